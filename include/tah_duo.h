@@ -390,7 +390,8 @@ typedef struct tah_sample_rows_args {
     const int32_t* add_prev;   /* optional int32 [rows]: a row whose entry is not 0 draws from logits_prev + logits, the sum
                                 * rounded to bf16 (the final logits of a token that took a second latent iteration) */
     const uint8_t* row_enable; /* optional, one byte per row: rows whose byte is 0 are skipped (outputs untouched) */
-    const float* uniforms;     /* float32 [rows], each in [0, 1): the caller's random numbers, one per row and call */
+    const float* uniforms;     /* float32 [rows], each in [0, 1): the caller's random numbers, one per row and call (with
+                                * uniform_step: [n_uniform_steps, rows]) */
     int64_t* tokens;           /* optional int64 [rows]: the drawn vocabulary index */
     float* probs;              /* optional float32 [rows, probs_row_stride]: the distribution drawn from (0 outside the filters) */
     int64_t logits_row_stride, prev_row_stride, probs_row_stride; /* elements */
@@ -398,6 +399,9 @@ typedef struct tah_sample_rows_args {
     float temperature;         /* > 0 */
     float top_p;               /* in (0, 1]; 1: no filter */
     float min_p;               /* in [0, 1]; 0: no filter */
+    const int32_t* uniform_step; /* optional int32 [rows]: row r's number is uniforms[uniform_step[r]][r] (an index outside the
+                                * table is moved to its nearest end), for batches whose rows are at tokens of different number */
+    int32_t n_uniform_steps;
 } tah_sample_rows_args;
 
 /* One token per row by temperature sampling with the min_p and top_p filters, in one launch and without a sort over
@@ -414,21 +418,25 @@ int tah_sample_rows(const tah_sample_rows_args* args, tah_stream_t stream);
 /* tah_qk_prep (append, one row per sequence) and tah_duo_decode in one launch, for a generation step: the workgroup
  * of a (query, kv head) prepares its query heads and the new K and V itself, stores K and V into the slabs and attends
  * over the cached rows and the new one.  `prep` and `dec` mean what they mean for the two calls (prep->q_out / k_out,
- * dec->q and the workspace are not used; prep->cache must be dec->c1 or dec->c2; row i of prep is query i of dec and
+ * dec->q is not used; prep->cache must be dec->c1 or dec->c2; row i of prep is query i of dec and
  * prep->slot_of[i], where not negative, is dec->q_slot[i]); cache contents and lengths are bit for bit those of the
  * two calls, the outputs too up to the last bit of a rare element (the same arithmetic in the same order, compiled
  * twice).  append_at: int32 [rows], the number of rows sequence i's segment of prep->cache holds before the
  * call, i.e. cache.len[slot] -- handed in because the workgroups of a sequence cannot read the length while one of
  * them advances it (len[slot] becomes append_at[i] + 1; a row whose append_at differs from the length sets
  * *prep->overflow to 2 where that flag is given: the slab then has a gap or an overwritten row; one query row per
- * slot and call).  Only for calls tah_duo_decode_step_supported() accepts (256
+ * slot and call).  For calls tah_duo_decode_step_supported() accepts (256
  * or more (query, kv head) pairs, slabs of at most 4096 rows, one or two query heads per kv head: cases
- * tah_duo_decode runs without split-K); others return TAH_E_SHAPE and the caller makes the two calls.  append_depth: NULL,
+ * tah_duo_decode runs without split-K), and with a workspace for fewer pairs or longer slabs: dec->workspace of at least
+ * tah_duo_decode_step_workspace_bytes() bytes, 16-byte aligned, zero before its first call and then left to these calls (it
+ * holds counters that every call returns to zero), one per sequence of calls that may overlap another (0: sizes no
+ * workspace helps).  Others return TAH_E_SHAPE and the caller makes the two calls.  append_depth: NULL,
  * or int32 [rows], 0 / 1 per row: the segment (dec->c1 / dec->c2) that row's K and V go to, for a batch whose rows are at
  * different latent iterations (append_at[i] then counts the rows of that segment, and prep->cache only has to be one of
  * the two).  Replaces, with
  * tah_qk_prep's and tah_duo_decode's lists, one more launch per layer and latent iteration. */
 int tah_duo_decode_step_supported(int32_t nq, int32_t hq, int32_t hkv, int32_t capacity1);
+size_t tah_duo_decode_step_workspace_bytes(int32_t nq, int32_t hq, int32_t hkv, int32_t capacity1, int32_t capacity2);
 int tah_duo_decode_step(const tah_qk_prep_args* prep, const tah_duo_decode_args* dec, const int32_t* append_at,
                         const int32_t* append_depth, tah_stream_t stream);
 

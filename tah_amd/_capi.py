@@ -232,6 +232,7 @@ class SampleRowsArgs(C.Structure):
         ("tokens", c_void_p), ("probs", c_void_p),
         ("logits_row_stride", c_int64), ("prev_row_stride", c_int64), ("probs_row_stride", c_int64),
         ("rows", c_int32), ("vocab", c_int32), ("temperature", c_float), ("top_p", c_float), ("min_p", c_float),
+        ("uniform_step", c_void_p), ("n_uniform_steps", c_int32),
     ]
 
 
@@ -357,6 +358,7 @@ PROTOTYPES = {
     "tah_qk_prep": (C.c_int, [C.POINTER(QkPrepArgs), c_void_p]),
     "tah_duo_decode_step": (C.c_int, [C.POINTER(QkPrepArgs), C.POINTER(DuoDecodeArgs), c_void_p, c_void_p, c_void_p]),
     "tah_duo_decode_step_supported": (C.c_int, [c_int32, c_int32, c_int32, c_int32]),
+    "tah_duo_decode_step_workspace_bytes": (C.c_size_t, [c_int32, c_int32, c_int32, c_int32, c_int32]),
     "tah_topk_mix": (C.c_int, [C.POINTER(TopkMixArgs), c_void_p]),
     "tah_qk_prep_bwd": (C.c_int, [C.POINTER(QkPrepBwdArgs), c_void_p]),
     "tah_sample_rows": (C.c_int, [C.POINTER(SampleRowsArgs), c_void_p]),

@@ -774,14 +774,19 @@ __global__ __launch_bounds__(256) void qk_prep_bwd_kernel(const PrepBwdParams p)
 }
 
 // ---- q/k preparation, append and attention of a decode step in one launch --------------------------------
-// What qk_prep_kernel (one row per sequence, append) followed by duo_decode_whole_kernel do, for calls the latter
-// takes: the workgroup of (query, kv head) prepares the G query heads and the new K and V of its kv head itself
-// (every 16-lane group of every wave repeats the few dozen operations: the prepared pieces are then where the row
-// loop wants them), one group stores K and V into the slabs for the steps to come, and the row loop takes the new
-// row from registers instead of reading back what is being written.  The place of the new row comes from the
-// caller (append_at[], the segment's length before the call): the eight workgroups of a sequence cannot read
-// len[] while one of them advances it.  Same arithmetic in the same order as the two kernels: the slabs get the
-// same bits, the outputs too except where the compiler contracted a multiply-add in one kernel and not the other.
+// What qk_prep_kernel (one row per sequence, append) followed by duo_decode_whole_kernel do: the workgroup of (query, kv
+// head) prepares the G query heads and the new K and V of its kv head itself, stores K and V into the slabs for the steps
+// to come, and the row loop takes the new row from LDS instead of reading back what is being written.  The place of the
+// new row comes from the caller (append_at[], the segment's length before the call): the eight workgroups of a sequence
+// cannot read len[] while one of them advances it.  Same arithmetic in the same order as the two kernels: the slabs
+// get the same bits, the outputs too except where the compiler contracted a multiply-add in one kernel and not the other.
+//
+// A call of a few sequences is a chain of dependent trips to memory, so the chain is kept short: wave 0 alone prepares,
+// all heads side by side, behind loads it issued first (every wave preparing everything for itself took 2 us of vector
+// issue, and the norm's row came back behind the cache rows), and where a sequence's rows lie is asked for together with
+// which sequence it is.  Measured in a replayed graph (16 / 8 heads), preparation + split-K + merge launches -> this one:
+// one sequence of 300 rows 13.6 -> 9.9 us, of 8000 18.4 -> 15.9 us; eight of up to 900 17.4 -> 14.0 us; 32 of up to 8000
+// (slabs of 8200) 152 -> 140 us.  The preparation by wave 0 is 2.5 to 3 us of that at few sequences.
 constexpr int kStepMaxGroup = 2;  // with four query heads per kv head the preparation no longer fits the 128 registers
 struct StepParams {
     PrepParams prep;
@@ -790,27 +795,65 @@ struct StepParams {
     const int32_t* append_at;
     const int32_t* append_depth;   // per row 0 / 1, or null: every row appends to segment `append_second`
     int32_t append_second;
+    float* part;                   // kSplit: partials [nq][hkv][nsplit][G][kPart] ...
+    int32_t* arrived;              // ... and workgroups of a pair that are done, [nq][hkv], 0 between calls
+    int32_t nsplit, fill;          // workgroups per pair at most, and as many as it takes to give every compute unit one
+    int32_t nslots1;               // slots of the depth-0 segment
 };
 
-template <int G>
+// Calls with too few (query, kv head) pairs to fill the chip, or slabs too long for one workgroup per pair: up to
+// kStepMaxSplit workgroups share a pair's rows (kSplit).  How many do is decided on the device from the rows there
+// are; the others leave at once.  The workgroup that finishes last merges the partials: they and the counter travel
+// through device-scope relaxed atomics, which go past the XCDs' L2 caches, so the hand-over needs no fence (a
+// device-scope fence writes the whole L2 back; it made the same idea cost 7 us).  The hand-over costs 3.9 us, a turn of the
+// sixteen waves 2.2 us: two turns stay with one workgroup (300 rows: 12.3 us against 14.0 shared by two), more are shared.
+// Once every compute unit has a workgroup a finer split only repeats the fixed 7 us: 32 x 8000 rows take 165 us at 1024
+// rows to a workgroup, 159 at 2048, 140 at 4096.
+constexpr int kStepMaxSplit = 32;
+constexpr int kStepRowsFew = 256;    // rows to a workgroup while the chip has idle compute units (one turn of its waves) ...
+constexpr int kStepRowsMany = 4096;  // ... and when all have work: the split only evens out their shares
+inline int step_fill(int nq, int hkv) { return (int)((kWholeMinPairs + (long)nq * hkv - 1) / ((long)nq * hkv)); }
+__host__ __device__ inline int step_splits_of(long rows, int fill) {
+    const long few = rows <= 2 * kStepRowsFew ? 1 : (rows + kStepRowsFew - 1) / kStepRowsFew, many = (rows + kStepRowsMany - 1) / kStepRowsMany;
+    const long n = few < fill ? few : fill, m = n > many ? n : many;
+    return (int)(m < 1 ? 1 : (m > kStepMaxSplit ? kStepMaxSplit : m));
+}
+
+template <int G, bool kSplit>
 __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const StepParams sp) {
     const PrepParams& pp = sp.prep;
     const DecParams& p = sp.dec;
     HIP_DYNAMIC_SHARED(unsigned char, smem_raw)
     float (*red)[G][kPart] = reinterpret_cast<float (*)[G][kPart]>(smem_raw);
-    __shared__ float xn_part[kWholeWaves];
+    __shared__ __align__(16) u32x4 ready[G + 2][16];  // the prepared query heads, K and V of the new row
     const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
     const int kq = lane / 16, dc = lane % 16;
     const int qi = blockIdx.x, hk = blockIdx.y;
-    // the row's data first: the loads fly while the bookkeeping is looked up
-    u32x4 xq[G];
+    // Wave 0 prepares the new row, a head per sixteen lanes (query heads, K, V); its loads go first, because a wave's loads
+    // return in order and everybody waits for what it makes of them.
+    constexpr int kPieces = G + 2;
+    const bool is_q = kq < G, is_v = kq > G;
+    u32x4 xin, wt, cs, sn, xn[4];
+    if (wave == 0) {
+        const int g = is_q ? kq : 0;
+        const __bf16* at = is_q ? pp.q + (int64_t)qi * pp.q_rs + (int64_t)(hk * G + g) * pp.q_hs
+                                : (is_v ? pp.v + (int64_t)qi * pp.v_rs + (int64_t)hk * pp.v_hs : pp.k + (int64_t)qi * pp.k_rs + (int64_t)hk * pp.k_hs);
+        xin = *reinterpret_cast<const u32x4*>(at + 8 * dc);
+        wt = *reinterpret_cast<const u32x4*>((is_q ? pp.qw : pp.kw) + 8 * dc);
+        cs = *reinterpret_cast<const u32x4*>(pp.cos + (int64_t)qi * pp.cs_rs + 8 * dc);
+        sn = *reinterpret_cast<const u32x4*>(pp.sin + (int64_t)qi * pp.cs_rs + 8 * dc);
+        if (pp.xn) {
+            const __bf16* xr = pp.xn + (int64_t)qi * pp.xn_rs;
 #pragma unroll
-    for (int g = 0; g < G; ++g) xq[g] = *reinterpret_cast<const u32x4*>(pp.q + (int64_t)qi * pp.q_rs + (int64_t)(hk * G + g) * pp.q_hs + 8 * dc);
-    u32x4 xk = *reinterpret_cast<const u32x4*>(pp.k + (int64_t)qi * pp.k_rs + (int64_t)hk * pp.k_hs + 8 * dc);
-    u32x4 xv = *reinterpret_cast<const u32x4*>(pp.v + (int64_t)qi * pp.v_rs + (int64_t)hk * pp.v_hs + 8 * dc);
-    const u32x4 cs = *reinterpret_cast<const u32x4*>(pp.cos + (int64_t)qi * pp.cs_rs + 8 * dc);
-    const u32x4 sn = *reinterpret_cast<const u32x4*>(pp.sin + (int64_t)qi * pp.cs_rs + 8 * dc);
-    const u32x4 qw = *reinterpret_cast<const u32x4*>(pp.qw + 8 * dc), kw = *reinterpret_cast<const u32x4*>(pp.kw + 8 * dc);
+            for (int i = 0; i < 4; ++i) {
+                const int c = (64 * i + lane) * 8;
+                xn[i] = *reinterpret_cast<const u32x4*>(xr + (c < pp.xn_cols ? c : 0));
+            }
+        }
+    }
+    // where the sequence's rows lie, asked for together with which sequence it is: row i of a generation step is slot i
+    const int guess = qi < sp.nslots1 ? qi : sp.nslots1 - 1;
+    int start1 = *(guess >= 0 ? p.c1.start + guess : p.q_slot + qi), len1 = *(guess >= 0 ? p.c1.len + guess : p.q_slot + qi);
     const int slot = p.q_slot[qi];
     const int qpos = p.q_pos[qi];
     const int qdepth = p.q_depth ? p.q_depth[qi] : p.depth;
@@ -820,65 +863,80 @@ __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const St
     const int adepth = sp.append_depth ? (sp.append_depth[qi] != 0 ? 1 : 0) : sp.append_second;  // uniform per workgroup
     const AppendParams& ap = sp.app[adepth];
     const bool cached = aslot >= 0, fits = cached && dst < ap.capacity;
+    if (slot >= 0 && slot != guess) {  // uniform per workgroup
+        start1 = p.c1.start[slot];
+        len1 = p.c1.len[slot];
+    }
     // rows of a segment: with the new row where this call appends (nobody may read len[] of that segment here)
     auto visible = [&](int seg) {
-        const Seg& sg = seg ? p.c2 : p.c1;
         if (slot < 0 || (seg && qdepth < 1)) return 0;  // (slot < 0: a query without a sequence)
-        const int n = (seg == adepth && cached) ? (fits ? dst + 1 : (dst < ap.capacity ? dst : ap.capacity)) : sg.len[slot];
+        const int n = (seg == adepth && cached) ? (fits ? dst + 1 : (dst < ap.capacity ? dst : ap.capacity)) : (seg ? p.c2.len[slot] : len1);
         return seg ? n : (qpos + 1 < n ? (qpos + 1 > 0 ? qpos + 1 : 0) : n);
     };
     constexpr int kBlock = 4 * kUnroll;
     // this wave's first block of cached rows goes on its way before the preparation below, which needs none of it
     const int nvis0 = visible(0);
-    const int64_t base0 = slot < 0 ? 0 : p.c1.start[slot];
+    int nact = 1, split = 0;  // workgroups at work on this pair, and which of them this one is
+    if constexpr (kSplit) {
+        split = blockIdx.z;
+        const int want = step_splits_of(nvis0 + visible(1), sp.fill);
+        nact = want > sp.nsplit ? sp.nsplit : want;
+        if (split >= nact) return;  // uniform per workgroup
+    }
+    const int row_first = (split * kWholeWaves + wave) * kBlock, row_step = nact * kWholeWaves * kBlock;
+    const int64_t base0 = slot < 0 ? 0 : start1;
     const __bf16* kbase0 = p.c1.k + base0 * p.c1.k_rs + (int64_t)hk * p.c1.k_hs + dc * 8;
     const __bf16* vbase0 = p.c1.v + base0 * p.c1.v_rs + (int64_t)hk * p.c1.v_hs + dc * 8;
     RowBlock<kUnroll> first;
-    const bool have_first = wave * kBlock < nvis0;  // uniform per wave
-    if (have_first) load_rows<kUnroll>(first, p.c1, false, kbase0, vbase0, nullptr, wave * kBlock, nvis0, kq);
-    float rin = 1.0f;
-    if (pp.xn) {
-        const __bf16* xr = pp.xn + (int64_t)qi * pp.xn_rs;
-        float ss = 0.f;
-        // summed as qk_prep_kernel's 256 threads sum it (same strides, same order), so that the factor has the same bits
-        if (tid < 256)
-            for (int c = tid * 8; c < pp.xn_cols; c += 256 * 8) {
-                const u32x4 x = *reinterpret_cast<const u32x4*>(xr + c);
+    const bool have_first = row_first < nvis0;  // uniform per wave
+    if (have_first) load_rows<kUnroll>(first, p.c1, false, kbase0, vbase0, nullptr, row_first, nvis0, kq);
+    if (wave == 0) {
+        if (pp.xn) {
+            // summed as qk_prep_kernel's 256 threads sum it (same strides, same order), so that the factor has the same bits
+            const __bf16* xr = pp.xn + (int64_t)qi * pp.xn_rs;
+            float ss[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) ss += bf16_lo(x[i]) * bf16_lo(x[i]) + bf16_hi(x[i]) * bf16_hi(x[i]);
+            for (int w = 0; w < 4; ++w) {
+                ss[w] = 0.f;
+                for (int c = (64 * w + lane) * 8; c < pp.xn_cols; c += 256 * 8) {
+                    const u32x4 x = c < 256 * 8 ? xn[w] : *reinterpret_cast<const u32x4*>(xr + c);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) ss[w] += bf16_lo(x[i]) * bf16_lo(x[i]) + bf16_hi(x[i]) * bf16_hi(x[i]);
+                }
             }
 #pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m);
-        if (lane == 0) xn_part[wave] = ss;
-        __syncthreads();
-        ss = (xn_part[0] + xn_part[1]) + (xn_part[2] + xn_part[3]);
-        rin = __builtin_amdgcn_rsqf(ss / (float)pp.xn_cols + pp.xn_eps);
+            for (int m = 32; m >= 1; m >>= 1)
 #pragma unroll
-        for (int g = 0; g < G; ++g) xq[g] = scale_piece(xq[g], rin);
-        xk = scale_piece(xk, rin);
-        xv = scale_piece(xv, rin);
-    }
-    const uint32_t sign = dc < 8 ? 0x80008000u : 0u;
-    u32x4 qv[G];
+                for (int w = 0; w < 4; ++w) ss[w] += __shfl_xor(ss[w], m);
+            const float total = (ss[0] + ss[1]) + (ss[2] + ss[3]);
+            xin = scale_piece(xin, __builtin_amdgcn_rsqf(total / (float)pp.xn_cols + pp.xn_eps));
+        }
+        u32x4 out = prep_head_piece(xin, wt, cs, sn, dc < 8 ? 0x80008000u : 0u, pp.eps);
 #pragma unroll
-    for (int g = 0; g < G; ++g) qv[g] = prep_head_piece(xq[g], qw, cs, sn, sign, pp.eps);
-    SubRow sub;
-    sub.k = prep_head_piece(xk, kw, cs, sn, sign, pp.eps);
-    sub.v = xv;
-    sub.pos = pos_new;
-    if (cached && !fits && pp.a.overflow && tid == 0 && hk == 0) *pp.a.overflow = 1;
-    if (fits && wave == 0 && kq == 0) {
-        const int64_t drow = (int64_t)const_i32(ap.start, aslot) + dst;
-        *reinterpret_cast<u32x4*>(ap.ck + drow * ap.ck_rs + (int64_t)hk * ap.ck_hs + 8 * dc) = sub.k;
-        *reinterpret_cast<u32x4*>(ap.cv + drow * ap.cv_rs + (int64_t)hk * ap.cv_hs + 8 * dc) = sub.v;
-        if (dc == 0 && hk == 0) {
-            if (ap.cpos && pp.a.pos_new) ap.cpos[(int64_t)aslot * ap.capacity + dst] = pos_new;
-            // (only this workgroup touches the length of the segment the row appends to)  A row placed anywhere but
-            // at the end of its slab leaves a gap of stale rows or overwrites cached ones: reported, not repaired.
-            if (ap.len[aslot] != dst && pp.a.overflow) *pp.a.overflow = 2;
-            ap.len[aslot] = dst + 1;
+        for (int i = 0; i < 4; ++i) out[i] = is_v ? xin[i] : out[i];
+        if (kq < kPieces) ready[kq][dc] = out;
+        if (cached && !fits && pp.a.overflow && tid == 0 && hk == 0 && split == 0) *pp.a.overflow = 1;
+        if (fits && split == 0 && kq >= G && kq < kPieces) {
+            const int64_t drow = (int64_t)const_i32(ap.start, aslot) + dst;
+            __bf16* to = is_v ? ap.cv + drow * ap.cv_rs + (int64_t)hk * ap.cv_hs : ap.ck + drow * ap.ck_rs + (int64_t)hk * ap.ck_hs;
+            *reinterpret_cast<u32x4*>(to + 8 * dc) = out;
+            if (dc == 0 && hk == 0 && !is_v) {
+                if (ap.cpos && pp.a.pos_new) ap.cpos[(int64_t)aslot * ap.capacity + dst] = pos_new;
+                // (only this workgroup touches the length of the segment the row appends to)  A row placed anywhere but
+                // at the end of its slab leaves a gap of stale rows or overwrites cached ones: reported, not repaired.
+                if (ap.len[aslot] != dst && pp.a.overflow) *pp.a.overflow = 2;
+                ap.len[aslot] = dst + 1;
+            }
         }
     }
+    __syncthreads();
+    u32x4 qv[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) qv[g] = ready[g][dc];
+    SubRow sub;
+    sub.k = ready[G][dc];
+    sub.v = ready[G + 1][dc];
+    sub.pos = pos_new;
     float m_run[G], l_run[G], acc[G][8];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
@@ -889,8 +947,8 @@ __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const St
     }
     // depth-0 segment: the block loaded above, then the wave's other turns
     sub.row = (adepth == 0 && fits) ? dst : -1;
-    if (have_first) attend_rows<G, kUnroll, true>(first, false, wave * kBlock, kq, qpos, p.scale_log2e, qv, m_run, l_run, acc, &sub);
-    for (int r_it = (wave + kWholeWaves) * kBlock; r_it < nvis0; r_it += kWholeWaves * kBlock)
+    if (have_first) attend_rows<G, kUnroll, true>(first, false, row_first, kq, qpos, p.scale_log2e, qv, m_run, l_run, acc, &sub);
+    for (int r_it = row_first + row_step; r_it < nvis0; r_it += row_step)
         consume_rows<G, kUnroll, true>(p.c1, false, kbase0, vbase0, nullptr, r_it, nvis0, kq, qpos, p.scale_log2e, qv, m_run, l_run, acc, &sub);
     // depth-1 segment
     const int nvis1 = visible(1);
@@ -900,7 +958,7 @@ __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const St
         const __bf16* kbase1 = p.c2.k + base1 * p.c2.k_rs + (int64_t)hk * p.c2.k_hs + dc * 8;
         const __bf16* vbase1 = p.c2.v + base1 * p.c2.v_rs + (int64_t)hk * p.c2.v_hs + dc * 8;
         const int32_t* posbase = p.c2.pos + (int64_t)slot * p.c2.capacity;
-        for (int r_it = wave * kBlock; r_it < nvis1; r_it += kWholeWaves * kBlock)
+        for (int r_it = row_first; r_it < nvis1; r_it += row_step)
             consume_rows<G, kUnroll, true>(p.c2, true, kbase1, vbase1, posbase, r_it, nvis1, kq, qpos, p.scale_log2e, qv, m_run, l_run, acc, &sub);
     }
     combine_row_groups<G>(m_run, l_run, acc);
@@ -910,6 +968,73 @@ __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const St
         const int g = e / kD, d = e % kD;
         float a, l, mx;
         merge16<G>(red, g, d, a, l, mx);
+        const int head = hk * G + g;
+        if (kSplit && nact > 1) {
+            float* out = sp.part + (((int64_t)qi * p.hkv + hk) * sp.nsplit + split) * (G * kPart) + g * kPart;
+            device_store(out + d, a);
+            if (d == 0) {
+                device_store(out + kD, mx);
+                device_store(out + kD + 1, l);
+            }
+            continue;
+        }
+        store_output(p, qi, head, d, l > 0.f ? a / l : 0.f);
+        if (p.lse && d == 0) p.lse[(int64_t)qi * p.hq + head] = l > 0.f ? (mx + fast_log2(l)) * kLn2 : kNegInf;
+    }
+    if constexpr (kSplit) {
+        if (nact == 1) return;
+        TAH_WAIT_VMEM();  // every wave's partials have left before its workgroup is counted
+        __syncthreads();
+        __shared__ int last;
+        int32_t* const count = sp.arrived + qi * p.hkv + hk;
+        if (tid == 0) last = device_add(count, 1) == nact - 1;
+        __syncthreads();
+        if (!last) return;
+        if (tid == 0) device_store(count, 0);  // ready for the next launch
+        // kLanes threads per element of the output take the partials in turn, their loads all on their way at once
+        constexpr int kElems = G * kD, kLanes = kWholeThreads / kElems, kTurns = kStepMaxSplit / kLanes;
+        const int e = tid % kElems, j0 = tid / kElems, g = e / kD, d = e % kD;
+        const float* base = sp.part + ((int64_t)qi * p.hkv + hk) * sp.nsplit * (G * kPart) + g * kPart;
+        float pa[kTurns], pm[kTurns], pl[kTurns];
+#pragma unroll
+        for (int t = 0; t < kTurns; ++t) {
+            const int j = j0 + t * kLanes;
+            const float* at = base + (int64_t)(j < nact ? j : 0) * (G * kPart);
+            pa[t] = device_load(at + d);
+            pm[t] = device_load(at + kD);
+            pl[t] = device_load(at + kD + 1);
+            if (j >= nact) pm[t] = kNegInf;
+        }
+        float mx = kNegInf, a = 0.f, l = 0.f;
+#pragma unroll
+        for (int t = 0; t < kTurns; ++t) mx = fmaxf(mx, pm[t]);
+        const float m_use = mx == kNegInf ? 0.f : mx;
+#pragma unroll
+        for (int t = 0; t < kTurns; ++t) {
+            const float w = fast_exp2(pm[t] - m_use);
+            a += w * pa[t];
+            l += w * pl[t];
+        }
+        // (the last reads of red are behind two barriers)
+        red[j0][g][d] = a;
+        if (d == 0) {
+            red[j0][g][kD] = mx;
+            red[j0][g][kD + 1] = l;
+        }
+        __syncthreads();
+        if (j0 != 0) return;
+        float am[kLanes];
+        mx = kNegInf;
+#pragma unroll
+        for (int j = 0; j < kLanes; ++j) mx = fmaxf(mx, am[j] = red[j][g][kD]);
+        const float top = mx == kNegInf ? 0.f : mx;
+        a = l = 0.f;
+#pragma unroll
+        for (int j = 0; j < kLanes; ++j) {
+            const float w = fast_exp2(am[j] - top);
+            a += w * red[j][g][d];
+            l += w * red[j][g][kD + 1];
+        }
         const int head = hk * G + g;
         store_output(p, qi, head, d, l > 0.f ? a / l : 0.f);
         if (p.lse && d == 0) p.lse[(int64_t)qi * p.hq + head] = l > 0.f ? (mx + fast_log2(l)) * kLn2 : kNegInf;
@@ -1215,11 +1340,23 @@ namespace {
 template <int G>
 int launch_step(const StepParams& sp, hipStream_t st) {
     constexpr int kRedBytes = 16 * G * kPart * (int)sizeof(float);
-    hipLaunchKernelGGL((duo_decode_step_kernel<G>), dim3(sp.dec.nq, sp.dec.hkv), dim3(kWholeThreads), kRedBytes, st, sp);
+    if (sp.part)
+        hipLaunchKernelGGL((duo_decode_step_kernel<G, true>), dim3(sp.dec.nq, sp.dec.hkv, sp.nsplit), dim3(kWholeThreads), kRedBytes, st, sp);
+    else
+        hipLaunchKernelGGL((duo_decode_step_kernel<G, false>), dim3(sp.dec.nq, sp.dec.hkv), dim3(kWholeThreads), kRedBytes, st, sp);
     return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
 }
+size_t step_counter_bytes(int nq, int hkv) { return ((size_t)nq * hkv * sizeof(int32_t) + 255) / 256 * 256; }  // then the partials
 }  // namespace
 }  // namespace tah
+
+extern "C" size_t tah_duo_decode_step_workspace_bytes(int32_t nq, int32_t hq, int32_t hkv, int32_t capacity1, int32_t capacity2) {
+    using namespace tah;
+    if (nq <= 0 || hq <= 0 || hkv <= 0 || hq % hkv || capacity1 <= 0 || capacity2 < 0) return 0;
+    const int g = hq / hkv;
+    if ((g != 1 && g != 2) || g > kStepMaxGroup || nq > 65535 || hkv > 65535) return 0;
+    return step_counter_bytes(nq, hkv) + (size_t)nq * hq * step_splits_of((long)capacity1 + capacity2, step_fill(nq, hkv)) * kPart * sizeof(float);
+}
 
 extern "C" int tah_duo_decode_step_supported(int32_t nq, int32_t hq, int32_t hkv, int32_t capacity1) {
     if (nq <= 0 || hq <= 0 || hkv <= 0 || hq % hkv) return 0;
@@ -1255,15 +1392,30 @@ extern "C" int tah_duo_decode_step(const tah_qk_prep_args* prep, const tah_duo_d
     // one row per sequence, appended to one of the two segments the queries read, in a call the one-workgroup kernel takes
     if (rc_p == 1 || rc_d == 1 || prep->rows != dec->nq || prep->hq != dec->hq || prep->hkv != dec->hkv) return TAH_E_SHAPE;
     if (!prep->append || !prep->append_one_row_per_seq || prep->nseq != prep->rows || !prep->v) return TAH_E_SHAPE;
-    if (!tah_duo_decode_step_supported(dec->nq, dec->hq, dec->hkv, dec->c1.capacity)) return TAH_E_SHAPE;
-    if (!append_at) return TAH_E_NULL;
     const bool have2 = dec->q_depth != nullptr || dec->depth >= 1;
+    sp.part = nullptr;
+    sp.arrived = nullptr;
+    sp.nsplit = 1;
+    sp.fill = 1;
+    if (!tah_duo_decode_step_supported(dec->nq, dec->hq, dec->hkv, dec->c1.capacity)) {
+        const int cap2 = have2 ? dec->c2.capacity : 0;
+        const size_t need = tah_duo_decode_step_workspace_bytes(dec->nq, dec->hq, dec->hkv, dec->c1.capacity, cap2);
+        if (!need || !dec->workspace) return TAH_E_SHAPE;
+        if (!aligned16(dec->workspace)) return TAH_E_ALIGN;
+        if (dec->workspace_bytes < need) return TAH_E_WORKSPACE;
+        sp.arrived = static_cast<int32_t*>(dec->workspace);
+        sp.part = reinterpret_cast<float*>(static_cast<unsigned char*>(dec->workspace) + step_counter_bytes(dec->nq, dec->hkv));
+        sp.fill = step_fill(dec->nq, dec->hkv);
+        sp.nsplit = step_splits_of((long)dec->c1.capacity + cap2, sp.fill);
+    }
+    if (!append_at) return TAH_E_NULL;
     if (prep->cache.k == dec->c1.k) sp.append_second = 0;
     else if (prep->cache.k == dec->c2.k && have2) sp.append_second = 1;
     else return TAH_E_SHAPE;
     if (append_depth && !have2) return TAH_E_SHAPE;  // rows that append to the depth-1 segment need it
     sp.app[0] = append_target(dec->c1);
     sp.app[1] = have2 ? append_target(dec->c2) : AppendParams{};
+    sp.nslots1 = dec->c1.nslots;
     sp.append_at = append_at;
     sp.append_depth = append_depth;
     hipStream_t st = static_cast<hipStream_t>(stream);

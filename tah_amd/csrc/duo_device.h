@@ -31,6 +31,18 @@ typedef __attribute__((address_space(3))) int lds_int;
 #define TAH_LDS_CAST(T, p) (reinterpret_cast<__attribute__((address_space(3))) T*>(p))
 #endif
 
+// Words that workgroups on different XCDs hand to each other inside one launch: device-scope relaxed atomics, which pass by
+// the caches that are not shared.  Order between them is the caller's (TAH_WAIT_VMEM between a store and what announces it).
+#ifdef TAH_CPU_EMU
+template <class T> inline void device_store(T* p, T v) { __atomic_store(p, &v, __ATOMIC_SEQ_CST); }
+template <class T> inline T device_load(const T* p) { T v; __atomic_load(const_cast<T*>(p), &v, __ATOMIC_SEQ_CST); return v; }
+inline int device_add(int32_t* p, int v) { return __atomic_fetch_add(p, v, __ATOMIC_SEQ_CST); }
+#else
+template <class T> __device__ __forceinline__ void device_store(T* p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <class T> __device__ __forceinline__ T device_load(const T* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ int device_add(int32_t* p, int v) { return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+#endif
+
 constexpr int kWave = 64;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;

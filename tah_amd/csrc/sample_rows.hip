@@ -39,6 +39,8 @@ struct SampleParams {
     const int32_t* add_prev;
     const uint8_t* row_enable;
     const float* uniforms;
+    const int32_t* uniform_step;  // rows take their number from a table [n_uniform_steps][rows], or null
+    int32_t n_uniform_steps;
     int64_t* tokens;
     float* probs;
     int64_t l_rs, p_rs, pr_rs;
@@ -415,7 +417,12 @@ __global__ __launch_bounds__(kSmpThreads) void sample_rows_kernel(const SamplePa
 
     // ---- the draw: the token at which the kept mass, in the same order, passes u Z --------------------------
     if (p.tokens) {
-        const float tu = p.uniforms[row] * Z;
+        int64_t ui = row;
+        if (p.uniform_step) {
+            const int s = p.uniform_step[row], top = p.n_uniform_steps - 1;
+            ui += (int64_t)(s < 0 ? 0 : s > top ? top : s) * p.rows;
+        }
+        const float tu = p.uniforms[ui] * Z;
         const int dcode = locate(tu, cut_code, 1);
         const uint32_t* cnt = group_counts(dcode);
         const uint32_t gbase = (dcode >> 10) * (uint32_t)kWinKeys + (uint32_t)(dcode & (kSmpThreads - 1)) * kBinsPerThread;
@@ -560,6 +567,8 @@ extern "C" int tah_sample_rows(const tah_sample_rows_args* a, tah_stream_t strea
     p.add_prev = a->add_prev;
     p.row_enable = a->row_enable;
     p.uniforms = a->uniforms;
+    p.uniform_step = a->uniform_step;
+    p.n_uniform_steps = a->n_uniform_steps;
     p.tokens = a->tokens;
     p.probs = a->probs;
     p.l_rs = a->logits_row_stride; p.p_rs = a->prev_row_stride; p.pr_rs = a->probs_row_stride;

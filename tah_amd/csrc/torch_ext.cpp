@@ -56,6 +56,7 @@ void load_library(const std::string& path, bool allow_host) {
     bind(g.qk_prep, "tah_qk_prep");
     bind(g.decode_step, "tah_duo_decode_step");
     bind(g.decode_step_supported, "tah_duo_decode_step_supported");
+    bind(g.decode_step_workspace_bytes, "tah_duo_decode_step_workspace_bytes");
     bind(g.topk_mix, "tah_topk_mix");
     bind(g.qk_prep_bwd, "tah_qk_prep_bwd");
     bind(g.sample_rows, "tah_sample_rows");
@@ -505,6 +506,11 @@ bool duo_decode_step_supported(int64_t nq, int64_t hq, int64_t hkv, int64_t capa
     return g.decode_step_supported((int32_t)nq, (int32_t)hq, (int32_t)hkv, (int32_t)capacity1) != 0;
 }
 
+int64_t duo_decode_step_workspace_bytes(int64_t nq, int64_t hq, int64_t hkv, int64_t capacity1, int64_t capacity2) {
+    need_lib();
+    return (int64_t)g.decode_step_workspace_bytes((int32_t)nq, (int32_t)hq, (int32_t)hkv, (int32_t)capacity1, (int32_t)capacity2);
+}
+
 // qk_prep (append, one row per sequence) + duo_decode in one launch (tah_duo_decode_step).  The slabs the new K/V go to
 // (ck, cv, ...) must be those of one of the two segments read.
 void duo_decode_step(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& q_weight, const Tensor& k_weight,
@@ -515,9 +521,10 @@ void duo_decode_step(const Tensor& q, const Tensor& k, const Tensor& v, const Te
                      const optional<Tensor>& append_depth, const Tensor& o, const optional<Tensor>& lse, const Tensor& q_slot, const Tensor& q_pos,
                      const optional<Tensor>& q_depth, int64_t depth, const Tensor& k1, const Tensor& v1, const Tensor& start1,
                      const Tensor& len1, const optional<Tensor>& k2, const optional<Tensor>& v2, const optional<Tensor>& pos2,
-                     const optional<Tensor>& start2, const optional<Tensor>& len2, double scale, const optional<Tensor>& o_packed) {
+                     const optional<Tensor>& start2, const optional<Tensor>& len2, double scale, const optional<Tensor>& o_packed,
+                     const optional<Tensor>& workspace) {
     need_lib();
-    Dev d; d.see(append_at); d.see(append_depth);
+    Dev d; d.see(append_at); d.see(append_depth); d.see(workspace);
     i32(append_at, "append_at");
     TORCH_CHECK(append_at.numel() == q.size(0), "duo_decode_step: append_at must have one entry per row");
     if (append_depth.has_value()) {
@@ -526,8 +533,13 @@ void duo_decode_step(const Tensor& q, const Tensor& k, const Tensor& v, const Te
     }
     const tah_qk_prep_args pa = prep_args(d, q, k, v, c10::nullopt, c10::nullopt, q_weight, k_weight, cos, sin, eps, ck, cv, cpos, start, len,
                                           overflow, cu_new, pos_new, slot_of, true, c10::nullopt, norm_input, norm_eps);
-    const tah_duo_decode_args da = decode_args(d, c10::nullopt, o, lse, q_slot, q_pos, q_depth, depth, k1, v1, start1, len1, k2, v2, pos2,
-                                               start2, len2, scale, o_packed);
+    tah_duo_decode_args da = decode_args(d, c10::nullopt, o, lse, q_slot, q_pos, q_depth, depth, k1, v1, start1, len1, k2, v2, pos2,
+                                         start2, len2, scale, o_packed);
+    if (workspace.has_value()) {
+        TORCH_CHECK(workspace->is_contiguous(), "duo_decode_step: the workspace must be contiguous");
+        da.workspace = workspace->data_ptr();
+        da.workspace_bytes = (size_t)workspace->numel() * workspace->element_size();
+    }
     check_rc(g.decode_step(&pa, &da, static_cast<const int32_t*>(append_at.data_ptr()),
                            append_depth.has_value() ? static_cast<const int32_t*>(append_depth->data_ptr()) : nullptr, d.stream()),
              "tah_duo_decode_step");
@@ -657,7 +669,7 @@ Tensor topk_values(const Tensor& logits, int64_t topk, const optional<Tensor>& i
 // `probs_out` (float32 [rows, V]) with the distribution drawn from when it is given; without `uniforms` only that
 void sample_rows(const Tensor& logits, const optional<Tensor>& logits_prev, const optional<Tensor>& add_prev,
                  const optional<Tensor>& uniforms, const optional<Tensor>& tokens_out, const optional<Tensor>& probs_out,
-                 const optional<Tensor>& row_enable, double temperature, double top_p, double min_p) {
+                 const optional<Tensor>& row_enable, double temperature, double top_p, double min_p, const optional<Tensor>& uniform_step) {
     need_lib();
     Dev d; d.see(logits);
     TORCH_CHECK(logits.dim() == 2 && logits.scalar_type() == at::kBFloat16 && logits.stride(1) == 1,
@@ -683,8 +695,18 @@ void sample_rows(const Tensor& logits, const optional<Tensor>& logits_prev, cons
     }
     if (uniforms.has_value()) {
         d.see(*uniforms);
-        TORCH_CHECK(uniforms->scalar_type() == at::kFloat && uniforms->is_contiguous() && uniforms->numel() == rows && tokens_out.has_value(),
-                    "sample_rows: uniforms must be a contiguous float32 [rows] tensor, given together with tokens_out");
+        if (uniform_step.has_value()) {
+            d.see(*uniform_step);
+            i32(*uniform_step, "sample_rows: uniform_step");
+            TORCH_CHECK(uniform_step->numel() == rows && uniforms->scalar_type() == at::kFloat && uniforms->is_contiguous() &&
+                            uniforms->dim() == 2 && uniforms->size(0) >= 1 && uniforms->size(1) == rows && tokens_out.has_value(),
+                        "sample_rows: with uniform_step [rows] uniforms must be a contiguous float32 [steps, rows] tensor, given together with tokens_out");
+            a.uniform_step = static_cast<const int32_t*>(uniform_step->data_ptr());
+            a.n_uniform_steps = (int32_t)uniforms->size(0);
+        } else {
+            TORCH_CHECK(uniforms->scalar_type() == at::kFloat && uniforms->is_contiguous() && uniforms->numel() == rows && tokens_out.has_value(),
+                        "sample_rows: uniforms must be a contiguous float32 [rows] tensor, given together with tokens_out");
+        }
         d.see(*tokens_out);
         TORCH_CHECK(tokens_out->scalar_type() == at::kLong && tokens_out->is_contiguous() && tokens_out->numel() == rows,
                     "sample_rows: tokens_out must be a contiguous int64 [rows] tensor");
@@ -1008,6 +1030,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("silu_mul", &silu_mul);
     m.def("duo_decode_step", &duo_decode_step);
     m.def("duo_decode_step_supported", &duo_decode_step_supported);
+    m.def("duo_decode_step_workspace_bytes", &duo_decode_step_workspace_bytes);
     m.def("step_begin", &step_begin);
     m.def("greedy_tick", &greedy_tick);
     m.def("decider_tail", &decider_tail);

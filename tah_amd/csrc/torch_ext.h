@@ -54,6 +54,7 @@ struct Api {
     Entry<decltype(&tah_qk_prep)> qk_prep;
     Entry<decltype(&tah_duo_decode_step)> decode_step;
     Entry<decltype(&tah_duo_decode_step_supported)> decode_step_supported;
+    Entry<decltype(&tah_duo_decode_step_workspace_bytes)> decode_step_workspace_bytes;
     Entry<decltype(&tah_topk_mix)> topk_mix;
     Entry<decltype(&tah_qk_prep_bwd)> qk_prep_bwd;
     Entry<decltype(&tah_sample_rows)> sample_rows;

@@ -39,7 +39,8 @@ import torch.nn.functional as F
 
 from . import ops
 from ._capi import TahDuoError
-from .kv_cache import KvSlabs, decode as _decode, decode_step as _decode_step, decode_step_supported, qk_norm_rope
+from .kv_cache import (KvSlabs, decode as _decode, decode_step as _decode_step, decode_step_supported, decode_step_workspace,
+                       qk_norm_rope)
 
 
 @dataclasses.dataclass
@@ -443,8 +444,13 @@ class TaHDecodeEngine(DecodeEngine):
         # depth-1 rows every sequence has cached (what each slabs1[l].len holds), kept once for the fused step kernel
         self.hard_len = torch.zeros(batch, dtype=torch.int32, device=dev)
         # q/k preparation, append and attention of a layer in one launch where the library takes the sizes
-        self.fused_step = bool(self.packed_linear and self.device.type == "cuda"
-                               and decode_step_supported(batch, cfg.hq, cfg.hkv, max_len))
+        # (small batches and long slabs: through a workspace of the engine's own, since engines may run side by side)
+        fused = self.packed_linear and self.device.type == "cuda"
+        self.step_workspace = None
+        if fused and not decode_step_supported(batch, cfg.hq, cfg.hkv, max_len):
+            self.step_workspace = decode_step_workspace(batch, cfg.hq, cfg.hkv, max_len, self.max_hard, self.device)
+            fused = self.step_workspace is not None
+        self.fused_step = bool(fused)
         if self.packed_linear:  # rows operands handed from kernel to kernel (32 rows each; rows past the batch stay zero)
             z = lambda n: torch.zeros(32 * n, dtype=torch.bfloat16, device=dev)
             self.xp, self.op, self.actp = z(cfg.hidden), z(cfg.hq * cfg.head_dim), z(cfg.intermediate)
@@ -471,6 +477,10 @@ class TaHDecodeEngine(DecodeEngine):
             self.eligible = torch.zeros(batch, dtype=torch.bool, device=dev)
             self.logits2 = [torch.zeros(batch, cfg.vocab, dtype=torch.bfloat16, device=dev) for _ in range(2)]
         self._tick_graphs = None
+        # Engines with a workspace draw a row's n-th token with the number a step-wise loop would draw it with: a table of the
+        # steps' uniforms, one row per token, so that sampled tokens do not depend on the schedule either.
+        self.uniforms = (torch.zeros(max_len + 1, batch, dtype=torch.float32, device=dev)
+                         if self.can_run_continuous and self.step_workspace is not None else None)
         self.decider = decider
         if decider is not None:
             if decider.hidden_states_size != cfg.hidden:
@@ -585,13 +595,13 @@ class TaHDecodeEngine(DecodeEngine):
                 _decode_step(q, k, v, L["qn"], L["kn"], cos, sin, c.rms_eps, cache=self.slabs1[l], cu_new=self.cu_rows,
                              append_at=self.append_at, append_depth=q_depth, q_slot=self.rows, q_pos=q_pos,
                              c1=self.slabs0[l], c2=self.slabs1[l], scale=self.scale, slot_of=slot_of, pos_new=pos,
-                             norm_input=x, norm_eps=c.rms_eps, q_depth=q_depth, out_packed=self.op)
+                             norm_input=x, norm_eps=c.rms_eps, q_depth=q_depth, out_packed=self.op, workspace=self.step_workspace)
             elif self.fused_step:
                 _decode_step(q, k, v, L["qn"], L["kn"], cos, sin, c.rms_eps, cache=cache, cu_new=self.cu_rows,
                              append_at=pos if depth == 0 else self.hard_len, q_slot=self.rows, q_pos=q_pos,
                              c1=self.slabs0[l], c2=self.slabs1[l], scale=self.scale, slot_of=slot_of,
                              pos_new=pos if depth == 1 else None, norm_input=x, norm_eps=c.rms_eps, q_depth=q_depth,
-                             out_packed=self.op)
+                             out_packed=self.op, workspace=self.step_workspace)
             else:
                 qo, _ = qk_norm_rope(q, k, L["qn"], L["kn"], cos, sin, c.rms_eps, v=v, cache=cache, cu_new=self.cu_rows,
                                      slot_of=slot_of, pos_new=pos if depth == 1 else None, one_row_per_seq=True,
@@ -817,11 +827,12 @@ class TaHDecodeEngine(DecodeEngine):
         greedy_fused = temperature <= 0.0 and self.fused_greedy and self.cfg.vocab % 8 == 0
         can_tick = self.can_run_continuous and self.fused_greedy and self.cfg.vocab % 8 == 0
         if continuous is None:
-            continuous = can_tick and self.use_fused_glue and not self.measure_without_attention
+            continuous = (can_tick and self.use_fused_glue and not self.measure_without_attention
+                          and (temperature <= 0.0 or self.uniforms is None or self._draws_by_step(temperature, filters)))
         if continuous:
             if not can_tick:
                 raise TahDuoError("continuous generation needs the fused attention and glue launches "
-                                  "(at most 32 rows, 256 (row, kv head) pairs, slabs of at most 4096 rows)")
+                                  "(at most 32 rows, one or two query heads per kv head)")
             return self._generate_ticks(first_logits, max_new_tokens, eos, use_graph and dev.type == "cuda",
                                         temperature=temperature, **filters)
         return super().generate(first_logits, max_new_tokens, temperature=temperature, eos=eos, use_graph=use_graph,
@@ -834,6 +845,11 @@ class TaHDecodeEngine(DecodeEngine):
     def _advanced(self, steps: int) -> None:
         self.host_positions += steps
         self.host_hard_rows += steps
+
+    def _draws_by_step(self, temperature: float, filters: dict) -> bool:
+        """Whether ticks draw from the table of uniforms: a draw is then one ``tah_sample_rows`` launch."""
+        return (self.uniforms is not None and temperature > 0.0 and self.fused_sampling and int(filters.get("top_k", 0)) == 0
+                and self.cfg.vocab <= self.SAMPLE_ROWS_MAX_VOCAB)
 
     # ── rows at different latent iterations in one batch ─────────────────
     def _tick(self, parity: int, eos: int, limit: int, temperature: float = 0.0, **filters):
@@ -858,10 +874,17 @@ class TaHDecodeEngine(DecodeEngine):
         if temperature > 0.0:
             # one draw per row from the final logits as the step-wise loop forms them (first iteration, plus the second
             # where there was one, summed in bf16); rows that only move on to their second iteration ignore theirs
-            chosen = self._draw(logits, temperature, prev=self.logits2[1 - parity], add_prev=self.phase, **filters).contiguous()
+            prev = dict(logits_prev=self.logits2[1 - parity], add_prev=self.phase)
+            if self._draws_by_step(temperature, filters):  # (out_len counts the tokens a row has: the next one's row of the table)
+                chosen = ops.sample_rows(logits, self.uniforms, temperature, top_p=float(filters.get("top_p", 1.0)),
+                                         min_p=float(filters.get("min_p", 0.0)), uniform_step=self.out_len, **prev)
+            else:
+                chosen = self._draw(logits, temperature, prev=prev["logits_prev"], add_prev=self.phase, **filters).contiguous()
         ops.greedy_tick(logits, self.logits2[1 - parity], eos, limit, hard_now=self.hard, phase=self.phase, tok=self.tok,
                         finished=self.finished, pos=self.pos, out_tokens=self.out_tokens, out_len=self.out_len,
                         hard_len=self.hard_len, n_hard=self.n_hard, n_steps=self.n_steps, chosen=chosen)
+
+    DRAW_AHEAD = 64  # ticks whose uniforms are drawn at a time; with an end-of-sequence token also how often the host looks
 
     def _launch_switches(self):
         return super()._launch_switches() + (self.use_fused_glue, self.static_scratch, self.measure_without_attention, id(self.decider))
@@ -872,6 +895,8 @@ class TaHDecodeEngine(DecodeEngine):
         if self._tick_graphs is not None and self._tick_key == key:
             return self._tick_graphs
         undo = self._hold_state()
+        if self._draws_by_step(temperature, filters):
+            torch.rand(self.B, device=self.device)  # what the warm-up step of ``capture`` draws
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(s):
@@ -912,8 +937,12 @@ class TaHDecodeEngine(DecodeEngine):
         self.finished |= reached
         n_min = max_new_tokens - 1
         graphs = self.capture_ticks(eos, limit, temperature, **filters) if (use_graph and n_min > 0) else None
-        ticks = 0
+        ticks, steps = 0, n_min  # steps: how many the step-wise loop would run
+        by_step = self._draws_by_step(temperature, filters)
         while n_min > 0:
+            if by_step and ticks % self.DRAW_AHEAD == 0:  # no row is at a later token than the tick's number
+                for i in range(ticks + 1, min(ticks + self.DRAW_AHEAD, n_min) + 1):
+                    self.uniforms[i].uniform_()
             if graphs is not None:
                 graphs[ticks % 2].replay()
             else:
@@ -921,12 +950,16 @@ class TaHDecodeEngine(DecodeEngine):
             ticks += 1
             if ticks >= n_min and (ticks - n_min) % check_every == 0 and bool(self.finished.all()):
                 break
+            if eos >= 0 and ticks % self.DRAW_AHEAD == 0 and bool(self.finished.all()):
+                steps = min(steps, max(1, -(-int(self.out_len.max()) // self.DRAW_AHEAD)) * self.DRAW_AHEAD)
+                break
             if ticks > 2 * n_min + check_every:
                 raise TahDuoError("generation did not finish within two passes per token")
         self.ticks = ticks
         self.finished &= self.out_len < limit  # rows stopped by the limit have not ended
-        self.host_positions += n_min
-        self.host_hard_rows += n_min
+        if eos >= 0 and self.step_workspace is not None:
+            self.tok.masked_fill_(self.finished & (self.out_len < steps), 0)  # (as rows that sat out steps have it there)
+        self._advanced(min(ticks, steps))  # (a row appends at most one token of each depth per tick)
         return self.out_tokens[:, :max_new_tokens]
 
 

@@ -18,7 +18,22 @@ def _slabs(B, cap, hkv, lens, with_pos, g, dev):
     return s
 
 
-def run(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2=64, full_slab=False):
+def _workspace(wanted, c1, c2, B, hq, hkv):
+    """What the call is handed as ``workspace=``: nothing, or for batches and slabs that the call takes only with one, that."""
+    from tah_amd import kv_cache
+    if not wanted:
+        return None
+    assert not kv_cache.decode_step_supported(B, hq, hkv, c1.capacity)
+    ws = kv_cache.decode_step_workspace(B, hq, hkv, c1.capacity, c2.capacity, c1.k.device)
+    assert ws is not None
+    return ws
+
+
+def _counters_are_back_at_zero(ws, B, hkv):
+    return ws is None or int(ws[:4 * B * hkv].view(torch.int32).abs().max()) == 0
+
+
+def run(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2=64, full_slab=False, workspace=False):
     """full_slab: the depth-0 slabs hold exactly the longest sequence, so that sequence's new row does not fit: both
     paths have to raise the overflow flag, leave slab and length alone and attend over what is cached."""
     from tah_amd import kv_cache
@@ -48,6 +63,7 @@ def run(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2=64, f
     active, hard = active.to(dev), hard.to(dev)
     minus1 = torch.full((B,), -1, dtype=torch.int32, device=dev)
     scale = 128 ** -0.5
+    ws = _workspace(workspace, c1, c2, B, hq, hkv)
     results = {}
     for depth in (0, 1):
         sel = active if depth == 0 else hard
@@ -62,7 +78,8 @@ def run(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2=64, f
             common = dict(cache=tgt, cu_new=cu, slot_of=slot_of, pos_new=pos if depth == 1 else None, norm_input=x, norm_eps=1e-6)
             if fused:
                 o = kv_cache.decode_step(q, k, v, qw, kw, cos, sin, 1e-6, append_at=tgt.len.clone(), q_slot=rows, q_pos=q_pos,
-                                         c1=a1, c2=a2, scale=scale, q_depth=q_depth, out_packed=packed, **common)
+                                         c1=a1, c2=a2, scale=scale, q_depth=q_depth, out_packed=packed, workspace=ws, **common)
+                assert _counters_are_back_at_zero(ws, B, hkv)
             else:
                 qo, _ = kv_cache.qk_norm_rope(q, k, qw, kw, cos, sin, 1e-6, v=v, one_row_per_seq=True, **common)
                 o = kv_cache.decode(qo, rows, q_pos, a1, a2, scale=scale, q_depth=q_depth, out_packed=packed)
@@ -91,12 +108,12 @@ def run(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2=64, f
         at[victim] -= 1
         kv_cache.decode_step(q, k, v, qw, kw, cos, sin, 1e-6, append_at=at, q_slot=rows, q_pos=torch.where(active, pos, minus1),
                              c1=a1, c2=a2, scale=scale, q_depth=torch.zeros(B, dtype=torch.int32, device=dev), cache=a1, cu_new=cu,
-                             slot_of=torch.where(active, rows, minus1), pos_new=None, norm_input=x, norm_eps=1e-6)
+                             slot_of=torch.where(active, rows, minus1), pos_new=None, norm_input=x, norm_eps=1e-6, workspace=ws)
         assert int(a1.overflow) == 2 and int(a1.len[victim]) == lens1[victim]
     return results
 
 
-def run_mixed(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2=64):
+def run_mixed(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2=64, workspace=False):
     """Rows at different latent iterations in one call (append_depth): rows at depth 0 append to the depth-0 slabs and
     see them, rows at depth 1 append to the depth-1 slabs (with their position) and see both.  Against two tah_qk_prep
     calls, one per depth with the other depth's rows masked out, followed by one tah_duo_decode."""
@@ -138,7 +155,8 @@ def run_mixed(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2
     b1, b2 = copy.deepcopy(c1), copy.deepcopy(c2)
     append_at = torch.where(depth, b2.len, b1.len)
     ob = kv_cache.decode_step(q, k, v, qw, kw, cos, sin, 1e-6, cache=b2, append_at=append_at, append_depth=q_depth, q_slot=rows,
-                              q_pos=q_pos, c1=b1, c2=b2, scale=scale, slot_of=slot_all, pos_new=pos, q_depth=q_depth, **common)
+                              q_pos=q_pos, c1=b1, c2=b2, scale=scale, slot_of=slot_all, pos_new=pos, q_depth=q_depth,
+                              workspace=_workspace(workspace, b1, b2, B, hq, hkv), **common)
     assert torch.allclose(oa.float(), ob.float(), rtol=2.0 ** -7, atol=2.0 ** -12) and (oa != ob).float().mean() < 1e-3
     for sa, sb in ((a1, b1), (a2, b2)):
         assert torch.equal(sa.k, sb.k) and torch.equal(sa.v, sb.v) and torch.equal(sa.len, sb.len) and int(sa.overflow) == int(sb.overflow) == 0

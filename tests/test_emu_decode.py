@@ -96,3 +96,17 @@ def test_fused_decode_step_equals_prep_then_decode_on_cpu_shim():
         decode_step_case.run("cpu", B=3, hq=16, hkv=8, seed=5)
         decode_step_case.run("cpu", B=2, hq=8, hkv=8, seed=6, full_slab=True)
         decode_step_case.run_mixed("cpu", B=4, hq=8, hkv=8, seed=7)
+
+
+def test_fused_decode_step_with_a_pairs_rows_shared_by_workgroups_on_cpu_shim():
+    """Fewer pairs than the one-workgroup kernel wants, slabs of 1500 rows: up to four workgroups per pair, the last one merges.
+    Without a workspace such calls are refused; too small a one is refused too."""
+    from tests import decode_step_case
+    from tah_amd import TahDuoError, kv_cache
+    with emu_util.emulated():
+        decode_step_case.run("cpu", B=3, hq=2, hkv=1, seed=8, max_len=1400, cap1=1500, cap2=700, workspace=True)
+        decode_step_case.run("cpu", B=2, hq=1, hkv=1, seed=9, max_len=600, cap2=300, full_slab=True, workspace=True)
+        decode_step_case.run_mixed("cpu", B=4, hq=2, hkv=1, seed=10, max_len=1400, cap1=1500, cap2=700, workspace=True)
+        with pytest.raises(TahDuoError):
+            decode_step_case.run("cpu", B=3, hq=2, hkv=1, seed=8)
+        assert kv_cache.decode_step_workspace(3, 4, 1, 1500, 700, "cpu") is None  # four query heads per kv head

@@ -420,6 +420,50 @@ def test_continuous_generation_with_sampling_gpu():
     assert min(len(set(toks[:, j].tolist())) for j in range(1, new)) > B // 4
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,max_len", [(1, 60), (5, 1200), (17, 60), (32, 4200)])
+def test_batches_that_need_a_workspace_generate_in_ticks_gpu(B, max_len):
+    """Small batches and long slabs: ticks by default, with the tokens, counters, cache lengths and random state that the
+    step-wise loop leaves, greedy and sampled, also over more tokens than uniforms are drawn ahead."""
+    from tah_amd.engine import EngineConfig, TaHDecodeEngine, Weights
+    cfg = EngineConfig(hidden=256, layers=2, hq=16, hkv=8, head_dim=128, intermediate=768, vocab=4096, decider_hidden=32)
+    w = Weights.random_init(cfg, "cuda", seed=6)
+    T = 21
+    new = 90 if max_len > 1000 else 24
+    ids = torch.randint(0, cfg.vocab, (B * T,), generator=torch.Generator().manual_seed(B)).cuda()
+    cu = torch.arange(0, B * T + 1, T, dtype=torch.int32, device="cuda")
+    for filters in ({}, dict(temperature=0.8, top_p=0.9), dict(temperature=0.8, top_k=20)):
+        runs = []
+        for continuous, use_graph in ((False, True), (None, True), (None, False)):
+            eng = TaHDecodeEngine(w, B, max_len, device="cuda")
+            assert eng.step_workspace is not None and eng.can_run_continuous
+            first, _ = eng.prefill(ids, cu, calibrate=0.25)
+            torch.manual_seed(3)
+            toks = eng.generate(first, new, continuous=continuous, use_graph=use_graph, **filters).clone()
+            runs.append((toks.cpu(), eng.out_len.cpu(), eng.pos.cpu(), int(eng.n_hard), [sl.len.tolist() for sl in eng.slabs0 + eng.slabs1],
+                         torch.cuda.get_rng_state() if use_graph else None))
+            assert hasattr(eng, "ticks") == (continuous is None and "top_k" not in filters)
+        for r in runs[1:] if not filters else runs[1:2]:
+            assert torch.equal(r[0], runs[0][0]) and torch.equal(r[1], runs[0][1]) and torch.equal(r[2], runs[0][2])
+            assert r[3:5] == runs[0][3:5] and (r[5] is None or torch.equal(r[5], runs[0][5]))
+
+
+@pytest.mark.gpu
+def test_ticks_end_soon_after_every_row_has_ended_gpu():
+    """With an end-of-sequence token the host looks every 64 ticks, as the step-wise loop does every 64 steps."""
+    from tah_amd.engine import EngineConfig, TaHDecodeEngine, Weights
+    cfg = EngineConfig(hidden=256, layers=2, hq=16, hkv=8, head_dim=128, intermediate=768, vocab=4096, decider_hidden=32)
+    w = Weights.random_init(cfg, "cuda", seed=6)
+    ids, cu = torch.arange(21).cuda(), torch.tensor([0, 21], dtype=torch.int32, device="cuda")
+    eng = TaHDecodeEngine(w, 1, 400, device="cuda")
+    first, _ = eng.prefill(ids, cu, calibrate=0.25)
+    eos = int(eng.generate(first, 8)[0, 5])
+    first, _ = eng.prefill(ids, cu)
+    toks = eng.generate(first, 300, eos=eos)
+    n = int(eng.out_len)
+    assert eng.ticks == 64 and n <= 5 and bool(eng.finished.all()) and int(toks[0, n:].abs().max()) == 0
+
+
 def _topk_sampling_case(device, V, rows=6, draws=True):
     """The distribution over the k largest logits that sample_topk draws from against the one the reference's filters
     leave on the whole row (utils.py:84-125), on rows without equal values; and the draws land where it is not zero."""

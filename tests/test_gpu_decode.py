@@ -132,3 +132,13 @@ def test_fused_decode_step_equals_prep_then_decode(B, hq, hkv):
     decode_step_case.run("cuda", B=B, hq=hq, hkv=hkv, seed=B + hq, max_len=3000, hidden=2048, cap1=4096, cap2=1024)
     decode_step_case.run("cuda", B=B, hq=hq, hkv=hkv, seed=B + hq + 1, max_len=500, hidden=512, cap2=512, full_slab=True)
     decode_step_case.run_mixed("cuda", B=B, hq=hq, hkv=hkv, seed=B + hq + 2, max_len=3000, hidden=2048, cap1=4096, cap2=1024)
+
+
+@pytest.mark.parametrize("B,hq,hkv,cap1", [(2, 16, 8, 700), (2, 16, 8, 20000), (5, 8, 8, 2100), (31, 16, 8, 1024), (3, 2, 1, 513),
+                                           (32, 16, 8, 8192)])
+def test_fused_decode_step_with_a_workspace_equals_prep_then_decode(B, hq, hkv, cap1):
+    """Batches with fewer pairs than compute units and slabs beyond 4096 rows: several workgroups share a pair's rows."""
+    from tests import decode_step_case
+    print(f"fused decode step with a workspace B={B} hq={hq} hkv={hkv} cap={cap1}", flush=True)
+    for case in (decode_step_case.run, decode_step_case.run_mixed):
+        case("cuda", B=B, hq=hq, hkv=hkv, seed=B + cap1, max_len=cap1 - 1, hidden=2048, cap1=cap1, cap2=max(64, cap1 // 4), workspace=True)
