@@ -26,7 +26,8 @@
 // reduction per kernel, and the rows' operand: every workgroup reads all 32 x K of it from L2, which the
 // per-CU L1 fill rate (about 100 GB/s) makes 1 us per 128 KB.  Splitting K over workgroups would cut that, but
 // the hand-over between workgroups (device-scope fence + counter, last one reduces) cost 7 us per split when
-// tried: the fence writes back and invalidates the whole L2 of the XCD.
+// tried: the fence writes back and invalidates the whole L2 of the XCD.  One to eight rows: 5.4 / 4.7 / 11.1 / 8.1 us
+// (kFold, H8 below).
 #include <hip/hip_runtime.h>
 
 #include "mixer_device.h"
@@ -79,7 +80,12 @@ __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + fast_exp2(
 // are at most 16 rows).  A layer with few column groups (n = 2048: 128) then fills the chip, and every compute
 // unit pulls half of the rows' operand; the second reader of a weight tile is placed on the same XCD, whose L2 has
 // it or is fetching it.
-template <int NC, int CH, int EPI, int PW, int NH>
+// H8 (one tile, sixteen rows, K known): a workgroup takes eight of the tile's sixteen columns, so a layer whose tiles would
+// occupy half of the compute units occupies all.  A load then covers two k steps of the eight columns (lanes c < 8 the
+// even one, the others the odd one: 128 contiguous bytes each), and each loaded operand is multiplied twice, by either
+// step's rows; of the first product the columns below 8 count, of the second those from 8 on.  At one to eight rows o
+// (8 MB) takes 5.0 -> 4.7 us, down (25 MB) 9.5 -> 8.1: 3.5 us of launch, latency and reduction and the weight at 5.6 TB/s.
+template <int NC, int CH, int EPI, int PW, int NH, bool H8 = false, bool kFold = false>
 __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParams p) {
     __shared__ __align__(16) float red[kLinWaves][NC][16 * NH][kTileCols];
     __shared__ float ssq[kLinWaves][16 * NH];
@@ -107,12 +113,13 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
     // The epilogue's own operands (residual, bias: 16 bytes each for a thread that writes results) are asked for here:
     // requested behind the reduction they would cost the kernel one trip to memory each, one after the other.
     constexpr bool kGateEpi = EPI == kGateUp16 || EPI == kGateUp24;
-    constexpr int kEpiUnits = EPI == kGateUp24 ? 3 : (kGateEpi ? 2 : 2 * NC);
+    constexpr int kEpiUnits = H8 ? 1 : EPI == kGateUp24 ? 3 : (kGateEpi ? 2 : 2 * NC);
+    constexpr int kCols = H8 ? 8 : NC * kTileCols;  // a plain layer's columns per workgroup
     bf16x8 res_early = {0, 0, 0, 0, 0, 0, 0, 0}, bias_early = {0, 0, 0, 0, 0, 0, 0, 0};
     if constexpr (!kGateEpi) {
         const bool writer = (int)threadIdx.x < 16 * NH * kEpiUnits;
         const int erow = 16 * half + (writer ? (int)threadIdx.x / kEpiUnits : 0);
-        const int en0 = group * NC * kTileCols + 8 * (writer ? (int)threadIdx.x % kEpiUnits : 0);
+        const int en0 = group * kCols + 8 * (writer ? (int)threadIdx.x % kEpiUnits : 0);
         const bool live_row = erow < p.rows;
         // (addresses picked by selects, so that no load sits under a branch)
         const __bf16* ra = (p.res && live_row) ? p.res + (int64_t)erow * p.res_rs + en0 : reinterpret_cast<const __bf16*>(px);
@@ -127,17 +134,21 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
     const int s0 = nst > 0 ? wave * per_wave : 0;  // a wave without steps still points at valid memory
     const bf16x8* wb[NC];
 #pragma unroll
-    for (int t = 0; t < NC; ++t) wb[t] = pw + ((int64_t)(group * NC + t) * steps + s0) * 64 + lane;
-    const bf16x8* xb = px + (int64_t)s0 * 128 + 64 * half + lane;
+    for (int t = 0; t < NC; ++t)
+        wb[t] = H8 ? pw + ((int64_t)(group / 2) * steps + s0 + c / 8) * 64 + 16 * kg + 8 * (group % 2) + c % 8
+                   : pw + ((int64_t)(group * NC + t) * steps + s0) * 64 + lane;
+    // kFold: the lanes of rows past the last one read row 0's operand again instead of their zeros (their results are not used):
+    // with up to eight rows a load then touches a half to a quarter of the bytes (q|k|v at one to eight rows 5.75 -> 5.4 us).
+    const bf16x8* xb = px + (int64_t)s0 * 128 + 64 * half + (kFold ? 16 * kg + (c < p.rows ? c : 0) : lane);
 
     struct Buf {
-        bf16x8 w[CH][NC], x[CH][NH];
+        bf16x8 w[H8 ? CH / 2 : CH][NC], x[CH][NH];
     };
-    f32x4 acc[NC][NH];
+    f32x4 acc[NC][H8 ? 2 : NH];  // (H8: of the even and of the odd steps)
 #pragma unroll
     for (int t = 0; t < NC; ++t)
 #pragma unroll
-        for (int h = 0; h < NH; ++h) acc[t][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int h = 0; h < (H8 ? 2 : NH); ++h) acc[t][h] = f32x4{0.f, 0.f, 0.f, 0.f};
     float ss0 = 0.f, ss1 = 0.f, sm0 = 0.f, sm1 = 0.f;
     const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
     // Loads of chunk ch.  Without a compile-time K a step past the wave's share reads step 0 of the wave's range
@@ -154,11 +165,11 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 0; s < CH; ++s) {
+        for (int s = 0; s < CH; s += H8 ? 2 : 1) {
             const int st = ch * CH + s;
             const int64_t sti = (PW > 0 || st < nst) ? st : 0;
 #pragma unroll
-            for (int t = 0; t < NC; ++t) b.w[s][t] = __builtin_nontemporal_load(wb[t] + sti * 64);
+            for (int t = 0; t < NC; ++t) b.w[H8 ? s / 2 : s][t] = __builtin_nontemporal_load(wb[t] + sti * 64);
         }
     };
     auto multiply = [&](int ch, Buf& b) __attribute__((always_inline)) {
@@ -180,8 +191,12 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
             }
 #pragma unroll
             for (int t = 0; t < NC; ++t) {
-                acc[t][0] = mfma16(a0, b.w[s][t], acc[t][0]);
-                if constexpr (NH == 2) acc[t][1] = mfma16(a1, b.w[s][t], acc[t][1]);
+                if constexpr (H8) {
+                    acc[t][s % 2] = mfma16(a0, b.w[s / 2][t], acc[t][s % 2]);
+                } else {
+                    acc[t][0] = mfma16(a0, b.w[s][t], acc[t][0]);
+                    if constexpr (NH == 2) acc[t][1] = mfma16(a1, b.w[s][t], acc[t][1]);
+                }
             }
         }
     };
@@ -221,7 +236,7 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
 #pragma unroll
         for (int h = 0; h < NH; ++h)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) red[wave][t][16 * h + 4 * kg + r][c] = acc[t][h][r];
+            for (int r = 0; r < 4; ++r) red[wave][t][16 * h + 4 * kg + r][c] = (H8 && c >= 8) ? acc[t][NH][r] : acc[t][h][r];
     if constexpr (EPI != kPlain) {
         // a lane's squares cover its 8 of every 32 k of rows c and 16 + c: add the four k groups
         ss0 += __shfl_xor(ss0, 16);
@@ -247,7 +262,7 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
 
     // ---- epilogue: one thread per (row, 8 output columns) -------------------------------------------------
     constexpr bool kGate = EPI == kGateUp16 || EPI == kGateUp24;
-    constexpr int kUnits = EPI == kGateUp24 ? 3 : (kGate ? 2 : 2 * NC);  // 8-column units of output per row and workgroup
+    constexpr int kUnits = H8 ? 1 : EPI == kGateUp24 ? 3 : (kGate ? 2 : 2 * NC);  // 8-column units of output per row and workgroup
     if (threadIdx.x >= 16 * NH * kUnits) return;
     const int lrow = threadIdx.x / kUnits, unit = threadIdx.x % kUnits;  // row inside the workgroup's rows
     const int row = 16 * half + lrow;
@@ -271,6 +286,15 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
             sg[i] += lo[i];
             sg[4 + i] += hi[i];
         }
+        if constexpr (H8) {  // the odd steps' sums
+            const f32x4 olo = *reinterpret_cast<const f32x4*>(&red[w][0][lrow][8]);
+            const f32x4 ohi = *reinterpret_cast<const f32x4*>(&red[w][0][lrow][12]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                sg[i] += olo[i];
+                sg[4 + i] += ohi[i];
+            }
+        }
         if constexpr (kGate) {
             const f32x4 ulo = *reinterpret_cast<const f32x4*>(&red[w][ut][lrow][uc]);
             const f32x4 uhi = *reinterpret_cast<const f32x4*>(&red[w][ut][lrow][uc + 4]);
@@ -281,7 +305,7 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
             }
         }
     }
-    const int n0 = group * (EPI == kGateUp24 ? kGroup24 : (kGate ? kTileCols : NC * kTileCols)) + 8 * unit;
+    const int n0 = group * (EPI == kGateUp24 ? kGroup24 : (kGate ? kTileCols : kCols)) + 8 * unit;
     const bool live = row < p.rows;
     bf16x8 out = zero8;
     if (live) {
@@ -357,6 +381,127 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
     }
 }
 
+// An output head (n >= kWideFromCols plain columns, K = 256 PW) for more than sixteen rows: a resident workgroup per
+// compute unit walks a range of column groups.  Its waves keep their slices of the rows' operand in registers -- read per
+// group it is as many bytes as the weights and shares the L1's fill rate with them -- and ask for the next group's weights
+// before they multiply and reduce this one's.  151936 x 2048, 32 rows: 114.5 -> 104.8 us (5.4 -> 5.9 TB/s), 24 rows
+// 111.7 -> 101.5; groups dealt out round robin instead of ranges 107.6 (two workgroups then write the halves of a line).
+// With sixteen rows the operand is half of that and many workgroups, two or three to a compute unit, stream better (93
+// against 98 us): they keep linear_rows_kernel.
+template <int EPI, int PW>
+__global__ __launch_bounds__(kLinThreads) void linear_wide_kernel(const LinParams p) {
+    static_assert(EPI == kPlain || EPI == kPlainNorm, "plain layers");
+    constexpr int NC = 2, NH = 2;
+    __shared__ __align__(16) float red[kLinWaves][NC][16 * NH][kTileCols];
+    __shared__ float ssq[kLinWaves][16 * NH];
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int c = lane % 16, kg = lane / 16;
+    constexpr int steps = kLinWaves * PW;
+    bf16x8 x[PW][NH];
+    {
+        const bf16x8* xb = p.x + (int64_t)wave * PW * 128 + lane;
+#pragma unroll
+        for (int s = 0; s < PW; ++s)
+#pragma unroll
+            for (int h = 0; h < NH; ++h) x[s][h] = xb[s * 128 + 64 * h];
+    }
+    struct Buf {
+        bf16x8 w[PW][NC];
+    };
+    auto issue = [&](int g, Buf& b) __attribute__((always_inline)) {
+        const bf16x8* wb = p.w + ((int64_t)g * NC * steps + wave * PW) * 64 + lane;
+#pragma unroll
+        for (int s = 0; s < PW; ++s)
+#pragma unroll
+            for (int t = 0; t < NC; ++t) b.w[s][t] = __builtin_nontemporal_load(wb + (int64_t)(t * steps + s) * 64);
+    };
+    // one thread per (row, 8 output columns)
+    constexpr int kUnits = 2 * NC;
+    const bool writer = (int)threadIdx.x < 16 * NH * kUnits;
+    const int row = threadIdx.x / kUnits, unit = threadIdx.x % kUnits;
+    float rin = 1.0f;
+    auto finish = [&](int g, Buf& b) __attribute__((always_inline)) {
+        f32x4 acc[NC][NH];
+#pragma unroll
+        for (int t = 0; t < NC; ++t)
+#pragma unroll
+            for (int h = 0; h < NH; ++h) acc[t][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < PW; ++s)
+#pragma unroll
+            for (int t = 0; t < NC; ++t)
+#pragma unroll
+                for (int h = 0; h < NH; ++h) acc[t][h] = mfma16(x[s][h], b.w[s][t], acc[t][h]);
+        __syncthreads();  // the group before has been read
+#pragma unroll
+        for (int t = 0; t < NC; ++t)
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) red[wave][t][16 * h + 4 * kg + r][c] = acc[t][h][r];
+        __syncthreads();
+        if (!writer || row >= p.rows) return;
+        float sum[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum[i] = 0.f;
+#pragma unroll
+        for (int w = 0; w < kLinWaves; ++w) {
+            const f32x4 lo = *reinterpret_cast<const f32x4*>(&red[w][unit / 2][row][8 * (unit % 2)]);
+            const f32x4 hi = *reinterpret_cast<const f32x4*>(&red[w][unit / 2][row][8 * (unit % 2) + 4]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                sum[i] += lo[i];
+                sum[4 + i] += hi[i];
+            }
+        }
+        bf16x8 out;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) out[i] = (__bf16)(sum[i] * rin);
+        *reinterpret_cast<bf16x8*>(p.y + (int64_t)row * p.y_rs + (int64_t)g * NC * kTileCols + 8 * unit) = out;
+    };
+    // (no workgroup is without a group)
+    int g = (int)((int64_t)blockIdx.x * p.groups / gridDim.x);
+    const int end = (int)((int64_t)(blockIdx.x + 1) * p.groups / gridDim.x);
+    Buf buf[2];
+    issue(g, buf[0]);
+    if constexpr (EPI == kPlainNorm) {
+        float ss[NH];
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            ss[h] = 0.f;
+#pragma unroll
+            for (int s = 0; s < PW; ++s)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) ss[h] += (float)x[s][h][i] * (float)x[s][h][i];
+            ss[h] += __shfl_xor(ss[h], 16);
+            ss[h] += __shfl_xor(ss[h], 32);
+            if (kg == 0) ssq[wave][16 * h + c] = ss[h];
+        }
+        __syncthreads();
+        if (writer) {
+            float t = 0.f;
+#pragma unroll
+            for (int w = 0; w < kLinWaves; ++w) t += ssq[w][row];
+            rin = __builtin_amdgcn_rsqf(t / (float)p.k + p.eps);
+        }
+    }
+    while (true) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int next = g + 1;
+            if (next < end) {
+                issue(next, buf[(i + 1) % 2]);
+                __builtin_amdgcn_sched_barrier(0);
+                finish(g, buf[i]);
+                ++g;
+            } else {
+                finish(g, buf[i]);
+                return;
+            }
+        }
+    }
+}
+
 // ---- re-ordering -----------------------------------------------------------------------------------------
 // Weight row behind column slot c of tile t of the packed order.
 __device__ __host__ inline int64_t packed_weight_row(int kind, int n, int tile, int c) {
@@ -399,10 +544,28 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 constexpr int kSplitRowsBelowGroups = 129;
 constexpr int kWideFromCols = 16384;  // plain layers from this many output columns on take 32 columns per workgroup
 
+template <int EPI, int PW>
+void launch_wide(LinParams& p, int groups, hipStream_t st) {
+    constexpr int kResident = 256;  // a workgroup per compute unit
+    p.groups = groups;
+    hipLaunchKernelGGL((linear_wide_kernel<EPI, PW>), dim3(groups < kResident ? groups : kResident), dim3(kLinThreads), 0, st, p);
+}
+
 template <int NC, int CH, int EPI, int PW>
 void launch(LinParams& p, int groups, int batch, hipStream_t st) {
     p.groups = groups;
-    if (p.rows <= 16)
+    if constexpr (NC == 1 && EPI == kPlain && PW > 0 && PW % 2 == 0) {
+        // (from nine rows on the doubled reads of the rows' operand outweigh it for short sums: K = 2048, sixteen rows 5.1 ->
+        // 5.5 us, where K = 4096 gains 7.6 -> 7.0 and K = 6144 9.5 -> 8.8)
+        if (groups * batch < kSplitRowsBelowGroups && (p.rows <= 8 || (p.rows <= 16 && PW >= 16))) {
+            p.groups = 2 * groups;
+            hipLaunchKernelGGL((linear_rows_kernel<1, PW, kPlain, PW, 1, true, true>), dim3(p.groups, batch), dim3(kLinThreads), 0, st, p);
+            return;
+        }
+    }
+    if (NC != 2 && PW > 0 && p.rows <= 8)  // (two tiles share the operand: nothing to gain)
+        hipLaunchKernelGGL((linear_rows_kernel<NC, CH, EPI, PW, 1, false, NC != 2 && (PW > 0)>), dim3(groups, batch), dim3(kLinThreads), 0, st, p);
+    else if (p.rows <= 16)
         hipLaunchKernelGGL((linear_rows_kernel<NC, CH, EPI, PW, 1>), dim3(groups, batch), dim3(kLinThreads), 0, st, p);
     else if (groups * batch < kSplitRowsBelowGroups)
         hipLaunchKernelGGL((linear_rows_kernel<NC, CH, EPI, PW, 1>), dim3(2 * groups, batch), dim3(kLinThreads), 0, st, p);
@@ -498,7 +661,10 @@ extern "C" int tah_linear_rows(const tah_linear_rows_args* a, tah_stream_t strea
     if (!gate_up && a->input_norm != TAH_NORM_LAYER && a->n >= kWideFromCols && a->n % (2 * kTileCols) == 0) {
         // an output head: two tiles per workgroup, the rows' operand is read half as often
         const int groups = a->n / (2 * kTileCols);
-        if (p.norm) {
+        if (pw == 8 && p.rows > 16 && batch == 1 && p.y && !p.yp && !p.res && !p.bias && p.act == TAH_ACT_NONE && !p.select) {
+            if (p.norm) launch_wide<kPlainNorm, 8>(p, groups, st);
+            else launch_wide<kPlain, 8>(p, groups, st);
+        } else if (p.norm) {
             if (pw == 8) launch<2, 2, kPlainNorm, 8>(p, groups, batch, st);
             else launch<2, 2, kPlainNorm, 0>(p, groups, batch, st);
         } else {

@@ -247,6 +247,29 @@ def test_packed_orders_gpu():
     _error_checks("cuda")
 
 
+# Few rows, K known at compile time: eight columns per workgroup (few column groups), rows past the last one read as row 0.
+FEW = [(1, 32, 2048, "residual"), (8, 48, 2048, "plain"), (9, 16, 2048, "residual"), (3, 16, 4096, "residual"), (16, 32, 6144, "residual"),
+       (8, 2064, 2048, "plain"), (5, 24, 2048, "gate_up_norm"), (8, 16, 2048, "plain_norm")]
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+@pytest.mark.parametrize("rows,n,k,kind", [c for c in FEW if c[1] < 100])
+def test_linear_rows_of_few_rows_on_cpu_shim(rows, n, k, kind):
+    with emu_util.emulated():
+        _linear_case("cpu", rows, n, k, kind)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n,k,kind", FEW + [
+    # (without a residual: added to products of up to 4, which the sum's order may move by one bf16 step of 2^-6, it can cancel
+    # them to a value whose own step is finer than that move)
+    (1, 2048, 2048, "plain"), (16, 2048, 6144, "plain"), (4, 6144, 2048, "gate_up_norm"),
+    # more than sixteen rows of an output head: a resident workgroup per compute unit, one, two or three column groups each
+    (17, 16384, 2048, "plain"), (32, 16416, 2048, "plain_norm"), (24, 32000, 2048, "plain"), (31, 151936, 2048, "plain_norm")])
+def test_linear_rows_of_few_rows_and_output_heads_gpu(rows, n, k, kind):
+    _linear_case("cuda", rows, n, k, kind, seed=n % 5)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,n,k,kind", CASES + [
     (32, 4096, 2048, "plain"), (32, 2048, 2048, "residual"), (32, 6144, 2048, "gate_up_norm"), (32, 2048, 6144, "residual"),
