@@ -125,3 +125,15 @@ def test_rows_copy_bit_exact(dtype, inner):
     want = torch.full_like(src, 7)
     want[rows.long()] = src[rows.long()]
     assert torch.equal(back, want)
+
+
+@pytest.mark.parametrize("hq,hkv,seqlens,p,drift", [(2, 1, [330], 0.3, 0.0), (4, 1, [193, 80], 1.0, 0.25)])
+def test_fwd_kernel_two_teams_per_tile_on_cpu_shim(hq, hkv, seqlens, p, drift):
+    """Small launches with at least four key tiles: two teams share a query tile's keys (also where the second team's exponent
+    reference is far from the first's)."""
+    from tah_amd import ops
+    case = make_varlen_case(33, seqlens, p, Hq=hq, Hkv=hkv, D=128)
+    dev = _to_dev(add_score_drift(case, drift) if drift else case)
+    with emu_util.emulated():
+        got = ops.duo_fwd_varlen(*varlen_args(dev))
+    _check(dev, got)

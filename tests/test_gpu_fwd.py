@@ -208,3 +208,15 @@ def test_tolerance_against_reference_bf16_path_and_bf16_rounded_oracle():
     assert mr["hip"] <= 1.05 * mr["ref_bf16"], mr
     assert worst_abs["hip"] <= max(1.05 * worst_abs["ref_bf16"], 1e-2), worst_abs
     assert mr["hip_vs_rounded"] <= 1.05 * mr["ref_vs_rounded"], mr
+
+
+@pytest.mark.parametrize("hq,hkv,seqlens,p,drift", [
+    (16, 8, [191], 0.5, 0.0), (16, 8, [192], 0.4, 0.0), (8, 8, [255], 0.1, 0.0), (16, 4, [257], 0.2, 0.0),   # around four key tiles
+    (16, 8, [449, 3, 64, 320], 0.2, 0.0), (16, 8, [1000], 0.0, 0.0), (2, 1, [640], 1.0, 0.0),
+    (16, 8, [900, 100], 0.1, 0.25), (16, 4, [700], 0.3, 0.02),     # the second team's exponent reference far from the first's
+    (16, 8, [2000, 2000], 0.1, 0.0), (16, 8, [3900], 0.05, 0.0)])  # on either side of one round of workgroups
+def test_fwd_two_teams_per_tile(hq, hkv, seqlens, p, drift):
+    print(f"case two teams hq={hq} hkv={hkv} seqlens={seqlens} p={p} drift={drift}", flush=True)
+    case = make_varlen_case(51, seqlens, p, Hq=hq, Hkv=hkv, D=128)
+    dev = to_device(add_score_drift(case, drift) if drift else case)
+    _check(dev, _run(dev), "two teams")
