@@ -1,5 +1,7 @@
 // Device-side helpers of the layer mechanisms in row_norm.hip, delta_rule.hip, latent_attn.hip, window_attn.hip and moe.hip.
 #pragma once
+#include <type_traits>
+
 #include "duo_device.h"
 #include "tah_mixers.h"
 
@@ -21,6 +23,22 @@ __device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
         v[4 + i] = b[i];
     }
 }
+// Eight elements as they lie in memory: loads that are on their way.
+template <class E> struct Eight;
+template <> struct Eight<__bf16> {
+    bf16x8 v;
+    __device__ __forceinline__ void load(const __bf16* p) { v = *reinterpret_cast<const bf16x8*>(p); }
+    __device__ __forceinline__ float operator[](int i) const { return (float)v[i]; }
+};
+template <> struct Eight<float> {
+    f32x4 a, b;
+    __device__ __forceinline__ void load(const float* p) {
+        a = *reinterpret_cast<const f32x4*>(p);
+        b = *reinterpret_cast<const f32x4*>(p + 4);
+    }
+    __device__ __forceinline__ float operator[](int i) const { return i < 4 ? a[i] : b[i - 4]; }
+};
+
 __device__ __forceinline__ bf16x8 to_bf16x8(const float (&v)[8]) {
     bf16x8 x;
 #pragma unroll
@@ -39,6 +57,31 @@ __device__ __host__ __forceinline__ int64_t rows_form_unit(int r, int c) {
 }
 // element of it
 __device__ __host__ __forceinline__ int64_t rows_form_elem(int r, int c) { return rows_form_unit(r, c) * 8 + c % 8; }
+
+// x of one lane, the same one for the whole wave
+__device__ __forceinline__ float lane_value(float x, int lane) {
+#ifdef TAH_CPU_EMU
+    return __shfl(x, lane);
+#else
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
+#endif
+}
+
+// Largest float / smallest int of a wave, in every lane, without a trip through LDS.
+template <class T, class F>
+__device__ __forceinline__ T wave_quick(T x, F pick) {
+    const auto from = [](T v, auto ctrl) {
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, true));
+    };
+    x = pick(x, from(x, std::integral_constant<int, 0xB1>{}));   // quad_perm [1,0,3,2]
+    x = pick(x, from(x, std::integral_constant<int, 0x4E>{}));   // quad_perm [2,3,0,1]
+    x = pick(x, from(x, std::integral_constant<int, 0x141>{}));  // row_half_mirror
+    x = pick(x, from(x, std::integral_constant<int, 0x140>{}));  // row_mirror
+    const auto at = [&](int lane) { return __builtin_bit_cast(T, __float_as_int(lane_value(__builtin_bit_cast(float, x), lane))); };
+    return pick(pick(at(0), at(16)), pick(at(32), at(48)));
+}
+__device__ __forceinline__ float wave_max_quick(float x) { return wave_quick(x, [](float a, float b) { return fmaxf(a, b); }); }
+__device__ __forceinline__ int wave_min_quick(int x) { return wave_quick(x, [](int a, int b) { return a < b ? a : b; }); }
 
 __device__ __forceinline__ float wave_sum(float x) {
 #pragma unroll

@@ -4,7 +4,8 @@
 //
 //  * moe_route_kernel: router logits in float32, their scores, the open groups of experts, the largest ones and their
 //    weights; RB rows per workgroup share the router's weights, and a wave takes EB experts at a time so that they share
-//    the rows' reads.
+//    the rows' reads.  Each of the largest is one maximum over the wave inside the vector pipe (four lane exchanges of
+//    registers and four lanes read out): as twelve exchanges through LDS each, eight of them took a third of the kernel.
 //  * moe_plan_kernel: counting sort of the (row, choice) pairs by expert, each expert's rows padded to whole tiles.
 //  * moe_tile_kernel: bf16 tiles of 128 places x 256 weight rows on the matrix cores, both operands staged through LDS
 //    by asynchronous copies, two stages ahead; gate and up rows of the same columns share a wave, which applies the gate.
@@ -20,6 +21,7 @@ constexpr int kMoeThreads = 256;
 constexpr int kMaxExperts = 1024;
 constexpr int kMaxTop = 64;
 constexpr int kGroupsPerLane = 4;  // groups of experts: at most 256
+constexpr int kUnitsHeld = 4;      // scores per lane that the selection keeps in registers (256 experts)
 constexpr int kTile = TAH_MOE_TILE;
 
 // LDS: rows [RB][cols] float32, logits [RB][experts + 1]
@@ -101,7 +103,14 @@ __global__ __launch_bounds__(kThreads) void moe_route_kernel(const tah_moe_route
                 gs[u] = gr < p.groups ? (size > 1 ? a + b : a) : kNegInf;
             }
             uint32_t open = 0;  // bit u: group lane + 64 u is open
-            for (int j = 0; j < p.keep; ++j) {
+            if (p.groups <= kWave) {  // a lane's group is open when fewer than `keep` are in front of it
+                int before = 0;
+                for (int g = 0; g < p.groups; ++g) {
+                    const float o = lane_value(gs[0], g);
+                    before += o > gs[0] || (o == gs[0] && g < lane);
+                }
+                open = gs[0] > kNegInf && before < p.keep;
+            } else for (int j = 0; j < p.keep; ++j) {
                 float bv = kNegInf;
                 int bi = 0x7fffffff;
 #pragma unroll
@@ -125,24 +134,35 @@ __global__ __launch_bounds__(kThreads) void moe_route_kernel(const tah_moe_route
         // the largest scores one after another, the lower index among equals; a chosen one leaves the race
         float mine = kNegInf, first = 0.f;
         int my_index = 0;
+        float v[kUnitsHeld];  // scores of experts lane, lane + 64, ... while they are in the race
+#pragma unroll
+        for (int u = 0; u < kUnitsHeld; ++u) v[u] = lane + kWave * u < experts ? zr[lane + kWave * u] : kNegInf;
+        const bool held = experts <= kUnitsHeld * kWave;
         for (int j = 0; j < top; ++j) {
             float bv = kNegInf;
             int bi = 0x7fffffff;
-            for (int e = lane; e < experts; e += kWave) {
-                const float v = zr[e];
-                if (v > bv) { bv = v; bi = e; }
-            }
+            if (held) {
 #pragma unroll
-            for (int m = 32; m >= 1; m >>= 1) {
-                const float ov = __shfl_xor(bv, m);
-                const int oi = __shfl_xor(bi, m);
-                if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
+                for (int u = 0; u < kUnitsHeld; ++u)
+                    if (v[u] > bv) { bv = v[u]; bi = lane + kWave * u; }
+            } else {
+                for (int e = lane; e < experts; e += kWave) {
+                    const float o = zr[e];
+                    if (o > bv) { bv = o; bi = e; }
+                }
             }
+            const float largest = wave_max_quick(bv);
+            bi = wave_min_quick(bv == largest ? bi : 0x7fffffff);
             if (bi >= experts) bi = j;  // (only when the logits are not numbers)
-            if (j == 0) first = bv;
-            if (lane == j) { mine = bv; my_index = bi; }
-            if (lane == 0) zr[bi] = kNegInf;
-            TAH_WAVE_LDS_SYNC();
+            if (j == 0) first = largest;
+            if (lane == j) { mine = largest; my_index = bi; }
+            if (held) {
+#pragma unroll
+                for (int u = 0; u < kUnitsHeld; ++u) v[u] = lane + kWave * u == bi ? kNegInf : v[u];
+            } else {
+                if (lane == 0) zr[bi] = kNegInf;
+                TAH_WAVE_LDS_SYNC();
+            }
         }
         const float w = lane < top ? expf(mine - first) : 0.f;
         const float sum = wave_sum(w);

@@ -75,47 +75,97 @@ __device__ __forceinline__ void group_sums(float (&s)[U], int units, int groups,
 
 constexpr int kMaxGroups = 256;
 
-// U: units per thread
-template <class E, int U, bool GROUPS>
+// U: units per thread.  kEarly: a few rows are a chain of trips to memory and little else, so a thread asks for everything
+// at once: row, norms, convolution, the expert rows as soon as their indices are there and the convolution's inputs as soon
+// as the position is.  (Threads whose columns lie behind the row's end read the row's start and use none of it.)
+template <class E, int U, bool GROUPS, bool kEarly>
 __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(const tah_residual_norm_args p) {
     __shared__ float red[kRowThreads / kWave], unit_sums[GROUPS ? U * kRowThreads : 1], group_sum[GROUPS ? kMaxGroups : 1];
+    constexpr int kExpertsAhead = kEarly ? 8 : 1, kTaps = 4;
     const int row = blockIdx.x, tid = threadIdx.x;
     const int units = p.cols / 8, group_units = GROUPS ? p.group_cols / 8 : units;
     const float count = GROUPS ? (float)(p.width / p.groups) : (float)p.width;
     float y[U][8], x[U][8];
-    const bool add = p.y || p.experts;
-    const float ys = p.y_scale ? p.y_scale[row] : 1.0f;
+    const bool add = p.y || p.experts, few_taps = kEarly && p.conv && p.taps <= kTaps;
+    Eight<float> x_in[U], coef[kEarly ? U : 1], next_coef[kEarly ? U : 1], conv_w[kEarly ? U : 1][kTaps];
+    Eight<E> y_in[U], conv_in[kEarly ? U : 1][kTaps];
+    int at[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int c = 8 * (tid + u * kRowThreads);
+        at[u] = c < p.cols ? c : 0;
+        x_in[u].load(p.x + (int64_t)row * p.cols + at[u]);
+        if (p.y) y_in[u].load(static_cast<const E*>(p.y) + (int64_t)row * p.y_row_stride + at[u]);
+    }
+    const float ys = p.y_scale ? p.y_scale[row] : 1.0f;
+    const int slot = p.conv ? p.slot[row] : -1, pos = p.conv ? p.pos[row] : -1;
+    if constexpr (kEarly) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) y[u][i] = x[u][i] = 0.f;
-        if (c < p.cols) {
-            load8(p.x + (int64_t)row * p.cols + c, x[u]);
-            if (p.y) {
-                load8(static_cast<const E*>(p.y) + (int64_t)row * p.y_row_stride + c, y[u]);
+        for (int u = 0; u < U; ++u) {
+            if (add) coef[u].load(p.coef + at[u]);
+            if (p.next_coef) next_coef[u].load(p.next_coef + at[u]);
+            if (few_taps) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) y[u][i] *= ys;
+                for (int d = 0; d < kTaps; ++d) conv_w[u][d].load(p.conv + (int64_t)(d < p.taps ? p.taps - 1 - d : 0) * p.cols + at[u]);
             }
         }
     }
+    const bool live = slot >= 0 && slot < p.nslots && pos >= 0;
+    E* const rings = p.conv ? static_cast<E*>(p.conv_state) + (int64_t)(live ? slot : 0) * p.taps * p.cols : nullptr;
+    if constexpr (kEarly) {
+        if (few_taps) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int d = 1; d < kTaps; ++d)
+                    conv_in[u][d].load(rings + (int64_t)(live && d < p.taps && d <= pos ? (pos - d) % p.taps : 0) * p.cols + at[u]);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[u][i] = 0.f;
+    if (p.y) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) y[u][i] = y_in[u][i] * ys;
+    }
     if (p.experts) {
-        for (int j = 0; j < p.top; ++j) {
-            const float w = p.weight[(int64_t)row * p.top + j];
-            const E* e = static_cast<const E*>(p.experts) + ((int64_t)p.index[(int64_t)row * p.top + j] * p.index_scale + (int64_t)row * p.index_row) * p.experts_row_stride;
+        for (int j0 = 0; j0 < p.top; j0 += kExpertsAhead) {
+            float w[kExpertsAhead];
+            int64_t from[kExpertsAhead];
+            Eight<E> v[kExpertsAhead][U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int c = 8 * (tid + u * kRowThreads);
-                if (c < p.cols) {
-                    float v[8];
-                    load8(e + c, v);
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) y[u][i] += w * v[i];
-                }
+            for (int k = 0; k < kExpertsAhead; ++k) {
+                const int64_t j = (int64_t)row * p.top + (j0 + k < p.top ? j0 + k : j0);
+                w[k] = p.weight[j];
+                from[k] = ((int64_t)p.index[j] * p.index_scale + (int64_t)row * p.index_row) * p.experts_row_stride;
             }
+#pragma unroll
+            for (int k = 0; k < kExpertsAhead; ++k)
+#pragma unroll
+                for (int u = 0; u < U; ++u) v[k][u].load(static_cast<const E*>(p.experts) + from[k] + at[u]);
+#pragma unroll
+            for (int k = 0; k < kExpertsAhead; ++k)
+                if (j0 + k < p.top) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) y[u][i] += w[k] * v[k][u][i];
+                }
         }
     }
     float s[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const bool in = 8 * (tid + u * kRowThreads) < p.cols;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            x[u][i] = in ? x_in[u][i] : 0.f;
+            y[u][i] = in ? y[u][i] : 0.f;
+        }
+    }
     if (add) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -132,10 +182,9 @@ __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(const tah_re
         if (c < p.cols) {
             if (add) {
                 const float r = 1.0f / sqrtf(s[u] / count + p.eps);
-                float k[8];
-                load8(p.coef + c, k);
+                if constexpr (!kEarly) coef[0].load(p.coef + c);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) x[u][i] += y[u][i] * r * k[i];
+                for (int i = 0; i < 8; ++i) x[u][i] += y[u][i] * r * coef[kEarly ? u : 0][i];
                 store8(p.x + (int64_t)row * p.cols + c, x[u]);
             }
 #pragma unroll
@@ -147,31 +196,40 @@ __global__ __launch_bounds__(kRowThreads) void residual_norm_kernel(const tah_re
     }
     if (!p.next_coef) return;
     group_sums<U, GROUPS>(s, units, p.groups, group_units, red, unit_sums, group_sum);
-    const int slot = p.conv ? p.slot[row] : -1, pos = p.conv ? p.pos[row] : -1;
-    const bool live = slot >= 0 && slot < p.nslots && pos >= 0;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int c = 8 * (tid + u * kRowThreads);
         if (c < p.cols) {
             const float rx = 1.0f / sqrtf(s[u] / count + p.eps);
             float k[8];
-            load8(p.next_coef + c, k);
+            if constexpr (!kEarly) next_coef[0].load(p.next_coef + c);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) k[i] *= x[u][i] * rx;
+            for (int i = 0; i < 8; ++i) k[i] = next_coef[kEarly ? u : 0][i] * (x[u][i] * rx);
             if (p.conv) {
-                E* const ring = static_cast<E*>(p.conv_state) + (int64_t)(live ? slot : 0) * p.taps * p.cols + c;
-                float h[8], w[8];
+                E* const ring = rings + c;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) k[i] = (float)(E)k[i];
-                load8(p.conv + (int64_t)(p.taps - 1) * p.cols + c, w);
                 if (live) store8(ring + (int64_t)(pos % p.taps) * p.cols, k);  // (in the place of a token no row reads any more)
+                if (kEarly && few_taps) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) k[i] += w[i] * k[i];
-                for (int d = 1; live && d < p.taps && d <= pos; ++d) {
-                    load8(ring + (int64_t)((pos - d) % p.taps) * p.cols, h);
-                    load8(p.conv + (int64_t)(p.taps - 1 - d) * p.cols + c, w);
+                    for (int i = 0; i < 8; ++i) k[i] += conv_w[kEarly ? u : 0][0][i] * k[i];
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) k[i] += w[i] * h[i];
+                    for (int d = 1; d < kTaps; ++d)
+                        if (live && d < p.taps && d <= pos) {
+#pragma unroll
+                            for (int i = 0; i < 8; ++i) k[i] += conv_w[kEarly ? u : 0][d][i] * conv_in[kEarly ? u : 0][d][i];
+                        }
+                } else {
+                    float h[8], w[8];
+                    load8(p.conv + (int64_t)(p.taps - 1) * p.cols + c, w);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) k[i] += w[i] * k[i];
+                    for (int d = 1; live && d < p.taps && d <= pos; ++d) {
+                        load8(ring + (int64_t)((pos - d) % p.taps) * p.cols, h);
+                        load8(p.conv + (int64_t)(p.taps - 1 - d) * p.cols + c, w);
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) k[i] += w[i] * h[i];
+                    }
                 }
             }
             if (p.normed) store8(static_cast<E*>(p.normed) + (int64_t)row * p.cols + c, k);
@@ -299,13 +357,17 @@ __global__ __launch_bounds__(kRowThreads) void activate_rows_kernel(const E* in,
     store8(out + (int64_t)row * out_rs + c, a);
 }
 
+constexpr int kEarlyRows = 256;  // a workgroup per compute unit: beyond it other rows fill the waiting, and registers are waves
+
 template <class E, bool GROUPS>
 void launch_residual(const tah_residual_norm_args& p, hipStream_t st) {
     const int units = (p.cols / 8 + kRowThreads - 1) / kRowThreads;
-    if (units <= 1) hipLaunchKernelGGL((residual_norm_kernel<E, 1, GROUPS>), dim3(p.rows), dim3(kRowThreads), 0, st, p);
-    else if (units <= 2) hipLaunchKernelGGL((residual_norm_kernel<E, 2, GROUPS>), dim3(p.rows), dim3(kRowThreads), 0, st, p);
-    else if (units <= 4) hipLaunchKernelGGL((residual_norm_kernel<E, 4, GROUPS>), dim3(p.rows), dim3(kRowThreads), 0, st, p);
-    else hipLaunchKernelGGL((residual_norm_kernel<E, kMaxUnits, GROUPS>), dim3(p.rows), dim3(kRowThreads), 0, st, p);
+    const bool early = p.rows <= kEarlyRows;
+    auto* const f = units <= 1   ? (early ? &residual_norm_kernel<E, 1, GROUPS, true> : &residual_norm_kernel<E, 1, GROUPS, false>)
+                    : units <= 2 ? (early ? &residual_norm_kernel<E, 2, GROUPS, true> : &residual_norm_kernel<E, 2, GROUPS, false>)
+                    : units <= 4 ? &residual_norm_kernel<E, 4, GROUPS, false>
+                                 : &residual_norm_kernel<E, kMaxUnits, GROUPS, false>;
+    hipLaunchKernelGGL(f, dim3(p.rows), dim3(kRowThreads), 0, st, p);
 }
 
 template <class E>

@@ -1,6 +1,7 @@
 """Layer mechanisms (tah_amd.mixers, include/tah_mixers.h), each alone, against the plain oracle: on the CPU execution build
 at small sizes, on the GPU at those and at larger ones."""
 import pytest
+import torch
 
 from tests import emu_util
 from tests import zedudra_cases as D
@@ -214,3 +215,46 @@ def test_activations_gpu(dtype):
 @pytest.mark.parametrize("case", range(len(EXPERTS_GPU)))
 def test_grouped_experts_gpu(dtype, case):
     D.moe_case("cuda", Z.DTYPES[dtype], *EXPERTS_GPU[case])
+
+
+def _route_case(dev, rows, experts, top, groups, keep, sigmoid=False):
+    """Scores that the inputs are (the router is the identity), many of them equal: the chosen ones against a plain ordering,
+    the lower index first among equals, groups by the sum of their two largest."""
+    from tah_amd.ops import _call
+    cols = (experts + 7) // 8 * 8
+    g = torch.Generator().manual_seed(experts + top)
+    z = torch.randint(-24, 25, (rows, experts), generator=g).float() / 8
+    if rows > 3:
+        z[1], z[2, :experts // 2] = 0.5, -1.0
+    x = torch.zeros(rows, cols)
+    x[:, :experts] = z
+    index, weight = torch.full((rows, top), -1, dtype=torch.int32, device=dev), torch.zeros(rows, top, device=dev)
+    _call("moe_route", x.to(dev), torch.eye(experts, cols).to(torch.bfloat16).to(dev), None, index, weight, None, int(sigmoid), groups, keep)
+    size = experts // groups
+    for r, s in enumerate((torch.sigmoid(z) if sigmoid else z).tolist()):
+        two = lambda i: sum(sorted(s[i * size:(i + 1) * size])[-2:])
+        best = sorted(range(groups), key=lambda i: (-two(i), i))[:keep]
+        allowed = [e for i in best for e in range(i * size, (i + 1) * size)]
+        want = sorted(allowed, key=lambda e: (-s[e], e))[:top]
+        assert index[r].tolist() == want, (r, index[r].tolist(), want)
+        v = torch.tensor([s[e] for e in want], dtype=torch.float64)
+        assert torch.allclose(weight[r].cpu().double(), v if sigmoid else torch.softmax(v, 0), rtol=1e-5)
+
+
+ROUTES = [(5, 8, 8, 1, 1), (4, 63, 5, 1, 1), (6, 64, 8, 8, 4), (4, 65, 64, 1, 1), (4, 128, 6, 64, 3), (4, 256, 8, 1, 1), (4, 260, 7, 65, 9), (5, 320, 3, 2, 1)]
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+@pytest.mark.parametrize("rows,experts,top,groups,keep", ROUTES[1:4] + ROUTES[6:7])
+def test_router_choice_among_equal_scores_on_cpu_shim(rows, experts, top, groups, keep):
+    with emu_util.emulated():
+        _route_case("cpu", rows, experts, top, groups, keep)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,experts,top,groups,keep", ROUTES + [(300, 64, 8, 8, 4), (300, 256, 8, 1, 1), (300, 300, 4, 75, 10)])
+def test_router_choice_among_equal_scores_gpu(rows, experts, top, groups, keep):
+    print(f"route rows={rows} experts={experts} top={top} groups={groups} keep={keep}", flush=True)
+    _route_case("cuda", rows, experts, top, groups, keep)
+    if groups == 1:
+        _route_case("cuda", rows, experts, top, groups, keep, sigmoid=True)
