@@ -5,7 +5,8 @@
 //  * moe_route_kernel: router logits in float32, their scores, the open groups of experts, the largest ones and their
 //    weights; RB rows per workgroup share the router's weights, and a wave takes EB experts at a time so that they share
 //    the rows' reads.  Each of the largest is one maximum over the wave inside the vector pipe (four lane exchanges of
-//    registers and four lanes read out): as twelve exchanges through LDS each, eight of them took a third of the kernel.
+//    registers and four lanes read out): as twelve exchanges through LDS each, eight of them took a third of the kernel.  64 experts, 2048 columns: a softmax router takes
+//    9.8 -> 7.1 us for one row, 10.2 -> 7.4 for 32, 78 -> 72 for 8192; grouped sigmoid scores 12.8 -> 8.1, 13.1 -> 8.4, 82 -> 70.
 //  * moe_plan_kernel: counting sort of the (row, choice) pairs by expert, each expert's rows padded to whole tiles.
 //  * moe_tile_kernel: bf16 tiles of 128 places x 256 weight rows on the matrix cores, both operands staged through LDS
 //    by asynchronous copies, two stages ahead; gate and up rows of the same columns share a wave, which applies the gate.
