@@ -541,7 +541,13 @@ typedef struct tah_greedy_step_args {
     int32_t* out_len;         /* [rows] += 1 for rows still unfinished after this step */
     int64_t* n_hard;          /* += hard rows among those that decoded */
     int64_t* n_steps;         /* += rows that decoded */
+    /* Optional: tah_greedy_workspace_bytes(rows) bytes, 8-byte aligned, zeroed once by the caller; each call leaves them
+     * zeroed.  For one call at a time: calls on different streams take different ones.  Several workgroups then share a
+     * row, and the launch also advances step_idx[0] (which must be writable) by one when all rows are done. */
+    void* workspace;
+    size_t workspace_bytes;
 } tah_greedy_step_args;
+size_t tah_greedy_workspace_bytes(int32_t rows);
 int tah_greedy_step(const tah_greedy_step_args* args, tah_stream_t stream);
 
 /* Start of a generation step (one token per sequence), in one launch: for row i, active[i] = !finished[i]; slot[i] = i
@@ -631,6 +637,8 @@ typedef struct tah_greedy_tick_args {
     int64_t* n_hard;
     int64_t* n_steps;
     const int64_t* chosen;    /* [rows] or NULL: take these tokens instead of the arg-max */
+    void* workspace;          /* optional, as in tah_greedy_step_args: several workgroups share a row */
+    size_t workspace_bytes;
 } tah_greedy_tick_args;
 int tah_greedy_tick(const tah_greedy_tick_args* args, tah_stream_t stream);
 

@@ -146,7 +146,7 @@ class GreedyTickArgs(C.Structure):
         ("rows", c_int32), ("vocab", c_int32), ("eos", c_int32), ("limit", c_int32),
         ("hard_now", c_void_p), ("phase", c_void_p), ("tok", c_void_p), ("finished", c_void_p), ("pos", c_void_p),
         ("out_tokens", c_void_p), ("out_stride", c_int64), ("out_len", c_void_p), ("hard_len", c_void_p),
-        ("n_hard", c_void_p), ("n_steps", c_void_p), ("chosen", c_void_p),
+        ("n_hard", c_void_p), ("n_steps", c_void_p), ("chosen", c_void_p), ("workspace", c_void_p), ("workspace_bytes", C.c_size_t),
     ]
 
 
@@ -209,6 +209,7 @@ class GreedyStepArgs(C.Structure):
         ("rows", c_int32), ("vocab", c_int32), ("eos", c_int32),
         ("tok", c_void_p), ("finished", c_void_p), ("pos", c_void_p), ("out_tokens", c_void_p), ("out_stride", c_int64),
         ("step_idx", c_void_p), ("out_cols", c_int32), ("out_len", c_void_p), ("n_hard", c_void_p), ("n_steps", c_void_p),
+        ("workspace", c_void_p), ("workspace_bytes", C.c_size_t),
     ]
 
 
@@ -340,6 +341,7 @@ PROTOTYPES = {
     "tah_duo_bwd_workspace_bytes": (C.c_size_t, [c_int32] * 9),
     "tah_duo_schedule_bytes": (C.c_size_t, [c_int32] * 7),
     "tah_duo_schedule_build": (C.c_int, [C.POINTER(DuoScheduleArgs), c_void_p]),
+    "tah_greedy_workspace_bytes": (C.c_size_t, [c_int32]),
     "tah_greedy_step": (C.c_int, [C.POINTER(GreedyStepArgs), c_void_p]),
     "tah_silu_mul_normed": (C.c_int, [c_void_p, c_void_p, c_int32, c_int32, c_int64, c_int64, c_void_p, c_int64, c_int32, c_float,
                                       c_void_p]),

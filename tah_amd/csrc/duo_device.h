@@ -37,10 +37,14 @@ typedef __attribute__((address_space(3))) int lds_int;
 template <class T> inline void device_store(T* p, T v) { __atomic_store(p, &v, __ATOMIC_SEQ_CST); }
 template <class T> inline T device_load(const T* p) { T v; __atomic_load(const_cast<T*>(p), &v, __ATOMIC_SEQ_CST); return v; }
 inline int device_add(int32_t* p, int v) { return __atomic_fetch_add(p, v, __ATOMIC_SEQ_CST); }
+inline void device_max(unsigned long long* p, unsigned long long v) {
+    for (unsigned long long now = device_load(p); now < v && !__atomic_compare_exchange_n(p, &now, v, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST);) {}
+}
 #else
 template <class T> __device__ __forceinline__ void device_store(T* p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 template <class T> __device__ __forceinline__ T device_load(const T* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ int device_add(int32_t* p, int v) { return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ void device_max(unsigned long long* p, unsigned long long v) { __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 #endif
 
 constexpr int kWave = 64;

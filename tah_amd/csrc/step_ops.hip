@@ -83,6 +83,8 @@ struct GreedyParams {
     int32_t out_cols;
     int32_t* out_len;
     unsigned long long *n_hard, *n_steps;
+    unsigned long long* best;  // several workgroups per row: [rows], 0 between calls ...
+    int32_t* count;            // ... and [rows + 1]
 };
 
 __device__ __forceinline__ void take_better(float& bv, int& bi, float v, int i) {
@@ -92,32 +94,35 @@ __device__ __forceinline__ void take_better(float& bv, int& bi, float v, int i) 
     }
 }
 
-// Arg-max over a row of logits a[0 .. vocab) -- of bf16(a + b) when b is given (the running sum of the iterations'
-// logits lives in the model dtype) -- by the whole workgroup; the lower index among equals.  Valid in thread 0.
-__device__ __forceinline__ int row_argmax(const __bf16* a, const __bf16* b, int vocab, float* wv, int* wi) {
+// Arg-max over the pieces [first, last) of eight of a row of logits a[0 .. vocab) -- of bf16(a + b) when b is given (the
+// running sum of the iterations' logits lives in the model dtype) -- and, with `tail`, over what is left behind the last whole piece,
+// by the whole workgroup; the lower index among equals.  Valid in thread 0; 0x7fffffff when nothing is above -inf.
+template <int kThreads>
+__device__ __forceinline__ int part_argmax(const __bf16* a, const __bf16* b, bool both, int vocab, int first, int last, bool tail, float* wv,
+                                           int* wi, float& best) {
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-    const bool both = b != nullptr;
     float bv = -__builtin_inff();
     int bi = 0x7fffffff;
-    const int nvec = vocab / 8;
-    // ten 16-byte pieces per pass, all loaded before the first is looked at (two passes over a vocabulary of 152 K):
-    // 32 workgroups read 19 MB, and what a thread waits for is memory latency
+    // ten 16-byte pieces per pass, all loaded before the first is looked at: what a thread waits for is memory latency
     constexpr int kAhead = 10;
-    for (int c0 = tid; c0 < nvec; c0 += kAhead * kGreedyThreads) {
+    for (int c0 = first + tid; c0 < last; c0 += kAhead * kThreads) {
         u32x4 x[kAhead], y[kAhead];
 #pragma unroll
         for (int u = 0; u < kAhead; ++u) {
-            const int c = c0 + u * kGreedyThreads;
-            x[u] = y[u] = u32x4{0u, 0u, 0u, 0u};
-            if (c < nvec) {
-                x[u] = *reinterpret_cast<const u32x4*>(a + 8 * c);
-                if (both) y[u] = *reinterpret_cast<const u32x4*>(b + 8 * c);
-            }
+            const int c = c0 + u * kThreads;
+            x[u] = u32x4{0u, 0u, 0u, 0u};
+            if (c < last) x[u] = *reinterpret_cast<const u32x4*>(a + 8 * c);
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {  // (behind the first ones: `both` may still be on its way)
+            const int c = c0 + u * kThreads;
+            y[u] = u32x4{0u, 0u, 0u, 0u};
+            if (both && c < last) y[u] = *reinterpret_cast<const u32x4*>(b + 8 * c);
         }
 #pragma unroll
         for (int u = 0; u < kAhead; ++u) {
-            const int c = c0 + u * kGreedyThreads;
-            if (c >= nvec) break;
+            const int c = c0 + u * kThreads;
+            if (c >= last) break;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 float lo = lo_f(x[u][q]), hi = hi_f(x[u][q]);
@@ -131,11 +136,12 @@ __device__ __forceinline__ int row_argmax(const __bf16* a, const __bf16* b, int 
             }
         }
     }
-    for (int i = nvec * 8 + tid; i < vocab; i += kGreedyThreads) {  // a tail that is not a multiple of 8
-        float v = (float)a[i];
-        if (both) v = (float)(__bf16)(v + (float)b[i]);
-        take_better(bv, bi, v, i);
-    }
+    if (tail)
+        for (int i = vocab / 8 * 8 + tid; i < vocab; i += kThreads) {  // a tail that is not a multiple of 8
+            float v = (float)a[i];
+            if (both) v = (float)(__bf16)(v + (float)b[i]);
+            take_better(bv, bi, v, i);
+        }
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) take_better(bv, bi, __shfl_xor(bv, m), __shfl_xor(bi, m));
     if (lane == 0) {
@@ -144,35 +150,102 @@ __device__ __forceinline__ int row_argmax(const __bf16* a, const __bf16* b, int 
     }
     __syncthreads();
     if (tid != 0) return 0;
-    for (int w = 1; w < kGreedyThreads / kWave; ++w) take_better(bv, bi, wv[w], wi[w]);
-    return bi == 0x7fffffff ? 0 : bi;
+    for (int w = 1; w < kThreads / kWave; ++w) take_better(bv, bi, wv[w], wi[w]);
+    best = bv;
+    return bi;
+}
+__device__ __forceinline__ int row_argmax(const __bf16* a, const __bf16* b, int vocab, float* wv, int* wi) {
+    float best;
+    const int i = part_argmax<kGreedyThreads>(a, b, b != nullptr, vocab, 0, vocab / 8, true, wv, wi, best);
+    return i == 0x7fffffff ? 0 : i;
+}
+
+// A row's arg-max shared by workgroups of 256 threads with ten pieces of 16 bytes each, all in flight at once.  One compute unit
+// takes 304 KB (a vocabulary of 151936) no faster than its own loads in flight allow, whatever else is idle: the greedy step of one such row
+// takes 12.9 us with one workgroup and 7.6 with eight, of 8 rows 13.5 and 8.3, of 32 rows 13.7 and 8.5, of 128 rows (the chip
+// is full either way) 16.8 and 15.7; behind the output head, with the launch between, 11-13 and 6.2-6.8.  What is left is trips to
+// memory one after the other: the logits, the maximum, the count, the answer.  Each
+// offers its best as one number, value above index, to a device-scope maximum; the last of the row to arrive has the
+// answer, returns true in thread 0 and leaves `best` and `count` at 0 for the next launch.  Every workgroup of the row comes here.
+constexpr int kArgmaxThreads = 256, kArgmaxPieces = 10 * kArgmaxThreads;
+__host__ __device__ inline int argmax_parts(int vocab) { return vocab / 8 > kArgmaxPieces ? (vocab / 8 + kArgmaxPieces - 1) / kArgmaxPieces : 1; }
+__device__ __forceinline__ bool shared_argmax(const __bf16* a, const __bf16* b, bool both, int vocab, int part, int parts, unsigned long long* best,
+                                              int32_t* count, float* wv, int* wi, int64_t& answer) {
+    const int pieces = vocab / 8, per = (pieces + parts - 1) / parts;
+    const int first = part * per, last = first + per < pieces ? first + per : pieces;
+    float v;
+    const int i = part_argmax<kArgmaxThreads>(a, b, both, vocab, first, last, part == parts - 1, wv, wi, v);
+    if (threadIdx.x != 0) return false;
+    if (i != 0x7fffffff) {
+        const uint32_t bits = __float_as_uint(v + 0.0f);  // (-0 and 0 are equal)
+        const uint32_t key = bits & 0x80000000u ? ~bits : bits | 0x80000000u;
+        device_max(best, (unsigned long long)key << 32 | (0xffffffffu - (uint32_t)i));
+        TAH_WAIT_VMEM();
+    }
+    if (device_add(count, 1) != parts - 1) return false;
+    const unsigned long long won = device_load(best);
+    device_store(best, 0ull);
+    device_store(count, 0);
+    answer = won ? (int64_t)(0xffffffffu - (uint32_t)won) : 0;
+    return true;
+}
+
+// the loop's bookkeeping for a row (tah/model/utils.py:228-262): a row ends with its end-of-sequence token, which is not
+// part of its output; rows that have ended write zeros
+struct GreedyRow {
+    bool active, hard;
+    int32_t out_len, pos;
+    int64_t column;
+};
+__device__ __forceinline__ GreedyRow greedy_row(const GreedyParams& p, int row) {
+    return {p.finished[row] == 0, p.hard != nullptr && p.hard[row] != 0, p.out_len[row], p.pos[row], p.step_idx[0]};
+}
+__device__ __forceinline__ void greedy_step_row(const GreedyParams& p, int row, const GreedyRow& r, int64_t nxt) {
+    bool done = !r.active;
+    if (r.active && p.eos >= 0 && nxt == p.eos) done = true;
+    const int64_t column = r.column;
+    const bool room = column >= 0 && column < p.out_cols;  // a step beyond the buffer ends the row instead of writing
+    if (!room) done = true;
+    p.finished[row] = done ? 1 : 0;
+    if (room) p.out_tokens[(int64_t)row * p.out_stride + column] = done ? 0 : nxt;
+    if (!done) p.out_len[row] = r.out_len + 1;
+    if (r.active) {
+        p.pos[row] = r.pos + 1;
+        atomicAdd(p.n_steps, 1ull);
+        if (r.hard) atomicAdd(p.n_hard, 1ull);
+    }
+    p.tok[row] = nxt;
 }
 
 __global__ __launch_bounds__(kGreedyThreads) void greedy_step_kernel(const GreedyParams p) {
     __shared__ float wv[kGreedyThreads / kWave];
     __shared__ int wi[kGreedyThreads / kWave];
     const int row = blockIdx.x, tid = threadIdx.x;
-    const bool active = p.finished[row] == 0;  // uniform per workgroup
-    const bool both = p.l1 != nullptr && p.hard != nullptr && p.hard[row] != 0;
+    const GreedyRow r = greedy_row(p, row);
     int64_t nxt = 0;
-    if (active) nxt = row_argmax(p.l0 + (int64_t)row * p.rs0, both ? p.l1 + (int64_t)row * p.rs1 : nullptr, p.vocab, wv, wi);
-    if (tid != 0) return;
-    // the loop's bookkeeping for this row (tah/model/utils.py:228-262): a row ends with its end-of-sequence token,
-    // which is not part of its output; rows that have ended write zeros
-    bool done = !active;
-    if (active && p.eos >= 0 && nxt == p.eos) done = true;
-    const int64_t column = p.step_idx[0];
-    const bool room = column >= 0 && column < p.out_cols;  // a step beyond the buffer ends the row instead of writing
-    if (!room) done = true;
-    p.finished[row] = done ? 1 : 0;
-    if (room) p.out_tokens[(int64_t)row * p.out_stride + column] = done ? 0 : nxt;
-    if (!done) p.out_len[row] += 1;
-    if (active) {
-        p.pos[row] += 1;
-        atomicAdd(p.n_steps, 1ull);
-        if (p.hard != nullptr && p.hard[row] != 0) atomicAdd(p.n_hard, 1ull);
+    if (r.active)  // (uniform per workgroup)
+        nxt = row_argmax(p.l0 + (int64_t)row * p.rs0, r.hard ? p.l1 + (int64_t)row * p.rs1 : nullptr, p.vocab, wv, wi);
+    __syncthreads();  // every thread has read the row's state before thread 0 changes it
+    if (tid == 0) greedy_step_row(p, row, r, nxt);
+}
+
+// The same with several workgroups per row, and the step counter advanced once all rows are done.  A row's state is read by all
+// of its workgroups up front, beside the logits, and changed by the last of them to arrive, the counter by the last row's.
+__global__ __launch_bounds__(kArgmaxThreads) void greedy_step_parts_kernel(const GreedyParams p) {
+    __shared__ float wv[kArgmaxThreads / kWave];
+    __shared__ int wi[kArgmaxThreads / kWave];
+    const int row = blockIdx.y, rows = gridDim.y;
+    const GreedyRow r = greedy_row(p, row);
+    int64_t nxt = 0;
+    // (rows that have ended are read as well: nothing then waits for `finished` before the logits are asked for)
+    if (!shared_argmax(p.l0 + (int64_t)row * p.rs0, p.l1 + (int64_t)row * p.rs1, r.hard, p.vocab, blockIdx.x, gridDim.x, p.best + row, p.count + row, wv, wi,
+                       nxt))
+        return;
+    greedy_step_row(p, row, r, r.active ? nxt : 0);
+    if (device_add(p.count + rows, 1) == rows - 1) {
+        *const_cast<int64_t*>(p.step_idx) = r.column + 1;
+        device_store(p.count + rows, 0);
     }
-    p.tok[row] = nxt;
 }
 
 
@@ -196,43 +269,68 @@ struct TickParams {
     int64_t out_stride;
     unsigned long long *n_hard, *n_steps;
     const int64_t* chosen;
+    unsigned long long* best;  // as in GreedyParams
+    int32_t* count;
 };
 
-__global__ __launch_bounds__(kGreedyThreads) void greedy_tick_kernel(const TickParams p) {
-    __shared__ float wv[kGreedyThreads / kWave];
-    __shared__ int wi[kGreedyThreads / kWave];
-    const int row = blockIdx.x, tid = threadIdx.x;
-    const bool ended = p.finished[row] != 0;
+struct TickRow {
+    bool ended, again, both;
+    int32_t out_len, pos, hard_len;
+};
+__device__ __forceinline__ TickRow tick_row(const TickParams& p, int row) {
     const int ph = p.phase[row];
-    const bool again = ph == 0 && p.hard_now[row] != 0;
-    __syncthreads();  // every thread has read the row's state before thread 0 changes it: the branches below are uniform
-    if (ended) return;
-    if (again) {  // the token takes a second iteration: next tick
-        if (tid == 0) p.phase[row] = 1;
+    return {p.finished[row] != 0, ph == 0 && p.hard_now[row] != 0, ph != 0, p.out_len[row], p.pos[row], p.hard_len[row]};
+}
+__device__ __forceinline__ void greedy_tick_row(const TickParams& p, int row, const TickRow& r, int64_t nxt) {
+    if (r.ended) return;
+    if (r.again) {  // the token takes a second iteration: next tick
+        p.phase[row] = 1;
         return;
     }
-    const bool both = ph != 0;
-    const int64_t nxt = p.chosen ? p.chosen[row]  // (uniform)
-                                 : row_argmax(p.cur + (int64_t)row * p.rs_cur, both ? p.prev + (int64_t)row * p.rs_prev : nullptr, p.vocab, wv, wi);
-    if (tid != 0) return;
     // a row ends with its end-of-sequence token, which is not part of its output (tah/model/utils.py:228-262),
     // or when it has `limit` tokens
     bool done = p.eos >= 0 && nxt == p.eos;
     if (!done) {
-        const int col = p.out_len[row];
+        const int col = r.out_len;
         p.out_tokens[(int64_t)row * p.out_stride + col] = nxt;
         p.out_len[row] = col + 1;
         done = col + 1 >= p.limit;
     }
     p.finished[row] = done ? 1 : 0;
-    p.pos[row] += 1;
+    p.pos[row] = r.pos + 1;
     p.tok[row] = nxt;
     p.phase[row] = 0;
     atomicAdd(p.n_steps, 1ull);
-    if (both) {
-        p.hard_len[row] += 1;  // the second iteration's K/V went into the depth-1 slabs during this tick
+    if (r.both) {
+        p.hard_len[row] = r.hard_len + 1;  // the second iteration's K/V went into the depth-1 slabs during this tick
         atomicAdd(p.n_hard, 1ull);
     }
+}
+
+__global__ __launch_bounds__(kGreedyThreads) void greedy_tick_kernel(const TickParams p) {
+    __shared__ float wv[kGreedyThreads / kWave];
+    __shared__ int wi[kGreedyThreads / kWave];
+    const int row = blockIdx.x, tid = threadIdx.x;
+    const TickRow r = tick_row(p, row);
+    __syncthreads();  // every thread has read the row's state before thread 0 changes it: the branches below are uniform
+    int64_t nxt = 0;
+    if (!r.ended && !r.again)
+        nxt = p.chosen ? p.chosen[row]  // (uniform)
+                       : row_argmax(p.cur + (int64_t)row * p.rs_cur, r.both ? p.prev + (int64_t)row * p.rs_prev : nullptr, p.vocab, wv, wi);
+    if (tid == 0) greedy_tick_row(p, row, r, nxt);
+}
+
+// The same with several workgroups per row, which read its state up front, beside the logits (also of a row that has ended or
+// that takes a second iteration); the last of them to arrive changes it.
+__global__ __launch_bounds__(kArgmaxThreads) void greedy_tick_parts_kernel(const TickParams p) {
+    __shared__ float wv[kArgmaxThreads / kWave];
+    __shared__ int wi[kArgmaxThreads / kWave];
+    const int row = blockIdx.y;
+    const TickRow r = tick_row(p, row);
+    int64_t nxt = 0;
+    if (shared_argmax(p.cur + (int64_t)row * p.rs_cur, p.prev + (int64_t)row * p.rs_prev, r.both, p.vocab, blockIdx.x, gridDim.x, p.best + row,
+                      p.count + row, wv, wi, nxt))
+        greedy_tick_row(p, row, r, nxt);
 }
 
 // ---------------------------------------------------------------------------
@@ -325,6 +423,8 @@ __global__ __launch_bounds__(64) void decider_tail_kernel(const DeciderTailParam
 }  // namespace
 }  // namespace tah
 
+extern "C" size_t tah_greedy_workspace_bytes(int32_t rows) { return rows <= 0 ? 0 : 8 * (size_t)rows + 4 * ((size_t)rows + 1); }
+
 extern "C" int tah_greedy_step(const tah_greedy_step_args* a, tah_stream_t stream) {
     using namespace tah;
     if (!a) return TAH_E_NULL;
@@ -347,6 +447,14 @@ extern "C" int tah_greedy_step(const tah_greedy_step_args* a, tah_stream_t strea
     p.out_cols = a->out_cols;
     p.n_hard = reinterpret_cast<unsigned long long*>(a->n_hard);
     p.n_steps = reinterpret_cast<unsigned long long*>(a->n_steps);
+    if (a->workspace) {
+        if (reinterpret_cast<uintptr_t>(a->workspace) & 7) return TAH_E_ALIGN;
+        if (a->workspace_bytes < tah_greedy_workspace_bytes(a->rows)) return TAH_E_WORKSPACE;
+        p.best = static_cast<unsigned long long*>(a->workspace);
+        p.count = reinterpret_cast<int32_t*>(p.best + a->rows);
+        hipLaunchKernelGGL(greedy_step_parts_kernel, dim3(argmax_parts(a->vocab), a->rows), dim3(kArgmaxThreads), 0, static_cast<hipStream_t>(stream), p);
+        return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
+    }
     hipLaunchKernelGGL(greedy_step_kernel, dim3(a->rows), dim3(kGreedyThreads), 0, static_cast<hipStream_t>(stream), p);
     return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
 }
@@ -442,6 +550,14 @@ extern "C" int tah_greedy_tick(const tah_greedy_tick_args* a, tah_stream_t strea
     p.n_hard = reinterpret_cast<unsigned long long*>(a->n_hard);
     p.n_steps = reinterpret_cast<unsigned long long*>(a->n_steps);
     p.chosen = a->chosen;
+    if (a->workspace && (reinterpret_cast<uintptr_t>(a->workspace) & 7)) return TAH_E_ALIGN;
+    if (a->workspace && a->workspace_bytes < tah_greedy_workspace_bytes(a->rows)) return TAH_E_WORKSPACE;
+    if (a->workspace && !a->chosen) {
+        p.best = static_cast<unsigned long long*>(a->workspace);
+        p.count = reinterpret_cast<int32_t*>(p.best + a->rows);
+        hipLaunchKernelGGL(greedy_tick_parts_kernel, dim3(argmax_parts(a->vocab), a->rows), dim3(kArgmaxThreads), 0, static_cast<hipStream_t>(stream), p);
+        return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
+    }
     hipLaunchKernelGGL(greedy_tick_kernel, dim3(a->rows), dim3(kGreedyThreads), 0, static_cast<hipStream_t>(stream), p);
     return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
 }

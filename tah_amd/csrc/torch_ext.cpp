@@ -759,9 +759,10 @@ Tensor silu_mul(const Tensor& gate_up, const optional<Tensor>& norm_input, doubl
 // Arg-max of the step's final logits and the generation loop's per-row bookkeeping, in place (tah_greedy_step).
 void greedy_step(const Tensor& logits0, const optional<Tensor>& logits1, const optional<Tensor>& hard, int64_t eos, const Tensor& tok,
                  const Tensor& finished, const Tensor& pos, const Tensor& out_tokens, const Tensor& step_idx, const Tensor& out_len,
-                 const Tensor& n_hard, const Tensor& n_steps) {
+                 const Tensor& n_hard, const Tensor& n_steps, const optional<Tensor>& workspace) {
     need_lib();
     Dev d;
+    d.see(workspace);
     for (const Tensor* t : {&logits0, &tok, &finished, &pos, &out_tokens, &step_idx, &out_len, &n_hard, &n_steps}) d.see(*t);
     d.see(logits1); d.see(hard);
     const int64_t rows = logits0.size(0), vocab = logits0.size(1);
@@ -790,6 +791,10 @@ void greedy_step(const Tensor& logits0, const optional<Tensor>& logits1, const o
     a.out_cols = (int32_t)out_tokens.size(1);
     a.out_len = static_cast<int32_t*>(out_len.data_ptr());
     a.n_hard = static_cast<int64_t*>(n_hard.data_ptr()); a.n_steps = static_cast<int64_t*>(n_steps.data_ptr());
+    if (workspace.has_value()) {
+        TORCH_CHECK(workspace->is_contiguous(), "greedy_step: workspace must be contiguous");
+        a.workspace = workspace->data_ptr(); a.workspace_bytes = (size_t)workspace->nbytes();
+    }
     check_rc(g.greedy_step(&a, d.stream()), "tah_greedy_step");
 }
 
@@ -849,9 +854,11 @@ void step_begin(const Tensor& tok, const Tensor& pos, const Tensor& finished, co
 // tah_greedy_tick: tokens and bookkeeping at the end of a tick whose rows are at different latent iterations.
 void greedy_tick(const Tensor& logits, const Tensor& logits_prev, int64_t eos, int64_t limit, const Tensor& hard_now, const Tensor& phase,
                  const Tensor& tok, const Tensor& finished, const Tensor& pos, const Tensor& out_tokens, const Tensor& out_len,
-                 const Tensor& hard_len, const Tensor& n_hard, const Tensor& n_steps, const optional<Tensor>& chosen) {
+                 const Tensor& hard_len, const Tensor& n_hard, const Tensor& n_steps, const optional<Tensor>& chosen,
+                 const optional<Tensor>& workspace) {
     need_lib();
     Dev d;
+    d.see(workspace);
     for (const Tensor* t : {&logits, &logits_prev, &hard_now, &phase, &tok, &finished, &pos, &out_tokens, &out_len, &hard_len, &n_hard, &n_steps}) d.see(*t);
     d.see(chosen);
     const int64_t rows = logits.size(0), vocab = logits.size(1);
@@ -878,6 +885,10 @@ void greedy_tick(const Tensor& logits, const Tensor& logits_prev, int64_t eos, i
     if (chosen.has_value()) {
         TORCH_CHECK(vec_of(*chosen, at::kLong, rows), "greedy_tick: chosen must be int64 [rows]");
         a.chosen = static_cast<const int64_t*>(chosen->data_ptr());
+    }
+    if (workspace.has_value()) {
+        TORCH_CHECK(workspace->is_contiguous(), "greedy_tick: workspace must be contiguous");
+        a.workspace = workspace->data_ptr(); a.workspace_bytes = (size_t)workspace->nbytes();
     }
     check_rc(g.greedy_tick(&a, d.stream()), "tah_greedy_tick");
 }

@@ -213,6 +213,7 @@ class DecodeEngine:
         self.step_idx = torch.zeros(1, dtype=torch.long, device=dev)
         self.out_tokens = torch.zeros(batch, max_len, dtype=torch.long, device=dev)  # generated tokens, column = step
         self.out_len = torch.zeros(batch, dtype=torch.int32, device=dev)             # tokens of each row before its end
+        self.greedy_workspace = ops.greedy_workspace(batch, dev)
         self.host_positions = 0  # upper bound on any sequence's length, kept on the host for capacity checks
         self._graph = None
 
@@ -322,8 +323,7 @@ class DecodeEngine:
         if temperature <= 0.0 and self.fused_greedy and l0.dtype == torch.bfloat16 and self.cfg.vocab % 8 == 0:
             # arg-max of the final logits and the bookkeeping below in one launch; the final logits are not formed
             ops.greedy_step(l0, l1, hard, eos, self.tok, self.finished, self.pos, self.out_tokens, self.step_idx, self.out_len,
-                            self.n_hard, self.n_steps)
-            self.step_idx += 1
+                            self.n_hard, self.n_steps, workspace=self.greedy_workspace)  # (advances step_idx)
             return
         if temperature > 0.0:  # final logits as step_logits forms them: l0, plus l1 for hard tokens (the sum in the logits' dtype)
             add = {} if l1 is None else dict(prev=l1, add_prev=hard.to(torch.int32))
@@ -882,7 +882,8 @@ class TaHDecodeEngine(DecodeEngine):
                 chosen = self._draw(logits, temperature, prev=prev["logits_prev"], add_prev=self.phase, **filters).contiguous()
         ops.greedy_tick(logits, self.logits2[1 - parity], eos, limit, hard_now=self.hard, phase=self.phase, tok=self.tok,
                         finished=self.finished, pos=self.pos, out_tokens=self.out_tokens, out_len=self.out_len,
-                        hard_len=self.hard_len, n_hard=self.n_hard, n_steps=self.n_steps, chosen=chosen)
+                        hard_len=self.hard_len, n_hard=self.n_hard, n_steps=self.n_steps, chosen=chosen,
+                        workspace=self.greedy_workspace)
 
     DRAW_AHEAD = 64  # ticks whose uniforms are drawn at a time; with an end-of-sequence token also how often the host looks
 

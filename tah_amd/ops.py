@@ -215,14 +215,15 @@ def step_begin(tok, pos, finished, embed, cos_table, sin_table, *, x, x_packed, 
 
 
 def greedy_tick(logits, logits_prev, eos: int, limit: int, *, hard_now, phase, tok, finished, pos, out_tokens, out_len, hard_len,
-                n_hard, n_steps, chosen=None) -> None:
+                n_hard, n_steps, chosen=None, workspace=None) -> None:
     """End of a tick in which every row advanced by one latent iteration of its own token (``tah_greedy_tick``), all
     updates in place: rows at phase 0 with ``hard_now`` move to phase 1; every other unfinished row gets its token (arg-max
     of ``logits``, or of ``bf16(logits_prev + logits)`` at phase 1) in ``out_tokens[row, out_len[row]]`` and the loop's
     bookkeeping; a row is finished at its end-of-sequence token or with ``limit`` tokens.  ``chosen`` (int64 [rows]):
-    tokens to take instead of the arg-max (sampled from the same final logits by the caller)."""
+    tokens to take instead of the arg-max (sampled from the same final logits by the caller).  ``workspace``: from
+    ``greedy_workspace``; several workgroups then share a row."""
     _call("greedy_tick", logits, logits_prev, int(eos), int(limit), hard_now, phase, tok, finished, pos, out_tokens, out_len,
-          hard_len, n_hard, n_steps, chosen)
+          hard_len, n_hard, n_steps, chosen, workspace)
 
 
 def decider_tail(hidden, w2, b2, threshold: float, *, hard, active=None, pos=None, hard_i32=None, slot=None, q_pos=None) -> None:
@@ -285,12 +286,20 @@ def linear_rows(w_packed: torch.Tensor, x_packed: torch.Tensor, rows: int, n: in
                  float(c0), float(c1))
 
 
-def greedy_step(logits0, logits1, hard, eos: int, tok, finished, pos, out_tokens, step_idx, out_len, n_hard, n_steps) -> None:
+def greedy_workspace(rows: int, device) -> torch.Tensor:
+    """What ``greedy_step`` and ``greedy_tick`` of ``rows`` rows keep between the workgroups of a row
+    (``tah_greedy_workspace_bytes``), zeroed: for one call at a time, one per stream."""
+    return torch.zeros((12 * rows + 4 + 7) // 8, dtype=torch.int64, device=device)
+
+
+def greedy_step(logits0, logits1, hard, eos: int, tok, finished, pos, out_tokens, step_idx, out_len, n_hard, n_steps,
+                workspace=None) -> None:
     """One greedy generation step after the logits (``tah_greedy_step``), all updates in place on the device.
 
     Per row: final logits = ``logits0`` (bf16 [rows, vocab]), or ``bf16(logits0 + logits1)`` where ``hard`` (bool
     [rows]) is set; ``tok`` = their arg-max (0 for finished rows); a row whose token is ``eos`` (>= 0) becomes
     ``finished`` and the token stays out of its output; ``out_tokens[:, step_idx]`` and ``out_len`` record the
-    output, ``pos`` advances for the rows that decoded, ``n_steps`` / ``n_hard`` count them.
+    output, ``pos`` advances for the rows that decoded, ``n_steps`` / ``n_hard`` count them.  With ``workspace`` (from
+    ``greedy_workspace``) several workgroups share a row and ``step_idx`` advances by one in the same launch.
     """
-    _call("greedy_step", logits0, logits1, hard, int(eos), tok, finished, pos, out_tokens, step_idx, out_len, n_hard, n_steps)
+    _call("greedy_step", logits0, logits1, hard, int(eos), tok, finished, pos, out_tokens, step_idx, out_len, n_hard, n_steps, workspace)

@@ -348,7 +348,7 @@ class StackEngine(DecodeEngine):
 
     # ── generation (DecodeEngine) ────────────────────────────────────────
     def _parts(self):
-        return self._single(self.tok, self.pos, self.finished), None, None, ~self.finished
+        return self._single(self.tok, self.pos, self.finished), None, None, self.act  # (which rows had not finished: embed_rows)
 
     def _advanced(self, steps: int) -> None:
         super()._advanced(steps)

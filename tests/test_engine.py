@@ -32,7 +32,7 @@ def _same_greedy(device, **size):
     assert bool(a[3].any())  # some row did finish
 
 
-def _greedy_step_case(device, rows=6, vocab=200, seed=0):
+def _greedy_step_case(device, rows=6, vocab=200, seed=0, workspace=False):
     """ops.greedy_step against the engine's own torch bookkeeping (engine.py:_step_inplace) on random logits with
     ties, rows already finished, rows that hit the end-of-sequence token and rows that took a second iteration."""
     from tah_amd import ops
@@ -42,6 +42,8 @@ def _greedy_step_case(device, rows=6, vocab=200, seed=0):
     l1p = (torch.randn(rows, padded, generator=g) * 3).to(torch.bfloat16)
     l0, l1 = l0p[:, :vocab], l1p[:, :vocab]
     l0[1, 7] = l0[1, 150] = 40.0               # a tie at the maximum: the lower index wins
+    if workspace:
+        l0[1, vocab - 1] = 40.0                # (and in the last workgroup's part)
     hard = torch.tensor([False, False, True, True, False, True])[:rows]
     finished = torch.tensor([False, False, False, True, False, False])[:rows]
     final = torch.where(hard[:, None], (l0 + l1).float(), l0.float())
@@ -50,8 +52,9 @@ def _greedy_step_case(device, rows=6, vocab=200, seed=0):
               out_tokens=torch.zeros(rows, 4, dtype=torch.long), step_idx=torch.tensor([2]), out_len=torch.full((rows,), 2, dtype=torch.int32),
               n_hard=torch.tensor(3), n_steps=torch.tensor(11))
     dev = {k: v.clone().to(device) for k, v in st.items()}
+    ws = ops.greedy_workspace(rows, device) if workspace else None
     ops.greedy_step(l0p.to(device)[:, :vocab], l1p.to(device)[:, :vocab], (hard & ~finished).to(device), eos, dev["tok"], dev["finished"], dev["pos"],
-                    dev["out_tokens"], dev["step_idx"], dev["out_len"], dev["n_hard"], dev["n_steps"])
+                    dev["out_tokens"], dev["step_idx"], dev["out_len"], dev["n_hard"], dev["n_steps"], workspace=ws)
     # the same step as the unfused loop writes it
     act = ~st["finished"]
     nxt = torch.where(act, final.argmax(-1), torch.zeros(rows, dtype=torch.long))
@@ -64,15 +67,21 @@ def _greedy_step_case(device, rows=6, vocab=200, seed=0):
     st["n_steps"] += act.sum()
     st["pos"] += act.to(torch.int32)
     st["tok"] = nxt
+    st["step_idx"] += int(workspace)
     for k in st:
         assert torch.equal(dev[k].cpu(), st[k]), k
     # a step beyond the last column of out_tokens (a captured step replayed too often) stores nothing and ends the rows
     dev["step_idx"].fill_(4)
     before = dev["out_tokens"].clone()
     ops.greedy_step(l0p.to(device)[:, :vocab], None, None, -1, dev["tok"], dev["finished"], dev["pos"],
-                    dev["out_tokens"], dev["step_idx"], dev["out_len"], dev["n_hard"], dev["n_steps"])
+                    dev["out_tokens"], dev["step_idx"], dev["out_len"], dev["n_hard"], dev["n_steps"], workspace=ws)
     assert torch.equal(dev["out_tokens"], before) and bool(dev["finished"].all())
     assert torch.equal(dev["out_len"].cpu(), st["out_len"])
+    assert ws is None or not bool(ws.any())  # left as it was found
+
+
+# one workgroup per row, whole pieces only / with a tail; several: the last one full, with a remainder, with only a tail
+SHARED = [200, 203, 3 * 20480, 20480 + 8, 2 * 20480 + 5, 151936]
 
 
 @pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
@@ -80,12 +89,16 @@ def test_greedy_step_kernel_on_cpu_shim():
     with emu_util.emulated():
         _greedy_step_case("cpu")
         _greedy_step_case("cpu", vocab=203, seed=1)   # a vocabulary that is not a multiple of 8
+        for vocab in SHARED[:2] + SHARED[3:5]:
+            _greedy_step_case("cpu", vocab=vocab, seed=vocab, workspace=True)
 
 
 @pytest.mark.gpu
 def test_greedy_step_kernel_gpu():
     _greedy_step_case("cuda", vocab=151936)
     _greedy_step_case("cuda", vocab=1003, seed=2)
+    for vocab in SHARED:
+        _greedy_step_case("cuda", vocab=vocab, seed=vocab, workspace=True)
 
 
 @pytest.mark.gpu

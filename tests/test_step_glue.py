@@ -87,7 +87,7 @@ def _step_begin_phase_case(dev, B=6, H=64, V=30, L=50):
     assert torch.equal(act, ~fin) and torch.equal(el, ~fin & ~second)
 
 
-def _greedy_tick_case(dev, B=7, V=304, limit=5, eos=11):
+def _greedy_tick_case(dev, B=7, V=304, limit=5, eos=11, workspace=False):
     """Every combination of finished / phase / hard_now, a row reaching the limit and a row hitting end-of-sequence."""
     from tah_amd import ops
     g = torch.Generator().manual_seed(6)
@@ -106,7 +106,9 @@ def _greedy_tick_case(dev, B=7, V=304, limit=5, eos=11):
     d = lambda t: t.clone().to(dev)
     st = dict(hard_now=d(hard), phase=d(phase), tok=d(tok), finished=d(fin), pos=d(pos), out_tokens=d(out), out_len=d(out_len),
               hard_len=d(hlen), n_hard=d(n_hard), n_steps=d(n_steps))
-    ops.greedy_tick(d(cur), d(prev), eos, limit, **st)
+    ws = ops.greedy_workspace(B, dev) if workspace else None
+    ops.greedy_tick(d(cur), d(prev), eos, limit, workspace=ws, **st)
+    assert ws is None or not bool(ws.any())  # left as it was found
     both = (cur.float() + prev.float()).to(BF)
     want_tok = {2: int(cur[2].float().argmax()), 3: int(both[3].float().argmax()), 4: int(both[4].float().argmax()), 5: eos,
                 6: int(cur[6].float().argmax())}
@@ -126,7 +128,7 @@ def _greedy_tick_case(dev, B=7, V=304, limit=5, eos=11):
     st = dict(hard_now=d(hard), phase=d(phase), tok=d(tok), finished=d(fin), pos=d(pos), out_tokens=d(out), out_len=d(out_len),
               hard_len=d(hlen), n_hard=d(n_hard), n_steps=d(n_steps))
     chosen = torch.tensor([70, 71, 72, 73, eos, 75, 76])
-    ops.greedy_tick(d(cur), d(prev), eos, limit, chosen=d(chosen), **st)
+    ops.greedy_tick(d(cur), d(prev), eos, limit, chosen=d(chosen), workspace=ws, **st)
     got = {k: v.cpu() for k, v in st.items()}
     assert got["tok"].tolist() == [99, 99, 72, 73, eos, 75, 76] and got["phase"].tolist() == [1, 0, 0, 0, 0, 0, 0]
     assert got["finished"].tolist() == [False, True, False, False, True, False, True]
@@ -142,6 +144,8 @@ def test_step_glue_on_cpu_shim():
         _decider_tail_case("cpu")
         _step_begin_phase_case("cpu")
         _greedy_tick_case("cpu")
+        _greedy_tick_case("cpu", workspace=True)
+        _greedy_tick_case("cpu", V=20480 + 8, workspace=True)  # two workgroups per row
 
 
 @pytest.mark.gpu
@@ -153,3 +157,5 @@ def test_step_glue_gpu():
     _step_begin_phase_case("cuda")
     _greedy_tick_case("cuda")
     _greedy_tick_case("cuda", V=151936)
+    _greedy_tick_case("cuda", V=20480 + 8, workspace=True)
+    _greedy_tick_case("cuda", V=151936, workspace=True)
