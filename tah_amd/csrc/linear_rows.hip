@@ -30,6 +30,8 @@
 // (kFold, H8 below).
 #include <hip/hip_runtime.h>
 
+#include <utility>
+
 #include "mixer_device.h"
 
 namespace tah {
@@ -74,6 +76,24 @@ __device__ __host__ __forceinline__ int64_t packed_rows_unit(int r, int k) {
 
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + fast_exp2(-x * kLog2e)); }
 
+// x[s][0] of step s: lane c of a k group takes what lane c + kRows * (s % kPer) of the group loaded (lanes past the group's end: 0)
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
+template <int kRows, int kShift>
+__device__ __forceinline__ bf16x8 from_lane_above(bf16x8 v) {
+    if constexpr (kShift == 0) return v;
+    else {
+        u32x4 u = __builtin_bit_cast(u32x4, v);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) u[q] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)u[q], 0x100 + kShift, 0xf, 0xf, true);  // row_shl
+        return __builtin_bit_cast(bf16x8, u);
+    }
+}
+template <int kPer, int kRows, class X, int... S>
+__device__ __forceinline__ void take_steps(const bf16x8* together, X& x, std::integer_sequence<int, S...>) {
+    ((x[S][0] = from_lane_above<kRows, kRows * (S % kPer)>(together[S / kPer])), ...);
+}
+
+
 // NC: weight tiles per workgroup (1 plain, 2 or 3 for gate|up).  CH: steps per chunk of loads.  PW: steps per wave
 // when K is known at compile time (K = 32 * 8 * PW), 0: any K % 32 == 0.  NH: row halves per workgroup -- 2: all 32
 // rows; 1: sixteen rows, the grid holds a workgroup per (column group, half) (or only the first half when there
@@ -84,8 +104,8 @@ __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + fast_exp2(
 // occupy half of the compute units occupies all.  A load then covers two k steps of the eight columns (lanes c < 8 the
 // even one, the others the odd one: 128 contiguous bytes each), and each loaded operand is multiplied twice, by either
 // step's rows; of the first product the columns below 8 count, of the second those from 8 on.  At one to eight rows o
-// (8 MB) takes 5.0 -> 4.7 us, down (25 MB) 9.5 -> 8.1: 3.5 us of launch, latency and reduction and the weight at 5.6 TB/s.
-template <int NC, int CH, int EPI, int PW, int NH, bool H8 = false, bool kFold = false>
+// (8 MB) takes 5.0 -> 4.7 us, down (25 MB) 9.5 -> 8.1 (both less again with the rows' operand folded, below).
+template <int NC, int CH, int EPI, int PW, int NH, bool H8 = false, int kFold = 0>
 __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParams p) {
     __shared__ __align__(16) float red[kLinWaves][NC][16 * NH][kTileCols];
     __shared__ float ssq[kLinWaves][16 * NH];
@@ -139,7 +159,13 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
                    : pw + ((int64_t)(group * NC + t) * steps + s0) * 64 + lane;
     // kFold: the lanes of rows past the last one read row 0's operand again instead of their zeros (their results are not used):
     // with up to eight rows a load then touches a half to a quarter of the bytes (q|k|v at one to eight rows 5.75 -> 5.4 us).
-    const bf16x8* xb = px + (int64_t)s0 * 128 + 64 * half + (kFold ? 16 * kg + (c < p.rows ? c : 0) : lane);
+    // Folded further where a wave's steps are one chunk: with one, two, four or eight rows (the next of these) the sixteen lanes of a k
+    // group hold sixteen, eight, four or two steps of them, so 24 steps take 2, 3, 6 or 12 loads instead of 24 -- behind those the
+    // weights' own would wait -- and a lane gets its step from its neighbours inside the vector pipe: down 8.2 -> 7.5 us at one to
+    // eight rows (of a bound of 7.0, the same kernel with two of its operand loads), q|k|v 5.8 -> 5.6, o 4.6 -> 4.45.
+    constexpr int kFoldRows = kFold > 0 && kFold < 16 ? kFold : 16, kPerLoad = kFoldRows < 16 ? 16 / kFoldRows : 0;
+    static_assert(kPerLoad == 0 || (CH == PW && NH == 1), "one chunk");
+    const bf16x8* xb = px + (int64_t)s0 * 128 + 64 * half + (kPerLoad ? (c / kFoldRows) * 128 + 16 * kg + c % kFoldRows : kFold ? 16 * kg + (c < p.rows ? c : 0) : lane);
 
     struct Buf {
         bf16x8 w[H8 ? CH / 2 : CH][NC], x[CH][NH];
@@ -156,12 +182,22 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
     auto issue = [&](int ch, Buf& b) __attribute__((always_inline)) {
         // the rows' operand first: it comes from L2 and is there long before the weights are, and a wave's loads
         // return in order -- behind the weight loads it would only arrive after their trip to HBM (down 11.2 -> 9.6 us)
+        bf16x8 together[kPerLoad ? (CH + kPerLoad - 1) / kPerLoad : 1];
+        if constexpr (kPerLoad > 0) {
 #pragma unroll
-        for (int s = 0; s < CH; ++s) {
-            const int st = ch * CH + s;
-            const int64_t sti = (PW > 0 || st < nst) ? st : 0;
-            b.x[s][0] = xb[sti * 128];
-            if constexpr (NH == 2) b.x[s][1] = xb[sti * 128 + 64];
+            for (int j = 0; j < (CH + kPerLoad - 1) / kPerLoad; ++j) {
+                int back = j * kPerLoad + c / kFoldRows - (CH - 1);  // a last load's steps past the chunk: the last step again
+                back = back > 0 ? back : 0;
+                together[j] = xb[(j * kPerLoad - back) * 128];
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < CH; ++s) {
+                const int st = ch * CH + s;
+                const int64_t sti = (PW > 0 || st < nst) ? st : 0;
+                b.x[s][0] = xb[sti * 128];
+                if constexpr (NH == 2) b.x[s][1] = xb[sti * 128 + 64];
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -170,6 +206,11 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
             const int64_t sti = (PW > 0 || st < nst) ? st : 0;
 #pragma unroll
             for (int t = 0; t < NC; ++t) b.w[H8 ? s / 2 : s][t] = __builtin_nontemporal_load(wb[t] + sti * 64);
+        }
+        if constexpr (kPerLoad > 0) {  // each step's rows move to the lanes of the first rows while the weights are on their way
+            __builtin_amdgcn_sched_barrier(0);
+            take_steps<kPerLoad, kFoldRows>(together, b.x, std::make_integer_sequence<int, CH>{});
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
     auto multiply = [&](int ch, Buf& b) __attribute__((always_inline)) {
@@ -551,6 +592,22 @@ void launch_wide(LinParams& p, int groups, hipStream_t st) {
     hipLaunchKernelGGL((linear_wide_kernel<EPI, PW>), dim3(groups < kResident ? groups : kResident), dim3(kLinThreads), 0, st, p);
 }
 
+// few rows: the rows operand folded as far as their number allows
+template <int NC, int CH, int EPI, int PW, bool H8>
+void launch_folded(const LinParams& p, int workgroups, int batch, hipStream_t st) {
+    const dim3 grid(workgroups, batch), block(kLinThreads);
+    if constexpr (PW > 0 && NC != 2) {
+        const auto run = [&](auto fold) { hipLaunchKernelGGL((linear_rows_kernel<NC, CH, EPI, PW, 1, H8, decltype(fold)::value>), grid, block, 0, st, p); };
+        if constexpr (CH == PW) {
+            if (p.rows <= 1) return run(std::integral_constant<int, 1>{});
+            if (p.rows <= 2) return run(std::integral_constant<int, 2>{});
+            if (p.rows <= 4) return run(std::integral_constant<int, 4>{});
+            if (p.rows <= 8) return run(std::integral_constant<int, 8>{});
+        }
+        run(std::integral_constant<int, 16>{});
+    }
+}
+
 template <int NC, int CH, int EPI, int PW>
 void launch(LinParams& p, int groups, int batch, hipStream_t st) {
     p.groups = groups;
@@ -559,12 +616,12 @@ void launch(LinParams& p, int groups, int batch, hipStream_t st) {
         // 5.5 us, where K = 4096 gains 7.6 -> 7.0 and K = 6144 9.5 -> 8.8)
         if (groups * batch < kSplitRowsBelowGroups && (p.rows <= 8 || (p.rows <= 16 && PW >= 16))) {
             p.groups = 2 * groups;
-            hipLaunchKernelGGL((linear_rows_kernel<1, PW, kPlain, PW, 1, true, true>), dim3(p.groups, batch), dim3(kLinThreads), 0, st, p);
+            launch_folded<1, PW, kPlain, PW, true>(p, p.groups, batch, st);
             return;
         }
     }
     if (NC != 2 && PW > 0 && p.rows <= 8)  // (two tiles share the operand: nothing to gain)
-        hipLaunchKernelGGL((linear_rows_kernel<NC, CH, EPI, PW, 1, false, NC != 2 && (PW > 0)>), dim3(groups, batch), dim3(kLinThreads), 0, st, p);
+        launch_folded<NC, CH, EPI, PW, false>(p, groups, batch, st);
     else if (p.rows <= 16)
         hipLaunchKernelGGL((linear_rows_kernel<NC, CH, EPI, PW, 1>), dim3(groups, batch), dim3(kLinThreads), 0, st, p);
     else if (groups * batch < kSplitRowsBelowGroups)

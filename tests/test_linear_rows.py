@@ -249,7 +249,10 @@ def test_packed_orders_gpu():
 
 # Few rows, K known at compile time: eight columns per workgroup (few column groups), rows past the last one read as row 0.
 FEW = [(1, 32, 2048, "residual"), (8, 48, 2048, "plain"), (9, 16, 2048, "residual"), (3, 16, 4096, "residual"), (16, 32, 6144, "residual"),
-       (8, 2064, 2048, "plain"), (5, 24, 2048, "gate_up_norm"), (8, 16, 2048, "plain_norm")]
+       (8, 2064, 2048, "plain"), (5, 24, 2048, "gate_up_norm"), (8, 16, 2048, "plain_norm"),
+       # one, two, four and eight rows' operand folded into a load, a row fewer, and the last load's steps past the end (24 of 32)
+       (1, 16, 6144, "residual"), (2, 32, 6144, "residual"), (3, 16, 2048, "plain_norm"), (4, 32, 6144, "residual"), (7, 16, 6144, "residual"),
+       (1, 16, 2048, "plain_norm"), (2, 48, 2048, "plain_norm")]
 
 
 @pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
