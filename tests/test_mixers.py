@@ -28,6 +28,7 @@ DELTA_GPU = DELTA_SMALL + [
     (delta(8, 2, 128, 128, 4), (200, 65), ((64, 17, 119), (65,))), (delta(2, 1, 256, 96, 4), (40, 40), ((40,), (17, 23))),
     (delta(3, 1, 17, 130, 1), (30, 9), ((16, 14), (9,))), (delta(2, 2, 100, 256, 5), (21, 2), ((5, 16), (2,))),
     (delta(5, 5, 32, 512, 3), (19, 18), ((19,), (2, 16))), (delta(4, 2, 128, 64, 4), (333, 97), ((96, 64, 173), (97,))),
+    (delta(2, 1, 224, 64, 4), (7, 5), ((7,), (5,))),   # a step holds two channels per thread, the last one too
     (delta(2, 1, 256, 32, 2), (161, 70), ((100, 61), (70,))), (delta(6, 3, 32, 48, 4), (520, 520), ((255, 265), (256, 264))),
 ]
 # (sizes, prompt, portions, decoded tokens, ring capacity)
