@@ -39,7 +39,7 @@
 extern "C" {
 #endif
 
-#define TAH_DUO_ABI_VERSION 9
+#define TAH_DUO_ABI_VERSION 10
 
 enum {
     TAH_OK = 0,
