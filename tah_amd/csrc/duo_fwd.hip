@@ -55,10 +55,6 @@ constexpr int kStageOff = (kBoundsOff + 64 + 255) / 256 * 256;  // output stagin
 constexpr int kSmemBytes = kStageOff + 8 * 8192;
 // The 4-wave variant (two workgroups per compute unit) stages its output over the K / V rings, which are dead by then.
 constexpr int kSmemBytes4 = kStageOff;
-constexpr int kTeamBytes = kStageOff;  // kSplit: the second team's rings
-constexpr int kSmemBytesSplit = 2 * kTeamBytes;
-constexpr int kSplitTiles = 4;  // fewer key tiles stay with one team
-static_assert(4 * 8192 + 4 * 66 * kWave * 4 <= kSmemBytesSplit, "partial sums behind the output staging");
 static_assert(4 * 8192 <= kPosRing, "the 4-wave variant's output staging must fit the K / V rings");
 
 struct FwdStream {
@@ -91,13 +87,9 @@ enum class Mask { kNone, kIndex, kPos, kDense };
 // the two drift freely against each other (the dispatcher starts them at different times and their tile counts
 // differ), one workgroup's prologue, epilogue and hand-over to its successor run under the other's tile loop, and a
 // workgroup needs one barrier per tile.  Each workgroup stages its own K / V tiles (twice the copies per MFMA).
-// kSplit (W = 4): two teams of four waves share a workgroup and a query tile; each walks half of the tile's key tiles
-// with rings of its own, and the second team's sums are merged into the first's through LDS.  For launches that leave
-// compute units idle, whose time is the longest chain of key tiles.
-template <int G, bool kDense, int W, bool kSplit = false>
-__global__ __launch_bounds__(64 * W * (kSplit ? 2 : 1)) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(const FwdParams p) {
+template <int G, bool kDense, int W>
+__global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(const FwdParams p) {
     static_assert(W == 8 || W == 4, "8 or 4 waves");
-    static_assert(!kSplit || (W == 4 && !kDense), "teams of four waves");
     static_assert(W >= G, "a workgroup holds every query head of its kv head");
     constexpr int BM = 32 * (W / G);
     constexpr int kRowsPerWave = kBN / W;       // rows of a K / V tile each wave copies
@@ -105,8 +97,7 @@ __global__ __launch_bounds__(64 * W * (kSplit ? 2 : 1)) TAH_WAVES_PER_EU(2, 2) v
     HIP_DYNAMIC_SHARED(unsigned char, smem)
 
     const int tid = threadIdx.x;
-    const int team = kSplit ? __builtin_amdgcn_readfirstlane(tid / (kWave * W)) : 0;
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave) - W * team;  // wave-uniform: lives in a scalar register
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // wave-uniform: lives in a scalar register
     const int lane = tid % kWave;
     const int half = lane / 32;
     const int col = lane % 32;
@@ -175,7 +166,7 @@ __global__ __launch_bounds__(64 * W * (kSplit ? 2 : 1)) TAH_WAVES_PER_EU(2, 2) v
     const int wmax1 = wave_reduce_max(qlim1);
     const int wmin1 = wave_reduce_min(row_ok ? qlim1 : 0x7fffffff);
     int* bounds = reinterpret_cast<int*>(smem + kBoundsOff);
-    if (lane == 0) bounds[wave] = wmax1;  // (both teams have the same rows)
+    if (lane == 0) bounds[wave] = wmax1;
     __syncthreads();
     int tmax1 = -1;
 #pragma unroll
@@ -190,13 +181,8 @@ __global__ __launch_bounds__(64 * W * (kSplit ? 2 : 1)) TAH_WAVES_PER_EU(2, 2) v
     // (all wave-uniform: moved to scalar registers so that the tile loops are scalar loops)
     const int n1 = __builtin_amdgcn_readfirstlane(tmax1 >= 0 ? tmax1 / kBN + 1 : 0);
     const int n2 = second ? (lk2 + kBN - 1) / kBN : 0;
-    const int nall = n1 + n2;
-    // this team's tiles: [tile0, ntiles)
-    const int tile_mid = kSplit && nall >= kSplitTiles ? (nall + 1) / 2 : nall;
-    const int tile0 = team ? tile_mid : 0, ntiles = kSplit && !team ? tile_mid : nall;
-    const int n1_end = n1 < ntiles ? n1 : ntiles;
-    int n_active = __builtin_amdgcn_readfirstlane(wmax1 >= 0 ? wmax1 / kBN + 1 : 0);
-    n_active = n_active < ntiles ? n_active : ntiles;
+    const int ntiles = n1 + n2;
+    const int n_active = __builtin_amdgcn_readfirstlane(wmax1 >= 0 ? wmax1 / kBN + 1 : 0);
     int n_plain = __builtin_amdgcn_readfirstlane(wmin1 >= kBN - 1 ? (wmin1 - (kBN - 1)) / kBN + 1 : 0);
     n_plain = n_plain < n_active ? n_plain : n_active;
     if constexpr (kDense) n_plain = 0;  // the mask is read for every tile
@@ -235,7 +221,6 @@ __global__ __launch_bounds__(64 * W * (kSplit ? 2 : 1)) TAH_WAVES_PER_EU(2, 2) v
     uint32_t my_chunk[kPieces];
 #pragma unroll
     for (int i = 0; i < kPieces; ++i) my_chunk[i] = (uint32_t)(((lane & 15) ^ row_swizzle(my_lrow + 4 * i)) * 16);
-    unsigned char* const ring = smem + team * kTeamBytes;
     auto issue_rows = [&](const __bf16* src, int64_t rs, int base, int left, unsigned char* dst) {
         const __bf16* tile0 = src + (int64_t)base * rs;
         const int last = left - 1 - base;  // >= 0: a tile starts inside its segment
@@ -247,7 +232,7 @@ __global__ __launch_bounds__(64 * W * (kSplit ? 2 : 1)) TAH_WAVES_PER_EU(2, 2) v
         }
     };
     auto issue_k = [&](int it) {  // K tile `it` -> K ring, plus the positions of depth-1 keys
-        unsigned char* kt = ring + kKRing + (it % kStages) * kKBytes;
+        unsigned char* kt = smem + kKRing + (it % kStages) * kKBytes;
         if (it < n1) {
             issue_rows(k1p, p.s1.k_rs, it * kBN, left1, kt);
         } else {
@@ -256,12 +241,12 @@ __global__ __launch_bounds__(64 * W * (kSplit ? 2 : 1)) TAH_WAVES_PER_EU(2, 2) v
             if (wave == 0) {
                 int r = base + lane;
                 r = r < lk2 ? r : lk2 - 1;
-                async_copy_4B(pos2p + r, ring + kPosRing + (it % kPosSlots) * (kBN * 4));
+                async_copy_4B(pos2p + r, smem + kPosRing + (it % kPosSlots) * (kBN * 4));
             }
         }
     };
     auto issue_v = [&](int it) {
-        unsigned char* vt = ring + kVRing + (it % kStages) * kVBytes;
+        unsigned char* vt = smem + kVRing + (it % kStages) * kVBytes;
         if (it < n1) issue_rows(v1p, p.s1.v_rs, it * kBN, left1, vt);
         else issue_rows(v2p, p.s2.v_rs, (it - n1) * kBN, left2, vt);
     };
@@ -292,7 +277,7 @@ __global__ __launch_bounds__(64 * W * (kSplit ? 2 : 1)) TAH_WAVES_PER_EU(2, 2) v
 
     // ---- matrix phase pieces -------------------------------------------------------------------
     auto qk = [&](int it) __attribute__((always_inline)) {  // S^T = K(it) Q^T
-        const unsigned char* kt = ring + kKRing + (it % kStages) * kKBytes;
+        const unsigned char* kt = smem + kKRing + (it % kStages) * kKBytes;
         const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt)
@@ -304,7 +289,7 @@ __global__ __launch_bounds__(64 * W * (kSplit ? 2 : 1)) TAH_WAVES_PER_EU(2, 2) v
                 sacc[mt] = mfma32(*reinterpret_cast<const bf16x8*>(kt + koff[s] + mt * 8192), qf[s], sacc[mt]);
     };
     auto pv = [&](int it) __attribute__((always_inline)) {  // O^T (128 d x 32 queries) += V(it)^T P^T
-        const unsigned char* vt = ring + kVRing + (it % kStages) * kVBytes;
+        const unsigned char* vt = smem + kVRing + (it % kStages) * kVBytes;
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
 #pragma unroll
@@ -366,7 +351,7 @@ __global__ __launch_bounds__(64 * W * (kSplit ? 2 : 1)) TAH_WAVES_PER_EU(2, 2) v
                     sacc[mt][r] = kk <= qlim1 ? sacc[mt][r] + mv * p.inv_scale : kNegInf;
                 }
         } else if constexpr (kMask == Mask::kPos) {
-            const int* kpos = reinterpret_cast<const int*>(ring + kPosRing + (it % kPosSlots) * (kBN * 4));
+            const int* kpos = reinterpret_cast<const int*>(smem + kPosRing + (it % kPosSlots) * (kBN * 4));
             const int nleft = lk2 - (it - n1) * kBN;  // keys of this tile that exist
 #pragma unroll
             for (int mt = 0; mt < 2; ++mt)
@@ -486,14 +471,14 @@ __global__ __launch_bounds__(64 * W * (kSplit ? 2 : 1)) TAH_WAVES_PER_EU(2, 2) v
             else if constexpr (kLate) step_late(t, tag, qk_tag);
             else step_early(t, tag, qk_tag);
         };
-        int t = tile0;
+        int t = 0;
         if constexpr (kLate) TAH_PHASE_BARRIER();  // before h = 1
-        if (next_active(tile0 - 1)) qk(tile0);
+        if (next_active(-1)) qk(0);
         for (; t < plain_q; ++t) step(t, PlainTag{}, WithQk{});
         for (; t < n_plain; ++t) step(t, PlainTag{}, NoQk{});
         for (; t < act_q; ++t) step(t, IndexTag{}, WithQk{});
         for (; t < n_active; ++t) step(t, IndexTag{}, NoQk{});
-        for (; t < n1_end; ++t) {
+        for (; t < n1; ++t) {
             if constexpr (W == 4) idle_single(t);
             else if constexpr (kLate) idle_late(t);
             else idle_early(t);
@@ -503,46 +488,17 @@ __global__ __launch_bounds__(64 * W * (kSplit ? 2 : 1)) TAH_WAVES_PER_EU(2, 2) v
         if constexpr (W == 8 && !kLate) TAH_PHASE_BARRIER();  // before h = 2*ntiles + 1
     };
 
-    if (tile0 < ntiles) issue_k(tile0);
+    if (ntiles > 0) issue_k(0);
     TAH_WAIT_VMEM();  // K(0) and the Q fragments are in: no ordinary load stays pending across the tile loop
-    if (nall > 0) {
+    if (ntiles > 0) {
         TAH_PHASE_BARRIER();  // before h = 0
-        issue(tile0);
+        issue(0);
         if (W == 4 || late_set(wave) == 0) run(std::false_type{});
         else run(std::true_type{});
-        if constexpr (kSplit)  // as many barriers as the team with more tiles (the first one)
-            for (int t = ntiles - tile0; t < tile_mid; ++t) TAH_PHASE_BARRIER();
     }
     if constexpr (W == 4) {  // the output staging below overlies the rings: every wave must be done reading them
         TAH_WAIT_VMEM();
         TAH_PHASE_BARRIER();
-    }
-    if constexpr (kSplit) {
-        if (tile_mid < nall) {  // (uniform per workgroup)
-            // one float per lane and register, behind the first team's output staging
-            float* const part = reinterpret_cast<float*>(smem + 4 * 8192) + wave * (66 * kWave) + lane;
-            if (team) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) part[(16 * i + r) * kWave] = oacc[i][r];
-                part[64 * kWave] = m_run;
-                part[65 * kWave] = l_run;
-            }
-            TAH_PHASE_BARRIER();
-            if (!team) {
-                const float m2 = part[64 * kWave], l2 = part[65 * kWave];
-                const float m_new = fmaxf(m_run, m2), m_use = m_new == kNegInf ? 0.f : m_new;
-                const float a1 = fast_exp2((m_run - m_use) * c), a2 = fast_exp2((m2 - m_use) * c);
-                m_run = m_new;
-                l_run = l_run * a1 + l2 * a2;
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) oacc[i][r] = oacc[i][r] * a1 + part[(16 * i + r) * kWave] * a2;
-            }
-        }
-        if (team) return;
     }
 #undef TAH_PHASE_BARRIER
 
@@ -619,13 +575,6 @@ int check_stream(const tah_duo_stream& s, bool second) {
     return TAH_OK;
 }
 
-// Up to this many 4-wave workgroups (two to a compute unit: one round of the chip) a launch takes as long as its longest
-// chain of key tiles, 1.6 us a tile, and two teams per workgroup halve the chain at 2.3 us for a tile of each: 16 / 8
-// heads, one sequence of 333 tokens 17.3 -> 16.5 us, 900 31.7 -> 26.1, 2048 55.4 -> 46.0, 3800 102 -> 86; depth-1
-// queries alone (10 % of 1024 to 3210 tokens) 87 -> 68.  Beyond it the second round costs more: 8 x 200 to 512 tokens
-// (576 workgroups) 23.3 -> 33.5.
-constexpr int kSplitBelow = 512;
-
 template <int G, bool kDense>
 int launch_fwd(const FwdParams& p, hipStream_t stream) {
     constexpr int BM = 32 * (8 / G);
@@ -635,13 +584,6 @@ int launch_fwd(const FwdParams& p, hipStream_t stream) {
     // duo-causal calls with up to four query heads per kv head: 4-wave workgroups, two per compute unit (same results
     // to the bit; measured 0-5 % faster than the 8-wave form, most with several short documents)
     if constexpr (!kDense && G <= 4) {
-        if (2 * tiles * p.hkv <= kSplitBelow && (int64_t)p.s1.total_k + p.s2.total_k >= kSplitTiles * kBN) {
-            if (hipFuncSetAttribute(reinterpret_cast<const void*>(&duo_fwd_kernel<G, kDense, 4, true>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytesSplit) != hipSuccess)
-                return TAH_E_LAUNCH;
-            hipLaunchKernelGGL((duo_fwd_kernel<G, kDense, 4, true>), dim3(p.hkv, 2 * tiles), dim3(512), kSmemBytesSplit, stream, p);
-            return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
-        }
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(&duo_fwd_kernel<G, kDense, 4>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes4) != hipSuccess)
             return TAH_E_LAUNCH;

@@ -47,6 +47,17 @@ def make_varlen_case(seed, seqlens, p_hard, Hq=16, Hkv=8, D=128, dtype=torch.flo
     )
 
 
+def first_sequence(case):
+    """A varlen case without its sequences behind the first one."""
+    n = {s: int(case["cu_" + s][1]) for s in ("q1", "k1", "q2", "k2")}
+    out = dict(case)
+    for name, s in (("q1", "q1"), ("k1", "k1"), ("v1", "k1"), ("q2", "q2"), ("k2", "k2"), ("v2", "k2"), ("pos_q2", "q2"), ("pos_k2", "k2")):
+        out[name] = case[name][:n[s]]
+    for s in n:
+        out["cu_" + s] = case["cu_" + s][:2]
+    return out
+
+
 def add_score_drift(case, nats_per_key):
     """Makes every depth-0 score grow with the key index by about `nats_per_key` (on top of the random
     part): all queries get a common direction u added, key j gets j * t * u.  A running-maximum softmax

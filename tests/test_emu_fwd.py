@@ -63,6 +63,22 @@ def test_fwd_kernel_moving_softmax_reference(nats_per_key):
     _check(dev, got)
 
 
+@pytest.mark.parametrize("rows,p", [(258, 0.1)])
+def test_fwd_of_a_head_does_not_depend_on_its_group(rows, p):
+    """Eight query heads of one kv head (8-wave workgroups) and the same heads four at a time (4-wave workgroups): the same
+    bits.  The probabilities are rounded to bf16 under a reference that moves along the keys, so this holds only if a
+    query's keys are always taken one after another from the first."""
+    from tah_amd import ops
+    eight = _to_dev(make_varlen_case(61, [rows], p, Hq=8, Hkv=1, D=128))
+    with emu_util.emulated():
+        want = ops.duo_fwd_varlen(*varlen_args(eight))
+        for h in (0, 4):
+            four = dict(eight, q1=eight["q1"][:, h:h + 4].contiguous(), q2=eight["q2"][:, h:h + 4].contiguous())
+            o1, lse1, o2, lse2 = ops.duo_fwd_varlen(*varlen_args(four))
+            assert torch.equal(o1, want[0][:, h:h + 4]) and torch.equal(lse1, want[1][h:h + 4])
+            assert torch.equal(o2, want[2][:, h:h + 4]) and torch.equal(lse2, want[3][h:h + 4])
+
+
 def test_fwd_kernel_cache_prefix_and_strided_views():
     from tah_amd import ops
     dev = _to_dev(make_varlen_case(7, [5, 40], 0.5, Hq=2, Hkv=1, D=128, seqlens_k=[90, 40], extra_k2=70))
@@ -128,9 +144,8 @@ def test_rows_copy_bit_exact(dtype, inner):
 
 
 @pytest.mark.parametrize("hq,hkv,seqlens,p,drift", [(2, 1, [330], 0.3, 0.0), (4, 1, [193, 80], 1.0, 0.25)])
-def test_fwd_kernel_two_teams_per_tile_on_cpu_shim(hq, hkv, seqlens, p, drift):
-    """Small launches with at least four key tiles: two teams share a query tile's keys (also where the second team's exponent
-    reference is far from the first's)."""
+def test_fwd_kernel_chains_of_key_tiles_on_cpu_shim(hq, hkv, seqlens, p, drift):
+    """Small launches with at least four key tiles (also where the exponent reference moves far along them)."""
     from tah_amd import ops
     case = make_varlen_case(33, seqlens, p, Hq=hq, Hkv=hkv, D=128)
     dev = _to_dev(add_score_drift(case, drift) if drift else case)
