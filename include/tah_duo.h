@@ -428,13 +428,15 @@ int tah_sample_rows(const tah_sample_rows_args* args, tah_stream_t stream);
  * slot and call).  For calls tah_duo_decode_step_supported() accepts (256
  * or more (query, kv head) pairs, slabs of at most 4096 rows, one or two query heads per kv head: cases
  * tah_duo_decode runs without split-K), and with a workspace for fewer pairs or longer slabs: dec->workspace of at least
- * tah_duo_decode_step_workspace_bytes() bytes, 16-byte aligned, zero before its first call and then left to these calls (it
- * holds counters that every call returns to zero), one per sequence of calls that may overlap another (0: sizes no
- * workspace helps).  Others return TAH_E_SHAPE and the caller makes the two calls.  append_depth: NULL,
+ * tah_duo_decode_step_workspace_bytes() bytes, 16-byte aligned, its first TAH_DUO_STEP_COUNTER_BYTES zero before its first
+ * call and then left to these calls (they hold counters that every call returns to zero; what lies behind needs no value, so
+ * one workspace, of the largest size, serves calls of different sizes in any order), one per sequence of calls that may
+ * overlap another (0: sizes no workspace helps).  Others return TAH_E_SHAPE and the caller makes the two calls.  append_depth: NULL,
  * or int32 [rows], 0 / 1 per row: the segment (dec->c1 / dec->c2) that row's K and V go to, for a batch whose rows are at
  * different latent iterations (append_at[i] then counts the rows of that segment, and prep->cache only has to be one of
  * the two).  Replaces, with
  * tah_qk_prep's and tah_duo_decode's lists, one more launch per layer and latent iteration. */
+#define TAH_DUO_STEP_COUNTER_BYTES 65536
 int tah_duo_decode_step_supported(int32_t nq, int32_t hq, int32_t hkv, int32_t capacity1);
 size_t tah_duo_decode_step_workspace_bytes(int32_t nq, int32_t hq, int32_t hkv, int32_t capacity1, int32_t capacity2);
 int tah_duo_decode_step(const tah_qk_prep_args* prep, const tah_duo_decode_args* dec, const int32_t* append_at,

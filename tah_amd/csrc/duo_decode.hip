@@ -1346,7 +1346,9 @@ int launch_step(const StepParams& sp, hipStream_t st) {
         hipLaunchKernelGGL((duo_decode_step_kernel<G, false>), dim3(sp.dec.nq, sp.dec.hkv), dim3(kWholeThreads), kRedBytes, st, sp);
     return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
 }
-size_t step_counter_bytes(int nq, int hkv) { return ((size_t)nq * hkv * sizeof(int32_t) + 255) / 256 * 256; }  // then the partials
+// The partials lie behind room for the counters of as many pairs as share rows at most, wherever a call's own counters end: a
+// counter's place then never holds what a call of another size left.  More pairs (64 to a compute unit) have a workgroup each.
+constexpr long kStepMaxPairs = TAH_DUO_STEP_COUNTER_BYTES / sizeof(int32_t);
 }  // namespace
 }  // namespace tah
 
@@ -1355,7 +1357,8 @@ extern "C" size_t tah_duo_decode_step_workspace_bytes(int32_t nq, int32_t hq, in
     if (nq <= 0 || hq <= 0 || hkv <= 0 || hq % hkv || capacity1 <= 0 || capacity2 < 0) return 0;
     const int g = hq / hkv;
     if ((g != 1 && g != 2) || g > kStepMaxGroup || nq > 65535 || hkv > 65535) return 0;
-    return step_counter_bytes(nq, hkv) + (size_t)nq * hq * step_splits_of((long)capacity1 + capacity2, step_fill(nq, hkv)) * kPart * sizeof(float);
+    if ((long)nq * hkv > kStepMaxPairs) return TAH_DUO_STEP_COUNTER_BYTES;
+    return TAH_DUO_STEP_COUNTER_BYTES + (size_t)nq * hq * step_splits_of((long)capacity1 + capacity2, step_fill(nq, hkv)) * kPart * sizeof(float);
 }
 
 extern "C" int tah_duo_decode_step_supported(int32_t nq, int32_t hq, int32_t hkv, int32_t capacity1) {
@@ -1403,10 +1406,12 @@ extern "C" int tah_duo_decode_step(const tah_qk_prep_args* prep, const tah_duo_d
         if (!need || !dec->workspace) return TAH_E_SHAPE;
         if (!aligned16(dec->workspace)) return TAH_E_ALIGN;
         if (dec->workspace_bytes < need) return TAH_E_WORKSPACE;
-        sp.arrived = static_cast<int32_t*>(dec->workspace);
-        sp.part = reinterpret_cast<float*>(static_cast<unsigned char*>(dec->workspace) + step_counter_bytes(dec->nq, dec->hkv));
-        sp.fill = step_fill(dec->nq, dec->hkv);
-        sp.nsplit = step_splits_of((long)dec->c1.capacity + cap2, sp.fill);
+        if ((long)dec->nq * dec->hkv <= kStepMaxPairs) {
+            sp.arrived = static_cast<int32_t*>(dec->workspace);
+            sp.part = reinterpret_cast<float*>(static_cast<unsigned char*>(dec->workspace) + TAH_DUO_STEP_COUNTER_BYTES);
+            sp.fill = step_fill(dec->nq, dec->hkv);
+            sp.nsplit = step_splits_of((long)dec->c1.capacity + cap2, sp.fill);
+        }
     }
     if (!append_at) return TAH_E_NULL;
     if (prep->cache.k == dec->c1.k) sp.append_second = 0;

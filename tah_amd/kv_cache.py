@@ -158,7 +158,8 @@ def decode_step(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_weight: tor
 
 def decode_step_workspace(nq: int, hq: int, hkv: int, capacity1: int, capacity2: int, device) -> Optional[torch.Tensor]:
     """The workspace :func:`decode_step` wants for a batch or slabs that :func:`decode_step_supported` does not take, or None for
-    sizes no workspace helps.  It is zero, and every call leaves its counters at zero."""
+    sizes no workspace helps.  It is zero, and every call leaves its counters at zero; one of the largest size serves
+    calls of all sizes, in any order."""
     n = int(_call("duo_decode_step_workspace_bytes", int(nq), int(hq), int(hkv), int(capacity1), int(capacity2)))
     return torch.zeros(n, dtype=torch.uint8, device=device) if n else None
 

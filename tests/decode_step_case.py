@@ -19,18 +19,28 @@ def _slabs(B, cap, hkv, lens, with_pos, g, dev):
 
 
 def _workspace(wanted, c1, c2, B, hq, hkv):
-    """What the call is handed as ``workspace=``: nothing, or for batches and slabs that the call takes only with one, that."""
+    """What the call is handed as ``workspace=``: nothing, or for batches and slabs that the call takes only with one, that.
+    ``wanted``: whether, or a workspace that other calls have used, or by how many bytes more than needed."""
     from tah_amd import kv_cache
-    if not wanted:
+    if wanted is False:
         return None
     assert not kv_cache.decode_step_supported(B, hq, hkv, c1.capacity)
     ws = kv_cache.decode_step_workspace(B, hq, hkv, c1.capacity, c2.capacity, c1.k.device)
     assert ws is not None
+    if isinstance(wanted, int) and wanted is not True:
+        return torch.zeros(ws.numel() + wanted, dtype=torch.uint8, device=ws.device)
+    if wanted is not True:
+        assert wanted.numel() >= ws.numel()
+        return wanted
     return ws
 
 
-def _counters_are_back_at_zero(ws, B, hkv):
-    return ws is None or int(ws[:4 * B * hkv].view(torch.int32).abs().max()) == 0
+COUNTER_BYTES = 65536  # TAH_DUO_STEP_COUNTER_BYTES
+
+
+def _counters_are_back_at_zero(ws):
+    """All that calls of any size may count in, not only this one's."""
+    return ws is None or int(ws[:COUNTER_BYTES].view(torch.int32).abs().max()) == 0
 
 
 def run(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2=64, full_slab=False, workspace=False):
@@ -79,7 +89,7 @@ def run(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2=64, f
             if fused:
                 o = kv_cache.decode_step(q, k, v, qw, kw, cos, sin, 1e-6, append_at=tgt.len.clone(), q_slot=rows, q_pos=q_pos,
                                          c1=a1, c2=a2, scale=scale, q_depth=q_depth, out_packed=packed, workspace=ws, **common)
-                assert _counters_are_back_at_zero(ws, B, hkv)
+                assert _counters_are_back_at_zero(ws)
             else:
                 qo, _ = kv_cache.qk_norm_rope(q, k, qw, kw, cos, sin, 1e-6, v=v, one_row_per_seq=True, **common)
                 o = kv_cache.decode(qo, rows, q_pos, a1, a2, scale=scale, q_depth=q_depth, out_packed=packed)
@@ -154,9 +164,10 @@ def run_mixed(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2
     oa = kv_cache.decode(qo, rows, q_pos, a1, a2, scale=scale, q_depth=q_depth)
     b1, b2 = copy.deepcopy(c1), copy.deepcopy(c2)
     append_at = torch.where(depth, b2.len, b1.len)
+    ws = _workspace(workspace, b1, b2, B, hq, hkv)
     ob = kv_cache.decode_step(q, k, v, qw, kw, cos, sin, 1e-6, cache=b2, append_at=append_at, append_depth=q_depth, q_slot=rows,
-                              q_pos=q_pos, c1=b1, c2=b2, scale=scale, slot_of=slot_all, pos_new=pos, q_depth=q_depth,
-                              workspace=_workspace(workspace, b1, b2, B, hq, hkv), **common)
+                              q_pos=q_pos, c1=b1, c2=b2, scale=scale, slot_of=slot_all, pos_new=pos, q_depth=q_depth, workspace=ws, **common)
+    assert _counters_are_back_at_zero(ws)
     assert torch.allclose(oa.float(), ob.float(), rtol=2.0 ** -7, atol=2.0 ** -12) and (oa != ob).float().mean() < 1e-3
     for sa, sb in ((a1, b1), (a2, b2)):
         assert torch.equal(sa.k, sb.k) and torch.equal(sa.v, sb.v) and torch.equal(sa.len, sb.len) and int(sa.overflow) == int(sb.overflow) == 0

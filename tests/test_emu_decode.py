@@ -104,9 +104,12 @@ def test_fused_decode_step_with_a_pairs_rows_shared_by_workgroups_on_cpu_shim():
     from tests import decode_step_case
     from tah_amd import TahDuoError, kv_cache
     with emu_util.emulated():
-        decode_step_case.run("cpu", B=3, hq=2, hkv=1, seed=8, max_len=1400, cap1=1500, cap2=700, workspace=True)
-        decode_step_case.run("cpu", B=2, hq=1, hkv=1, seed=9, max_len=600, cap2=300, full_slab=True, workspace=True)
-        decode_step_case.run_mixed("cpu", B=4, hq=2, hkv=1, seed=10, max_len=1400, cap1=1500, cap2=700, workspace=True)
+        ws = kv_cache.decode_step_workspace(3, 2, 1, 1500, 700, "cpu")  # the largest of three sizes serves all
+        decode_step_case.run("cpu", B=2, hq=1, hkv=1, seed=9, max_len=600, cap2=300, full_slab=True, workspace=ws)
+        decode_step_case.run("cpu", B=3, hq=2, hkv=1, seed=8, max_len=1400, cap1=1500, cap2=700, workspace=ws)
+        decode_step_case.run_mixed("cpu", B=4, hq=2, hkv=1, seed=10, max_len=1400, cap1=1500, cap2=700, workspace=ws)
+        with pytest.raises(TahDuoError):
+            decode_step_case.run("cpu", B=3, hq=2, hkv=1, seed=8, workspace=-16)
         with pytest.raises(TahDuoError):
             decode_step_case.run("cpu", B=3, hq=2, hkv=1, seed=8)
         assert kv_cache.decode_step_workspace(3, 4, 1, 1500, 700, "cpu") is None  # four query heads per kv head

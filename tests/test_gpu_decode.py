@@ -142,3 +142,16 @@ def test_fused_decode_step_with_a_workspace_equals_prep_then_decode(B, hq, hkv, 
     print(f"fused decode step with a workspace B={B} hq={hq} hkv={hkv} cap={cap1}", flush=True)
     for case in (decode_step_case.run, decode_step_case.run_mixed):
         case("cuda", B=B, hq=hq, hkv=hkv, seed=B + cap1, max_len=cap1 - 1, hidden=2048, cap1=cap1, cap2=max(64, cap1 // 4), workspace=True)
+
+
+def test_fused_decode_steps_of_several_sizes_share_a_workspace():
+    """Few pairs, then more, then few: what a call leaves behind its counters must not be taken for another call's counters."""
+    from tests import decode_step_case
+    from tah_amd import kv_cache
+    sizes = [(2, 16, 8, 700), (16, 16, 8, 900), (3, 2, 1, 513), (31, 16, 8, 1024), (2, 4, 2, 4500), (2, 16, 8, 700)]
+    needs = [kv_cache.decode_step_workspace(B, hq, hkv, cap, cap // 4, "cuda") for B, hq, hkv, cap in sizes]
+    ws = max(needs, key=lambda t: t.numel())
+    for B, hq, hkv, cap in sizes:
+        print(f"shared workspace B={B} hq={hq} hkv={hkv} cap={cap}", flush=True)
+        for case in (decode_step_case.run, decode_step_case.run_mixed):
+            case("cuda", B=B, hq=hq, hkv=hkv, seed=B + cap, max_len=cap - 1, hidden=2048, cap1=cap, cap2=cap // 4, workspace=ws)
