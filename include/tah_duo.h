@@ -401,7 +401,7 @@ typedef struct tah_sample_rows_args {
     float min_p;               /* in [0, 1]; 0: no filter */
     const int32_t* uniform_step; /* optional int32 [rows]: row r's number is uniforms[uniform_step[r]][r] (an index outside the
                                 * table is moved to its nearest end), for batches whose rows are at tokens of different number */
-    int32_t n_uniform_steps;
+    int32_t n_uniform_steps;   /* with uniform_step: at least 1 (TAH_E_SHAPE otherwise) */
 } tah_sample_rows_args;
 
 /* One token per row by temperature sampling with the min_p and top_p filters, in one launch and without a sort over

@@ -556,9 +556,11 @@ extern "C" int tah_sample_rows(const tah_sample_rows_args* a, tah_stream_t strea
     if (a->rows == 0) return TAH_OK;
     if (!a->logits || (!a->tokens && !a->probs) || (a->tokens && !a->uniforms)) return TAH_E_NULL;
     if (a->add_prev && !a->logits_prev) return TAH_E_NULL;
+    if (a->tokens && a->uniform_step && a->n_uniform_steps < 1) return TAH_E_SHAPE;  // (no row to move an index to)
     if ((reinterpret_cast<uintptr_t>(a->logits) & 1) || (reinterpret_cast<uintptr_t>(a->logits_prev) & 1) ||
         (reinterpret_cast<uintptr_t>(a->tokens) & 7) || (reinterpret_cast<uintptr_t>(a->probs) & 3) ||
-        (reinterpret_cast<uintptr_t>(a->uniforms) & 3) || (reinterpret_cast<uintptr_t>(a->add_prev) & 3))
+        (reinterpret_cast<uintptr_t>(a->uniforms) & 3) || (reinterpret_cast<uintptr_t>(a->add_prev) & 3) ||
+        (reinterpret_cast<uintptr_t>(a->uniform_step) & 3))
         return TAH_E_ALIGN;
     if (a->probs && a->probs_row_stride < a->vocab) return TAH_E_SHAPE;
     SampleParams p;

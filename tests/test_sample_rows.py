@@ -110,6 +110,35 @@ def test_sample_rows_row_enable_and_refusals_on_cpu_shim():
     assert out[1] == -5 and out[0] == full[0] and out[2] == full[2]
 
 
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_sample_rows_numbers_from_a_table_on_cpu_shim():
+    """Rows at different steps of a table of numbers draw as with their own numbers handed over; an index outside the table is
+    moved to its nearest end; a table without a row, or a misaligned index array, is refused."""
+    import ctypes as C
+    from tah_amd import _capi, ops
+    x = torch.from_numpy(make_rows(10, 5, 800, "flat")).to(torch.bfloat16)
+    table = torch.from_numpy(np.random.default_rng(110).random((4, 5)).astype(np.float32))
+    step = torch.tensor([2, -3, 0, 7, 3], dtype=torch.int32)
+    rows = torch.arange(5)
+    own = table[step.long().clamp(0, 3), rows].contiguous()
+    with emu_util.emulated() as lib:
+        got = ops.sample_rows(x, table, 0.7, uniform_step=step)
+        assert torch.equal(got, ops.sample_rows(x, own, 0.7))
+        assert not torch.equal(got, ops.sample_rows(x, table[0].contiguous(), 0.7))  # (the numbers do decide)
+        tokens = torch.zeros(5, dtype=torch.int64)
+        a = _capi.SampleRowsArgs()
+        a.logits, a.logits_row_stride, a.rows, a.vocab = x.data_ptr(), 800, 5, 800
+        a.temperature, a.top_p = 0.7, 1.0
+        a.uniforms = table[2].data_ptr()  # (in the middle: a row in front of it exists)
+        a.uniform_step, a.tokens = step.data_ptr(), tokens.data_ptr()
+        for n in (0, -1):
+            a.n_uniform_steps = n
+            assert lib.tah_sample_rows(C.byref(a), None) == -2  # TAH_E_SHAPE
+        a.n_uniform_steps = 1
+        a.uniform_step = step.data_ptr() + 2
+        assert lib.tah_sample_rows(C.byref(a), None) == -3      # TAH_E_ALIGN
+
+
 GPU_CASES = [
     (20, 4, 151936, "peaked", 0.6, 0.95, 0.0, False),
     (21, 4, 151936, "flat", 0.6, 0.95, 0.0, True),
