@@ -1003,7 +1003,10 @@ __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const St
             pa[t] = device_load(at + d);
             pm[t] = device_load(at + kD);
             pl[t] = device_load(at + kD + 1);
-            if (j >= nact) pm[t] = kNegInf;
+            if (j >= nact) {  // (0 as well, not only weighed by 0: part 0 may hold an infinity)
+                pm[t] = kNegInf;
+                pa[t] = pl[t] = 0.f;
+            }
         }
         float mx = kNegInf, a = 0.f, l = 0.f;
 #pragma unroll

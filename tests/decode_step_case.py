@@ -43,8 +43,9 @@ def _counters_are_back_at_zero(ws):
     return ws is None or int(ws[:COUNTER_BYTES].view(torch.int32).abs().max()) == 0
 
 
-def run(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2=64, full_slab=False, workspace=False):
-    """full_slab: the depth-0 slabs hold exactly the longest sequence, so that sequence's new row does not fit: both
+def run(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2=64, full_slab=False, workspace=False, infinite=False):
+    """infinite: one cached value of the last sequence is +inf, and so its output there.
+    full_slab: the depth-0 slabs hold exactly the longest sequence, so that sequence's new row does not fit: both
     paths have to raise the overflow flag, leave slab and length alone and attend over what is cached."""
     from tah_amd import kv_cache
     g = torch.Generator().manual_seed(seed)
@@ -55,6 +56,8 @@ def run(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2=64, f
     lens2 = [int(torch.randint(0, min(l, cap2 - 1) + 1, (1,), generator=g)) for l in lens1]
     c1 = _slabs(B, cap1, hkv, lens1, False, g, dev)
     c2 = _slabs(B, cap2, hkv, lens2, True, g, dev)
+    if infinite:
+        c1.v[B - 1, 0, 1, 7] = float("inf")
     for b in range(B):  # depth-1 rows sit at increasing positions below the sequence's length
         c2.pos[b, :lens2[b]] = torch.sort(torch.randperm(lens1[b], generator=g)[:lens2[b]]).values.to(torch.int32)
     rn = lambda *s: torch.randn(*s, generator=g).to(BF).to(dev)
@@ -94,6 +97,9 @@ def run(dev, *, B, hq, hkv, seed=0, max_len=90, hidden=256, cap1=128, cap2=64, f
                 qo, _ = kv_cache.qk_norm_rope(q, k, qw, kw, cos, sin, 1e-6, v=v, one_row_per_seq=True, **common)
                 o = kv_cache.decode(qo, rows, q_pos, a1, a2, scale=scale, q_depth=q_depth, out_packed=packed)
             out.append((o, packed, a1, a2))
+            if infinite and (depth == 0 or bool(hard[B - 1])):
+                seen = o[B - 1].float()
+                assert bool((seen[:hq // hkv, 7] == float("inf")).all()) and not bool(seen.isnan().any())
         (oa, pa, a1, a2), (ob, pb, b1, b2) = out
         assert torch.allclose(oa.float(), ob.float(), rtol=2.0 ** -7, atol=2.0 ** -12), f"depth {depth}: outputs differ"
         assert (oa != ob).float().mean() < 1e-3, f"depth {depth}: more than a rare last bit differs"
