@@ -821,7 +821,8 @@ class TaHDecodeEngine(DecodeEngine):
                  use_graph: bool = True, check_every: int = 64, continuous: Optional[bool] = None, **filters):
         """As in :class:`DecodeEngine`.  ``continuous`` (default: whenever the engine can): rows do not wait for each other's second latent iterations
         -- see :meth:`_generate_ticks`.  Greedy decoding gives the same tokens per row either way; sampled tokens come from
-        the same per-row distributions but from other random draws (a tick draws for every row, a step once per token)."""
+        the same per-row distributions but from other random draws (a tick draws for every row, a step once per token).
+        ``check_every`` counts ticks there."""
         self._check_room(max_new_tokens)
         dev = self.device
         greedy_fused = temperature <= 0.0 and self.fused_greedy and self.cfg.vocab % 8 == 0
@@ -833,7 +834,7 @@ class TaHDecodeEngine(DecodeEngine):
             if not can_tick:
                 raise TahDuoError("continuous generation needs the fused attention and glue launches "
                                   "(at most 32 rows, one or two query heads per kv head)")
-            return self._generate_ticks(first_logits, max_new_tokens, eos, use_graph and dev.type == "cuda",
+            return self._generate_ticks(first_logits, max_new_tokens, eos, use_graph and dev.type == "cuda", check_every=check_every,
                                         temperature=temperature, **filters)
         return super().generate(first_logits, max_new_tokens, temperature=temperature, eos=eos, use_graph=use_graph,
                                 check_every=check_every, **filters)
@@ -885,7 +886,8 @@ class TaHDecodeEngine(DecodeEngine):
                         hard_len=self.hard_len, n_hard=self.n_hard, n_steps=self.n_steps, chosen=chosen,
                         workspace=self.greedy_workspace)
 
-    DRAW_AHEAD = 64  # ticks whose uniforms are drawn at a time; with an end-of-sequence token also how often the host looks
+    DRAW_AHEAD = 64  # ticks whose uniforms are drawn at a time
+    LAST_TICKS = 8   # how often the host looks once the fastest possible row could be done
 
     def _launch_switches(self):
         return super()._launch_switches() + (self.use_fused_glue, self.static_scratch, self.measure_without_attention, id(self.decider))
@@ -914,14 +916,15 @@ class TaHDecodeEngine(DecodeEngine):
         self._tick_graphs, self._tick_key = graphs, key
         return graphs
 
-    def _generate_ticks(self, first_logits: torch.Tensor, max_new_tokens: int, eos: int, use_graph: bool, check_every: int = 8,
+    def _generate_ticks(self, first_logits: torch.Tensor, max_new_tokens: int, eos: int, use_graph: bool, check_every: int = 64,
                         temperature: float = 0.0, **filters):
         """Generation in ticks.  The reference's loop (tah_model.py:580-706 inside utils.py:228-262) keeps the
         batch in step: every token costs the batch a first iteration and, if any row calls it hard, a second one --
         here a full pass over the weights for the one row in twelve that needs it.  Rows do not interact, so each row
         can run its own sequence of passes: a tick is one pass in which every row does the next iteration it needs.  A
         token costs its row 1 + [hard] ticks instead of 2, and the tokens are the ones the step-wise loop produces.
-        The host looks every ``check_every`` ticks, once the fastest possible row could be done, whether all are."""
+        With ``eos`` the host looks every ``check_every`` ticks whether all rows are done, and in any case every
+        ``LAST_TICKS`` ticks once the fastest possible row could be."""
         B = self.B
         self.out_tokens.zero_()
         self.out_len.zero_()
@@ -949,12 +952,13 @@ class TaHDecodeEngine(DecodeEngine):
             else:
                 self._tick(ticks % 2, eos, limit, temperature, **filters)
             ticks += 1
-            if ticks >= n_min and (ticks - n_min) % check_every == 0 and bool(self.finished.all()):
+            if ticks >= n_min and (ticks - n_min) % self.LAST_TICKS == 0 and bool(self.finished.all()):
                 break
-            if eos >= 0 and ticks % self.DRAW_AHEAD == 0 and bool(self.finished.all()):
-                steps = min(steps, max(1, -(-int(self.out_len.max()) // self.DRAW_AHEAD)) * self.DRAW_AHEAD)
+            if eos >= 0 and ticks % check_every == 0 and bool(self.finished.all()):
+                every = abs(check_every)
+                steps = min(steps, max(1, -(-int(self.out_len.max()) // every)) * every)
                 break
-            if ticks > 2 * n_min + check_every:
+            if ticks > 2 * n_min + self.LAST_TICKS:
                 raise TahDuoError("generation did not finish within two passes per token")
         self.ticks = ticks
         self.finished &= self.out_len < limit  # rows stopped by the limit have not ended

@@ -477,6 +477,22 @@ def test_ticks_end_soon_after_every_row_has_ended_gpu():
     assert eng.ticks == 64 and n <= 5 and bool(eng.finished.all()) and int(toks[0, n:].abs().max()) == 0
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("check_every", [3, 10, 100])
+def test_ticks_look_as_often_as_the_caller_asks_gpu(check_every):
+    from tah_amd.engine import EngineConfig, TaHDecodeEngine, Weights
+    cfg = EngineConfig(hidden=256, layers=2, hq=16, hkv=8, head_dim=128, intermediate=768, vocab=4096, decider_hidden=32)
+    w = Weights.random_init(cfg, "cuda", seed=6)
+    ids, cu = torch.arange(21).cuda(), torch.tensor([0, 21], dtype=torch.int32, device="cuda")
+    eng = TaHDecodeEngine(w, 1, 400, device="cuda")
+    w.threshold = 2.0  # no token takes a second iteration
+    first, _ = eng.prefill(ids, cu)
+    eos = int(eng.generate(first, 8)[0, 5])
+    first, _ = eng.prefill(ids, cu)
+    eng.generate(first, 300, eos=eos, check_every=check_every)
+    assert bool(eng.finished.all()) and int(eng.n_hard) == 0 and eng.ticks == -(-int(eng.out_len) // check_every) * check_every
+
+
 def _topk_sampling_case(device, V, rows=6, draws=True):
     """The distribution over the k largest logits that sample_topk draws from against the one the reference's filters
     leave on the whole row (utils.py:84-125), on rows without equal values; and the draws land where it is not zero."""
