@@ -820,9 +820,11 @@ class TaHDecodeEngine(DecodeEngine):
     def generate(self, first_logits: torch.Tensor, max_new_tokens: int, *, temperature: float = 0.0, eos: int = -1,
                  use_graph: bool = True, check_every: int = 64, continuous: Optional[bool] = None, **filters):
         """As in :class:`DecodeEngine`.  ``continuous`` (default: whenever the engine can): rows do not wait for each other's second latent iterations
-        -- see :meth:`_generate_ticks`.  Greedy decoding gives the same tokens per row either way; sampled tokens come from
-        the same per-row distributions but from other random draws (a tick draws for every row, a step once per token).
-        ``check_every`` counts ticks there."""
+        -- see :meth:`_generate_ticks`.  Greedy decoding gives the same tokens per row either way.  So does sampling without a
+        top-k filter on an engine that has a workspace for the attention launch (small batches, long slabs), whose
+        generator is left as the step-wise loop leaves it; such an engine runs other filters step-wise by default.  On
+        other engines sampled tokens come from the same per-row distributions but from other random draws (a tick draws
+        for every row, a step once per token).  ``check_every`` counts ticks there."""
         self._check_room(max_new_tokens)
         dev = self.device
         greedy_fused = temperature <= 0.0 and self.fused_greedy and self.cfg.vocab % 8 == 0
@@ -886,7 +888,7 @@ class TaHDecodeEngine(DecodeEngine):
                         hard_len=self.hard_len, n_hard=self.n_hard, n_steps=self.n_steps, chosen=chosen,
                         workspace=self.greedy_workspace)
 
-    DRAW_AHEAD = 64  # ticks whose uniforms are drawn at a time
+    DRAW_AHEAD = 64  # ticks whose uniforms are drawn at a time at most
     LAST_TICKS = 8   # how often the host looks once the fastest possible row could be done
 
     def _launch_switches(self):
@@ -943,9 +945,13 @@ class TaHDecodeEngine(DecodeEngine):
         graphs = self.capture_ticks(eos, limit, temperature, **filters) if (use_graph and n_min > 0) else None
         ticks, steps = 0, n_min  # steps: how many the step-wise loop would run
         by_step = self._draws_by_step(temperature, filters)
+        ahead = min(self.DRAW_AHEAD, abs(check_every)) if eos >= 0 else self.DRAW_AHEAD
+        random_state = {}  # of the generator, before each step the step-wise loop might end in front of
         while n_min > 0:
-            if by_step and ticks % self.DRAW_AHEAD == 0:  # no row is at a later token than the tick's number
-                for i in range(ticks + 1, min(ticks + self.DRAW_AHEAD, n_min) + 1):
+            if by_step and ticks % ahead == 0:  # no row is at a later token than the tick's number
+                for i in range(ticks + 1, min(ticks + ahead, n_min) + 1):
+                    if eos >= 0 and (i - 1) % check_every == 0:
+                        random_state[i - 1] = torch.cuda.get_rng_state(self.device)
                     self.uniforms[i].uniform_()
             if graphs is not None:
                 graphs[ticks % 2].replay()
@@ -955,16 +961,19 @@ class TaHDecodeEngine(DecodeEngine):
             if ticks >= n_min and (ticks - n_min) % self.LAST_TICKS == 0 and bool(self.finished.all()):
                 break
             if eos >= 0 and ticks % check_every == 0 and bool(self.finished.all()):
-                every = abs(check_every)
-                steps = min(steps, max(1, -(-int(self.out_len.max()) // every)) * every)
                 break
             if ticks > 2 * n_min + self.LAST_TICKS:
                 raise TahDuoError("generation did not finish within two passes per token")
         self.ticks = ticks
+        if eos >= 0 and n_min > 0:  # (a row of n tokens met its end in step n)
+            every = abs(check_every)
+            steps = min(n_min, max(1, -(-int(self.out_len.max()) // every)) * every)
+        if steps in random_state:  # numbers of later steps were drawn for nothing
+            torch.cuda.set_rng_state(random_state[steps], self.device)
         self.finished &= self.out_len < limit  # rows stopped by the limit have not ended
         if eos >= 0 and self.step_workspace is not None:
             self.tok.masked_fill_(self.finished & (self.out_len < steps), 0)  # (as rows that sat out steps have it there)
-        self._advanced(min(ticks, steps))  # (a row appends at most one token of each depth per tick)
+        self._advanced(steps)  # (a row appends at most one token of each depth per step)
         return self.out_tokens[:, :max_new_tokens]
 
 

@@ -493,6 +493,40 @@ def test_ticks_look_as_often_as_the_caller_asks_gpu(check_every):
     assert bool(eng.finished.all()) and int(eng.n_hard) == 0 and eng.ticks == -(-int(eng.out_len) // check_every) * check_every
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("check_every", [1, 7, 64, 100])
+@pytest.mark.parametrize("filters", [{}, dict(temperature=1.0, top_p=0.95)])
+def test_ticks_with_an_end_of_sequence_token_leave_what_the_stepwise_loop_leaves_gpu(filters, check_every):
+    """Rows that end before the limit: ticks look as often as the caller asked, and tokens, per-row state, the host's counts and
+    the random state are those of the step-wise loop, also where hard tokens need more ticks than there are tokens."""
+    from tah_amd.engine import EngineConfig, TaHDecodeEngine, Weights
+    cfg = EngineConfig(hidden=256, layers=2, hq=16, hkv=8, head_dim=128, intermediate=768, vocab=4096, decider_hidden=32)
+    w = Weights.random_init(cfg, "cuda", seed=6)
+    B, T, new = (1, 21, 150) if filters else (3, 21, 150)
+    ids = torch.randint(0, cfg.vocab, (T,), generator=torch.Generator().manual_seed(5)).repeat(B).cuda()
+    cu = torch.arange(0, B * T + 1, T, dtype=torch.int32, device="cuda")
+    eng = TaHDecodeEngine(w, B, T + new, device="cuda")
+    first, _ = eng.prefill(ids, cu, calibrate=0.6)
+    torch.manual_seed(3)
+    free = eng.generate(first, new, **filters)[0].tolist()
+    met = [free.index(t) for t in free]  # where a token is met first
+    ends = [max(i for i in met if i <= j) for j in (60, new - 2)]  # the last one met by then
+    for eos in [free[i] for i in ends] + [int(first[0].argmax()), cfg.vocab - 1 if cfg.vocab - 1 not in free else -1]:
+        runs = []
+        for continuous, use_graph in ((False, True), (None, True)):
+            eng = TaHDecodeEngine(w, B, T + new, device="cuda")
+            first, _ = eng.prefill(ids, cu)
+            torch.manual_seed(3)
+            toks = eng.generate(first, new, eos=eos, continuous=continuous, use_graph=use_graph, check_every=check_every, **filters)
+            runs.append([toks.tolist(), eng.out_len.tolist(), eng.pos.tolist(), eng.finished.tolist(), eng.tok.tolist(), int(eng.n_hard),
+                         int(eng.n_steps), [sl.len.tolist() for sl in eng.slabs0 + eng.slabs1], eng.host_positions, eng.host_hard_rows,
+                         torch.cuda.get_rng_state().tolist()])
+            assert hasattr(eng, "ticks") == (continuous is None)
+        assert runs[0] == runs[1], eos
+        if eos >= 0 and eng.out_len.max() < 70:  # all rows have ended: soon after that the loop did
+            assert eng.ticks < 2 * 70 + check_every
+
+
 def _topk_sampling_case(device, V, rows=6, draws=True):
     """The distribution over the k largest logits that sample_topk draws from against the one the reference's filters
     leave on the whole row (utils.py:84-125), on rows without equal values; and the draws land where it is not zero."""
