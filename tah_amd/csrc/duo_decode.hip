@@ -983,7 +983,7 @@ __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const St
     }
     if constexpr (kSplit) {
         if (nact == 1) return;
-        TAH_WAIT_VMEM();  // every wave's partials have left before its workgroup is counted
+        device_settle();  // every wave's partials have left before its workgroup is counted
         __syncthreads();
         __shared__ int last;
         int32_t* const count = sp.arrived + qi * p.hkv + hk;

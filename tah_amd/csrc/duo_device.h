@@ -32,7 +32,7 @@ typedef __attribute__((address_space(3))) int lds_int;
 #endif
 
 // Words that workgroups on different XCDs hand to each other inside one launch: device-scope relaxed atomics, which pass by
-// the caches that are not shared.  Order between them is the caller's (TAH_WAIT_VMEM between a store and what announces it).
+// the caches that are not shared.  Order between them is the caller's (device_settle between a store and what announces it).
 #ifdef TAH_CPU_EMU
 template <class T> inline void device_store(T* p, T v) { __atomic_store(p, &v, __ATOMIC_SEQ_CST); }
 template <class T> inline T device_load(const T* p) { T v; __atomic_load(const_cast<T*>(p), &v, __ATOMIC_SEQ_CST); return v; }
@@ -46,6 +46,19 @@ template <class T> __device__ __forceinline__ T device_load(const T* p) { return
 __device__ __forceinline__ int device_add(int32_t* p, int v) { return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void device_max(unsigned long long* p, unsigned long long v) { __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 #endif
+
+#ifndef TAH_WAIT_VMEM
+// s_waitcnt vmcnt(0) (expcnt/lgkmcnt untouched) as a builtin, so the compiler's own wait-count
+// bookkeeping also learns that no ordinary load is pending past this point.
+#define TAH_WAIT_VMEM() __builtin_amdgcn_s_waitcnt(0x0F70)
+#endif
+// What this thread has stored or added for other workgroups is there.  The wait alone says nothing to the compiler about memory:
+// the fences, which cost no instruction, keep what stands before it before it and what stands behind it behind it.
+__device__ __forceinline__ void device_settle() {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    TAH_WAIT_VMEM();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
 
 constexpr int kWave = 64;
 constexpr float kLog2e = 1.4426950408889634f;
@@ -229,11 +242,6 @@ __device__ __forceinline__ void async_copy_4B(const void* sbase, uint32_t voff, 
 #endif
 #ifndef TAH_WAVES_PER_EU
 #define TAH_WAVES_PER_EU(lo, hi) __attribute__((amdgpu_waves_per_eu(lo, hi)))
-#endif
-#ifndef TAH_WAIT_VMEM
-// s_waitcnt vmcnt(0) (expcnt/lgkmcnt untouched) as a builtin, so the compiler's own wait-count
-// bookkeeping also learns that no ordinary load is pending past this point.
-#define TAH_WAIT_VMEM() __builtin_amdgcn_s_waitcnt(0x0F70)
 #endif
 #ifndef TAH_WAIT_VMEM_N
 // s_waitcnt vmcnt(n), n <= 15: all but the n most recently issued loads / asynchronous copies have landed

@@ -180,9 +180,11 @@ __device__ __forceinline__ bool shared_argmax(const __bf16* a, const __bf16* b, 
         const uint32_t bits = __float_as_uint(v + 0.0f);  // (-0 and 0 are equal)
         const uint32_t key = bits & 0x80000000u ? ~bits : bits | 0x80000000u;
         device_max(best, (unsigned long long)key << 32 | (0xffffffffu - (uint32_t)i));
-        TAH_WAIT_VMEM();
+        device_settle();
     }
-    if (device_add(count, 1) != parts - 1) return false;
+    const int before = device_add(count, 1);
+    device_settle();  // (the maximum is read only by who knows to be the last)
+    if (before != parts - 1) return false;
     const unsigned long long won = device_load(best);
     device_store(best, 0ull);
     device_store(count, 0);
