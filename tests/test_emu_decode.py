@@ -96,6 +96,8 @@ def test_fused_decode_step_equals_prep_then_decode_on_cpu_shim():
         decode_step_case.run("cpu", B=3, hq=16, hkv=8, seed=5)
         decode_step_case.run("cpu", B=2, hq=8, hkv=8, seed=6, full_slab=True)
         decode_step_case.run_mixed("cpu", B=4, hq=8, hkv=8, seed=7)
+        decode_step_case.run("cpu", B=3, hq=8, hkv=8, seed=5, slots=[4, 1, 0])
+        decode_step_case.run("cpu", B=3, hq=8, hkv=8, seed=5, slots=[1, -1, 0])  # fewer slots than rows
 
 
 def test_fused_decode_step_with_a_pairs_rows_shared_by_workgroups_on_cpu_shim():
@@ -108,6 +110,7 @@ def test_fused_decode_step_with_a_pairs_rows_shared_by_workgroups_on_cpu_shim():
         decode_step_case.run("cpu", B=2, hq=1, hkv=1, seed=9, max_len=600, cap2=300, full_slab=True, workspace=ws)
         decode_step_case.run("cpu", B=3, hq=2, hkv=1, seed=8, max_len=1400, cap1=1500, cap2=700, workspace=ws)
         decode_step_case.run_mixed("cpu", B=4, hq=2, hkv=1, seed=10, max_len=1400, cap1=1500, cap2=700, workspace=ws)
+        decode_step_case.run_mixed("cpu", B=3, hq=2, hkv=1, seed=11, max_len=700, cap1=720, cap2=300, workspace=True, slots=[5, 2, 0])
         decode_step_case.run("cpu", B=2, hq=2, hkv=1, seed=16, max_len=1000, cap1=1024, workspace=True, infinite=True)
         with pytest.raises(TahDuoError):
             decode_step_case.run("cpu", B=3, hq=2, hkv=1, seed=8, workspace=-16)

@@ -144,6 +144,19 @@ def test_fused_decode_step_with_a_workspace_equals_prep_then_decode(B, hq, hkv, 
         case("cuda", B=B, hq=hq, hkv=hkv, seed=B + cap1, max_len=cap1 - 1, hidden=2048, cap1=cap1, cap2=max(64, cap1 // 4), workspace=True)
 
 
+@pytest.mark.parametrize("B,hq,hkv,cap1,workspace", [(32, 16, 8, 900, False), (40, 8, 8, 300, False), (5, 16, 8, 900, True), (32, 16, 8, 4500, True)])
+def test_fused_decode_step_of_sequences_in_any_slot(B, hq, hkv, cap1, workspace):
+    """The launch asks for the place of slot i's rows before it knows which slot row i is: rows in other slots and in slots
+    beyond the batch."""
+    from tests import decode_step_case
+    print(f"fused decode step, permuted slots B={B} hq={hq} hkv={hkv} cap={cap1}", flush=True)
+    g = torch.Generator().manual_seed(B)
+    slots = torch.randperm(B + 7, generator=g)[:B].tolist()
+    for case in (decode_step_case.run, decode_step_case.run_mixed):
+        case("cuda", B=B, hq=hq, hkv=hkv, seed=B + cap1, max_len=cap1 - 1, hidden=2048, cap1=cap1, cap2=max(64, cap1 // 4), workspace=workspace,
+             slots=slots)
+
+
 def test_fused_decode_steps_of_several_sizes_share_a_workspace():
     """Few pairs, then more, then few: what a call leaves behind its counters must not be taken for another call's counters."""
     from tests import decode_step_case
