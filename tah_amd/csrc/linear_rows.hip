@@ -26,8 +26,8 @@
 // reduction per kernel, and the rows' operand: every workgroup reads all 32 x K of it from L2, which the
 // per-CU L1 fill rate (about 100 GB/s) makes 1 us per 128 KB.  Splitting K over workgroups would cut that, but
 // the hand-over between workgroups (device-scope fence + counter, last one reduces) cost 7 us per split when
-// tried: the fence writes back and invalidates the whole L2 of the XCD.  One to eight rows: 5.4 / 4.7 / 11.1 / 8.1 us
-// (kFold, H8 below).
+// tried: the fence writes back and invalidates the whole L2 of the XCD.  One to eight rows: 5.2 / 4.6 / 11.5 / 7.6 us
+// (kFold, H8 below), 5.7 / 5.1 / 11.7 / 9.6 without those.
 #include <hip/hip_runtime.h>
 
 #include <utility>
@@ -104,7 +104,7 @@ __device__ __forceinline__ void take_steps(const bf16x8* together, X& x, std::in
 // occupy half of the compute units occupies all.  A load then covers two k steps of the eight columns (lanes c < 8 the
 // even one, the others the odd one: 128 contiguous bytes each), and each loaded operand is multiplied twice, by either
 // step's rows; of the first product the columns below 8 count, of the second those from 8 on.  At one to eight rows o
-// (8 MB) takes 5.0 -> 4.7 us, down (25 MB) 9.5 -> 8.1 (both less again with the rows' operand folded, below).
+// (8 MB) takes 5.05 -> 4.65 us, down (25 MB) 9.6 -> 7.6, with the rows' operand folded (below); down at sixteen rows 9.5 -> 8.5.
 template <int NC, int CH, int EPI, int PW, int NH, bool H8 = false, int kFold = 0>
 __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParams p) {
     __shared__ __align__(16) float red[kLinWaves][NC][16 * NH][kTileCols];
@@ -158,11 +158,11 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
         wb[t] = H8 ? pw + ((int64_t)(group / 2) * steps + s0 + c / 8) * 64 + 16 * kg + 8 * (group % 2) + c % 8
                    : pw + ((int64_t)(group * NC + t) * steps + s0) * 64 + lane;
     // kFold: the lanes of rows past the last one read row 0's operand again instead of their zeros (their results are not used):
-    // with up to eight rows a load then touches a half to a quarter of the bytes (q|k|v at one to eight rows 5.75 -> 5.4 us).
+    // with up to eight rows a load then touches a half to a quarter of the bytes (gate|up at one to eight rows 11.7 -> 11.5 us).
     // Folded further where a wave's steps are one chunk: with one, two, four or eight rows (the next of these) the sixteen lanes of a k
     // group hold sixteen, eight, four or two steps of them, so 24 steps take 2, 3, 6 or 12 loads instead of 24 -- behind those the
-    // weights' own would wait -- and a lane gets its step from its neighbours inside the vector pipe: down 8.2 -> 7.5 us at one to
-    // eight rows (of a bound of 7.0, the same kernel with two of its operand loads), q|k|v 5.8 -> 5.6, o 4.6 -> 4.45.
+    // weights' own would wait -- and a lane gets its step from its neighbours inside the vector pipe: down 8.2 -> 7.6 us at one to
+    // eight rows (of a bound of 7.0, the same kernel with two of its operand loads), q|k|v 5.7 -> 5.2.
     constexpr int kFoldRows = kFold > 0 && kFold < 16 ? kFold : 16, kPerLoad = kFoldRows < 16 ? 16 / kFoldRows : 0;
     static_assert(kPerLoad == 0 || (CH == PW && NH == 1), "one chunk");
     const bf16x8* xb = px + (int64_t)s0 * 128 + 64 * half + (kPerLoad ? (c / kFoldRows) * 128 + 16 * kg + c % kFoldRows : kFold ? 16 * kg + (c < p.rows ? c : 0) : lane);
@@ -425,8 +425,8 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
 // An output head (n >= kWideFromCols plain columns, K = 256 PW) for more than sixteen rows: a resident workgroup per
 // compute unit walks a range of column groups.  Its waves keep their slices of the rows' operand in registers -- read per
 // group it is as many bytes as the weights and shares the L1's fill rate with them -- and ask for the next group's weights
-// before they multiply and reduce this one's.  151936 x 2048, 32 rows: 114.5 -> 104.8 us (5.4 -> 5.9 TB/s), 24 rows
-// 111.7 -> 101.5; groups dealt out round robin instead of ranges 107.6 (two workgroups then write the halves of a line).
+// before they multiply and reduce this one's.  151936 x 2048, 32 rows: 116 -> 105 us (5.4 -> 5.9 TB/s), 24 rows
+// 114 -> 105, inside a step 102 (6.1 TB/s); groups dealt out round robin instead of ranges 107.6 (two workgroups then write the halves of a line).
 // With sixteen rows the operand is half of that and many workgroups, two or three to a compute unit, stream better (93
 // against 98 us): they keep linear_rows_kernel.
 template <int EPI, int PW>
