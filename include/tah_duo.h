@@ -519,6 +519,32 @@ typedef struct tah_linear_rows_args {
 } tah_linear_rows_args;
 int tah_linear_rows(const tah_linear_rows_args* args, tah_stream_t stream);
 
+/* The linear layers between two attentions of a decode step in one launch, at most eight rows:
+ *   mid = residual + attn Wo^T;  act = silu(g) * u of mid's RMS-normed rows;  out = mid + act Wdown^T;  qkv = out Wqkv^T
+ * with the sums and roundings of the four tah_linear_rows calls (o with residual, gate|up with TAH_NORM_RMS, down with
+ * residual, the next layer's q|k|v), the same bits.  wqkv_packed NULL: without the last one.  Sizes: tah_linear_chain_supported.
+ * `handover`: TAH_LINEAR_CHAIN_HANDOVER_BYTES of scratch.
+ * `arrived`: TAH_LINEAR_CHAIN_WORDS words that are zero when the launch starts and not zero behind it; `clear`: other such
+ * words, which the launch sets to zero (those of the launch that comes next on the stream).  No two results may overlap
+ * each other, the residual or attn_packed (TAH_E_SHAPE). */
+#define TAH_LINEAR_CHAIN_TILES 256
+#define TAH_LINEAR_CHAIN_WORDS (3 * TAH_LINEAR_CHAIN_TILES * 8)
+#define TAH_LINEAR_CHAIN_HANDOVER_BYTES(hidden, ff) (16 * (2 * (hidden) + (ff)))
+typedef struct tah_linear_chain_args {
+    const void *wo_packed, *wgu_packed, *wdown_packed, *wqkv_packed; /* from tah_linear_pack_weight */
+    const void* attn_packed;  /* packed rows [32 * o_cols] */
+    const void* residual;     /* bf16 [rows, hidden] */
+    void *mid, *out, *qkv;    /* bf16 [rows, hidden], [rows, hidden], [rows, qkv_cols] */
+    void* handover;
+    void* out_packed;         /* packed rows [32 * hidden] of `out`, or NULL */
+    int64_t residual_row_stride, mid_row_stride, out_row_stride, qkv_row_stride; /* elements */
+    int32_t rows, hidden, o_cols, ff, qkv_cols;
+    float norm_eps;
+    int32_t *arrived, *clear;
+} tah_linear_chain_args;
+int tah_linear_chain_supported(int32_t rows, int32_t hidden, int32_t o_cols, int32_t ff, int32_t qkv_cols);
+int tah_linear_chain(const tah_linear_chain_args* args, tah_stream_t stream);
+
 /* One greedy generation step after the logits exist: per row, the final logits (first-iteration logits, plus
  * the second iteration's for rows that took one, summed in bf16 as the model's logits buffers are,
  * tah/model/tah_model.py:543,628), their arg-max (the lower index among equals), and the generation loop's

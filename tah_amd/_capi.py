@@ -124,6 +124,19 @@ class LinearRowsArgs(C.Structure):
     ]
 
 
+class LinearChainArgs(C.Structure):
+    """``tah_linear_chain_args``"""
+
+    _fields_ = [
+        ("wo_packed", c_void_p), ("wgu_packed", c_void_p), ("wdown_packed", c_void_p), ("wqkv_packed", c_void_p),
+        ("attn_packed", c_void_p), ("residual", c_void_p), ("mid", c_void_p), ("out", c_void_p), ("qkv", c_void_p),
+        ("handover", c_void_p), ("out_packed", c_void_p),
+        ("residual_row_stride", c_int64), ("mid_row_stride", c_int64), ("out_row_stride", c_int64), ("qkv_row_stride", c_int64),
+        ("rows", c_int32), ("hidden", c_int32), ("o_cols", c_int32), ("ff", c_int32), ("qkv_cols", c_int32), ("norm_eps", c_float),
+        ("arrived", c_void_p), ("clear", c_void_p),
+    ]
+
+
 class StepBeginArgs(C.Structure):
     """``tah_step_begin_args``"""
 
@@ -356,6 +369,8 @@ PROTOTYPES = {
     "tah_linear_pack_weight": (C.c_int, [c_void_p, c_int64, c_void_p, c_int32, c_int32, c_int32, c_void_p]),
     "tah_linear_pack_rows": (C.c_int, [c_void_p, c_int64, c_void_p, c_int32, c_int32, c_void_p]),
     "tah_linear_rows": (C.c_int, [C.POINTER(LinearRowsArgs), c_void_p]),
+    "tah_linear_chain_supported": (C.c_int, [c_int32] * 5),
+    "tah_linear_chain": (C.c_int, [C.POINTER(LinearChainArgs), c_void_p]),
     "tah_kv_append": (C.c_int, [C.POINTER(KvAppendArgs), c_void_p]),
     "tah_qk_prep": (C.c_int, [C.POINTER(QkPrepArgs), c_void_p]),
     "tah_duo_decode_step": (C.c_int, [C.POINTER(QkPrepArgs), C.POINTER(DuoDecodeArgs), c_void_p, c_void_p, c_void_p]),

@@ -37,6 +37,7 @@ typedef __attribute__((address_space(3))) int lds_int;
 template <class T> inline void device_store(T* p, T v) { __atomic_store(p, &v, __ATOMIC_SEQ_CST); }
 template <class T> inline T device_load(const T* p) { T v; __atomic_load(const_cast<T*>(p), &v, __ATOMIC_SEQ_CST); return v; }
 inline int device_add(int32_t* p, int v) { return __atomic_fetch_add(p, v, __ATOMIC_SEQ_CST); }
+inline void device_or(uint32_t* p, uint32_t v) { __atomic_fetch_or(p, v, __ATOMIC_SEQ_CST); }
 inline void device_max(unsigned long long* p, unsigned long long v) {
     for (unsigned long long now = device_load(p); now < v && !__atomic_compare_exchange_n(p, &now, v, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST);) {}
 }
@@ -44,6 +45,7 @@ inline void device_max(unsigned long long* p, unsigned long long v) {
 template <class T> __device__ __forceinline__ void device_store(T* p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 template <class T> __device__ __forceinline__ T device_load(const T* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ int device_add(int32_t* p, int v) { return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ void device_or(uint32_t* p, uint32_t v) { __hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void device_max(unsigned long long* p, unsigned long long v) { __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 #endif
 
@@ -51,6 +53,17 @@ __device__ __forceinline__ void device_max(unsigned long long* p, unsigned long 
 // s_waitcnt vmcnt(0) (expcnt/lgkmcnt untouched) as a builtin, so the compiler's own wait-count
 // bookkeeping also learns that no ordinary load is pending past this point.
 #define TAH_WAIT_VMEM() __builtin_amdgcn_s_waitcnt(0x0F70)
+#endif
+#ifdef TAH_CPU_EMU
+#define TAH_WAIT_LDS() ((void)0)
+#define TAH_SLEEP(n) ((void)0)
+#define TAH_OPAQUE_S(p) ((void)0)
+#define TAH_GLOBAL
+#else
+#define TAH_WAIT_LDS() __builtin_amdgcn_s_waitcnt(0xC07F)  // s_waitcnt lgkmcnt(0), loads from memory stay on their way
+#define TAH_SLEEP(n) __builtin_amdgcn_s_sleep(n)
+#define TAH_OPAQUE_S(p) asm volatile("" : "+s"(p))  // a value that stays in scalar registers, apart from those it was made of
+#define TAH_GLOBAL __attribute__((address_space(1)))
 #endif
 // What this thread has stored or added for other workgroups is there.  The wait alone says nothing to the compiler about memory:
 // the fences, which cost no instruction, keep what stands before it before it and what stands behind it behind it.

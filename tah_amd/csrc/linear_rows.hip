@@ -543,6 +543,452 @@ __global__ __launch_bounds__(kLinThreads) void linear_wide_kernel(const LinParam
     }
 }
 
+// ---- a layer's four linear layers in one launch ------------------------------------------------------------
+// o + residual, gate|up + SiLU, down + residual and the next layer's q|k|v of at most eight rows.  As four launches each of
+// them pays its start, the first bytes' way and its reduction with the memory pipe empty; here the next phase's weights,
+// which depend on nothing, are on their way while a phase's results travel between the workgroups.  2048 / 6144 / 4096 (100 MB) in a
+// captured sequence of layers: 23.7 us at one row, 25.7 at eight, against 28.1 as four launches; the weights alone take 16 us at
+// 6.2 TB/s.  What bounds it now: the three hand-overs, each from the last workgroup's sums to the first product of the next phase 3.5
+// to 4 us (a store that has arrived 0.7 to 1, the slowest workgroup another 1, bit and poll 1.5, the rows 0.7), of which the weights
+// asked for ahead hide one and parts of two.  From nine rows on the rows' operand that everybody reads past the L2s would cost
+// more than the launches (eight rows already lose 2 us): they keep four launches.
+//  * A workgroup takes the same tile number of every phase (2048 / 6144: 256 tiles in each, one to a compute unit).  Eight waves
+//    multiply as in linear_rows_kernel (same slices of K, same order of sums: the same bits); a ninth reduces, stores and
+//    waits for the other workgroups, so that no wait for a store or a flag stands behind the weights' loads.
+//  * A tile's results and then its bit in `arrived` are stored with device_store, past the XCDs' own L2 caches; readers use
+//    device_load.  No fence: that would write back and invalidate the L2.
+//  * Every wait ends, whatever is resident: a workgroup that has waited kChainPolls polls computes missing tiles itself.  All that
+//    such a tile reads is there (the phase before it is complete, or the waiting workgroup would not be here), and its
+//    result is the same bits whoever stores it and however often, because no phase's result lies on another phase's
+//    operands (tah_linear_chain refuses such calls).  So one workgroup alone would finish the launch.
+//  * `arrived` is zero at the start; the words of the next launch (`clear`) are zeroed on the way.
+constexpr int kChainTiles = TAH_LINEAR_CHAIN_TILES;  // tiles of a phase at most
+// `arrived`: a bit per tile, four to a word, every word on a line of its own: a line's writes take their turns among the reads of
+// everybody who waits (32 tiles to a line 31.4 us a launch, sixteen 27.6, eight 25.0, four 24.0; a byte per tile on two lines 38.5)
+constexpr int kChainBits = 4, kChainLine = 32, kChainPhaseWords = kChainTiles / kChainBits * kChainLine;
+static_assert(3 * kChainPhaseWords == TAH_LINEAR_CHAIN_WORDS, "header");
+constexpr int kChainThreads = kLinThreads + kWave;
+#ifdef TAH_CPU_EMU
+constexpr int kChainPolls = 2;  // (workgroups run one after another there)
+#else
+constexpr int kChainPolls = 128;  // about 150 us: several times a whole launch
+#endif
+
+constexpr int kChainSleep = 1;    // x 64 cycles between polls
+
+struct ChainParams {
+    const bf16x8 *w0, *w1, *w2, *w3;  // packed weights
+    const bf16x8* x0;                 // packed rows: attention output
+    unsigned long long *x1, *x2, *x3; // results on their way to the next phase (handed_over)
+    bf16x8* out_packed;               // packed rows of `out`, or null
+    const __bf16* res;                // rows the o layer adds to
+    __bf16 *mid, *out, *y;            // row-major: o + residual, down + residual, q|k|v
+    int64_t res_rs, mid_rs, out_rs, y_rs;
+    uint32_t* arrived;
+    int32_t* clear;
+    int32_t rows, tiles0, tiles1, tiles2, tiles3;
+    float eps;
+};
+
+// Where columns col ... col + 3 of a row lie between two phases, in 8-byte words.  Nothing but the rows (rounded up to F), and
+// a wave's 8-byte load of 64 operands' halves covers 512 bytes that lie together: every compute unit reads all of it past the L2s,
+// and in the packed rows form (16 of 256 bytes used by one row) those requests took 1.5 us of a phase.
+template <int F>
+__device__ __forceinline__ int handed_over(int row, int col) {
+    const int unit = (col / 8) * F + row;
+    return ((unit / 64) * 2 + (col % 8) / 4) * 64 + unit % 64;
+}
+// A wave has this many loads of weights on their way at most: 32 KB per compute unit keep the memory busy, and what the ninth wave
+// stores and asks for has no longer queue than that before it (all at once: the stores took 6.8 us to arrive, not 1.2).
+constexpr int kChainWindow = 4;
+
+// A wave's part of one tile: PW steps of K, NC column tiles (H8: one, and half of its columns, as in linear_rows_kernel), rows
+// folded to F.
+template <int PW, int NC, bool H8, int F>
+struct ChainTile {
+    static constexpr int kLoads = H8 ? PW / 2 : PW, kPer = 16 / F, kXLoads = (PW + kPer - 1) / kPer;
+    bf16x8 w[kLoads][NC], x[kXLoads];
+    float ss;
+    f32x4 acc[NC][H8 ? 2 : 1];
+
+    template <int kFrom, int kTo>
+    __device__ __forceinline__ void ask_weights(const bf16x8* pw, int tile, int wave, int lane) {
+        // (a base that is the same for the whole wave and 32-bit offsets: one address register for all loads)
+        const int c = lane % 16, kg = lane / 16;
+        constexpr int steps = kLinWaves * PW;
+        const uint32_t own = 16 * (H8 ? 64 * (c / 8) + 16 * kg + c % 8 : lane);
+#pragma unroll
+        for (int i = kFrom; i < kTo; ++i)
+#pragma unroll
+            for (int t = 0; t < NC; ++t) {
+                const bf16x8* at = H8 ? pw + ((int64_t)(tile / 2) * steps + wave * PW + 2 * i) * 64 + 8 * (tile % 2)
+                                      : pw + ((int64_t)(tile * NC + t) * steps + wave * PW + i) * 64;
+                uintptr_t base = reinterpret_cast<uintptr_t>(at);
+                TAH_OPAQUE_S(base);
+                w[i][t] = __builtin_nontemporal_load(reinterpret_cast<const TAH_GLOBAL bf16x8*>(reinterpret_cast<const TAH_GLOBAL char*>(base) + own));
+            }
+    }
+    __device__ __forceinline__ void ask_weights(const bf16x8* pw, int tile, int wave, int lane) { ask_weights<0, kLoads>(pw, tile, wave, lane); }
+    // the same with at most kChainWindow of the wave's loads on their way
+    template <int kFrom, int kTo>
+    __device__ __forceinline__ void trickle_weights(const bf16x8* pw, int tile, int wave, int lane) {
+        if constexpr (kFrom < kTo) {
+            __builtin_amdgcn_sched_barrier(0);
+            TAH_WAIT_VMEM_N(kChainWindow - NC);
+            ask_weights<kFrom, kFrom + 1>(pw, tile, wave, lane);
+            __builtin_amdgcn_sched_barrier(0);
+            trickle_weights<kFrom + 1, kTo>(pw, tile, wave, lane);
+        }
+    }
+    __device__ __forceinline__ static int step_of(int j, int c) {
+        const int step = j * kPer + c / F;
+        return (j + 1) * kPer > PW && step >= PW ? PW - 1 : step;  // a last load's steps past the slice: the last step again
+    }
+    __device__ __forceinline__ void ask_rows(const bf16x8* px, int wave, int lane) {
+        const int c = lane % 16, kg = lane / 16;
+#pragma unroll
+        for (int j = 0; j < kXLoads; ++j) x[j] = px[wave * PW * 128 + (uint32_t)(step_of(j, c) * 128 + 16 * kg + c % F)];
+    }
+    __device__ __forceinline__ void ask_rows(const unsigned long long* px, int wave, int lane) {
+        const int c = lane % 16, kg = lane / 16;
+        typedef __attribute__((__vector_size__(2 * sizeof(unsigned long long)))) unsigned long long u64x2;
+#pragma unroll
+        for (int j = 0; j < kXLoads; ++j) {
+            const uint32_t at = handed_over<F>(c % F, 32 * (wave * PW + step_of(j, c)) + 8 * kg);
+            u64x2 v;
+            v[0] = device_load(px + at);
+            v[1] = device_load(px + at + 64);
+            x[j] = __builtin_bit_cast(bf16x8, v);
+        }
+    }
+    __device__ __forceinline__ void start() {
+        ss = 0.f;
+#pragma unroll
+        for (int t = 0; t < NC; ++t)
+#pragma unroll
+            for (int h = 0; h < (H8 ? 2 : 1); ++h) acc[t][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    template <bool kNorm, int S>
+    __device__ __forceinline__ void step() {
+        const bf16x8 a = from_lane_above<F, F * (S % kPer)>(x[S / kPer]);
+        if constexpr (kNorm) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) ss += (float)a[i] * (float)a[i];
+        }
+#pragma unroll
+        for (int t = 0; t < NC; ++t) {
+            if constexpr (H8) acc[t][S % 2] = mfma16(a, w[S / 2][t], acc[t][S % 2]);
+            else acc[t][0] = mfma16(a, w[S][t], acc[t][0]);
+        }
+    }
+    template <bool kNorm, int kFrom, int... S>
+    __device__ __forceinline__ void steps(std::integer_sequence<int, S...>) { (step<kNorm, kFrom + S>(), ...); }
+    template <bool kNorm, int kFrom, int kTo>
+    __device__ __forceinline__ void multiply() { steps<kNorm, kFrom>(std::make_integer_sequence<int, kTo - kFrom>{}); }
+    template <bool kNorm>
+    __device__ __forceinline__ void park(float (*red)[3][16][kTileCols], float (*ssq)[16], int wave, int lane) {
+        const int c = lane % 16, kg = lane / 16;
+#pragma unroll
+        for (int t = 0; t < NC; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (4 * kg < F) red[wave][t][4 * kg + r][c] = (H8 && c >= 8) ? acc[t][H8 ? 1 : 0][r] : acc[t][0][r];
+        if constexpr (kNorm) {
+            ss += __shfl_xor(ss, 16);
+            ss += __shfl_xor(ss, 32);
+            if (kg == 0) ssq[wave][c] = ss;
+        }
+    }
+};
+
+// LDS between the waves of a workgroup: loads from memory stay on their way across it
+__device__ __forceinline__ void chain_barrier() {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    TAH_WAIT_LDS();
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
+// PWO, PWH, PWF: query columns, hidden size and MLP width over 256.  kNext: with the q|k|v phase.
+template <int F, int PWO, int PWH, int PWF, bool kNext>
+__global__ __launch_bounds__(kChainThreads) void linear_chain_kernel(const ChainParams p) {
+    __shared__ __align__(16) float red[kLinWaves][3][16][kTileCols];
+    __shared__ float ssq[kLinWaves][16];
+    __shared__ int command;  // a tile of the phase before to compute, or -1: go on
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const int tile = blockIdx.x;
+    using O = ChainTile<PWO, 1, true, F>;
+    using GateUp = ChainTile<PWH, 3, false, F>;
+    using Down = ChainTile<PWF, 1, true, F>;
+    using Qkv = ChainTile<PWH, 1, false, F>;
+    // (a workgroup without a tile in a phase multiplies another's and stores nothing)
+    const int t0 = tile < p.tiles0 ? tile : 0, t1 = tile < p.tiles1 ? tile : 0, t2 = tile < p.tiles2 ? tile : 0, t3 = tile < p.tiles3 ? tile : 0;
+
+    if (wave < kLinWaves) {
+        // until the phase before is complete, with tiles that others should have computed; the weights on their way are asked for
+        // again behind those (they share registers with them)
+        auto wait = [&](auto help, auto ask_again) __attribute__((always_inline)) {
+            chain_barrier();
+            int missing = command;
+            if (missing >= 0) {
+                do {
+                    help(missing);
+                    chain_barrier();
+                    chain_barrier();
+                    missing = command;
+                } while (missing >= 0);
+                ask_again();
+            }
+        };
+        auto help0 = [&](int missing) __attribute__((always_inline)) {
+            O o;
+            o.ask_rows(p.x0, wave, lane);
+            o.ask_weights(p.w0, missing, wave, lane);
+            o.start();
+            o.template multiply<false, 0, PWO>();
+            o.template park<false>(red, ssq, wave, lane);
+        };
+        auto help1 = [&](int missing) __attribute__((always_inline)) {
+            GateUp g;
+            g.ask_rows(p.x1, wave, lane);
+            g.ask_weights(p.w1, missing, wave, lane);
+            g.start();
+            g.template multiply<true, 0, PWH>();
+            g.template park<true>(red, ssq, wave, lane);
+        };
+        auto help2 = [&](int missing) __attribute__((always_inline)) {
+            Down d;
+            d.ask_rows(p.x2, wave, lane);
+            d.ask_weights(p.w2, missing, wave, lane);
+            d.start();
+            d.template multiply<false, 0, PWF>();
+            d.template park<false>(red, ssq, wave, lane);
+        };
+        constexpr int kDownAhead = Down::kLoads / 3, kQkvAhead = kNext ? Qkv::kLoads / 2 : 0;  // (nine waves leave 168 registers)
+        GateUp gu;
+        Down down;
+        Qkv qkv;
+        {
+            O o;
+            o.ask_rows(p.x0, wave, lane);
+            __builtin_amdgcn_sched_barrier(0);
+            o.ask_weights(p.w0, t0, wave, lane);
+            __builtin_amdgcn_sched_barrier(0);
+            o.start();
+            o.template multiply<false, 0, PWO>();
+            o.template park<false>(red, ssq, wave, lane);
+            chain_barrier();
+            gu.template trickle_weights<0, PWH>(p.w1, t1, wave, lane);
+            down.template trickle_weights<0, kDownAhead>(p.w2, t2, wave, lane);
+        }
+        wait(help0, [&]() __attribute__((always_inline)) { 
+            gu.ask_weights(p.w1, t1, wave, lane);
+            down.template ask_weights<0, kDownAhead>(p.w2, t2, wave, lane);
+        });
+        gu.ask_rows(p.x1, wave, lane);
+        gu.start();
+        gu.template multiply<true, 0, PWH>();
+        gu.template park<true>(red, ssq, wave, lane);
+        chain_barrier();
+        down.template trickle_weights<kDownAhead, Down::kLoads>(p.w2, t2, wave, lane);
+        qkv.template trickle_weights<0, kQkvAhead>(p.w3, t3, wave, lane);
+
+        wait(help1, [&]() __attribute__((always_inline)) { 
+            down.ask_weights(p.w2, t2, wave, lane);
+            qkv.template ask_weights<0, kQkvAhead>(p.w3, t3, wave, lane);
+        });
+        down.ask_rows(p.x2, wave, lane);
+        chain_barrier();
+        if constexpr (kNext) qkv.template ask_weights<kQkvAhead, Qkv::kLoads>(p.w3, t3, wave, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        down.start();
+        down.template multiply<false, 0, PWF>();
+        down.template park<false>(red, ssq, wave, lane);
+        chain_barrier();
+
+        if constexpr (kNext) {
+            wait(help2, [&]() __attribute__((always_inline)) { qkv.ask_weights(p.w3, t3, wave, lane); });
+            qkv.ask_rows(p.x3, wave, lane);
+            qkv.start();
+            qkv.template multiply<false, 0, PWH>();
+            qkv.template park<false>(red, ssq, wave, lane);
+            chain_barrier();
+        }
+        return;
+    }
+
+    // ---- the ninth wave: a lane per (row, 2 columns) of the eight-column tiles, per (row, 4 columns) of the others; all partial
+    // sums are asked for before the first is added, in the order of linear_rows_kernel ----
+    typedef __attribute__((__vector_size__(2 * sizeof(float)))) float f32x2;
+    typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+    typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
+    for (int i = (int)blockIdx.x * kWave + lane; i < TAH_LINEAR_CHAIN_WORDS; i += (int)gridDim.x * kWave) p.clear[i] = 0;
+    // rows past the last one are zeros in the rows form that stays
+    if (p.out_packed && tile < p.tiles2 && lane >= p.rows && lane < kLinRows) p.out_packed[packed_rows_unit(lane, 8 * tile)] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    const int row2 = lane / 4, col2 = 2 * (lane % 4);
+    const bool live2 = row2 < p.rows;
+    auto sum_even_odd = [&](float* s) __attribute__((always_inline)) {
+        f32x2 part[kLinWaves][2];
+#pragma unroll
+        for (int w = 0; w < kLinWaves; ++w)
+#pragma unroll
+            for (int odd = 0; odd < 2; ++odd) part[w][odd] = *reinterpret_cast<const f32x2*>(&red[w][0][row2][8 * odd + col2]);
+        __builtin_amdgcn_sched_barrier(0);
+        s[0] = s[1] = 0.f;
+#pragma unroll
+        for (int w = 0; w < kLinWaves; ++w)
+#pragma unroll
+            for (int odd = 0; odd < 2; ++odd) {
+                s[0] += part[w][odd][0];
+                s[1] += part[w][odd][1];
+            }
+    };
+    auto ask4 = [&](f32x4 (&part)[kLinWaves], int t, int row, int col) __attribute__((always_inline)) {
+#pragma unroll
+        for (int w = 0; w < kLinWaves; ++w) part[w] = *reinterpret_cast<const f32x4*>(&red[w][t][row][col]);
+    };
+    auto sum4 = [&](const f32x4 (&part)[kLinWaves]) __attribute__((always_inline)) {
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < kLinWaves; ++w) s += part[w];
+        return s;
+    };
+    auto announce = [&](int phase, int of) __attribute__((always_inline)) {
+        device_settle();  // the results are there before the word that says so
+        if (lane == 0) device_or(p.arrived + phase * kChainPhaseWords + of / kChainBits * kChainLine, 1u << (of % kChainBits));
+    };
+    auto hand_over2 = [&](unsigned long long* to, int of, bf16x2 o) __attribute__((always_inline)) {
+        device_store(reinterpret_cast<uint32_t*>(to + handed_over<F>(row2, 8 * of + col2)) + (col2 % 4) / 2, __builtin_bit_cast(uint32_t, o));
+    };
+    auto plus = [&](const float* s, bf16x2 r) __attribute__((always_inline)) {
+        bf16x2 o;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) o[i] = (__bf16)((float)(__bf16)s[i] + (float)r[i]);
+        return o;
+    };
+    auto finish0 = [&](int of, bf16x2 r) __attribute__((always_inline)) {
+        bf16x2 o = r;
+        if (live2) {
+            float s[2];
+            sum_even_odd(s);
+            o = plus(s, r);
+            hand_over2(p.x1, of, o);
+            device_store(reinterpret_cast<uint32_t*>(p.mid + (int64_t)row2 * p.mid_rs + 8 * of + col2), __builtin_bit_cast(uint32_t, o));
+        }
+        announce(0, of);
+        return o;
+    };
+    auto finish1 = [&](int of) __attribute__((always_inline)) {
+        const int row = lane / 6, col = 4 * (lane % 6);
+        if (row < p.rows) {
+            // tiles: gate 0-15 | gate 16-23, up 16-23 | up 0-15
+            const bool last = col >= 16;
+            f32x4 g[kLinWaves], u[kLinWaves];
+            float sq[kLinWaves];
+            ask4(g, last ? 1 : 0, row, last ? col - 16 : col);
+            ask4(u, last ? 1 : 2, row, last ? col - 8 : col);
+#pragma unroll
+            for (int w = 0; w < kLinWaves; ++w) sq[w] = ssq[w][row];
+            __builtin_amdgcn_sched_barrier(0);
+            const f32x4 sg = sum4(g), su = sum4(u);
+            float ss = 0.f;
+#pragma unroll
+            for (int w = 0; w < kLinWaves; ++w) ss += sq[w];
+            const float rin = __builtin_amdgcn_rsqf(ss / (float)(256 * PWH) + p.eps);
+            bf16x4 o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = (__bf16)((float)(__bf16)silu_f((float)(__bf16)(sg[i] * rin)) * (float)(__bf16)(su[i] * rin));
+            device_store(p.x2 + handed_over<F>(row, kGroup24 * of + col), __builtin_bit_cast(unsigned long long, o));
+        }
+        announce(1, of);
+    };
+    auto finish2 = [&](int of, bf16x2 r) __attribute__((always_inline)) {
+        if (live2) {
+            float s[2];
+            sum_even_odd(s);
+            const bf16x2 o = plus(s, r);
+            if (kNext) hand_over2(p.x3, of, o);
+            if (p.out_packed) *reinterpret_cast<bf16x2*>(reinterpret_cast<__bf16*>(p.out_packed + packed_rows_unit(row2, 8 * of)) + col2) = o;
+            *reinterpret_cast<bf16x2*>(p.out + (int64_t)row2 * p.out_rs + 8 * of + col2) = o;
+        }
+        if (kNext) announce(2, of);
+    };
+    // until all tiles of a phase have arrived; a tile that does not come is computed here
+    auto wait = [&](int phase, int tiles, auto finish) __attribute__((always_inline)) {
+        // a word per lane
+        const int first = kChainBits * lane, mine = tiles - first < kChainBits ? tiles - first : kChainBits;
+        const uint32_t* const word = p.arrived + phase * kChainPhaseWords + lane * kChainLine;
+        uint32_t absent = mine > 0 ? (1u << mine) - 1u : 0u;
+        for (int polls = 0;;) {
+            if (absent != 0) absent &= ~device_load(word);  // (a word that is complete is not read again: reads are in the writers' way)
+            int missing = absent != 0 ? first + __builtin_ctz(absent) : -1;
+            const unsigned long long some = __ballot(missing >= 0);
+            if (some == 0) break;
+            if (++polls >= kChainPolls) {
+                missing = __shfl(missing, __builtin_ctzll(some));
+                if (lane == 0) command = missing;
+                chain_barrier();
+                chain_barrier();
+                finish(missing);
+                polls = kChainPolls - 1;  // (the others of its kind are late as well)
+            } else {
+                TAH_SLEEP(kChainSleep);
+            }
+        }
+        if (lane == 0) command = -1;
+        chain_barrier();
+        if (phase == 1) chain_barrier();  // (between the waves' loads of the rows and those of weights)
+    };
+    auto residual = [&](int of) __attribute__((always_inline)) {
+        bf16x2 r = {0, 0};
+        if (live2) r = *reinterpret_cast<const bf16x2*>(p.res + (int64_t)row2 * p.res_rs + 8 * of + col2);
+        return r;
+    };
+    bf16x2 mid = residual(t0);
+    chain_barrier();
+    if (tile < p.tiles0) mid = finish0(tile, mid);
+    wait(0, p.tiles0, [&](int of) __attribute__((always_inline)) { finish0(of, residual(of)); });
+    chain_barrier();
+    if (tile < p.tiles1) finish1(tile);
+    wait(1, p.tiles1, finish1);
+    chain_barrier();
+    if (tile < p.tiles2) finish2(tile, mid);  // (tiles0 = tiles2: its own columns of o + residual are still here)
+    if constexpr (kNext) {
+        wait(2, p.tiles2, [&](int of) __attribute__((always_inline)) {
+            uint32_t r = 0;
+            if (live2) r = device_load(reinterpret_cast<const uint32_t*>(p.mid + (int64_t)row2 * p.mid_rs + 8 * of + col2));
+            finish2(of, __builtin_bit_cast(bf16x2, r));
+        });
+        chain_barrier();
+        const int row = lane / 4, col = 4 * (lane % 4);
+        if (tile < p.tiles3 && row < p.rows) {
+            f32x4 part[kLinWaves];
+            ask4(part, 0, row, col);
+            __builtin_amdgcn_sched_barrier(0);
+            const f32x4 s = sum4(part);
+            bf16x4 o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = (__bf16)s[i];
+            *reinterpret_cast<bf16x4*>(p.y + (int64_t)row * p.y_rs + kTileCols * tile + col) = o;
+        }
+    }
+}
+
+template <int PWO, int PWH, int PWF>
+void launch_chain(const ChainParams& p, bool next, hipStream_t st) {
+    int tiles = p.tiles0 > p.tiles1 ? p.tiles0 : p.tiles1;
+    tiles = tiles > p.tiles3 ? tiles : p.tiles3;
+    const auto run = [&](auto fold) {
+        constexpr int F = decltype(fold)::value;
+        if (next) hipLaunchKernelGGL((linear_chain_kernel<F, PWO, PWH, PWF, true>), dim3(tiles), dim3(kChainThreads), 0, st, p);
+        else hipLaunchKernelGGL((linear_chain_kernel<F, PWO, PWH, PWF, false>), dim3(tiles), dim3(kChainThreads), 0, st, p);
+    };
+    if (p.rows <= 1) run(std::integral_constant<int, 1>{});
+    else if (p.rows <= 2) run(std::integral_constant<int, 2>{});
+    else if (p.rows <= 4) run(std::integral_constant<int, 4>{});
+    else run(std::integral_constant<int, 8>{});
+}
+
 // ---- re-ordering -----------------------------------------------------------------------------------------
 // Weight row behind column slot c of tile t of the packed order.
 __device__ __host__ inline int64_t packed_weight_row(int kind, int n, int tile, int c) {
@@ -756,5 +1202,83 @@ extern "C" int tah_linear_rows(const tah_linear_rows_args* a, tah_stream_t strea
         if (pw == 8) launch<2, 4, kGateUp16, 8>(p, groups, batch, st);
         else launch<2, 2, kGateUp16, 0>(p, groups, batch, st);
     }
+    return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
+}
+
+extern "C" int tah_linear_chain_supported(int32_t rows, int32_t hidden, int32_t o_cols, int32_t ff, int32_t qkv_cols) {
+    using namespace tah;
+    if (rows < 1 || rows > 8 || qkv_cols < 0 || qkv_cols % kTileCols != 0 || qkv_cols > kTileCols * kChainTiles) return 0;
+#ifdef TAH_CPU_EMU
+    if (hidden == 512 && o_cols == 512 && ff == 1536) return 1;  // (a size the execution on the CPU gets through)
+#endif
+    return hidden == 2048 && o_cols == 2048 && ff == 6144;
+}
+
+extern "C" int tah_linear_chain(const tah_linear_chain_args* a, tah_stream_t stream) {
+    using namespace tah;
+    if (!a) return TAH_E_NULL;
+    if (a->rows == 0) return TAH_OK;
+    const bool next = a->wqkv_packed != nullptr;
+    if (!tah_linear_chain_supported(a->rows, a->hidden, a->o_cols, a->ff, next ? a->qkv_cols : 0) || (next && a->qkv_cols == 0)) return TAH_E_SHAPE;
+    const void* needed[] = {a->wo_packed, a->wgu_packed, a->wdown_packed, a->attn_packed, a->residual, a->mid, a->out, a->handover, a->arrived, a->clear, next ? a->qkv : a->out, next ? a->wqkv_packed : a->out};
+    for (const void* q : needed) {
+        if (!q) return TAH_E_NULL;
+        if (!aligned16(q)) return TAH_E_ALIGN;
+    }
+    if (!aligned16(a->out_packed)) return TAH_E_ALIGN;
+    if ((a->residual_row_stride | a->mid_row_stride | a->out_row_stride) % 8 != 0 || (next && a->qkv_row_stride % 8 != 0)) return TAH_E_ALIGN;
+    if (a->residual_row_stride < a->hidden || a->mid_row_stride < a->hidden || a->out_row_stride < a->hidden || (next && a->qkv_row_stride < a->qkv_cols))
+        return TAH_E_SHAPE;
+    // what a phase writes may be written again while later phases run: no result may lie on an operand or on another result
+    struct Range { const char* at; int64_t bytes; };
+    const auto rows_of = [&](const void* q, int64_t stride, int64_t cols) { return Range{static_cast<const char*>(q), 2 * ((a->rows - 1) * stride + cols)}; };
+    const int64_t word_bytes = (int64_t)TAH_LINEAR_CHAIN_WORDS * 4;
+    const Range none{nullptr, 0};
+    const Range written[] = {rows_of(a->mid, a->mid_row_stride, a->hidden), rows_of(a->out, a->out_row_stride, a->hidden),
+                             {static_cast<const char*>(a->handover), (int64_t)TAH_LINEAR_CHAIN_HANDOVER_BYTES(a->hidden, a->ff)},
+                             {reinterpret_cast<const char*>(a->arrived), word_bytes}, {reinterpret_cast<const char*>(a->clear), word_bytes},
+                             a->out_packed ? Range{static_cast<const char*>(a->out_packed), 64 * (int64_t)a->hidden} : none,
+                             next ? rows_of(a->qkv, a->qkv_row_stride, a->qkv_cols) : none};
+    const Range read[] = {rows_of(a->residual, a->residual_row_stride, a->hidden), {static_cast<const char*>(a->attn_packed), 64 * (int64_t)a->o_cols}};
+    const auto meet = [](const Range& x, const Range& y) { return x.bytes > 0 && y.bytes > 0 && x.at < y.at + y.bytes && y.at < x.at + x.bytes; };
+    for (int i = 0; i < 7; ++i) {
+        for (int j = i + 1; j < 7; ++j)
+            if (meet(written[i], written[j])) return TAH_E_SHAPE;
+        for (const Range& q : read)
+            if (meet(written[i], q)) return TAH_E_SHAPE;
+    }
+    ChainParams p{};
+    p.w0 = static_cast<const bf16x8*>(a->wo_packed);
+    p.w1 = static_cast<const bf16x8*>(a->wgu_packed);
+    p.w2 = static_cast<const bf16x8*>(a->wdown_packed);
+    p.w3 = static_cast<const bf16x8*>(a->wqkv_packed);
+    p.x0 = static_cast<const bf16x8*>(a->attn_packed);
+    p.x1 = static_cast<unsigned long long*>(a->handover);
+    p.x2 = p.x1 + 2 * (int64_t)a->hidden;  // (eight rows' 8-byte words of each)
+    p.x3 = p.x2 + 2 * (int64_t)a->ff;
+    p.out_packed = static_cast<bf16x8*>(a->out_packed);
+    p.res = static_cast<const __bf16*>(a->residual);
+    p.mid = static_cast<__bf16*>(a->mid);
+    p.out = static_cast<__bf16*>(a->out);
+    p.y = static_cast<__bf16*>(a->qkv);
+    p.res_rs = a->residual_row_stride;
+    p.mid_rs = a->mid_row_stride;
+    p.out_rs = a->out_row_stride;
+    p.y_rs = a->qkv_row_stride;
+    p.arrived = reinterpret_cast<uint32_t*>(a->arrived);
+    p.clear = a->clear;
+    p.rows = a->rows;
+    p.tiles0 = p.tiles2 = a->hidden / 8;
+    p.tiles1 = a->ff / kGroup24;
+    p.tiles3 = next ? a->qkv_cols / kTileCols : 0;
+    p.eps = a->norm_eps;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+#ifdef TAH_CPU_EMU
+    if (a->hidden == 512) {
+        launch_chain<2, 2, 6>(p, next, st);
+        return TAH_OK;
+    }
+#endif
+    launch_chain<8, 8, 24>(p, next, st);
     return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
 }

@@ -47,6 +47,8 @@ void load_library(const std::string& path, bool allow_host) {
     bind(g.linear_pack_weight, "tah_linear_pack_weight");
     bind(g.linear_pack_rows, "tah_linear_pack_rows");
     bind(g.linear_rows, "tah_linear_rows");
+    bind(g.linear_chain_supported, "tah_linear_chain_supported");
+    bind(g.linear_chain, "tah_linear_chain");
     bind(g.fwd_masked, "tah_duo_fwd_masked");
     bind(g.bwd_masked, "tah_duo_bwd_masked");
     bind(g.decode_workspace_bytes, "tah_duo_decode_workspace_bytes");
@@ -1008,6 +1010,56 @@ optional<Tensor> linear_rows(const Tensor& w_packed, const Tensor& x_packed, int
     return y;
 }
 
+bool linear_chain_supported(int64_t rows, int64_t hidden, int64_t o_cols, int64_t ff, int64_t qkv_cols) {
+    need_lib();
+    const auto fits = [](int64_t v) { return v >= 0 && v <= 0x7fffffff; };
+    return fits(rows) && fits(hidden) && fits(o_cols) && fits(ff) && fits(qkv_cols) &&
+           g.linear_chain_supported((int32_t)rows, (int32_t)hidden, (int32_t)o_cols, (int32_t)ff, (int32_t)qkv_cols) != 0;
+}
+
+// The linear layers between two attentions of a decode step; returns the next layer's q|k|v rows (nothing without its weight).
+optional<Tensor> linear_chain(const Tensor& wo, const Tensor& wgu, const Tensor& wdown, const optional<Tensor>& wqkv, const Tensor& attn_packed,
+                              const Tensor& residual, const Tensor& mid, const Tensor& out, const Tensor& handover,
+                              const optional<Tensor>& out_packed, const Tensor& arrived, const Tensor& clear, double norm_eps) {
+    need_lib();
+    Dev d; d.see(wo); d.see(wgu); d.see(wdown); d.see(wqkv); d.see(attn_packed); d.see(residual); d.see(mid); d.see(out); d.see(handover);
+    d.see(out_packed); d.see(arrived); d.see(clear);
+    const auto rows_form = [](const Tensor& t) { return t.scalar_type() == at::kBFloat16 && t.is_contiguous() && t.numel() % 1024 == 0; };
+    TORCH_CHECK(residual.dim() == 2 && residual.size(1) > 0 && rows_form(attn_packed), "linear_chain: residual is [rows, hidden]; attn_packed a rows operand");
+    const int64_t rows = residual.size(0), hidden = residual.size(1), o_cols = attn_packed.numel() / 32, ff = wdown.numel() / hidden;
+    TORCH_CHECK(!out_packed.has_value() || packed_vec(*out_packed, 32 * hidden), "linear_chain: out_packed must be a contiguous bf16 tensor of 32 * hidden elements");
+    TORCH_CHECK(handover.scalar_type() == at::kBFloat16 && handover.is_contiguous() && 2 * handover.numel() >= TAH_LINEAR_CHAIN_HANDOVER_BYTES(hidden, ff),
+                "linear_chain: handover holds 8 * (2 * hidden + ff) bf16 elements");
+    for (const Tensor* t : {&residual, &mid, &out})
+        TORCH_CHECK(t->dim() == 2 && t->size(0) == rows && t->size(1) == hidden && t->scalar_type() == at::kBFloat16 && (t->numel() == 0 || t->stride(1) == 1),
+                    "linear_chain: residual, mid and out are bf16 [rows, hidden]");
+    TORCH_CHECK(packed_vec(wo, hidden * o_cols) && packed_vec(wgu, 2 * ff * hidden) && packed_vec(wdown, hidden * ff),
+                "linear_chain: weights must come from linear_pack_weight for these sizes");
+    int64_t qkv_cols = 0;
+    optional<Tensor> y;
+    if (wqkv.has_value()) {
+        TORCH_CHECK(wqkv->numel() % hidden == 0 && packed_vec(*wqkv, wqkv->numel()), "linear_chain: weights must come from linear_pack_weight for these sizes");
+        qkv_cols = wqkv->numel() / hidden;
+        y = at::empty({rows, qkv_cols}, residual.options());
+    }
+    for (const Tensor* t : {&arrived, &clear})
+        TORCH_CHECK(t->scalar_type() == at::kInt && t->is_contiguous() && t->numel() == TAH_LINEAR_CHAIN_WORDS, "linear_chain: arrived and clear are int32 [",
+                    TAH_LINEAR_CHAIN_WORDS, "]");
+    TORCH_CHECK(linear_chain_supported(rows, hidden, o_cols, ff, qkv_cols), "linear_chain: sizes it is not built for");
+    const auto stride = [&](const Tensor& t) { return rows > 1 ? t.stride(0) : hidden; };
+    tah_linear_chain_args a{};
+    a.wo_packed = ptr(wo); a.wgu_packed = ptr(wgu); a.wdown_packed = ptr(wdown); a.wqkv_packed = ptr(wqkv);
+    a.attn_packed = ptr(attn_packed); a.residual = ptr(residual); a.residual_row_stride = stride(residual);
+    a.mid = mptr(mid); a.mid_row_stride = stride(mid); a.out = mptr(out); a.out_row_stride = stride(out);
+    a.qkv = y.has_value() ? mptr(*y) : nullptr; a.qkv_row_stride = qkv_cols;
+    a.handover = mptr(handover); a.out_packed = out_packed.has_value() ? mptr(*out_packed) : nullptr;
+    a.rows = (int32_t)rows; a.hidden = (int32_t)hidden; a.o_cols = (int32_t)o_cols; a.ff = (int32_t)ff; a.qkv_cols = (int32_t)qkv_cols;
+    a.norm_eps = (float)norm_eps;
+    a.arrived = static_cast<int32_t*>(mptr(arrived)); a.clear = static_cast<int32_t*>(mptr(clear));
+    check_rc(g.linear_chain(&a, d.stream()), "tah_linear_chain");
+    return y;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -1048,5 +1100,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("linear_pack_weight", &linear_pack_weight);
     m.def("linear_pack_rows", &linear_pack_rows);
     m.def("linear_rows", &linear_rows);
+    m.def("linear_chain_supported", &linear_chain_supported);
+    m.def("linear_chain", &linear_chain);
     tah_ext::bind_mixers(m);
 }

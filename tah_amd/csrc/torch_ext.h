@@ -45,6 +45,8 @@ struct Api {
     Entry<decltype(&tah_linear_pack_weight)> linear_pack_weight;
     Entry<decltype(&tah_linear_pack_rows)> linear_pack_rows;
     Entry<decltype(&tah_linear_rows)> linear_rows;
+    Entry<decltype(&tah_linear_chain_supported)> linear_chain_supported;
+    Entry<decltype(&tah_linear_chain)> linear_chain;
     Entry<decltype(&tah_duo_fwd_masked)> fwd_masked;
     Entry<decltype(&tah_duo_bwd_masked)> bwd_masked;
     Entry<decltype(&tah_duo_decode_workspace_bytes)> decode_workspace_bytes;

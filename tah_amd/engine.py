@@ -454,6 +454,16 @@ class TaHDecodeEngine(DecodeEngine):
         if self.packed_linear:  # rows operands handed from kernel to kernel (32 rows each; rows past the batch stay zero)
             z = lambda n: torch.zeros(32 * n, dtype=torch.bfloat16, device=dev)
             self.xp, self.op, self.actp = z(cfg.hidden), z(cfg.hq * cfg.head_dim), z(cfg.intermediate)
+        # the linear layers between two attentions in one launch where the library takes the sizes.  Its words of arrival: every
+        # layer's launch zeroes the next layer's, the last one the first's for the next pass.
+        self.linear_chain = bool(self.packed_linear and cfg.layers > 1 and self.device.type == "cuda" and
+                                 ops.linear_chain_supported(batch, cfg.hidden, cfg.hq * cfg.head_dim, cfg.intermediate,
+                                                            (cfg.hq + 2 * cfg.hkv) * cfg.head_dim))
+        if self.linear_chain:
+            self.handover = torch.empty(8 * (2 * cfg.hidden + cfg.intermediate), dtype=torch.bfloat16, device=dev)
+            self.x_mid, *self.x_turn = [torch.zeros(batch, cfg.hidden, dtype=torch.bfloat16, device=dev) for _ in range(3)]
+            self.arrived = torch.zeros(cfg.layers, ops.LINEAR_CHAIN_WORDS, dtype=torch.int32, device=dev)
+            self.pass_open = False  # a pass has begun and not ended: the words are not to be relied on
         # the step's element-wise glue in two launches (tah_step_begin, tah_decider_tail) and the decider's first layer
         # on the linear-layer kernel, instead of some twenty torch launches; needs the packed rows
         self.fused_glue = bool(self.packed_linear and weights.lm_head_p is not None and
@@ -577,17 +587,22 @@ class TaHDecodeEngine(DecodeEngine):
         return self._rms(x, self.w.norm)
 
     def _pass_single_packed(self, x, pos, depth: int, slot_of, q_pos, q_depth, cos, sin, rows_packed: bool = False):
-        """The same pass with the four linear layers of a layer on ``ops.linear_rows``: seven launches per layer.  The
-        hidden state lives twice, row-major in ``x`` (updated in place; read by the q/k preparation for the norm
-        factor) and as rows operand in ``self.xp``; attention output and MLP activation exist as rows operands only."""
+        """The same pass with the four linear layers of a layer on ``ops.linear_rows``, or those from one attention to the next
+        in one launch (``ops.linear_chain``).  The hidden state lives twice, row-major in ``x`` (updated in place, or in
+        ``self.x_turn``; read by the q/k preparation for the norm factor) and as rows operand in ``self.xp``; attention output and MLP activation exist as rows operands only."""
         c = self.cfg
         B, H, I = x.shape[0], c.hidden, c.intermediate
         n_qkv, n_o = (c.hq + 2 * c.hkv) * c.head_dim, c.hq * c.head_dim
         x = x.contiguous()
         xp = self.xp if rows_packed else ops.linear_pack_rows(x, out=self.xp)  # rows_packed: self.xp already holds x
         self._keep_hidden(0, x)
+        chain, qkv = self.linear_chain, None
+        if chain:
+            if self.pass_open:
+                self.arrived.zero_()
+            self.pass_open = True
         for l, L in enumerate(self.w.layers):
-            q, k, v = self._split_qkv(ops.linear_rows(L["wqkv_p"], xp, B, n_qkv, H))
+            q, k, v = self._split_qkv(ops.linear_rows(L["wqkv_p"], xp, B, n_qkv, H) if qkv is None else qkv)
             cache = self.slabs1[l] if depth == 1 else self.slabs0[l]
             if self.measure_without_attention:  # timing aid: the step minus its q/k preparation and decode kernels
                 ops.linear_pack_rows(q.reshape(B, n_o), out=self.op)
@@ -608,10 +623,21 @@ class TaHDecodeEngine(DecodeEngine):
                                      norm_input=x, norm_eps=c.rms_eps)
                 _decode(qo, self.rows, q_pos, self.slabs0[l], self.slabs1[l], scale=self.scale, q_depth=q_depth,
                         static_scratch=self.static_scratch, out_packed=self.op)
+            if chain:
+                last = l + 1 == c.layers
+                x_next = self.x_turn[l % 2]
+                qkv = ops.linear_chain(L["wo_p"], L["wgu_p"], L["wdown_p"], None if last else self.w.layers[l + 1]["wqkv_p"], self.op, x,
+                                       mid=self.x_mid, out=x_next, handover=self.handover, out_packed=xp if last else None,
+                                       arrived=self.arrived[l], clear=self.arrived[0 if last else l + 1], norm_eps=c.rms_eps)
+                x = x_next
+                self._keep_hidden(l + 1, x)
+                continue
             ops.linear_rows(L["wo_p"], self.op, B, H, n_o, residual=x, out=x, out_packed=xp)
             ops.linear_rows(L["wgu_p"], xp, B, I, H, gate_up=True, out_packed=self.actp, want_out=False, norm_eps=c.rms_eps)
             ops.linear_rows(L["wdown_p"], self.actp, B, H, I, residual=x, out=x, out_packed=xp)
             self._keep_hidden(l + 1, x)
+        if chain:
+            self.pass_open = False
         return x  # before the final norm; self.xp holds the same rows as operand
 
     def _head(self, h):
@@ -892,7 +918,7 @@ class TaHDecodeEngine(DecodeEngine):
     LAST_TICKS = 8   # how often the host looks once the fastest possible row could be done
 
     def _launch_switches(self):
-        return super()._launch_switches() + (self.use_fused_glue, self.static_scratch, self.measure_without_attention, id(self.decider))
+        return super()._launch_switches() + (self.use_fused_glue, self.static_scratch, self.measure_without_attention, self.linear_chain, id(self.decider))
 
     def capture_ticks(self, eos: int, limit: int, temperature: float = 0.0, **filters):
         """The tick as two HIP graphs, one per logits buffer, after a warm-up tick whose state changes are undone."""

@@ -286,6 +286,27 @@ def linear_rows(w_packed: torch.Tensor, x_packed: torch.Tensor, rows: int, n: in
                  float(c0), float(c1))
 
 
+LINEAR_CHAIN_WORDS = 6144  # TAH_LINEAR_CHAIN_WORDS
+
+
+def linear_chain_supported(rows: int, hidden: int, o_cols: int, ff: int, qkv_cols: int) -> bool:
+    """Whether ``linear_chain`` takes these sizes."""
+    return bool(_call("linear_chain_supported", int(rows), int(hidden), int(o_cols), int(ff), int(qkv_cols)))
+
+
+def linear_chain(wo_packed, wgu_packed, wdown_packed, wqkv_packed, attn_packed, residual, *, mid, out, handover, arrived, clear,
+                 norm_eps: float, out_packed=None):
+    """The linear layers between two attentions of a decode step in one launch (``tah_linear_chain``), at most eight rows.
+
+    ``mid = residual + attn @ wo.T``; the MLP of mid's RMS-normed rows (the norm's weight sits in the gate|up weight);
+    ``out = mid + act @ wdown.T``; returns ``out @ wqkv.T`` (None without ``wqkv_packed``): the same bits as four
+    ``linear_rows`` calls.  ``residual``, ``mid`` and ``out`` bf16 [rows, hidden] are different tensors; ``handover`` bf16
+    [8 * (2 * hidden + ff)] is scratch; ``out_packed`` [32 * hidden] also receives ``out`` as a rows operand.  ``arrived`` int32 [LINEAR_CHAIN_WORDS]: zeros before the call, not
+    behind it; ``clear``: other such words, which the call zeroes (for the call that comes next on the stream)."""
+    return _call("linear_chain", wo_packed, wgu_packed, wdown_packed, wqkv_packed, attn_packed, residual, mid, out, handover,
+                 out_packed, arrived, clear, float(norm_eps))
+
+
 def greedy_workspace(rows: int, device) -> torch.Tensor:
     """What ``greedy_step`` and ``greedy_tick`` of ``rows`` rows keep between the workgroups of a row
     (``tah_greedy_workspace_bytes``), zeroed: for one call at a time, one per stream."""

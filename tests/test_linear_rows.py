@@ -306,3 +306,100 @@ def test_linear_rows_through_the_c_abi_gpu():
     _close(h.cpu(), reference(x, w, residual=res))
     assert torch.equal(unpack_rows(yp.cpu(), n), h.cpu())
     assert torch.equal(ops.linear_pack_weight(dw), wp) and torch.equal(ops.linear_pack_rows(dx), xp)
+
+
+# ── the linear layers between two attentions in one launch (tah_linear_chain) ──
+# rows on both sides of each of its kernels' row counts; q|k|v narrower than the other phases; without q|k|v
+CHAIN_CASES = [(1, 4096, False), (2, 4096, True), (3, 16, False), (4, 0, True), (5, 4096, True), (8, 4096, False), (8, 0, False)]
+
+
+def _chain_case(dev, rows, hidden, o_cols, ff, n_qkv, views, launches=2):
+    """Against the four ``linear_rows`` launches: the same bits (512 columns, on the CPU only: ``linear_rows`` adds even and odd steps
+    up together there, a neighbouring bf16 value).  ``views``: row-major tensors with strides of their own."""
+    from tah_amd import ops
+    same = torch.equal if hidden == 2048 else lambda a, b: torch.allclose(a.float(), b.float(), rtol=2.0 ** -6, atol=2.0 ** -6)
+    pack = lambda n, k, seed, gu=False: ops.linear_pack_weight(_rand(((2 if gu else 1) * n, k), seed, k ** -0.5).to(dev), gate_up=gu)
+    wo, wgu, wdown = pack(hidden, o_cols, 21), pack(ff, hidden, 22, True), pack(hidden, ff, 23)
+    wqkv = pack(n_qkv, hidden, 24) if n_qkv else None
+    empty = lambda: torch.full((rows, hidden + 64), 7.0, dtype=BF, device=dev)[:, 8:hidden + 8] if views else torch.full((rows, hidden), 7.0, dtype=BF, device=dev)
+    form = lambda n: torch.full((32 * n,), 7.0, dtype=BF, device=dev)
+    words = torch.zeros(2, ops.LINEAR_CHAIN_WORDS, dtype=torch.int32, device=dev)
+    words[1] = 5  # what the launch before left there
+    for i in range(launches):
+        attn, res = ops.linear_pack_rows(_rand((rows, o_cols), 31 + i).to(dev)), empty()
+        res.copy_(_rand((rows, hidden), 41 + i))
+        before = res.clone()
+        mid, out, between, out_p = empty(), empty(), torch.full((8 * (2 * hidden + ff),), 7.0, dtype=BF, device=dev), form(hidden)
+        got = ops.linear_chain(wo, wgu, wdown, wqkv, attn, res, mid=mid, out=out, handover=between, out_packed=out_p if i != 1 else None,
+                               arrived=words[i % 2], clear=words[1 - i % 2], norm_eps=1e-6)
+        x, xp, ap = before.clone(), form(hidden), form(ff)
+        ops.linear_rows(wo, attn, rows, hidden, o_cols, residual=x, out=x, out_packed=xp)
+        assert same(mid, x)
+        ops.linear_rows(wgu, xp, rows, ff, hidden, gate_up=True, out_packed=ap, want_out=False, norm_eps=1e-6)
+        ops.linear_rows(wdown, ap, rows, hidden, ff, residual=x, out=x, out_packed=xp)
+        assert same(out, x) and (i == 1 or same(out_p, xp)) and torch.equal(res, before)
+        if n_qkv:
+            assert same(got, ops.linear_rows(wqkv, xp, rows, n_qkv, hidden))
+        else:
+            assert got is None
+        assert not words[1 - i % 2].any()
+        assert words[i % 2].view(3, 64, 32)[:2, :hidden // 32, 0].eq(15).all()
+
+
+def _chain_errors(dev):
+    from tah_amd import ops
+    from tah_amd._capi import TahDuoError
+    z = lambda *s: torch.zeros(*s, dtype=BF, device=dev)
+    w = lambda n: torch.zeros(n, dtype=torch.int32, device=dev)
+    good = dict(mid=z(2, 2048), out=z(2, 2048), handover=z(8 * (2 * 2048 + 6144)), out_packed=z(32 * 2048),
+                arrived=w(ops.LINEAR_CHAIN_WORDS), clear=w(ops.LINEAR_CHAIN_WORDS), norm_eps=1e-6)
+    head = (z(2048 * 2048), z(2 * 6144 * 2048), z(2048 * 6144), None, z(32 * 2048))
+    res = z(2, 2048)
+    for bad in (dict(mid=res), dict(out=res), dict(out=good["mid"]), dict(out_packed=head[4]), dict(handover=head[4]), dict(handover=z(8 * 6144)),
+                dict(clear=good["arrived"]), dict(arrived=w(64))):
+        with pytest.raises((TahDuoError, RuntimeError)):
+            ops.linear_chain(*head, res, **{**good, **bad})
+    with pytest.raises((TahDuoError, RuntimeError)):
+        ops.linear_chain(*head, z(9, 2048), **{**good, "mid": z(9, 2048), "out": z(9, 2048)})
+    assert not ops.linear_chain_supported(9, 2048, 2048, 6144, 0) and not ops.linear_chain_supported(1, 2048, 2048, 6144, 8)
+    assert not ops.linear_chain_supported(1, 1024, 2048, 6144, 0) and not ops.linear_chain_supported(1, 2048, 2048, 6144, 16 * 257)
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_linear_chain_on_the_cpu_shim():
+    """Workgroups run one after another there: the first one's waits all end by computing the others' tiles itself."""
+    with emu_util.emulated():
+        _chain_errors("cpu")
+        _chain_case("cpu", 7, 512, 512, 1536, 16, True, launches=1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n_qkv,views", CHAIN_CASES)
+def test_linear_chain_gpu(rows, n_qkv, views):
+    _chain_case("cuda", rows, 2048, 2048, 6144, n_qkv, views, launches=5)
+    _chain_errors("cuda")
+
+
+@pytest.mark.gpu
+def test_linear_chains_side_by_side_gpu():
+    """Two streams' launches share the compute units: whichever workgroups are resident, both finish with the same bits."""
+    from tah_amd import ops
+    pack = lambda n, k, seed, gu=False: ops.linear_pack_weight(_rand(((2 if gu else 1) * n, k), seed, k ** -0.5).cuda(), gate_up=gu)
+    weights = pack(2048, 2048, 51), pack(6144, 2048, 52, True), pack(2048, 6144, 53), pack(4096, 2048, 54)
+    attn, res = ops.linear_pack_rows(_rand((2, 2048), 55).cuda()), _rand((2, 2048), 56).cuda()
+    z = lambda *s: torch.zeros(*s, dtype=BF, device="cuda")
+    sets = [dict(mid=z(2, 2048), out=z(2, 2048), handover=z(8 * (2 * 2048 + 6144))) for _ in range(3)]
+    words = torch.zeros(3, 2, ops.LINEAR_CHAIN_WORDS, dtype=torch.int32, device="cuda")
+    run = lambda s, i: ops.linear_chain(*weights, attn, res, arrived=words[s][i % 2], clear=words[s][1 - i % 2], norm_eps=1e-6, **sets[s])
+    want = run(2, 0)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    got = [[], []]
+    for i in range(50):
+        for s, stream in enumerate(streams):
+            with torch.cuda.stream(stream):
+                got[s].append(run(s, i))
+    torch.cuda.synchronize()
+    for one in got:
+        assert all(torch.equal(q, want) for q in one)
+    assert torch.equal(sets[0]["out"], sets[2]["out"]) and torch.equal(sets[1]["out"], sets[2]["out"])
