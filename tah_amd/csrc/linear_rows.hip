@@ -66,6 +66,8 @@ struct LinParams {
     int32_t yp_col_step;    // columns a product's packed result is moved by (results side by side in one rows form)
     const int32_t* select;  // run only products whose index is listed here, or null
     int32_t n_select;
+    int32_t grid_y, batches; // workgroups along y: one per product or, by_list, one per entry of a list that is shorter than the
+    bool by_list;            // products are: 7 of 8 of 64 experts' workgroups would start only to leave (1.7 us of 11 a launch at one row)
     float c0, c1;           // constants of the activation
 };
 
@@ -112,11 +114,18 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
     __shared__ float ssum[EPI == kPlainLayerNorm ? kLinWaves : 1][16 * NH];
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int c = lane % 16, kg = lane / 16;
-    const int batch = blockIdx.y;
+    int batch = blockIdx.y;
     if (p.select) {  // (every wave looks for itself: the answer is the same in all of them)
         bool hit = false;
-        for (int i = lane; i < p.n_select; i += kWave) hit |= p.select[i] == batch;
-        if (__ballot(hit) == 0) return;
+        if (p.by_list) {
+            const int at = batch;
+            batch = p.select[at];
+            for (int i = lane; i < at; i += kWave) hit |= p.select[i] == batch;  // listed before: that workgroup's
+            if (__ballot(hit) != 0 || batch < 0 || batch >= p.batches) return;
+        } else {
+            for (int i = lane; i < p.n_select; i += kWave) hit |= p.select[i] == batch;
+            if (__ballot(hit) == 0) return;
+        }
     }
     const bf16x8* const pw = p.w + batch * (p.w_bs / 8);
     const bf16x8* const px = p.x + batch * (p.x_bs / 8);
@@ -1040,8 +1049,8 @@ void launch_wide(LinParams& p, int groups, hipStream_t st) {
 
 // few rows: the rows operand folded as far as their number allows
 template <int NC, int CH, int EPI, int PW, bool H8>
-void launch_folded(const LinParams& p, int workgroups, int batch, hipStream_t st) {
-    const dim3 grid(workgroups, batch), block(kLinThreads);
+void launch_folded(const LinParams& p, int workgroups, hipStream_t st) {
+    const dim3 grid(workgroups, p.grid_y), block(kLinThreads);
     if constexpr (PW > 0 && NC != 2) {
         const auto run = [&](auto fold) { hipLaunchKernelGGL((linear_rows_kernel<NC, CH, EPI, PW, 1, H8, decltype(fold)::value>), grid, block, 0, st, p); };
         if constexpr (CH == PW) {
@@ -1062,18 +1071,18 @@ void launch(LinParams& p, int groups, int batch, hipStream_t st) {
         // 5.5 us, where K = 4096 gains 7.6 -> 7.0 and K = 6144 9.5 -> 8.8)
         if (groups * batch < kSplitRowsBelowGroups && (p.rows <= 8 || (p.rows <= 16 && PW >= 16))) {
             p.groups = 2 * groups;
-            launch_folded<1, PW, kPlain, PW, true>(p, p.groups, batch, st);
+            launch_folded<1, PW, kPlain, PW, true>(p, p.groups, st);
             return;
         }
     }
     if (NC != 2 && PW > 0 && p.rows <= 8)  // (two tiles share the operand: nothing to gain)
-        launch_folded<NC, CH, EPI, PW, false>(p, groups, batch, st);
+        launch_folded<NC, CH, EPI, PW, false>(p, groups, st);
     else if (p.rows <= 16)
-        hipLaunchKernelGGL((linear_rows_kernel<NC, CH, EPI, PW, 1>), dim3(groups, batch), dim3(kLinThreads), 0, st, p);
+        hipLaunchKernelGGL((linear_rows_kernel<NC, CH, EPI, PW, 1>), dim3(groups, p.grid_y), dim3(kLinThreads), 0, st, p);
     else if (groups * batch < kSplitRowsBelowGroups)
-        hipLaunchKernelGGL((linear_rows_kernel<NC, CH, EPI, PW, 1>), dim3(2 * groups, batch), dim3(kLinThreads), 0, st, p);
+        hipLaunchKernelGGL((linear_rows_kernel<NC, CH, EPI, PW, 1>), dim3(2 * groups, p.grid_y), dim3(kLinThreads), 0, st, p);
     else
-        hipLaunchKernelGGL((linear_rows_kernel<NC, CH, EPI, PW, 2>), dim3(groups, batch), dim3(kLinThreads), 0, st, p);
+        hipLaunchKernelGGL((linear_rows_kernel<NC, CH, EPI, PW, 2>), dim3(groups, p.grid_y), dim3(kLinThreads), 0, st, p);
 }
 
 }  // namespace
@@ -1158,6 +1167,9 @@ extern "C" int tah_linear_rows(const tah_linear_rows_args* a, tah_stream_t strea
     p.yp_col_step = a->out_packed_col_step;
     p.select = a->n_select > 0 ? a->batch_select : nullptr;
     p.n_select = a->n_select;
+    p.batches = batch;
+    p.by_list = p.select && a->n_select < batch;
+    p.grid_y = p.by_list ? a->n_select : batch;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int steps = a->k / kStepK;
     const int pw = steps % kLinWaves == 0 ? steps / kLinWaves : 0;  // compile-time K for the sizes of the end-to-end model

@@ -403,3 +403,34 @@ def test_linear_chains_side_by_side_gpu():
     for one in got:
         assert all(torch.equal(q, want) for q in one)
     assert torch.equal(sets[0]["out"], sets[2]["out"]) and torch.equal(sets[1]["out"], sets[2]["out"])
+
+
+# ── products chosen by a list shorter than the products (a workgroup per entry) and by a longer one ──
+def _select_case(dev, rows, n, k, gate_up, lists):
+    from tah_amd import ops
+    batch = 8
+    w = torch.cat([ops.linear_pack_weight(_rand(((2 if gate_up else 1) * n, k), 61 + b, k ** -0.5).to(dev), gate_up=gate_up) for b in range(batch)])
+    xp = ops.linear_pack_rows(_rand((rows, k), 60).to(dev))
+    run = lambda **kw: ops.linear_rows(w, xp, rows, n, k, gate_up=gate_up, batch=batch, shared_rows=True, **kw)
+    want = run()
+    for chosen in lists:
+        out = torch.full((batch, rows, n), 5.0, dtype=BF, device=dev)
+        run(out=out, select=torch.tensor(chosen, dtype=torch.int32, device=dev))
+        for b in range(batch):
+            assert torch.equal(out[b], want[b]) if b in chosen else bool((out[b] == 5.0).all())
+
+
+# one entry, repeats, entries that name no product; as many entries as products and more
+SELECT_LISTS = [[7], [5, 0, 5, 2, 0], [-1, 3, 8, 1 << 30], list(range(7)), [4] * 8, [6, 1] * 40]
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_linear_rows_select_on_the_cpu_shim():
+    with emu_util.emulated():
+        _select_case("cpu", 3, 16, 64, False, SELECT_LISTS[1:3])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n,k,gate_up", [(1, 768, 2048, True), (9, 48, 2048, True), (20, 96, 320, True), (1, 2048, 768, False), (8, 64, 2048, False), (32, 32, 96, False)])
+def test_linear_rows_select_gpu(rows, n, k, gate_up):
+    _select_case("cuda", rows, n, k, gate_up, SELECT_LISTS)
