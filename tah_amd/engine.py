@@ -586,6 +586,13 @@ class TaHDecodeEngine(DecodeEngine):
             self._keep_hidden(l + 1, x)
         return self._rms(x, self.w.norm)
 
+    def _close_pass(self) -> None:
+        """Zeroes the words of arrival if a pass ended between two of its launches (an exception): before the next pass, and
+        before graphs, which hold passes that began with zeros, are replayed."""
+        if self.linear_chain and self.pass_open:
+            self.arrived.zero_()
+            self.pass_open = False
+
     def _pass_single_packed(self, x, pos, depth: int, slot_of, q_pos, q_depth, cos, sin, rows_packed: bool = False):
         """The same pass with the four linear layers of a layer on ``ops.linear_rows``, or those from one attention to the next
         in one launch (``ops.linear_chain``).  The hidden state lives twice, row-major in ``x`` (updated in place, or in
@@ -598,8 +605,7 @@ class TaHDecodeEngine(DecodeEngine):
         self._keep_hidden(0, x)
         chain, qkv = self.linear_chain, None
         if chain:
-            if self.pass_open:
-                self.arrived.zero_()
+            self._close_pass()
             self.pass_open = True
         for l, L in enumerate(self.w.layers):
             q, k, v = self._split_qkv(ops.linear_rows(L["wqkv_p"], xp, B, n_qkv, H) if qkv is None else qkv)
@@ -851,6 +857,7 @@ class TaHDecodeEngine(DecodeEngine):
         generator is left as the step-wise loop leaves it; such an engine runs other filters step-wise by default.  On
         other engines sampled tokens come from the same per-row distributions but from other random draws (a tick draws
         for every row, a step once per token).  ``check_every`` counts ticks there."""
+        self._close_pass()
         self._check_room(max_new_tokens)
         dev = self.device
         greedy_fused = temperature <= 0.0 and self.fused_greedy and self.cfg.vocab % 8 == 0

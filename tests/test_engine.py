@@ -661,3 +661,32 @@ def test_engine_at_the_end_to_end_shape_gpu():
     print(f"end-to-end shape, error / logit range: rows with one iteration max {plain:.3e}; rows with two: max {second[0]:.3e}, "
           f"mean {second[1]:.3e}", flush=True)
     assert plain <= 3e-2 and second[0] <= 0.4 and second[1] <= 6e-2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [1, 3, 8])
+def test_linear_layers_in_one_launch_change_no_bit_gpu(batch):
+    """Eager and replayed, also behind a pass that ended between two launches (its words of arrival are still set)."""
+    import torch
+    from tah_amd.engine import EngineConfig, TaHDecodeEngine, Weights
+
+    w = Weights.random_init(EngineConfig(layers=3, vocab=4096), "cuda", seed=3)
+    g = torch.Generator().manual_seed(batch)
+    lens = [17 + 9 * i for i in range(batch)]
+    ids = torch.randint(0, 4096, (sum(lens),), generator=g).cuda()
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+
+    def run(chain, use_graph, broken=False):
+        e = TaHDecodeEngine(w, batch, 128)
+        assert e.linear_chain
+        e.linear_chain = chain
+        first, _ = e.prefill(ids, cu, calibrate=0.2)
+        if broken:
+            e.arrived.fill_(15)
+            e.pass_open = True
+        tokens = e.generate(first, 20, use_graph=use_graph)
+        return [tokens] + [s.k for s in e.slabs0] + [s.v for s in e.slabs1]
+
+    want = run(False, True)
+    for chain, use_graph, broken in ((True, True, False), (True, False, False), (True, True, True), (True, False, True)):
+        assert all(torch.equal(a, b) for a, b in zip(run(chain, use_graph, broken), want)), (chain, use_graph, broken)
