@@ -525,8 +525,8 @@ int tah_linear_rows(const tah_linear_rows_args* args, tah_stream_t stream);
  * residual, the next layer's q|k|v), the same bits.  wqkv_packed NULL: without the last one.  Sizes: tah_linear_chain_supported.
  * `handover`: TAH_LINEAR_CHAIN_HANDOVER_BYTES of scratch.
  * `arrived`: TAH_LINEAR_CHAIN_WORDS words that are zero when the launch starts and not zero behind it; `clear`: other such
- * words, which the launch sets to zero (those of the launch that comes next on the stream).  No two results may overlap
- * each other, the residual or attn_packed (TAH_E_SHAPE). */
+ * words, which the launch sets to zero (those of the launch that comes next on the stream; rows == 0 does that and nothing
+ * else).  No two results may overlap each other, the residual or attn_packed (TAH_E_SHAPE). */
 #define TAH_LINEAR_CHAIN_TILES 256
 #define TAH_LINEAR_CHAIN_WORDS (3 * TAH_LINEAR_CHAIN_TILES * 8)
 #define TAH_LINEAR_CHAIN_HANDOVER_BYTES(hidden, ff) (16 * (2 * (hidden) + (ff)))

@@ -983,6 +983,11 @@ __global__ __launch_bounds__(kChainThreads) void linear_chain_kernel(const Chain
     }
 }
 
+// what is left of a launch without rows: the words of the next one
+__global__ __launch_bounds__(kLinThreads) void linear_chain_clear_kernel(int32_t* clear) {
+    for (int i = threadIdx.x; i < TAH_LINEAR_CHAIN_WORDS; i += kLinThreads) clear[i] = 0;
+}
+
 template <int PWO, int PWH, int PWF>
 void launch_chain(const ChainParams& p, bool next, hipStream_t st) {
     int tiles = p.tiles0 > p.tiles1 ? p.tiles0 : p.tiles1;
@@ -1229,7 +1234,12 @@ extern "C" int tah_linear_chain_supported(int32_t rows, int32_t hidden, int32_t 
 extern "C" int tah_linear_chain(const tah_linear_chain_args* a, tah_stream_t stream) {
     using namespace tah;
     if (!a) return TAH_E_NULL;
-    if (a->rows == 0) return TAH_OK;
+    if (a->rows == 0) {
+        if (!a->clear) return TAH_OK;
+        if (reinterpret_cast<uintptr_t>(a->clear) % sizeof(int32_t) != 0) return TAH_E_ALIGN;
+        hipLaunchKernelGGL(linear_chain_clear_kernel, dim3(1), dim3(kLinThreads), 0, static_cast<hipStream_t>(stream), a->clear);
+        return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
+    }
     const bool next = a->wqkv_packed != nullptr;
     if (!tah_linear_chain_supported(a->rows, a->hidden, a->o_cols, a->ff, next ? a->qkv_cols : 0) || (next && a->qkv_cols == 0)) return TAH_E_SHAPE;
     const void* needed[] = {a->wo_packed, a->wgu_packed, a->wdown_packed, a->attn_packed, a->residual, a->mid, a->out, a->handover, a->arrived, a->clear, next ? a->qkv : a->out, next ? a->wqkv_packed : a->out};

@@ -366,6 +366,17 @@ def _chain_errors(dev):
 
 
 @pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_linear_chain_without_rows_clears_the_next_words_on_the_cpu_shim():
+    """The launch behind an empty one finds zeros too."""
+    from tah_amd import _capi, ops
+    words = torch.full((2, ops.LINEAR_CHAIN_WORDS), 15, dtype=torch.int32)
+    with emu_util.emulated() as lib:
+        assert lib.tah_linear_chain(ctypes.byref(_capi.LinearChainArgs(arrived=words[0].data_ptr(), clear=words[1].data_ptr())), None) == 0
+        assert lib.tah_linear_chain(ctypes.byref(_capi.LinearChainArgs()), None) == 0
+    assert bool((words[0] == 15).all()) and not words[1].any()
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
 def test_linear_chain_on_the_cpu_shim():
     """Workgroups run one after another there: the first one's waits all end by computing the others' tiles itself."""
     with emu_util.emulated():
