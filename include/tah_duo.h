@@ -526,7 +526,7 @@ int tah_linear_rows(const tah_linear_rows_args* args, tah_stream_t stream);
  * `handover`: TAH_LINEAR_CHAIN_HANDOVER_BYTES of scratch.
  * `arrived`: TAH_LINEAR_CHAIN_WORDS words that are zero when the launch starts and not zero behind it; `clear`: other such
  * words, which the launch sets to zero (those of the launch that comes next on the stream; rows == 0 does that and nothing
- * else).  No two results may overlap each other, the residual or attn_packed (TAH_E_SHAPE). */
+ * else).  No two results may overlap each other, and none the residual, attn_packed or a weight (TAH_E_SHAPE). */
 #define TAH_LINEAR_CHAIN_TILES 256
 #define TAH_LINEAR_CHAIN_WORDS (3 * TAH_LINEAR_CHAIN_TILES * 8)
 #define TAH_LINEAR_CHAIN_HANDOVER_BYTES(hidden, ff) (16 * (2 * (hidden) + (ff)))

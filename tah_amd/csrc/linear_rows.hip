@@ -1261,7 +1261,10 @@ extern "C" int tah_linear_chain(const tah_linear_chain_args* a, tah_stream_t str
                              {reinterpret_cast<const char*>(a->arrived), word_bytes}, {reinterpret_cast<const char*>(a->clear), word_bytes},
                              a->out_packed ? Range{static_cast<const char*>(a->out_packed), 64 * (int64_t)a->hidden} : none,
                              next ? rows_of(a->qkv, a->qkv_row_stride, a->qkv_cols) : none};
-    const Range read[] = {rows_of(a->residual, a->residual_row_stride, a->hidden), {static_cast<const char*>(a->attn_packed), 64 * (int64_t)a->o_cols}};
+    const auto weight_of = [](const void* w, int64_t n, int64_t k) { return Range{static_cast<const char*>(w), 2 * n * k}; };
+    const Range read[] = {rows_of(a->residual, a->residual_row_stride, a->hidden), {static_cast<const char*>(a->attn_packed), 64 * (int64_t)a->o_cols},
+                          weight_of(a->wo_packed, a->hidden, a->o_cols), weight_of(a->wgu_packed, 2 * (int64_t)a->ff, a->hidden),
+                          weight_of(a->wdown_packed, a->hidden, a->ff), next ? weight_of(a->wqkv_packed, a->qkv_cols, a->hidden) : none};
     const auto meet = [](const Range& x, const Range& y) { return x.bytes > 0 && y.bytes > 0 && x.at < y.at + y.bytes && y.at < x.at + x.bytes; };
     for (int i = 0; i < 7; ++i) {
         for (int j = i + 1; j < 7; ++j)

@@ -377,6 +377,21 @@ def test_linear_chain_without_rows_clears_the_next_words_on_the_cpu_shim():
 
 
 @pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+@pytest.mark.parametrize("which", range(4))
+def test_linear_chain_refuses_results_on_a_weight_on_the_cpu_shim(which):
+    """A late workgroup reads its weights after others' results are stored: on the last rows of any of them."""
+    from tah_amd import ops
+    from tah_amd._capi import TahDuoError
+    z = lambda *s: torch.zeros(*s, dtype=BF)
+    weights = (z(512 * 512), z(2 * 1536 * 512), z(512 * 1536), z(16 * 512))
+    words = torch.zeros(2, ops.LINEAR_CHAIN_WORDS, dtype=torch.int32)
+    with emu_util.emulated():
+        with pytest.raises((TahDuoError, RuntimeError)):
+            ops.linear_chain(*weights, z(32 * 512), z(1, 512), mid=z(1, 512), out=weights[which][-512:].view(1, 512),
+                             handover=z(8 * (2 * 512 + 1536)), arrived=words[0], clear=words[1], norm_eps=1e-6)
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
 def test_linear_chain_on_the_cpu_shim():
     """Workgroups run one after another there: the first one's waits all end by computing the others' tiles itself."""
     with emu_util.emulated():
