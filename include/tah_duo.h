@@ -39,7 +39,7 @@
 extern "C" {
 #endif
 
-#define TAH_DUO_ABI_VERSION 10
+#define TAH_DUO_ABI_VERSION 11
 
 enum {
     TAH_OK = 0,
@@ -541,6 +541,7 @@ typedef struct tah_linear_chain_args {
     int32_t rows, hidden, o_cols, ff, qkv_cols;
     float norm_eps;
     int32_t *arrived, *clear;
+    int32_t polls;            /* a workgroup that has looked this often for the others' tiles computes what is missing; 0: the library's number */
 } tah_linear_chain_args;
 int tah_linear_chain_supported(int32_t rows, int32_t hidden, int32_t o_cols, int32_t ff, int32_t qkv_cols);
 int tah_linear_chain(const tah_linear_chain_args* args, tah_stream_t stream);

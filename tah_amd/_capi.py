@@ -8,7 +8,7 @@ from __future__ import annotations
 
 import ctypes as C
 
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 c_void_p, c_int32, c_int64, c_float = C.c_void_p, C.c_int32, C.c_int64, C.c_float
 
@@ -133,7 +133,7 @@ class LinearChainArgs(C.Structure):
         ("handover", c_void_p), ("out_packed", c_void_p),
         ("residual_row_stride", c_int64), ("mid_row_stride", c_int64), ("out_row_stride", c_int64), ("qkv_row_stride", c_int64),
         ("rows", c_int32), ("hidden", c_int32), ("o_cols", c_int32), ("ff", c_int32), ("qkv_cols", c_int32), ("norm_eps", c_float),
-        ("arrived", c_void_p), ("clear", c_void_p),
+        ("arrived", c_void_p), ("clear", c_void_p), ("polls", c_int32),
     ]
 
 

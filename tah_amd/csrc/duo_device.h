@@ -37,7 +37,10 @@ typedef __attribute__((address_space(3))) int lds_int;
 template <class T> inline void device_store(T* p, T v) { __atomic_store(p, &v, __ATOMIC_SEQ_CST); }
 template <class T> inline T device_load(const T* p) { T v; __atomic_load(const_cast<T*>(p), &v, __ATOMIC_SEQ_CST); return v; }
 inline int device_add(int32_t* p, int v) { return __atomic_fetch_add(p, v, __ATOMIC_SEQ_CST); }
-inline void device_or(uint32_t* p, uint32_t v) { __atomic_fetch_or(p, v, __ATOMIC_SEQ_CST); }
+inline void device_or(uint32_t* p, uint32_t v) {  // (one thread of a block calls it)
+    __atomic_fetch_or(p, v, __ATOMIC_SEQ_CST);
+    emu::g_ors.push_back(p);
+}
 inline void device_max(unsigned long long* p, unsigned long long v) {
     for (unsigned long long now = device_load(p); now < v && !__atomic_compare_exchange_n(p, &now, v, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST);) {}
 }

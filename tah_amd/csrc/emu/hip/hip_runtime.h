@@ -91,8 +91,14 @@ extern thread_local WaveCtx* t_wave;
 extern thread_local int t_lane;
 extern dim3 g_blockDim, g_gridDim;
 extern BlockCtx* g_block;
+// For tests of kernels whose blocks wait for each other: launches run blocks first ... first + count - 1 (along x) only, and the
+// addresses of the words that device_or was called on, in order.
+extern unsigned g_first_block, g_block_count;
+extern std::vector<const void*> g_ors;
 
 #ifdef TAH_EMU_IMPL
+unsigned g_first_block = 0, g_block_count = ~0u;
+std::vector<const void*> g_ors;
 thread_local emu_idx t_threadIdx, t_blockIdx;
 thread_local WaveCtx* t_wave;
 thread_local int t_lane;
@@ -135,7 +141,7 @@ void launch(K kernel, dim3 grid, dim3 block, size_t shmem, Args... args) {
         t_lane = tid % WAVE;
         for (unsigned bz = 0; bz < grid.z; ++bz)
             for (unsigned by = 0; by < grid.y; ++by)
-                for (unsigned bx = 0; bx < grid.x; ++bx) {
+                for (unsigned bx = g_first_block; bx < grid.x && bx - g_first_block < g_block_count; ++bx) {
                     t_blockIdx = {bx, by, bz};
                     pthread_barrier_wait(&ctx.bar);
                     kernel(args...);

@@ -566,10 +566,15 @@ __global__ __launch_bounds__(kLinThreads) void linear_wide_kernel(const LinParam
 //    waits for the other workgroups, so that no wait for a store or a flag stands behind the weights' loads.
 //  * A tile's results and then its bit in `arrived` are stored with device_store, past the XCDs' own L2 caches; readers use
 //    device_load.  No fence: that would write back and invalidate the L2.
-//  * Every wait ends, whatever is resident: a workgroup that has waited kChainPolls polls computes missing tiles itself.  All that
+//  * Every wait ends, whatever is resident: a workgroup that has waited kChainLook polls looks which of the missing tiles belong to
+//    workgroups that have not begun (another stream's work holds their compute units) and computes one of them after the other; after
+//    kChainPolls polls it computes whatever is missing.  Those that wait start at different tiles (chain_pick).  All that
 //    such a tile reads is there (the phase before it is complete, or the waiting workgroup would not be here), and its
-//    result is the same bits whoever stores it and however often, because no phase's result lies on another phase's
-//    operands (tah_linear_chain refuses such calls).  So one workgroup alone would finish the launch.
+//    result is the same bits whoever stores it and however often, because no result lies on an operand or on another
+//    result (tah_linear_chain refuses such calls).  So one workgroup alone would finish the launch.
+//    Two engines of eight layers on two streams, a tick of each: 480 us at one row (454 as four launches a layer), 557 to 609 at
+//    eight (480); one such engine alone 290 and 324 (330 and 350).  When every workgroup waited its 128 polls and all took the same
+//    tile: 483 to 573 and 672 to 1275.  kChainLook = 3, 5, 16: the same within those ranges.
 //  * `arrived` is zero at the start; the words of the next launch (`clear`) are zeroed on the way.
 constexpr int kChainTiles = TAH_LINEAR_CHAIN_TILES;  // tiles of a phase at most
 // `arrived`: a bit per tile, four to a word, every word on a line of its own: a line's writes take their turns among the reads of
@@ -577,12 +582,13 @@ constexpr int kChainTiles = TAH_LINEAR_CHAIN_TILES;  // tiles of a phase at most
 constexpr int kChainBits = 4, kChainLine = 32, kChainPhaseWords = kChainTiles / kChainBits * kChainLine;
 static_assert(3 * kChainPhaseWords == TAH_LINEAR_CHAIN_WORDS, "header");
 constexpr int kChainThreads = kLinThreads + kWave;
+constexpr int kChainBegun = 1;    // word of a line, phase 0: the workgroups of these tiles have begun
 #ifdef TAH_CPU_EMU
-constexpr int kChainPolls = 2;  // (workgroups run one after another there)
+constexpr int kChainPolls = 2, kChainLook = 1;  // (workgroups run one after another there)
 #else
 constexpr int kChainPolls = 128;  // about 150 us: several times a whole launch
+constexpr int kChainLook = 8;     // about 9 us: twice what a hand-over takes
 #endif
-
 constexpr int kChainSleep = 1;    // x 64 cycles between polls
 
 struct ChainParams {
@@ -595,7 +601,7 @@ struct ChainParams {
     int64_t res_rs, mid_rs, out_rs, y_rs;
     uint32_t* arrived;
     int32_t* clear;
-    int32_t rows, tiles0, tiles1, tiles2, tiles3;
+    int32_t rows, tiles0, tiles1, tiles2, tiles3, polls;
     float eps;
 };
 
@@ -709,6 +715,31 @@ struct ChainTile {
         }
     }
 };
+
+// One of the tiles that `take` names (a lane's kChainBits of them), -1: none.  Workgroups that see the same ones take different ones as
+// far as there are any, so that what is missing gets less by as many tiles as there are workgroups that wait (each the first one: they
+// all computed the same tile, a hundred missing ones took a hundred turns).
+__device__ __forceinline__ int chain_pick(uint32_t take) {
+    unsigned long long has[kChainBits];
+    int total = 0;
+#pragma unroll
+    for (int b = 0; b < kChainBits; ++b) {
+        has[b] = __ballot((take >> b & 1u) != 0);
+        total += __builtin_popcountll(has[b]);
+    }
+    if (total == 0) return -1;
+    int nth = (int)blockIdx.x % total, tile = -1;
+#pragma unroll
+    for (int b = 0; b < kChainBits; ++b) {
+        const int n = __builtin_popcountll(has[b]);
+        if (tile < 0 && nth < n) {
+            for (int i = 0; i < nth; ++i) has[b] &= has[b] - 1;
+            tile = kChainBits * __builtin_ctzll(has[b]) + b;
+        }
+        nth -= n;
+    }
+    return tile;
+}
 
 // LDS between the waves of a workgroup: loads from memory stay on their way across it
 __device__ __forceinline__ void chain_barrier() {
@@ -831,6 +862,7 @@ __global__ __launch_bounds__(kChainThreads) void linear_chain_kernel(const Chain
     typedef __attribute__((__vector_size__(2 * sizeof(float)))) float f32x2;
     typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
     typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
+    if (lane == 0) device_or(p.arrived + tile / kChainBits * kChainLine + kChainBegun, 1u << (tile % kChainBits));
     for (int i = (int)blockIdx.x * kWave + lane; i < TAH_LINEAR_CHAIN_WORDS; i += (int)gridDim.x * kWave) p.clear[i] = 0;
     // rows past the last one are zeros in the rows form that stays
     if (p.out_packed && tile < p.tiles2 && lane >= p.rows && lane < kLinRows) p.out_packed[packed_rows_unit(lane, 8 * tile)] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
@@ -923,23 +955,26 @@ __global__ __launch_bounds__(kChainThreads) void linear_chain_kernel(const Chain
         if (kNext) announce(2, of);
     };
     // until all tiles of a phase have arrived; a tile that does not come is computed here
+    int look = kChainLook;
     auto wait = [&](int phase, int tiles, auto finish) __attribute__((always_inline)) {
         // a word per lane
         const int first = kChainBits * lane, mine = tiles - first < kChainBits ? tiles - first : kChainBits;
         const uint32_t* const word = p.arrived + phase * kChainPhaseWords + lane * kChainLine;
         uint32_t absent = mine > 0 ? (1u << mine) - 1u : 0u;
-        for (int polls = 0;;) {
+        for (int polls = 1;; ++polls) {
             if (absent != 0) absent &= ~device_load(word);  // (a word that is complete is not read again: reads are in the writers' way)
-            int missing = absent != 0 ? first + __builtin_ctz(absent) : -1;
-            const unsigned long long some = __ballot(missing >= 0);
-            if (some == 0) break;
-            if (++polls >= kChainPolls) {
-                missing = __shfl(missing, __builtin_ctzll(some));
+            if (__ballot(absent != 0) == 0) break;
+            uint32_t take = 0;
+            if (polls >= p.polls) take = absent;
+            else if (polls >= look && absent != 0) take = absent & ~device_load(p.arrived + lane * kChainLine + kChainBegun);
+            const int missing = chain_pick(take);
+            if (missing >= 0) {
                 if (lane == 0) command = missing;
                 chain_barrier();
                 chain_barrier();
                 finish(missing);
-                polls = kChainPolls - 1;  // (the others of its kind are late as well)
+                if (lane == missing / kChainBits) absent &= ~(1u << (missing % kChainBits));  // (the word may not say so yet)
+                look = 1;  // (workgroups have not begun: looked for at once from now on)
             } else {
                 TAH_SLEEP(kChainSleep);
             }
@@ -1296,6 +1331,7 @@ extern "C" int tah_linear_chain(const tah_linear_chain_args* a, tah_stream_t str
     p.tiles0 = p.tiles2 = a->hidden / 8;
     p.tiles1 = a->ff / kGroup24;
     p.tiles3 = next ? a->qkv_cols / kTileCols : 0;
+    p.polls = a->polls > 0 ? a->polls : kChainPolls;
     p.eps = a->norm_eps;
     hipStream_t st = static_cast<hipStream_t>(stream);
 #ifdef TAH_CPU_EMU

@@ -1020,7 +1020,7 @@ bool linear_chain_supported(int64_t rows, int64_t hidden, int64_t o_cols, int64_
 // The linear layers between two attentions of a decode step; returns the next layer's q|k|v rows (nothing without its weight).
 optional<Tensor> linear_chain(const Tensor& wo, const Tensor& wgu, const Tensor& wdown, const optional<Tensor>& wqkv, const Tensor& attn_packed,
                               const Tensor& residual, const Tensor& mid, const Tensor& out, const Tensor& handover,
-                              const optional<Tensor>& out_packed, const Tensor& arrived, const Tensor& clear, double norm_eps) {
+                              const optional<Tensor>& out_packed, const Tensor& arrived, const Tensor& clear, double norm_eps, int64_t polls) {
     need_lib();
     Dev d; d.see(wo); d.see(wgu); d.see(wdown); d.see(wqkv); d.see(attn_packed); d.see(residual); d.see(mid); d.see(out); d.see(handover);
     d.see(out_packed); d.see(arrived); d.see(clear);
@@ -1046,6 +1046,7 @@ optional<Tensor> linear_chain(const Tensor& wo, const Tensor& wgu, const Tensor&
         TORCH_CHECK(t->scalar_type() == at::kInt && t->is_contiguous() && t->numel() == TAH_LINEAR_CHAIN_WORDS, "linear_chain: arrived and clear are int32 [",
                     TAH_LINEAR_CHAIN_WORDS, "]");
     TORCH_CHECK(linear_chain_supported(rows, hidden, o_cols, ff, qkv_cols), "linear_chain: sizes it is not built for");
+    TORCH_CHECK(polls >= 0 && polls <= 0x7fffffff, "linear_chain: polls must not be negative");
     const auto stride = [&](const Tensor& t) { return rows > 1 ? t.stride(0) : hidden; };
     tah_linear_chain_args a{};
     a.wo_packed = ptr(wo); a.wgu_packed = ptr(wgu); a.wdown_packed = ptr(wdown); a.wqkv_packed = ptr(wqkv);
@@ -1056,6 +1057,7 @@ optional<Tensor> linear_chain(const Tensor& wo, const Tensor& wgu, const Tensor&
     a.rows = (int32_t)rows; a.hidden = (int32_t)hidden; a.o_cols = (int32_t)o_cols; a.ff = (int32_t)ff; a.qkv_cols = (int32_t)qkv_cols;
     a.norm_eps = (float)norm_eps;
     a.arrived = static_cast<int32_t*>(mptr(arrived)); a.clear = static_cast<int32_t*>(mptr(clear));
+    a.polls = (int32_t)polls;
     check_rc(g.linear_chain(&a, d.stream()), "tah_linear_chain");
     return y;
 }

@@ -295,16 +295,18 @@ def linear_chain_supported(rows: int, hidden: int, o_cols: int, ff: int, qkv_col
 
 
 def linear_chain(wo_packed, wgu_packed, wdown_packed, wqkv_packed, attn_packed, residual, *, mid, out, handover, arrived, clear,
-                 norm_eps: float, out_packed=None):
+                 norm_eps: float, out_packed=None, polls: int = 0):
     """The linear layers between two attentions of a decode step in one launch (``tah_linear_chain``), at most eight rows.
 
     ``mid = residual + attn @ wo.T``; the MLP of mid's RMS-normed rows (the norm's weight sits in the gate|up weight);
     ``out = mid + act @ wdown.T``; returns ``out @ wqkv.T`` (None without ``wqkv_packed``): the same bits as four
     ``linear_rows`` calls.  ``residual``, ``mid`` and ``out`` bf16 [rows, hidden] are different tensors; ``handover`` bf16
-    [8 * (2 * hidden + ff)] is scratch; ``out_packed`` [32 * hidden] also receives ``out`` as a rows operand.  ``arrived`` int32 [LINEAR_CHAIN_WORDS]: zeros before the call, not
-    behind it; ``clear``: other such words, which the call zeroes (for the call that comes next on the stream)."""
+    [8 * (2 * hidden + ff)] is scratch; ``out_packed`` [32 * hidden] also receives ``out`` as a rows operand.  ``arrived`` int32
+    [LINEAR_CHAIN_WORDS]: zeros before the call, not behind it; ``clear``: other such words, which the call zeroes (for the
+    call that comes next on the stream).  ``polls``: how often a workgroup looks for the others' tiles before it computes
+    what is missing itself (0: the library's number)."""
     return _call("linear_chain", wo_packed, wgu_packed, wdown_packed, wqkv_packed, attn_packed, residual, mid, out, handover,
-                 out_packed, arrived, clear, float(norm_eps))
+                 out_packed, arrived, clear, float(norm_eps), int(polls))
 
 
 def greedy_workspace(rows: int, device) -> torch.Tensor:

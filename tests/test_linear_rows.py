@@ -7,6 +7,7 @@ different order from the float64 ones, so a result may land on the neighbouring 
 most elements have to agree exactly.  The CPU tests run the kernels on the CPU execution shim; the GPU tests call the
 library through the extension and through ctypes.
 """
+import contextlib
 import ctypes
 
 import numpy as np
@@ -313,7 +314,7 @@ def test_linear_rows_through_the_c_abi_gpu():
 CHAIN_CASES = [(1, 4096, False), (2, 4096, True), (3, 16, False), (4, 0, True), (5, 4096, True), (8, 4096, False), (8, 0, False)]
 
 
-def _chain_case(dev, rows, hidden, o_cols, ff, n_qkv, views, launches=2):
+def _chain_case(dev, rows, hidden, o_cols, ff, n_qkv, views, launches=2, polls=0):
     """Against the four ``linear_rows`` launches: the same bits (512 columns, on the CPU only: ``linear_rows`` adds even and odd steps
     up together there, a neighbouring bf16 value).  ``views``: row-major tensors with strides of their own."""
     from tah_amd import ops
@@ -331,7 +332,7 @@ def _chain_case(dev, rows, hidden, o_cols, ff, n_qkv, views, launches=2):
         before = res.clone()
         mid, out, between, out_p = empty(), empty(), torch.full((8 * (2 * hidden + ff),), 7.0, dtype=BF, device=dev), form(hidden)
         got = ops.linear_chain(wo, wgu, wdown, wqkv, attn, res, mid=mid, out=out, handover=between, out_packed=out_p if i != 1 else None,
-                               arrived=words[i % 2], clear=words[1 - i % 2], norm_eps=1e-6)
+                               arrived=words[i % 2], clear=words[1 - i % 2], norm_eps=1e-6, polls=polls)
         x, xp, ap = before.clone(), form(hidden), form(ff)
         ops.linear_rows(wo, attn, rows, hidden, o_cols, residual=x, out=x, out_packed=xp)
         assert same(mid, x)
@@ -397,6 +398,76 @@ def test_linear_chain_on_the_cpu_shim():
     with emu_util.emulated():
         _chain_errors("cpu")
         _chain_case("cpu", 7, 512, 512, 1536, 16, True, launches=1)
+
+
+@contextlib.contextmanager
+def _only_blocks(lib, first, count):
+    lib.tah_emu_run_blocks(first, count)
+    try:
+        yield
+    finally:
+        lib.tah_emu_run_blocks(0, 0xffffffff)
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_linear_chain_waiters_take_different_tiles_on_the_cpu_shim():
+    """Three workgroups that each see the same three tiles missing begin with a different one; tiles of workgroups that have begun
+    are left to them until the polls are used up."""
+    from tah_amd import _capi, ops
+    z = lambda *s: torch.zeros(*s, dtype=BF)
+    weights = (z(512 * 512), z(2 * 1536 * 512), z(512 * 1536))
+    missing = [5, 18, 40]
+    with emu_util.emulated() as lib:
+        def taken(block, begun, polls):
+            words = torch.zeros(2, ops.LINEAR_CHAIN_WORDS, dtype=torch.int32)
+            lines = words[0].view(3, 64, 32)
+            lines[:2, :, 0] = 15
+            for t in missing:
+                lines[0, t // 4, 0] &= ~(1 << t % 4)
+            lines[0, :, 1] = 15 if begun else lines[0, :, 0]
+            with _only_blocks(lib, block, 1):
+                ops.linear_chain(*weights, None, z(32 * 512), z(1, 512), mid=z(1, 512), out=z(1, 512), handover=z(8 * (2 * 512 + 1536)),
+                                 arrived=words[0], clear=words[1], norm_eps=1e-6, polls=polls)
+                at = (ctypes.c_void_p * 64)()
+                n = lib.tah_emu_ors(at, 64)
+            words_at = [(a - words.data_ptr()) // 4 for a in at[:n]]
+            line = [w // 32 for w in words_at if w < 64 * 32 and w % 32 == 0]  # phase 0, without the workgroup's own
+            assert line[0] == block // 4 and sorted(line[1:]) == sorted(t // 4 for t in missing)
+            return line[1]
+        assert sorted(taken(b, False, 0) for b in range(3)) == sorted(t // 4 for t in missing)
+        assert sorted(taken(b, True, 1) for b in range(3)) == sorted(t // 4 for t in missing)
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+@pytest.mark.parametrize("rows,n_qkv", [(1, 0), (2, 16), (4, 0)])
+def test_linear_chain_by_one_workgroup_on_the_cpu_shim(rows, n_qkv):
+    """What the first workgroup computes in the others' place, before they run themselves (all tiles but those of q|k|v)."""
+    from tah_amd import ops
+    dense = [_rand(s, 21 + i, s[1] ** -0.5) for i, s in enumerate([(512, 512), (2 * 1536, 512), (512, 1536), (16, 512)])]
+    attn, res = _rand((rows, 512), 31), _rand((rows, 512), 41)
+    mid, out = [torch.full((rows, 512), 7.0, dtype=BF) for _ in range(2)]
+    words = torch.zeros(2, ops.LINEAR_CHAIN_WORDS, dtype=torch.int32)
+    with emu_util.emulated() as lib:
+        packed = [ops.linear_pack_weight(w, gate_up=i == 1) for i, w in enumerate(dense)]
+        attn_p = ops.linear_pack_rows(attn)
+        with _only_blocks(lib, 0, 1):
+            got = ops.linear_chain(*packed[:3], packed[3] if n_qkv else None, attn_p, res, mid=mid, out=out,
+                                   handover=torch.full((8 * (2 * 512 + 1536),), 7.0, dtype=BF), arrived=words[0], clear=words[1], norm_eps=1e-6)
+    close = lambda a, b: torch.allclose(a.float(), b.float(), rtol=2.0 ** -6, atol=2.0 ** -6)
+    _close(mid, reference(attn, dense[0], residual=res))
+    if n_qkv:  # (without q|k|v nobody waits for down's tiles)
+        assert close(out, reference(reference(mid, dense[1], gate_up=True, norm_eps=1e-6), dense[2], residual=mid))
+        assert close(got, reference(out, dense[3]))
+    else:
+        assert close(out[:, :8], reference(reference(mid, dense[1], gate_up=True, norm_eps=1e-6), dense[2], residual=mid)[:, :8])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("n_qkv", [4096, 0])
+def test_linear_chain_tiles_of_others_gpu(rows, n_qkv):
+    """A wait that gives up at its first look: whoever finds a tile missing computes it, the same bits."""
+    _chain_case("cuda", rows, 2048, 2048, 6144, n_qkv, rows == 3, launches=5, polls=1)
 
 
 @pytest.mark.gpu
