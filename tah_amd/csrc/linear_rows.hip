@@ -618,13 +618,14 @@ __device__ __forceinline__ int handed_over(int row, int col) {
 constexpr int kChainWindow = 4;
 
 // A wave's part of one tile: PW steps of K, NC column tiles (H8: one, and half of its columns, as in linear_rows_kernel), rows
-// folded to F.
-template <int PW, int NC, bool H8, int F>
+// folded to F.  kApart: even and odd steps are summed apart, as H8 does (a whole tile then leaves them in red's first two).
+template <int PW, int NC, bool H8, int F, bool kApart = H8>
 struct ChainTile {
+    static_assert(NC == 1 || !kApart, "");
     static constexpr int kLoads = H8 ? PW / 2 : PW, kPer = 16 / F, kXLoads = (PW + kPer - 1) / kPer;
     bf16x8 w[kLoads][NC], x[kXLoads];
     float ss;
-    f32x4 acc[NC][H8 ? 2 : 1];
+    f32x4 acc[NC][kApart ? 2 : 1];
 
     template <int kFrom, int kTo>
     __device__ __forceinline__ void ask_weights(const bf16x8* pw, int tile, int wave, int lane) {
@@ -681,7 +682,7 @@ struct ChainTile {
 #pragma unroll
         for (int t = 0; t < NC; ++t)
 #pragma unroll
-            for (int h = 0; h < (H8 ? 2 : 1); ++h) acc[t][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int h = 0; h < (kApart ? 2 : 1); ++h) acc[t][h] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     template <bool kNorm, int S>
     __device__ __forceinline__ void step() {
@@ -692,8 +693,8 @@ struct ChainTile {
         }
 #pragma unroll
         for (int t = 0; t < NC; ++t) {
-            if constexpr (H8) acc[t][S % 2] = mfma16(a, w[S / 2][t], acc[t][S % 2]);
-            else acc[t][0] = mfma16(a, w[S][t], acc[t][0]);
+            constexpr int half = kApart ? S % 2 : 0;
+            acc[t][half] = mfma16(a, w[H8 ? S / 2 : S][t], acc[t][half]);
         }
     }
     template <bool kNorm, int kFrom, int... S>
@@ -707,7 +708,10 @@ struct ChainTile {
         for (int t = 0; t < NC; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                if (4 * kg < F) red[wave][t][4 * kg + r][c] = (H8 && c >= 8) ? acc[t][H8 ? 1 : 0][r] : acc[t][0][r];
+                if (4 * kg < F) {
+                    red[wave][t][4 * kg + r][c] = (H8 && c >= 8) ? acc[t][H8 ? 1 : 0][r] : acc[t][0][r];
+                    if constexpr (kApart && !H8) red[wave][1][4 * kg + r][c] = acc[t][1][r];
+                }
         if constexpr (kNorm) {
             ss += __shfl_xor(ss, 16);
             ss += __shfl_xor(ss, 32);
@@ -749,8 +753,10 @@ __device__ __forceinline__ void chain_barrier() {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
-// PWO, PWH, PWF: query columns, hidden size and MLP width over 256.  kNext: with the q|k|v phase.
-template <int F, int PWO, int PWH, int PWF, bool kNext>
+// PWO, PWH, PWF: query columns, hidden size and MLP width over 256.  NEXT: the q|k|v phase (kNextApart: of so few columns that
+// linear_rows takes eight at a time and sums even and odd steps apart).
+enum { kNextNone, kNextWhole, kNextApart };
+template <int F, int PWO, int PWH, int PWF, int NEXT>
 __global__ __launch_bounds__(kChainThreads) void linear_chain_kernel(const ChainParams p) {
     __shared__ __align__(16) float red[kLinWaves][3][16][kTileCols];
     __shared__ float ssq[kLinWaves][16];
@@ -760,7 +766,8 @@ __global__ __launch_bounds__(kChainThreads) void linear_chain_kernel(const Chain
     using O = ChainTile<PWO, 1, true, F>;
     using GateUp = ChainTile<PWH, 3, false, F>;
     using Down = ChainTile<PWF, 1, true, F>;
-    using Qkv = ChainTile<PWH, 1, false, F>;
+    constexpr bool kNext = NEXT != kNextNone;
+    using Qkv = ChainTile<PWH, 1, false, F, NEXT == kNextApart>;
     // (a workgroup without a tile in a phase multiplies another's and stores nothing)
     const int t0 = tile < p.tiles0 ? tile : 0, t1 = tile < p.tiles1 ? tile : 0, t2 = tile < p.tiles2 ? tile : 0, t3 = tile < p.tiles3 ? tile : 0;
 
@@ -1006,10 +1013,15 @@ __global__ __launch_bounds__(kChainThreads) void linear_chain_kernel(const Chain
         chain_barrier();
         const int row = lane / 4, col = 4 * (lane % 4);
         if (tile < p.tiles3 && row < p.rows) {
-            f32x4 part[kLinWaves];
+            f32x4 s = {0.f, 0.f, 0.f, 0.f}, part[kLinWaves], odd[kLinWaves];
             ask4(part, 0, row, col);
+            if constexpr (NEXT == kNextApart) ask4(odd, 1, row, col);
             __builtin_amdgcn_sched_barrier(0);
-            const f32x4 s = sum4(part);
+#pragma unroll
+            for (int w = 0; w < kLinWaves; ++w) {
+                s += part[w];
+                if constexpr (NEXT == kNextApart) s += odd[w];
+            }
             bf16x4 o;
 #pragma unroll
             for (int i = 0; i < 4; ++i) o[i] = (__bf16)s[i];
@@ -1024,13 +1036,15 @@ __global__ __launch_bounds__(kLinThreads) void linear_chain_clear_kernel(int32_t
 }
 
 template <int PWO, int PWH, int PWF>
-void launch_chain(const ChainParams& p, bool next, hipStream_t st) {
+void launch_chain(const ChainParams& p, int next, hipStream_t st) {
     int tiles = p.tiles0 > p.tiles1 ? p.tiles0 : p.tiles1;
     tiles = tiles > p.tiles3 ? tiles : p.tiles3;
     const auto run = [&](auto fold) {
         constexpr int F = decltype(fold)::value;
-        if (next) hipLaunchKernelGGL((linear_chain_kernel<F, PWO, PWH, PWF, true>), dim3(tiles), dim3(kChainThreads), 0, st, p);
-        else hipLaunchKernelGGL((linear_chain_kernel<F, PWO, PWH, PWF, false>), dim3(tiles), dim3(kChainThreads), 0, st, p);
+        const dim3 grid(tiles), block(kChainThreads);
+        if (next == kNextApart) hipLaunchKernelGGL((linear_chain_kernel<F, PWO, PWH, PWF, kNextApart>), grid, block, 0, st, p);
+        else if (next) hipLaunchKernelGGL((linear_chain_kernel<F, PWO, PWH, PWF, kNextWhole>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((linear_chain_kernel<F, PWO, PWH, PWF, kNextNone>), grid, block, 0, st, p);
     };
     if (p.rows <= 1) run(std::integral_constant<int, 1>{});
     else if (p.rows <= 2) run(std::integral_constant<int, 2>{});
@@ -1333,13 +1347,14 @@ extern "C" int tah_linear_chain(const tah_linear_chain_args* a, tah_stream_t str
     p.tiles3 = next ? a->qkv_cols / kTileCols : 0;
     p.polls = a->polls > 0 ? a->polls : kChainPolls;
     p.eps = a->norm_eps;
+    const int form = !next ? kNextNone : p.tiles3 < kSplitRowsBelowGroups ? kNextApart : kNextWhole;
     hipStream_t st = static_cast<hipStream_t>(stream);
 #ifdef TAH_CPU_EMU
     if (a->hidden == 512) {
-        launch_chain<2, 2, 6>(p, next, st);
+        launch_chain<2, 2, 6>(p, form, st);
         return TAH_OK;
     }
 #endif
-    launch_chain<8, 8, 24>(p, next, st);
+    launch_chain<8, 8, 24>(p, form, st);
     return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
 }

@@ -478,6 +478,14 @@ def test_linear_chain_gpu(rows, n_qkv, views):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 2, 4, 8])
+@pytest.mark.parametrize("n_qkv", [128, 2048, 2064])
+def test_linear_chain_narrow_qkv_gpu(rows, n_qkv):
+    """Up to 2048 columns of q|k|v and above: ``linear_rows`` sums even and odd steps apart up to there."""
+    _chain_case("cuda", rows, 2048, 2048, 6144, n_qkv, False)
+
+
+@pytest.mark.gpu
 def test_linear_chains_side_by_side_gpu():
     """Two streams' launches share the compute units: whichever workgroups are resident, both finish with the same bits."""
     from tah_amd import ops
