@@ -463,7 +463,7 @@ class TaHDecodeEngine(DecodeEngine):
             self.handover = torch.empty(8 * (2 * cfg.hidden + cfg.intermediate), dtype=torch.bfloat16, device=dev)
             self.x_mid, *self.x_turn = [torch.zeros(batch, cfg.hidden, dtype=torch.bfloat16, device=dev) for _ in range(3)]
             self.arrived = torch.zeros(cfg.layers, ops.LINEAR_CHAIN_WORDS, dtype=torch.int32, device=dev)
-            self.pass_open = False  # a pass has begun and not ended: the words are not to be relied on
+        self.pass_open = False  # a pass has begun and not ended: the words are not to be relied on
         # the step's element-wise glue in two launches (tah_step_begin, tah_decider_tail) and the decider's first layer
         # on the linear-layer kernel, instead of some twenty torch launches; needs the packed rows
         self.fused_glue = bool(self.packed_linear and weights.lm_head_p is not None and
@@ -587,9 +587,10 @@ class TaHDecodeEngine(DecodeEngine):
         return self._rms(x, self.w.norm)
 
     def _close_pass(self) -> None:
-        """Zeroes the words of arrival if a pass ended between two of its launches (an exception): before the next pass, and
-        before graphs, which hold passes that began with zeros, are replayed."""
-        if self.linear_chain and self.pass_open:
+        """Zeroes the words of arrival if a pass ended between two of its launches (an exception): at once, for graphs a caller
+        holds, whose passes began with zeros; and, if that could not be (while a graph is captured), before the next pass, and
+        before graphs are captured or handed out."""
+        if self.pass_open:
             self.arrived.zero_()
             self.pass_open = False
 
@@ -597,16 +598,28 @@ class TaHDecodeEngine(DecodeEngine):
         """The same pass with the four linear layers of a layer on ``ops.linear_rows``, or those from one attention to the next
         in one launch (``ops.linear_chain``).  The hidden state lives twice, row-major in ``x`` (updated in place, or in
         ``self.x_turn``; read by the q/k preparation for the norm factor) and as rows operand in ``self.xp``; attention output and MLP activation exist as rows operands only."""
-        c = self.cfg
-        B, H, I = x.shape[0], c.hidden, c.intermediate
-        n_qkv, n_o = (c.hq + 2 * c.hkv) * c.head_dim, c.hq * c.head_dim
         x = x.contiguous()
         xp = self.xp if rows_packed else ops.linear_pack_rows(x, out=self.xp)  # rows_packed: self.xp already holds x
         self._keep_hidden(0, x)
-        chain, qkv = self.linear_chain, None
-        if chain:
-            self._close_pass()
-            self.pass_open = True
+        if not self.linear_chain:
+            return self._layers_packed(x, xp, pos, depth, slot_of, q_pos, q_depth, cos, sin, False)
+        self._close_pass()
+        self.pass_open = True
+        try:
+            x = self._layers_packed(x, xp, pos, depth, slot_of, q_pos, q_depth, cos, sin, True)
+        except BaseException:
+            if not (x.is_cuda and torch.cuda.is_current_stream_capturing()):
+                self._close_pass()
+            raise
+        self.pass_open = False
+        return x
+
+    def _layers_packed(self, x, xp, pos, depth: int, slot_of, q_pos, q_depth, cos, sin, chain: bool):
+        """The layers of ``_pass_single_packed``; ``chain``: on ``ops.linear_chain``."""
+        c = self.cfg
+        B, H, I = x.shape[0], c.hidden, c.intermediate
+        n_qkv, n_o = (c.hq + 2 * c.hkv) * c.head_dim, c.hq * c.head_dim
+        qkv = None
         for l, L in enumerate(self.w.layers):
             q, k, v = self._split_qkv(ops.linear_rows(L["wqkv_p"], xp, B, n_qkv, H) if qkv is None else qkv)
             cache = self.slabs1[l] if depth == 1 else self.slabs0[l]
@@ -642,8 +655,6 @@ class TaHDecodeEngine(DecodeEngine):
             ops.linear_rows(L["wgu_p"], xp, B, I, H, gate_up=True, out_packed=self.actp, want_out=False, norm_eps=c.rms_eps)
             ops.linear_rows(L["wdown_p"], self.actp, B, H, I, residual=x, out=x, out_packed=xp)
             self._keep_hidden(l + 1, x)
-        if chain:
-            self.pass_open = False
         return x  # before the final norm; self.xp holds the same rows as operand
 
     def _head(self, h):
@@ -874,6 +885,10 @@ class TaHDecodeEngine(DecodeEngine):
         return super().generate(first_logits, max_new_tokens, temperature=temperature, eos=eos, use_graph=use_graph,
                                 check_every=check_every, **filters)
 
+    def capture(self, temperature: float = 0.0, eos: int = -1, **filters):
+        self._close_pass()
+        return super().capture(temperature, eos, **filters)
+
     def _check_room(self, max_new_tokens: int) -> None:
         if self.host_positions + max_new_tokens > self.max_len or self.host_hard_rows + max_new_tokens > self.max_hard:
             raise TahDuoError("generation would outgrow the KV slabs: construct the engine with a larger max_len / max_hard")
@@ -929,6 +944,7 @@ class TaHDecodeEngine(DecodeEngine):
 
     def capture_ticks(self, eos: int, limit: int, temperature: float = 0.0, **filters):
         """The tick as two HIP graphs, one per logits buffer, after a warm-up tick whose state changes are undone."""
+        self._close_pass()
         key = (eos, limit, self.w.threshold, temperature, tuple(sorted(filters.items()))) + self._launch_switches()
         if self._tick_graphs is not None and self._tick_key == key:
             return self._tick_graphs

@@ -690,3 +690,66 @@ def test_linear_layers_in_one_launch_change_no_bit_gpu(batch):
     want = run(False, True)
     for chain, use_graph, broken in ((True, True, False), (True, False, False), (True, True, True), (True, False, True)):
         assert all(torch.equal(a, b) for a, b in zip(run(chain, use_graph, broken), want)), (chain, use_graph, broken)
+
+
+def _break_off(e, monkeypatch, at=1):
+    """A step whose linear layers raise in layer ``at``, behind launches that have left their words of arrival."""
+    from tah_amd import ops
+    real, calls = ops.linear_chain, []
+
+    def chain(*args, **kw):
+        if len(calls) == at:
+            raise KeyboardInterrupt
+        calls.append(1)
+        if e.device.type == "cuda":
+            return real(*args, **kw)
+        kw["arrived"].fill_(15)
+        return torch.zeros(e.B, (e.cfg.hq + 2 * e.cfg.hkv) * e.cfg.head_dim, dtype=torch.bfloat16)
+
+    with monkeypatch.context() as m:
+        m.setattr(ops, "linear_chain", chain)
+        with pytest.raises(KeyboardInterrupt):
+            e._step_inplace(0.0, -1)
+    assert len(calls) == at
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_no_words_of_arrival_are_left_by_a_pass_that_broke_off_on_cpu_shim(monkeypatch):
+    """Graphs that a caller holds, and those that ``capture`` and ``capture_ticks`` hand out again, begin with zeros."""
+    from tah_amd.engine import EngineConfig, TaHDecodeEngine, Weights
+    cfg = EngineConfig(hidden=256, layers=2, hq=2, hkv=1, head_dim=128, intermediate=256, vocab=96, decider_hidden=32)
+    with emu_util.emulated(), torch.no_grad():
+        e = TaHDecodeEngine(Weights.random_init(cfg, "cpu", seed=1), 1, 8, device="cpu")
+        e.linear_chain, e.handover, e.x_mid, e.x_turn = True, None, None, [None, None]
+        e.arrived, e.pass_open = torch.zeros(cfg.layers, 64, dtype=torch.int32), False
+        _break_off(e, monkeypatch)
+        assert not e.arrived.any() and not e.pass_open
+        e._graph, e._graph_key = "step", (0.0, -1, ()) + e._launch_switches()
+        e._tick_graphs, e._tick_key = "ticks", (-1, 8, e.w.threshold, 0.0, ()) + e._launch_switches()
+        for capture, graph in ((lambda: e.capture(), "step"), (lambda: e.capture_ticks(-1, 8), "ticks")):
+            e.arrived.fill_(15)
+            e.pass_open = True
+            assert capture() == graph and not e.arrived.any() and not e.pass_open
+
+
+@pytest.mark.gpu
+def test_graphs_behind_a_pass_that_broke_off_gpu(monkeypatch):
+    from tah_amd.engine import EngineConfig, TaHDecodeEngine, Weights
+    e = TaHDecodeEngine(Weights.random_init(EngineConfig(layers=3, vocab=4096), "cuda", seed=3), 2, 128)
+    ids = torch.randint(0, 4096, (50,), generator=torch.Generator().manual_seed(1)).cuda()
+    with torch.no_grad():
+        first, _ = e.prefill(ids, torch.tensor([0, 30, 50], dtype=torch.int32).cuda(), calibrate=0.2)
+        e.generate(first, 4)
+        e.finished.zero_()
+        graphs = e.capture_ticks(-1, 100)
+        undo = e._hold_state()
+        graphs[0].replay()
+        want = e.logits2[0].clone()
+        undo()
+        _break_off(e, monkeypatch)
+        assert not e.arrived.any() and not e.pass_open
+        undo()
+        for _ in range(3):
+            graphs[0].replay()
+            assert torch.equal(e.logits2[0], want)
+            undo()
