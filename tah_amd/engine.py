@@ -458,7 +458,7 @@ class TaHDecodeEngine(DecodeEngine):
         # layer's launch zeroes the next layer's, the last one the first's for the next pass.
         self.linear_chain = bool(self.packed_linear and cfg.layers > 1 and self.device.type == "cuda" and
                                  ops.linear_chain_supported(batch, cfg.hidden, cfg.hq * cfg.head_dim, cfg.intermediate,
-                                                            (cfg.hq + 2 * cfg.hkv) * cfg.head_dim))
+                                                            (cfg.hq + 2 * cfg.hkv) * cfg.head_dim, device=dev))
         if self.linear_chain:
             self.handover = torch.empty(8 * (2 * cfg.hidden + cfg.intermediate), dtype=torch.bfloat16, device=dev)
             self.x_mid, *self.x_turn = [torch.zeros(batch, cfg.hidden, dtype=torch.bfloat16, device=dev) for _ in range(3)]

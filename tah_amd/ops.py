@@ -286,11 +286,17 @@ def linear_rows(w_packed: torch.Tensor, x_packed: torch.Tensor, rows: int, n: in
                  float(c0), float(c1))
 
 
+LINEAR_CHAIN_TILES = 256   # TAH_LINEAR_CHAIN_TILES
 LINEAR_CHAIN_WORDS = 6144  # TAH_LINEAR_CHAIN_WORDS
 
 
-def linear_chain_supported(rows: int, hidden: int, o_cols: int, ff: int, qkv_cols: int) -> bool:
-    """Whether ``linear_chain`` takes these sizes."""
+def linear_chain_supported(rows: int, hidden: int, o_cols: int, ff: int, qkv_cols: int, device=None) -> bool:
+    """Whether ``linear_chain`` takes these sizes and, with a ``device``, whether that has a compute unit for each of its workgroups
+    (at most LINEAR_CHAIN_TILES).  With fewer (a partition of the card) the launch ends with the same results, but every
+    workgroup that has to wait for a compute unit has its tiles computed twice; four ``linear_rows`` calls only take turns."""
+    if device is not None and torch.device(device).type == "cuda":
+        if torch.cuda.get_device_properties(device).multi_processor_count < LINEAR_CHAIN_TILES:
+            return False
     return bool(_call("linear_chain_supported", int(rows), int(hidden), int(o_cols), int(ff), int(qkv_cols)))
 
 

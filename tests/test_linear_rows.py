@@ -366,6 +366,16 @@ def _chain_errors(dev):
     assert not ops.linear_chain_supported(1, 1024, 2048, 6144, 0) and not ops.linear_chain_supported(1, 2048, 2048, 6144, 16 * 257)
 
 
+def test_linear_chain_wants_a_compute_unit_for_each_workgroup(monkeypatch):
+    import types
+    from tah_amd import ops
+    sizes = (1, 2048, 2048, 6144, 4096)
+    for units, want in ((256, True), (304, True), (255, False), (32, False)):
+        monkeypatch.setattr(torch.cuda, "get_device_properties", lambda device: types.SimpleNamespace(multi_processor_count=units))
+        assert ops.linear_chain_supported(*sizes, device="cuda:0") is want
+    assert ops.linear_chain_supported(*sizes) and ops.linear_chain_supported(*sizes, device="cpu")
+
+
 @pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
 def test_linear_chain_without_rows_clears_the_next_words_on_the_cpu_shim():
     """The launch behind an empty one finds zeros too."""
