@@ -543,7 +543,8 @@ typedef struct tah_linear_chain_args {
     int32_t *arrived, *clear;
     int32_t polls;            /* a workgroup that has looked this often for the others' tiles computes what is missing; 0: the library's number */
 } tah_linear_chain_args;
-/* Whether the sizes are taken (hidden and o_cols 2048, ff 6144: what the kernel is built for).  The launch wants a compute unit for each
+/* Whether the sizes are taken: rows 1 to 8, hidden and o_cols 2048, ff 6144 (the kernel is built for this layer alone), qkv_cols a
+ * multiple of 16 up to 4096.  The launch wants a compute unit for each
  * of its TAH_LINEAR_CHAIN_TILES workgroups; with fewer it ends with the same results, slower than four tah_linear_rows calls. */
 int tah_linear_chain_supported(int32_t rows, int32_t hidden, int32_t o_cols, int32_t ff, int32_t qkv_cols);
 int tah_linear_chain(const tah_linear_chain_args* args, tah_stream_t stream);

@@ -67,7 +67,8 @@ struct LinParams {
     const int32_t* select;  // run only products whose index is listed here, or null
     int32_t n_select;
     int32_t grid_y, batches; // workgroups along y: one per product or, by_list, one per entry of a list that is shorter than the
-    bool by_list;            // products are: 7 of 8 of 64 experts' workgroups would start only to leave (1.7 us of 11 a launch at one row)
+    bool by_list;            // products are: seven of eight of 64 experts' workgroups would start only to leave (one row, eight experts of
+                             // 2048 x 768, in a captured sequence: gate|up 10.3 -> 8.8 us a launch, down 8.4 -> 5.4; eight rows 10.9 -> 9.5, 9.2 -> 5.7)
     float c0, c1;           // constants of the activation
 };
 
@@ -556,11 +557,13 @@ __global__ __launch_bounds__(kLinThreads) void linear_wide_kernel(const LinParam
 // o + residual, gate|up + SiLU, down + residual and the next layer's q|k|v of at most eight rows.  As four launches each of
 // them pays its start, the first bytes' way and its reduction with the memory pipe empty; here the next phase's weights,
 // which depend on nothing, are on their way while a phase's results travel between the workgroups.  2048 / 6144 / 4096 (100 MB) in a
-// captured sequence of layers: 23.7 us at one row, 25.7 at eight, against 28.1 as four launches; the weights alone take 16 us at
-// 6.2 TB/s.  What bounds it now: the three hand-overs, each from the last workgroup's sums to the first product of the next phase 3.5
+// captured sequence of layers, against four launches: 24.1 us at one row (28.0), 24.0 at two (28.3), 24.4 at three and four (28.2),
+// 25.5 at five and eight (28.9, 28.4); the weights alone take 16 us at 6.2 TB/s.  What bounds it now: the three hand-overs, each from the last workgroup's sums to the first product of the next phase 3.5
 // to 4 us (a store that has arrived 0.7 to 1, the slowest workgroup another 1, bit and poll 1.5, the rows 0.7), of which the weights
-// asked for ahead hide one and parts of two.  From nine rows on the rows' operand that everybody reads past the L2s would cost
-// more than the launches (eight rows already lose 2 us): they keep four launches.
+// asked for ahead hide one and parts of two.  From nine rows on it is four launches (31 us): the ninth wave's lanes hold ten rows of
+// gate|up's results, and everybody reads the rows' operand past the L2s (eight rows already lose 1.4 us).  A form for them is not
+// built, so what it would take is not known.  Nor is one for other layer sizes: K per wave is a template argument, and 2048 / 2048 /
+// 6144 is the layer that this library's generation workloads have.
 //  * A workgroup takes the same tile number of every phase (2048 / 6144: 256 tiles in each, one to a compute unit).  Eight waves
 //    multiply as in linear_rows_kernel (same slices of K, same order of sums: the same bits); a ninth reduces, stores and
 //    waits for the other workgroups, so that no wait for a store or a flag stands behind the weights' loads.
@@ -613,8 +616,10 @@ __device__ __forceinline__ int handed_over(int row, int col) {
     const int unit = (col / 8) * F + row;
     return ((unit / 64) * 2 + (col % 8) / 4) * 64 + unit % 64;
 }
-// A wave has this many loads of weights on their way at most: 32 KB per compute unit keep the memory busy, and what the ninth wave
-// stores and asks for has no longer queue than that before it (all at once: the stores took 6.8 us to arrive, not 1.2).
+// While the ninth wave stores results and asks for others', a wave has this many loads of weights on their way at most: 32 KB per
+// compute unit keep the memory busy, and those stores have no longer queue than that before them (all at once: they took 6.8 us to
+// arrive, not 1.2).  o's weights at the start, q|k|v's second half and what is asked for again behind a tile of another workgroup go
+// out all at once: the ninth wave has nothing to store then.
 constexpr int kChainWindow = 4;
 
 // A wave's part of one tile: PW steps of K, NC column tiles (H8: one, and half of its columns, as in linear_rows_kernel), rows

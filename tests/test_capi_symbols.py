@@ -48,6 +48,7 @@ def test_struct_sizes_match_c_layout(tmp_path):
              "tah_duo_decode_args": _capi.DuoDecodeArgs, "tah_qk_prep_args": _capi.QkPrepArgs, "tah_topk_mix_args": _capi.TopkMixArgs,
              "tah_kv_append_args": _capi.KvAppendArgs, "tah_additive_mask": _capi.AdditiveMask,
              "tah_greedy_step_args": _capi.GreedyStepArgs, "tah_linear_rows_args": _capi.LinearRowsArgs,
+             "tah_linear_chain_args": _capi.LinearChainArgs,
              "tah_step_begin_args": _capi.StepBeginArgs, "tah_decider_tail_args": _capi.DeciderTailArgs,
              "tah_greedy_tick_args": _capi.GreedyTickArgs, "tah_sample_rows_args": _capi.SampleRowsArgs,
              "tah_qk_prep_bwd_args": _capi.QkPrepBwdArgs, "tah_embed_rows_args": _capi.EmbedRowsArgs,
