@@ -558,8 +558,8 @@ __global__ __launch_bounds__(kLinThreads) void linear_wide_kernel(const LinParam
 // them pays its start, the first bytes' way and its reduction with the memory pipe empty; here the next phase's weights,
 // which depend on nothing, are on their way while a phase's results travel between the workgroups.  2048 / 6144 / 4096 (100 MB) in a
 // captured sequence of layers, against four launches: 24.1 us at one row (28.0), 24.0 at two (28.3), 24.4 at three and four (28.2),
-// 25.5 at five and eight (28.9, 28.4); the weights alone take 16 us at 6.2 TB/s.  What bounds it now: the three hand-overs, each from the last workgroup's sums to the first product of the next phase 3.5
-// to 4 us (a store that has arrived 0.7 to 1, the slowest workgroup another 1, bit and poll 1.5, the rows 0.7), of which the weights
+// 25.5 at five and eight (28.9, 28.4); the weights alone take 16 us at 6.2 TB/s.  What bounds it
+// now: the three hand-overs, each from the last workgroup's sums to the first product of the next phase 3.5 to 4 us (a store that has arrived 0.7 to 1, the slowest workgroup another 1, bit and poll 1.5, the rows 0.7), of which the weights
 // asked for ahead hide one and parts of two.  From nine rows on it is four launches (31 us): the ninth wave's lanes hold ten rows of
 // gate|up's results, and everybody reads the rows' operand past the L2s (eight rows already lose 1.4 us).  A form for them is not
 // built, so what it would take is not known.  Nor is one for other layer sizes: K per wave is a template argument, and 2048 / 2048 /
