@@ -371,21 +371,24 @@ __global__ __launch_bounds__(kKvThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dkd
 
     int seq = 0, key0 = 0, key_end = 0;
     bool second = false;
+    const CallBounds cb = call_bounds(p);
     int slot = (int)blockIdx.y;  // without a table: early (heavy) key tiles of each sequence first
     // (the table's order: the key tile seen by the most query rows first)
     sched_lookup(p.sched, true, p.nseq, G, p.s1.total_q, p.s2.total_q, p.s1.total_k, p.s2.total_k, (int)gridDim.y,
                  (int)blockIdx.y, slot);
-    if (!(p.s1.total_k > 0 && find_tile(p.s1.cu_k, p.nseq, kBK, slot, seq, key0, key_end))) {
-        if (!(p.s2.total_k > 0 && find_tile(p.s2.cu_k, p.nseq, kBK, slot, seq, key0, key_end))) return;
+    if (!(p.s1.total_k > 0 && find_tile(p.s1.cu_k, p.nseq, kBK, slot, seq, key0, key_end, cb.k1))) {
+        if (!(p.s2.total_k > 0 && find_tile(p.s2.cu_k, p.nseq, kBK, slot, seq, key0, key_end, cb.k2))) return;
         second = true;
     }
     const BwdStream& ks = second ? p.s2 : p.s1;
-    const int k_lo = ks.cu_k[seq];
-    const int lk1 = p.s1.cu_k[seq + 1] - p.s1.cu_k[seq];
-    const int q1_lo = p.s1.total_q > 0 ? p.s1.cu_q[seq] : 0;
-    const int lq1 = p.s1.total_q > 0 ? p.s1.cu_q[seq + 1] - q1_lo : 0;
-    const int q2_lo = p.s2.total_q > 0 ? p.s2.cu_q[seq] : 0;
-    const int lq2 = p.s2.total_q > 0 ? p.s2.cu_q[seq + 1] - q2_lo : 0;
+    const LaneBounds key1 = bounds_at(cb.k1, p.s1.cu_k, seq);
+    const int k_lo = second ? bounds_at(cb.k2, p.s2.cu_k, seq).lo : key1.lo;
+    const int lk1 = key1.hi - key1.lo;
+    LaneBounds own1{0, 0}, own2{0, 0};
+    if (p.s1.total_q > 0) own1 = bounds_at(cb.q1, p.s1.cu_q, seq);
+    if (p.s2.total_q > 0) own2 = bounds_at(cb.q2, p.s2.cu_q, seq);
+    const int q1_lo = own1.lo, lq1 = own1.hi - q1_lo;
+    const int q2_lo = own2.lo, lq2 = own2.hi - q2_lo;
     const int off = lk1 - lq1;  // position of depth-0 query i is i + off
 
     // my key (accumulator column) and its position
@@ -813,27 +816,30 @@ __global__ __launch_bounds__(kLqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
 
     int seq = 0, row0 = 0, row_end = 0;
     bool second = false;
+    const CallBounds cb = call_bounds(p);
     int slot = (int)(gridDim.y - 1 - blockIdx.y);  // without a table: late (heavy) tiles of each sequence first
     // (the table's order: heaviest tile of the whole call first)
     sched_lookup(p.sched, false, p.nseq, G, p.s1.total_q, p.s2.total_q, p.s1.total_k, p.s2.total_k, (int)gridDim.y,
                  (int)blockIdx.y, slot);
-    if (!(p.s1.total_q > 0 && find_tile(p.s1.cu_q, p.nseq, BM, slot, seq, row0, row_end))) {
-        if (!(p.s2.total_q > 0 && find_tile(p.s2.cu_q, p.nseq, BM, slot, seq, row0, row_end))) return;
+    if (!(p.s1.total_q > 0 && find_tile(p.s1.cu_q, p.nseq, BM, slot, seq, row0, row_end, cb.q1))) {
+        if (!(p.s2.total_q > 0 && find_tile(p.s2.cu_q, p.nseq, BM, slot, seq, row0, row_end, cb.q2))) return;
         second = true;
     }
     const BwdStream& qs = second ? p.s2 : p.s1;
-    const int q_lo = const_i32(qs.cu_q, seq);
-    const int k1_lo = const_i32(p.s1.cu_k, seq);
-    const int lk1 = const_i32(p.s1.cu_k, seq + 1) - k1_lo;
-    const int lq1 = p.s1.total_q > 0 ? const_i32(p.s1.cu_q, seq + 1) - const_i32(p.s1.cu_q, seq) : 0;
+    LaneBounds own1{0, 0};
+    if (p.s1.total_q > 0) own1 = bounds_at(cb.q1, p.s1.cu_q, seq);
+    const LaneBounds own = second ? bounds_at(cb.q2, p.s2.cu_q, seq) : own1, key1 = bounds_at(cb.k1, p.s1.cu_k, seq);
+    const int q_lo = own.lo, q_end = own.hi;
+    const int k1_lo = key1.lo, lk1 = key1.hi - k1_lo, lq1 = own1.hi - own1.lo;
     const int off = lk1 - lq1;  // position of depth-0 query row i of the sequence is i + off
     const __bf16* k1p = p.s1.k + (int64_t)k1_lo * p.s1.k_rs + (int64_t)hk * p.s1.k_hs;
     const int left1 = p.s1.total_k - k1_lo;
     int lk2 = 0, left2 = 0;
     const __bf16* k2p = nullptr;
     if (second) {
-        const int k2_lo = const_i32(p.s2.cu_k, seq);
-        lk2 = const_i32(p.s2.cu_k, seq + 1) - k2_lo;
+        const LaneBounds key2 = bounds_at(cb.k2, p.s2.cu_k, seq);
+        const int k2_lo = key2.lo;
+        lk2 = key2.hi - k2_lo;
         k2p = p.s2.k + (int64_t)k2_lo * p.s2.k_rs + (int64_t)hk * p.s2.k_hs;
         left2 = p.s2.total_k - k2_lo;
     }
@@ -846,7 +852,6 @@ __global__ __launch_bounds__(kLqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
     const bool unit_ok = utile < ntiles_wg;
     // 64-key steps that hold a key visible to some row of 64-row tile t (depth-0 rows see positions <= row + off)
     // (the position of depth-1 row: pos_q, ascending inside a sequence, so a tile's last row has its largest)
-    const int q_end = const_i32(qs.cu_q, seq + 1);
     auto steps_of = [&](int t) {
         int reach = 64 * t + 63 + off;  // largest position a row of the tile has
         if (second) {

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace tah {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
@@ -324,14 +326,39 @@ __device__ __forceinline__ float wave_sum_xor32(float x) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-__device__ __forceinline__ int wave_reduce_max(int x) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) { int y = __shfl_xor(x, m); x = x > y ? x : y; }
-    return x;
+// x of one lane, the same one for the whole wave
+__device__ __forceinline__ int lane_value(int x, int lane) {
+#ifdef TAH_CPU_EMU
+    return __shfl(x, lane);
+#else
+    return __builtin_amdgcn_readlane(x, lane);
+#endif
 }
-__device__ __forceinline__ int wave_reduce_min(int x) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) { int y = __shfl_xor(x, m); x = x < y ? x : y; }
+__device__ __forceinline__ float lane_value(float x, int lane) { return __int_as_float(lane_value(__float_as_int(x), lane)); }
+
+// Largest / smallest of a wave, in every lane, without a trip through LDS (each of the six exchanges of a shuffle tree is one).
+template <class T, class F>
+__device__ __forceinline__ T wave_quick(T x, F pick) {
+    const auto from = [](T v, auto ctrl) {
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, true));
+    };
+    x = pick(x, from(x, std::integral_constant<int, 0xB1>{}));   // quad_perm [1,0,3,2]
+    x = pick(x, from(x, std::integral_constant<int, 0x4E>{}));   // quad_perm [2,3,0,1]
+    x = pick(x, from(x, std::integral_constant<int, 0x141>{}));  // row_half_mirror
+    x = pick(x, from(x, std::integral_constant<int, 0x140>{}));  // row_mirror
+    const auto at = [&](int lane) { return lane_value(x, lane); };
+    return pick(pick(at(0), at(16)), pick(at(32), at(48)));
+}
+__device__ __forceinline__ int wave_reduce_max(int x) { return wave_quick(x, [](int a, int b) { return a > b ? a : b; }); }
+__device__ __forceinline__ int wave_reduce_min(int x) { return wave_quick(x, [](int a, int b) { return a < b ? a : b; }); }
+// Sum over this lane and those below it, likewise.
+__device__ __forceinline__ int wave_prefix_sum(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1, 2, 4, 8: inside sixteen lanes
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
     return x;
 }
 
@@ -344,42 +371,72 @@ __device__ __forceinline__ int wave_reduce_min(int x) {
 #endif
 __device__ __forceinline__ int32_t const_i32(const int32_t* a, int i) { return ((const TAH_CONST_AS int32_t*)a)[i]; }
 
+// Boundaries of a wave's 64 sequences from b0 on, one per lane (no sequence: an empty one).  Asked for without a branch, so that a
+// kernel can have those of all its streams on their way at once.
+struct LaneBounds {
+    int lo, hi;
+};
+__device__ __forceinline__ LaneBounds lane_bounds(const int32_t* cu, int b0, int nseq) {
+    const int b = b0 + (int)(threadIdx.x % kWave);
+    const bool there = b < nseq;
+    LaneBounds x;
+    x.lo = cu[there ? b : b0];
+    x.hi = cu[there ? b + 1 : b0];
+    x.lo = there ? x.lo : 0;
+    x.hi = there ? x.hi : 0;
+    return x;
+}
+
 // Locate tile `slot` among sequences whose lengths are cu[b+1]-cu[b], `bm` rows
 // per tile.  On success fills seq/row0/row_end and returns true; otherwise
 // subtracts the number of tiles in this stream from `slot` and returns false.
 // Every lane of the wave must call it with the same arguments: the lanes take 64 sequences at a time (one pair of
 // loads and a prefix sum over the lanes), so that a batch of hundreds of short sequences costs a workgroup a few
-// steps and not one scalar load pair per sequence.
-__device__ __forceinline__ bool find_tile(const int32_t* cu, int nseq, int bm, int& slot, int& seq, int& row0, int& row_end) {
-    const int lane = (int)(threadIdx.x % kWave);
+// steps and not one scalar load pair per sequence.  `first`: lane_bounds(cu, 0, nseq), nseq > 0.
+__device__ __forceinline__ bool find_tile(const int32_t* cu, int nseq, int bm, int& slot, int& seq, int& row0, int& row_end, LaneBounds first) {
     for (int b0 = 0; b0 < nseq; b0 += kWave) {
-        const int b = b0 + lane;
-        int lo = 0, hi = 0;
-        if (b < nseq) {
-            lo = cu[b];
-            hi = cu[b + 1];
-        }
-        const int n = (hi - lo + bm - 1) / bm;
-        int incl = n;  // tiles of sequences b0 .. b
-#pragma unroll
-        for (int o = 1; o < kWave; o <<= 1) {
-            const int v = __shfl_up(incl, o);
-            if (lane >= o) incl += v;
-        }
-        const int tot = __builtin_amdgcn_readfirstlane(__shfl(incl, kWave - 1));
+        const LaneBounds x = b0 == 0 ? first : lane_bounds(cu, b0, nseq);
+        const int n = (x.hi - x.lo + bm - 1) / bm;
+        const int incl = wave_prefix_sum(n);  // tiles of sequences b0 .. b
+        const int tot = lane_value(incl, kWave - 1);
         if (slot < tot) {
             const int src = __builtin_ctzll(__ballot(slot < incl));  // the first sequence whose tiles reach past `slot`
-            const int lo_s = __builtin_amdgcn_readfirstlane(__shfl(lo, src));
-            const int hi_s = __builtin_amdgcn_readfirstlane(__shfl(hi, src));
-            const int before = __builtin_amdgcn_readfirstlane(__shfl(incl - n, src));
+            const int lo_s = lane_value(x.lo, src), hi_s = lane_value(x.hi, src);
             seq = b0 + src;
-            row0 = lo_s + (slot - before) * bm;
+            row0 = lo_s + (slot - (lane_value(incl, src) - lane_value(n, src))) * bm;
             row_end = row0 + bm < hi_s ? row0 + bm : hi_s;
             return true;
         }
         slot -= tot;
     }
     return false;
+}
+__device__ __forceinline__ bool find_tile(const int32_t* cu, int nseq, int bm, int& slot, int& seq, int& row0, int& row_end) {
+    return nseq > 0 && find_tile(cu, nseq, bm, slot, seq, row0, row_end, lane_bounds(cu, 0, nseq));
+}
+
+// The first 64 sequences' boundaries in both streams of a varlen call, asked for at once (a stream without queries or keys may
+// come without them): a workgroup's start is a chain of trips to memory, and which tile it is, where its sequence's keys lie and
+// how many there are then follow from one of them.
+struct CallBounds {
+    LaneBounds q1, k1, q2, k2;
+};
+template <class P>
+__device__ __forceinline__ CallBounds call_bounds(const P& p) {
+    const bool q2 = p.s2.total_q > 0, k2 = q2 || p.s2.total_k > 0;
+    CallBounds x;
+    x.q1 = lane_bounds(p.s1.total_q > 0 ? p.s1.cu_q : p.s1.cu_k, 0, p.nseq);
+    x.k1 = lane_bounds(p.s1.cu_k, 0, p.nseq);
+    x.q2 = lane_bounds(q2 ? p.s2.cu_q : p.s1.cu_k, 0, p.nseq);
+    x.k2 = lane_bounds(k2 ? p.s2.cu_k : p.s1.cu_k, 0, p.nseq);
+    return x;
+}
+// Those of one sequence (the same one for the whole wave)
+__device__ __forceinline__ LaneBounds bounds_at(const LaneBounds& first, const int32_t* cu, int seq) {
+    LaneBounds x;
+    x.lo = seq < kWave ? lane_value(first.lo, seq % kWave) : const_i32(cu, seq);
+    x.hi = seq < kWave ? lane_value(first.hi, seq % kWave) : const_i32(cu, seq + 1);
+    return x;
 }
 
 // ---------------------------------------------------------------------------
@@ -409,12 +466,15 @@ inline __host__ __device__ int sched_slots(int nseq, int bm, int total_1, int to
 __device__ __forceinline__ bool sched_lookup(const int32_t* sched, bool key_tiles, int nseq, int group, int total_q1,
                                              int total_q2, int total_k1, int total_k2, int slots, int idx, int& slot) {
     if (!sched) return false;
-    if (const_i32(sched, 0) != kSchedMagic || const_i32(sched, kSchedNseq) != nseq || const_i32(sched, kSchedGroup) != group ||
-        const_i32(sched, kSchedTotalQ1) != total_q1 || const_i32(sched, kSchedTotalQ2) != total_q2 ||
-        const_i32(sched, kSchedTotalK1) != total_k1 || const_i32(sched, kSchedTotalK2) != total_k2 ||
-        const_i32(sched, key_tiles ? kSchedKSlots : kSchedQSlots) != slots)
-        return false;
-    const int base = kSchedHeaderWords + (key_tiles ? 2 * const_i32(sched, kSchedQSlots) : 0);
+    // (all of the header is asked for before any of it is compared)
+    int h[kSchedKSlots + 1];
+#pragma unroll
+    for (int i = 0; i <= kSchedKSlots; ++i) h[i] = const_i32(sched, i);
+    const int other = (h[0] ^ kSchedMagic) | (h[kSchedNseq] ^ nseq) | (h[kSchedGroup] ^ group) | (h[kSchedTotalQ1] ^ total_q1) |
+                      (h[kSchedTotalQ2] ^ total_q2) | (h[kSchedTotalK1] ^ total_k1) | (h[kSchedTotalK2] ^ total_k2) |
+                      (h[key_tiles ? kSchedKSlots : kSchedQSlots] ^ slots);
+    if (other != 0) return false;
+    const int base = kSchedHeaderWords + (key_tiles ? 2 * h[kSchedQSlots] : 0);
     const int x = const_i32(sched, base + 2 * idx);
     if (x < 0 || x >= slots) return false;  // (not a table this library wrote)
     slot = x;

@@ -58,28 +58,6 @@ __device__ __host__ __forceinline__ int64_t rows_form_unit(int r, int c) {
 // element of it
 __device__ __host__ __forceinline__ int64_t rows_form_elem(int r, int c) { return rows_form_unit(r, c) * 8 + c % 8; }
 
-// x of one lane, the same one for the whole wave
-__device__ __forceinline__ float lane_value(float x, int lane) {
-#ifdef TAH_CPU_EMU
-    return __shfl(x, lane);
-#else
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
-#endif
-}
-
-// Largest float / smallest int of a wave, in every lane, without a trip through LDS.
-template <class T, class F>
-__device__ __forceinline__ T wave_quick(T x, F pick) {
-    const auto from = [](T v, auto ctrl) {
-        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, true));
-    };
-    x = pick(x, from(x, std::integral_constant<int, 0xB1>{}));   // quad_perm [1,0,3,2]
-    x = pick(x, from(x, std::integral_constant<int, 0x4E>{}));   // quad_perm [2,3,0,1]
-    x = pick(x, from(x, std::integral_constant<int, 0x141>{}));  // row_half_mirror
-    x = pick(x, from(x, std::integral_constant<int, 0x140>{}));  // row_mirror
-    const auto at = [&](int lane) { return __builtin_bit_cast(T, __float_as_int(lane_value(__builtin_bit_cast(float, x), lane))); };
-    return pick(pick(at(0), at(16)), pick(at(32), at(48)));
-}
 __device__ __forceinline__ float wave_max_quick(float x) { return wave_quick(x, [](float a, float b) { return fmaxf(a, b); }); }
 __device__ __forceinline__ int wave_min_quick(int x) { return wave_quick(x, [](int a, int b) { return a < b ? a : b; }); }
 

@@ -127,3 +127,17 @@ def test_fwd_bwd_headline_seq8192_vs_torch_fp32():
     ((r1 * do1.float()).sum() + (r2 * do2.float()).sum()).backward()
     want = [leaf[n].grad.cpu().numpy() for n in ("q1", "k1", "v1", "q2", "k2", "v2")]
     print("headline fwd+bwd:", check_grads(got, want), flush=True)
+
+
+@pytest.mark.parametrize("nseq", [64, 65, 129])
+def test_boundaries_of_more_sequences_than_a_wave_has_lanes(nseq):
+    """A workgroup takes its sequence's boundaries from the first 64 that its lanes hold, or reads them: empty and one-token
+    sequences on both sides of that line, prefixes in the cache, outputs' gradients against the oracle."""
+    lens = [(7 * i) % 90 + 1 for i in range(nseq)]
+    more = [n + (5 * i) % 40 for i, n in enumerate(lens)]
+    lens[0] = lens[-2] = 1
+    print(f"boundaries nseq={nseq}", flush=True)
+    dev = to_device(make_varlen_case(31 + nseq, lens, 0.2, Hq=4, Hkv=2, D=128, seqlens_k=more, extra_k2=3 * nseq))
+    got, want = run_bwd(dev, nseq)
+    torch.cuda.synchronize()
+    print(check_grads(got, want), flush=True)
