@@ -56,6 +56,12 @@ constexpr int kSmemBytes = kStageOff + 8 * 8192;
 // The 4-wave variant (two workgroups per compute unit) stages its output over the K / V rings, which are dead by then.
 constexpr int kSmemBytes4 = kStageOff;
 static_assert(4 * 8192 <= kPosRing, "the 4-wave variant's output staging must fit the K / V rings");
+// kPair: what the two waves of 32 query rows hand each other, per pair: probabilities (four operands of 64 lanes), and a number per
+// query and wave.
+constexpr int kPairP = kStageOff;
+constexpr int kPairPBytes = 4 * kWave * 16;
+constexpr int kPairNum = kPairP + 2 * kPairPBytes;
+constexpr int kSmemBytesPair = kPairNum + 2 * 2 * 32 * 4;
 
 struct FwdStream {
     const __bf16 *q, *k, *v;
@@ -87,11 +93,18 @@ enum class Mask { kNone, kIndex, kPos, kDense };
 // the two drift freely against each other (the dispatcher starts them at different times and their tile counts
 // differ), one workgroup's prologue, epilogue and hand-over to its successor run under the other's tile loop, and a
 // workgroup needs one barrier per tile.  Each workgroup stages its own K / V tiles (twice the copies per MFMA).
-template <int G, bool kDense, int W>
+// kPair (4 waves, up to two query heads per kv head): a launch with fewer workgroups than compute units takes as long as its longest
+// tile, one key tile after another with a single wave on each SIMD.  Two waves then share 32 query rows: each takes half of a key
+// tile's keys for the scores and the softmax and half of the output's columns for the product with V, so half of the matrix and
+// vector work stands one behind the other; the maxima and the probabilities travel through LDS, two barriers a tile.  A row's
+// keys are taken in the same order under the same reference, and every sum has the terms and the order of the other forms: the same bits.
+template <int G, bool kDense, int W, bool kPair = false>
 __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(const FwdParams p) {
     static_assert(W == 8 || W == 4, "8 or 4 waves");
-    static_assert(W >= G, "a workgroup holds every query head of its kv head");
-    constexpr int BM = 32 * (W / G);
+    constexpr int kTeams = kPair ? 2 : 1, kBlocks = W / kTeams;  // kBlocks: (head, 32 rows) per workgroup
+    static_assert(kBlocks >= G && (!kPair || (W == 4 && !kDense)), "a workgroup holds every query head of its kv head");
+    constexpr int kKeyBlocks = 2 / kTeams, kDimBlocks = 4 / kTeams;  // of 32, per wave: keys of a tile, columns of the output
+    constexpr int BM = 32 * (kBlocks / G);
     constexpr int kRowsPerWave = kBN / W;       // rows of a K / V tile each wave copies
     constexpr int kPieces = kRowsPerWave / 4;   // in pieces of 4 rows (one copy instruction each)
     HIP_DYNAMIC_SHARED(unsigned char, smem)
@@ -102,6 +115,7 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     const int half = lane / 32;
     const int col = lane % 32;
     const int hk = blockIdx.x;
+    const int team = kPair ? wave / kBlocks : 0, block = wave % kBlocks;
 
     // ---- which tile am I ---------------------------------------------------
     // (all boundaries in one trip, together with the table, and scalar arithmetic on them: 333 rows, where the last workgroup's start was
@@ -110,8 +124,8 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     const bool has1 = p.s1.total_q > 0, has2 = p.s2.total_q > 0;
     int seq = 0, row0 = 0, row_end = 0;
     bool second = false;
-    // (the launch-order table lists tiles of 256 / G rows: a 4-wave workgroup takes one half of an entry)
-    constexpr int kPerEntry = 8 / W;
+    // (the launch-order table lists tiles of 256 / G rows: a 4-wave workgroup takes one half of an entry, or a quarter)
+    constexpr int kPerEntry = 8 / kBlocks;
     int slot;
     if (sched_lookup(p.sched, false, p.nseq, G, p.s1.total_q, p.s2.total_q, p.s1.total_k, p.s2.total_k,
                      (int)gridDim.y / kPerEntry, (int)blockIdx.y / kPerEntry, slot)) {
@@ -132,8 +146,8 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     }
     const FwdStream& qs = second ? p.s2 : p.s1;
 
-    const int head = hk * G + wave % G;
-    const int rblk = wave / G;
+    const int head = hk * G + block % G;
+    const int rblk = block / G;
     // depth-0 key segment of this sequence (position of a key = its local index)
     const LaneBounds key1 = bounds_at(cb.k1, p.s1.cu_k, seq);
     const int k1_lo = key1.lo, lk1 = key1.hi - k1_lo;
@@ -214,13 +228,15 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
         for (int s = 0; s < 8; ++s) qf[s] = ld_global_16B(qrow + 16 * s);
     }
 
-    f32x16 oacc[4];
+    f32x16 oacc[kDimBlocks];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < kDimBlocks; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
     float m_run = kNegInf;  // running max of raw scores
-    float l_run = 0.f;      // this lane's share of the running denominator
+    float l_run[kKeyBlocks];  // this lane's share of the running denominator, keys 0-31 and 32-63 of the tiles apart
+#pragma unroll
+    for (int mt = 0; mt < kKeyBlocks; ++mt) l_run[mt] = 0.f;
     const float c = p.scale_log2e;
 
     // ---- asynchronous global -> LDS copies (no registers, no ds_write) ------------------------
@@ -272,32 +288,34 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     int koff[8];       // K row `col` (+32 per mt), chunk 2s + half
 #pragma unroll
     for (int s8 = 0; s8 < 8; ++s8) koff[s8] = rowmajor128_off(col, 2 * s8 + half);
-    int voff_lo[4], voff_hi[4];  // V rows 4*half + r/4 (+8), columns 32*dt + 16*grp + 4*(r%4), +16 rows per step
+    int voff_lo[kDimBlocks], voff_hi[kDimBlocks];  // V rows 4*half + r/4 (+8), columns 32*dt + 16*grp + 4*(r%4), +16 rows per step
     {
         const int r16 = lane & 15, grp = (lane >> 4) & 1;
         const int vrow = 4 * half + (r16 >> 2);
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-            const int vcol = 32 * dt + 16 * grp + 4 * (r16 & 3);
+        for (int dt = 0; dt < kDimBlocks; ++dt) {
+            const int vcol = 32 * (kDimBlocks * team + dt) + 16 * grp + 4 * (r16 & 3);
             voff_lo[dt] = rowmajor128_off(vrow, vcol >> 3) + (vcol & 7) * 2;
             voff_hi[dt] = rowmajor128_off(vrow + 8, vcol >> 3) + (vcol & 7) * 2;
         }
     }
 
-    f32x16 sacc[2];    // S^T of the tile in flight: written by M(t-1), consumed by X(t)
-    bf16x8 pfrag[4];   // its probabilities: written by X(t), consumed by M(t)
+    f32x16 sacc[kKeyBlocks];  // S^T of the tile in flight: written by M(t-1), consumed by X(t)
+    bf16x8 pfrag[4];          // its probabilities: written by X(t), consumed by M(t) (kPair: through LDS, [operand][lane])
+    [[maybe_unused]] bf16x8* const pair_p = reinterpret_cast<bf16x8*>(smem + kPairP + (block % 2) * kPairPBytes) + lane;
+    [[maybe_unused]] float* const pair_num = reinterpret_cast<float*>(smem + kPairNum) + (block % 2) * 64 + col;  // [wave of the pair][query]
 
     // ---- matrix phase pieces -------------------------------------------------------------------
     auto qk = [&](int it) __attribute__((always_inline)) {  // S^T = K(it) Q^T
-        const unsigned char* kt = smem + kKRing + (it % kStages) * kKBytes;
+        const unsigned char* kt = smem + kKRing + (it % kStages) * kKBytes + team * 8192;
         const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
+        for (int mt = 0; mt < kKeyBlocks; ++mt)
             sacc[mt] = mfma32(*reinterpret_cast<const bf16x8*>(kt + koff[0] + mt * 8192), qf[0], zero);
 #pragma unroll
         for (int s = 1; s < 8; ++s)
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt)
+            for (int mt = 0; mt < kKeyBlocks; ++mt)
                 sacc[mt] = mfma32(*reinterpret_cast<const bf16x8*>(kt + koff[s] + mt * 8192), qf[s], sacc[mt]);
     };
     auto pv = [&](int it) __attribute__((always_inline)) {  // O^T (128 d x 32 queries) += V(it)^T P^T
@@ -305,7 +323,7 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
 #pragma unroll
-            for (int dt = 0; dt < 4; ++dt) {
+            for (int dt = 0; dt < kDimBlocks; ++dt) {
                 const bf16x4 lo = lds_read_tr16(vt + voff_lo[dt] + st * 4096);
                 const bf16x4 hi = lds_read_tr16(vt + voff_hi[dt] + st * 4096);
                 oacc[dt] = mfma32(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), pfrag[st], oacc[dt]);
@@ -317,17 +335,21 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     auto matrix = [&](int t, auto qk_tag) __attribute__((always_inline)) {
         constexpr bool kQk = decltype(qk_tag)::value;
         __builtin_amdgcn_s_setprio(kMatrixPrio);  // the matrix pipe is the scarce one: its wave issues first
+        if constexpr (kPair) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pfrag[i] = pair_p[i * kWave];
+        }
         pv(t);
         if constexpr (kQk) qk(t + 1);
-        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, kPair ? 12 : 8, 0);
 #pragma unroll
-        for (int i = 0; i < 12; ++i) {
+        for (int i = 0; i < 4 * kDimBlocks - 4; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
         }
         if constexpr (kQk) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
+            for (int i = 0; i < 8 * kKeyBlocks; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             }
@@ -340,19 +362,19 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     auto next_active = [&](int t) { return t + 1 < n_active || (t + 1 >= n1 && t + 1 < ntiles); };
 
     // ---- vector phase: mask, online softmax (one query per lane column, two lanes per query) ----
-    auto softmax = [&](int it, auto mask_tag) __attribute__((always_inline)) {
+    auto mask_scores = [&](int it, auto mask_tag) __attribute__((always_inline)) {
         constexpr Mask kMask = decltype(mask_tag)::value;
         if constexpr (kMask == Mask::kIndex) {
-            const int base = it * kBN;
+            const int base = it * kBN + 32 * team;
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt)
+            for (int mt = 0; mt < kKeyBlocks; ++mt)
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     sacc[mt][r] = base + 32 * mt + acc_row(half, r) <= qlim1 ? sacc[mt][r] : kNegInf;
         } else if constexpr (kMask == Mask::kDense) {
             const int base = it * kBN;
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt)
+            for (int mt = 0; mt < kKeyBlocks; ++mt)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int kk = base + 32 * mt + acc_row(half, r);
@@ -363,22 +385,27 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
                     sacc[mt][r] = kk <= qlim1 ? sacc[mt][r] + mv * p.inv_scale : kNegInf;
                 }
         } else if constexpr (kMask == Mask::kPos) {
-            const int* kpos = reinterpret_cast<const int*>(smem + kPosRing + (it % kPosSlots) * (kBN * 4));
-            const int nleft = lk2 - (it - n1) * kBN;  // keys of this tile that exist
+            const int* kpos = reinterpret_cast<const int*>(smem + kPosRing + (it % kPosSlots) * (kBN * 4)) + 32 * team;
+            const int nleft = lk2 - (it - n1) * kBN - 32 * team;  // keys of this tile that exist
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt)
+            for (int mt = 0; mt < kKeyBlocks; ++mt)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int kk = 32 * mt + acc_row(half, r);
                     sacc[mt][r] = (kk < nleft && kpos[kk] <= qlim2) ? sacc[mt][r] : kNegInf;
                 }
         }
+    };
+    auto score_max = [&]() __attribute__((always_inline)) {
         float mx = kNegInf;
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
+        for (int mt = 0; mt < kKeyBlocks; ++mt)
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sacc[mt][r]);
-        mx = wave_max_xor32(mx);
+        return wave_max_xor32(mx);
+    };
+    // probabilities of masked scores, given the largest score of every query of the wave
+    auto probabilities = [&](float mx) __attribute__((always_inline)) {
         // Lazy reference: the exponent reference m_run follows the true row maximum only when that
         // has grown by more than kLazy (log2 units) for some row of the wave; until then
         // probabilities may reach 2^kLazy, which fp32 sums and bf16 operands absorb, and the 64
@@ -391,23 +418,28 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
         const float alpha = fast_exp2((m_run - m_use) * c);  // 1 when nothing changes, 0 from -inf
         m_run = m_next;
         const float mc = m_use * c;
-        float psum = 0.f;
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
+        for (int mt = 0; mt < kKeyBlocks; ++mt) {
+            float psum = 0.f;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const float e = fast_exp2(sacc[mt][r] * c - mc);
                 psum += e;
                 pfrag[2 * mt + r / 8][r % 8] = (__bf16)e;
             }
-        l_run = l_run * alpha + psum;
+            l_run[mt] = l_run[mt] * alpha + psum;
+        }
         f32x16* const op = oacc;  // (asm operands alone do not make a lambda capture the array)
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) TAH_SCALE16_IF(op[dt], alpha, any_grow);
+        for (int dt = 0; dt < kDimBlocks; ++dt) TAH_SCALE16_IF(op[dt], alpha, any_grow);
         // Pin the results here: without a use inside this phase the optimiser sinks the whole
         // computation to its first consumer, i.e. past the barrier into the matrix phase.
-        TAH_KEEP_HERE4(pfrag[0], pfrag[1], pfrag[2], pfrag[3]);
-        TAH_KEEP_HERE4(op[0], op[1], op[2], op[3]);
+        if constexpr (!kPair) TAH_KEEP_HERE4(pfrag[0], pfrag[1], pfrag[2], pfrag[3]);
+        TAH_KEEP_HERE4(op[0], op[1], op[kDimBlocks - 2], op[kDimBlocks - 1]);
+    };
+    auto softmax = [&](int it, auto mask_tag) __attribute__((always_inline)) {
+        mask_scores(it, mask_tag);
+        probabilities(score_max());
     };
     using PlainTag = std::integral_constant<Mask, Mask::kNone>;
     using IndexTag = std::integral_constant<Mask, kDense ? Mask::kDense : Mask::kIndex>;
@@ -441,6 +473,29 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
         TAH_PHASE_BARRIER();
         issue(t + 1);
         matrix(t, qk_tag);
+    };
+    // kPair: the barrier between the maxima and the probabilities, and the one that publishes those and the copies.  What stands behind
+    // either is written by nobody before the other.
+    [[maybe_unused]] auto step_pair = [&](int t, auto tag, auto qk_tag) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        mask_scores(t, tag);
+        const float mx = score_max();
+        if (half == 0) pair_num[32 * team] = mx;
+        TAH_PHASE_BARRIER();
+        probabilities(fmaxf(mx, pair_num[32 * (1 - team)]));
+        pair_p[(2 * team) * kWave] = pfrag[0];
+        pair_p[(2 * team + 1) * kWave] = pfrag[1];
+        TAH_WAIT_VMEM();
+        TAH_PHASE_BARRIER();
+        issue(t + 1);
+        matrix(t, qk_tag);
+    };
+    [[maybe_unused]] auto idle_pair = [&](int t) __attribute__((always_inline)) {
+        TAH_PHASE_BARRIER();
+        TAH_WAIT_VMEM();
+        TAH_PHASE_BARRIER();
+        issue(t + 1);
+        if (next_active(t)) qk(t + 1);
     };
     auto idle_single = [&](int t) __attribute__((always_inline)) {
         TAH_WAIT_VMEM();
@@ -479,7 +534,8 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     auto run = [&](auto late_tag) __attribute__((always_inline)) {
         constexpr bool kLate = decltype(late_tag)::value;
         auto step = [&](int t, auto tag, auto qk_tag) __attribute__((always_inline)) {
-            if constexpr (W == 4) step_single(t, tag, qk_tag);
+            if constexpr (kPair) step_pair(t, tag, qk_tag);
+            else if constexpr (W == 4) step_single(t, tag, qk_tag);
             else if constexpr (kLate) step_late(t, tag, qk_tag);
             else step_early(t, tag, qk_tag);
         };
@@ -491,7 +547,8 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
         for (; t < act_q; ++t) step(t, IndexTag{}, WithQk{});
         for (; t < n_active; ++t) step(t, IndexTag{}, NoQk{});
         for (; t < n1; ++t) {
-            if constexpr (W == 4) idle_single(t);
+            if constexpr (kPair) idle_pair(t);
+            else if constexpr (W == 4) idle_single(t);
             else if constexpr (kLate) idle_late(t);
             else idle_early(t);
         }
@@ -508,43 +565,55 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
         if (W == 4 || late_set(wave) == 0) run(std::false_type{});
         else run(std::true_type{});
     }
+    float l_part[2];  // the denominators of the keys 0-31 and 32-63 of all tiles
+#pragma unroll
+    for (int mt = 0; mt < kKeyBlocks; ++mt) l_part[mt] = wave_sum_xor32(l_run[mt]);
+    if constexpr (kPair) {
+        if (half == 0) pair_num[32 * team] = l_part[0];  // (the last maxima were read before the last barrier)
+    }
     if constexpr (W == 4) {  // the output staging below overlies the rings: every wave must be done reading them
         TAH_WAIT_VMEM();
         TAH_PHASE_BARRIER();
     }
 #undef TAH_PHASE_BARRIER
+    if constexpr (kPair) {
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) l_part[mt] = pair_num[32 * mt];
+    }
 
     // ---- epilogue -----------------------------------------------------------
-    const float l_tot = wave_sum_xor32(l_run);
+    const float l_tot = l_part[0] + l_part[1];
     const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
     // The accumulators hold O^T (a lane owns one query row, four values of d at a time): written out
     // directly every store instruction would touch 32 rows with 8 bytes each.  The wave turns its
-    // 32 x 128 tile through a private piece of LDS instead (16-byte chunks of a row XOR-swizzled by the
-    // row number, so that neither side runs into bank conflicts) and stores whole rows: 4 rows x 256
+    // 32 x 128 tile (kPair: 32 x 64) through a private piece of LDS instead (16-byte chunks of a row XOR-swizzled by the
+    // row number, so that neither side runs into bank conflicts) and stores whole rows: 4 rows x 256 (8 x 128)
     // contiguous bytes per instruction.  Nobody else reads or writes this piece: no barrier.
+    constexpr int kRowBytes = 64 * kDimBlocks, kChunks = kRowBytes / 16;  // of a row, and 16-byte chunks of it
     unsigned char* stage = smem + (W == 4 ? 0 : kStageOff) + wave * 8192;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int dt = 0; dt < kDimBlocks; ++dt)
 #pragma unroll
         for (int g4 = 0; g4 < 4; ++g4) {
             bf16x4 v4;
 #pragma unroll
             for (int b = 0; b < 4; ++b) v4[b] = (__bf16)(oacc[dt][4 * g4 + b] * inv);
-            *reinterpret_cast<bf16x4*>(stage + col * 256 + (((4 * dt + g4) ^ (col & 15)) * 16) + half * 8) = v4;
+            *reinterpret_cast<bf16x4*>(stage + col * kRowBytes + (((4 * dt + g4) ^ (col & (kChunks - 1))) * 16) + half * 8) = v4;
         }
     TAH_WAVE_LDS_SYNC();  // the reads below are of other lanes' writes
     {
-        const int ch = lane & 15;
-        __bf16* obase = qs.o + (int64_t)head * qs.o_hs + ch * 8;
+        constexpr int kRowsAtOnce = kWave / kChunks;
+        const int ch = lane % kChunks;
+        __bf16* obase = qs.o + (int64_t)head * qs.o_hs + kRowBytes / 2 * team + ch * 8;
         const int tile_row0 = row0 + rblk * 32;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int r = 4 * i + (lane >> 4);
-            const bf16x8 v = *reinterpret_cast<const bf16x8*>(stage + r * 256 + ((ch ^ (r & 15)) * 16));
+        for (int i = 0; i < 32 / kRowsAtOnce; ++i) {
+            const int r = kRowsAtOnce * i + lane / kChunks;
+            const bf16x8 v = *reinterpret_cast<const bf16x8*>(stage + r * kRowBytes + ((ch ^ (r & (kChunks - 1))) * 16));
             if (tile_row0 + r < row_end) st_global_16B(obase + (int64_t)(tile_row0 + r) * qs.o_rs, v);
         }
     }
-    if (row_ok && half == 0)
+    if (row_ok && half == 0 && team == 0)
         qs.lse[(int64_t)head * qs.total_q + row] = l_tot > 0.f ? (m_run * c + fast_log2(l_tot)) * kLn2 : kNegInf;
 }
 
@@ -587,12 +656,33 @@ int check_stream(const tah_duo_stream& s, bool second) {
     return TAH_OK;
 }
 
+// Launches that take kPair (workgroups counted as that form launches them, 256 compute units of two each): while all of them are resident
+// at once, and where sequences are long, so that a workgroup's tiles and not its start fill its time, up to three and a half
+// per compute unit.  16 / 8 heads, 6 % hard tokens, us without and with it: 333 rows 15.9 -> 13.3, 512 19.6 -> 16.1, 1024 32.1 -> 25.2, 2048
+// 55.7 -> 47.2, 3000 79.4 -> 69.2 (832 workgroups), 3500 92.4 -> 91.1 (960), 4096 111.8 -> 110.2 (1120); four sequences of 256 13.6 -> 12.2 (512),
+// five of 300 16.1 -> 16.6 (672), six 16.5 -> 18.5 (832), four of 512 22.2 -> 19.4 (768), five 23.1 -> 23.8 (992), four of 1000 37.6 -> 44.5 (1280);
+// depth-1 queries alone, 881 of four sequences 86 -> 69 (320), 2568 of four 109 -> 116 (768).
+constexpr long kPairWorkgroups = 576, kPairWorkgroupsLong = 896;
+constexpr int kPairLongRows = 512;
+inline bool pair_launch(const FwdParams& p, long workgroups) {
+    return workgroups <= kPairWorkgroups || (workgroups <= kPairWorkgroupsLong && p.s1.total_q / p.nseq >= kPairLongRows);
+}
+
 template <int G, bool kDense>
 int launch_fwd(const FwdParams& p, hipStream_t stream) {
     constexpr int BM = 32 * (8 / G);
     int tiles = 0;  // upper bound on sum_b ceil(len_b / BM), no device read needed
     if (p.s1.total_q > 0) tiles += p.s1.total_q / BM + p.nseq;
     if (p.s2.total_q > 0) tiles += p.s2.total_q / BM + p.nseq;
+    if constexpr (!kDense && G <= 2) {
+        if (pair_launch(p, 4l * p.hkv * tiles)) {
+            if (hipFuncSetAttribute(reinterpret_cast<const void*>(&duo_fwd_kernel<G, kDense, 4, true>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytesPair) != hipSuccess)
+                return TAH_E_LAUNCH;
+            hipLaunchKernelGGL((duo_fwd_kernel<G, kDense, 4, true>), dim3(p.hkv, 4 * tiles), dim3(256), kSmemBytesPair, stream, p);
+            return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
+        }
+    }
     // duo-causal calls with up to four query heads per kv head: 4-wave workgroups, two per compute unit (same results
     // to the bit; measured 0-5 % faster than the 8-wave form, most with several short documents)
     if constexpr (!kDense && G <= 4) {

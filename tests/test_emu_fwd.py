@@ -152,3 +152,18 @@ def test_fwd_kernel_chains_of_key_tiles_on_cpu_shim(hq, hkv, seqlens, p, drift):
     with emu_util.emulated():
         got = ops.duo_fwd_varlen(*varlen_args(dev))
     _check(dev, got)
+
+
+@pytest.mark.parametrize("lens,p", [([97], 0.3), ([64, 1, 33], 0.5)])
+def test_two_waves_to_the_same_rows_give_the_bits_of_one(lens, p):
+    """Few workgroups: two waves share 32 query rows (two heads of a kv head, and one).  The same heads four at a time run with a
+    wave to 32 rows: the same bits, outputs and LSE, with a reference that moves (tile edges, idle waves, one-row sequences)."""
+    from tah_amd import ops
+    four = _to_dev(add_score_drift(make_varlen_case(71, lens, p, Hq=4, Hkv=1, D=128), 0.2))
+    with emu_util.emulated():
+        want = ops.duo_fwd_varlen(*varlen_args(four))
+        for h, n in ((0, 2), (2, 2), (3, 1)):
+            part = dict(four, q1=four["q1"][:, h:h + n].contiguous(), q2=four["q2"][:, h:h + n].contiguous())
+            o1, lse1, o2, lse2 = ops.duo_fwd_varlen(*varlen_args(part))
+            assert torch.equal(o1, want[0][:, h:h + n]) and torch.equal(lse1, want[1][h:h + n])
+            assert torch.equal(o2, want[2][:, h:h + n]) and torch.equal(lse2, want[3][h:h + n])
