@@ -32,6 +32,7 @@ from __future__ import annotations
 
 import dataclasses
 import math
+import weakref
 from typing import List, Optional, Tuple
 
 import torch
@@ -194,6 +195,45 @@ def rope_tables(max_len: int, head_dim: int, theta: float, device, dtype=torch.b
     return emb.cos().to(dtype).to(device), emb.sin().to(dtype).to(device)
 
 
+_PLAIN = (int, float, str, bool, type(None), torch.dtype, torch.device)
+
+
+def _leaves(x, out: list, seen: set) -> list:
+    """What a captured step may hold of ``x``, in a fixed order: plain values, tensors with their addresses, and objects that are
+    neither (kernel objects), the latter two weakly.  Containers and this package's objects are walked, engines are not."""
+    if isinstance(x, _PLAIN):
+        out.append(x)
+    elif isinstance(x, torch.Tensor):
+        out.append((weakref.ref(x), x.data_ptr()))
+    elif isinstance(x, dict):
+        for k, v in x.items():
+            out.append(k)
+            _leaves(v, out, seen)
+    elif isinstance(x, (list, tuple)):
+        out.append(len(x))
+        for v in x:
+            _leaves(v, out, seen)
+    elif isinstance(x, DecodeEngine):
+        pass
+    elif type(x).__module__.startswith("tah_amd.") and hasattr(x, "__dict__"):
+        if id(x) not in seen:
+            seen.add(id(x))
+            for k, v in vars(x).items():
+                out.append(k)
+                _leaves(v, out, seen)
+    else:
+        out.append((weakref.ref(x), None))
+    return out
+
+
+def _same_leaves(a: list, b: list) -> bool:
+    def same(x, y):
+        if isinstance(x, tuple) and isinstance(y, tuple) and isinstance(x[0], weakref.ref):
+            return x[0]() is not None and x[0]() is y[0]() and x[1] == y[1]
+        return type(x) is type(y) and x == y  # (keys of dictionaries may be tuples of plain values)
+    return len(a) == len(b) and all(same(x, y) for x, y in zip(a, b))
+
+
 class DecodeEngine:
     """What every model's engine shares: the generation state of a batch of rows (on the device), sampling, the greedy
     step's bookkeeping, the loop, and its step captured in a HIP graph.  A model's engine provides ``_parts``, one step
@@ -216,6 +256,7 @@ class DecodeEngine:
         self.greedy_workspace = ops.greedy_workspace(batch, dev)
         self.host_positions = 0  # upper bound on any sequence's length, kept on the host for capacity checks
         self._graph = None
+        self._graph_over = None  # what the captured step holds, where another batch may replay it
 
     def _parts(self):
         """One step of all rows on the engine's own state: (logits, logits of a second iteration or None, which rows
@@ -225,6 +266,26 @@ class DecodeEngine:
     def _hold_state(self):
         """Called before a warm-up step; returns a function that undoes what the step changed."""
         raise NotImplementedError
+
+    # attributes that change from call to call and are no part of a captured step
+    _BETWEEN_STEPS = ("host_positions", "host_hard_rows", "ticks", "binding", "pool", "pass_open", "decision_logits", "draw_again",
+                      "_positions_on_device", "_graph", "_graph_key", "_graph_over", "_tick_graphs", "_tick_key", "_tick_over")
+
+    def _captured_over(self) -> list:
+        """Everything of the engine and its weights that a captured step may hold."""
+        out, seen = [], {id(self)}
+        for k, v in vars(self).items():
+            if k not in self._BETWEEN_STEPS:
+                out.append(k)
+                _leaves(v, out, seen)
+        return out
+
+    def _new_batch(self) -> None:
+        """A new batch begins: a step captured for an earlier one is kept where all that it holds is still the engine's (a step of
+        generate_1's size takes 1.8 ms to warm up and capture, one of 32 rows 4.5) and where replaying it leaves the random
+        numbers as capturing it would."""
+        if self._graph is not None and not (self._graph_over is not None and _same_leaves(self._graph_over, self._captured_over())):
+            self._graph = self._graph_over = None
 
     def _launch_switches(self):
         """Every attribute that changes which kernels a captured step launches: part of the graph keys, so that
@@ -402,6 +463,7 @@ class DecodeEngine:
         with torch.cuda.graph(g):
             self._step_inplace(temperature, eos, **filters)
         self._graph, self._graph_key = g, key
+        self._graph_over = self._captured_over() if temperature <= 0.0 else None  # (draws inside a step: the warm-up took some too)
         return g
 
 
@@ -487,6 +549,8 @@ class TaHDecodeEngine(DecodeEngine):
             self.eligible = torch.zeros(batch, dtype=torch.bool, device=dev)
             self.logits2 = [torch.zeros(batch, cfg.vocab, dtype=torch.bfloat16, device=dev) for _ in range(2)]
         self._tick_graphs = None
+        self._tick_over = None
+        self.draw_again = False  # kept graphs: the numbers that their warm-up would have drawn for this batch are not drawn yet
         # Engines with a workspace draw a row's n-th token with the number a step-wise loop would draw it with: a table of the
         # steps' uniforms, one row per token, so that sampled tokens do not depend on the schedule either.
         self.uniforms = (torch.zeros(max_len + 1, batch, dtype=torch.float32, device=dev)
@@ -765,8 +829,7 @@ class TaHDecodeEngine(DecodeEngine):
         self.n_hard.zero_()
         self.n_steps.zero_()
         self.host_hard_rows = 0
-        self._graph = None  # (its warm-up step belongs to the old batch's state)
-        self._tick_graphs = None
+        self._new_batch()
         self.phase.zero_()
         seq = torch.repeat_interleave(torch.arange(B, device=dev), torch.tensor(lens, device=dev))
         pos = (torch.arange(N, device=dev) - cu.long()[seq]).to(torch.int32)
@@ -844,6 +907,14 @@ class TaHDecodeEngine(DecodeEngine):
         return logits_last.float(), hard
 
     # ── generation ───────────────────────────────────────────────────────
+    def _new_batch(self) -> None:
+        if self.decider is not None:  # (leaves the last decision's logits where a capture puts them)
+            self._graph = self._tick_graphs = None
+        super()._new_batch()
+        if self._tick_graphs is not None and not (self._tick_over is not None and _same_leaves(self._tick_over, self._captured_over())):
+            self._tick_graphs = self._tick_over = None
+        self.draw_again = self._tick_graphs is not None
+
     def _state(self):
         return super()._state() + (self.hard_len, self.phase)
 
@@ -946,10 +1017,15 @@ class TaHDecodeEngine(DecodeEngine):
         """The tick as two HIP graphs, one per logits buffer, after a warm-up tick whose state changes are undone."""
         self._close_pass()
         key = (eos, limit, self.w.threshold, temperature, tuple(sorted(filters.items()))) + self._launch_switches()
+        by_step = self._draws_by_step(temperature, filters)
         if self._tick_graphs is not None and self._tick_key == key:
+            if self.draw_again and by_step:
+                torch.rand(self.B, device=self.device)
+            self.draw_again = False
             return self._tick_graphs
+        self.draw_again = False
         undo = self._hold_state()
-        if self._draws_by_step(temperature, filters):
+        if by_step:
             torch.rand(self.B, device=self.device)  # what the warm-up step of ``capture`` draws
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
@@ -965,6 +1041,7 @@ class TaHDecodeEngine(DecodeEngine):
                 self._tick(parity, eos, limit, temperature, **filters)
             graphs.append(g)
         self._tick_graphs, self._tick_key = graphs, key
+        self._tick_over = self._captured_over() if temperature <= 0.0 or by_step else None
         return graphs
 
     def _generate_ticks(self, first_logits: torch.Tensor, max_new_tokens: int, eos: int, use_graph: bool, check_every: int = 64,

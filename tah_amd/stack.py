@@ -324,7 +324,7 @@ class StackEngine(DecodeEngine):
         self._positions_on_device = False
         self.n_hard.zero_()
         self.n_steps.zero_()
-        self._graph = None
+        self._new_batch()
         step = portion or max(lens)
         first = torch.empty(self.B, self.cfg.vocab, dtype=torch.float32, device=self.device)
         for at in range(0, max(lens), step):

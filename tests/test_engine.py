@@ -753,3 +753,51 @@ def test_graphs_behind_a_pass_that_broke_off_gpu(monkeypatch):
             graphs[0].replay()
             assert torch.equal(e.logits2[0], want)
             undo()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("temperature", [0.0, 0.7])
+def test_a_captured_tick_serves_the_next_batch_gpu(temperature):
+    """Batches one after another on one engine, the captured ticks kept between them or dropped: the same tokens and the same state of the
+    generator behind them.  Kept they are while the engine's weights, buffers and switches are the ones captured."""
+    from tah_amd.engine import EngineConfig, TaHDecodeEngine, Weights
+    g = torch.Generator().manual_seed(2)
+    batches = [(torch.randint(0, 4096, (n,), generator=g).cuda(), torch.tensor([0, a, n], dtype=torch.int32).cuda()) for n, a in ((50, 30), (21, 4), (77, 50))]
+
+    def run(keep):
+        e = TaHDecodeEngine(Weights.random_init(EngineConfig(layers=3, vocab=4096), "cuda", seed=3), 2, 128)
+        e.w.threshold = 0.5
+        torch.manual_seed(7)
+        out, graphs = [], []
+        for ids, cu in batches:
+            if not keep:
+                e._tick_graphs = None
+            first, _ = e.prefill(ids, cu)
+            out.append(e.generate(first, 20, temperature=temperature).clone())
+            graphs.append(e._tick_graphs)
+        return e, graphs, out + [torch.rand(3, device="cuda")]
+
+    with torch.no_grad():
+        e, graphs, got = run(True)
+        assert graphs[0] is graphs[1] and graphs[1] is graphs[2]
+        for a, b in zip(got, run(False)[2]):
+            assert torch.equal(a, b)
+
+        def next_batch():
+            was = e._tick_graphs
+            first, _ = e.prefill(*batches[0])
+            tokens = e.generate(first, 20, temperature=0.0)
+            assert e._tick_graphs is not None
+            return e._tick_graphs is was, tokens.clone()
+
+        next_batch()
+        kept, want = next_batch()
+        assert kept
+        e.w.layers[1]["wo_p"] = e.w.layers[1]["wo_p"].clone()  # the same numbers elsewhere
+        kept, same = next_batch()
+        assert not kept and torch.equal(want, same) and next_batch()[0]
+        e.w.threshold = 0.3
+        assert not next_batch()[0] and next_batch()[0]
+        e.use_fused_glue = True  # (as it was)
+        e.linear_chain = False
+        assert not next_batch()[0]

@@ -317,3 +317,24 @@ def test_trace_runner_refuses_a_format_the_model_does_not_run_in(tmp_path):
     from tah_amd import trace
     (tmp_path / "config.json").write_text(json.dumps({"architectures": ["Qwen3ForCausalLM"]}))
     assert trace.main(["--model", str(tmp_path), "--dtype", "float32", "--out", str(tmp_path), "--max-tokens", "4"], io.StringIO(""), io.StringIO()) == 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", ["zozosun odd", "zedudra odd"])
+def test_a_captured_step_serves_the_next_batch_gpu(which):
+    """Batches one after another, the captured step kept between them: the tokens of an engine that captures for each."""
+    cfg, t, eng, check = setup(which, "bf16", "cuda", 2, 60)
+    batches = [[Z.tokens_of(cfg, n, 50 + n) for n in pair] for pair in ((17, 5), (3, 24), (9, 9))]
+    graphs, kept, fresh = [], [], []
+    with torch.no_grad():
+        for keep, out in ((True, kept), (False, fresh)):
+            eng._graph = None
+            for a, b in batches:
+                if not keep:
+                    eng._graph = None
+                first, _ = eng.prefill(torch.tensor(list(a) + list(b)).cuda(), torch.tensor([0, len(a), len(a) + len(b)], dtype=torch.int32).cuda())
+                out.append(eng.generate(first, 12).clone())
+                if keep:
+                    graphs.append(eng._graph)
+    assert graphs[0] is not None and all(g is graphs[0] for g in graphs)
+    assert all(torch.equal(a, b) for a, b in zip(kept, fresh))
