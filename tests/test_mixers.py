@@ -259,3 +259,20 @@ def test_router_choice_among_equal_scores_gpu(rows, experts, top, groups, keep):
     _route_case("cuda", rows, experts, top, groups, keep)
     if groups == 1:
         _route_case("cuda", rows, experts, top, groups, keep, sigmoid=True)
+
+
+# a shared expert of the experts' padded size is one more product of their launches: fewer, as many and more choices than products
+SHARED_AMONG = [(1, 64, 40, 8, 2, 40), (4, 64, 40, 8, 2, 50), (5, 96, 33, 8, 2, 64), (3, 32, 32, 2, 1, 32)]
+
+
+@needs_clang
+@pytest.mark.parametrize("case", range(len(SHARED_AMONG)))
+def test_shared_expert_among_the_experts_on_cpu_shim(case):
+    with emu_util.emulated():
+        Z.moe_case("cpu", Z.BF, *SHARED_AMONG[case])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", SHARED_AMONG + [(8, 2048, 768, 64, 8, 768), (1, 2048, 768, 64, 8, 768), (32, 2048, 768, 16, 8, 768)])
+def test_shared_expert_among_the_experts_gpu(case):
+    Z.moe_case("cuda", Z.BF, *case)
