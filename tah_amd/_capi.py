@@ -387,6 +387,8 @@ PROTOTYPES = {
     # include/tah_mixers.h
     "tah_embed_rows": (C.c_int, [C.POINTER(EmbedRowsArgs), c_void_p]),
     "tah_residual_norm": (C.c_int, [C.POINTER(ResidualNormArgs), c_void_p]),
+    "tah_norm_linear_supported": (C.c_int, [c_int32, c_int32, c_int32]),
+    "tah_norm_linear": (C.c_int, [C.POINTER(ResidualNormArgs), c_void_p, C.POINTER(LinearRowsArgs), c_void_p]),
     "tah_activate_rows": (C.c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int32, c_int32, c_int32, c_float, c_float, c_int32, c_void_p]),
     "tah_conv_rows": (C.c_int, [c_void_p, c_void_p, c_void_p, C.POINTER(Portions), c_void_p, c_int32, c_int32, c_int32, c_int32, c_void_p]),
     "tah_delta_step": (C.c_int, [C.POINTER(DeltaLayer), c_void_p, c_void_p, c_int32, c_void_p, c_int64, c_void_p, c_int32, c_void_p]),

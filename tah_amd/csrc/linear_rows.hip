@@ -32,7 +32,7 @@
 
 #include <utility>
 
-#include "mixer_device.h"
+#include "residual_row.h"
 
 namespace tah {
 namespace {
@@ -1035,6 +1035,99 @@ __global__ __launch_bounds__(kChainThreads) void linear_chain_kernel(const Chain
     }
 }
 
+// ---- a norm of the residual stream and the linear layer behind it in one launch ----------------------------
+// One or two rows: a decode step of such a model is a chain of launches of 4.4 us and more, most of it their start and the first trip to
+// memory, and a norm of a few rows is a launch of its own for 8 KB.  Here every workgroup of the layer makes the normed rows for
+// itself (28 KB a row, with experts 60, with a convolution 72) while its weights are on their way, and the first one stores what is kept: the
+// new residual rows and the convolution's input.  Same arithmetic in the same order as tah_residual_norm and tah_linear_rows: the same bits.
+// One row in a captured step of four layers, as two launches and as one: 2048 -> 6144 behind a plain norm 4.4 + 8.0 -> 8.9 us, 2048 -> 3616 behind
+// a norm with convolution (and experts) 4.4 + 4.9 -> 7.9: a step 305.9 -> 298.8 us, two rows 329.8 -> 324.2; of the other design, 2048 -> 6144, 342.4 ->
+// 334.9 and 369.1 -> 361.9.  Three and four rows: the rows' bytes cost more than the launch (350.5 -> 359.3, 369.6 -> 378.4).  More than two
+// workgroups to a compute unit: the rows are made three times over (2048 -> 12352, one row: a step 334.9 -> 344.2).
+constexpr int kNormLinearRows = 2, kNormLinearWorkgroups = 512;
+constexpr int kNormLinearSteps = 8;  // K = 256 kNormLinearSteps = a thread's eight columns for 256 threads
+struct NormLinear {
+    tah_residual_norm_args n;
+    float* x_out;
+    const bf16x8* w;
+    __bf16* y;
+    bf16x8* yp;
+    int64_t y_rs;
+    int32_t act;
+    float c0, c1;
+};
+
+// kMore: with experts or a convolution, whose loads take the registers of a second workgroup on the compute unit
+template <int F, bool GROUPS, bool H8, bool kMore>
+__global__ __launch_bounds__(kLinThreads, kMore ? 2 : 4) void norm_linear_kernel(const NormLinear p) {
+    constexpr int PW = kNormLinearSteps;
+    static_assert(F <= kLinThreads / kRowThreads, "all rows at a time");
+    using Tile = ChainTile<PW, 1, H8, F, H8>;
+    __shared__ __align__(16) float red[kLinWaves][3][16][kTileCols];
+    __shared__ __align__(16) bf16x8 rows_lds[PW * kLinWaves * 4 * F];  // [step][k group][row]
+    __shared__ ResidualLds<1, GROUPS> lds[kLinThreads / kRowThreads];
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const int part = wave / (kRowThreads / kWave), c = lane % 16, kg = lane / 16;
+    tah_residual_norm_args n = p.n;
+    if constexpr (!kMore) {
+        n.experts = nullptr;
+        n.conv = nullptr;
+    }
+    Tile t;
+    const int r = F == 1 ? 0 : part;  // (of one row both halves of the workgroup make it)
+    const bool own = r < p.n.rows && (F > 1 || part == 0);
+    residual_row<__bf16, 1, GROUPS, true>(
+        n, r < p.n.rows ? r : p.n.rows - 1, threadIdx.x % kRowThreads, lds[part], blockIdx.x == 0 && own, p.x_out,
+        [&]() __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_barrier(0);
+            t.ask_weights(p.w, blockIdx.x, wave, lane);
+            __builtin_amdgcn_sched_barrier(0);
+        },
+        [&](int col, const float (&v)[8]) __attribute__((always_inline)) {
+            if (own) rows_lds[(col / kStepK * 4 + col % kStepK / 8) * F + r] = to_bf16x8(v);
+        });
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < Tile::kXLoads; ++j) t.x[j] = rows_lds[((wave * PW + Tile::step_of(j, c)) * 4 + kg) * F + c % F];
+    t.start();
+    t.template multiply<false, 0, PW>();
+    t.template park<false>(red, nullptr, wave, lane);
+    __syncthreads();
+    // a lane per row (rows past the last one are zeros in the rows form) and eight columns
+    constexpr int kUnits = H8 ? 1 : 2;
+    if ((int)threadIdx.x >= kLinRows * kUnits) return;
+    const int row = threadIdx.x % kLinRows, unit = threadIdx.x / kLinRows, n0 = (int)blockIdx.x * 8 * kUnits + 8 * unit;
+    bf16x8 out = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (row < p.n.rows) {
+        float s[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s[i] = 0.f;
+#pragma unroll
+        for (int w = 0; w < kLinWaves; ++w)
+#pragma unroll
+            for (int half = 0; half < (H8 ? 2 : 1); ++half) {  // (H8: the even and the odd steps' sums)
+                const f32x4 lo = *reinterpret_cast<const f32x4*>(&red[w][0][row][8 * (H8 ? half : unit)]);
+                const f32x4 hi = *reinterpret_cast<const f32x4*>(&red[w][0][row][8 * (H8 ? half : unit) + 4]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    s[i] += lo[i];
+                    s[4 + i] += hi[i];
+                }
+            }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) out[i] = (__bf16)s[i];
+        if (p.act == TAH_ACT_GELU_TANH) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) out[i] = (__bf16)gelu_tanh_exact((float)out[i]);
+        } else if (p.act == TAH_ACT_XIELU) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) out[i] = (__bf16)xielu((float)out[i], p.c0, p.c1);
+        }
+        if (p.y) *reinterpret_cast<bf16x8*>(p.y + (int64_t)row * p.y_rs + n0) = out;
+    }
+    if (p.yp) p.yp[packed_rows_unit(row, n0)] = out;
+}
+
 // what is left of a launch without rows: the words of the next one
 __global__ __launch_bounds__(kLinThreads) void linear_chain_clear_kernel(int32_t* clear) {
     for (int i = threadIdx.x; i < TAH_LINEAR_CHAIN_WORDS; i += kLinThreads) clear[i] = 0;
@@ -1273,6 +1366,60 @@ extern "C" int tah_linear_rows(const tah_linear_rows_args* a, tah_stream_t strea
         if (pw == 8) launch<2, 4, kGateUp16, 8>(p, groups, batch, st);
         else launch<2, 2, kGateUp16, 0>(p, groups, batch, st);
     }
+    return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
+}
+
+extern "C" int tah_norm_linear_supported(int32_t rows, int32_t cols, int32_t n) {
+    using namespace tah;
+    return rows >= 1 && rows <= kNormLinearRows && cols == kNormLinearSteps * kLinWaves * kStepK && n > 0 && n % kTileCols == 0 &&
+           n / kTileCols <= kNormLinearWorkgroups;
+}
+
+extern "C" int tah_norm_linear(const tah_residual_norm_args* norm, float* x_out, const tah_linear_rows_args* a, tah_stream_t stream) {
+    using namespace tah;
+    if (!norm || !a || !x_out) return TAH_E_NULL;
+    if (const int rc = check_residual(*norm)) return rc;
+    if (!tah_norm_linear_supported(norm->rows, norm->cols, a->n) || norm->dtype != TAH_DT_BF16 || a->rows != norm->rows || a->k != norm->cols) return TAH_E_SHAPE;
+    // (what a workgroup of another tile still reads: nothing but x_out, the convolution's input and the layer's result is written)
+    if (norm->xe || norm->x_packed || norm->normed || norm->normed_packed) return TAH_E_SHAPE;
+    if (a->kind != TAH_LINEAR_PLAIN || a->batch > 1 || a->residual || a->bias || a->input_norm != TAH_NORM_NONE || a->n_select != 0 ||
+        (a->activation != TAH_ACT_NONE && a->activation != TAH_ACT_GELU_TANH && a->activation != TAH_ACT_XIELU) || (a->out_packed && a->n % kStepK != 0) ||
+        (a->out && a->out_row_stride < a->n))
+        return TAH_E_SHAPE;
+    if (!a->w_packed || (!a->out && !a->out_packed)) return TAH_E_NULL;
+    if (!aligned16(x_out) || !aligned16(a->w_packed) || !aligned16(a->out) || !aligned16(a->out_packed) || (a->out && a->out_row_stride % 8 != 0))
+        return TAH_E_ALIGN;
+    struct Range { const char* at; int64_t bytes; };
+    const auto of = [](const void* q, int64_t bytes) { return Range{static_cast<const char*>(q), q ? bytes : 0}; };
+    const int64_t last = norm->rows - 1;
+    const Range written[] = {of(x_out, 4ll * norm->rows * norm->cols), of(a->out, 2 * (last * a->out_row_stride + a->n)), of(a->out_packed, 64ll * a->n)};
+    const Range read[] = {of(norm->x, 4ll * norm->rows * norm->cols), of(norm->y, 2 * (last * norm->y_row_stride + norm->cols)),
+                          of(norm->coef, 4ll * norm->cols), of(norm->next_coef, 4ll * norm->cols), of(a->w_packed, 2ll * a->n * a->k)};
+    const auto meet = [](const Range& x, const Range& y) { return x.bytes > 0 && y.bytes > 0 && x.at < y.at + y.bytes && y.at < x.at + x.bytes; };
+    for (const Range& w : written)
+        for (const Range& r : read)
+            if (meet(w, r)) return TAH_E_SHAPE;
+    NormLinear p{};
+    p.n = *norm;
+    p.x_out = x_out;
+    p.w = static_cast<const bf16x8*>(a->w_packed);
+    p.y = static_cast<__bf16*>(a->out);
+    p.yp = static_cast<bf16x8*>(a->out_packed);
+    p.y_rs = a->out_row_stride;
+    p.act = a->activation;
+    p.c0 = a->act_c[0]; p.c1 = a->act_c[1];
+    const bool h8 = a->n / kTileCols < kSplitRowsBelowGroups;  // (as tah_linear_rows takes such a layer)
+    const auto launch = [&](auto fold, auto groups, auto half, auto more) {
+        hipLaunchKernelGGL((norm_linear_kernel<decltype(fold)::value, decltype(groups)::value, decltype(half)::value, decltype(more)::value>),
+                           dim3(a->n / (h8 ? 8 : kTileCols)), dim3(kLinThreads), 0, static_cast<hipStream_t>(stream), p);
+    };
+    const auto run = [&](auto fold, auto groups, auto half) {
+        norm->conv || norm->experts ? launch(fold, groups, half, std::true_type{}) : launch(fold, groups, half, std::false_type{});
+    };
+    const auto by_tile = [&](auto fold, auto groups) { h8 ? run(fold, groups, std::true_type{}) : run(fold, groups, std::false_type{}); };
+    const auto by_groups = [&](auto fold) { norm->groups > 1 ? by_tile(fold, std::true_type{}) : by_tile(fold, std::false_type{}); };
+    if (norm->rows <= 1) by_groups(std::integral_constant<int, 1>{});
+    else by_groups(std::integral_constant<int, 2>{});
     return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
 }
 

@@ -44,6 +44,8 @@ struct Api {
     Entry<decltype(&tah_decider_tail)> decider_tail;
     Entry<decltype(&tah_linear_pack_weight)> linear_pack_weight;
     Entry<decltype(&tah_linear_pack_rows)> linear_pack_rows;
+    Entry<decltype(&tah_norm_linear_supported)> norm_linear_supported;
+    Entry<decltype(&tah_norm_linear)> norm_linear;
     Entry<decltype(&tah_linear_rows)> linear_rows;
     Entry<decltype(&tah_linear_chain_supported)> linear_chain_supported;
     Entry<decltype(&tah_linear_chain)> linear_chain;

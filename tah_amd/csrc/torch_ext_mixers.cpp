@@ -75,19 +75,18 @@ struct InputConv {
     }
 };
 
-void residual_norm(const Tensor& x, const optional<Tensor>& coef, int64_t width, double eps, const optional<Tensor>& y, const optional<Tensor>& y_scale,
+// tah_residual_norm_args from tensors.  (elem: the element type where nothing is given in it)
+tah_residual_norm_args residual_args(Dev& d, const Tensor* elem, const Tensor& x, const optional<Tensor>& coef, int64_t width, double eps, const optional<Tensor>& y, const optional<Tensor>& y_scale,
                    const optional<Tensor>& experts, const optional<Tensor>& index, const optional<Tensor>& weight, const optional<Tensor>& xe,
                    const optional<Tensor>& x_packed, const optional<Tensor>& next_coef, const optional<Tensor>& normed,
                    const optional<Tensor>& normed_packed, int64_t index_scale, int64_t index_row, int64_t groups, int64_t group_cols,
                    const InputConv* conv, const optional<Tensor>& slot, const optional<Tensor>& pos) {
-    need_lib();
-    Dev d; d.see(x); d.see(coef); d.see(y); d.see(y_scale); d.see(experts); d.see(index); d.see(weight); d.see(xe); d.see(x_packed);
+    d.see(x); d.see(coef); d.see(y); d.see(y_scale); d.see(experts); d.see(index); d.see(weight); d.see(xe); d.see(x_packed);
     d.see(next_coef); d.see(normed); d.see(normed_packed); d.see(slot); d.see(pos);
     TORCH_CHECK(x.dim() == 2, "residual_norm: x must be [rows, cols]");
     const int64_t rows = x.size(0), cols = x.size(1);
     // (the element type is that of whatever is given in it)
     const optional<Tensor>* const elems[] = {&y, &experts, &xe, &normed, &x_packed, &normed_packed};
-    const Tensor* elem = nullptr;
     for (const auto* t : elems)
         if (!elem && t->has_value()) elem = &**t;
     TORCH_CHECK(elem, "residual_norm: nothing to add and nothing to write");
@@ -120,7 +119,48 @@ void residual_norm(const Tensor& x, const optional<Tensor>& coef, int64_t width,
         a.conv = at_<float>(conv->w); a.conv_state = mptr(conv->state); a.slot = at_<int32_t>(slot); a.pos = at_<int32_t>(pos);
         a.taps = (int32_t)conv->w.size(0); a.nslots = (int32_t)conv->state.size(0);
     }
+    return a;
+}
+
+void residual_norm(const Tensor& x, const optional<Tensor>& coef, int64_t width, double eps, const optional<Tensor>& y, const optional<Tensor>& y_scale,
+                   const optional<Tensor>& experts, const optional<Tensor>& index, const optional<Tensor>& weight, const optional<Tensor>& xe,
+                   const optional<Tensor>& x_packed, const optional<Tensor>& next_coef, const optional<Tensor>& normed,
+                   const optional<Tensor>& normed_packed, int64_t index_scale, int64_t index_row, int64_t groups, int64_t group_cols,
+                   const InputConv* conv, const optional<Tensor>& slot, const optional<Tensor>& pos) {
+    need_lib();
+    Dev d;
+    const tah_residual_norm_args a = residual_args(d, nullptr, x, coef, width, eps, y, y_scale, experts, index, weight, xe, x_packed, next_coef, normed,
+                                                   normed_packed, index_scale, index_row, groups, group_cols, conv, slot, pos);
     check_rc(g.residual_norm(&a, d.stream()), "tah_residual_norm");
+}
+
+bool norm_linear_supported(int64_t rows, int64_t cols, int64_t n) {
+    need_lib();
+    const auto fits = [](int64_t v) { return v >= 0 && v <= 0x7fffffff; };
+    return fits(rows) && fits(cols) && fits(n) && g.norm_linear_supported((int32_t)rows, (int32_t)cols, (int32_t)n) != 0;
+}
+
+// The norm, and the linear layer w_packed [n, cols] behind it: its row-major result, or nothing where only out_packed is asked for.
+optional<Tensor> norm_linear(const Tensor& x, const Tensor& x_out, const optional<Tensor>& coef, int64_t width, double eps, const optional<Tensor>& y,
+                             const optional<Tensor>& y_scale, const optional<Tensor>& experts, const optional<Tensor>& index, const optional<Tensor>& weight,
+                             const optional<Tensor>& next_coef, int64_t index_scale, int64_t index_row, int64_t groups, int64_t group_cols,
+                             const InputConv* conv, const optional<Tensor>& slot, const optional<Tensor>& pos, const Tensor& w_packed, int64_t n,
+                             const optional<Tensor>& out_packed, bool want_out, int64_t activation, double act_c0, double act_c1) {
+    need_lib();
+    Dev d; d.see(x_out); d.see(w_packed); d.see(out_packed);
+    const tah_residual_norm_args a = residual_args(d, &w_packed, x, coef, width, eps, y, y_scale, experts, index, weight, c10::nullopt, c10::nullopt, next_coef,
+                                                   c10::nullopt, c10::nullopt, index_scale, index_row, groups, group_cols, conv, slot, pos);
+    flat(x_out, at::kFloat, (int64_t)a.rows * a.cols, "norm_linear: x_out"); flat(w_packed, at::kBFloat16, n * a.cols, "norm_linear: w_packed");
+    flat(out_packed, at::kBFloat16, 32 * n, "norm_linear: out_packed");
+    TORCH_CHECK(want_out || out_packed.has_value(), "norm_linear: nothing to write");
+    optional<Tensor> out;
+    if (want_out) out = at::empty({(int64_t)a.rows, n}, w_packed.options());
+    tah_linear_rows_args l{};
+    l.w_packed = ptr(w_packed); l.out = out.has_value() ? mptr(*out) : nullptr; l.out_row_stride = out.has_value() ? n : 0; l.out_packed = any(out_packed);
+    l.rows = a.rows; l.n = (int32_t)n; l.k = a.cols; l.kind = TAH_LINEAR_PLAIN; l.activation = (int32_t)activation;
+    l.act_c[0] = (float)act_c0; l.act_c[1] = (float)act_c1;
+    check_rc(g.norm_linear(&a, at_<float>(x_out), &l, d.stream()), "tah_norm_linear");
+    return out;
 }
 
 Tensor activate_rows(const Tensor& in, int64_t kind, const optional<Tensor>& out_, double c0, double c1) {
@@ -421,6 +461,8 @@ void bind_mixers(py::module_& m) {
     m.def("embed_rows", &embed_rows);
     py::class_<InputConv>(m, "InputConv").def(py::init<Tensor, Tensor>());
     m.def("residual_norm", &residual_norm);
+    m.def("norm_linear_supported", &norm_linear_supported);
+    m.def("norm_linear", &norm_linear);
     m.def("conv_rows", &conv_rows);
     m.def("activate_rows", &activate_rows);
     m.def("moe_route", &moe_route);

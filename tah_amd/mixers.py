@@ -117,6 +117,10 @@ class Step:
     starts: Optional[list] = None              # ... and on the host: (length, first position) per sequence
     contexts: Dict[int, tuple] = dataclasses.field(default_factory=dict)  # latent rows portions can see, per ring
     normed: bool = False
+    # A sum and norm of the residual rows that is not launched yet (packed rows): the layer that reads its result launches it with its
+    # own product (``linear``), anything else ``settle``s it.  x_other: where the former leaves the residual rows.
+    pending: Optional["Norm"] = None
+    x_other: Optional[torch.Tensor] = None
 
     @property
     def n(self) -> int:
@@ -125,6 +129,25 @@ class Step:
     @property
     def packed(self) -> bool:
         return self.xp is not None
+
+    def settle(self) -> None:
+        p, self.pending = self.pending, None
+        if p is not None:
+            reads_norm = p.norm is not None
+            _call("residual_norm", self.x, *p.front, None, None if reads_norm else self.xp, p.norm, self.xe if reads_norm else None,
+                  self.xp if reads_norm else None, *p.tail)
+
+    def linear(self, layer: Linear, out_packed: Optional[torch.Tensor] = None, want_out: bool = True, act: Optional[Activation] = None):
+        """A dense layer of the rows operand."""
+        p, kw = self.pending, act.rows if act is not None else {}
+        if p is not None and not set(kw) - {"gelu_tanh", "xielu"} and _call("norm_linear_supported", self.n, self.x.shape[1], layer.n):
+            self.pending = None
+            code, c = (3, (0.0, 0.0)) if "gelu_tanh" in kw else (4, kw["xielu"]) if "xielu" in kw else (0, (0.0, 0.0))
+            out = _call("norm_linear", self.x, self.x_other, *p.front, p.norm, *p.tail, layer.packed, layer.n, out_packed, want_out, code, *c)
+            self.x, self.x_other = self.x_other, self.x
+            return out
+        self.settle()
+        return layer.rows(self.xp, self.n, out_packed=out_packed, want_out=want_out, **kw)
 
 
 @dataclasses.dataclass
@@ -137,6 +160,15 @@ class Sublayer:
     weight: Optional[torch.Tensor] = None
     index_scale: int = 1
     index_row: int = 0
+
+
+@dataclasses.dataclass
+class Norm:
+    """Arguments of a ``residual_norm`` call between its rows and its results: what is added, the norm in front of the next sublayer
+    (None: it reads the residual rows), groups and convolution."""
+    front: tuple
+    norm: Optional[torch.Tensor]
+    tail: tuple
 
 
 # ── gated delta rule ─────────────────────────────────────────────────────────────────────────────────────────────────
@@ -189,7 +221,7 @@ class DeltaMixer:
         def rows(self, st: Step) -> Sublayer:
             m = self.m
             if st.packed:
-                proj = m.proj.rows(st.xp, st.n)
+                proj = st.linear(m.proj)
                 _call_on(self.layer.step, proj, st.slot, st.pos, None, self.op)
                 return Sublayer(m.o.rows(self.op, st.n))
             out = torch.empty(st.n, m.width_o, dtype=st.xe.dtype, device=st.x.device)
@@ -287,7 +319,7 @@ class LatentAttention:
         def rows(self, st: Step) -> Sublayer:
             m, H, n = self.m, self.m.spec.heads, st.n
             if st.packed:
-                proj = m.proj.rows(st.xp, n)
+                proj = st.linear(m.proj)
                 self._prep(proj, st, slot=st.slot, q_packed=self.qp)
                 q = m.uk_rows.rows(self.qp, n)   # [H, n, rank_p]
                 _call_on(self.layer.decode, st.slot, st.pos, q, proj, 0, self.cp, None, self.workspace)
@@ -411,7 +443,7 @@ class WindowAttention:
         def rows(self, st: Step) -> Sublayer:
             m = self.m
             if st.packed:
-                _call_on(self.layer.decode, m.proj.rows(st.xp, st.n), st.slot, st.pos, None, self.op, self.workspace)
+                _call_on(self.layer.decode, st.linear(m.proj), st.slot, st.pos, None, self.op, self.workspace)
                 return Sublayer(m.o.rows(self.op, st.n))
             out = torch.empty(st.n, m.width_o, dtype=st.xe.dtype, device=st.x.device)
             _call_on(self.layer.decode, m.proj(st.xe), st.slot, st.pos, out, None, self.workspace)
@@ -444,7 +476,7 @@ class DenseMlp:
         def rows(self, st: Step) -> Sublayer:
             if not st.packed:
                 return self.portions(st)
-            self.m.up.rows(st.xp, st.n, out_packed=self.ap, want_out=False, **self.m.act.rows)
+            st.linear(self.m.up, out_packed=self.ap, want_out=False, act=self.m.act)
             return Sublayer(self.m.down.rows(self.ap, st.n))
 
         def portions(self, st: Step) -> Sublayer:
@@ -537,6 +569,7 @@ class MoeMlp:
             m, n = self.m, st.n
             if not st.packed:
                 return self.portions(st)
+            st.settle()
             picked = self.chosen[1:1 + n * m.top]
             index, weight, sg = self._route(st, picked.view(n, m.top))
             select = self.chosen[:1 + n * m.top] if m.shared_among else picked

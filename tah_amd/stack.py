@@ -20,7 +20,7 @@ from . import ops
 from ._capi import TahDuoError
 from .engine import DecodeEngine
 from .kv_cache import InputTail, SlotPool
-from .mixers import Linear, LatentAttention, Step, Sublayer, pad_to, padded
+from .mixers import Linear, LatentAttention, Norm, Step, Sublayer, pad_to, padded
 from .ops import _call
 
 
@@ -146,6 +146,7 @@ class StackEngine(DecodeEngine):
         z = lambda *s, dt=torch.float32: torch.zeros(*s, dtype=dt, device=dev)
         i32 = lambda: z(batch, dt=torch.int32)
         self.x = z(batch, cols)
+        self.x_other = z(batch, cols) if self.packed else None
         self.xe = z(batch, cols, dt=self.dtype) if self.packed or self.normed else self.x
         self.slot, self.qpos, self.act = i32(), i32(), z(batch, dt=torch.bool)
         self.xp = z(32 * cols, dt=self.dtype) if self.packed else None
@@ -181,14 +182,18 @@ class StackEngine(DecodeEngine):
         """A sublayer's result into the residual stream, and from it what the next sublayer (or the output head) reads."""
         m, (norm, conv, last) = self.cfg, front
         geometry = (m.groups, m.columns.group_cols)
-        args = (st.x, coef, m.width, m.eps, r.y, r.y_scale, r.experts, r.index, r.weight)
-        tail = (r.index_scale, r.index_row, *geometry)
+        st.settle()
+        what = (coef, m.width, m.eps, r.y, r.y_scale, r.experts, r.index, r.weight)
+        args, tail = (st.x, *what), (r.index_scale, r.index_row, *geometry)
+        if st.packed and not last:
+            st.pending = Norm(what, norm, (*tail, conv, st.slot if conv else None, st.pos if conv else None))
+            return
         if last:
             _call("residual_norm", *args, None, None, norm, None if st.packed else h, self.hp if st.packed else None, *tail, None, None, None)
         elif norm is None:  # (in float32 the element-type rows are the residual rows themselves)
-            _call("residual_norm", *args, st.xe if self.packed and not st.packed else None, st.xp, None, None, None, *tail, None, None, None)
+            _call("residual_norm", *args, st.xe if self.packed else None, None, None, None, None, *tail, None, None, None)
         elif conv is None or st.slot is not None:
-            _call("residual_norm", *args, None, None, norm, st.xe, st.xp, *tail, conv, st.slot if conv else None, st.pos if conv else None)
+            _call("residual_norm", *args, None, None, norm, st.xe, None, *tail, conv, st.slot if conv else None, st.pos if conv else None)
         else:
             n = torch.empty_like(st.xe)
             _call("residual_norm", *args, None, None, norm, n, None, *tail, None, None, None)
@@ -217,7 +222,7 @@ class StackEngine(DecodeEngine):
             sl = slice(a, b)
             _call("embed_rows", tok[sl], m.embed, self.x[sl], None, None if self.normed else self.xp, pos[sl], finished[sl], self.slot[sl], self.qpos[sl],
                   self.act[sl], a, m.embed_scale)
-            st = Step(self.x[sl], self.xe[sl], self.qpos[sl], self.xp, slot=self.slot[sl])
+            st = Step(self.x[sl], self.xe[sl], self.qpos[sl], self.xp, slot=self.slot[sl], x_other=self.x_other[sl] if self.packed else None)
             self._layers(st, self.h[sl])
             if self.packed:
                 m.head.rows(self.hp, b - a, out=self.logits[sl])
