@@ -35,6 +35,7 @@ constexpr int kChunkSmall = 256;       // ... and when there are not (few sequen
                                        // times the workgroups, so that enough loads are in flight
 constexpr int kDecThreads = 256;     // 4 waves x (chunk / 4) rows
 constexpr int kUnroll = 4;           // loads of 4 rows in flight per wave and tensor
+constexpr int kBlock = 4 * kUnroll;  // rows per wave and turn
 constexpr int kPart = kD + 2;        // acc[128], m, l  (floats per partial)
 
 
@@ -109,13 +110,6 @@ __device__ __forceinline__ int visible_len(const DecParams& p, bool second, int 
     return qdepth >= 1 ? p.c2.len[slot] : 0;
 }
 
-// kSub: row sub->row of the segment is not taken from memory but from sub->k / v / pos (the token the same
-// workgroup is appending while it attends: what the loads return for that row is discarded).
-struct SubRow {
-    int row;  // -1: none in this segment
-    int pos;
-    u32x4 k, v;
-};
 // The loads of 4 U rows from r_it on (one row per 16-lane group and load; rows at or past row_end are clamped into
 // the slab and flagged).
 template <int U>
@@ -147,21 +141,9 @@ __device__ __forceinline__ void load_rows(RowBlock<U>& b, const Seg& sg, bool se
 // Scores, online softmax and the weighted sum of V for a loaded block, for the G query heads of the kv head at
 // once.  m / l / acc: running maximum (log2 domain), sum and un-normalised output of this lane's row group, 8
 // values of d per lane.
-template <int G, int U, bool kSub = false>
+template <int G, int U>
 __device__ __forceinline__ void attend_rows(RowBlock<U>& b, bool second, int r_it, int kq, int qpos, float scale_log2e, const u32x4 (&qv)[G],
-                                            float (&m_run)[G], float (&l_run)[G], float (&acc)[G][8], const SubRow* sub = nullptr) {
-    if constexpr (kSub) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const bool hit = r_it + u * 4 + kq == sub->row;
-            b.pos[u] = hit ? sub->pos : b.pos[u];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                b.k[u][i] = hit ? sub->k[i] : b.k[u][i];
-                b.v[u][i] = hit ? sub->v[i] : b.v[u][i];
-            }
-        }
-    }
+                                            float (&m_run)[G], float (&l_run)[G], float (&acc)[G][8]) {
     float s[U][G];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -203,13 +185,13 @@ __device__ __forceinline__ void attend_rows(RowBlock<U>& b, bool second, int r_i
 }
 // Sixteen-lane groups of a wave each take one cache row per load (4 rows x 256 B = 1 KiB per instruction); U such
 // loads of K and of V are in flight per wave: load, then attend.
-template <int G, int U, bool kSub = false>
+template <int G, int U>
 __device__ __forceinline__ void consume_rows(const Seg& sg, bool second, const __bf16* kbase, const __bf16* vbase, const int32_t* posbase,
                                              int r_it, int row_end, int kq, int qpos, float scale_log2e, const u32x4 (&qv)[G],
-                                             float (&m_run)[G], float (&l_run)[G], float (&acc)[G][8], const SubRow* sub = nullptr) {
+                                             float (&m_run)[G], float (&l_run)[G], float (&acc)[G][8]) {
     RowBlock<U> b;
     load_rows<U>(b, sg, second, kbase, vbase, posbase, r_it, row_end, kq);
-    attend_rows<G, U, kSub>(b, second, r_it, kq, qpos, scale_log2e, qv, m_run, l_run, acc, sub);
+    attend_rows<G, U>(b, second, r_it, kq, qpos, scale_log2e, qv, m_run, l_run, acc);
 }
 
 // The 16 (wave, row group) partials of a workgroup into LDS: red[16][G][kPart].
@@ -329,26 +311,222 @@ __device__ __forceinline__ void store_output(const DecParams& p, int qi, int hea
 constexpr int kWholeWaves = 16;
 constexpr int kWholeThreads = kWholeWaves * kWave;
 
-// The four row groups of a wave (lanes 16 apart hold the same slice of d) into one partial, left in every lane.
-template <int G>
-__device__ __forceinline__ void combine_row_groups(float (&m_run)[G], float (&l_run)[G], float (&acc)[G][8]) {
+// A wave takes blocks of sixteen cache rows.  Q.K of a block runs on the matrix cores: its rows against the G query heads, each of
+// them in 16 / G of the 16 columns, so that lane (kq, dc) gets the scores of rows 4 kq ... + 4 for head dc % G -- the rows of V that its row
+// group weighs, 8 of the 128 values in each lane.  The softmax of a score is one lane's work then, not sixteen lanes', and the
+// other heads' weights come from lanes beside it by a turn of the row.  The matrix product's sums are of the same
+// bfloat16 products in float32, the four steps apart and then added in pairs (one chain through all four left the log-sum-exp 2 %
+// further from its 64-bit value); weights and the sum of V stay float32 on the vector units.  What this is for: four waves
+// share a SIMD, and with dot products on the vector units (four v_dot2 and four row adds a score) a turn of sixteen waves, 256 rows, took
+// 3.0 us of issue behind its loads, now 1.9; the fused step's launches went with it from 9.4 to 7.9 us (one sequence of 300 rows),
+// 13.1 to 11.2 (eight of 100 ... 1000) and 17.2 to 15.9 (32 of 512 ... 600, 4.6 TB/s).  The split-K launch keeps attend_rows:
+// several workgroups to a compute unit hide its issue behind memory (64 sequences of 1024 ... 16384 rows: 422 us, with this form 414, but
+// 490 instead of 473 on slabs just written, whose lines leave the caches for K's).
+// Row sub.row of the segment is not taken from memory but from sub.k / v / pos (the token the same
+// workgroup is appending while it attends: what the loads return for that row is discarded).
+struct SubRow {
+    int row;  // -1: none in this segment
+    int pos;
+    const u32x4 *k, *v;  // the prepared row, in LDS
+};
+// The loads of 16 rows from r_it on (rows at or past row_end are clamped into the slab and flagged).  kbase: the kv head's part of
+// the segment's first row.  V: 16 bytes of the rows 4 kq + u.  K: the matrix product wants 16 bytes of row dc for each of its steps, which
+// as a load is half a 128-byte line of sixteen rows; instead a load takes whole lines of eight rows, and lanes eight apart
+// exchange halves (take_rows) once they are there.  K stays in the caches where a launch's keys are few
+// (stream_keys): its halves of a row come by two loads, and the tokens that take another iteration in this step ask for the same rows again.
+struct TileBlock {
+    u32x4 k[4], v[4];
+    int pos[4];
+    bool ok[4];
+};
+__device__ __forceinline__ void load_tile(TileBlock& b, const Seg& sg, bool second, const __bf16* kbase, const __bf16* vbase,
+                                          const int32_t* posbase, int r_it, int row_end, int kq, int dc, bool stream) {
+    // all of K (and the positions) before V: a wave's loads return in order, and the scores need K only
+    const __bf16* krow[2];
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        float mx = fmaxf(m_run[g], __shfl_xor(m_run[g], 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float w = fast_exp2(m_run[g] - (mx == kNegInf ? 0.f : mx));
-        float l = l_run[g] * w;
-        l += __shfl_xor(l, 16);
-        l += __shfl_xor(l, 32);
-        l_run[g] = l;
-        m_run[g] = mx;
+    for (int u = 0; u < 2; ++u) {
+        const int r = r_it + 8 * u + dc % 8;
+        krow[u] = kbase + (int64_t)(r < row_end ? r : row_end - 1) * sg.k_rs + 8 * kq + 32 * (dc / 8);  // keep tail loads inside the slab
+    }
+    int rl[4];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            float a = acc[g][i] * w;
-            a += __shfl_xor(a, 16);
-            a += __shfl_xor(a, 32);
-            acc[g][i] = a;
+    for (int u = 0; u < 4; ++u) {
+        const int rv = r_it + 4 * kq + u;
+        b.ok[u] = rv < row_end;
+        rl[u] = b.ok[u] ? rv : row_end - 1;
+        b.pos[u] = 0;
+    }
+    if (stream) {  // uniform
+        TAH_APART();  // (loads that differ in the hint only are made one otherwise, without it)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) b.k[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(krow[u % 2] + 64 * (u / 2)));
+        TAH_APART();
+    } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) b.k[u] = *reinterpret_cast<const u32x4*>(krow[u % 2] + 64 * (u / 2));
+    }
+    if (second) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) b.pos[u] = posbase[rl[u]];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)  // (streaming loads: every row is read exactly once)
+        b.v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vbase + (int64_t)rl[u] * sg.v_rs + 8 * dc));
+    // all eight loads are on their way before the first is waited for (left alone, the compiler put two of V's behind the scores)
+    __builtin_amdgcn_sched_barrier(0);
+}
+// K as loaded -> k[u]: values 32 u + 8 kq ... + 8 of row dc.
+__device__ __forceinline__ void take_rows(u32x4 (&k)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; u += 2)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int a = (int)k[u][i], c = (int)k[u + 1][i];
+            // row_ror:8, written in the lanes dc >= 8 and dc < 8 only
+            k[u][i] = (uint32_t)__builtin_amdgcn_update_dpp(a, c, 0x128, 0xf, 0xc, false);
+            k[u + 1][i] = (uint32_t)__builtin_amdgcn_update_dpp(c, a, 0x128, 0xf, 0x3, false);
         }
+}
+// Lane (kq, dc)'s part of the G query heads: 16 bytes of head dc % G for each step of the matrix product (head g at q + g * stride).
+template <int G>
+__device__ __forceinline__ void load_query(u32x4 (&qv)[4], const __bf16* q, int64_t stride, int kq, int dc) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) qv[u] = *reinterpret_cast<const u32x4*>(q + (dc % G) * stride + 32 * u + 8 * kq);
+}
+// Running maximum (log2 domain) and sum of head dc % G over this lane's row group, and the group's un-normalised output: acc[k] is
+// 8 values of d of head (dc + k) % G.
+template <int G>
+struct TileState {
+    float m = kNegInf, l = 0.f, acc[G][8] = {};
+};
+// The value of the lane whose head is k further (the same row group).
+template <int K>
+__device__ __forceinline__ float head_turn(float x) {
+    if constexpr (K == 0) return x;
+    else return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + 16 - K, 0xf, 0xf, true));  // row_ror
+}
+template <int G, int K = 0, class F>
+__device__ __forceinline__ void for_heads(F&& f) {
+    f(std::integral_constant<int, K>{});
+    if constexpr (K + 1 < G) for_heads<G, K + 1>(f);
+}
+// Scores, online softmax and the weighted sum of V for a loaded block, for the G query heads of the kv head at once.
+template <int G>
+__device__ __forceinline__ void attend_tile(TileBlock& b, bool second, int r_it, int kq, int dc, int qpos, float scale_log2e, const u32x4 (&qv)[4],
+                                            TileState<G>& st, const SubRow& sub) {
+    take_rows(b.k);
+    const int hit = sub.row - r_it;
+    if (hit >= 0 && hit < kBlock) {  // uniform per wave
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const u32x4 k = sub.k[4 * u + kq], v = sub.v[dc];
+            const bool mine = hit == 4 * kq + u;
+            b.pos[u] = mine ? sub.pos : b.pos[u];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                b.k[u][i] = hit == dc ? k[i] : b.k[u][i];
+                b.v[u][i] = mine ? v[i] : b.v[u][i];
+            }
+        }
+    }
+    const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+    f32x4 part[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+        part[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b.k[u]), __builtin_bit_cast(bf16x8, qv[u]), none, 0, 0, 0);
+    f32x4 s = (part[0] + part[1]) + (part[2] + part[3]);
+    float mx = st.m;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        s[u] = b.ok[u] && (!second || b.pos[u] <= qpos) ? s[u] * scale_log2e : kNegInf;
+        mx = fmaxf(mx, s[u]);
+    }
+    const float m_use = mx == kNegInf ? 0.f : mx;
+    const float alpha = fast_exp2(st.m - m_use);
+    st.m = mx;
+    float pr[4], psum = 0.f;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        pr[u] = fast_exp2(s[u] - m_use);
+        psum += pr[u];
+    }
+    st.l = st.l * alpha + psum;
+    for_heads<G>([&](auto k) {
+        constexpr int K = decltype(k)::value;
+        const float al = head_turn<K>(alpha);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) st.acc[K][i] *= al;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const float w = head_turn<K>(pr[u]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                st.acc[K][2 * i] += w * bf16_lo(b.v[u][i]);
+                st.acc[K][2 * i + 1] += w * bf16_hi(b.v[u][i]);
+            }
+        }
+    });
+}
+// Eight loads of 1 KiB in flight per wave: load, then attend.
+template <int G>
+__device__ __forceinline__ void consume_tile(const Seg& sg, bool second, const __bf16* kbase, const __bf16* vbase, const int32_t* posbase,
+                                             int r_it, int row_end, int kq, int dc, int qpos, float scale_log2e, const u32x4 (&qv)[4],
+                                             TileState<G>& st, const SubRow& sub, bool stream) {
+    TileBlock b;
+    load_tile(b, sg, second, kbase, vbase, posbase, r_it, row_end, kq, dc, stream);
+    attend_tile<G>(b, second, r_it, kq, dc, qpos, scale_log2e, qv, st, sub);
+}
+
+// The four row groups of a wave into one partial, red[grp] of a workgroup's sixteen ([G][kPart]).  Lanes sixteen apart hold the same
+// values of d; a swap of two values between them and one add leave each with the total of one, so two rounds leave every lane two of its
+// eight (summing all eight in every lane was 0.4 us of vector issue at sixteen waves).
+template <int G>
+__device__ __forceinline__ void park_wave(float (*red)[G][kPart], int grp, int kq, int dc, const TileState<G>& st) {
+    const float mx = wave_max_xor32(wave_max_xor16(st.m));
+    const float w = fast_exp2(st.m - (mx == kNegInf ? 0.f : mx));
+    const float l = wave_sum_xor32(wave_sum_xor16(st.l * w));
+    const auto bits = [](float x) { return __float_as_uint(x); };
+    for_heads<G>([&](auto k) {
+        constexpr int K = decltype(k)::value;
+        const float wk = head_turn<K>(w);
+        float t[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {  // even row groups: value i, odd: i + 4
+            const auto r = __builtin_amdgcn_permlane16_swap(bits(st.acc[K][i] * wk), bits(st.acc[K][i + 4] * wk), false, false);
+            t[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {  // row groups 0, 1: t[i], 2, 3: t[i + 2]
+            const auto r = __builtin_amdgcn_permlane32_swap(bits(t[i]), bits(t[i + 2]), false, false);
+            red[grp][(dc + K) % G][dc * 8 + (kq % 2) * 4 + (kq / 2) * 2 + i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        }
+    });
+    if (kq == 0 && dc < G) {
+        red[grp][dc][kD] = mx;
+        red[grp][dc][kD + 1] = l;
+    }
+}
+
+// Element d of head g (the same head throughout a wave) merged over a workgroup's sixteen partials: un-normalised output, sum,
+// maximum.  Lane j weighs part j % 16; the weights go round from there (sixteen weights in every lane are 0.2 us of exponentials).
+template <int G>
+__device__ __forceinline__ void merge_waves(float (*red)[G][kPart], int g, int d, int lane, float& a, float& l, float& mx) {
+    const float m_part = red[lane % kWholeWaves][g][kD], l_part = red[lane % kWholeWaves][g][kD + 1];
+    float part[kWholeWaves];
+#pragma unroll
+    for (int j = 0; j < kWholeWaves; ++j) part[j] = red[j][g][d];
+    mx = kNegInf;
+#pragma unroll
+    for (int j = 0; j < kWholeWaves; ++j) mx = fmaxf(mx, lane_value(m_part, j));
+    const float w = fast_exp2(m_part - (mx == kNegInf ? 0.f : mx));
+    a = 0.f;
+    l = 0.f;
+#pragma unroll
+    for (int j = 0; j < kWholeWaves; ++j) {
+        const float wj = lane_value(w, j);
+        a += wj * part[j];
+        l += wj * lane_value(l_part, j);
     }
 }
 
@@ -362,38 +540,27 @@ __global__ __launch_bounds__(kWholeThreads) void duo_decode_whole_kernel(const D
     const int slot = p.q_slot[qi];
     const int qpos = p.q_pos[qi];
     const int qdepth = p.q_depth ? p.q_depth[qi] : p.depth;
-    u32x4 qv[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-        qv[g] = *reinterpret_cast<const u32x4*>(p.q + (int64_t)qi * p.q_rs + (int64_t)(hk * G + g) * p.q_hs + dc * 8);
-    float m_run[G], l_run[G], acc[G][8];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        m_run[g] = kNegInf;
-        l_run[g] = 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[g][i] = 0.f;
-    }
-    constexpr int kBlock = 4 * kUnroll;  // rows per wave and turn
+    u32x4 qv[4];
+    load_query<G>(qv, p.q + (int64_t)qi * p.q_rs + (int64_t)(hk * G) * p.q_hs, p.q_hs, kq, dc);
+    TileState<G> st;
     for (int seg = 0; seg < 2; ++seg) {
         const bool second = seg == 1;
         const int nvis = visible_len(p, second, slot, qpos, qdepth);
         if (nvis <= 0) continue;  // uniform per workgroup
         const Seg& sg = second ? p.c2 : p.c1;
         const int64_t base_row = sg.start[slot];
-        const __bf16* kbase = sg.k + base_row * sg.k_rs + (int64_t)hk * sg.k_hs + dc * 8;
-        const __bf16* vbase = sg.v + base_row * sg.v_rs + (int64_t)hk * sg.v_hs + dc * 8;
+        const __bf16* kbase = sg.k + base_row * sg.k_rs + (int64_t)hk * sg.k_hs;
+        const __bf16* vbase = sg.v + base_row * sg.v_rs + (int64_t)hk * sg.v_hs;
         const int32_t* posbase = second ? sg.pos + (int64_t)slot * sg.capacity : nullptr;
         for (int r_it = wave * kBlock; r_it < nvis; r_it += kWholeWaves * kBlock)
-            consume_rows<G, kUnroll>(sg, second, kbase, vbase, posbase, r_it, nvis, kq, qpos, p.scale_log2e, qv, m_run, l_run, acc);
+            consume_tile<G>(sg, second, kbase, vbase, posbase, r_it, nvis, kq, dc, qpos, p.scale_log2e, qv, st, SubRow{-1, 0, nullptr, nullptr}, false);
     }
-    combine_row_groups<G>(m_run, l_run, acc);
-    if (kq == 0) park_partials<G>(red, wave, dc, m_run, l_run, acc);
+    park_wave<G>(red, wave, kq, dc, st);
     __syncthreads();
     for (int e = tid; e < G * kD; e += kWholeThreads) {
         const int g = e / kD, d = e % kD;
         float a, l, mx;
-        merge16<G>(red, g, d, a, l, mx);
+        merge_waves<G>(red, g, d, lane, a, l, mx);
         const int head = hk * G + g;
         store_output(p, qi, head, d, l > 0.f ? a / l : 0.f);
         if (p.lse && d == 0) p.lse[(int64_t)qi * p.hq + head] = l > 0.f ? (mx + fast_log2(l)) * kLn2 : kNegInf;
@@ -783,10 +950,13 @@ __global__ __launch_bounds__(256) void qk_prep_bwd_kernel(const PrepBwdParams p)
 //
 // A call of a few sequences is a chain of dependent trips to memory, so the chain is kept short: wave 0 alone prepares,
 // all heads side by side, behind loads it issued first (every wave preparing everything for itself took 2 us of vector
-// issue, and the norm's row came back behind the cache rows), and where a sequence's rows lie is asked for together with
-// which sequence it is.  Measured in a replayed graph (16 / 8 heads), preparation + split-K + merge launches -> this one:
-// one sequence of 300 rows 13.6 -> 9.9 us, of 8000 18.4 -> 15.9 us; eight of up to 900 17.4 -> 14.0 us; 32 of up to 8000
-// (slabs of 8200) 152 -> 140 us.  The preparation by wave 0 is 2.5 to 3 us of that at few sequences.
+// issue, and the norm's row came back behind the cache rows), where a sequence's rows lie is asked for together with
+// which sequence it is, and no load in front of the first block stands under a branch (the compiler waits for everything
+// at those).  Measured in a replayed graph (16 / 8 heads), preparation + split-K + merge launches -> this one, both with scores on the
+// vector units (attend_rows has what the matrix cores made of it): one sequence of 300 rows 13.6 -> 9.9 us, of 8000
+// 18.4 -> 15.9 us; eight of up to 900 17.4 -> 14.0 us; 32 of up to 8000 (slabs of 8200) 152 -> 140 us.  One sequence of 300 rows now:
+// the addresses are known at 1.5 us, the new row is prepared at 2.8, the first block is there at 3.8 and attended at
+// 6.0, the output is written at 7.1.
 constexpr int kStepMaxGroup = 2;  // with four query heads per kv head the preparation no longer fits the 128 registers
 struct StepParams {
     PrepParams prep;
@@ -798,7 +968,7 @@ struct StepParams {
     float* part;                   // kSplit: partials [nq][hkv][nsplit][G][kPart] ...
     int32_t* arrived;              // ... and workgroups of a pair that are done, [nq][hkv], 0 between calls
     int32_t nsplit, fill;          // workgroups per pair at most, and as many as it takes to give every compute unit one
-    int32_t nslots1;               // slots of the depth-0 segment
+    int32_t nslots1, nslots2;      // slots of the depth-0 segment and, 0 without one, of the depth-1 segment
 };
 
 // Calls with too few (query, kv head) pairs to fill the chip, or slabs too long for one workgroup per pair: up to
@@ -806,7 +976,7 @@ struct StepParams {
 // are; the others leave at once.  The workgroup that finishes last merges the partials: they and the counter travel
 // through device-scope relaxed atomics, which go past the XCDs' L2 caches, so the hand-over needs no fence (a
 // device-scope fence writes the whole L2 back; it made the same idea cost 7 us).  The hand-over costs 3.9 us, a turn of the
-// sixteen waves 2.2 us: two turns stay with one workgroup (300 rows: 12.3 us against 14.0 shared by two), more are shared.
+// sixteen waves cost 2.2 us when these lines were drawn and costs less since: two turns stay with one workgroup (300 rows: 12.3 us against 14.0 shared by two), more are shared.
 // Once every compute unit has a workgroup a finer split only repeats the fixed 7 us: 32 x 8000 rows take 165 us at 1024
 // rows to a workgroup, 159 at 2048, 140 at 4096.
 constexpr int kStepMaxSplit = 32;
@@ -818,6 +988,12 @@ __host__ __device__ inline int step_splits_of(long rows, int fill) {
     const long n = few < fill ? few : fill, m = n > many ? n : many;
     return (int)(m < 1 ? 1 : (m > kStepMaxSplit ? kStepMaxSplit : m));
 }
+
+// Keys too many for the L2 caches (8 x 4 MB) to hold until they are asked for again are streamed: 28 MB and more of them, taken from the
+// workgroup's own context.  A step of a generation on a model of eight layers, kept / streamed: 8 sequences of 200 ... 300 rows (4 MB)
+// 400 / 403 us, 32 of them (16 MB) 514 / 519, 8 of 1000 ... 1500 (20 MB) 447 / 452; 32 of 500 ... 600 (36 MB) 575 / 564, 32 of
+// 1000 ... 1500 (82 MB) 717 / 698, 8 of 3000 ... 8000 (90 MB) 672 / 659.
+__device__ __forceinline__ bool stream_keys(int rows, int nq, int hkv) { return (int64_t)rows * nq * hkv * (kD * 2) >= 28 * 1000 * 1000; }
 
 template <int G, bool kSplit>
 __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const StepParams sp) {
@@ -835,11 +1011,15 @@ __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const St
     const bool is_q = kq < G, is_v = kq > G;
     u32x4 xin, wt, cs, sn, xn[4];
     if (wave == 0) {
-        const int g = is_q ? kq : 0;
-        const __bf16* at = is_q ? pp.q + (int64_t)qi * pp.q_rs + (int64_t)(hk * G + g) * pp.q_hs
-                                : (is_v ? pp.v + (int64_t)qi * pp.v_rs + (int64_t)hk * pp.v_hs : pp.k + (int64_t)qi * pp.k_rs + (int64_t)hk * pp.k_hs);
-        xin = *reinterpret_cast<const u32x4*>(at + 8 * dc);
-        wt = *reinterpret_cast<const u32x4*>((is_q ? pp.qw : pp.kw) + 8 * dc);
+        // (picked as distances from the first query head: as a choice of pointers the compiler made branches of it, with a
+        // trip to the arguments inside each)
+        auto bytes = [](const void* ptr) { return (int64_t)(uintptr_t)ptr; };
+        const int64_t at_q = bytes(pp.q + (int64_t)qi * pp.q_rs + (int64_t)(hk * G) * pp.q_hs);
+        const int64_t to_k = bytes(pp.k + (int64_t)qi * pp.k_rs + (int64_t)hk * pp.k_hs) - at_q;
+        const int64_t to_v = bytes(pp.v + (int64_t)qi * pp.v_rs + (int64_t)hk * pp.v_hs) - at_q;
+        const int64_t to_q = (int64_t)kq * pp.q_hs * 2, to_kw = bytes(pp.kw) - bytes(pp.qw);
+        xin = *reinterpret_cast<const u32x4*>((uintptr_t)(at_q + (is_q ? to_q : (is_v ? to_v : to_k)) + 16 * dc));
+        wt = *reinterpret_cast<const u32x4*>((uintptr_t)(bytes(pp.qw) + (is_q ? 0 : to_kw) + 16 * dc));
         cs = *reinterpret_cast<const u32x4*>(pp.cos + (int64_t)qi * pp.cs_rs + 8 * dc);
         sn = *reinterpret_cast<const u32x4*>(pp.sin + (int64_t)qi * pp.cs_rs + 8 * dc);
         if (pp.xn) {
@@ -852,28 +1032,38 @@ __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const St
         }
     }
     // where the sequence's rows lie, asked for together with which sequence it is: row i of a generation step is slot i
-    const int guess = qi < sp.nslots1 ? qi : sp.nslots1 - 1;
-    int start1 = *(guess >= 0 ? p.c1.start + guess : p.q_slot + qi), len1 = *(guess >= 0 ? p.c1.len + guess : p.q_slot + qi);
-    const int slot = p.q_slot[qi];
-    const int qpos = p.q_pos[qi];
-    const int qdepth = p.q_depth ? p.q_depth[qi] : p.depth;
-    const int aslot = pp.a.slot_of ? pp.a.slot_of[qi] : qi;  // < 0: the row is not cached
-    const int dst = sp.append_at[qi];
-    const int pos_new = pp.a.pos_new ? pp.a.pos_new[qi] : 0;
-    const int adepth = sp.append_depth ? (sp.append_depth[qi] != 0 ? 1 : 0) : sp.append_second;  // uniform per workgroup
+    // (the addresses picked by selects: a branch would be waited for)
+    const int guess1 = qi < sp.nslots1 ? qi : sp.nslots1 - 1, guess2 = qi < sp.nslots2 ? qi : sp.nslots2 - 1;
+    const int32_t* const nowhere = p.q_slot + qi;
+    const int first1 = *(guess1 >= 0 ? p.c1.start + guess1 : nowhere), held1 = *(guess1 >= 0 ? p.c1.len + guess1 : nowhere);
+    const int first2 = *(guess2 >= 0 ? p.c2.start + guess2 : nowhere), held2 = *(guess2 >= 0 ? p.c2.len + guess2 : nowhere);
+    const int slot_row = *nowhere, pos_row = p.q_pos[qi], at_row = sp.append_at[qi];
+    const int depth_row = *(p.q_depth ? p.q_depth + qi : nowhere), aslot_row = *(pp.a.slot_of ? pp.a.slot_of + qi : nowhere);
+    const int new_row = *(pp.a.pos_new ? pp.a.pos_new + qi : nowhere), second_row = *(sp.append_depth ? sp.append_depth + qi : nowhere);
+    // uniform per workgroup, and said to be: what is picked by them below then comes by scalar loads and branches
+    auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    const int slot = uniform(slot_row), qpos = uniform(pos_row), dst = uniform(at_row);
+    const int qdepth = p.q_depth ? uniform(depth_row) : p.depth;
+    const int aslot = pp.a.slot_of ? uniform(aslot_row) : qi;  // < 0: the row is not cached
+    const int pos_new = pp.a.pos_new ? uniform(new_row) : 0;
+    const int adepth = sp.append_depth ? (uniform(second_row) != 0 ? 1 : 0) : sp.append_second;
+    int start1 = uniform(first1), len1 = uniform(held1), start2 = uniform(first2), len2 = uniform(held2);
     const AppendParams& ap = sp.app[adepth];
     const bool cached = aslot >= 0, fits = cached && dst < ap.capacity;
-    if (slot >= 0 && slot != guess) {  // uniform per workgroup
-        start1 = p.c1.start[slot];
-        len1 = p.c1.len[slot];
+    if (slot >= 0 && slot != guess1) {
+        start1 = uniform(p.c1.start[slot]);
+        len1 = uniform(p.c1.len[slot]);
+    }
+    if (slot >= 0 && slot != guess2 && qdepth >= 1) {
+        start2 = uniform(p.c2.start[slot]);
+        len2 = uniform(p.c2.len[slot]);
     }
     // rows of a segment: with the new row where this call appends (nobody may read len[] of that segment here)
     auto visible = [&](int seg) {
         if (slot < 0 || (seg && qdepth < 1)) return 0;  // (slot < 0: a query without a sequence)
-        const int n = (seg == adepth && cached) ? (fits ? dst + 1 : (dst < ap.capacity ? dst : ap.capacity)) : (seg ? p.c2.len[slot] : len1);
+        const int n = (seg == adepth && cached) ? (fits ? dst + 1 : (dst < ap.capacity ? dst : ap.capacity)) : (seg ? len2 : len1);
         return seg ? n : (qpos + 1 < n ? (qpos + 1 > 0 ? qpos + 1 : 0) : n);
     };
-    constexpr int kBlock = 4 * kUnroll;
     // this wave's first block of cached rows goes on its way before the preparation below, which needs none of it
     const int nvis0 = visible(0);
     int nact = 1, split = 0;  // workgroups at work on this pair, and which of them this one is
@@ -885,11 +1075,18 @@ __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const St
     }
     const int row_first = (split * kWholeWaves + wave) * kBlock, row_step = nact * kWholeWaves * kBlock;
     const int64_t base0 = slot < 0 ? 0 : start1;
-    const __bf16* kbase0 = p.c1.k + base0 * p.c1.k_rs + (int64_t)hk * p.c1.k_hs + dc * 8;
-    const __bf16* vbase0 = p.c1.v + base0 * p.c1.v_rs + (int64_t)hk * p.c1.v_hs + dc * 8;
-    RowBlock<kUnroll> first;
+    const __bf16* kbase0 = p.c1.k + base0 * p.c1.k_rs + (int64_t)hk * p.c1.k_hs;
+    const __bf16* vbase0 = p.c1.v + base0 * p.c1.v_rs + (int64_t)hk * p.c1.v_hs;
+    const bool stream = stream_keys(nvis0 + visible(1), p.nq, p.hkv);
+    TileBlock first;
     const bool have_first = row_first < nvis0;  // uniform per wave
-    if (have_first) load_rows<kUnroll>(first, p.c1, false, kbase0, vbase0, nullptr, row_first, nvis0, kq);
+    // (asked for in any case, by waves without a block a row that is there: with a branch around these loads the compiler does not know
+    // how many are on their way behind the norm's row, and wave 0 waited for all of them before it prepared)
+    const __bf16* const some = pp.q + (int64_t)qi * pp.q_rs + (int64_t)(hk * G) * pp.q_hs;
+    load_tile(first, p.c1, false, nvis0 > 0 ? kbase0 : some, nvis0 > 0 ? vbase0 : some, nullptr, row_first, nvis0 > 0 ? nvis0 : 1, kq, dc, stream);
+    // where the new row goes and what its segment's length says, for wave 0 behind the barrier
+    const int append_start = *(cached ? ap.start + aslot : nowhere), append_len = *(cached ? ap.len + aslot : nowhere);
+    u32x4 prepared;
     if (wave == 0) {
         if (pp.xn) {
             // summed as qk_prep_kernel's 256 threads sum it (same strides, same order), so that the factor has the same bits
@@ -898,76 +1095,76 @@ __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const St
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
                 ss[w] = 0.f;
-                for (int c = (64 * w + lane) * 8; c < pp.xn_cols; c += 256 * 8) {
-                    const u32x4 x = c < 256 * 8 ? xn[w] : *reinterpret_cast<const u32x4*>(xr + c);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) ss[w] += bf16_lo(x[i]) * bf16_lo(x[i]) + bf16_hi(x[i]) * bf16_hi(x[i]);
+                for (int i = 0; i < 4; ++i) ss[w] += bf16_lo(xn[w][i]) * bf16_lo(xn[w][i]) + bf16_hi(xn[w][i]) * bf16_hi(xn[w][i]);
+                ss[w] = (64 * w + lane) * 8 < pp.xn_cols ? ss[w] : 0.f;
+            }
+            // (the rest of a longer row, in a loop of its own: a load in the loop above made wave 0 wait for its cache rows)
+            if (pp.xn_cols > 256 * 8) {
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    for (int c = (256 + 64 * w + lane) * 8; c < pp.xn_cols; c += 256 * 8) {
+                        const u32x4 x = *reinterpret_cast<const u32x4*>(xr + c);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) ss[w] += bf16_lo(x[i]) * bf16_lo(x[i]) + bf16_hi(x[i]) * bf16_hi(x[i]);
+                    }
                 }
             }
 #pragma unroll
-            for (int m = 32; m >= 1; m >>= 1)
-#pragma unroll
-                for (int w = 0; w < 4; ++w) ss[w] += __shfl_xor(ss[w], m);
+            for (int w = 0; w < 4; ++w) ss[w] = wave_sum_tree(ss[w]);
             const float total = (ss[0] + ss[1]) + (ss[2] + ss[3]);
             xin = scale_piece(xin, __builtin_amdgcn_rsqf(total / (float)pp.xn_cols + pp.xn_eps));
         }
-        u32x4 out = prep_head_piece(xin, wt, cs, sn, dc < 8 ? 0x80008000u : 0u, pp.eps);
+        prepared = prep_head_piece(xin, wt, cs, sn, dc < 8 ? 0x80008000u : 0u, pp.eps);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) out[i] = is_v ? xin[i] : out[i];
-        if (kq < kPieces) ready[kq][dc] = out;
+        for (int i = 0; i < 4; ++i) prepared[i] = is_v ? xin[i] : prepared[i];
+        if (kq < kPieces) ready[kq][dc] = prepared;
+    }
+    __syncthreads();
+    if (wave == 0) {  // the append, which nobody waits for
         if (cached && !fits && pp.a.overflow && tid == 0 && hk == 0 && split == 0) *pp.a.overflow = 1;
         if (fits && split == 0 && kq >= G && kq < kPieces) {
-            const int64_t drow = (int64_t)const_i32(ap.start, aslot) + dst;
+            const int64_t drow = (int64_t)append_start + dst;
             __bf16* to = is_v ? ap.cv + drow * ap.cv_rs + (int64_t)hk * ap.cv_hs : ap.ck + drow * ap.ck_rs + (int64_t)hk * ap.ck_hs;
-            *reinterpret_cast<u32x4*>(to + 8 * dc) = out;
+            *reinterpret_cast<u32x4*>(to + 8 * dc) = prepared;
             if (dc == 0 && hk == 0 && !is_v) {
                 if (ap.cpos && pp.a.pos_new) ap.cpos[(int64_t)aslot * ap.capacity + dst] = pos_new;
                 // (only this workgroup touches the length of the segment the row appends to)  A row placed anywhere but
                 // at the end of its slab leaves a gap of stale rows or overwrites cached ones: reported, not repaired.
-                if (ap.len[aslot] != dst && pp.a.overflow) *pp.a.overflow = 2;
+                if (append_len != dst && pp.a.overflow) *pp.a.overflow = 2;
                 ap.len[aslot] = dst + 1;
             }
         }
     }
-    __syncthreads();
-    u32x4 qv[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) qv[g] = ready[g][dc];
+    u32x4 qv[4];
+    load_query<G>(qv, reinterpret_cast<const __bf16*>(ready[0]), kD, kq, dc);
     SubRow sub;
-    sub.k = ready[G][dc];
-    sub.v = ready[G + 1][dc];
+    sub.k = ready[G];
+    sub.v = ready[G + 1];
     sub.pos = pos_new;
-    float m_run[G], l_run[G], acc[G][8];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        m_run[g] = kNegInf;
-        l_run[g] = 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[g][i] = 0.f;
-    }
+    TileState<G> st;
     // depth-0 segment: the block loaded above, then the wave's other turns
     sub.row = (adepth == 0 && fits) ? dst : -1;
-    if (have_first) attend_rows<G, kUnroll, true>(first, false, row_first, kq, qpos, p.scale_log2e, qv, m_run, l_run, acc, &sub);
+    if (have_first) attend_tile<G>(first, false, row_first, kq, dc, qpos, p.scale_log2e, qv, st, sub);
     for (int r_it = row_first + row_step; r_it < nvis0; r_it += row_step)
-        consume_rows<G, kUnroll, true>(p.c1, false, kbase0, vbase0, nullptr, r_it, nvis0, kq, qpos, p.scale_log2e, qv, m_run, l_run, acc, &sub);
+        consume_tile<G>(p.c1, false, kbase0, vbase0, nullptr, r_it, nvis0, kq, dc, qpos, p.scale_log2e, qv, st, sub, stream);
     // depth-1 segment
     const int nvis1 = visible(1);
     if (nvis1 > 0) {  // uniform per workgroup
         sub.row = (adepth == 1 && fits) ? dst : -1;
-        const int64_t base1 = p.c2.start[slot];
-        const __bf16* kbase1 = p.c2.k + base1 * p.c2.k_rs + (int64_t)hk * p.c2.k_hs + dc * 8;
-        const __bf16* vbase1 = p.c2.v + base1 * p.c2.v_rs + (int64_t)hk * p.c2.v_hs + dc * 8;
+        const int64_t base1 = start2;
+        const __bf16* kbase1 = p.c2.k + base1 * p.c2.k_rs + (int64_t)hk * p.c2.k_hs;
+        const __bf16* vbase1 = p.c2.v + base1 * p.c2.v_rs + (int64_t)hk * p.c2.v_hs;
         const int32_t* posbase = p.c2.pos + (int64_t)slot * p.c2.capacity;
         for (int r_it = row_first; r_it < nvis1; r_it += row_step)
-            consume_rows<G, kUnroll, true>(p.c2, true, kbase1, vbase1, posbase, r_it, nvis1, kq, qpos, p.scale_log2e, qv, m_run, l_run, acc, &sub);
+            consume_tile<G>(p.c2, true, kbase1, vbase1, posbase, r_it, nvis1, kq, dc, qpos, p.scale_log2e, qv, st, sub, stream);
     }
-    combine_row_groups<G>(m_run, l_run, acc);
-    if (kq == 0) park_partials<G>(red, wave, dc, m_run, l_run, acc);
+    park_wave<G>(red, wave, kq, dc, st);
     __syncthreads();
     for (int e = tid; e < G * kD; e += kWholeThreads) {
         const int g = e / kD, d = e % kD;
         float a, l, mx;
-        merge16<G>(red, g, d, a, l, mx);
+        merge_waves<G>(red, g, d, lane, a, l, mx);
         const int head = hk * G + g;
         if (kSplit && nact > 1) {
             float* out = sp.part + (((int64_t)qi * p.hkv + hk) * sp.nsplit + split) * (G * kPart) + g * kPart;
@@ -1424,6 +1621,7 @@ extern "C" int tah_duo_decode_step(const tah_qk_prep_args* prep, const tah_duo_d
     sp.app[0] = append_target(dec->c1);
     sp.app[1] = have2 ? append_target(dec->c2) : AppendParams{};
     sp.nslots1 = dec->c1.nslots;
+    sp.nslots2 = have2 ? dec->c2.nslots : 0;
     sp.append_at = append_at;
     sp.append_depth = append_depth;
     hipStream_t st = static_cast<hipStream_t>(stream);

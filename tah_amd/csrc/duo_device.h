@@ -63,10 +63,12 @@ __device__ __forceinline__ void device_max(unsigned long long* p, unsigned long 
 #define TAH_WAIT_LDS() ((void)0)
 #define TAH_SLEEP(n) ((void)0)
 #define TAH_OPAQUE_S(p) ((void)0)
+#define TAH_APART() ((void)0)
 #define TAH_GLOBAL
 #else
 #define TAH_WAIT_LDS() __builtin_amdgcn_s_waitcnt(0xC07F)  // s_waitcnt lgkmcnt(0), loads from memory stay on their way
 #define TAH_SLEEP(n) __builtin_amdgcn_s_sleep(n)
+#define TAH_APART() asm volatile("; apart")  // no instruction: keeps what stands in one branch from being merged with its like in the other
 #define TAH_OPAQUE_S(p) asm volatile("" : "+s"(p))  // a value that stays in scalar registers, apart from those it was made of
 #define TAH_GLOBAL __attribute__((address_space(1)))
 #endif
@@ -324,6 +326,28 @@ __device__ __forceinline__ float wave_max_xor32(float x) {
 __device__ __forceinline__ float wave_sum_xor32(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// the same over lanes l and l^16 (v_permlane16_swap)
+__device__ __forceinline__ float wave_max_xor16(float x) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float wave_sum_xor16(float x) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// Sum over a wave in every lane, in the pairs of a shuffle tree from 32 down to 1 (the same bits) without its trips through LDS.  Behind the
+// pairs 32, 16 and 8 apart lanes that differ in those bits hold the same number, so turning a row by 4, 2 and 1 is the pairs that far apart.
+__device__ __forceinline__ float wave_sum_tree(float x) {
+    x = wave_sum_xor16(wave_sum_xor32(x));
+    const auto turned = [](float v, auto by) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + decltype(by)::value, 0xf, 0xf, true));  // row_ror
+    };
+    x += turned(x, std::integral_constant<int, 8>{});
+    x += turned(x, std::integral_constant<int, 4>{});
+    x += turned(x, std::integral_constant<int, 2>{});
+    return x + turned(x, std::integral_constant<int, 1>{});
 }
 
 // x of one lane, the same one for the whole wave

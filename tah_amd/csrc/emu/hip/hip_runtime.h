@@ -298,11 +298,24 @@ inline emu_u32pair emu_permlane32_swap(unsigned a, unsigned b, bool, bool) {
     return l < 32 ? emu_u32pair{{lo[0], hi[0]}} : emu_u32pair{{lo[1], hi[1]}};
 }
 #define __builtin_amdgcn_permlane32_swap emu_permlane32_swap
+// v_permlane16_swap(a, b): the same between neighbouring rows of sixteen lanes
+inline emu_u32pair emu_permlane16_swap(unsigned a, unsigned b, bool, bool) {
+    unsigned mine[2] = {a, b};
+    memcpy(emu::t_wave->box[emu::t_lane], mine, 8);
+    emu::wave_sync();
+    const int l = emu::t_lane;
+    unsigned lo[2], hi[2];
+    memcpy(lo, emu::t_wave->box[l & ~16], 8);
+    memcpy(hi, emu::t_wave->box[l | 16], 8);
+    emu::wave_sync();
+    return (l & 16) == 0 ? emu_u32pair{{lo[0], hi[0]}} : emu_u32pair{{lo[1], hi[1]}};
+}
+#define __builtin_amdgcn_permlane16_swap emu_permlane16_swap
 inline int __float_as_int(float x) { int i; memcpy(&i, &x, 4); return i; }
 inline float __int_as_float(int i) { float x; memcpy(&x, &i, 4); return x; }
 // DPP lane selects used by the kernels: quad_perm, row_shl/shr/ror, row_mirror, row_half_mirror, row_bcast:15/31 (rows that
 // row_mask leaves out keep `old`).
-inline int emu_update_dpp(int old, int src, int ctrl, int row_mask, int, bool bound_ctrl) {
+inline int emu_update_dpp(int old, int src, int ctrl, int row_mask, int bank_mask, bool bound_ctrl) {
     const int l = emu::t_lane, row = l & ~15, i = l & 15;
     int from = -1;
     if (ctrl < 0x100) from = (l & ~3) + ((ctrl >> (2 * (l & 3))) & 3);
@@ -315,7 +328,7 @@ inline int emu_update_dpp(int old, int src, int ctrl, int row_mask, int, bool bo
     else if (ctrl == 0x143) from = row >= 32 ? 31 : -1;
     else { fprintf(stderr, "emu: unsupported dpp_ctrl 0x%x\n", ctrl); abort(); }
     const int got = emu::exchange(src, from < 0 ? l : from);
-    if (!(row_mask >> (l / 16) & 1)) return old;
+    if (!(row_mask >> (l / 16) & 1) || !(bank_mask >> (i / 4) & 1)) return old;
     return from < 0 ? (bound_ctrl ? 0 : old) : got;
 }
 #define __builtin_amdgcn_update_dpp emu_update_dpp

@@ -168,3 +168,26 @@ def test_fused_decode_steps_of_several_sizes_share_a_workspace():
         print(f"shared workspace B={B} hq={hq} hkv={hkv} cap={cap}", flush=True)
         for case in (decode_step_case.run, decode_step_case.run_mixed):
             case("cuda", B=B, hq=hq, hkv=hkv, seed=B + cap, max_len=cap - 1, hidden=2048, cap1=cap, cap2=cap // 4, workspace=ws)
+
+
+@pytest.mark.parametrize("hq,hkv", [(8, 8), (16, 8), (16, 4), (16, 2)])
+@pytest.mark.parametrize("copies", [1, 4])  # split rows, and (up to four query heads) one workgroup per pair
+def test_blocks_of_sixteen_rows_that_are_not_full(hq, hkv, copies):
+    """A wave's block is sixteen rows, a workgroup's turn 64 or 256 of them: contexts of one row, and at and beside those edges."""
+    lens = [1, 2, 7, 8, 9, 15, 16, 17, 31, 33, 63, 65, 255, 256, 257, 273] * copies
+    print(f"blocks hq={hq} hkv={hkv} copies={copies}", flush=True)
+    c = make_decode_case(7 * hq + hkv, lens, 0.2, Hq=hq, Hkv=hkv, hard_new=[b % 3 == 0 for b in range(len(lens))])
+    got = run_decode(c, 300, 128, True)
+    w0, wl0, w1, wl1 = oracle_decode_c(c)
+    assert_close(got[0], w0, "decode o depth0")
+    assert_close(got[2], w1, "decode o depth1")
+    np.testing.assert_allclose(got[1].cpu().numpy(), wl0, atol=5e-3, rtol=1e-3)
+    np.testing.assert_allclose(got[3].cpu().numpy(), wl1, atol=5e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("hidden", [8, 2040, 2056, 4104])
+def test_fused_decode_step_norm_of_rows_of_any_length(hidden):
+    """The input norm's row is read in pieces of 2048 values: less than one, one and a bit, two and a bit."""
+    from tests import decode_step_case
+    print(f"decode step, norm over {hidden}", flush=True)
+    decode_step_case.run("cuda", B=32, hq=16, hkv=8, seed=hidden, max_len=300, hidden=hidden, cap1=512, cap2=128)
