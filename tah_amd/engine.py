@@ -281,11 +281,15 @@ class DecodeEngine:
         return out
 
     def _new_batch(self) -> None:
-        """A new batch begins: a step captured for an earlier one is kept where all that it holds is still the engine's (a step of
-        generate_1's size takes 1.8 ms to warm up and capture, one of 32 rows 4.5) and where replaying it leaves the random
-        numbers as capturing it would."""
-        if self._graph is not None and not (self._graph_over is not None and _same_leaves(self._graph_over, self._captured_over())):
-            self._graph = self._graph_over = None
+        """A new batch begins: a step captured for an earlier one may serve it (one row's step of eight layers takes 1.8 ms to warm up and
+        capture, one of 32 rows 4.5) where replaying it leaves the random numbers as capturing it would.  Whether all that it
+        holds is still the engine's is asked where it is handed out (``_holds``)."""
+        if self._graph_over is None:
+            self._graph = None
+
+    def _holds(self, over: Optional[list]) -> bool:
+        """Whether a step captured over ``over`` may be replayed now.  (None: only the batch that it was captured for asks.)"""
+        return over is None or _same_leaves(over, self._captured_over())
 
     def _launch_switches(self):
         """Every attribute that changes which kernels a captured step launches: part of the graph keys, so that
@@ -449,7 +453,7 @@ class DecodeEngine:
         """Captures one generation step in a HIP graph (after a warm-up step run on a side stream whose state
         changes are undone, so that library workspaces exist before the capture)."""
         key = (temperature, eos, tuple(sorted(filters.items()))) + self._launch_switches()
-        if self._graph is not None and self._graph_key == key:
+        if self._graph is not None and self._graph_key == key and self._holds(self._graph_over):
             return self._graph
         undo = self._hold_state()
         s = torch.cuda.Stream()
@@ -911,8 +915,8 @@ class TaHDecodeEngine(DecodeEngine):
         if self.decider is not None:  # (leaves the last decision's logits where a capture puts them)
             self._graph = self._tick_graphs = None
         super()._new_batch()
-        if self._tick_graphs is not None and not (self._tick_over is not None and _same_leaves(self._tick_over, self._captured_over())):
-            self._tick_graphs = self._tick_over = None
+        if self._tick_over is None:
+            self._tick_graphs = None
         self.draw_again = self._tick_graphs is not None
 
     def _state(self):
@@ -1018,7 +1022,7 @@ class TaHDecodeEngine(DecodeEngine):
         self._close_pass()
         key = (eos, limit, self.w.threshold, temperature, tuple(sorted(filters.items()))) + self._launch_switches()
         by_step = self._draws_by_step(temperature, filters)
-        if self._tick_graphs is not None and self._tick_key == key:
+        if self._tick_graphs is not None and self._tick_key == key and self._holds(self._tick_over):
             if self.draw_again and by_step:
                 torch.rand(self.B, device=self.device)
             self.draw_again = False

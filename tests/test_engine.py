@@ -801,3 +801,77 @@ def test_a_captured_tick_serves_the_next_batch_gpu(temperature):
         e.use_fused_glue = True  # (as it was)
         e.linear_chain = False
         assert not next_batch()[0]
+
+
+@pytest.fixture
+def captured_nothing(monkeypatch):
+    """``capture`` and ``capture_ticks`` on the host alone: streams and graphs are stand-ins, the step and the tick do nothing."""
+    import contextlib
+    import types
+
+    from tah_amd.engine import DecodeEngine, TaHDecodeEngine
+    stream = types.SimpleNamespace(wait_stream=lambda s: None)
+    for name, stand_in in dict(Stream=lambda: stream, current_stream=lambda: stream, stream=lambda s: contextlib.nullcontext(), synchronize=lambda: None,
+                               CUDAGraph=type("Graph", (), {}), graph=lambda g: contextlib.nullcontext()).items():
+        monkeypatch.setattr(torch.cuda, name, stand_in)
+    monkeypatch.setattr(DecodeEngine, "_step_inplace", lambda self, *args, **kw: None)
+    monkeypatch.setattr(TaHDecodeEngine, "_tick", lambda self, *args, **kw: None)
+
+
+def _small_engine(**kw):
+    from tah_amd.engine import EngineConfig, TaHDecodeEngine, Weights
+    cfg = EngineConfig(hidden=256, layers=2, hq=2, hkv=1, head_dim=128, intermediate=256, vocab=96, decider_hidden=32)
+    return TaHDecodeEngine(Weights.random_init(cfg, "cpu", seed=1), 1, 8, device="cpu", **kw)
+
+
+_HAND_OUTS = {"step": lambda e: e.capture(), "ticks": lambda e: e.capture_ticks(-1, 8)}
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+@pytest.mark.parametrize("which", list(_HAND_OUTS))
+def test_a_kept_graph_is_compared_where_it_is_handed_out_on_cpu_shim(which, captured_nothing):
+    """What a caller, or ``prefill(calibrate=)`` itself, changes once the new batch has begun."""
+    hand_out = _HAND_OUTS[which]
+    with emu_util.emulated(), torch.no_grad():
+        e = _small_engine()
+
+        def kept_when(change):
+            was = hand_out(e)
+            e._new_batch()
+            change()
+            return hand_out(e) is was
+
+        assert kept_when(lambda: None)
+        assert not kept_when(lambda: setattr(e.w, "threshold", e.w.threshold + 0.125))
+        assert not kept_when(lambda: e.w.layers[1].update(wqkv=e.w.layers[1]["wqkv"].clone()))
+        assert not kept_when(lambda: setattr(e, "cos", e.cos.clone()))
+        assert kept_when(lambda: None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("continuous", [False, True])
+def test_a_kept_graph_sees_what_changed_behind_the_prefill_gpu(continuous):
+    """A second batch whose prefill moves the decider's threshold, and one whose weights are replaced between prefill and generate: the tokens
+    of an engine that captures for each batch."""
+    from tah_amd.engine import EngineConfig, TaHDecodeEngine, Weights
+    ids = torch.randint(0, 4096, (50,), generator=torch.Generator().manual_seed(2)).cuda()
+    cu = torch.tensor([0, 30, 50], dtype=torch.int32).cuda()
+
+    def run(keep):
+        e = TaHDecodeEngine(Weights.random_init(EngineConfig(layers=3, vocab=4096), "cuda", seed=3), 2, 128)
+        out = []
+        for p, replace in ((0.6, False), (0.05, False), (0.05, True)):
+            first, _ = e.prefill(ids, cu, calibrate=p)
+            if replace:
+                e.w.layers[1]["wo_p"] = torch.zeros_like(e.w.layers[1]["wo_p"])
+                e.w.layers[1]["wdown_p"] = torch.zeros_like(e.w.layers[1]["wdown_p"])
+            if not keep:
+                e._graph = e._tick_graphs = None
+            out.append((e.generate(first, 20, continuous=continuous).clone(), int(e.n_hard)))
+        return out
+
+    with torch.no_grad():
+        got, want = run(True), run(False)
+    for (tokens, hard), (tokens_want, hard_want) in zip(got, want):
+        assert torch.equal(tokens, tokens_want) and hard == hard_want
+    assert got[0][1] != got[1][1]
