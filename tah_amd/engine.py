@@ -1014,8 +1014,8 @@ class TaHDecodeEngine(DecodeEngine):
     DRAW_AHEAD = 64  # ticks whose uniforms are drawn at a time at most
     LAST_TICKS = 8   # how often the host looks once the fastest possible row could be done
 
-    def _launch_switches(self):
-        return super()._launch_switches() + (self.use_fused_glue, self.static_scratch, self.measure_without_attention, self.linear_chain, id(self.decider))
+    def _launch_switches(self):  # (the threshold, too, is part of a launch: a number among its arguments)
+        return super()._launch_switches() + (self.w.threshold, self.use_fused_glue, self.static_scratch, self.measure_without_attention, self.linear_chain, id(self.decider))
 
     def capture_ticks(self, eos: int, limit: int, temperature: float = 0.0, **filters):
         """The tick as two HIP graphs, one per logits buffer, after a warm-up tick whose state changes are undone."""

@@ -848,6 +848,18 @@ def test_a_kept_graph_is_compared_where_it_is_handed_out_on_cpu_shim(which, capt
         assert kept_when(lambda: None)
 
 
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+@pytest.mark.parametrize("draw", [{}, dict(temperature=0.7), dict(temperature=0.7, top_k=3)])
+def test_a_step_captured_with_another_threshold_is_not_handed_out_on_cpu_shim(draw, captured_nothing):
+    """On one and the same batch; drawn steps are not compared further."""
+    with emu_util.emulated(), torch.no_grad():
+        e = _small_engine()
+        was = e.capture(**draw)
+        assert e.capture(**draw) is was
+        e.w.threshold += 0.125
+        assert e.capture(**draw) is not was
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("continuous", [False, True])
 def test_a_kept_graph_sees_what_changed_behind_the_prefill_gpu(continuous):
