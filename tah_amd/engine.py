@@ -200,7 +200,8 @@ _PLAIN = (int, float, str, bool, type(None), torch.dtype, torch.device)
 
 def _leaves(x, out: list, seen: set) -> list:
     """What a captured step may hold of ``x``, in a fixed order: plain values, tensors with their addresses, and objects that are
-    neither (kernel objects), the latter two weakly.  Containers and this package's objects are walked, engines are not."""
+    neither (kernel objects), the latter two weakly.  Containers and this package's objects are walked, engines are not.
+    ``TypeError`` where something cannot be told from its like later on: it has no weak references."""
     if isinstance(x, _PLAIN):
         out.append(x)
     elif isinstance(x, torch.Tensor):
@@ -271,13 +272,17 @@ class DecodeEngine:
     _BETWEEN_STEPS = ("host_positions", "host_hard_rows", "ticks", "binding", "pool", "pass_open", "decision_logits", "draw_again",
                       "_positions_on_device", "_graph", "_graph_key", "_graph_over", "_tick_graphs", "_tick_key", "_tick_over")
 
-    def _captured_over(self) -> list:
-        """Everything of the engine and its weights that a captured step may hold."""
+    def _captured_over(self) -> Optional[list]:
+        """Everything of the engine and its weights that a captured step may hold; None where some of it cannot be told from its
+        like later on (a captured step then serves the batch that it was captured for)."""
         out, seen = [], {id(self)}
-        for k, v in vars(self).items():
-            if k not in self._BETWEEN_STEPS:
-                out.append(k)
-                _leaves(v, out, seen)
+        try:
+            for k, v in vars(self).items():
+                if k not in self._BETWEEN_STEPS:
+                    out.append(k)
+                    _leaves(v, out, seen)
+        except TypeError:
+            return None
         return out
 
     def _new_batch(self) -> None:
@@ -289,7 +294,7 @@ class DecodeEngine:
 
     def _holds(self, over: Optional[list]) -> bool:
         """Whether a step captured over ``over`` may be replayed now.  (None: only the batch that it was captured for asks.)"""
-        return over is None or _same_leaves(over, self._captured_over())
+        return over is None or _same_leaves(over, self._captured_over() or [])
 
     def _launch_switches(self):
         """Every attribute that changes which kernels a captured step launches: part of the graph keys, so that

@@ -1,4 +1,5 @@
 """Decode engine: the iteration loop for one token per sequence on the native kernels."""
+import numpy as np
 import pytest
 import torch
 
@@ -858,6 +859,24 @@ def test_a_step_captured_with_another_threshold_is_not_handed_out_on_cpu_shim(dr
         assert e.capture(**draw) is was
         e.w.threshold += 0.125
         assert e.capture(**draw) is not was
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_values_without_weak_references_on_cpu_shim(captured_nothing):
+    """As a threshold, and on the engine, its weights and its configuration: captured as before, kept for one batch."""
+    with emu_util.emulated(), torch.no_grad():
+        e = _small_engine()
+        places = [(e.w, "threshold", np.float32(0.375)), (e.w, "threshold", np.int64(1))]
+        places += [(owner, "note", value) for owner in (e, e.w, e.cfg) for value in (b"note", range(3))]
+        for owner, name, value in places:
+            before = getattr(owner, name, None)
+            setattr(owner, name, value)
+            for hand_out in _HAND_OUTS.values():
+                was = hand_out(e)
+                assert hand_out(e) is was
+                e._new_batch()
+                assert hand_out(e) is not was
+            setattr(owner, name, before)
 
 
 @pytest.mark.gpu
