@@ -258,6 +258,7 @@ class DecodeEngine:
         self.host_positions = 0  # upper bound on any sequence's length, kept on the host for capacity checks
         self._graph = None
         self._graph_over = None  # what the captured step holds, where another batch may replay it
+        self._graph_carried = False  # it is of an earlier batch, and this one has not been handed it yet
 
     def _parts(self):
         """One step of all rows on the engine's own state: (logits, logits of a second iteration or None, which rows
@@ -269,8 +270,8 @@ class DecodeEngine:
         raise NotImplementedError
 
     # attributes that change from call to call and are no part of a captured step
-    _BETWEEN_STEPS = ("host_positions", "host_hard_rows", "ticks", "binding", "pool", "pass_open", "decision_logits", "draw_again",
-                      "_positions_on_device", "_graph", "_graph_key", "_graph_over", "_tick_graphs", "_tick_key", "_tick_over")
+    _BETWEEN_STEPS = ("host_positions", "host_hard_rows", "ticks", "binding", "pool", "pass_open", "decision_logits", "_positions_on_device",
+                      "_graph", "_graph_key", "_graph_over", "_graph_carried", "_tick_graphs", "_tick_key", "_tick_over", "_ticks_carried")
 
     def _captured_over(self) -> Optional[list]:
         """Everything of the engine and its weights that a captured step may hold; None where some of it cannot be told from its
@@ -291,10 +292,11 @@ class DecodeEngine:
         holds is still the engine's is asked where it is handed out (``_holds``)."""
         if self._graph_over is None:
             self._graph = None
+        self._graph_carried = self._graph is not None
 
-    def _holds(self, over: Optional[list]) -> bool:
-        """Whether a step captured over ``over`` may be replayed now.  (None: only the batch that it was captured for asks.)"""
-        return over is None or _same_leaves(over, self._captured_over() or [])
+    def _holds(self, over: list) -> bool:
+        """Whether a step captured over ``over`` for an earlier batch may be replayed.  (Asked once a batch: 1.8 ms for 28 layers.)"""
+        return _same_leaves(over, self._captured_over() or [])
 
     def _launch_switches(self):
         """Every attribute that changes which kernels a captured step launches: part of the graph keys, so that
@@ -458,7 +460,8 @@ class DecodeEngine:
         """Captures one generation step in a HIP graph (after a warm-up step run on a side stream whose state
         changes are undone, so that library workspaces exist before the capture)."""
         key = (temperature, eos, tuple(sorted(filters.items()))) + self._launch_switches()
-        if self._graph is not None and self._graph_key == key and self._holds(self._graph_over):
+        if self._graph is not None and self._graph_key == key and (not self._graph_carried or self._holds(self._graph_over)):
+            self._graph_carried = False
             return self._graph
         undo = self._hold_state()
         s = torch.cuda.Stream()
@@ -471,7 +474,7 @@ class DecodeEngine:
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g):
             self._step_inplace(temperature, eos, **filters)
-        self._graph, self._graph_key = g, key
+        self._graph, self._graph_key, self._graph_carried = g, key, False
         self._graph_over = self._captured_over() if temperature <= 0.0 else None  # (draws inside a step: the warm-up took some too)
         return g
 
@@ -559,7 +562,8 @@ class TaHDecodeEngine(DecodeEngine):
             self.logits2 = [torch.zeros(batch, cfg.vocab, dtype=torch.bfloat16, device=dev) for _ in range(2)]
         self._tick_graphs = None
         self._tick_over = None
-        self.draw_again = False  # kept graphs: the numbers that their warm-up would have drawn for this batch are not drawn yet
+        # of an earlier batch, and not handed out yet: the numbers that their warm-up would have drawn for this batch are not drawn
+        self._ticks_carried = False
         # Engines with a workspace draw a row's n-th token with the number a step-wise loop would draw it with: a table of the
         # steps' uniforms, one row per token, so that sampled tokens do not depend on the schedule either.
         self.uniforms = (torch.zeros(max_len + 1, batch, dtype=torch.float32, device=dev)
@@ -922,7 +926,7 @@ class TaHDecodeEngine(DecodeEngine):
         super()._new_batch()
         if self._tick_over is None:
             self._tick_graphs = None
-        self.draw_again = self._tick_graphs is not None
+        self._ticks_carried = self._tick_graphs is not None
 
     def _state(self):
         return super()._state() + (self.hard_len, self.phase)
@@ -1027,12 +1031,11 @@ class TaHDecodeEngine(DecodeEngine):
         self._close_pass()
         key = (eos, limit, self.w.threshold, temperature, tuple(sorted(filters.items()))) + self._launch_switches()
         by_step = self._draws_by_step(temperature, filters)
-        if self._tick_graphs is not None and self._tick_key == key and self._holds(self._tick_over):
-            if self.draw_again and by_step:
+        if self._tick_graphs is not None and self._tick_key == key and (not self._ticks_carried or self._holds(self._tick_over)):
+            if self._ticks_carried and by_step:
                 torch.rand(self.B, device=self.device)
-            self.draw_again = False
+            self._ticks_carried = False
             return self._tick_graphs
-        self.draw_again = False
         undo = self._hold_state()
         if by_step:
             torch.rand(self.B, device=self.device)  # what the warm-up step of ``capture`` draws
@@ -1049,7 +1052,7 @@ class TaHDecodeEngine(DecodeEngine):
             with torch.cuda.graph(g):
                 self._tick(parity, eos, limit, temperature, **filters)
             graphs.append(g)
-        self._tick_graphs, self._tick_key = graphs, key
+        self._tick_graphs, self._tick_key, self._ticks_carried = graphs, key, False
         self._tick_over = self._captured_over() if temperature <= 0.0 or by_step else None
         return graphs
 

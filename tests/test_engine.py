@@ -830,7 +830,7 @@ _HAND_OUTS = {"step": lambda e: e.capture(), "ticks": lambda e: e.capture_ticks(
 
 @pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
 @pytest.mark.parametrize("which", list(_HAND_OUTS))
-def test_a_kept_graph_is_compared_where_it_is_handed_out_on_cpu_shim(which, captured_nothing):
+def test_a_kept_graph_is_compared_where_it_is_handed_out_on_cpu_shim(which, captured_nothing, monkeypatch):
     """What a caller, or ``prefill(calibrate=)`` itself, changes once the new batch has begun."""
     hand_out = _HAND_OUTS[which]
     with emu_util.emulated(), torch.no_grad():
@@ -847,6 +847,10 @@ def test_a_kept_graph_is_compared_where_it_is_handed_out_on_cpu_shim(which, capt
         assert not kept_when(lambda: e.w.layers[1].update(wqkv=e.w.layers[1]["wqkv"].clone()))
         assert not kept_when(lambda: setattr(e, "cos", e.cos.clone()))
         assert kept_when(lambda: None)
+        # and once a batch: to the next generate of the batch the key is enough
+        was = hand_out(e)
+        monkeypatch.setattr(e, "_captured_over", None)
+        assert hand_out(e) is was
 
 
 @pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
