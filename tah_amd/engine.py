@@ -32,6 +32,7 @@ from __future__ import annotations
 
 import dataclasses
 import math
+import types
 import weakref
 from typing import List, Optional, Tuple
 
@@ -196,12 +197,13 @@ def rope_tables(max_len: int, head_dim: int, theta: float, device, dtype=torch.b
 
 
 _PLAIN = (int, float, str, bool, type(None), torch.dtype, torch.device)
+_FIXED = (type, types.ModuleType, types.FunctionType, types.BuiltinFunctionType)
 
 
 def _leaves(x, out: list, seen: set) -> list:
     """What a captured step may hold of ``x``, in a fixed order: plain values, tensors with their addresses, and objects that are
-    neither (kernel objects), the latter two weakly.  Containers and this package's objects are walked, engines are not.
-    ``TypeError`` where something cannot be told from its like later on: it has no weak references."""
+    neither, the latter two weakly.  Containers and what objects have for attributes are walked, engines are not.  ``TypeError``
+    where something cannot be told from its like later on: it has no weak references, or may change and shows nothing of it."""
     if isinstance(x, _PLAIN):
         out.append(x)
     elif isinstance(x, torch.Tensor):
@@ -216,14 +218,18 @@ def _leaves(x, out: list, seen: set) -> list:
             _leaves(v, out, seen)
     elif isinstance(x, DecodeEngine):
         pass
-    elif type(x).__module__.startswith("tah_amd.") and hasattr(x, "__dict__"):
+    elif isinstance(x, _FIXED) or type(x).__module__ == "tah_amd._C":  # (kernel objects hold what they were made of)
+        out.append((weakref.ref(x), None))
+    elif hasattr(x, "__dict__"):
         if id(x) not in seen:
             seen.add(id(x))
+            if not type(x).__module__.startswith("tah_amd."):  # (and may have more than that)
+                out.append((weakref.ref(x), None))
             for k, v in vars(x).items():
                 out.append(k)
                 _leaves(v, out, seen)
     else:
-        out.append((weakref.ref(x), None))
+        raise TypeError(f"a {type(x).__name__} may change unseen")
     return out
 
 
@@ -282,7 +288,7 @@ class DecodeEngine:
                 if k not in self._BETWEEN_STEPS:
                     out.append(k)
                     _leaves(v, out, seen)
-        except TypeError:
+        except (TypeError, RecursionError):
             return None
         return out
 

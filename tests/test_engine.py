@@ -883,6 +883,45 @@ def test_values_without_weak_references_on_cpu_shim(captured_nothing):
             setattr(owner, name, before)
 
 
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_objects_of_other_modules_are_looked_into_on_cpu_shim(captured_nothing):
+    """Weights of a class of the caller's own, objects with attributes, with slots and with neither on the engine."""
+    from tah_amd.engine import EngineConfig, TaHDecodeEngine, Weights
+
+    class OwnWeights(Weights):
+        pass
+
+    class Own:
+        pass
+
+    class Slots:
+        __slots__ = ("scale", "__weakref__")
+
+    round_and_round = []
+    round_and_round.append(round_and_round)
+    with emu_util.emulated(), torch.no_grad():
+        cfg = EngineConfig(hidden=256, layers=2, hq=2, hkv=1, head_dim=128, intermediate=256, vocab=96, decider_hidden=32)
+        e = TaHDecodeEngine(OwnWeights.random_init(cfg, "cpu", seed=1), 1, 8, device="cpu")
+        e.w.__class__ = OwnWeights
+        e.own = Own()
+        e.own.scale, e.own.tensor = 1.0, torch.zeros(3)
+
+        def kept_when(change):
+            was = e.capture()
+            e._new_batch()
+            change()
+            return e.capture() is was
+
+        assert kept_when(lambda: None)
+        assert not kept_when(lambda: e.w.layers[1].update(wqkv=e.w.layers[1]["wqkv"].clone()))
+        assert not kept_when(lambda: setattr(e.own, "scale", 2.0))
+        assert not kept_when(lambda: setattr(e.own, "tensor", torch.zeros(3)))
+        assert kept_when(lambda: None)
+        for unknown in (Slots(), np.zeros(2), round_and_round):
+            e.own = unknown
+            assert not kept_when(lambda: None)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("continuous", [False, True])
 def test_a_kept_graph_sees_what_changed_behind_the_prefill_gpu(continuous):
