@@ -968,7 +968,7 @@ struct StepParams {
     float* part;                   // kSplit: partials [nq][hkv][nsplit][G][kPart] ...
     int32_t* arrived;              // ... and workgroups of a pair that are done, [nq][hkv], 0 between calls
     int32_t nsplit, fill;          // workgroups per pair at most, and as many as it takes to give every compute unit one
-    int32_t nslots1, nslots2;      // slots of the depth-0 segment and, 0 without one, of the depth-1 segment
+    int32_t nslots1, nslots2;      // slots of the depth-0 and the depth-1 segment; 0 where there is none or it holds no row
 };
 
 // Calls with too few (query, kv head) pairs to fill the chip, or slabs too long for one workgroup per pair: up to
@@ -1050,14 +1050,17 @@ __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const St
     int start1 = uniform(first1), len1 = uniform(held1), start2 = uniform(first2), len2 = uniform(held2);
     const AppendParams& ap = sp.app[adepth];
     const bool cached = aslot >= 0, fits = cached && dst < ap.capacity;
-    if (slot >= 0 && slot != guess1) {
+    // (a segment that holds no row may come without its pointers)
+    if (slot >= 0 && slot != guess1 && p.c1.capacity > 0) {
         start1 = uniform(p.c1.start[slot]);
         len1 = uniform(p.c1.len[slot]);
     }
-    if (slot >= 0 && slot != guess2 && qdepth >= 1) {
+    if (slot >= 0 && slot != guess2 && qdepth >= 1 && p.c2.capacity > 0) {
         start2 = uniform(p.c2.start[slot]);
         len2 = uniform(p.c2.len[slot]);
     }
+    len1 = p.c1.capacity > 0 ? len1 : 0;
+    len2 = p.c2.capacity > 0 ? len2 : 0;
     // rows of a segment: with the new row where this call appends (nobody may read len[] of that segment here)
     auto visible = [&](int seg) {
         if (slot < 0 || (seg && qdepth < 1)) return 0;  // (slot < 0: a query without a sequence)
@@ -1085,7 +1088,7 @@ __global__ __launch_bounds__(kWholeThreads) void duo_decode_step_kernel(const St
     const __bf16* const some = pp.q + (int64_t)qi * pp.q_rs + (int64_t)(hk * G) * pp.q_hs;
     load_tile(first, p.c1, false, nvis0 > 0 ? kbase0 : some, nvis0 > 0 ? vbase0 : some, nullptr, row_first, nvis0 > 0 ? nvis0 : 1, kq, dc, stream);
     // where the new row goes and what its segment's length says, for wave 0 behind the barrier
-    const int append_start = *(cached ? ap.start + aslot : nowhere), append_len = *(cached ? ap.len + aslot : nowhere);
+    const int append_start = *(fits ? ap.start + aslot : nowhere), append_len = *(fits ? ap.len + aslot : nowhere);
     u32x4 prepared;
     if (wave == 0) {
         if (pp.xn) {
@@ -1620,8 +1623,8 @@ extern "C" int tah_duo_decode_step(const tah_qk_prep_args* prep, const tah_duo_d
     if (append_depth && !have2) return TAH_E_SHAPE;  // rows that append to the depth-1 segment need it
     sp.app[0] = append_target(dec->c1);
     sp.app[1] = have2 ? append_target(dec->c2) : AppendParams{};
-    sp.nslots1 = dec->c1.nslots;
-    sp.nslots2 = have2 ? dec->c2.nslots : 0;
+    sp.nslots1 = dec->c1.capacity > 0 ? dec->c1.nslots : 0;
+    sp.nslots2 = have2 && dec->c2.capacity > 0 ? dec->c2.nslots : 0;
     sp.append_at = append_at;
     sp.append_depth = append_depth;
     hipStream_t st = static_cast<hipStream_t>(stream);

@@ -116,3 +116,72 @@ def test_fused_decode_step_with_a_pairs_rows_shared_by_workgroups_on_cpu_shim():
         with pytest.raises(TahDuoError):
             decode_step_case.run("cpu", B=3, hq=2, hkv=1, seed=8)
         assert kv_cache.decode_step_workspace(3, 4, 1, 1500, 700, "cpu") is None  # four query heads per kv head
+
+
+def test_fused_decode_step_with_an_empty_segment_without_pointers_on_cpu_shim():
+    """A depth-1 segment of no capacity, described by null pointers: beside queries of depth 0, and as the place of a new row that
+    does not fit.  And a depth-0 segment of that kind beside a depth-1 segment that takes the rows."""
+    import ctypes as C
+
+    from tah_amd import _capi, kv_cache
+    from tah_amd.kv_cache import KvSlabs
+    B, hq, hkv = 2, 8, 8
+    g = torch.Generator().manual_seed(4)
+    rn = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32)
+    q, k, v, qw, kw = rn(B, hq, 128), rn(B, hkv, 128), rn(B, hkv, 128), rn(128), rn(128)
+    ang = torch.randn(B, 128, generator=g)
+    cos, sin = ang.cos().to(torch.bfloat16), ang.sin().to(torch.bfloat16)
+    rows, cu, pos = i32(0, 1), i32(0, 1, 2), i32(20, 33)
+    scale = 128 ** -0.5
+
+    def slabs(with_pos=False):
+        s = KvSlabs(B, 48, hkv, 128, with_pos=with_pos, device="cpu")
+        gs = torch.Generator().manual_seed(5)
+        s.k.copy_(torch.randn(s.k.shape, generator=gs).to(torch.bfloat16))
+        s.v.copy_(torch.randn(s.v.shape, generator=gs).to(torch.bfloat16))
+        s.len.copy_(pos)
+        if with_pos:
+            s.pos.copy_(torch.arange(48, dtype=torch.int32))
+        return s
+
+    def segment(s):
+        if s is None:
+            return _capi.KvSegment(nslots=B)
+        ptr = lambda t: None if t is None else t.data_ptr()
+        return _capi.KvSegment(ptr(s.k), ptr(s.v), ptr(s.pos), ptr(s.start), ptr(s.len), s.k.stride(2), s.k.stride(1), s.v.stride(2), s.v.stride(1),
+                               s.capacity, B)
+
+    def step(lib, c1, c2, cache, q_slot, q_depth, append_at, append_depth=None, pos_new=None):
+        o = torch.zeros(B, hq, 128, dtype=torch.bfloat16)
+        prep = _capi.QkPrepArgs(q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), q_weight=qw.data_ptr(), k_weight=kw.data_ptr(), cos=cos.data_ptr(),
+                                sin=sin.data_ptr(), cos_sin_row_stride=128, eps=1e-6, rows=B, hq=hq, hkv=hkv, d=128, append=1, nseq=B,
+                                append_one_row_per_seq=1, cu_new=cu.data_ptr(), slot_of=q_slot.data_ptr(), cache=segment(cache),
+                                overflow=cache.overflow.data_ptr(), pos_new=None if pos_new is None else pos_new.data_ptr())
+        for name in ("q", "k", "v"):
+            setattr(prep, f"{name}_row_stride", (hq if name == "q" else hkv) * 128)
+            setattr(prep, f"{name}_head_stride", 128)
+        dec = _capi.DuoDecodeArgs(o=o.data_ptr(), o_row_stride=hq * 128, o_head_stride=128, q_slot=rows.data_ptr(), q_pos=pos.data_ptr(),
+                                  q_depth=q_depth.data_ptr(), c1=segment(c1), c2=segment(c2), nq=B, hq=hq, hkv=hkv, d=128, scale=scale)
+        assert lib.tah_duo_decode_step(C.byref(prep), C.byref(dec), append_at.data_ptr(), None if append_depth is None else append_depth.data_ptr(), None) == 0
+        return o
+
+    with emu_util.emulated() as lib:
+        def whole(c1, q_slot):
+            return kv_cache.decode_step(q, k, v, qw, kw, cos, sin, 1e-6, cache=c1, cu_new=cu, append_at=c1.len.clone(), q_slot=rows, q_pos=pos, c1=c1,
+                                        c2=None, scale=scale, slot_of=q_slot)
+        a, b = slabs(), slabs()
+        want = whole(a, rows)
+        assert torch.equal(step(lib, b, None, b, rows, i32(0, 0), pos.clone()), want)
+        assert torch.equal(a.k, b.k) and torch.equal(a.len, b.len) and int(b.overflow) == 0
+        # row 0 appends to the depth-1 segment: no room, so it attends over what is cached
+        a, b = slabs(), slabs()
+        want = whole(a, i32(-1, 1))
+        assert torch.equal(step(lib, b, None, b, rows, i32(1, 0), i32(0, 33), i32(1, 0)), want)
+        assert torch.equal(a.k, b.k) and torch.equal(a.len, b.len) and int(b.overflow) == 1
+        # no depth-0 rows: what the call gives over a depth-0 segment without any
+        a, b, none = slabs(True), slabs(True), slabs()
+        none.len.zero_()
+        want = step(lib, none, a, a, rows, i32(1, 1), pos.clone(), pos_new=pos)
+        assert torch.equal(step(lib, None, b, b, rows, i32(1, 1), pos.clone(), pos_new=pos), want)
+        assert torch.equal(a.k, b.k) and torch.equal(a.len, b.len)
