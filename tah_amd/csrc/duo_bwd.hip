@@ -371,7 +371,7 @@ __global__ __launch_bounds__(kKvThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dkd
 
     int seq = 0, key0 = 0, key_end = 0;
     bool second = false;
-    const CallBounds cb = call_bounds(p);
+    const CallBounds cb = call_bounds(p, p.s2.total_q > 0 || p.s2.total_k > 0);
     int slot = (int)blockIdx.y;  // without a table: early (heavy) key tiles of each sequence first
     // (the table's order: the key tile seen by the most query rows first)
     sched_lookup(p.sched, true, p.nseq, G, p.s1.total_q, p.s2.total_q, p.s1.total_k, p.s2.total_k, (int)gridDim.y,
@@ -816,7 +816,7 @@ __global__ __launch_bounds__(kLqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
 
     int seq = 0, row0 = 0, row_end = 0;
     bool second = false;
-    const CallBounds cb = call_bounds(p);
+    const CallBounds cb = call_bounds(p, p.s2.total_q > 0);
     int slot = (int)(gridDim.y - 1 - blockIdx.y);  // without a table: late (heavy) tiles of each sequence first
     // (the table's order: heaviest tile of the whole call first)
     sched_lookup(p.sched, false, p.nseq, G, p.s1.total_q, p.s2.total_q, p.s1.total_k, p.s2.total_k, (int)gridDim.y,

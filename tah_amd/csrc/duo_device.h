@@ -441,13 +441,13 @@ __device__ __forceinline__ bool find_tile(const int32_t* cu, int nseq, int bm, i
 
 // The first 64 sequences' boundaries in both streams of a varlen call, asked for at once (a stream without queries or keys may
 // come without them): a workgroup's start is a chain of trips to memory, and which tile it is, where its sequence's keys lie and
-// how many there are then follow from one of them.
+// how many there are then follow from one of them.  k2: whether the caller looks at the depth-1 keys' boundaries.
 struct CallBounds {
     LaneBounds q1, k1, q2, k2;
 };
 template <class P>
-__device__ __forceinline__ CallBounds call_bounds(const P& p) {
-    const bool q2 = p.s2.total_q > 0, k2 = q2 || p.s2.total_k > 0;
+__device__ __forceinline__ CallBounds call_bounds(const P& p, bool k2) {
+    const bool q2 = p.s2.total_q > 0;
     CallBounds x;
     x.q1 = lane_bounds(p.s1.total_q > 0 ? p.s1.cu_q : p.s1.cu_k, 0, p.nseq);
     x.k1 = lane_bounds(p.s1.cu_k, 0, p.nseq);

@@ -120,7 +120,7 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     // ---- which tile am I ---------------------------------------------------
     // (all boundaries in one trip, together with the table, and scalar arithmetic on them: 333 rows, where the last workgroup's start was
     // 2.7 of 16 us, 16.95 -> 16.1 us; 4 x 4096 rows, 3.8 us a workgroup, 316 -> 312; 8192 forward and backward 1231 -> 1222)
-    const CallBounds cb = call_bounds(p);
+    const CallBounds cb = call_bounds(p, p.s2.total_q > 0);  // (keys of a depth without queries may come without boundaries)
     const bool has1 = p.s1.total_q > 0, has2 = p.s2.total_q > 0;
     int seq = 0, row0 = 0, row_end = 0;
     bool second = false;

@@ -167,3 +167,23 @@ def test_two_waves_to_the_same_rows_give_the_bits_of_one(lens, p):
             o1, lse1, o2, lse2 = ops.duo_fwd_varlen(*varlen_args(part))
             assert torch.equal(o1, want[0][:, h:h + n]) and torch.equal(lse1, want[1][h:h + n])
             assert torch.equal(o2, want[2][:, h:h + n]) and torch.equal(lse2, want[3][h:h + n])
+
+
+def test_fwd_of_depth0_queries_beside_depth1_keys_without_boundaries():
+    """Depth-1 keys that no query looks at, described by their number alone: the outputs of the call without them."""
+    import ctypes as C
+
+    from tah_amd import _capi, ops
+    dev = _to_dev(make_varlen_case(73, [40], 0.0, Hq=2, Hkv=1, D=128))
+    with emu_util.emulated() as lib:
+        want = ops.duo_fwd_varlen(*varlen_args(dev))
+        o, lse = torch.zeros_like(want[0]), torch.zeros_like(want[1])
+        q, k, v = dev["q1"], dev["k1"], dev["v1"]
+        s1 = _capi.DuoStream(q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), o=o.data_ptr(), lse=lse.data_ptr(), cu_q=dev["cu_q1"].data_ptr(),
+                             cu_k=dev["cu_k1"].data_ptr(), total_q=q.shape[0], total_k=k.shape[0])
+        for name, t in (("q", q), ("k", k), ("v", v), ("o", o)):
+            setattr(s1, f"{name}_row_stride", t.stride(0))
+            setattr(s1, f"{name}_head_stride", t.stride(1))
+        a = _capi.DuoFwdArgs(s1=s1, s2=_capi.DuoStream(total_k=7), nseq=1, hq=2, hkv=1, d=128, scale=dev["scale"])
+        assert lib.tah_duo_fwd_varlen(C.byref(a), None) == 0
+    assert torch.equal(o, want[0]) and torch.equal(lse, want[1])
