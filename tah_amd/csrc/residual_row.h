@@ -1,6 +1,6 @@
 // A row of the residual stream on its way past a norm: the sum with a sublayer's normed result and the norm and short convolution in
 // front of the next sublayer.  Shared by residual_norm_kernel (row_norm.hip), which writes what the next launch reads, and by
-// kernels whose workgroups each make a row's operand for themselves (linear_rows.hip, moe.hip).
+// norm_linear_kernel (linear_rows.hip), whose workgroups each make the rows' operand for themselves.
 #pragma once
 #include "mixer_device.h"
 
@@ -58,6 +58,15 @@ __device__ __forceinline__ void group_sums(float (&s)[U], int tid, int units, in
             s[u] = lds.group_sum[g < groups ? g : groups - 1];  // (columns behind the last group hold zeros)
         }
     }
+}
+
+// Sum of the squares of a unit's columns.  The roundings are written out: left to the compiler, one kernel fused the first square
+// into the sum and another the second, the last bit of a norm hung on that, and two kernels that must agree did not have to.
+__device__ __forceinline__ float sum_of_squares(const float (&v)[8]) {
+    float s = fmaf(v[0], v[0], v[1] * v[1]);
+#pragma unroll
+    for (int i = 2; i < 8; ++i) s = fmaf(v[i], v[i], s);
+    return s;
 }
 
 // What tah_residual_norm does with one row, by kRowThreads threads.  U: units of eight columns per thread.  kEarly: a few rows are a
@@ -157,11 +166,7 @@ __device__ __forceinline__ void residual_row(const tah_residual_norm_args& p, in
     }
     if (add) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            s[u] = 0.f;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) s[u] += y[u][i] * y[u][i];
-        }
+        for (int u = 0; u < U; ++u) s[u] = sum_of_squares(y[u]);
         group_sums<U, GROUPS>(s, tid, units, p.groups, group_units, lds);
     }
 #pragma unroll
@@ -178,8 +183,7 @@ __device__ __forceinline__ void residual_row(const tah_residual_norm_args& p, in
             } else if (write && x_out != p.x) {
                 store8(x_out + (int64_t)row * p.cols + c, x[u]);
             }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) sx += x[u][i] * x[u][i];
+            sx = sum_of_squares(x[u]);
             if (write && p.xe) store8(static_cast<E*>(p.xe) + (int64_t)row * p.cols + c, x[u]);
             if (write && p.x_packed) static_cast<bf16x8*>(p.x_packed)[rows_form_unit(row, c)] = to_bf16x8(x[u]);
             if (!p.next_coef) emit(c, x[u]);

@@ -276,3 +276,24 @@ def test_shared_expert_among_the_experts_on_cpu_shim(case):
 @pytest.mark.parametrize("case", SHARED_AMONG + [(8, 2048, 768, 64, 8, 768), (1, 2048, 768, 64, 8, 768), (32, 2048, 768, 16, 8, 768)])
 def test_shared_expert_among_the_experts_gpu(case):
     Z.moe_case("cuda", Z.BF, *case)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("cols,width,groups", [(2048, 2048, 1), (2048, 2048, 8), (2048, 2040, 5), (4096, 4096, 8), (8192, 8192, 8), (16384, 16384, 1)])
+def test_a_rows_norm_does_not_depend_on_how_many_rows_the_call_has_gpu(dtype, cols, width, groups):
+    """Calls of up to 256 rows ask for everything at once, others do not: two kernels, the same bits of a row.  (The residual rows
+    in float32: they show the last bit of the norm in front of the sum, and so does the float32 result of the one behind it.)"""
+    from tah_amd.ops import _call
+    g = torch.Generator().manual_seed(cols + groups)
+    r = lambda *s: torch.nn.functional.pad(torch.randn(*s, width, generator=g), (0, cols - width)).cuda()
+    x, y, coef, norm = r(300), r(300).to(dtype), r(), r()
+
+    def run(rows):
+        out, normed = x[:rows].clone(), torch.zeros(rows, cols, dtype=dtype, device="cuda")
+        _call("residual_norm", out, coef, width, 1e-5, y[:rows], None, None, None, None, None, None, norm, normed, None, 1, 0, groups,
+              width // groups if groups > 1 else cols, None, None, None)
+        return out, normed
+
+    (a, na), (b, nb) = run(300), run(64)
+    assert torch.equal(a[:64], b) and torch.equal(na[:64], nb)
