@@ -87,7 +87,8 @@ typedef struct tah_residual_norm_args {
 int tah_residual_norm(const tah_residual_norm_args* args, tah_stream_t stream);
 /* tah_residual_norm and, on the operand that comes out of it (the normed row, or without next_coef the new residual row), tah_linear_rows
  * in one launch, for a few rows of tah_norm_linear_supported() sizes, bf16: the bits of the two calls.  The new residual rows go to
- * x_out [rows, cols], which like `linear`'s results lies on nothing that either reads; norm->xe, x_packed, normed and
+ * x_out [rows, cols], which like `linear`'s results lies on nothing that either reads (TAH_E_SHAPE where it does; on the experts' rows, whose
+ * extent the call does not know, the caller sees to it); norm->xe, x_packed, normed and
  * normed_packed are NULL.  linear: a plain layer (TAH_LINEAR_PLAIN) without residual, bias, norm or batch, with no activation,
  * TAH_ACT_GELU_TANH or TAH_ACT_XIELU; its x_packed is not read.  Rows of one call belong to different slots. */
 int tah_norm_linear_supported(int32_t rows, int32_t cols, int32_t n);

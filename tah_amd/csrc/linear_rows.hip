@@ -1393,8 +1393,13 @@ extern "C" int tah_norm_linear(const tah_residual_norm_args* norm, float* x_out,
     const auto of = [](const void* q, int64_t bytes) { return Range{static_cast<const char*>(q), q ? bytes : 0}; };
     const int64_t last = norm->rows - 1;
     const Range written[] = {of(x_out, 4ll * norm->rows * norm->cols), of(a->out, 2 * (last * a->out_row_stride + a->n)), of(a->out_packed, 64ll * a->n)};
+    // (how far the experts' rows reach only their indices say)
+    const int64_t choices = norm->experts ? 4ll * norm->rows * norm->top : 0, per_row = norm->conv ? 4ll * norm->rows : 0;
+    const int64_t taps = norm->conv ? (int64_t)norm->taps * norm->cols : 0;
     const Range read[] = {of(norm->x, 4ll * norm->rows * norm->cols), of(norm->y, 2 * (last * norm->y_row_stride + norm->cols)),
-                          of(norm->coef, 4ll * norm->cols), of(norm->next_coef, 4ll * norm->cols), of(a->w_packed, 2ll * a->n * a->k)};
+                          of(norm->coef, 4ll * norm->cols), of(norm->next_coef, 4ll * norm->cols), of(a->w_packed, 2ll * a->n * a->k),
+                          of(norm->y_scale, 4ll * norm->rows), of(norm->index, choices), of(norm->weight, choices), of(norm->slot, per_row),
+                          of(norm->pos, per_row), of(norm->conv, 4 * taps), of(norm->conv_state, 2 * taps * norm->nslots)};
     const auto meet = [](const Range& x, const Range& y) { return x.bytes > 0 && y.bytes > 0 && x.at < y.at + y.bytes && y.at < x.at + x.bytes; };
     for (const Range& w : written)
         for (const Range& r : read)

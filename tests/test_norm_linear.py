@@ -87,6 +87,33 @@ def test_norm_linear_refuses_results_on_operands_on_cpu_shim():
             st.linear(Linear(torch.zeros(32, COLS, dtype=torch.bfloat16)))
 
 
+@needs_clang
+def test_norm_linear_refuses_results_on_what_a_row_comes_with_on_cpu_shim():
+    """The factor, the experts' choice, slot, position, convolution and its inputs: in the residual rows' place and in the layer's result's."""
+    import ctypes as C
+
+    from tah_amd import _capi
+    TAPS, SLOTS, N = 3, 2, 32
+    mem = torch.zeros(4 << 20, dtype=torch.uint8)
+    at = lambda k: mem.data_ptr() + (k << 18)   # places a quarter of a megabyte apart
+    names = ["x", "y", "y_scale", "experts", "index", "weight", "coef", "next_coef", "conv", "conv_state", "slot", "pos"]
+    place = {name: at(i) for i, name in enumerate(names)}
+    ends = {"y_scale": 4, "index": 8, "weight": 8, "slot": 4, "pos": 4, "conv": 4 * TAPS * COLS, "conv_state": 2 * SLOTS * TAPS * COLS, "coef": 4 * COLS}
+    with emu_util.emulated() as lib:
+        def call(x_out, out):
+            n = _capi.ResidualNormArgs(**place, y_row_stride=COLS, experts_row_stride=COLS, rows=1, width=COLS, cols=COLS, top=2, index_scale=1, eps=1e-5,
+                                       groups=1, group_cols=COLS, taps=TAPS, nslots=SLOTS, dtype=0)
+            a = _capi.LinearRowsArgs(w_packed=at(12), out=out, out_row_stride=N, rows=1, n=N, k=COLS)
+            return lib.tah_norm_linear(C.byref(n), x_out, C.byref(a), None)
+
+        assert call(at(13), at(14)) == 0
+        for name, size in ends.items():
+            for offset in {0, (size - 1) // 16 * 16}:  # (results are 16-byte aligned)
+                assert call(place[name] + offset, at(14)) == _capi.TAH_E_SHAPE, name
+                assert call(at(13), place[name] + offset) == _capi.TAH_E_SHAPE, name
+        assert int(mem[14 << 18:].sum()) == 0
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", CASES)
 def test_norm_and_linear_layer_in_one_launch_gpu(case):
