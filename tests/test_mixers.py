@@ -279,6 +279,34 @@ def test_shared_expert_among_the_experts_gpu(case):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,width,ff,experts,top", [(1, 64, 32, 8, 2), (1, 2048, 768, 64, 8), (8, 2048, 768, 64, 8), (17, 2048, 768, 16, 8), (32, 256, 96, 16, 8)])
+def test_shared_expert_among_the_experts_has_the_bits_of_launches_of_its_own_gpu(rows, width, ff, experts, top):
+    from tah_amd import ops
+    from tah_amd.mixers import GatedMlp, MoeMlp, PackedBatch, Router, Step
+
+    class Engine:
+        packed, device = True, torch.device("cuda")
+    g = torch.Generator().manual_seed(rows + width)
+    w = lambda *s: (torch.randn(*s, generator=g) * s[-1] ** -0.5).to(torch.bfloat16).cuda()
+    routed = {"router": 3 * w(experts, width), "gate": w(experts, ff, width), "up": w(experts, ff, width), "down": w(experts, width, ff)}
+    shared = {"gate": w(ff, width), "up": w(ff, width), "down": w(width, ff), "sg": 2 * w(1, width)}
+    x = torch.randn(rows, width, generator=g).to(torch.bfloat16).cuda()
+    zeros = torch.zeros(rows, dtype=torch.int32, device="cuda")
+    step = lambda: Step(x.float(), x, zeros, ops.linear_pack_rows(x), slot=zeros)
+    m = MoeMlp(Router(top), routed, shared, width)
+    assert m.shared_among
+    got = m.bind(Engine).rows(step())
+    # the same weights, the shared expert in two launches beside the experts'
+    m.shared_among, m.shared = False, GatedMlp(shared, width)
+    m.gate_up_rows, m.down_rows = PackedBatch(m.gate_up, gate_up=True), PackedBatch(m.down)
+    want = m.bind(Engine).rows(step())
+    assert torch.equal(got.y, want.y) and torch.equal(got.index, want.index) and torch.equal(got.weight, want.weight) and torch.equal(got.y_scale, want.y_scale)
+    assert got.index_scale == want.index_scale and got.index_row == want.index_row
+    at = (want.index.long() * want.index_scale + torch.arange(rows, device="cuda")[:, None] * want.index_row).flatten()
+    assert torch.equal(got.experts[at], want.experts[at])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("cols,width,groups", [(2048, 2048, 1), (2048, 2048, 8), (2048, 2040, 5), (4096, 4096, 8), (8192, 8192, 8), (16384, 16384, 1)])
 def test_a_rows_norm_does_not_depend_on_how_many_rows_the_call_has_gpu(dtype, cols, width, groups):

@@ -20,6 +20,9 @@ CASES = [
     (1, 8192, (16, 2048), 8, (4, [0]), True, True, True, {}),
     (1, 12352, (1, 2048), 0, None, True, False, False, {}),
 ]
+# neither experts nor convolution: wide layers and narrow ones, groups and none
+CASES += [(rows, n, groups, 0, None, True, False, normed, act) for rows in (1, 2) for n, act in ((6144, {"xielu": (0.7, 1.1)}), (2048, {}))
+          for groups, normed in (((8, 2048), True), ((1, 2048), False))]
 
 
 def norm_linear_case(dev, rows, n, geometry, top, conv, with_y, scaled, normed, act, seed=3):
@@ -68,7 +71,7 @@ def norm_linear_case(dev, rows, n, geometry, top, conv, with_y, scaled, normed, 
 
 
 @needs_clang
-@pytest.mark.parametrize("case", [0, 6])
+@pytest.mark.parametrize("case", [0, 6, 10])
 def test_norm_and_linear_layer_in_one_launch_on_cpu_shim(case):
     rows, n, *rest = CASES[case]
     with emu_util.emulated():
