@@ -1045,7 +1045,7 @@ __global__ __launch_bounds__(kChainThreads) void linear_chain_kernel(const Chain
 // 334.9 and 369.1 -> 361.9.  Three and four rows: the rows' bytes cost more than the launch (350.5 -> 359.3, 369.6 -> 378.4).  More than two
 // workgroups to a compute unit: the rows are made three times over (2048 -> 12352, one row: a step 334.9 -> 344.2).
 constexpr int kNormLinearRows = 2, kNormLinearWorkgroups = 512;
-constexpr int kNormLinearSteps = 8;  // K = 256 kNormLinearSteps = a thread's eight columns for 256 threads
+constexpr int kNormLinearSteps = 8;  // K = 256 kNormLinearSteps = a thread's eight columns for 256 threads (no other width is built or measured)
 struct NormLinear {
     tah_residual_norm_args n;
     float* x_out;
