@@ -9,7 +9,9 @@
  *
  * Layout.  Tokens are packed ("varlen"): sequence b owns rows
  * [cu[b], cu[b+1]) of a [rows, heads, D] bf16 tensor whose innermost D elements
- * are contiguous; row and head strides are given in elements.  Only valid tokens
+ * are contiguous; row and head strides are given in elements.  (Boundaries given as
+ * pairs, `cu_pairs`: rows [cu[2b], cu[2b+1]), ascending, with rows in between that belong
+ * to no sequence and are neither read nor written -- padded batches where they lie.)  Only valid tokens
  * are packed, so within a sequence the depth-0 ("iteration 1") key at local
  * index j has position j, and a depth-0 query at local index i has position
  * i + (Lk1 - Lq1) (queries are the newest rows of the sequence).  Depth-1
@@ -39,7 +41,7 @@
 extern "C" {
 #endif
 
-#define TAH_DUO_ABI_VERSION 11
+#define TAH_DUO_ABI_VERSION 12
 
 enum {
     TAH_OK = 0,
@@ -76,6 +78,7 @@ typedef struct tah_duo_fwd_args {
     tah_duo_stream s2;      /* depth 1: hard tokens; total_q may be 0 */
     int32_t nseq, hq, hkv, d;
     float scale;            /* softmax scale, head_dim**-0.5 in Qwen3 */
+    int32_t cu_pairs;       /* 0, or the sum of 1, 2, 4, 8 for s1.cu_q, s1.cu_k, s2.cu_q, s2.cu_k that hold pairs */
     const void* schedule;   /* launch-order table from tah_duo_schedule_build for these boundaries, or NULL */
 } tah_duo_fwd_args;
 
@@ -116,6 +119,7 @@ typedef struct tah_duo_schedule_args {
     const int32_t* pos_q2;  /* int32 [total_q2] positions of the depth-1 query rows */
     int32_t nseq, hq, hkv;  /* nseq <= 4095 */
     int32_t total_q1, total_k1, total_q2, total_k2;
+    int32_t cu_pairs;       /* as in tah_duo_fwd_args */
     void* schedule;         /* >= tah_duo_schedule_bytes(...) bytes, 4-byte aligned */
     size_t schedule_bytes;
 } tah_duo_schedule_args;
@@ -700,6 +704,45 @@ int tah_pad_rows_build(const int32_t* cu, const int32_t* seq_of, int32_t n, cons
 int tah_rows_copy(const void* src, const int32_t* src_rows, void* dst, const int32_t* dst_rows,
                   const uint8_t* dst_enable, int32_t n, const int32_t* n_dev, int64_t row_bytes,
                   int64_t src_stride_bytes, int64_t dst_stride_bytes, tah_stream_t stream);
+
+/* tah_hard_index_build with, from the same launch, where an entry went and where a row's entries lie (either may be NULL):
+ * rank[b*S + s] = the entry's number or -1, and spans = B pairs (flat index of the row's first True entry, that plus their
+ * number), then 1 if the True entries of some row do not lie together, else 0.  pos, flat, seq may be NULL (flat not with spans). */
+typedef struct tah_mask_index_args {
+    const uint8_t* mask;
+    int32_t B, S;
+    int32_t *pos, *flat, *seq, *cu;
+    int32_t* rank;   /* [B*S] */
+    int32_t* spans;  /* [2*B + 1] */
+} tah_mask_index_args;
+int tah_mask_index_build(const tah_mask_index_args* args, tah_stream_t stream);
+
+/* The right-padded (B, width) form of a mask's entries (tah/model/tah_model.py:117-134) as tables: left[b*width + j] = flat
+ * index of row b's j-th entry, back[f] = b*width + j for that entry, both -1 where there is none, pad = 1 where left is -1. */
+int tah_left_index_build(const int32_t* cu, const int32_t* flat, const int32_t* rank, int32_t B, int32_t S, int32_t width,
+                         int32_t* left, int32_t* back, uint8_t* pad, tah_stream_t stream);
+
+/* Rows of several tensors by one table: dst[r] = src[index[r]] for r < rows (and r < *n_dev when given), zeros where
+ * index[r] < 0.  dst rows lie one behind the other.  Bit-exact. */
+#define TAH_SELECT_TENSORS 6
+typedef struct tah_select_rows {
+    const void* src;
+    void* dst;
+    int64_t row_bytes, src_stride_bytes;
+} tah_select_rows;
+int tah_rows_select(const tah_select_rows* tensors, int32_t n, const int32_t* index, int32_t rows, const int32_t* n_dev,
+                    tah_stream_t stream);
+
+/* Sets the rows between sequences to zero: of every tensor those that lie in no [pairs[2b], pairs[2b+1]), b < nseq (ascending).
+ * Rows are contiguous, row_bytes a multiple of 16. */
+#define TAH_GAP_TENSORS 6
+typedef struct tah_gap_rows {
+    void* rows;
+    const int32_t* pairs;  /* int32 [2 * nseq] */
+    int64_t row_bytes;
+    int32_t total;         /* rows */
+} tah_gap_rows;
+int tah_zero_gaps(const tah_gap_rows* tensors, int32_t n, int32_t nseq, tah_stream_t stream);
 
 #ifdef __cplusplus
 }

@@ -8,7 +8,7 @@ from __future__ import annotations
 
 import ctypes as C
 
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 c_void_p, c_int32, c_int64, c_float = C.c_void_p, C.c_int32, C.c_int64, C.c_float
 
@@ -38,7 +38,7 @@ class DuoFwdArgs(C.Structure):
     _fields_ = [
         ("s1", DuoStream), ("s2", DuoStream),
         ("nseq", c_int32), ("hq", c_int32), ("hkv", c_int32), ("d", c_int32),
-        ("scale", c_float),
+        ("scale", c_float), ("cu_pairs", c_int32),
         ("schedule", c_void_p),
     ]
 
@@ -50,6 +50,7 @@ class DuoScheduleArgs(C.Structure):
         ("cu_q1", c_void_p), ("cu_k1", c_void_p), ("cu_q2", c_void_p), ("cu_k2", c_void_p), ("pos_q2", c_void_p),
         ("nseq", c_int32), ("hq", c_int32), ("hkv", c_int32),
         ("total_q1", c_int32), ("total_k1", c_int32), ("total_q2", c_int32), ("total_k2", c_int32),
+        ("cu_pairs", c_int32),
         ("schedule", c_void_p), ("schedule_bytes", C.c_size_t),
     ]
 
@@ -382,6 +383,10 @@ PROTOTYPES = {
     "tah_silu_mul": (C.c_int, [c_void_p, c_void_p, c_int32, c_int32, c_int64, c_int64, c_void_p]),
     "tah_hard_index_build": (C.c_int, [c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "tah_pad_rows_build": (C.c_int, [c_void_p, c_void_p, c_int32, c_void_p, c_int32, c_void_p, c_void_p, c_void_p]),
+    "tah_mask_index_build": (C.c_int, [c_void_p, c_void_p]),
+    "tah_left_index_build": (C.c_int, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "tah_rows_select": (C.c_int, [c_void_p, c_int32, c_void_p, c_int32, c_void_p, c_void_p]),
+    "tah_zero_gaps": (C.c_int, [c_void_p, c_int32, c_int32, c_void_p]),
     "tah_rows_copy": (C.c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_int64, c_int64,
                                 c_int64, c_void_p]),
     # include/tah_mixers.h

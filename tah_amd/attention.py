@@ -22,6 +22,7 @@ not valid get zeros.
 """
 from __future__ import annotations
 
+import types
 from typing import Optional, Tuple
 
 import torch
@@ -35,12 +36,13 @@ from .pack import HardIndex
 class _DuoAttnVarlen(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q1, k1, v1, q2, k2, v2, cu_q1, cu_k1, pos_q2, pos_k2, cu_q2, cu_k2, scale, schedule=None,
-                max_seqlen_k1=0, max_seqlen_k2=0):
+                max_seqlen_k1=0, max_seqlen_k2=0, pairs=0):
         o1, lse1, o2, lse2 = ops.duo_fwd_varlen(q1, k1, v1, cu_q1, cu_k1, q2, k2, v2, pos_q2, pos_k2, cu_q2, cu_k2, scale,
-                                                schedule)
+                                                schedule, pairs)
         ctx.save_for_backward(q1, k1, v1, o1, lse1, q2, k2, v2, o2, lse2, cu_q1, cu_k1, pos_q2, pos_k2, cu_q2, cu_k2)
         ctx.scale = scale
         ctx.schedule = schedule
+        ctx.pairs = pairs
         ctx.max_k = (int(max_seqlen_k1), int(max_seqlen_k2))
         ctx.mark_non_differentiable(lse1, lse2)
         return o1, o2, lse1, lse2
@@ -48,15 +50,16 @@ class _DuoAttnVarlen(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do1, do2, _dl1, _dl2):
         q1, k1, v1, o1, lse1, q2, k2, v2, o2, lse2, cu_q1, cu_k1, pos_q2, pos_k2, cu_q2, cu_k2 = ctx.saved_tensors
-        c = lambda g, like: (torch.zeros_like(like) if g is None else g.contiguous())
+        c = lambda g, like: (torch.zeros_like(like) if g is None else _readable(g.contiguous()))
         dq1, dk1, dv1, dq2, dk2, dv2 = ops.duo_bwd_varlen(
             q1, k1, v1, o1, lse1, c(do1, o1), cu_q1, cu_k1, q2, k2, v2, o2, lse2, c(do2, o2),
-            pos_q2, pos_k2, cu_q2, cu_k2, ctx.scale, ctx.schedule, max_seqlen_k1=ctx.max_k[0], max_seqlen_k2=ctx.max_k[1])
-        return dq1, dk1, dv1, dq2, dk2, dv2, None, None, None, None, None, None, None, None, None, None
+            pos_q2, pos_k2, cu_q2, cu_k2, ctx.scale, ctx.schedule, max_seqlen_k1=ctx.max_k[0], max_seqlen_k2=ctx.max_k[1],
+            pairs=ctx.pairs)
+        return (dq1, dk1, dv1, dq2, dk2, dv2) + (None,) * 11
 
 
 def duo_attn_varlen(q1, k1, v1, cu_q1, cu_k1, q2, k2, v2, pos_q2, pos_k2, cu_q2, cu_k2, scale: float,
-                    return_lse: bool = False, schedule=None, max_seqlen_k1: int = 0, max_seqlen_k2: int = 0):
+                    return_lse: bool = False, schedule=None, max_seqlen_k1: int = 0, max_seqlen_k2: int = 0, pairs: int = 0):
     """Duo-causal attention on packed varlen bf16 tensors, differentiable.
 
     Depth-0 stream: q1 [T1q,Hq,D], k1/v1 [T1k,Hkv,D], cu_q1/cu_k1 int32 [nseq+1].
@@ -66,10 +69,11 @@ def duo_attn_varlen(q1, k1, v1, cu_q1, cu_k1, q2, k2, v2, pos_q2, pos_k2, cu_q2,
     :func:`tah_amd.ops.duo_schedule` built for these boundaries (forward and backward use it), or None.
     ``max_seqlen_k1`` / ``max_seqlen_k2``: upper bounds on one sequence's key rows per depth (0: unknown); they only
     make the backward pass's dS workspace smaller (:func:`tah_amd.ops.duo_bwd_varlen`).
+    ``pairs``: which boundaries are (first row, one past the last) pairs (:func:`tah_amd.ops.duo_fwd_varlen`).
     Returns (o1, o2).
     """
     o1, o2, lse1, lse2 = _DuoAttnVarlen.apply(q1, k1, v1, q2, k2, v2, cu_q1, cu_k1, pos_q2, pos_k2, cu_q2, cu_k2,
-                                              float(scale), schedule, max_seqlen_k1, max_seqlen_k2)
+                                              float(scale), schedule, max_seqlen_k1, max_seqlen_k2, int(pairs))
     return (o1, o2, lse1, lse2) if return_lse else (o1, o2)
 
 
@@ -111,6 +115,7 @@ class DuoMask:
         self.position_ids, self.valid_mask, self.cache, self.iter_depth = position_ids, valid_mask, cache, iter_depth
         self._packed = None  # per-step packing metadata, shared by all decoder layers
         self._sched = None   # launch-order table of the step's varlen calls, likewise
+        self._empty = None   # boundaries and positions of no rows
         self._merge = None   # where the rows of depths 1 .. iter_depth go in their common packing (depth >= 2)
 
     def dense(self, dtype: torch.dtype = torch.float32) -> Optional[torch.Tensor]:
@@ -202,6 +207,12 @@ def _rows(x: torch.Tensor) -> torch.Tensor:
     return x.transpose(1, 2).reshape(B * T, H, D)
 
 
+def _readable(r: torch.Tensor) -> torch.Tensor:
+    """[n, H, D] rows as the kernels take them where they lie: itself, or a copy if its strides or its address are not theirs."""
+    fits = r.stride(2) == 1 and r.stride(0) % 8 == 0 and r.stride(1) % 8 == 0 and 0 <= r.stride(0) < 1 << 23 and r.data_ptr() % 16 == 0
+    return r if fits or r.numel() == 0 else r.clone(memory_format=torch.contiguous_format)
+
+
 # Blocks of at most this many rows are packed without reading their valid count back (see _Packed).
 NO_SYNC_ROWS = 4096
 
@@ -209,18 +220,27 @@ NO_SYNC_ROWS = 4096
 class _Packed:
     """Valid-row packing of one (B, T) block: row ids, per-sequence offsets, int32 positions.
 
+    A padded block (every sequence's valid rows lie together, depth 0: no positions) is not moved at all: the kernels take its rows where
+    they lie, ``cu`` then holds (first row, one past the last) pairs, ``paired``.  Its pad rows come out as zeros, as from a scatter, and
+    what they hold is not read.  Two layers of four sequences of 1024 to 3210 rows, forward and backward: 2.62 -> 2.05 ms with
+    :class:`_BlockAttn` (row moves, clears and the gradients of empty slices were 0.5 of it, and the host's 105 launches behind the hard
+    tokens' read-back the rest).  Blocks that are mostly padding are packed: the dS
+    workspace of the backward grows with the rows a block has, and its pad rows are cleared in every result.
+
     With ``tah_amd.pack.HOST_SYNC`` off nothing is read back from the device: packed tensors keep the full
-    B*T rows (zero beyond the valid count, so that a key tile never mixes in uninitialised rows), the kernels
-    find the real extent in ``cu``, and the row copies stop at the count held on the device."""
+    B*T rows, the kernels find the real extent in ``cu`` (and read no row behind it: those are undefined), and the row copies
+    stop at the count held on the device."""
 
     def __init__(self, valid: Optional[torch.Tensor], pos: Optional[torch.Tensor], B: int, T: int, device):
         self.B, self.T = B, T
+        self.valid, self.given_pos = valid, pos
         self.n_dev = None
         if valid is not None and tuple(valid.shape) != (B, T):
             raise TahDuoError(f"valid mask of shape {tuple(valid.shape)} for a block of {B} x {T} rows")
         if pos is not None and pos.numel() != B * T:
             raise TahDuoError(f"positions of shape {tuple(pos.shape)} for a block of {B} x {T} rows")
         all_valid = valid is None
+        self.paired = False
         if not all_valid:
             # a small block (the packed hard tokens of a step) is packed by its upper bound, B * T rows: reading the count
             # back would stall the host on everything queued so far to save copying a few pad rows
@@ -229,35 +249,31 @@ class _Packed:
         if all_valid:
             self.rows, self.n = None, B * T
             self.cu = torch.arange(0, (B + 1) * T, T, dtype=torch.int32, device=device)
+        elif pos is None and idx.intervals is not None and 2 * idx.n >= B * T:
+            self.rows, self.n, self.cu, self.paired = None, B * T, idx.intervals, True
         else:
-            self.rows, self.n, self.cu, self.n_dev = idx.flat, idx.bound, idx.cu, idx.n_dev
+            self.rows, self.n, self.cu, self.n_dev, self.rank = idx.flat, idx.bound, idx.cu, idx.n_dev, idx.rank
         self.pos = None
         if pos is not None:
-            p32 = pos.to(torch.int32).contiguous().view(B * T, 1)
-            if self.rows is not None:
-                out = torch.zeros((self.n, 1), dtype=torch.int32, device=device)
-                ops.rows_copy(p32, self.rows, out, None, self.n, None, self.n_dev)
-                p32 = out
-            self.pos = p32.view(-1)
+            p32 = pos.to(torch.int32).contiguous().view(B * T)
+            self.pos = p32 if self.rows is None else ops.rows_select([p32], self.rows, self.n, self.n_dev)[0]
+
+    def unmoved(self, x: torch.Tensor) -> torch.Tensor:
+        """The rows of a (B, H, T, D) block as the attention call takes them, where they lie or for it to pack."""
+        r = _rows(x)
+        return _readable(r) if self.paired else r
 
     def pack(self, x: torch.Tensor) -> torch.Tensor:
         r = _rows(x)
         if self.rows is None:
-            return r
+            return _readable(r) if self.paired else r
         return _GatherRows.apply(r.contiguous(), self.rows, self.n, self.n_dev)
-
-    def unpack(self, o: torch.Tensor, Hq: int, D: int) -> torch.Tensor:
-        """[n, Hq, D] -> (B, T, Hq, D) with zeros at rows that were not packed."""
-        if self.rows is None:
-            return o.view(self.B, self.T, Hq, D)
-        return _ScatterRows.apply(o, self.rows, self.n, self.B * self.T, self.n_dev).view(self.B, self.T, Hq, D)
 
 
 class _GatherRows(torch.autograd.Function):
     @staticmethod
     def forward(ctx, src, rows, n, n_dev=None):
-        alloc = torch.empty if n_dev is None else torch.zeros  # rows past a device-side count stay zero
-        out = alloc((n,) + tuple(src.shape[1:]), dtype=src.dtype, device=src.device)
+        out = torch.empty((n,) + tuple(src.shape[1:]), dtype=src.dtype, device=src.device)  # (rows past a device-side count: read by nobody)
         ops.rows_copy(src, rows, out, None, n, None, n_dev)
         ctx.save_for_backward(rows, n_dev)
         ctx.n, ctx.total = n, src.shape[0]
@@ -271,26 +287,59 @@ class _GatherRows(torch.autograd.Function):
         return gs, None, None, None
 
 
-class _ScatterRows(torch.autograd.Function):
+class _BlockAttn(torch.autograd.Function):
+    """Attention of one depth's (B, T) block of query rows, the rows packed and unpacked around the kernels: one launch takes the
+    query rows, and the position-carrying keys and values of the same rows, out of their blocks, one puts the output back among
+    zeros; the same for the gradients.  As autograd nodes and clears of their own around the attention, the four moves of a depth-1
+    call and their gradients were 22 launches and 0.25 ms of the host's time.  ``b``: what :func:`_attend_block` gathered.  Rows past a
+    count that stays on the device are undefined, and nobody reads them: the kernels stop at a segment's last row."""
+
     @staticmethod
-    def forward(ctx, src, rows, n, total, n_dev=None):
-        out = torch.zeros((total,) + tuple(src.shape[1:]), dtype=src.dtype, device=src.device)
-        ops.rows_copy(src.contiguous(), None, out, rows, n, None, n_dev)
-        ctx.save_for_backward(rows, n_dev)
-        ctx.n = n
-        return out
+    def forward(ctx, b, q, k1, v1, k2, v2):
+        rows = [q, k2, v2]
+        for pack, at in b.packs:
+            for i, t in zip(at, ops.rows_select([rows[i] for i in at], pack.rows, pack.n, pack.n_dev)):
+                rows[i] = t
+        qp, k2p, v2p = rows
+        none = qp.new_empty((0,) + tuple(qp.shape[1:]))
+        if b.second:
+            _, _, o, lse = ops.duo_fwd_varlen(none, k1, v1, b.none_cu, b.cu_k1, qp, k2p, v2p, b.pos_q, b.pos_k, b.cu_q, b.cu_k2, b.scale,
+                                              b.schedule, b.pairs)
+        else:
+            o, lse, _, _ = ops.duo_fwd_varlen(qp, k1, v1, b.cu_q, b.cu_k1, none, k2p, v2p, b.none_pos, b.none_pos, b.none_cu, b.none_cu, b.scale,
+                                              b.schedule, b.pairs)
+        ctx.save_for_backward(qp, k1, v1, k2p, v2p, o, lse)
+        ctx.b = b
+        out = o if b.pack_q.rows is None else ops.rows_select([o], b.pack_q.rank, b.pack_q.B * b.pack_q.T)[0]
+        return out.view(b.pack_q.B, b.pack_q.T, *out.shape[1:])
 
     @staticmethod
     def backward(ctx, g):
-        rows, n_dev = ctx.saved_tensors
-        alloc = torch.empty if n_dev is None else torch.zeros
-        gs = alloc((ctx.n,) + tuple(g.shape[1:]), dtype=g.dtype, device=g.device)
-        ops.rows_copy(g.contiguous(), rows, gs, None, ctx.n, None, n_dev)
-        return gs, None, None, None, None
+        b = ctx.b
+        qp, k1, v1, k2p, v2p, o, lse = ctx.saved_tensors
+        pack = b.pack_q
+        g = _readable(g.reshape(pack.B * pack.T, *g.shape[2:]).contiguous())
+        if pack.rows is not None:
+            g = ops.rows_select([g], pack.rows, pack.n, pack.n_dev)[0]
+        none = qp.new_empty((0,) + tuple(qp.shape[1:]))
+        no_lse = lse.new_empty((lse.shape[0], 0))
+        if b.second:
+            grads = ops.duo_bwd_varlen(none, k1, v1, none, no_lse, none, b.none_cu, b.cu_k1, qp, k2p, v2p, o, lse, g, b.pos_q, b.pos_k, b.cu_q,
+                                       b.cu_k2, b.scale, b.schedule, max_seqlen_k1=b.max_k1, max_seqlen_k2=b.max_k2, pairs=b.pairs)
+            rows = [grads[3], grads[4], grads[5]]
+        else:
+            grads = ops.duo_bwd_varlen(qp, k1, v1, o, lse, g, b.cu_q, b.cu_k1, none, k2p, v2p, none, no_lse, none, b.none_pos, b.none_pos, b.none_cu,
+                                       b.none_cu, b.scale, b.schedule, max_seqlen_k1=b.max_k1, max_seqlen_k2=b.max_k2, pairs=b.pairs)
+            rows = [grads[0], None, None]
+        for pack, at in b.packs:
+            for i, t in zip(at, ops.rows_select([rows[i] for i in at], pack.rank, pack.B * pack.T)):
+                rows[i] = t
+        return None, rows[0], grads[1], grads[2], rows[1], rows[2]
 
 
 def _segment(cache: TaHDuoCache, layer_idx: int, depth: int, B: int, with_pos: bool):
-    """All rows written at (layer, depth), packed per sequence: k, v [rows,Hkv,D], cu int32, pos int32 or None.
+    """All rows written at (layer, depth), packed per sequence: k, v [rows,Hkv,D], cu int32, pos int32 or None, and whether
+    ``cu`` holds pairs (:class:`_Packed`; never with positions).
 
     One chunk (prefill / training, the only case on the backward path) packs without copies when every
     token is valid; several chunks (a cache grown by earlier calls) are concatenated per sequence.
@@ -314,13 +363,13 @@ def _segment(cache: TaHDuoCache, layer_idx: int, depth: int, B: int, with_pos: b
         # and under autograd their gradients then meet at the packed tensor (one scatter back, not one per call).
         # (Training only: without gradients the copy would only hold memory for as long as the cache lives.)
         if pk.rows is None or not (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad)):
-            return pk.pack(k), pk.pack(v), pk.cu, pk.pos
+            return pk.pack(k), pk.pack(v), pk.cu, pk.pos, pk.paired
         slot = (layer_idx, depth)
         kept = cache._kv_packed.get(slot)
         if kept is None or kept[0] is not k or kept[1] is not v or kept[2] is not pk or kept[3] != (k._version, v._version):
             kept = (k, v, pk, (k._version, v._version), pk.pack(k), pk.pack(v))
             cache._kv_packed[slot] = kept
-        return kept[4], kept[5], pk.cu, pk.pos
+        return kept[4], kept[5], pk.cu, pk.pos, pk.paired
     k = torch.cat([c[0] for c in chunks], dim=2)
     v = torch.cat([c[1] for c in chunks], dim=2)
     T = k.shape[2]
@@ -328,7 +377,7 @@ def _segment(cache: TaHDuoCache, layer_idx: int, depth: int, B: int, with_pos: b
     valid = torch.cat([c[3] if c[3] is not None else one(c, 1) for c in chunks], dim=1)
     pos = torch.cat([c[2] if c[2] is not None else one(c, 0) for c in chunks], dim=1) if with_pos else None
     pk = _Packed(valid, pos, B, T, dev)
-    return pk.pack(k), pk.pack(v), pk.cu, pk.pos
+    return pk.pack(k), pk.pack(v), pk.cu, pk.pos, pk.paired
 
 
 def _merge_plan(m: "DuoMask", segs, B: int):
@@ -372,7 +421,7 @@ def _sparse_keys(m: "DuoMask", cache: TaHDuoCache, layer: int, depth: int, B: in
         raise TahDuoError(f"no keys cached for layer {layer} at depths {first}..{depth}")
     bound = sum(cache.get_cache_length(layer, d) for d in range(first, depth + 1))
     if len(segs) == 1:
-        return segs[0] + (bound,)
+        return segs[0][:4] + (bound,)
     dest, cu, pos = _merge_plan(m, segs, B)
     kcat, vcat = torch.cat([sg[0] for sg in segs]), torch.cat([sg[1] for sg in segs])
     return torch.zeros_like(kcat).index_copy(0, dest, kcat), torch.zeros_like(vcat).index_copy(0, dest, vcat), cu, pos, bound
@@ -443,29 +492,62 @@ def duo_attention_forward(module, query: torch.Tensor, key: torch.Tensor, value:
     pq = m._packed
     if not isinstance(pq, _Packed):
         raise TahDuoError("a DuoMask cannot be shared between the decode path and the varlen path")
-    q = pq.pack(query)
-    zc = torch.zeros(B + 1, dtype=torch.int32, device=dev)
-    zi = torch.zeros(0, dtype=torch.int32, device=dev)
-    e_q = q[:0]
-    if depth == 0 and ranks:
-        k1, v1, cu_k1, _ = _segment(cache, layer, 0, B, with_pos=False)
-        Hkv = k1.shape[1]
-        e_k = k1[:0]
-        sched = _schedule_of(m, (pq.cu, cu_k1, zc, zc, zi, Hq, Hkv, q.shape[0], k1.shape[0], 0))
-        o, _ = duo_attn_varlen(q, k1, v1, pq.cu, cu_k1, e_q, e_k, e_k, zi, zi, zc, zc, scale, schedule=sched,
-                               max_seqlen_k1=cache.get_cache_length(layer, 0))
+    return _attend_block(m, cache, layer, pq, query, scale, ranks), None
+
+
+def _attend_block(m: "DuoMask", cache: TaHDuoCache, layer: int, pq: _Packed, query: torch.Tensor, scale: float, ranks: bool) -> torch.Tensor:
+    """The general path of :func:`duo_attention_forward`: packed varlen kernels, (B, Tq, Hq, D)."""
+    B, Hq, _, D = query.shape
+    depth, dev = m.iter_depth, query.device
+    if m._empty is None:
+        m._empty = (torch.zeros(B + 1, dtype=torch.int32, device=dev), torch.zeros(0, dtype=torch.int32, device=dev))
+    b = types.SimpleNamespace(second=depth >= 1 or not ranks, scale=scale, pack_q=pq, cu_q=pq.cu, pos_q=pq.pos, packs=[])
+    b.none_cu, b.none_pos = m._empty
+    q = pq.unmoved(query)
+    n_q = q.shape[0] if pq.rows is None else pq.n
+    k1_paired = False
+    if ranks:
+        k1, v1, b.cu_k1, _, k1_paired = _segment(cache, layer, 0, B, with_pos=False)
+        b.max_k1 = cache.get_cache_length(layer, 0)
+    at_q = [0]  # of (q, k2, v2): what the pack of the query rows moves
+    if b.second:
+        own = _own_keys(cache, layer, depth, pq) if ranks else None
+        if own is not None:
+            k2, v2, b.max_k2 = own
+            b.cu_k2, b.pos_k, n_k2 = pq.cu, pq.pos, n_q
+            at_q = [0, 1, 2]
+        else:
+            k2, v2, b.cu_k2, b.pos_k, b.max_k2 = _sparse_keys(m, cache, layer, depth, B, first=1 if ranks else 0)
+            n_k2 = k2.shape[0]
+        if not ranks:  # no key without a position of its own
+            k1, v1, b.cu_k1, b.max_k1 = k2.detach()[:0], v2.detach()[:0], b.none_cu, 0
     else:
-        k2, v2, cu_k2, pos_k2, bound_k2 = _sparse_keys(m, cache, layer, depth, B, first=1 if ranks else 0)
-        Hkv = k2.shape[1]
-        if ranks:
-            k1, v1, cu_k1, _ = _segment(cache, layer, 0, B, with_pos=False)
-            bound_k1 = cache.get_cache_length(layer, 0)
-        else:  # no key without a position of its own
-            k1, v1, cu_k1, bound_k1 = k2[:0], v2[:0], zc, 0
-        sched = _schedule_of(m, (zc, cu_k1, pq.cu, cu_k2, pq.pos, Hq, Hkv, 0, k1.shape[0], k2.shape[0]))
-        _, o = duo_attn_varlen(e_q, k1, v1, zc, cu_k1, q, k2, v2, pq.pos, pos_k2, pq.cu, cu_k2, scale, schedule=sched,
-                               max_seqlen_k1=bound_k1, max_seqlen_k2=bound_k2)
-    return pq.unpack(o, Hq, D), None
+        k2 = v2 = k1.detach()[:0]
+        b.max_k2 = n_k2 = 0
+    Hkv = k1.shape[1]
+    if b.second:
+        b.pairs = 2 if k1_paired else 0
+        b.schedule = _schedule_of(m, (b.none_cu, b.cu_k1, pq.cu, b.cu_k2, pq.pos, Hq, Hkv, 0, k1.shape[0], n_k2), b.pairs)
+    else:
+        b.pairs = (1 if pq.paired else 0) + (2 if k1_paired else 0)
+        b.schedule = _schedule_of(m, (pq.cu, b.cu_k1, b.none_cu, b.none_cu, b.none_pos, Hq, Hkv, n_q, k1.shape[0], 0), b.pairs)
+    if pq.rows is not None:
+        b.packs.append((pq, at_q))
+    return _BlockAttn.apply(b, q, k1, v1, k2, v2)
+
+
+def _own_keys(cache: TaHDuoCache, layer: int, depth: int, pq: _Packed):
+    """(k, v, upper bound of a sequence's rows), not moved, where the keys that a query at ``depth`` sees beside the depth-0 ones are one
+    block with the queries' own rows (their valid mask and positions: a model's second iteration), else None."""
+    if depth != 1 or not cache.has_rows(layer, 1):
+        return None
+    chunks = cache.chunks(layer, 1)
+    if len(chunks) != 1:
+        return None
+    k, v, pos, valid = chunks[0]
+    if valid is not pq.valid or pos is not pq.given_pos or pos is None or k.shape[2] != pq.T:
+        return None
+    return pq.unmoved(k), pq.unmoved(v), cache.get_cache_length(layer, 1)
 
 
 # Calls with at least this many (query row, kv head) pairs get a launch-order table: below it a launch has about
@@ -476,17 +558,17 @@ SCHEDULE_MIN_ROW_HEADS = 49152
 SCHEDULE_MIN_MEAN_ROWS = 256
 
 
-def _schedule_of(m: "DuoMask", args):
+def _schedule_of(m: "DuoMask", args, pairs: int = 0):
     """The launch-order table of this mask's varlen calls: built at the first layer, shared by the others (the
     boundaries of queries and cached keys are the same in every layer of a step) and by the backward pass."""
     cu_q1, cu_k1, cu_q2, cu_k2, pos_q2, hq, hkv, tq1, tk1, tk2 = args
-    rows, nseq = tq1 + pos_q2.shape[0], max(1, cu_k1.numel() - 1)
+    rows, nseq = tq1 + pos_q2.shape[0], max(1, cu_k1.numel() // 2 if pairs & 2 else cu_k1.numel() - 1)
     if rows * hkv < SCHEDULE_MIN_ROW_HEADS or rows < SCHEDULE_MIN_MEAN_ROWS * nseq:
         return None
-    key = (tq1, tk1, pos_q2.shape[0], tk2, hq, hkv, cu_k1.data_ptr(), cu_k2.data_ptr())
+    key = (tq1, tk1, pos_q2.shape[0], tk2, hq, hkv, cu_k1.data_ptr(), cu_k2.data_ptr(), pairs)
     memo = getattr(m, "_sched", None)
     if memo is None or memo[0] != key:
-        memo = (key, ops.duo_schedule(cu_q1, cu_k1, cu_q2, cu_k2, pos_q2, hq, hkv, tq1, tk1, tk2), (cu_k1, cu_k2))
+        memo = (key, ops.duo_schedule(cu_q1, cu_k1, cu_q2, cu_k2, pos_q2, hq, hkv, tq1, tk1, tk2, pairs), (cu_k1, cu_k2))
         m._sched = memo
     return memo[1]
 

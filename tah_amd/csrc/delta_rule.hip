@@ -583,7 +583,7 @@ __global__ __launch_bounds__(kChunkThreads) void delta_chunk_kernel(const tah_de
     __shared__ __align__(16) float al[kChunk][kChunk + 4];
     __shared__ float gl[kChunk], bl[kChunk], be[kChunk];  // G, beta, beta exp(G)
     int slot = blockIdx.x, b = 0, row0 = 0, row_end = 0;
-    if (!find_tile(P.cu, P.nseq, kChunk, slot, b, row0, row_end)) return;
+    if (!find_tile(P.cu, 0, P.nseq, kChunk, slot, b, row0, row_end)) return;
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, c = lane % 16, g = lane / 16;
     const int h = blockIdx.y, kh = h / (L.heads / L.kv_heads), n = row_end - row0;
     float* const out = work + ((int64_t)blockIdx.x * L.heads + h) * chunk_floats(D, L.vdim);

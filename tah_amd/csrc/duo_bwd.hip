@@ -42,6 +42,7 @@ struct BwdStream {
     int64_t q_rs, q_hs, k_rs, k_hs, v_rs, v_hs, o_rs, o_hs;
     int64_t do_rs, do_hs, dq_rs, dq_hs, dk_rs, dk_hs, dv_rs, dv_hs;
     int32_t total_q, total_k;
+    int32_t q_shift, k_shift;  // of the boundaries (lane_bounds)
 };
 struct BwdParams {
     BwdStream s1, s2;
@@ -64,8 +65,8 @@ struct BwdParams {
 // recomputes S and dP: 5 products per (query tile, key tile) pair instead of 7.
 // The workspace is a table of 16 KiB blocks, one per (64 query rows, query head, 128 keys):
 //   block = ((qslot * hq + head) * ds_kt + ktile)
-//   qslot = cu_q1[seq] / 64 + seq + tile                  depth-0 query rows  (ds_q1slots slots)
-//           ds_q1slots + cu_q2[seq] / 64 + seq + tile     depth-1 query rows
+//   qslot = first row / 64 + seq + tile                   depth-0 query rows  (ds_q1slots slots)
+//           ds_q1slots + first row / 64 + seq + tile      depth-1 query rows
 //   ktile = key tile inside its sequence (depth 0), ds_kt1 + key tile (depth 1)
 // (cu / 64 + seq numbers the 64-row tiles of successive sequences without collisions and needs no prefix
 // sum over tile counts.)  Inside a block wave w = 4 * (query half) + (32-key block) of the key-tile kernel
@@ -144,28 +145,26 @@ __global__ __launch_bounds__(kDqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
     // (the table's order: heaviest tile of the whole call first)
     sched_lookup(p.sched, false, p.nseq, G, p.s1.total_q, p.s2.total_q, p.s1.total_k, p.s2.total_k, (int)gridDim.y,
                  (int)blockIdx.y, slot);
-    if (!(p.s1.total_q > 0 && find_tile(p.s1.cu_q, p.nseq, BM, slot, seq, row0, row_end))) {
-        if (!(p.s2.total_q > 0 && find_tile(p.s2.cu_q, p.nseq, BM, slot, seq, row0, row_end))) return;
+    if (!(p.s1.total_q > 0 && find_tile(p.s1.cu_q, p.s1.q_shift, p.nseq, BM, slot, seq, row0, row_end))) {
+        if (!(p.s2.total_q > 0 && find_tile(p.s2.cu_q, p.s2.q_shift, p.nseq, BM, slot, seq, row0, row_end))) return;
         second = true;
     }
     const BwdStream& qs = second ? p.s2 : p.s1;
     const int head = hk * G + wave % G;
     const int rblk = wave / G;
-    const int k1_lo = p.s1.cu_k[seq];
-    const int lk1 = p.s1.cu_k[seq + 1] - k1_lo;
+    const int k1_lo = p.s1.cu_k[seq << p.s1.k_shift];
+    const int lk1 = p.s1.cu_k[(seq << p.s1.k_shift) + 1] - k1_lo;
     const __bf16* k1p = p.s1.k + (int64_t)k1_lo * p.s1.k_rs + (int64_t)hk * p.s1.k_hs;
     const __bf16* v1p = p.s1.v + (int64_t)k1_lo * p.s1.v_rs + (int64_t)hk * p.s1.v_hs;
-    const int left1 = p.s1.total_k - k1_lo;
-    int lk2 = 0, left2 = 0;
+    int lk2 = 0;
     const __bf16 *k2p = nullptr, *v2p = nullptr;
     const int32_t* pos2p = nullptr;
     if (second) {
-        const int k2_lo = p.s2.cu_k[seq];
-        lk2 = p.s2.cu_k[seq + 1] - k2_lo;
+        const int k2_lo = p.s2.cu_k[seq << p.s2.k_shift];
+        lk2 = p.s2.cu_k[(seq << p.s2.k_shift) + 1] - k2_lo;
         k2p = p.s2.k + (int64_t)k2_lo * p.s2.k_rs + (int64_t)hk * p.s2.k_hs;
         v2p = p.s2.v + (int64_t)k2_lo * p.s2.v_rs + (int64_t)hk * p.s2.v_hs;
         pos2p = p.s2.pos_k + k2_lo;
-        left2 = p.s2.total_k - k2_lo;
     }
 
     const int row = row0 + rblk * 32 + col;
@@ -175,8 +174,7 @@ __global__ __launch_bounds__(kDqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
     if (second) {
         qpos = qs.pos_q[row_ld];
     } else {
-        const int q_lo = qs.cu_q[seq];
-        qpos = (row_ld - q_lo) + (lk1 - (qs.cu_q[seq + 1] - q_lo));
+        qpos = row_ld + (lk1 - qs.cu_q[(seq << qs.q_shift) + 1]);
     }
     const int qlim1 = row_ok ? ((qpos < lk1 - 1 && !kDense) ? qpos : lk1 - 1) : -1;
     const int qlim2 = row_ok ? qpos : -1;
@@ -200,7 +198,7 @@ __global__ __launch_bounds__(kDqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
     const unsigned char* mask_row = nullptr;  // additive-mask mode: this lane's mask row
     if constexpr (kDense) {
         const int64_t e = (int64_t)seq * p.mask_sb + (int64_t)head * p.mask_sh +
-                          (int64_t)(row_ld - qs.cu_q[seq]) * p.mask_sq;
+                          (int64_t)(row_ld - qs.cu_q[seq << qs.q_shift]) * p.mask_sq;
         mask_row = static_cast<const unsigned char*>(p.mask) + e * (p.mask_f32 ? 4 : 2);
     }
 
@@ -227,7 +225,7 @@ __global__ __launch_bounds__(kDqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
 
     // asynchronous global -> LDS copy of one K/V tile (both row-major, swizzled), as in the forward
     // kernel: (wave-uniform pointer to the tile's first row) + (per-lane byte offset), rows past the
-    // end of the array repeat its last row (finite data, masked by index)
+    // end of the segment repeat its last row (what lies behind it may be anything; masked by index)
     const int my_lrow = 8 * wave + (lane >> 4);  // second piece: 4 rows further down
     const uint32_t my_chunk0 = (uint32_t)(((lane & 15) ^ row_swizzle(my_lrow)) * 16);
     const uint32_t my_chunk1 = (uint32_t)(((lane & 15) ^ row_swizzle(my_lrow + 4)) * 16);
@@ -238,7 +236,7 @@ __global__ __launch_bounds__(kDqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
         const int64_t vrs = s0 ? p.s1.v_rs : p.s2.v_rs;
         const __bf16* kt0 = (s0 ? k1p : k2p) + (int64_t)base * krs;
         const __bf16* vt0 = (s0 ? v1p : v2p) + (int64_t)base * vrs;
-        const int last = (s0 ? left1 : left2) - 1 - base;  // >= 0: a tile starts inside its segment
+        const int last = (s0 ? lk1 : lk2) - 1 - base;  // >= 0: a tile starts inside its segment
         unsigned char* kt = smem + buf * kDqStage;
         unsigned char* vt = kt + kTileBytes;
         const uint32_t r0 = (uint32_t)(my_lrow < last ? my_lrow : last) & 63u;
@@ -371,22 +369,22 @@ __global__ __launch_bounds__(kKvThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dkd
 
     int seq = 0, key0 = 0, key_end = 0;
     bool second = false;
-    const CallBounds cb = call_bounds(p, p.s2.total_q > 0 || p.s2.total_k > 0);
+    const CallBounds cb = call_bounds(p);
     int slot = (int)blockIdx.y;  // without a table: early (heavy) key tiles of each sequence first
     // (the table's order: the key tile seen by the most query rows first)
     sched_lookup(p.sched, true, p.nseq, G, p.s1.total_q, p.s2.total_q, p.s1.total_k, p.s2.total_k, (int)gridDim.y,
                  (int)blockIdx.y, slot);
-    if (!(p.s1.total_k > 0 && find_tile(p.s1.cu_k, p.nseq, kBK, slot, seq, key0, key_end, cb.k1))) {
-        if (!(p.s2.total_k > 0 && find_tile(p.s2.cu_k, p.nseq, kBK, slot, seq, key0, key_end, cb.k2))) return;
+    if (!(p.s1.total_k > 0 && find_tile(p.s1.cu_k, p.s1.k_shift, p.nseq, kBK, slot, seq, key0, key_end, cb.k1))) {
+        if (!(p.s2.total_k > 0 && find_tile(p.s2.cu_k, p.s2.k_shift, p.nseq, kBK, slot, seq, key0, key_end, cb.k2))) return;
         second = true;
     }
     const BwdStream& ks = second ? p.s2 : p.s1;
-    const LaneBounds key1 = bounds_at(cb.k1, p.s1.cu_k, seq);
-    const int k_lo = second ? bounds_at(cb.k2, p.s2.cu_k, seq).lo : key1.lo;
+    const LaneBounds key1 = bounds_at(cb.k1, p.s1.cu_k, p.s1.k_shift, seq);
+    const int k_lo = second ? bounds_at(cb.k2, p.s2.cu_k, p.s2.k_shift, seq).lo : key1.lo;
     const int lk1 = key1.hi - key1.lo;
     LaneBounds own1{0, 0}, own2{0, 0};
-    if (p.s1.total_q > 0) own1 = bounds_at(cb.q1, p.s1.cu_q, seq);
-    if (p.s2.total_q > 0) own2 = bounds_at(cb.q2, p.s2.cu_q, seq);
+    if (p.s1.total_q > 0) own1 = bounds_at(cb.q1, p.s1.cu_q, p.s1.q_shift, seq);
+    if (p.s2.total_q > 0) own2 = bounds_at(cb.q2, p.s2.cu_q, p.s2.q_shift, seq);
     const int q1_lo = own1.lo, lq1 = own1.hi - q1_lo;
     const int q2_lo = own2.lo, lq2 = own2.hi - q2_lo;
     const int off = lk1 - lq1;  // position of depth-0 query i is i + off
@@ -816,32 +814,30 @@ __global__ __launch_bounds__(kLqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
 
     int seq = 0, row0 = 0, row_end = 0;
     bool second = false;
-    const CallBounds cb = call_bounds(p, p.s2.total_q > 0);
+    const CallBounds cb = call_bounds(p);
     int slot = (int)(gridDim.y - 1 - blockIdx.y);  // without a table: late (heavy) tiles of each sequence first
     // (the table's order: heaviest tile of the whole call first)
     sched_lookup(p.sched, false, p.nseq, G, p.s1.total_q, p.s2.total_q, p.s1.total_k, p.s2.total_k, (int)gridDim.y,
                  (int)blockIdx.y, slot);
-    if (!(p.s1.total_q > 0 && find_tile(p.s1.cu_q, p.nseq, BM, slot, seq, row0, row_end, cb.q1))) {
-        if (!(p.s2.total_q > 0 && find_tile(p.s2.cu_q, p.nseq, BM, slot, seq, row0, row_end, cb.q2))) return;
+    if (!(p.s1.total_q > 0 && find_tile(p.s1.cu_q, p.s1.q_shift, p.nseq, BM, slot, seq, row0, row_end, cb.q1))) {
+        if (!(p.s2.total_q > 0 && find_tile(p.s2.cu_q, p.s2.q_shift, p.nseq, BM, slot, seq, row0, row_end, cb.q2))) return;
         second = true;
     }
     const BwdStream& qs = second ? p.s2 : p.s1;
     LaneBounds own1{0, 0};
-    if (p.s1.total_q > 0) own1 = bounds_at(cb.q1, p.s1.cu_q, seq);
-    const LaneBounds own = second ? bounds_at(cb.q2, p.s2.cu_q, seq) : own1, key1 = bounds_at(cb.k1, p.s1.cu_k, seq);
+    if (p.s1.total_q > 0) own1 = bounds_at(cb.q1, p.s1.cu_q, p.s1.q_shift, seq);
+    const LaneBounds own = second ? bounds_at(cb.q2, p.s2.cu_q, p.s2.q_shift, seq) : own1, key1 = bounds_at(cb.k1, p.s1.cu_k, p.s1.k_shift, seq);
     const int q_lo = own.lo, q_end = own.hi;
     const int k1_lo = key1.lo, lk1 = key1.hi - k1_lo, lq1 = own1.hi - own1.lo;
     const int off = lk1 - lq1;  // position of depth-0 query row i of the sequence is i + off
     const __bf16* k1p = p.s1.k + (int64_t)k1_lo * p.s1.k_rs + (int64_t)hk * p.s1.k_hs;
-    const int left1 = p.s1.total_k - k1_lo;
-    int lk2 = 0, left2 = 0;
+    int lk2 = 0;
     const __bf16* k2p = nullptr;
     if (second) {
-        const LaneBounds key2 = bounds_at(cb.k2, p.s2.cu_k, seq);
+        const LaneBounds key2 = bounds_at(cb.k2, p.s2.cu_k, p.s2.k_shift, seq);
         const int k2_lo = key2.lo;
         lk2 = key2.hi - k2_lo;
         k2p = p.s2.k + (int64_t)k2_lo * p.s2.k_rs + (int64_t)hk * p.s2.k_hs;
-        left2 = p.s2.total_k - k2_lo;
     }
 
     // my unit: 64-row tile `tile` of the sequence's query rows (all wave-uniform)
@@ -881,7 +877,7 @@ __global__ __launch_bounds__(kLqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
         const int ks = s0 ? s : s - n1;  // 64-key step inside its segment
         const int64_t krs = s0 ? p.s1.k_rs : p.s2.k_rs;
         const __bf16* kt0 = (s0 ? k1p : k2p) + (int64_t)ks * kBN * krs;
-        const int last = (s0 ? left1 : left2) - 1 - ks * kBN;
+        const int last = (s0 ? lk1 : lk2) - 1 - ks * kBN;
         auto* kt = smem + stage * kLqStage;
         const uint32_t r0 = (uint32_t)(my_lrow < last ? my_lrow : last) & 63u;
         const uint32_t r1 = (uint32_t)(my_lrow + 4 < last ? my_lrow + 4 : last) & 63u;
@@ -977,7 +973,7 @@ __global__ __launch_bounds__(kLqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
     }
 }
 
-BwdStream to_dev(const tah_duo_stream& s, const tah_duo_bwd_stream& g) {
+BwdStream to_dev(const tah_duo_stream& s, const tah_duo_bwd_stream& g, int pairs) {
     BwdStream d;
     d.q = static_cast<const __bf16*>(s.q);
     d.k = static_cast<const __bf16*>(s.k);
@@ -1000,6 +996,8 @@ BwdStream to_dev(const tah_duo_stream& s, const tah_duo_bwd_stream& g) {
     d.dv_rs = g.dv_row_stride; d.dv_hs = g.dv_head_stride;
     d.total_q = s.total_q;
     d.total_k = s.total_k;
+    d.q_shift = pairs & 1;
+    d.k_shift = pairs >> 1 & 1;
     return d;
 }
 
@@ -1085,6 +1083,7 @@ int dispatch_bwd(const tah_duo_bwd_args* a, const tah_additive_mask* m, tah_stre
     if (f.d != kD || f.nseq < 0 || f.hq <= 0 || f.hkv <= 0 || f.hq % f.hkv != 0) return TAH_E_SHAPE;
     const int g = f.hq / f.hkv;
     if (g != 1 && g != 2 && g != 4 && g != 8) return TAH_E_SHAPE;
+    if (f.cu_pairs & ~15) return TAH_E_SHAPE;
     if (kDense) {
         if (!m || !m->mask) return TAH_E_NULL;
         if (f.s2.total_q != 0 || f.s2.total_k != 0 || (m->dtype != 0 && m->dtype != 1) || f.scale == 0.f) return TAH_E_SHAPE;
@@ -1093,9 +1092,10 @@ int dispatch_bwd(const tah_duo_bwd_args* a, const tah_additive_mask* m, tah_stre
     if (int rc = check_bwd_stream(f.s1, a->g1, false)) return rc;
     if (int rc = check_bwd_stream(f.s2, a->g2, true)) return rc;
     BwdParams p;
-    p.s1 = to_dev(f.s1, a->g1);
-    p.s2 = to_dev(f.s2, a->g2);
+    p.s1 = to_dev(f.s1, a->g1, f.cu_pairs);
+    p.s2 = to_dev(f.s2, a->g2, f.cu_pairs >> 2);
     p.nseq = f.nseq;
+    fill_absent_bounds(p, p.s2.total_q > 0 || p.s2.total_k > 0);
     p.hq = f.hq;
     p.hkv = f.hkv;
     p.scale = f.scale;

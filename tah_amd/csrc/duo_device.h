@@ -396,30 +396,32 @@ __device__ __forceinline__ int wave_prefix_sum(int x) {
 __device__ __forceinline__ int32_t const_i32(const int32_t* a, int i) { return ((const TAH_CONST_AS int32_t*)a)[i]; }
 
 // Boundaries of a wave's 64 sequences from b0 on, one per lane (no sequence: an empty one).  Asked for without a branch, so that a
-// kernel can have those of all its streams on their way at once.
+// kernel can have those of all its streams on their way at once.  Sequence b's rows are cu[b << shift] ... cu[(b << shift) + 1]: shift 0
+// for sequences one behind the other, 1 for (first row, one past the last) pairs with rows between sequences that belong to none.  nseq > b0.
 struct LaneBounds {
     int lo, hi;
 };
-__device__ __forceinline__ LaneBounds lane_bounds(const int32_t* cu, int b0, int nseq) {
+__device__ __forceinline__ LaneBounds lane_bounds(const int32_t* cu, int b0, int nseq, int shift) {
     const int b = b0 + (int)(threadIdx.x % kWave);
     const bool there = b < nseq;
     LaneBounds x;
-    x.lo = cu[there ? b : b0];
-    x.hi = cu[there ? b + 1 : b0];
+    const int at = (there ? b : b0) << shift;
+    x.lo = cu[at];
+    x.hi = cu[at + 1];
     x.lo = there ? x.lo : 0;
     x.hi = there ? x.hi : 0;
     return x;
 }
 
-// Locate tile `slot` among sequences whose lengths are cu[b+1]-cu[b], `bm` rows
+// Locate tile `slot` among sequences with the boundaries lane_bounds reads, `bm` rows
 // per tile.  On success fills seq/row0/row_end and returns true; otherwise
 // subtracts the number of tiles in this stream from `slot` and returns false.
 // Every lane of the wave must call it with the same arguments: the lanes take 64 sequences at a time (one pair of
 // loads and a prefix sum over the lanes), so that a batch of hundreds of short sequences costs a workgroup a few
-// steps and not one scalar load pair per sequence.  `first`: lane_bounds(cu, 0, nseq), nseq > 0.
-__device__ __forceinline__ bool find_tile(const int32_t* cu, int nseq, int bm, int& slot, int& seq, int& row0, int& row_end, LaneBounds first) {
+// steps and not one scalar load pair per sequence.  `first`: lane_bounds(cu, 0, nseq, shift), nseq > 0.
+__device__ __forceinline__ bool find_tile(const int32_t* cu, int shift, int nseq, int bm, int& slot, int& seq, int& row0, int& row_end, LaneBounds first) {
     for (int b0 = 0; b0 < nseq; b0 += kWave) {
-        const LaneBounds x = b0 == 0 ? first : lane_bounds(cu, b0, nseq);
+        const LaneBounds x = b0 == 0 ? first : lane_bounds(cu, b0, nseq, shift);
         const int n = (x.hi - x.lo + bm - 1) / bm;
         const int incl = wave_prefix_sum(n);  // tiles of sequences b0 .. b
         const int tot = lane_value(incl, kWave - 1);
@@ -435,31 +437,41 @@ __device__ __forceinline__ bool find_tile(const int32_t* cu, int nseq, int bm, i
     }
     return false;
 }
-__device__ __forceinline__ bool find_tile(const int32_t* cu, int nseq, int bm, int& slot, int& seq, int& row0, int& row_end) {
-    return nseq > 0 && find_tile(cu, nseq, bm, slot, seq, row0, row_end, lane_bounds(cu, 0, nseq));
+__device__ __forceinline__ bool find_tile(const int32_t* cu, int shift, int nseq, int bm, int& slot, int& seq, int& row0, int& row_end) {
+    return nseq > 0 && find_tile(cu, shift, nseq, bm, slot, seq, row0, row_end, lane_bounds(cu, 0, nseq, shift));
 }
 
-// The first 64 sequences' boundaries in both streams of a varlen call, asked for at once (a stream without queries or keys may
-// come without them): a workgroup's start is a chain of trips to memory, and which tile it is, where its sequence's keys lie and
-// how many there are then follow from one of them.  k2: whether the caller looks at the depth-1 keys' boundaries.
+// The first 64 sequences' boundaries in both streams of a varlen call, asked for at once: a workgroup's start is a chain of trips to
+// memory, and which tile it is, where its sequence's keys lie and how many there are then follow from one of them.
 struct CallBounds {
     LaneBounds q1, k1, q2, k2;
 };
 template <class P>
-__device__ __forceinline__ CallBounds call_bounds(const P& p, bool k2) {
-    const bool q2 = p.s2.total_q > 0;
+__device__ __forceinline__ CallBounds call_bounds(const P& p) {
     CallBounds x;
-    x.q1 = lane_bounds(p.s1.total_q > 0 ? p.s1.cu_q : p.s1.cu_k, 0, p.nseq);
-    x.k1 = lane_bounds(p.s1.cu_k, 0, p.nseq);
-    x.q2 = lane_bounds(q2 ? p.s2.cu_q : p.s1.cu_k, 0, p.nseq);
-    x.k2 = lane_bounds(k2 ? p.s2.cu_k : p.s1.cu_k, 0, p.nseq);
+    x.q1 = lane_bounds(p.s1.cu_q, 0, p.nseq, p.s1.q_shift);
+    x.k1 = lane_bounds(p.s1.cu_k, 0, p.nseq, p.s1.k_shift);
+    x.q2 = lane_bounds(p.s2.cu_q, 0, p.nseq, p.s2.q_shift);
+    x.k2 = lane_bounds(p.s2.cu_k, 0, p.nseq, p.s2.k_shift);
     return x;
 }
+// Boundaries that a call may come without (no queries, no keys that anybody looks at): call_bounds reads the depth-0 keys' in their place.
+// (Chosen on the host: a choice between pointers in a kernel became a branch with a trip to the arguments inside.)
+template <class P>
+void fill_absent_bounds(P& p, bool k2) {
+    auto same = [&](const int32_t*& cu, int32_t& shift) {
+        cu = p.s1.cu_k;
+        shift = p.s1.k_shift;
+    };
+    if (p.s1.total_q == 0) same(p.s1.cu_q, p.s1.q_shift);
+    if (p.s2.total_q == 0) same(p.s2.cu_q, p.s2.q_shift);
+    if (!k2) same(p.s2.cu_k, p.s2.k_shift);
+}
 // Those of one sequence (the same one for the whole wave)
-__device__ __forceinline__ LaneBounds bounds_at(const LaneBounds& first, const int32_t* cu, int seq) {
+__device__ __forceinline__ LaneBounds bounds_at(const LaneBounds& first, const int32_t* cu, int shift, int seq) {
     LaneBounds x;
-    x.lo = seq < kWave ? lane_value(first.lo, seq % kWave) : const_i32(cu, seq);
-    x.hi = seq < kWave ? lane_value(first.hi, seq % kWave) : const_i32(cu, seq + 1);
+    x.lo = seq < kWave ? lane_value(first.lo, seq % kWave) : const_i32(cu, seq << shift);
+    x.hi = seq < kWave ? lane_value(first.hi, seq % kWave) : const_i32(cu, (seq << shift) + 1);
     return x;
 }
 

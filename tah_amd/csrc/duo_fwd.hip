@@ -70,6 +70,7 @@ struct FwdStream {
     const int32_t *cu_q, *cu_k, *pos_q, *pos_k;
     int64_t q_rs, q_hs, k_rs, k_hs, v_rs, v_hs, o_rs, o_hs;
     int32_t total_q, total_k;
+    int32_t q_shift, k_shift;  // of the boundaries (lane_bounds)
 };
 struct FwdParams {
     FwdStream s1, s2;
@@ -120,7 +121,7 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     // ---- which tile am I ---------------------------------------------------
     // (all boundaries in one trip, together with the table, and scalar arithmetic on them: 333 rows, where the last workgroup's start was
     // 2.7 of 16 us, 16.95 -> 16.1 us; 4 x 4096 rows, 3.8 us a workgroup, 316 -> 312; 8192 forward and backward 1231 -> 1222)
-    const CallBounds cb = call_bounds(p, p.s2.total_q > 0);  // (keys of a depth without queries may come without boundaries)
+    const CallBounds cb = call_bounds(p);
     const bool has1 = p.s1.total_q > 0, has2 = p.s2.total_q > 0;
     int seq = 0, row0 = 0, row_end = 0;
     bool second = false;
@@ -130,8 +131,8 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     if (sched_lookup(p.sched, false, p.nseq, G, p.s1.total_q, p.s2.total_q, p.s1.total_k, p.s2.total_k,
                      (int)gridDim.y / kPerEntry, (int)blockIdx.y / kPerEntry, slot)) {
         // the table's order: heaviest tile of the whole call first; its tiles have kPerEntry * BM rows
-        if (!(has1 && find_tile(p.s1.cu_q, p.nseq, kPerEntry * BM, slot, seq, row0, row_end, cb.q1))) {
-            if (!(has2 && find_tile(p.s2.cu_q, p.nseq, kPerEntry * BM, slot, seq, row0, row_end, cb.q2))) return;
+        if (!(has1 && find_tile(p.s1.cu_q, p.s1.q_shift, p.nseq, kPerEntry * BM, slot, seq, row0, row_end, cb.q1))) {
+            if (!(has2 && find_tile(p.s2.cu_q, p.s2.q_shift, p.nseq, kPerEntry * BM, slot, seq, row0, row_end, cb.q2))) return;
             second = true;
         }
         row0 += BM * ((int)blockIdx.y % kPerEntry);
@@ -139,8 +140,8 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
         row_end = row0 + BM < row_end ? row0 + BM : row_end;
     } else {
         slot = (int)(gridDim.y - 1 - blockIdx.y);  // late (heavy) tiles of each sequence first
-        if (!(has1 && find_tile(p.s1.cu_q, p.nseq, BM, slot, seq, row0, row_end, cb.q1))) {
-            if (!(has2 && find_tile(p.s2.cu_q, p.nseq, BM, slot, seq, row0, row_end, cb.q2))) return;
+        if (!(has1 && find_tile(p.s1.cu_q, p.s1.q_shift, p.nseq, BM, slot, seq, row0, row_end, cb.q1))) {
+            if (!(has2 && find_tile(p.s2.cu_q, p.s2.q_shift, p.nseq, BM, slot, seq, row0, row_end, cb.q2))) return;
             second = true;
         }
     }
@@ -149,23 +150,21 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     const int head = hk * G + block % G;
     const int rblk = block / G;
     // depth-0 key segment of this sequence (position of a key = its local index)
-    const LaneBounds key1 = bounds_at(cb.k1, p.s1.cu_k, seq);
+    const LaneBounds key1 = bounds_at(cb.k1, p.s1.cu_k, p.s1.k_shift, seq);
     const int k1_lo = key1.lo, lk1 = key1.hi - k1_lo;
     const __bf16* k1p = p.s1.k + (int64_t)k1_lo * p.s1.k_rs + (int64_t)hk * p.s1.k_hs;
     const __bf16* v1p = p.s1.v + (int64_t)k1_lo * p.s1.v_rs + (int64_t)hk * p.s1.v_hs;
-    const int left1 = p.s1.total_k - k1_lo;  // rows from the segment start to the end of the array
     // depth-1 key segment (explicit positions), only seen by depth-1 queries
-    int lk2 = 0, left2 = 0;
+    int lk2 = 0;
     const __bf16 *k2p = nullptr, *v2p = nullptr;
     const int32_t* pos2p = nullptr;
     if (second) {
-        const LaneBounds key2 = bounds_at(cb.k2, p.s2.cu_k, seq);
+        const LaneBounds key2 = bounds_at(cb.k2, p.s2.cu_k, p.s2.k_shift, seq);
         const int k2_lo = key2.lo;
         lk2 = key2.hi - k2_lo;
         k2p = p.s2.k + (int64_t)k2_lo * p.s2.k_rs + (int64_t)hk * p.s2.k_hs;
         v2p = p.s2.v + (int64_t)k2_lo * p.s2.v_rs + (int64_t)hk * p.s2.v_hs;
         pos2p = p.s2.pos_k + k2_lo;
-        left2 = p.s2.total_k - k2_lo;
     }
 
     // ---- my query row, its position, the tile's position bounds ------------
@@ -173,7 +172,7 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     const int row = wrow0 + col;
     const bool row_ok = row < row_end;
     const int row_ld = row_ok ? row : row_end - 1;  // tiles are never empty
-    const LaneBounds own = second ? bounds_at(cb.q2, p.s2.cu_q, seq) : bounds_at(cb.q1, p.s1.cu_q, seq);
+    const LaneBounds own = second ? bounds_at(cb.q2, p.s2.cu_q, p.s2.q_shift, seq) : bounds_at(cb.q1, p.s1.cu_q, p.s1.q_shift, seq);
     // last visible depth-0 key index of a position (additive-mask mode: every key of the sequence, the mask decides)
     auto limit1 = [&](int pos) __attribute__((always_inline)) { return (pos < lk1 - 1 && !kDense) ? pos : lk1 - 1; };
     int qpos, wmax1, wmin1, tmax1;
@@ -242,7 +241,7 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     // ---- asynchronous global -> LDS copies (no registers, no ds_write) ------------------------
     // A tile is 16 blocks of 4 rows, two per wave; lane l fills row 4*blk + l/16, physical chunk
     // l%16, i.e. fetches logical chunk (l%16) ^ row_swizzle(row) of that row.  Rows past the end
-    // of the segment are clamped to the last row of the array (finite data, masked by index).
+    // of the segment are clamped to its last row (what lies behind it may be anything; masked by index).
     // The source is addressed as (wave-uniform pointer to the tile's first row) + (per-lane byte
     // offset < 2^30: row strides are limited to 2^23 elements by the host-side checks).
     const int my_lrow = kRowsPerWave * wave + (lane >> 4);  // piece i: 4 * i rows further down
@@ -262,10 +261,10 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     auto issue_k = [&](int it) {  // K tile `it` -> K ring, plus the positions of depth-1 keys
         unsigned char* kt = smem + kKRing + (it % kStages) * kKBytes;
         if (it < n1) {
-            issue_rows(k1p, p.s1.k_rs, it * kBN, left1, kt);
+            issue_rows(k1p, p.s1.k_rs, it * kBN, lk1, kt);
         } else {
             const int base = (it - n1) * kBN;
-            issue_rows(k2p, p.s2.k_rs, base, left2, kt);
+            issue_rows(k2p, p.s2.k_rs, base, lk2, kt);
             if (wave == 0) {
                 int r = base + lane;
                 r = r < lk2 ? r : lk2 - 1;
@@ -275,8 +274,8 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
     };
     auto issue_v = [&](int it) {
         unsigned char* vt = smem + kVRing + (it % kStages) * kVBytes;
-        if (it < n1) issue_rows(v1p, p.s1.v_rs, it * kBN, left1, vt);
-        else issue_rows(v2p, p.s2.v_rs, (it - n1) * kBN, left2, vt);
+        if (it < n1) issue_rows(v1p, p.s1.v_rs, it * kBN, lk1, vt);
+        else issue_rows(v2p, p.s2.v_rs, (it - n1) * kBN, lk2, vt);
     };
     // start of even half-phase 2u: K(u+1) replaces K(u-1), V(u) replaces V(u-2)
     auto issue = [&](int u) {
@@ -617,7 +616,7 @@ __global__ __launch_bounds__(64 * W) TAH_WAVES_PER_EU(2, 2) void duo_fwd_kernel(
         qs.lse[(int64_t)head * qs.total_q + row] = l_tot > 0.f ? (m_run * c + fast_log2(l_tot)) * kLn2 : kNegInf;
 }
 
-FwdStream to_dev(const tah_duo_stream& s) {
+FwdStream to_dev(const tah_duo_stream& s, int pairs) {
     FwdStream d;
     d.q = static_cast<const __bf16*>(s.q);
     d.k = static_cast<const __bf16*>(s.k);
@@ -634,6 +633,8 @@ FwdStream to_dev(const tah_duo_stream& s) {
     d.o_rs = s.o_row_stride; d.o_hs = s.o_head_stride;
     d.total_q = s.total_q;
     d.total_k = s.total_k;
+    d.q_shift = pairs & 1;
+    d.k_shift = pairs >> 1 & 1;
     return d;
 }
 
@@ -705,6 +706,7 @@ int dispatch_fwd(const tah_duo_fwd_args* a, const tah_additive_mask* m, tah_stre
     if (a->d != kD || a->nseq < 0 || a->hq <= 0 || a->hkv <= 0 || a->hq % a->hkv != 0) return TAH_E_SHAPE;
     const int g = a->hq / a->hkv;
     if (g != 1 && g != 2 && g != 4 && g != 8) return TAH_E_SHAPE;
+    if (a->cu_pairs & ~15) return TAH_E_SHAPE;
     if (int rc = check_stream(a->s1, false)) return rc;
     if (int rc = check_stream(a->s2, true)) return rc;
     if (a->s2.total_q > 0 && (!a->s1.cu_k || (a->s1.total_k > 0 && (!a->s1.k || !a->s1.v)))) return TAH_E_NULL;
@@ -714,9 +716,10 @@ int dispatch_fwd(const tah_duo_fwd_args* a, const tah_additive_mask* m, tah_stre
     }
     if (a->nseq == 0 || (a->s1.total_q == 0 && a->s2.total_q == 0)) return TAH_OK;
     FwdParams p;
-    p.s1 = to_dev(a->s1);
-    p.s2 = to_dev(a->s2);
+    p.s1 = to_dev(a->s1, a->cu_pairs);
+    p.s2 = to_dev(a->s2, a->cu_pairs >> 2);
     p.nseq = a->nseq;
+    fill_absent_bounds(p, p.s2.total_q > 0);  // (keys of a depth without queries may come without boundaries)
     p.hq = a->hq;
     p.hkv = a->hkv;
     p.scale_log2e = a->scale * kLog2e;

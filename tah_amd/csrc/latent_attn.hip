@@ -234,7 +234,7 @@ __global__ __launch_bounds__(W * kWave) void attend_tile_kernel(const AttendTile
         tile = blockIdx.x % p.slots;
         h = blockIdx.x / p.slots;
     }
-    if (!find_tile(p.cu, p.nseq, kTileRows, tile, b, row0, row_end)) return;
+    if (!find_tile(p.cu, 0, p.nseq, kTileRows, tile, b, row0, row_end)) return;
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, c = lane % 16, g = lane / 16;
     const int dq = p.dim_pad + p.rot_pad, nq = kExact ? NQ : dq / 32, nv = kExact ? NV : p.vdim_pad / 16;
     const int ks = dq + 8, vs = p.vdim_pad + 16;  // row strides in LDS: what a read takes from several rows lies in different banks

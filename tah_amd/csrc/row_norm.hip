@@ -48,7 +48,7 @@ template <class E>
 __global__ __launch_bounds__(kWave) void conv_rows_kernel(const E* h, const float* conv, E* state, const tah_portions P, E* out, int cols, int taps,
                                                           int nslots) {
     int tile = blockIdx.y, b = 0, row0 = 0, row_end = 0;
-    if (!find_tile(P.cu, P.nseq, kConvRows, tile, b, row0, row_end)) return;
+    if (!find_tile(P.cu, 0, P.nseq, kConvRows, tile, b, row0, row_end)) return;
     const int c = 8 * (blockIdx.x * kWave + threadIdx.x);
     if (c >= cols) return;
     const int first = P.cu[b], last = P.cu[b + 1], slot = P.slot[b], pos0 = P.pos0[b];
@@ -91,7 +91,7 @@ template <class E>
 __global__ __launch_bounds__(kWave) void conv_few_rows_kernel(const E* h, const float* conv, E* state, const tah_portions P, E* out, int cols, int taps,
                                                               int nslots) {
     int tile = blockIdx.y, b = 0, row0 = 0, row_end = 0;
-    if (!find_tile(P.cu, P.nseq, kFewRows, tile, b, row0, row_end)) return;
+    if (!find_tile(P.cu, 0, P.nseq, kFewRows, tile, b, row0, row_end)) return;
     const int c = 8 * (blockIdx.x * kWave + threadIdx.x);
     if (c >= cols) return;
     const int first = P.cu[b], last = P.cu[b + 1], slot = P.slot[b], pos0 = P.pos0[b];

@@ -30,6 +30,7 @@ struct SchedParams {
     const int32_t *cu_q1, *cu_k1, *cu_q2, *cu_k2, *pos_q2;
     int32_t nseq, group, bm;
     int32_t total_q1, total_k1, total_q2, total_k2;
+    int32_t shift_q1, shift_k1, shift_q2, shift_k2;  // of the boundaries (lane_bounds)
     int32_t q_slots, k_slots;
     int32_t* out;
 };
@@ -64,20 +65,20 @@ __device__ int block_exclusive_scan(int* a, int n, int* tmp) {
     return total;
 }
 
-__device__ __forceinline__ int seg_len(const int32_t* cu, int total, int b) { return total > 0 ? cu[b + 1] - cu[b] : 0; }
+__device__ __forceinline__ int seg_len(const int32_t* cu, int shift, int total, int b) { return total > 0 ? cu[(b << shift) + 1] - cu[b << shift] : 0; }
 __device__ __forceinline__ int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 // Tile steps of tile i (rows i*tile .. of its segment) of sequence b in stream `second`.
 template <bool kKeyTiles>
 __device__ int tile_steps(const SchedParams& p, bool second, int b, int i, int tile) {
-    const int lq1 = seg_len(p.cu_q1, p.total_q1, b), lk1 = seg_len(p.cu_k1, p.total_k1, b);
-    const int lq2 = seg_len(p.cu_q2, p.total_q2, b), lk2 = seg_len(p.cu_k2, p.total_k2, b);
+    const int lq1 = seg_len(p.cu_q1, p.shift_q1, p.total_q1, b), lk1 = seg_len(p.cu_k1, p.shift_k1, p.total_k1, b);
+    const int lq2 = seg_len(p.cu_q2, p.shift_q2, p.total_q2, b), lk2 = seg_len(p.cu_k2, p.shift_k2, p.total_k2, b);
     const int off = lk1 - lq1;  // position of depth-0 query row r is r + off
     if (!kKeyTiles) {
         // query tile: depth-0 keys up to the position of its last row (+ every depth-1 key tile for depth-1 rows)
         const int lq = second ? lq2 : lq1;
         const int last_row = ((i + 1) * tile < lq ? (i + 1) * tile : lq) - 1;
-        int last_pos = second ? p.pos_q2[p.cu_q2[b] + last_row] : last_row + off;
+        int last_pos = second ? p.pos_q2[p.cu_q2[b << p.shift_q2] + last_row] : last_row + off;
         last_pos = last_pos < lk1 - 1 ? last_pos : lk1 - 1;
         return (last_pos >= 0 ? last_pos / kStep + 1 : 0) + (second ? ceil_div(lk2, kStep) : 0);
     }
@@ -91,12 +92,12 @@ __device__ int tile_steps(const SchedParams& p, bool second, int b, int i, int t
 
 // One sorted list: tiles of `tile` rows over segments cu_a (stream 0) and cu_b (stream 1), `slots` pairs at out.
 template <bool kKeyTiles>
-__device__ void build_list(const SchedParams& p, const int32_t* cu_a, int total_a, const int32_t* cu_b, int total_b,
+__device__ void build_list(const SchedParams& p, const int32_t* cu_a, int shift_a, int total_a, const int32_t* cu_b, int shift_b, int total_b,
                            int tile, int slots, int32_t* out, int* off_a, int* off_b, int* bins, int* tmp) {
     const int tid = threadIdx.x;
     for (int b = tid; b <= p.nseq; b += kSchedThreads) {
-        off_a[b] = b < p.nseq ? ceil_div(seg_len(cu_a, total_a, b), tile) : 0;
-        off_b[b] = b < p.nseq ? ceil_div(seg_len(cu_b, total_b, b), tile) : 0;
+        off_a[b] = b < p.nseq ? ceil_div(seg_len(cu_a, shift_a, total_a, b), tile) : 0;
+        off_b[b] = b < p.nseq ? ceil_div(seg_len(cu_b, shift_b, total_b, b), tile) : 0;
     }
     for (int c = tid; c < kSchedBins; c += kSchedThreads) bins[c] = 0;
     __syncthreads();
@@ -147,8 +148,8 @@ __global__ __launch_bounds__(kSchedThreads) void schedule_build_kernel(const Sch
     __shared__ int off_a[kSchedMaxSeq + 1], off_b[kSchedMaxSeq + 1], bins[kSchedBins], tmp[kSchedThreads];
     int32_t* q_list = p.out + kSchedHeaderWords;
     int32_t* k_list = q_list + 2 * p.q_slots;
-    build_list<false>(p, p.cu_q1, p.total_q1, p.cu_q2, p.total_q2, p.bm, p.q_slots, q_list, off_a, off_b, bins, tmp);
-    build_list<true>(p, p.cu_k1, p.total_k1, p.cu_k2, p.total_k2, kSchedKeyTile, p.k_slots, k_list, off_a, off_b, bins, tmp);
+    build_list<false>(p, p.cu_q1, p.shift_q1, p.total_q1, p.cu_q2, p.shift_q2, p.total_q2, p.bm, p.q_slots, q_list, off_a, off_b, bins, tmp);
+    build_list<true>(p, p.cu_k1, p.shift_k1, p.total_k1, p.cu_k2, p.shift_k2, p.total_k2, kSchedKeyTile, p.k_slots, k_list, off_a, off_b, bins, tmp);
     if (threadIdx.x < kSchedHeaderWords) {
         int32_t h = 0;
         switch (threadIdx.x) {
@@ -189,7 +190,7 @@ extern "C" int tah_duo_schedule_build(const tah_duo_schedule_args* a, tah_stream
     using namespace tah;
     if (!a || !a->schedule) return TAH_E_NULL;
     if (!sched_shape_ok(a->nseq, a->hq, a->hkv, a->total_q1, a->total_k1, a->total_q2, a->total_k2)) return TAH_E_SHAPE;
-    if (a->nseq > kSchedMaxSeq) return TAH_E_SHAPE;
+    if (a->nseq > kSchedMaxSeq || (a->cu_pairs & ~15)) return TAH_E_SHAPE;
     if ((a->total_q1 > 0 && !a->cu_q1) || (a->total_k1 > 0 && !a->cu_k1) || (a->total_q2 > 0 && (!a->cu_q2 || !a->pos_q2)) ||
         (a->total_k2 > 0 && !a->cu_k2))
         return TAH_E_NULL;
@@ -202,6 +203,7 @@ extern "C" int tah_duo_schedule_build(const tah_duo_schedule_args* a, tah_stream
     p.group = a->hq / a->hkv;
     p.bm = 32 * (8 / p.group);
     p.total_q1 = a->total_q1; p.total_k1 = a->total_k1; p.total_q2 = a->total_q2; p.total_k2 = a->total_k2;
+    p.shift_q1 = a->cu_pairs & 1; p.shift_k1 = a->cu_pairs >> 1 & 1; p.shift_q2 = a->cu_pairs >> 2 & 1; p.shift_k2 = a->cu_pairs >> 3 & 1;
     p.q_slots = sched_slots(a->nseq, p.bm, a->total_q1, a->total_q2);
     p.k_slots = sched_slots(a->nseq, kSchedKeyTile, a->total_k1, a->total_k2);
     p.out = static_cast<int32_t*>(a->schedule);

@@ -66,6 +66,10 @@ void load_library(const std::string& path, bool allow_host) {
     bind(g.sample_rows, "tah_sample_rows");
     bind(g.silu_mul, "tah_silu_mul");
     bind(g.hard_index_build, "tah_hard_index_build");
+    bind(g.mask_index_build, "tah_mask_index_build");
+    bind(g.left_index_build, "tah_left_index_build");
+    bind(g.rows_select, "tah_rows_select");
+    bind(g.zero_gaps, "tah_zero_gaps");
     bind(g.pad_rows_build, "tah_pad_rows_build");
     bind(g.rows_copy, "tah_rows_copy");
     bind(g.embed_rows, "tah_embed_rows");
@@ -123,17 +127,39 @@ const void* schedule_ptr(const optional<Tensor>& schedule) {
     return ptr(*schedule);
 }
 
+// Sequences of a varlen call; `pairs`: which of the four boundary tensors hold (first row, one past the last) pairs (cu_pairs).
+int64_t sequences(const Tensor& cu_q1, const Tensor& cu_k1, const Tensor& cu_q2, const Tensor& cu_k2, int64_t pairs) {
+    TORCH_CHECK(pairs >= 0 && pairs <= 15, "cu_pairs must be a sum of 1, 2, 4 and 8");
+    const int64_t nseq = pairs & 1 ? cu_q1.numel() / 2 : cu_q1.numel() - 1;
+    const Tensor* const cu[] = {&cu_q1, &cu_k1, &cu_q2, &cu_k2};
+    for (int i = 0; i < 4; ++i)
+        TORCH_CHECK(cu[i]->numel() == (pairs >> i & 1 ? 2 * nseq : nseq + 1), "cu_seqlens tensors must all have nseq+1 entries (pairs: 2 nseq)");
+    return nseq;
+}
+
+// Rows between the sequences of padded results: zeros.
+struct Gaps {
+    tah_gap_rows rows[TAH_GAP_TENSORS];
+    int n = 0;
+    void add(bool padded, const Tensor& t, const Tensor& pairs) {
+        if (!padded || t.numel() == 0) return;
+        rows[n++] = {t.data_ptr(), static_cast<const int32_t*>(pairs.data_ptr()), t.stride(0) * (int64_t)t.element_size(), (int32_t)t.size(0)};
+    }
+    void zero(int64_t nseq, tah_stream_t stream) {
+        if (n > 0) check_rc(g.zero_gaps(rows, n, (int32_t)nseq, stream), "tah_zero_gaps");
+    }
+};
+
 // Launch-order table for the varlen calls that use these boundaries (tah_duo_schedule_build).
 Tensor duo_schedule(const Tensor& cu_q1, const Tensor& cu_k1, const Tensor& cu_q2, const Tensor& cu_k2, const Tensor& pos_q2,
-                    int64_t hq, int64_t hkv, int64_t total_q1, int64_t total_k1, int64_t total_k2) {
+                    int64_t hq, int64_t hkv, int64_t total_q1, int64_t total_k1, int64_t total_k2, int64_t pairs) {
     need_lib();
     i32(cu_q1, "cu_q1"); i32(cu_k1, "cu_k1"); i32(cu_q2, "cu_q2"); i32(cu_k2, "cu_k2"); i32(pos_q2, "pos_q2");
     Dev d;
     for (const Tensor* t : {&cu_q1, &cu_k1, &cu_q2, &cu_k2, &pos_q2}) d.see(*t);
-    const int64_t nseq = cu_q1.numel() - 1;
-    TORCH_CHECK(cu_k1.numel() == nseq + 1 && cu_q2.numel() == nseq + 1 && cu_k2.numel() == nseq + 1,
-                "cu_seqlens tensors must all have nseq+1 entries");
+    const int64_t nseq = sequences(cu_q1, cu_k1, cu_q2, cu_k2, pairs);
     tah_duo_schedule_args a{};
+    a.cu_pairs = (int32_t)pairs;
     a.cu_q1 = static_cast<const int32_t*>(cu_q1.data_ptr()); a.cu_k1 = static_cast<const int32_t*>(cu_k1.data_ptr());
     a.cu_q2 = static_cast<const int32_t*>(cu_q2.data_ptr()); a.cu_k2 = static_cast<const int32_t*>(cu_k2.data_ptr());
     a.pos_q2 = static_cast<const int32_t*>(ptr(pos_q2));
@@ -150,16 +176,14 @@ Tensor duo_schedule(const Tensor& cu_q1, const Tensor& cu_k1, const Tensor& cu_q
 std::tuple<Tensor, Tensor, Tensor, Tensor> duo_fwd_varlen(const Tensor& q1, const Tensor& k1, const Tensor& v1, const Tensor& cu_q1,
                                                           const Tensor& cu_k1, const Tensor& q2, const Tensor& k2, const Tensor& v2,
                                                           const Tensor& pos_q2, const Tensor& pos_k2, const Tensor& cu_q2,
-                                                          const Tensor& cu_k2, double scale, const optional<Tensor>& schedule) {
+                                                          const Tensor& cu_k2, double scale, const optional<Tensor>& schedule, int64_t pairs) {
     need_lib();
     thd(q1, "q1"); thd(k1, "k1"); thd(v1, "v1"); thd(q2, "q2"); thd(k2, "k2"); thd(v2, "v2");
     i32(cu_q1, "cu_q1"); i32(cu_k1, "cu_k1"); i32(cu_q2, "cu_q2"); i32(cu_k2, "cu_k2"); i32(pos_q2, "pos_q2"); i32(pos_k2, "pos_k2");
     Dev d;
     for (const Tensor* t : {&q1, &k1, &v1, &q2, &k2, &v2, &cu_q1, &cu_k1, &cu_q2, &cu_k2, &pos_q2, &pos_k2}) d.see(*t);
     d.see(schedule);
-    const int64_t nseq = cu_q1.numel() - 1;
-    TORCH_CHECK(cu_k1.numel() == nseq + 1 && cu_q2.numel() == nseq + 1 && cu_k2.numel() == nseq + 1,
-                "cu_seqlens tensors must all have nseq+1 entries");
+    const int64_t nseq = sequences(cu_q1, cu_k1, cu_q2, cu_k2, pairs);
     TORCH_CHECK(pos_q2.numel() == q2.size(0) && pos_k2.numel() == k2.size(0) && k1.sizes() == v1.sizes() && k2.sizes() == v2.sizes(),
                 "inconsistent row counts");
     const int64_t hq = q1.size(1), dd = q1.size(2);
@@ -172,7 +196,12 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> duo_fwd_varlen(const Tensor& q1, cons
     fill_stream(a.s2, q2, k2, v2, o2, lse2, cu_q2, cu_k2, &pos_q2, &pos_k2);
     a.nseq = (int32_t)nseq; a.hq = (int32_t)hq; a.hkv = (int32_t)k1.size(1); a.d = (int32_t)dd; a.scale = (float)scale;
     a.schedule = schedule_ptr(schedule);
+    a.cu_pairs = (int32_t)pairs;
     check_rc(g.fwd_varlen(&a, d.stream()), "tah_duo_fwd_varlen");
+    Gaps gaps;
+    gaps.add(pairs & 1, o1, cu_q1);
+    gaps.add(pairs & 4, o2, cu_q2);
+    gaps.zero(nseq, d.stream());
     return {o1, lse1, o2, lse2};
 }
 
@@ -189,7 +218,7 @@ std::vector<Tensor> duo_bwd_varlen(const Tensor& q1, const Tensor& k1, const Ten
                                    const Tensor& v2, const Tensor& o2, const Tensor& lse2, const Tensor& do2, const Tensor& pos_q2,
                                    const Tensor& pos_k2, const Tensor& cu_q2, const Tensor& cu_k2, double scale,
                                    const optional<Tensor>& schedule, const optional<Tensor>& ds_workspace,
-                                   int64_t max_seqlen_k1, int64_t max_seqlen_k2) {
+                                   int64_t max_seqlen_k1, int64_t max_seqlen_k2, int64_t pairs) {
     need_lib();
     for (auto p : {std::make_pair(&q1, "q1"), {&k1, "k1"}, {&v1, "v1"}, {&o1, "o1"}, {&do1, "do1"}, {&q2, "q2"}, {&k2, "k2"},
                    {&v2, "v2"}, {&o2, "o2"}, {&do2, "do2"}})
@@ -211,7 +240,7 @@ std::vector<Tensor> duo_bwd_varlen(const Tensor& q1, const Tensor& k1, const Ten
     tah_duo_bwd_args a{};
     fill_stream(a.fwd.s1, q1, k1, v1, o1, lse1, cu_q1, cu_k1, nullptr, nullptr);
     fill_stream(a.fwd.s2, q2, k2, v2, o2, lse2, cu_q2, cu_k2, &pos_q2, &pos_k2);
-    a.fwd.nseq = (int32_t)(cu_q1.numel() - 1); a.fwd.hq = (int32_t)hq; a.fwd.hkv = (int32_t)k1.size(1); a.fwd.d = (int32_t)q1.size(2);
+    a.fwd.nseq = (int32_t)sequences(cu_q1, cu_k1, cu_q2, cu_k2, pairs); a.fwd.cu_pairs = (int32_t)pairs; a.fwd.hq = (int32_t)hq; a.fwd.hkv = (int32_t)k1.size(1); a.fwd.d = (int32_t)q1.size(2);
     a.fwd.scale = (float)scale;
     a.fwd.schedule = schedule_ptr(schedule);
     fill_bwd_stream(a.g1, do1, dq1, dk1, dv1, delta1);
@@ -225,6 +254,14 @@ std::vector<Tensor> duo_bwd_varlen(const Tensor& q1, const Tensor& k1, const Ten
         a.max_seqlen_k2 = (int32_t)max_seqlen_k2;
     }
     check_rc(g.bwd_varlen(&a, d.stream()), "tah_duo_bwd_varlen");
+    Gaps gaps;
+    gaps.add(pairs & 1, dq1, cu_q1);
+    gaps.add(pairs & 2, dk1, cu_k1);
+    gaps.add(pairs & 2, dv1, cu_k1);
+    gaps.add(pairs & 4, dq2, cu_q2);
+    gaps.add(pairs & 8, dk2, cu_k2);
+    gaps.add(pairs & 8, dv2, cu_k2);
+    gaps.zero(a.fwd.nseq, d.stream());
     return {dq1, dk1, dv1, dq2, dk2, dv2};
 }
 
@@ -563,6 +600,74 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> hard_index_build(const Tensor& mask) 
                                 static_cast<int32_t*>(cu.data_ptr()), d.stream()),
              "tah_hard_index_build");
     return {pos, flat, seq, cu};
+}
+
+// (pos, flat, seq, rank, cu and spans one behind the other)
+std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> mask_index_build(const Tensor& mask) {
+    need_lib();
+    Dev d; d.see(mask);
+    TORCH_CHECK(mask.dim() == 2 && (mask.scalar_type() == at::kBool || mask.scalar_type() == at::kByte),
+                "mask must be a (B, S) bool or uint8 tensor");
+    auto m = mask.contiguous();
+    const int64_t B = m.size(0), S = m.size(1), cap = std::max<int64_t>(B * S, 1);
+    auto io = m.options().dtype(at::kInt);
+    auto pos = at::empty({cap}, io), flat = at::empty({cap}, io), seq = at::empty({cap}, io), rank = at::empty({cap}, io);
+    auto info = at::empty({3 * B + 2}, io);
+    tah_mask_index_args a{};
+    a.mask = static_cast<const uint8_t*>(ptr(m)); a.B = (int32_t)B; a.S = (int32_t)S;
+    a.pos = static_cast<int32_t*>(pos.data_ptr()); a.flat = static_cast<int32_t*>(flat.data_ptr()); a.seq = static_cast<int32_t*>(seq.data_ptr());
+    a.rank = static_cast<int32_t*>(rank.data_ptr());
+    a.cu = static_cast<int32_t*>(info.data_ptr()); a.spans = a.cu + B + 1;
+    check_rc(g.mask_index_build(&a, d.stream()), "tah_mask_index_build");
+    return {pos, flat, seq, rank, info};
+}
+
+std::tuple<Tensor, Tensor, Tensor> left_index_build(const Tensor& cu, const Tensor& flat, const Tensor& rank, int64_t S, int64_t width) {
+    need_lib();
+    i32(cu, "cu"); i32(flat, "flat"); i32(rank, "rank");
+    Dev d; d.see(cu); d.see(flat); d.see(rank);
+    const int64_t B = cu.numel() - 1;
+    TORCH_CHECK(B >= 0 && S >= 0 && width >= 0 && rank.numel() >= B * S, "left_index_build: rank must hold B * S entries");
+    auto left = at::empty({B * width}, cu.options()), back = at::empty({B * S}, cu.options());
+    auto pad = at::empty({B, width}, cu.options().dtype(at::kBool));
+    check_rc(g.left_index_build(static_cast<const int32_t*>(cu.data_ptr()), static_cast<const int32_t*>(ptr(flat)), static_cast<const int32_t*>(ptr(rank)),
+                                (int32_t)B, (int32_t)S, (int32_t)width, static_cast<int32_t*>(mptr(left)), static_cast<int32_t*>(mptr(back)),
+                                static_cast<uint8_t*>(mptr(pad)), d.stream()),
+             "tah_left_index_build");
+    return {left, back, pad};
+}
+
+std::vector<Tensor> rows_select(const std::vector<Tensor>& srcs, const Tensor& index, int64_t rows, const optional<Tensor>& n_dev) {
+    need_lib();
+    i32(index, "index");
+    Dev d; d.see(index); d.see(n_dev);
+    TORCH_CHECK(rows >= 0 && index.numel() >= rows && rows < (1ll << 31), "rows_select: index must hold an entry per row of the results");
+    TORCH_CHECK(srcs.size() <= TAH_SELECT_TENSORS, "rows_select: at most ", TAH_SELECT_TENSORS, " tensors");
+    std::vector<Tensor> out, copies;  // (copies: kept until the launch is in)
+    tah_select_rows moves[TAH_SELECT_TENSORS];
+    for (const Tensor& src : srcs) {
+        d.see(src);
+        TORCH_CHECK(src.dim() >= 1, "rows_select: tensors of rows");
+        auto sizes = src.sizes().vec();
+        sizes[0] = rows;
+        // rows that are not contiguous: those of a copy
+        int64_t elems = 1;
+        bool whole = true;
+        for (int64_t i = src.dim() - 1; i > 0; --i) {
+            whole = whole && (src.size(i) == 1 || src.stride(i) == elems);
+            elems *= src.size(i);
+        }
+        if (!whole) copies.push_back(src.contiguous());
+        const Tensor& from = whole ? src : copies.back();
+        auto to = at::empty(sizes, src.options());
+        const int64_t es = (int64_t)src.element_size();
+        moves[out.size()] = {ptr(from), mptr(to), elems * es, (from.size(0) > 1 ? from.stride(0) : elems) * es};
+        out.push_back(to);
+    }
+    check_rc(g.rows_select(moves, (int32_t)out.size(), static_cast<const int32_t*>(index.data_ptr()), (int32_t)rows, static_cast<const int32_t*>(ptr(n_dev)),
+                           d.stream()),
+             "tah_rows_select");
+    return out;
 }
 
 Tensor pad_rows_build(const Tensor& cu, const Tensor& seq_of, int64_t n, int64_t width, const optional<Tensor>& n_dev,
@@ -1088,6 +1193,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("kv_append", &kv_append);
     m.def("qk_prep", &qk_prep);
     m.def("hard_index_build", &hard_index_build);
+    m.def("mask_index_build", &mask_index_build);
+    m.def("left_index_build", &left_index_build);
+    m.def("rows_select", &rows_select);
     m.def("pad_rows_build", &pad_rows_build);
     m.def("rows_copy", &rows_copy);
     m.def("topk_mix", &topk_mix);

@@ -64,6 +64,10 @@ struct Api {
     Entry<decltype(&tah_sample_rows)> sample_rows;
     Entry<decltype(&tah_silu_mul)> silu_mul;
     Entry<decltype(&tah_hard_index_build)> hard_index_build;
+    Entry<decltype(&tah_mask_index_build)> mask_index_build;
+    Entry<decltype(&tah_left_index_build)> left_index_build;
+    Entry<decltype(&tah_rows_select)> rows_select;
+    Entry<decltype(&tah_zero_gaps)> zero_gaps;
     Entry<decltype(&tah_pad_rows_build)> pad_rows_build;
     Entry<decltype(&tah_rows_copy)> rows_copy;
     Entry<decltype(&tah_embed_rows)> embed_rows;

@@ -223,7 +223,7 @@ __global__ __launch_bounds__(kTileThreads) TAH_WAVES_PER_EU(NQ <= 4 ? 2 : 1, 8) 
     if (g >= L.kv_heads) return;
     const int hpt = p.heads_per_tile, h0 = g * per + (gc % p.chunks) * hpt, h_end = (g + 1) * per;
     const int ptiles = kTileQueries / hpt;  // tiles of 16 positions
-    if (!find_tile(p.c.P.cu, p.c.P.nseq, 16 * ptiles, tile, b, row0, row_end)) return;
+    if (!find_tile(p.c.P.cu, 0, p.c.P.nseq, 16 * ptiles, tile, b, row0, row_end)) return;
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, c = lane % 16, gq = lane / 16;
     const int nq = kExact ? NQ : L.key_dim / 32, nv = kExact ? NV : L.value_dim / 16;
     const int ks = tile_stride(L.row), koff = L.row - L.key_dim;

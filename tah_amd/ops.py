@@ -26,29 +26,33 @@ lib = _lib.lib  # the extension with the library loaded (kernel objects: Portion
 MAX_SCHEDULE_SEQS = 4095
 
 
-def duo_schedule(cu_q1, cu_k1, cu_q2, cu_k2, pos_q2, hq: int, hkv: int, total_q1: int, total_k1: int, total_k2: int):
+def duo_schedule(cu_q1, cu_k1, cu_q2, cu_k2, pos_q2, hq: int, hkv: int, total_q1: int, total_k1: int, total_k2: int, pairs: int = 0):
     """Launch-order table for the varlen calls over these boundaries: every tile of both depths, heaviest first.
 
     Built on the device from the boundary tensors (no read-back); pass it as ``schedule=`` to :func:`duo_fwd_varlen` /
     :func:`duo_bwd_varlen` for as long as the boundaries, ``pos_q2`` and the row counts stay the same -- one table
     serves every layer and the backward pass of a batch.  It only changes the order in which tiles are started.
+    ``pairs``: as in :func:`duo_fwd_varlen`.
     Returns ``None`` for a single sequence (its tiles are already in that order) or more than 4095 sequences.
     """
-    nseq = cu_q1.numel() - 1
+    nseq = cu_q1.numel() // 2 if pairs & 1 else cu_q1.numel() - 1
     if nseq <= 1 or nseq > MAX_SCHEDULE_SEQS:
         return None
-    return _call("duo_schedule", cu_q1, cu_k1, cu_q2, cu_k2, pos_q2, int(hq), int(hkv), int(total_q1), int(total_k1), int(total_k2))
+    return _call("duo_schedule", cu_q1, cu_k1, cu_q2, cu_k2, pos_q2, int(hq), int(hkv), int(total_q1), int(total_k1), int(total_k2), int(pairs))
 
 
-def duo_fwd_varlen(q1, k1, v1, cu_q1, cu_k1, q2, k2, v2, pos_q2, pos_k2, cu_q2, cu_k2, scale: float, schedule=None
-                   ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+def duo_fwd_varlen(q1, k1, v1, cu_q1, cu_k1, q2, k2, v2, pos_q2, pos_k2, cu_q2, cu_k2, scale: float, schedule=None,
+                   pairs: int = 0) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """Duo-causal attention forward on packed varlen bf16 tensors.
 
     q1 [T1q,Hq,D], k1/v1 [T1k,Hkv,D], cu_q1/cu_k1 int32 [nseq+1]: depth-0 stream.
     q2 [T2q,Hq,D], k2/v2 [T2k,Hkv,D], pos_q2/pos_k2 int32, cu_q2/cu_k2: depth-1 stream
-    (hard tokens).  ``schedule``: table from :func:`duo_schedule` or None.  Returns o1, lse1 [Hq,T1q], o2, lse2 [Hq,T2q].
+    (hard tokens).  ``schedule``: table from :func:`duo_schedule` or None.  ``pairs``: the sum of 1, 2, 4, 8 for
+    cu_q1, cu_k1, cu_q2, cu_k2 that hold (first row, one past the last) pairs, int32 [2 * nseq], ascending, with rows in between that
+    belong to no sequence: what they hold is not read, their rows of o are zeros (of lse undefined).
+    Returns o1, lse1 [Hq,T1q], o2, lse2 [Hq,T2q].
     """
-    return _call("duo_fwd_varlen", q1, k1, v1, cu_q1, cu_k1, q2, k2, v2, pos_q2, pos_k2, cu_q2, cu_k2, float(scale), schedule)
+    return _call("duo_fwd_varlen", q1, k1, v1, cu_q1, cu_k1, q2, k2, v2, pos_q2, pos_k2, cu_q2, cu_k2, float(scale), schedule, int(pairs))
 
 
 # The backward pass can hand dS from the dK/dV kernel to the dQ kernel through a workspace instead of computing the
@@ -78,23 +82,23 @@ def _ds_workspace(device, nbytes: int):
 
 
 def duo_bwd_varlen(q1, k1, v1, o1, lse1, do1, cu_q1, cu_k1, q2, k2, v2, o2, lse2, do2, pos_q2, pos_k2, cu_q2, cu_k2,
-                   scale: float, schedule=None, ds_workspace=None, max_seqlen_k1: int = 0, max_seqlen_k2: int = 0):
+                   scale: float, schedule=None, ds_workspace=None, max_seqlen_k1: int = 0, max_seqlen_k2: int = 0, pairs: int = 0):
     """Backward of :func:`duo_fwd_varlen`; returns dq1, dk1, dv1, dq2, dk2, dv2 (bf16).
 
     ``ds_workspace``: a uint8 tensor of at least :func:`duo_bwd_workspace_bytes` bytes, ``False`` for the three-kernel
     backward, or None: the package's own buffer when ``DS_EXCHANGE`` is on and the call fits ``DS_EXCHANGE_MAX_BYTES``.
     ``max_seqlen_k1`` / ``max_seqlen_k2``: upper bounds on one sequence's key rows per depth (0: unknown); they only
-    make the workspace smaller.
+    make the workspace smaller.  ``pairs``: as in :func:`duo_fwd_varlen` (gradients of rows in between are zeros).
     """
     if ds_workspace is None and DS_EXCHANGE:
-        need = duo_bwd_workspace_bytes(cu_q1.numel() - 1, q1.shape[1], k1.shape[1], q1.shape[0], k1.shape[0], q2.shape[0],
+        need = duo_bwd_workspace_bytes(cu_q1.numel() // 2 if pairs & 1 else cu_q1.numel() - 1, q1.shape[1], k1.shape[1], q1.shape[0], k1.shape[0], q2.shape[0],
                                        k2.shape[0], max_seqlen_k1, max_seqlen_k2)
         if 0 < need <= DS_EXCHANGE_MAX_BYTES:
             ds_workspace = _ds_workspace(q1.device, need)
     if ds_workspace is False:
         ds_workspace = None
     return tuple(_call("duo_bwd_varlen", q1, k1, v1, o1, lse1, do1, cu_q1, cu_k1, q2, k2, v2, o2, lse2, do2, pos_q2, pos_k2,
-                       cu_q2, cu_k2, float(scale), schedule, ds_workspace, int(max_seqlen_k1), int(max_seqlen_k2)))
+                       cu_q2, cu_k2, float(scale), schedule, ds_workspace, int(max_seqlen_k1), int(max_seqlen_k2), int(pairs)))
 
 
 def duo_fwd_masked(q, k, v, mask, nseq: int, scale: float):
@@ -117,6 +121,25 @@ def hard_index_build(mask: torch.Tensor):
     Only the first cu[B] entries of pos/flat/seq are defined.  No host sync.
     """
     return _call("hard_index_build", mask)
+
+
+def mask_index_build(mask: torch.Tensor):
+    """:func:`hard_index_build` and, from the same launch, rank int32 [B*S cap] (an entry's number, -1: none); the boundaries
+    come in one int32 tensor [3 B + 2]: ``cu``, then B pairs (flat index of the row's first True entry, that plus their number), then 1
+    if some row's True entries do not lie together.  Returns pos, flat, seq, rank, boundaries.  No host sync."""
+    return _call("mask_index_build", mask)
+
+
+def left_index_build(cu: torch.Tensor, flat: torch.Tensor, rank: torch.Tensor, S: int, width: int):
+    """The right-padded (B, width) form of a mask's entries as tables: left int32 [B*width] (flat index of the entry there), back
+    int32 [B*S] (its place), both -1 where there is none, and the padding, bool [B, width]."""
+    return _call("left_index_build", cu, flat, rank, int(S), int(width))
+
+
+def rows_select(srcs, index: torch.Tensor, rows: int, n_dev: Optional[torch.Tensor] = None):
+    """Rows of up to six tensors by one table, one launch: out[r] = src[index[r]] for r < rows, zeros where index[r] < 0.  ``n_dev``
+    (device int32, one element): results from there on are undefined."""
+    return _call("rows_select", list(srcs), index, int(rows), n_dev)
 
 
 def pad_rows_build(cu: torch.Tensor, seq_of: torch.Tensor, n: int, width: int, n_dev: Optional[torch.Tensor] = None,

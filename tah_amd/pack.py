@@ -23,6 +23,9 @@ from ._capi import TahDuoError
 HOST_SYNC = True
 
 
+# Tensors that one launch moves at most (TAH_SELECT_TENSORS).
+MOVE_TENSORS = 6
+
 # The index of a mask is asked for several times within one model step (queries and keys of an attention call pack by
 # the same valid mask; scatter_back follows gather_active with the same mask): the last few are kept, keyed by the
 # mask tensor itself and its version counter, so that each mask is compacted -- and its count read back -- once.
@@ -35,11 +38,14 @@ class HardIndex:
 
     pos[r]  position (column) of the r-th True entry in row-major order (int32)
     flat[r] its flat index b*S + s, seq[r] its row b, cu[b] entries before row b
+    rank[b*S + s] that entry's r, -1 where the mask is False
     n, width: total count and the largest per-row count (host ints; reading them
     is the one host sync of the pack, as in tah_model.py:116).  With ``sync=False``
     nothing is read back: ``n`` and ``width`` are None, ``n_max`` = B*S bounds the
     count, ``count`` is the count on the device (one int32) and pos / flat / seq keep
     their full capacity (entries past the count are undefined).
+    intervals  int32 [2 B] on the device, (flat index of the row's first True entry, that plus their number), if every row's
+    True entries lie together (a padded batch); None if they do not, or nothing is read back.
     """
 
     @classmethod
@@ -62,19 +68,21 @@ class HardIndex:
             mask = mask != 0
         self.B, self.S = mask.shape
         self.mask = mask.contiguous()
-        pos, flat, seq, cu = ops.hard_index_build(self.mask)
-        self.cu = cu
+        pos, flat, seq, self.rank, info = ops.mask_index_build(self.mask)
+        cu = self.cu = info[: self.B + 1]
         self.count = cu[self.B:]
         self.n_max = self.B * self.S
         self.synced = HOST_SYNC if sync is None else sync
         if self.synced:
-            cu_host = cu.cpu()
+            host = info.cpu()
+            cu_host = host[: self.B + 1]
+            self.intervals = None if int(host[-1]) else info[self.B + 1: 3 * self.B + 1]
             self.n = int(cu_host[-1])
             counts = cu_host[1:] - cu_host[:-1]
             self.width = int(counts.max()) if self.B > 0 else 0
             self.pos, self.flat, self.seq = pos[: self.n], flat[: self.n], seq[: self.n]
         else:
-            self.n = self.width = None
+            self.n = self.width = self.intervals = None
             self.pos, self.flat, self.seq = pos[: self.n_max], flat[: self.n_max], seq[: self.n_max]
         self._pad_rows: Optional[torch.Tensor] = None
 
@@ -132,6 +140,28 @@ class _RowsMove(torch.autograd.Function):
         return grad_src, None, None, None, None, None, None, None
 
 
+class _RowsSelect(torch.autograd.Function):
+    """out[r] = src[index[r]], zeros where that is negative, for several tensors in one launch.  ``back``: the table of the other
+    direction (every source row goes to one row of the result at most)."""
+
+    @staticmethod
+    def forward(ctx, index, rows, back, *srcs):
+        ctx.save_for_backward(back)
+        ctx.totals = [s.shape[0] for s in srcs]
+        out = ops.rows_select(srcs, index, rows)
+        ctx.mark_non_differentiable(*[o for i, o in enumerate(out) if not ctx.needs_input_grad[3 + i]])
+        return tuple(out)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        (back,) = ctx.saved_tensors
+        at = [i for i in range(len(grads)) if ctx.needs_input_grad[3 + i]]
+        out = [None] * len(grads)
+        for i, g in zip(at, ops.rows_select([grads[i] for i in at], back, ctx.totals[at[0]]) if at else ()):
+            out[i] = g
+        return (None, None, None, *out)
+
+
 def _flat_rows(t: torch.Tensor, lead: int) -> torch.Tensor:
     """(B, S, ...) -> (B*S, ...) contiguous; 2-D tensors become (B*S, 1)."""
     t = t.contiguous()
@@ -156,6 +186,17 @@ def gather_active(current_iter_mask: torch.Tensor, *tensors, pad_value=0, max_ac
         raise TahDuoError("gather_active: with tah_amd.pack.HOST_SYNC = False the packed width must be given (max_active)")
     idx = HardIndex.of(current_iter_mask, sync=max_active is None)
     B, S = idx.B, idx.S
+    given = [t for t in tensors if t is not None]
+    if max_active is None and pad_value == 0 and idx.n and len(given) <= MOVE_TENSORS:
+        # one launch for the tables and the padding, one for all tensors: the host's time here stands between a model's two iterations,
+        # behind the read-back of the width (two tables, three tensors as clears and copies: eleven launches, 0.25 ms of the host)
+        for t in given:
+            if t.shape[0] != B or t.shape[1] != S:
+                raise TahDuoError(f"gather_active: tensor shape {tuple(t.shape)} does not start with ({B}, {S})")
+        W = idx.width
+        left, back, pad_mask = ops.left_index_build(idx.cu, idx.flat, idx.rank, S, W)
+        moved = iter(_RowsSelect.apply(left, B * W, back, *[_flat_rows(t, B * S) for t in given]) if given else ())
+        return (pad_mask, *[None if t is None else next(moved).view(B, W, *t.shape[2:]) for t in tensors])
     overflow = None
     if max_active is None:
         W, n, n_dev, pad_rows = idx.width, idx.n, None, (idx.pad_rows if idx.n else None)
