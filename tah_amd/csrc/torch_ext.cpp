@@ -400,6 +400,28 @@ void duo_decode(const Tensor& q, const Tensor& o, const optional<Tensor>& lse, c
     }
 }
 
+// The same with results and workspace from torch's allocator, in one crossing from Python: a call of a few sequences is two launches of 10 us
+// together, and the host took 11 for it (a call for the workspace's size, the stream, two allocations and a table of workspaces from
+// Python); 8 now.
+std::tuple<Tensor, optional<Tensor>> duo_decode_alloc(const Tensor& q, const Tensor& q_slot, const Tensor& q_pos, const optional<Tensor>& q_depth,
+                                                      int64_t depth, const Tensor& k1, const Tensor& v1, const Tensor& start1, const Tensor& len1,
+                                                      const optional<Tensor>& k2, const optional<Tensor>& v2, const optional<Tensor>& pos2,
+                                                      const optional<Tensor>& start2, const optional<Tensor>& len2, double scale, bool want_lse) {
+    need_lib();
+    thd(q, "q");
+    Tensor o = at::empty({q.size(0), q.size(1), q.size(2)}, q.options());
+    optional<Tensor> lse;
+    if (want_lse) lse = at::empty({q.size(0), q.size(1)}, q.options().dtype(at::kFloat));
+    Dev d;
+    tah_duo_decode_args a = decode_args(d, q, o, lse, q_slot, q_pos, q_depth, depth, k1, v1, start1, len1, k2, v2, pos2, start2, len2, scale, c10::nullopt);
+    const int64_t bytes = (int64_t)g.decode_workspace_bytes(a.nq, a.hq, a.c1.capacity, a.c2.capacity);
+    const Tensor workspace = at::empty({std::max<int64_t>(bytes, 16)}, q.options().dtype(at::kByte));
+    a.workspace = workspace.data_ptr();
+    a.workspace_bytes = (size_t)workspace.numel();
+    check_rc(g.decode(&a, d.stream()), "tah_duo_decode");
+    return {o, lse};
+}
+
 void kv_append(const Tensor& k_new, const Tensor& v_new, const Tensor& cu_new, const optional<Tensor>& pos_new,
                const optional<Tensor>& slot_of, const Tensor& ck, const Tensor& cv, const optional<Tensor>& cpos, const Tensor& start,
                const Tensor& len, const Tensor& overflow) {
@@ -1189,6 +1211,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("duo_fwd_masked", &duo_fwd_masked);
     m.def("duo_bwd_masked", &duo_bwd_masked);
     m.def("decode_workspace_bytes", &decode_workspace_bytes);
+    m.def("duo_decode_alloc", &duo_decode_alloc);
     m.def("duo_decode", &duo_decode);
     m.def("kv_append", &kv_append);
     m.def("qk_prep", &qk_prep);

@@ -181,10 +181,15 @@ def decode(q: torch.Tensor, q_slot: torch.Tensor, q_pos: torch.Tensor, c1: KvSla
     """
     if q.dim() != 3:
         raise _capi.TahDuoError("decode: q must be [nq, Hq, D]")
-    nq, hq, d = q.shape
     need2 = q_depth is not None or depth >= 1
     if need2 and c2 is None:
         raise _capi.TahDuoError("depth-1 queries need the depth-1 cache")
+    two = (c2.k, c2.v, c2.pos, c2.start, c2.len) if need2 else (None,) * 5
+    if out is None and lse_out is None and out_packed is None and not static_scratch:
+        o, lse = _call("duo_decode_alloc", q, q_slot, q_pos, q_depth, int(depth), c1.k, c1.v, c1.start, c1.len, *two, float(scale),
+                       return_lse)
+        return (o, lse) if return_lse else o
+    nq, hq, d = q.shape
     o = out if out is not None else torch.empty((nq, hq, d), dtype=q.dtype, device=q.device)
     if o.shape != (nq, hq, d) or o.dtype != q.dtype or o.stride(2) != 1:
         raise _capi.TahDuoError("decode: out must be a [nq, Hq, D] tensor of q's dtype")
@@ -197,7 +202,6 @@ def decode(q: torch.Tensor, q_slot: torch.Tensor, q_pos: torch.Tensor, c1: KvSla
         if ws is None or ws.numel() < nbytes:
             ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=q.device)
             _WORKSPACES[key] = ws
-    two = (c2.k, c2.v, c2.pos, c2.start, c2.len) if need2 else (None,) * 5
     _call("duo_decode", q, o, lse, q_slot, q_pos, q_depth, int(depth), c1.k, c1.v, c1.start, c1.len, *two, ws, float(scale),
           out_packed)
     return (o, lse) if return_lse else o
