@@ -13,7 +13,7 @@
 //  * moe_plain_kernel: the same product in float32 arithmetic (the float32 form of a model).
 #include <hip/hip_runtime.h>
 
-#include "mixer_device.h"
+#include "residual_row.h"
 
 namespace tah {
 namespace {
@@ -25,6 +25,100 @@ constexpr int kGroupsPerLane = 4;  // groups of experts: at most 256
 constexpr int kUnitsHeld = 4;      // scores per lane that the selection keeps in registers (256 experts)
 constexpr int kTile = TAH_MOE_TILE;
 
+// One row's experts from its logits, by one wave.  zr: the logits in LDS, behind them the shared expert's where there is a gate.
+__device__ __forceinline__ void choose_experts(const tah_moe_route_args& p, float* const zr, int row, int lane) {
+    const int experts = p.experts, top = p.top;
+            if (p.gate_w && lane == 0) p.shared_gate[row] = sigmoid_exact(zr[experts]);
+            if (p.score == TAH_MOE_SIGMOID) {
+                for (int e = lane; e < experts; e += kWave) zr[e] = sigmoid_exact(zr[e]);
+                TAH_WAVE_LDS_SYNC();
+            }
+            if (p.keep < p.groups) {
+                // a lane's groups: the sum of their two largest scores; then the best groups one after another, and the others'
+                // experts leave the race
+                const int size = experts / p.groups;
+                float gs[kGroupsPerLane];
+    #pragma unroll
+                for (int u = 0; u < kGroupsPerLane; ++u) {
+                    const int gr = lane + kWave * u;
+                    float a = kNegInf, b = kNegInf;
+                    for (int i = 0; gr < p.groups && i < size; ++i) {
+                        const float v = zr[gr * size + i];
+                        b = fmaxf(b, fminf(a, v));
+                        a = fmaxf(a, v);
+                    }
+                    gs[u] = gr < p.groups ? (size > 1 ? a + b : a) : kNegInf;
+                }
+                uint32_t open = 0;  // bit u: group lane + 64 u is open
+                if (p.groups <= kWave) {  // a lane's group is open when fewer than `keep` are in front of it
+                    int before = 0;
+                    for (int g = 0; g < p.groups; ++g) {
+                        const float o = lane_value(gs[0], g);
+                        before += o > gs[0] || (o == gs[0] && g < lane);
+                    }
+                    open = gs[0] > kNegInf && before < p.keep;
+                } else for (int j = 0; j < p.keep; ++j) {
+                    float bv = kNegInf;
+                    int bi = 0x7fffffff;
+    #pragma unroll
+                    for (int u = 0; u < kGroupsPerLane; ++u)
+                        if (!(open >> u & 1) && gs[u] > bv) { bv = gs[u]; bi = lane + kWave * u; }
+    #pragma unroll
+                    for (int m = 32; m >= 1; m >>= 1) {
+                        const float ov = __shfl_xor(bv, m);
+                        const int oi = __shfl_xor(bi, m);
+                        if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
+                    }
+                    if (bi % kWave == lane && bi < p.groups) open |= 1u << (bi / kWave);
+                }
+    #pragma unroll
+                for (int u = 0; u < kGroupsPerLane; ++u) {
+                    const int gr = lane + kWave * u;
+                    for (int i = 0; gr < p.groups && !(open >> u & 1) && i < size; ++i) zr[gr * size + i] = kNegInf;
+                }
+                TAH_WAVE_LDS_SYNC();
+            }
+            // the largest scores one after another, the lower index among equals; a chosen one leaves the race
+            float mine = kNegInf, first = 0.f;
+            int my_index = 0;
+            float v[kUnitsHeld];  // scores of experts lane, lane + 64, ... while they are in the race
+    #pragma unroll
+            for (int u = 0; u < kUnitsHeld; ++u) v[u] = lane + kWave * u < experts ? zr[lane + kWave * u] : kNegInf;
+            const bool held = experts <= kUnitsHeld * kWave;
+            for (int j = 0; j < top; ++j) {
+                float bv = kNegInf;
+                int bi = 0x7fffffff;
+                if (held) {
+    #pragma unroll
+                    for (int u = 0; u < kUnitsHeld; ++u)
+                        if (v[u] > bv) { bv = v[u]; bi = lane + kWave * u; }
+                } else {
+                    for (int e = lane; e < experts; e += kWave) {
+                        const float o = zr[e];
+                        if (o > bv) { bv = o; bi = e; }
+                    }
+                }
+                const float largest = wave_max_quick(bv);
+                bi = wave_min_quick(bv == largest ? bi : 0x7fffffff);
+                if (bi >= experts) bi = j;  // (only when the logits are not numbers)
+                if (j == 0) first = largest;
+                if (lane == j) { mine = largest; my_index = bi; }
+                if (held) {
+    #pragma unroll
+                    for (int u = 0; u < kUnitsHeld; ++u) v[u] = lane + kWave * u == bi ? kNegInf : v[u];
+                } else {
+                    if (lane == 0) zr[bi] = kNegInf;
+                    TAH_WAVE_LDS_SYNC();
+                }
+            }
+            const float w = lane < top ? expf(mine - first) : 0.f;
+            const float sum = wave_sum(w);
+            if (lane < top) {
+                p.index[(int64_t)row * top + lane] = my_index;
+                p.weight[(int64_t)row * top + lane] = p.score == TAH_MOE_SIGMOID ? mine : w / sum;
+            }
+}
+
 // LDS: rows [RB][cols] float32, logits [RB][experts + 1]
 template <class X, class E, int RB, int EB, int kThreads>
 __global__ __launch_bounds__(kThreads) void moe_route_kernel(const tah_moe_route_args p) {
@@ -32,7 +126,7 @@ __global__ __launch_bounds__(kThreads) void moe_route_kernel(const tah_moe_route
     const X* const x = static_cast<const X*>(p.x);
     const E* const router = static_cast<const E*>(p.router);
     const E* const gate_w = static_cast<const E*>(p.gate_w);
-    const int rows = p.rows, cols = p.cols, experts = p.experts, top = p.top;
+    const int rows = p.rows, cols = p.cols, experts = p.experts;
     float* const xs = sm;
     float* const z = sm + RB * cols;
     constexpr int kWaves = kThreads / kWave;
@@ -82,96 +176,87 @@ __global__ __launch_bounds__(kThreads) void moe_route_kernel(const tah_moe_route
         const int row = row0 + r;
         if (row >= rows) break;
         float* const zr = z + r * zs;
-        if (gate_w && lane == 0) p.shared_gate[row] = sigmoid_exact(zr[experts]);
-        if (p.score == TAH_MOE_SIGMOID) {
-            for (int e = lane; e < experts; e += kWave) zr[e] = sigmoid_exact(zr[e]);
-            TAH_WAVE_LDS_SYNC();
-        }
-        if (p.keep < p.groups) {
-            // a lane's groups: the sum of their two largest scores; then the best groups one after another, and the others'
-            // experts leave the race
-            const int size = experts / p.groups;
-            float gs[kGroupsPerLane];
+        choose_experts(p, zr, row, lane);
+    }
+}
+
+// ---- the norm in front of a router and the router in one launch ---------------------------------------------
+// A few rows of a decode step: a workgroup makes its row's norm, leaves what the experts read and chooses them.  Two launches of 4.7 and
+// 10.4 us (64 experts and a shared one's gate, 2048 columns, one row or eight in a captured step) were each a chain of trips to memory, the
+// second one bounded by what one compute unit's L1 takes in (266 KB of weights, 2 us) behind the row's trip.  Here the row's loads
+// go first and all of the router's weights behind them, in registers (PER experts a wave, kRouteBlocks loads each), on their way while the norm
+// is made: 10.7 and 10.5 us (1 row, 8 rows); what is left is the products' vector work (2 us) and the choice.  Same arithmetic in the same order as the two: the same bits.
+constexpr int kNormRouteThreads = 512, kRouteWaves = kNormRouteThreads / kWave;
+constexpr int kRouteBlocks = 4;       // of 512 columns: rows of up to 2048 (a unit of eight columns per thread of the norm)
+constexpr int kNormRouteExperts = 9;  // per wave: 72 with the gate, as many as leave registers for the norm
+constexpr int kNormRouteRows = 32;
+
+struct NormRoute {
+    tah_residual_norm_args n;
+    tah_moe_route_args r;
+    float* x_out;
+};
+
+template <bool GROUPS, int PER>
+__global__ __launch_bounds__(kNormRouteThreads) void moe_norm_route_kernel(const NormRoute p) {
+    __shared__ __align__(16) float xs[kRouteBlocks * 8 * kWave];
+    __shared__ float z[kRouteWaves * kNormRouteExperts];
+    __shared__ ResidualLds<1, GROUPS> lds[kNormRouteThreads / kRowThreads];
+    const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, row = blockIdx.x, part = tid / kRowThreads;
+    const int cols = p.r.cols, experts = p.r.experts, total = experts + (p.r.gate_w ? 1 : 0);
+    const __bf16* const router = static_cast<const __bf16*>(p.r.router);
+    bf16x8 w[PER][kRouteBlocks];
+    tah_residual_norm_args n = p.n;
+    n.experts = nullptr;
+    n.conv = nullptr;
+    const bool normed = n.next_coef != nullptr;
+    // (both halves of the workgroup make the row; one stores it)
+    residual_row<__bf16, 1, GROUPS, true>(
+        n, row, tid % kRowThreads, lds[part], part == 0, p.x_out,
+        [&]() __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int u = 0; u < kGroupsPerLane; ++u) {
-                const int gr = lane + kWave * u;
-                float a = kNegInf, b = kNegInf;
-                for (int i = 0; gr < p.groups && i < size; ++i) {
-                    const float v = zr[gr * size + i];
-                    b = fmaxf(b, fminf(a, v));
-                    a = fmaxf(a, v);
-                }
-                gs[u] = gr < p.groups ? (size > 1 ? a + b : a) : kNegInf;
-            }
-            uint32_t open = 0;  // bit u: group lane + 64 u is open
-            if (p.groups <= kWave) {  // a lane's group is open when fewer than `keep` are in front of it
-                int before = 0;
-                for (int g = 0; g < p.groups; ++g) {
-                    const float o = lane_value(gs[0], g);
-                    before += o > gs[0] || (o == gs[0] && g < lane);
-                }
-                open = gs[0] > kNegInf && before < p.keep;
-            } else for (int j = 0; j < p.keep; ++j) {
-                float bv = kNegInf;
-                int bi = 0x7fffffff;
+            for (int x = 0; x < PER; ++x) {
+                const int e = wave * PER + x;
+                const __bf16* const from = e < experts ? router + (int64_t)e * cols : (e < total ? static_cast<const __bf16*>(p.r.gate_w) : router);
 #pragma unroll
-                for (int u = 0; u < kGroupsPerLane; ++u)
-                    if (!(open >> u & 1) && gs[u] > bv) { bv = gs[u]; bi = lane + kWave * u; }
-#pragma unroll
-                for (int m = 32; m >= 1; m >>= 1) {
-                    const float ov = __shfl_xor(bv, m);
-                    const int oi = __shfl_xor(bi, m);
-                    if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-                }
-                if (bi % kWave == lane && bi < p.groups) open |= 1u << (bi / kWave);
-            }
-#pragma unroll
-            for (int u = 0; u < kGroupsPerLane; ++u) {
-                const int gr = lane + kWave * u;
-                for (int i = 0; gr < p.groups && !(open >> u & 1) && i < size; ++i) zr[gr * size + i] = kNegInf;
-            }
-            TAH_WAVE_LDS_SYNC();
-        }
-        // the largest scores one after another, the lower index among equals; a chosen one leaves the race
-        float mine = kNegInf, first = 0.f;
-        int my_index = 0;
-        float v[kUnitsHeld];  // scores of experts lane, lane + 64, ... while they are in the race
-#pragma unroll
-        for (int u = 0; u < kUnitsHeld; ++u) v[u] = lane + kWave * u < experts ? zr[lane + kWave * u] : kNegInf;
-        const bool held = experts <= kUnitsHeld * kWave;
-        for (int j = 0; j < top; ++j) {
-            float bv = kNegInf;
-            int bi = 0x7fffffff;
-            if (held) {
-#pragma unroll
-                for (int u = 0; u < kUnitsHeld; ++u)
-                    if (v[u] > bv) { bv = v[u]; bi = lane + kWave * u; }
-            } else {
-                for (int e = lane; e < experts; e += kWave) {
-                    const float o = zr[e];
-                    if (o > bv) { bv = o; bi = e; }
+                for (int b = 0; b < kRouteBlocks; ++b) {
+                    const int c = 8 * lane + 8 * kWave * b;
+                    w[x][b] = *reinterpret_cast<const bf16x8*>(from + (c < cols ? c : 0));
                 }
             }
-            const float largest = wave_max_quick(bv);
-            bi = wave_min_quick(bv == largest ? bi : 0x7fffffff);
-            if (bi >= experts) bi = j;  // (only when the logits are not numbers)
-            if (j == 0) first = largest;
-            if (lane == j) { mine = largest; my_index = bi; }
-            if (held) {
+            __builtin_amdgcn_sched_barrier(0);
+        },
+        [&](int c, const float (&v)[8]) __attribute__((always_inline)) {
+            if (part != 0) return;
+            float y[8];
 #pragma unroll
-                for (int u = 0; u < kUnitsHeld; ++u) v[u] = lane + kWave * u == bi ? kNegInf : v[u];
-            } else {
-                if (lane == 0) zr[bi] = kNegInf;
-                TAH_WAVE_LDS_SYNC();
-            }
-        }
-        const float w = lane < top ? expf(mine - first) : 0.f;
-        const float sum = wave_sum(w);
-        if (lane < top) {
-            p.index[(int64_t)row * top + lane] = my_index;
-            p.weight[(int64_t)row * top + lane] = p.score == TAH_MOE_SIGMOID ? mine : w / sum;
+            for (int i = 0; i < 8; ++i) y[i] = normed ? (float)(__bf16)v[i] : v[i];  // (as the router reads the row from memory)
+            store8(xs + c, y);
+        });
+    __syncthreads();
+    float s[PER];
+#pragma unroll
+    for (int x = 0; x < PER; ++x) s[x] = 0.f;
+#pragma unroll
+    for (int b = 0; b < kRouteBlocks; ++b) {
+        const int c = 8 * lane + 8 * kWave * b;
+        if (c < cols) {
+            float y[8];
+            load8(xs + c, y);
+#pragma unroll
+            for (int x = 0; x < PER; ++x)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) s[x] += (float)w[x][b][i] * y[i];
         }
     }
+#pragma unroll
+    for (int x = 0; x < PER; ++x) {
+        const float t = wave_sum_tree(s[x]);
+        if (lane == 0 && wave * PER + x < total) z[wave * PER + x] = t;
+    }
+    __syncthreads();
+    if (wave == 0) choose_experts(p.r, z, row, lane);
 }
 
 constexpr int kPlanThreads = 1024;
@@ -434,6 +519,18 @@ void launch_route(const tah_moe_route_args& a, hipStream_t st) {
         hipLaunchKernelGGL((moe_route_kernel<X, E, 1, 2, 1024>), dim3(a.rows), dim3(1024), lds(1), st, a);
 }
 
+// What tah_moe_route's sizes and rule have to be.
+int check_route(const tah_moe_route_args& a) {
+    if (a.rows < 0 || a.cols <= 0 || a.cols % 8 != 0 || a.experts <= 0 || a.experts > kMaxExperts || a.top <= 0 || a.top > kMaxTop ||
+        a.top > a.experts || (a.dtype != TAH_DT_BF16 && a.dtype != TAH_DT_F32) || (a.score != TAH_MOE_SOFTMAX && a.score != TAH_MOE_SIGMOID))
+        return TAH_E_SHAPE;
+    if (a.groups <= 0 || a.groups > kWave * kGroupsPerLane || a.experts % a.groups != 0 || a.keep <= 0 || a.keep > a.groups ||
+        a.top > a.experts / a.groups * a.keep)
+        return TAH_E_SHAPE;
+    if ((size_t)(a.cols + a.experts + 1) * sizeof(float) > 65536) return TAH_E_SHAPE;
+    return TAH_OK;
+}
+
 int tile_capacity(int64_t pairs, int experts) { return (int)(pairs / kTile + (experts < pairs ? experts : pairs)); }
 
 }  // namespace
@@ -442,13 +539,7 @@ int tile_capacity(int64_t pairs, int experts) { return (int)(pairs / kTile + (ex
 extern "C" int tah_moe_route(const tah_moe_route_args* a, tah_stream_t stream) {
     using namespace tah;
     if (!a) return TAH_E_NULL;
-    if (a->rows < 0 || a->cols <= 0 || a->cols % 8 != 0 || a->experts <= 0 || a->experts > kMaxExperts || a->top <= 0 || a->top > kMaxTop ||
-        a->top > a->experts || (a->dtype != TAH_DT_BF16 && a->dtype != TAH_DT_F32) || (a->score != TAH_MOE_SOFTMAX && a->score != TAH_MOE_SIGMOID))
-        return TAH_E_SHAPE;
-    if (a->groups <= 0 || a->groups > kWave * kGroupsPerLane || a->experts % a->groups != 0 || a->keep <= 0 || a->keep > a->groups ||
-        a->top > a->experts / a->groups * a->keep)
-        return TAH_E_SHAPE;
-    if ((size_t)(a->cols + a->experts + 1) * sizeof(float) > 65536) return TAH_E_SHAPE;
+    if (const int rc = check_route(*a)) return rc;
     if (a->rows == 0) return TAH_OK;
     if (!a->x || !a->router || !a->index || !a->weight || (a->gate_w && !a->shared_gate)) return TAH_E_NULL;
     if (!aligned_16(a->x) || !aligned_16(a->router) || !aligned_16(a->gate_w)) return TAH_E_ALIGN;
@@ -456,6 +547,48 @@ extern "C" int tah_moe_route(const tah_moe_route_args* a, tah_stream_t stream) {
     if (a->dtype == TAH_DT_F32) launch_route<float, float>(*a, st);
     else if (a->x_elem) launch_route<__bf16, __bf16>(*a, st);
     else launch_route<float, __bf16>(*a, st);
+    return launch_status();
+}
+
+extern "C" int tah_norm_route_supported(int32_t rows, int32_t cols, int32_t experts, int32_t gate) {
+    using namespace tah;
+    return rows >= 0 && rows <= kNormRouteRows && cols > 0 && cols % 8 == 0 && cols <= 8 * kRowThreads && experts > 0 &&
+           experts + (gate ? 1 : 0) <= kRouteWaves * kNormRouteExperts;
+}
+
+extern "C" int tah_norm_route(const tah_residual_norm_args* norm, float* x_out, const tah_moe_route_args* a, tah_stream_t stream) {
+    using namespace tah;
+    if (!norm || !a || !x_out) return TAH_E_NULL;
+    if (const int rc = check_residual(*norm)) return rc;
+    if (const int rc = check_route(*a)) return rc;
+    if (!tah_norm_route_supported(a->rows, a->cols, a->experts, a->gate_w != nullptr) || norm->dtype != TAH_DT_BF16 || a->dtype != TAH_DT_BF16 ||
+        norm->rows != a->rows || norm->cols != a->cols || norm->experts || norm->conv || (a->x_elem != 0) != (norm->next_coef != nullptr))
+        return TAH_E_SHAPE;
+    if (a->rows == 0) return TAH_OK;
+    // (a workgroup reads its row twice over while it stores the new one)
+    const auto meet = [&](const void* x, int64_t bytes) {
+        const char *at = static_cast<const char*>(x), *to = reinterpret_cast<const char*>(x_out);
+        return x && bytes > 0 && at < to + 4ll * norm->rows * norm->cols && to < at + bytes;
+    };
+    if (meet(norm->x, 4ll * norm->rows * norm->cols) || meet(norm->y, 2 * ((norm->rows - 1ll) * norm->y_row_stride + norm->cols)) ||
+        meet(norm->coef, 4ll * norm->cols) || meet(norm->next_coef, 4ll * norm->cols) || meet(norm->y_scale, 4ll * norm->rows) ||
+        meet(a->router, 2ll * a->experts * a->cols) || meet(a->gate_w, 2ll * a->cols))
+        return TAH_E_SHAPE;
+    if (!a->router || !a->index || !a->weight || (a->gate_w && !a->shared_gate)) return TAH_E_NULL;
+    if (!aligned_16(a->router) || !aligned_16(a->gate_w) || !aligned_16(x_out)) return TAH_E_ALIGN;
+    const NormRoute p{*norm, *a, x_out};
+    const int per = (a->experts + (a->gate_w ? 1 : 0) + kRouteWaves - 1) / kRouteWaves;
+    const auto launch = [&](auto groups, auto of) {
+        hipLaunchKernelGGL((moe_norm_route_kernel<decltype(groups)::value, decltype(of)::value>), dim3(a->rows), dim3(kNormRouteThreads), 0,
+                           static_cast<hipStream_t>(stream), p);
+    };
+    const auto run = [&](auto groups) {
+        if (per <= 2) launch(groups, std::integral_constant<int, 2>{});
+        else if (per <= 5) launch(groups, std::integral_constant<int, 5>{});
+        else launch(groups, std::integral_constant<int, kNormRouteExperts>{});
+    };
+    if (norm->groups > 1) run(std::true_type{});
+    else run(std::false_type{});
     return launch_status();
 }
 

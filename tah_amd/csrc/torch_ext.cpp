@@ -49,6 +49,8 @@ void load_library(const std::string& path, bool allow_host) {
     bind(g.linear_rows, "tah_linear_rows");
     bind(g.norm_linear_supported, "tah_norm_linear_supported");
     bind(g.norm_linear, "tah_norm_linear");
+    bind(g.norm_route_supported, "tah_norm_route_supported");
+    bind(g.norm_route, "tah_norm_route");
     bind(g.linear_chain_supported, "tah_linear_chain_supported");
     bind(g.linear_chain, "tah_linear_chain");
     bind(g.fwd_masked, "tah_duo_fwd_masked");

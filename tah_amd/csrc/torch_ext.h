@@ -46,6 +46,8 @@ struct Api {
     Entry<decltype(&tah_linear_pack_rows)> linear_pack_rows;
     Entry<decltype(&tah_norm_linear_supported)> norm_linear_supported;
     Entry<decltype(&tah_norm_linear)> norm_linear;
+    Entry<decltype(&tah_norm_route_supported)> norm_route_supported;
+    Entry<decltype(&tah_norm_route)> norm_route;
     Entry<decltype(&tah_linear_rows)> linear_rows;
     Entry<decltype(&tah_linear_chain_supported)> linear_chain_supported;
     Entry<decltype(&tah_linear_chain)> linear_chain;

@@ -426,6 +426,34 @@ void moe_route(const Tensor& x, const Tensor& router, const optional<Tensor>& ga
     check_rc(g.moe_route(&a, d.stream()), "tah_moe_route");
 }
 
+bool norm_route_supported(int64_t rows, int64_t cols, int64_t experts, bool gate) {
+    need_lib();
+    const auto fits = [](int64_t v) { return v >= 0 && v <= 0x7fffffff; };
+    return fits(rows) && fits(cols) && fits(experts) && g.norm_route_supported((int32_t)rows, (int32_t)cols, (int32_t)experts, gate) != 0;
+}
+
+// The norm, and the choice of experts behind it.
+void norm_route(const Tensor& x, const Tensor& x_out, const optional<Tensor>& coef, int64_t width, double eps, const optional<Tensor>& y,
+                const optional<Tensor>& y_scale, const optional<Tensor>& x_packed, const optional<Tensor>& next_coef, const optional<Tensor>& normed,
+                const optional<Tensor>& normed_packed, int64_t groups, int64_t group_cols, const Tensor& router, const optional<Tensor>& gate_w,
+                const Tensor& index, const Tensor& weight, const optional<Tensor>& shared_gate, int64_t score, int64_t of_groups, int64_t keep) {
+    need_lib();
+    Dev d; d.see(x_out); d.see(router); d.see(gate_w); d.see(index); d.see(weight); d.see(shared_gate);
+    const optional<Tensor> none;
+    const tah_residual_norm_args n = residual_args(d, &router, x, coef, width, eps, y, y_scale, none, none, none, none, x_packed, next_coef, normed,
+                                                   normed_packed, 1, 0, groups, group_cols, nullptr, none, none);
+    const int64_t rows = n.rows, cols = n.cols, top = index.size(1);
+    TORCH_CHECK(router.dim() == 2 && router.size(1) == cols && index.dim() == 2, "norm_route: router [experts, cols], index [rows, top]");
+    flat(x_out, at::kFloat, rows * cols, "norm_route: x_out"); flat(router, at::kBFloat16, -1, "norm_route: router");
+    flat(gate_w, at::kBFloat16, cols, "norm_route: gate_w"); flat(index, at::kInt, rows * top, "norm_route: index");
+    flat(weight, at::kFloat, rows * top, "norm_route: weight"); flat(shared_gate, at::kFloat, rows, "norm_route: shared_gate");
+    TORCH_CHECK(gate_w.has_value() == shared_gate.has_value(), "norm_route: gate_w and shared_gate come together");
+    const tah_moe_route_args a{nullptr, ptr(router), any(gate_w), at_<int32_t>(index), at_<float>(weight), at_<float>(shared_gate), (int32_t)rows,
+                               (int32_t)cols, (int32_t)router.size(0), (int32_t)top, (int32_t)of_groups, (int32_t)keep, (int32_t)score,
+                               next_coef.has_value(), TAH_DT_BF16};
+    check_rc(g.norm_route(&n, at_<float>(x_out), &a, d.stream()), "tah_norm_route");
+}
+
 // -> source [places], tile_expert [tiles and their number], place [rows, top]
 std::vector<Tensor> moe_plan(const Tensor& index, int64_t experts) {
     need_lib();
@@ -466,6 +494,8 @@ void bind_mixers(py::module_& m) {
     m.def("conv_rows", &conv_rows);
     m.def("activate_rows", &activate_rows);
     m.def("moe_route", &moe_route);
+    m.def("norm_route_supported", &norm_route_supported);
+    m.def("norm_route", &norm_route);
     m.def("moe_plan", &moe_plan);
     m.def("moe_linear", &moe_linear);
     py::class_<Portions>(m, "Portions").def(py::init<Tensor, Tensor, Tensor, Tensor>());

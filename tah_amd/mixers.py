@@ -149,6 +149,21 @@ class Step:
         self.settle()
         return layer.rows(self.xp, self.n, out_packed=out_packed, want_out=want_out, **kw)
 
+    def route(self, router: torch.Tensor, shared_gate: Optional[torch.Tensor], index, weight, sg, rule: "Router") -> None:
+        """The rows' experts; what the experts read is settled behind it."""
+        p = self.pending
+        if (p is not None and p.front[5] is None and p.tail[4] is None  # (neither experts' rows nor a convolution)
+                and _call("norm_route_supported", self.n, self.x.shape[1], router.shape[0], shared_gate is not None)):
+            self.pending = None
+            reads_norm = p.norm is not None
+            coef, width, eps, y, y_scale, *_ = p.front
+            _call("norm_route", self.x, self.x_other, coef, width, eps, y, y_scale, None if reads_norm else self.xp, p.norm, self.xe if reads_norm else None,
+                  self.xp if reads_norm else None, *p.tail[2:4], router, shared_gate, index, weight, sg, int(rule.sigmoid), rule.groups, rule.keep)
+            self.x, self.x_other = self.x_other, self.x
+            return
+        self.settle()
+        _call("moe_route", self.xe if self.normed else self.x, router, shared_gate, index, weight, sg, int(rule.sigmoid), rule.groups, rule.keep)
+
 
 @dataclasses.dataclass
 class Sublayer:
@@ -562,14 +577,13 @@ class MoeMlp:
                 index = torch.empty(st.n, m.top, dtype=torch.int32, device=dev)
             weight = torch.empty(st.n, m.top, dtype=torch.float32, device=dev)
             sg = torch.empty(st.n, dtype=torch.float32, device=dev) if m.shared else None
-            _call("moe_route", st.xe if st.normed else st.x, m.router, m.shared_gate, index, weight, sg, int(m.rule.sigmoid), m.rule.groups, m.rule.keep)
+            st.route(m.router, m.shared_gate, index, weight, sg, m.rule)
             return index, weight, sg
 
         def rows(self, st: Step) -> Sublayer:
             m, n = self.m, st.n
             if not st.packed:
                 return self.portions(st)
-            st.settle()
             picked = self.chosen[1:1 + n * m.top]
             index, weight, sg = self._route(st, picked.view(n, m.top))
             select = self.chosen[:1 + n * m.top] if m.shared_among else picked
