@@ -235,6 +235,12 @@ int tah_window_append(const tah_window_layer* layer, const tah_portions* p, cons
 size_t tah_window_decode_workspace(const tah_window_layer* layer, int32_t rows);
 int tah_window_decode(const tah_window_layer* layer, const tah_window_rows* rows, void* out, int64_t out_row_stride, void* out_packed,
                       void* workspace, size_t workspace_bytes, tah_stream_t stream);
+/* The same and tah_linear_rows on the result (the output projection, k = heads * value_dim; its x_packed is not read), for a few rows whose
+ * keys are split over workgroups: the parts are merged in the projection's launch.  The bits of the two calls.  linear: a plain layer as
+ * tah_norm_linear takes it; its results lie on nothing that the call reads (TAH_E_SHAPE where they do). */
+int tah_window_decode_linear_supported(const tah_window_layer* layer, int32_t rows, int32_t n);
+int tah_window_decode_linear(const tah_window_layer* layer, const tah_window_rows* rows, const struct tah_linear_rows_args* linear, void* workspace,
+                             size_t workspace_bytes, tah_stream_t stream);
 
 /* ---- mixture of experts -------------------------------------------------------------------------------------- *
  * tah_moe_route: logits x . router in float32; scores are the logits (TAH_MOE_SOFTMAX) or their sigmoids (TAH_MOE_SIGMOID).

@@ -413,6 +413,8 @@ PROTOTYPES = {
     "tah_window_append": (C.c_int, [C.POINTER(WindowLayer), C.POINTER(Portions), C.POINTER(WindowRows), c_void_p]),
     "tah_window_decode_workspace": (C.c_size_t, [C.POINTER(WindowLayer), c_int32]),
     "tah_window_decode": (C.c_int, [C.POINTER(WindowLayer), C.POINTER(WindowRows), c_void_p, c_int64, c_void_p, c_void_p, C.c_size_t, c_void_p]),
+    "tah_window_decode_linear_supported": (C.c_int, [C.POINTER(WindowLayer), c_int32, c_int32]),
+    "tah_window_decode_linear": (C.c_int, [C.POINTER(WindowLayer), C.POINTER(WindowRows), C.POINTER(LinearRowsArgs), c_void_p, C.c_size_t, c_void_p]),
     "tah_moe_route": (C.c_int, [C.POINTER(MoeRouteArgs), c_void_p]),
     "tah_norm_route_supported": (C.c_int, [c_int32, c_int32, c_int32, c_int32]),
     "tah_norm_route": (C.c_int, [C.POINTER(ResidualNormArgs), c_void_p, C.POINTER(MoeRouteArgs), c_void_p]),

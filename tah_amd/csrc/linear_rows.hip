@@ -1035,6 +1035,51 @@ __global__ __launch_bounds__(kChainThreads) void linear_chain_kernel(const Chain
     }
 }
 
+// What a plain layer's tile leaves of at most two rows: sums, activation, row-major and / or rows form.
+struct LinearOut {
+    __bf16* y;
+    bf16x8* yp;
+    int64_t y_rs;
+    int32_t act, rows;
+    float c0, c1;
+};
+template <bool H8>
+__device__ __forceinline__ void finish_plain_tile(const LinearOut& p, const float (*red)[3][16][kTileCols]) {
+    // a lane per row (rows past the last one are zeros in the rows form) and eight columns
+    constexpr int kUnits = H8 ? 1 : 2;
+    if ((int)threadIdx.x >= kLinRows * kUnits) return;
+    const int row = threadIdx.x % kLinRows, unit = threadIdx.x / kLinRows, n0 = (int)blockIdx.x * 8 * kUnits + 8 * unit;
+    bf16x8 out = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (row < p.rows) {
+        float s[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s[i] = 0.f;
+#pragma unroll
+        for (int w = 0; w < kLinWaves; ++w)
+#pragma unroll
+            for (int half = 0; half < (H8 ? 2 : 1); ++half) {  // (H8: the even and the odd steps' sums)
+                const f32x4 lo = *reinterpret_cast<const f32x4*>(&red[w][0][row][8 * (H8 ? half : unit)]);
+                const f32x4 hi = *reinterpret_cast<const f32x4*>(&red[w][0][row][8 * (H8 ? half : unit) + 4]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    s[i] += lo[i];
+                    s[4 + i] += hi[i];
+                }
+            }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) out[i] = (__bf16)s[i];
+        if (p.act == TAH_ACT_GELU_TANH) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) out[i] = (__bf16)gelu_tanh_exact((float)out[i]);
+        } else if (p.act == TAH_ACT_XIELU) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) out[i] = (__bf16)xielu((float)out[i], p.c0, p.c1);
+        }
+        if (p.y) *reinterpret_cast<bf16x8*>(p.y + (int64_t)row * p.y_rs + n0) = out;
+    }
+    if (p.yp) p.yp[packed_rows_unit(row, n0)] = out;
+}
+
 // ---- a norm of the residual stream and the linear layer behind it in one launch ----------------------------
 // One or two rows: a decode step of such a model is a chain of launches of 4.4 us and more, most of it their start and the first trip to
 // memory, and a norm of a few rows is a launch of its own for 8 KB.  Here every workgroup of the layer makes the normed rows for
@@ -1050,11 +1095,7 @@ struct NormLinear {
     tah_residual_norm_args n;
     float* x_out;
     const bf16x8* w;
-    __bf16* y;
-    bf16x8* yp;
-    int64_t y_rs;
-    int32_t act;
-    float c0, c1;
+    LinearOut out;
 };
 
 // kMore: with experts or a convolution, whose loads take the registers of a second workgroup on the compute unit
@@ -1093,39 +1134,78 @@ __global__ __launch_bounds__(kLinThreads, kMore ? 2 : 4) void norm_linear_kernel
     t.template multiply<false, 0, PW>();
     t.template park<false>(red, nullptr, wave, lane);
     __syncthreads();
-    // a lane per row (rows past the last one are zeros in the rows form) and eight columns
-    constexpr int kUnits = H8 ? 1 : 2;
-    if ((int)threadIdx.x >= kLinRows * kUnits) return;
-    const int row = threadIdx.x % kLinRows, unit = threadIdx.x / kLinRows, n0 = (int)blockIdx.x * 8 * kUnits + 8 * unit;
-    bf16x8 out = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (row < p.n.rows) {
-        float s[8];
+    finish_plain_tile<H8>(p.out, red);
+}
+
+// ---- the parts of a windowed attention's split call and the output projection behind them in one launch -------
+// One or two rows: merging a call's parts was a launch of 4.7 us for 42 KB a row, and the projection behind it another of 4.5. Here
+// every workgroup of the projection merges the row for itself (a compute unit takes 42 KB in in 0.4 us), its weights on their way.  The
+// same bits as window_merge_kernel and tah_linear_rows leave.  From three rows on the parts cost more than the launch: two launches.
+// One row of 16 heads in five parts, 2048 -> 2048, in a captured step: 4.7 + 4.5 -> 5.5 us.
+template <int F, bool H8>
+__global__ __launch_bounds__(kLinThreads) void merge_linear_kernel(const MergeLinear p, const LinearOut out, const bf16x8* weights) {
+    constexpr int PW = kNormLinearSteps, kCols = 4 * F, kAhead = 8;  // columns per thread; parts on their way
+    using Tile = ChainTile<PW, 1, H8, F, H8>;
+    __shared__ __align__(16) float red[kLinWaves][3][16][kTileCols];
+    __shared__ __align__(16) bf16x8 rows_lds[PW * kLinWaves * 4 * F];  // [step][k group][row]
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const int c = lane % 16, kg = lane / 16;
+    constexpr int kPerRow = kLinThreads / F;
+    const int r = (int)threadIdx.x / kPerRow, col = kCols * ((int)threadIdx.x % kPerRow), h = col / p.value_dim, vs = p.value_dim + 4;
+    const int row = r < out.rows ? r : out.rows - 1;
+    const float* const base = p.part + ((int64_t)row * p.heads + h) * p.splits * vs;
+    const int x = col % p.value_dim;
+    f32x4 v[kAhead][F];
+    float vm[kAhead], vl[kAhead];
+    auto ask = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) s[i] = 0.f;
+        for (int i = 0; i < kAhead; ++i) {
+            const float* const at = base + (int64_t)(s0 + i < p.splits ? s0 + i : p.splits - 1) * vs;
 #pragma unroll
-        for (int w = 0; w < kLinWaves; ++w)
-#pragma unroll
-            for (int half = 0; half < (H8 ? 2 : 1); ++half) {  // (H8: the even and the odd steps' sums)
-                const f32x4 lo = *reinterpret_cast<const f32x4*>(&red[w][0][row][8 * (H8 ? half : unit)]);
-                const f32x4 hi = *reinterpret_cast<const f32x4*>(&red[w][0][row][8 * (H8 ? half : unit) + 4]);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    s[i] += lo[i];
-                    s[4 + i] += hi[i];
-                }
-            }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) out[i] = (__bf16)s[i];
-        if (p.act == TAH_ACT_GELU_TANH) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) out[i] = (__bf16)gelu_tanh_exact((float)out[i]);
-        } else if (p.act == TAH_ACT_XIELU) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) out[i] = (__bf16)xielu((float)out[i], p.c0, p.c1);
+            for (int f = 0; f < F; ++f) v[i][f] = *reinterpret_cast<const f32x4*>(at + x + 4 * f);
+            vm[i] = at[p.value_dim];
+            vl[i] = at[p.value_dim + 1];
         }
-        if (p.y) *reinterpret_cast<bf16x8*>(p.y + (int64_t)row * p.y_rs + n0) = out;
+    };
+    ask(0);
+    const __bf16 gate = p.gate ? p.gate[(int64_t)row * p.gate_rs + h] : (__bf16)0.f;
+    Tile t;
+    __builtin_amdgcn_sched_barrier(0);
+    t.ask_weights(weights, blockIdx.x, wave, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    PartsSum<kCols> sum;
+    for (int s0 = 0;;) {
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+            if (s0 + i >= p.splits) continue;
+            float w[kCols];
+#pragma unroll
+            for (int e = 0; e < kCols; ++e) w[e] = v[i][e / 4][e % 4];
+            sum.add(vm[i], vl[i], w);
+        }
+        s0 += kAhead;
+        if (s0 >= p.splits) break;
+        ask(s0);
     }
-    if (p.yp) p.yp[packed_rows_unit(row, n0)] = out;
+    const float inv = sum.factor(p.gate != nullptr, (float)gate);
+    if (r < out.rows) {
+        __bf16* const to = reinterpret_cast<__bf16*>(&rows_lds[(col / kStepK * 4 + col % kStepK / 8) * F + r]) + col % 8;
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            bf16x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = (__bf16)(sum.y[4 * f + e] * inv);
+            *reinterpret_cast<bf16x4*>(to + 4 * f) = o;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < Tile::kXLoads; ++j) t.x[j] = rows_lds[((wave * PW + Tile::step_of(j, c)) * 4 + kg) * F + c % F];
+    t.start();
+    t.template multiply<false, 0, PW>();
+    t.template park<false>(red, nullptr, wave, lane);
+    __syncthreads();
+    finish_plain_tile<H8>(out, red);
 }
 
 // what is left of a launch without rows: the words of the next one
@@ -1375,6 +1455,40 @@ extern "C" int tah_norm_linear_supported(int32_t rows, int32_t cols, int32_t n) 
            n / kTileCols <= kNormLinearWorkgroups;
 }
 
+namespace tah {
+namespace {
+// What a plain layer's arguments say beside its sizes, as tah_norm_linear and the merge's projection take them.
+int check_plain(const tah_linear_rows_args& a) {
+    if (a.kind != TAH_LINEAR_PLAIN || a.batch > 1 || a.residual || a.bias || a.input_norm != TAH_NORM_NONE || a.n_select != 0 ||
+        (a.activation != TAH_ACT_NONE && a.activation != TAH_ACT_GELU_TANH && a.activation != TAH_ACT_XIELU) || (a.out_packed && a.n % kStepK != 0) ||
+        (a.out && a.out_row_stride < a.n))
+        return TAH_E_SHAPE;
+    if (!a.w_packed || (!a.out && !a.out_packed)) return TAH_E_NULL;
+    if (!aligned16(a.w_packed) || !aligned16(a.out) || !aligned16(a.out_packed) || (a.out && a.out_row_stride % 8 != 0)) return TAH_E_ALIGN;
+    return TAH_OK;
+}
+LinearOut linear_out(const tah_linear_rows_args& a) {
+    return LinearOut{static_cast<__bf16*>(a.out), static_cast<bf16x8*>(a.out_packed), a.out_row_stride, a.activation, a.rows, a.act_c[0], a.act_c[1]};
+}
+}  // namespace
+
+bool merge_linear_fits(int rows, int k, int n) { return tah_norm_linear_supported(rows, k, n) != 0; }
+
+int merge_linear(const MergeLinear& p, const tah_linear_rows_args& a, hipStream_t st) {
+    if (const int rc = check_plain(a)) return rc;
+    if (!merge_linear_fits(a.rows, a.k, a.n) || a.k != p.heads * p.value_dim) return TAH_E_SHAPE;
+    const bool h8 = a.n / kTileCols < kSplitRowsBelowGroups;  // (as tah_linear_rows takes such a layer)
+    const auto launch = [&](auto fold, auto half) {
+        hipLaunchKernelGGL((merge_linear_kernel<decltype(fold)::value, decltype(half)::value>), dim3(a.n / (h8 ? 8 : kTileCols)), dim3(kLinThreads), 0, st, p,
+                           linear_out(a), static_cast<const bf16x8*>(a.w_packed));
+    };
+    const auto run = [&](auto fold) { h8 ? launch(fold, std::true_type{}) : launch(fold, std::false_type{}); };
+    if (a.rows <= 1) run(std::integral_constant<int, 1>{});
+    else run(std::integral_constant<int, 2>{});
+    return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
+}
+}  // namespace tah
+
 extern "C" int tah_norm_linear(const tah_residual_norm_args* norm, float* x_out, const tah_linear_rows_args* a, tah_stream_t stream) {
     using namespace tah;
     if (!norm || !a || !x_out) return TAH_E_NULL;
@@ -1382,13 +1496,8 @@ extern "C" int tah_norm_linear(const tah_residual_norm_args* norm, float* x_out,
     if (!tah_norm_linear_supported(norm->rows, norm->cols, a->n) || norm->dtype != TAH_DT_BF16 || a->rows != norm->rows || a->k != norm->cols) return TAH_E_SHAPE;
     // (what a workgroup of another tile still reads: nothing but x_out, the convolution's input and the layer's result is written)
     if (norm->xe || norm->x_packed || norm->normed || norm->normed_packed) return TAH_E_SHAPE;
-    if (a->kind != TAH_LINEAR_PLAIN || a->batch > 1 || a->residual || a->bias || a->input_norm != TAH_NORM_NONE || a->n_select != 0 ||
-        (a->activation != TAH_ACT_NONE && a->activation != TAH_ACT_GELU_TANH && a->activation != TAH_ACT_XIELU) || (a->out_packed && a->n % kStepK != 0) ||
-        (a->out && a->out_row_stride < a->n))
-        return TAH_E_SHAPE;
-    if (!a->w_packed || (!a->out && !a->out_packed)) return TAH_E_NULL;
-    if (!aligned16(x_out) || !aligned16(a->w_packed) || !aligned16(a->out) || !aligned16(a->out_packed) || (a->out && a->out_row_stride % 8 != 0))
-        return TAH_E_ALIGN;
+    if (const int rc = check_plain(*a)) return rc;
+    if (!aligned16(x_out)) return TAH_E_ALIGN;
     struct Range { const char* at; int64_t bytes; };
     const auto of = [](const void* q, int64_t bytes) { return Range{static_cast<const char*>(q), q ? bytes : 0}; };
     const int64_t last = norm->rows - 1;
@@ -1408,11 +1517,7 @@ extern "C" int tah_norm_linear(const tah_residual_norm_args* norm, float* x_out,
     p.n = *norm;
     p.x_out = x_out;
     p.w = static_cast<const bf16x8*>(a->w_packed);
-    p.y = static_cast<__bf16*>(a->out);
-    p.yp = static_cast<bf16x8*>(a->out_packed);
-    p.y_rs = a->out_row_stride;
-    p.act = a->activation;
-    p.c0 = a->act_c[0]; p.c1 = a->act_c[1];
+    p.out = linear_out(*a);
     const bool h8 = a->n / kTileCols < kSplitRowsBelowGroups;  // (as tah_linear_rows takes such a layer)
     const auto launch = [&](auto fold, auto groups, auto half, auto more) {
         hipLaunchKernelGGL((norm_linear_kernel<decltype(fold)::value, decltype(groups)::value, decltype(half)::value, decltype(more)::value>),

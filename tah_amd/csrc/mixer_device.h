@@ -150,6 +150,36 @@ __device__ __forceinline__ float groups_sum(float x) {
     return x + __shfl_xor(x, 32);
 }
 
+// ---- the parts of a split windowed attention ----
+// A row's running sum over parts, each of sums v under its own maximum vm and a denominator vl (0: it saw nothing).  The roundings are written
+// out: two kernels merge parts, and what one of them fused the other did not have to.
+template <int N>
+struct PartsSum {
+    float m = kNoScore, l = 0.f, y[N] = {};
+    __device__ __forceinline__ void add(float vm, float vl, const float (&v)[N]) {
+        if (!(vl > 0.f)) return;
+        const float mn = fmaxf(m, vm), a = fast_exp2(m - mn), b = fast_exp2(vm - mn);
+        m = mn;
+        l = fmaf(l, a, vl * b);
+#pragma unroll
+        for (int e = 0; e < N; ++e) y[e] = fmaf(y[e], a, v[e] * b);
+    }
+    // what the sums are multiplied by: one over the denominator, times the head's gate
+    __device__ __forceinline__ float factor(bool gated, float gate) const {
+        const float inv = l > 0.f ? 1.0f / l : 0.f;
+        return gated ? inv * sigmoid_exact(gate) : inv;
+    }
+};
+struct MergeLinear {
+    const float* part;   // [rows][heads][splits][value_dim + 4]: sums, the maximum, the sum of weights
+    const __bf16* gate;  // [rows, gate_rs]: a gate per head, or null
+    int64_t gate_rs;
+    int32_t heads, splits, value_dim;
+};
+// A plain linear layer of at most two merged rows in the merge's launch (linear_rows.hip), and whether its sizes are taken.
+bool merge_linear_fits(int rows, int k, int n);
+int merge_linear(const MergeLinear& p, const tah_linear_rows_args& a, hipStream_t st);
+
 inline bool aligned_16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 inline int launch_status() { return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH; }
 

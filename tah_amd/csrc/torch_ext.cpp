@@ -93,6 +93,8 @@ void load_library(const std::string& path, bool allow_host) {
     bind(g.window_append, "tah_window_append");
     bind(g.window_decode_workspace, "tah_window_decode_workspace");
     bind(g.window_decode, "tah_window_decode");
+    bind(g.window_decode_linear_supported, "tah_window_decode_linear_supported");
+    bind(g.window_decode_linear, "tah_window_decode_linear");
     bind(g.moe_route, "tah_moe_route");
     bind(g.moe_places, "tah_moe_places");
     bind(g.moe_plan, "tah_moe_plan");

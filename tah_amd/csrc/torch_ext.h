@@ -91,6 +91,8 @@ struct Api {
     Entry<decltype(&tah_window_append)> window_append;
     Entry<decltype(&tah_window_decode_workspace)> window_decode_workspace;
     Entry<decltype(&tah_window_decode)> window_decode;
+    Entry<decltype(&tah_window_decode_linear_supported)> window_decode_linear_supported;
+    Entry<decltype(&tah_window_decode_linear)> window_decode_linear;
     Entry<decltype(&tah_moe_route)> moe_route;
     Entry<decltype(&tah_moe_places)> moe_places;
     Entry<decltype(&tah_moe_plan)> moe_plan;

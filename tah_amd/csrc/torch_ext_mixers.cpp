@@ -407,6 +407,25 @@ struct WindowLayer {
         check_rc(g.window_decode(&L, &r, any(out), rs, any(out_packed), any(workspace), workspace.has_value() ? (size_t)workspace->numel() : 0, d.stream()),
                  "tah_window_decode");
     }
+    bool decode_linear_supported(int64_t n, int64_t cols) const {
+        need_lib();
+        const auto fits = [](int64_t v) { return v >= 0 && v <= 0x7fffffff; };
+        return fits(n) && fits(cols) && g.window_decode_linear_supported(&L, (int32_t)n, (int32_t)cols) != 0;
+    }
+    // attention and the output projection w_packed [n, heads * value_dim] -> [rows, n]
+    Tensor decode_linear(const Tensor& proj, const Tensor& slot, const Tensor& pos, const Tensor& w_packed, int64_t n, const Tensor& workspace) const {
+        need_lib();
+        Dev d; d.see(w_packed); d.see(workspace);
+        const tah_window_rows r = rows(d, proj, pos, slot);
+        flat(w_packed, at::kBFloat16, n * width(), "WindowLayer.decode_linear: w_packed");
+        flat(workspace, at::kByte, -1, "WindowLayer.decode_linear: workspace");
+        Tensor out = at::empty({(int64_t)r.rows, n}, w_packed.options());
+        tah_linear_rows_args l{};
+        l.w_packed = ptr(w_packed); l.out = mptr(out); l.out_row_stride = n;
+        l.rows = r.rows; l.n = (int32_t)n; l.k = (int32_t)width(); l.kind = TAH_LINEAR_PLAIN;
+        check_rc(g.window_decode_linear(&L, &r, &l, mptr(workspace), (size_t)workspace.numel(), d.stream()), "tah_window_decode_linear");
+        return out;
+    }
 };
 
 void moe_route(const Tensor& x, const Tensor& router, const optional<Tensor>& gate_w, const Tensor& index, const Tensor& weight,
@@ -514,7 +533,9 @@ void bind_mixers(py::module_& m) {
         .def(py::init<Tensor, Tensor, Tensor, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, double, int64_t, int64_t, int64_t>())
         .def("portions", &WindowLayer::portions)
         .def("decode_workspace", &WindowLayer::decode_workspace)
-        .def("decode", &WindowLayer::decode);
+        .def("decode", &WindowLayer::decode)
+        .def("decode_linear_supported", &WindowLayer::decode_linear_supported)
+        .def("decode_linear", &WindowLayer::decode_linear);
 }
 
 }  // namespace tah_ext

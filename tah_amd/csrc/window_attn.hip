@@ -635,7 +635,7 @@ __global__ __launch_bounds__(kWave) void window_merge_kernel(const WindowDecode 
     const __bf16* const proj = static_cast<const __bf16*>(p.R.proj) + (int64_t)row * p.R.proj_row_stride;
     const float* const base = p.part + ((int64_t)row * p.L.heads + h) * p.splits * vs;
     for (int x = 8 * threadIdx.x; x < p.L.value_dim; x += 8 * kWave) {
-        float m = kNoScore, l = 0.f, y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        PartsSum<8> sum;
         for (int s0 = 0; s0 < p.splits; s0 += 4) {
             float v[4][8], vm[4], vl[4];
 #pragma unroll
@@ -646,19 +646,13 @@ __global__ __launch_bounds__(kWave) void window_merge_kernel(const WindowDecode 
                 vl[i] = at[p.L.value_dim + 1];
             }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (s0 + i >= p.splits || !(vl[i] > 0.f)) continue;
-                const float mn = fmaxf(m, vm[i]), a = fast_exp2(m - mn), b = fast_exp2(vm[i] - mn);
-                m = mn;
-                l = l * a + vl[i] * b;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) y[e] = y[e] * a + v[i][e] * b;
-            }
+            for (int i = 0; i < 4; ++i)
+                if (s0 + i < p.splits) sum.add(vm[i], vl[i], v[i]);
         }
-        float inv = l > 0.f ? 1.0f / l : 0.f;
-        if (p.R.g_col >= 0) inv *= sigmoid_exact((float)proj[p.R.g_col + h]);
+        const float inv = sum.factor(p.R.g_col >= 0, p.R.g_col >= 0 ? (float)proj[p.R.g_col + h] : 0.f);
+        float y[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) y[e] *= inv;
+        for (int e = 0; e < 8; ++e) y[e] = sum.y[e] * inv;
         const int col = h * p.L.value_dim + x;
         if (p.out) store8(p.out + row * p.out_rs + col, y);
         if (p.out_packed) reinterpret_cast<bf16x8*>(p.out_packed)[rows_form_unit(row, col)] = to_bf16x8(y);
@@ -814,6 +808,28 @@ extern "C" size_t tah_window_decode_workspace(const tah_window_layer* L, int32_t
     return most;
 }
 
+namespace tah {
+namespace {
+// The split launch of a decode call: parts in the workspace, or with one split the results themselves.
+int launch_parts(const tah_window_layer* L, const tah_window_rows* R, WindowDecode& d, void* workspace, size_t workspace_bytes, hipStream_t st) {
+    d.L = *L; d.R = *R;
+    d.scale_log2 = L->scale * kLog2e;
+    d.chunks = (L->heads / L->kv_heads + 15) / 16;
+    decode_split(*L, R->rows, d.splits, d.keys_per_split);
+    if (d.splits > 1) {
+        if (!workspace || !aligned_16(workspace) || workspace_bytes < (size_t)R->rows * L->heads * d.splits * (L->value_dim + 4) * sizeof(float))
+            return TAH_E_WORKSPACE;
+        d.part = static_cast<float*>(workspace);
+    }
+    // (units per lane and row: row / 64, rounded up)
+    if (L->key_dim == 128 && L->value_dim == 128 && L->row <= 192) return launch_decode<4, 8, 3, 8, true>(d, st);
+    if (L->key_dim <= 64 && L->value_dim <= 64) return launch_decode<2, 4, 2, 8, false>(d, st);
+    if (L->row <= 256) return launch_decode<8, 16, 4, 8, false>(d, st);
+    return launch_decode<8, 16, 8, 4, false>(d, st);
+}
+}  // namespace
+}  // namespace tah
+
 extern "C" int tah_window_decode(const tah_window_layer* L, const tah_window_rows* R, void* out, int64_t out_rs, void* out_packed, void* workspace,
                                  size_t workspace_bytes, tah_stream_t stream) {
     using namespace tah;
@@ -832,23 +848,45 @@ extern "C" int tah_window_decode(const tah_window_layer* L, const tah_window_row
         return launch_status();
     }
     WindowDecode d{};
-    d.L = *L; d.R = *R;
     d.out = static_cast<__bf16*>(out); d.out_packed = static_cast<__bf16*>(out_packed); d.out_rs = out_rs;
-    d.scale_log2 = L->scale * kLog2e;
-    d.chunks = (L->heads / L->kv_heads + 15) / 16;
-    decode_split(*L, R->rows, d.splits, d.keys_per_split);
-    if (d.splits > 1) {
-        if (!workspace || !aligned_16(workspace) || workspace_bytes < (size_t)R->rows * L->heads * d.splits * (L->value_dim + 4) * sizeof(float))
-            return TAH_E_WORKSPACE;
-        d.part = static_cast<float*>(workspace);
-    }
-    // (units per lane and row: row / 64, rounded up)
-    int rc;
-    if (L->key_dim == 128 && L->value_dim == 128 && L->row <= 192) rc = launch_decode<4, 8, 3, 8, true>(d, st);
-    else if (L->key_dim <= 64 && L->value_dim <= 64) rc = launch_decode<2, 4, 2, 8, false>(d, st);
-    else if (L->row <= 256) rc = launch_decode<8, 16, 4, 8, false>(d, st);
-    else rc = launch_decode<8, 16, 8, 4, false>(d, st);
+    const int rc = launch_parts(L, R, d, workspace, workspace_bytes, st);
     if (rc != TAH_OK || d.splits == 1) return rc;
     hipLaunchKernelGGL(window_merge_kernel, dim3(L->heads, R->rows), dim3(kWave), 0, st, d);
     return launch_status();
 }
+
+extern "C" int tah_window_decode_linear_supported(const tah_window_layer* L, int32_t rows, int32_t n) {
+    using namespace tah;
+    if (check_layer(L) != TAH_OK || !on_tiles(L) || rows <= 0) return 0;
+    int splits, keys;
+    decode_split(*L, rows, splits, keys);
+    return splits > 1 && merge_linear_fits(rows, L->heads * L->value_dim, n);
+}
+
+extern "C" int tah_window_decode_linear(const tah_window_layer* L, const tah_window_rows* R, const tah_linear_rows_args* a, void* workspace,
+                                        size_t workspace_bytes, tah_stream_t stream) {
+    using namespace tah;
+    if (const int rc = check_layer(L)) return rc;
+    if (const int rc = check_rows(L, R)) return rc;
+    if (!a) return TAH_E_NULL;
+    if (R->rows == 0) return TAH_OK;
+    if (!tah_window_decode_linear_supported(L, R->rows, a->n) || a->rows != R->rows || a->k != L->heads * L->value_dim) return TAH_E_SHAPE;
+    if (!R->slot) return TAH_E_NULL;
+    // (the projection's workgroups read the parts and the gates while others store)
+    const auto meet = [&](const void* x, int64_t nx, const void* y, int64_t ny) {
+        const char *p = static_cast<const char*>(x), *q = static_cast<const char*>(y);
+        return p && q && p < q + ny && q < p + nx;
+    };
+    const int64_t proj = 2 * ((R->rows - 1) * R->proj_row_stride + (R->g_col >= 0 ? R->g_col + (int64_t)L->heads : 0));
+    const int64_t out = 2 * ((a->rows - 1) * a->out_row_stride + a->n), packed = 64ll * a->n;
+    if (meet(a->out, out, workspace, (int64_t)workspace_bytes) || meet(a->out_packed, packed, workspace, (int64_t)workspace_bytes) ||
+        meet(a->out, out, R->proj, proj) || meet(a->out_packed, packed, R->proj, proj) || meet(a->out, out, a->w_packed, 2ll * a->n * a->k) ||
+        meet(a->out_packed, packed, a->w_packed, 2ll * a->n * a->k))
+        return TAH_E_SHAPE;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    WindowDecode d{};
+    if (const int rc = launch_parts(L, R, d, workspace, workspace_bytes, st)) return rc;
+    const __bf16* const gates = R->g_col >= 0 ? static_cast<const __bf16*>(R->proj) + R->g_col : nullptr;
+    return merge_linear(MergeLinear{d.part, gates, R->proj_row_stride, L->heads, d.splits, L->value_dim}, *a, st);
+}
+

@@ -454,9 +454,12 @@ class WindowAttention:
             z = lambda n, dt=engine.dtype: torch.zeros(n, dtype=dt, device=engine.device)
             self.workspace = z(max(int(self.layer.decode_workspace(min(engine.B, ops.LINEAR_MAX_ROWS))), 16), torch.uint8)
             self.op = z(32 * m.width_o) if engine.packed else None
+            self.layer_width = s.heads * m.value_dim
 
         def rows(self, st: Step) -> Sublayer:
             m = self.m
+            if st.packed and m.o.k == self.layer_width and self.layer.decode_linear_supported(st.n, m.o.n):
+                return Sublayer(_call_on(self.layer.decode_linear, st.linear(m.proj), st.slot, st.pos, m.o.packed, m.o.n, self.workspace))
             if st.packed:
                 _call_on(self.layer.decode, st.linear(m.proj), st.slot, st.pos, None, self.op, self.workspace)
                 return Sublayer(m.o.rows(self.op, st.n))
