@@ -809,18 +809,24 @@ __global__ __launch_bounds__(kKvThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dkd
 // MFMA per 512 bytes of it, so what matters is the number of bytes on their way); a wave then forms
 // dQ[64 rows x 64 d] += dS[64 x 64 keys] K[64 keys x 64 d] from transpose reads of both (dS lies key-major,
 // K row-major, and both operands want the keys along a lane's registers): 16 MFMAs.
-constexpr int kLqThreads = 512;
-constexpr int kLqUnits = 4;
-constexpr int kLqStageDs = kLqUnits * 8192;            // per unit: 64 rows x 64 keys of dS
-constexpr int kLqStage = kTileBytes + kLqStageDs;      // K rows of the step + dS
-constexpr int kLqStages = 3;
-constexpr int kLqSmem = kLqStages * kLqStage;
-constexpr int kLqCopies = 6;                           // asynchronous copies per wave and step
+// Launches of at most kLqFewWorkgroups workgroups of four units take workgroups of two (G <= 2), twice as many: a step of four waves reads
+// half as much out of LDS and stages 32 KB instead of 48, four steps deep instead of three.  Every row's sum is the same: the same bits.
+// Whole backward, 16 / 8 heads, us with four and with two: 333 rows 48.9 -> 47.7 (32 workgroups of four), 1024 89 -> 85, 2048 159 -> 150, 3000 227 -> 214,
+// 4096 336 -> 315 (280), 6000 542 -> 537 (400), eight of 512 94.5 -> 95.7 (392); 10 % of four sequences' rows at depth 1 160 -> 139 (88).
+constexpr int kLqUnitsFew = 2;
+constexpr long kLqFewWorkgroups = 320;
+constexpr int lq_threads(int units) { return units * 128; }
+constexpr int lq_stage(int units) { return kTileBytes + units * 8192; }  // K rows of the step, and per unit 64 rows x 64 keys of dS
+constexpr int lq_stages(int units) { return units == 4 ? 3 : 4; }
+constexpr int lq_smem(int units) { return lq_stages(units) * lq_stage(units); }
 
-template <int G>
-__global__ __launch_bounds__(kLqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_from_ds_kernel(const BwdParams p) {
-    static_assert(G == 1 || G == 2 || G == 4, "four (64-row tile, head) units per workgroup");
-    constexpr int BM = 32 * (8 / G);
+template <int G, int kUnits = 4>
+__global__ __launch_bounds__(lq_threads(kUnits)) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_from_ds_kernel(const BwdParams p) {
+    static_assert(kUnits % G == 0, "a workgroup's (64-row tile, head) units: every head of its kv head");
+    constexpr int BM = 64 * kUnits / G;
+    constexpr int kLqStage = lq_stage(kUnits), kLqStages = lq_stages(kUnits);
+    constexpr int kWaves = 2 * kUnits, kPieces = kBN / 4 / kWaves;  // K rows a wave copies, in pieces of four
+    constexpr int kLqCopies = kPieces + 4;                          // asynchronous copies per wave and step
     HIP_DYNAMIC_SHARED(unsigned char, smem_array)
     TAH_LDS_ZERO_BASED(smem, smem_array);
     const int tid = threadIdx.x, lane = tid % kWave;
@@ -831,13 +837,23 @@ __global__ __launch_bounds__(kLqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
     int seq = 0, row0 = 0, row_end = 0;
     bool second = false;
     const CallBounds cb = call_bounds(p);
-    int slot = (int)(gridDim.y - 1 - blockIdx.y);  // without a table: late (heavy) tiles of each sequence first
-    // (the table's order: heaviest tile of the whole call first)
-    sched_lookup(p.sched, false, p.nseq, G, p.s1.total_q, p.s2.total_q, p.s1.total_k, p.s2.total_k, (int)gridDim.y,
-                 (int)blockIdx.y, slot);
-    if (!(p.s1.total_q > 0 && find_tile(p.s1.cu_q, p.s1.q_shift, p.nseq, BM, slot, seq, row0, row_end, cb.q1))) {
-        if (!(p.s2.total_q > 0 && find_tile(p.s2.cu_q, p.s2.q_shift, p.nseq, BM, slot, seq, row0, row_end, cb.q2))) return;
+    // (the table's order: heaviest tile of the whole call first; its tiles have kPerEntry * BM rows)
+    constexpr int kPerEntry = 4 / kUnits;
+    int slot, tile_rows = kPerEntry * BM;
+    const bool table = sched_lookup(p.sched, false, p.nseq, G, p.s1.total_q, p.s2.total_q, p.s1.total_k, p.s2.total_k,
+                                    (int)gridDim.y / kPerEntry, (int)blockIdx.y / kPerEntry, slot);
+    if (!table) {
+        slot = (int)(gridDim.y - 1 - blockIdx.y);  // late (heavy) tiles of each sequence first
+        tile_rows = BM;
+    }
+    if (!(p.s1.total_q > 0 && find_tile(p.s1.cu_q, p.s1.q_shift, p.nseq, tile_rows, slot, seq, row0, row_end, cb.q1))) {
+        if (!(p.s2.total_q > 0 && find_tile(p.s2.cu_q, p.s2.q_shift, p.nseq, tile_rows, slot, seq, row0, row_end, cb.q2))) return;
         second = true;
+    }
+    if (kPerEntry > 1 && table) {
+        row0 += BM * ((int)blockIdx.y % kPerEntry);
+        if (row0 >= row_end) return;
+        row_end = row0 + BM < row_end ? row0 + BM : row_end;
     }
     const BwdStream& qs = second ? p.s2 : p.s1;
     LaneBounds own1{0, 0};
@@ -885,9 +901,10 @@ __global__ __launch_bounds__(kLqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
 
     // asynchronous copies of one step: K rows as in the dQ kernel (4 rows per copy, two copies per wave), then four
     // 1 KiB pieces of my unit's dS: piece pi = 4 * dh + j covers the key-tile kernel's wave (pi / 4, 2 * hh + (pi % 4) / 2)
-    const int my_lrow = 8 * wave + (lane >> 4);
-    const uint32_t my_chunk0 = (uint32_t)(((lane & 15) ^ row_swizzle(my_lrow)) * 16);
-    const uint32_t my_chunk1 = (uint32_t)(((lane & 15) ^ row_swizzle(my_lrow + 4)) * 16);
+    const int my_lrow = 4 * kPieces * wave + (lane >> 4);
+    uint32_t my_chunk[kPieces];
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) my_chunk[i] = (uint32_t)(((lane & 15) ^ row_swizzle(my_lrow + 4 * i)) * 16);
     auto issue_step = [&](int s, int stage) {
         const bool s0 = s < n1;
         const int ks = s0 ? s : s - n1;  // 64-key step inside its segment
@@ -895,11 +912,12 @@ __global__ __launch_bounds__(kLqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
         const __bf16* kt0 = (s0 ? k1p : k2p) + (int64_t)ks * kBN * krs;
         const int last = (s0 ? lk1 : lk2) - 1 - ks * kBN;
         auto* kt = smem + stage * kLqStage;
-        const uint32_t r0 = (uint32_t)(my_lrow < last ? my_lrow : last) & 63u;
-        const uint32_t r1 = (uint32_t)(my_lrow + 4 < last ? my_lrow + 4 : last) & 63u;
         const uint32_t krs2 = (uint32_t)(krs * 2) & 0xffffffu;
-        async_copy_16B(kt0, r0 * krs2 + my_chunk0, kt + (2 * wave) * 1024);
-        async_copy_16B(kt0, r1 * krs2 + my_chunk1, kt + (2 * wave + 1) * 1024);
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+            const uint32_t r = (uint32_t)(my_lrow + 4 * i < last ? my_lrow + 4 * i : last) & 63u;
+            async_copy_16B(kt0, r * krs2 + my_chunk[i], kt + (kPieces * wave + i) * 1024);
+        }
         const int ktile = (s0 ? 0 : p.ds_kt1) + ks / 2, hh = ks % 2;
         const unsigned char* blk = ds_unit + (int64_t)ktile * kDsBlockBytes;
         auto* dst = kt + kTileBytes + unit * 8192 + dh * 4096;
@@ -959,16 +977,20 @@ __global__ __launch_bounds__(kLqThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dq_
         }
     };
 
-    if (nsteps > 0) issue_step(0, 0);
-    if (nsteps > 1) issue_step(1, 1);
+#pragma unroll
+    for (int s = 0; s < kLqStages - 1; ++s)
+        if (s < nsteps) issue_step(s, s);
     int stage = 0;
     for (int s = 0; s < nsteps; ++s) {
-        // the copies of step s are in; those of step s + 1 (the last kLqCopies this wave issued) may still be on their way
-        if (s + 1 < nsteps) TAH_WAIT_VMEM_N(kLqCopies); else TAH_WAIT_VMEM();
+        // the copies of step s are in; those of the steps behind it (the last this wave issued) may still be on their way
+        const int behind = nsteps - 1 - s;
+        if (behind >= kLqStages - 2) TAH_WAIT_VMEM_N((kLqStages - 2) * kLqCopies);
+        else if (kLqStages > 3 && behind == 1) TAH_WAIT_VMEM_N(kLqCopies);
+        else TAH_WAIT_VMEM();
         __syncthreads();
-        if (s + 2 < nsteps) issue_step(s + 2, stage == 0 ? 2 : stage - 1);
+        if (behind >= kLqStages - 1) issue_step(s + kLqStages - 1, stage == 0 ? kLqStages - 1 : stage - 1);
         if (s >= n1 ? unit_ok : s < my_n1) compute(stage);
-        stage = stage == 2 ? 0 : stage + 1;
+        stage = stage == kLqStages - 1 ? 0 : stage + 1;
     }
 
     if (unit_ok) {
@@ -1061,11 +1083,21 @@ int launch_bwd(const BwdParams& p, hipStream_t st) {
                     return TAH_E_LAUNCH;
                 hipLaunchKernelGGL((duo_bwd_dkdv_kernel<G, false, true>), dim3(p.hkv, ktiles), dim3(kKvThreads), kKvSmem, st, p);
             }
+            if constexpr (G <= kLqUnitsFew) {
+                if (qtiles > 0 && (long)p.hkv * qtiles <= kLqFewWorkgroups) {
+                    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&duo_bwd_dq_from_ds_kernel<G, kLqUnitsFew>),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, lq_smem(kLqUnitsFew)) != hipSuccess)
+                        return TAH_E_LAUNCH;
+                    hipLaunchKernelGGL((duo_bwd_dq_from_ds_kernel<G, kLqUnitsFew>), dim3(p.hkv, 4 / kLqUnitsFew * qtiles),
+                                       dim3(lq_threads(kLqUnitsFew)), lq_smem(kLqUnitsFew), st, p);
+                    return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
+                }
+            }
             if (qtiles > 0) {
                 if (hipFuncSetAttribute(reinterpret_cast<const void*>(&duo_bwd_dq_from_ds_kernel<G>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLqSmem) != hipSuccess)
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, lq_smem(4)) != hipSuccess)
                     return TAH_E_LAUNCH;
-                hipLaunchKernelGGL((duo_bwd_dq_from_ds_kernel<G>), dim3(p.hkv, qtiles), dim3(kLqThreads), kLqSmem, st, p);
+                hipLaunchKernelGGL((duo_bwd_dq_from_ds_kernel<G>), dim3(p.hkv, qtiles), dim3(lq_threads(4)), lq_smem(4), st, p);
             }
             return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
         }

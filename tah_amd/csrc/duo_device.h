@@ -264,8 +264,8 @@ __device__ __forceinline__ void async_copy_4B(const void* sbase, uint32_t voff, 
 #define TAH_WAVES_PER_EU(lo, hi) __attribute__((amdgpu_waves_per_eu(lo, hi)))
 #endif
 #ifndef TAH_WAIT_VMEM_N
-// s_waitcnt vmcnt(n), n <= 15: all but the n most recently issued loads / asynchronous copies have landed
-#define TAH_WAIT_VMEM_N(n) __builtin_amdgcn_s_waitcnt(0x0F70 | (n))
+// s_waitcnt vmcnt(n), n <= 63: all but the n most recently issued loads / asynchronous copies have landed
+#define TAH_WAIT_VMEM_N(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | ((n) >> 4 << 14))
 #endif
 
 // LDS tile of R rows x 128 bf16 (256 B per row, 16 chunks of 16 B).  The chunk index is XORed

@@ -95,3 +95,30 @@ def test_ds_exchange_against_three_kernel_backward_on_cpu_shim(hq, hkv, seqlens,
         if n[1] != "q":
             assert torch.equal(new[i], old[i]), n
     assert any(not torch.equal(new[i], old[i]) for i in (0, 3)) or dev["q1"].shape[0] < 8
+
+
+@pytest.mark.parametrize("lens,p", [([70, 1, 129], 0.3), ([140], 0.6)])
+def test_two_units_to_a_workgroup_give_the_bits_of_four(lens, p):
+    """Few workgroups: dQ's hold two (64 rows, head) units (two heads of a kv head, or two tiles of one).  The same heads four at a time
+    run four: the same dQ bits, with a launch-order table and without (ragged last tiles, one-row sequences, more steps than stages)."""
+    from tah_amd import ops
+    four = _to_dev(make_varlen_case(77, lens, p, Hq=4, Hkv=1, D=128))
+
+    def grads(dev, heads, table):
+        g = torch.Generator().manual_seed(9)
+        do1, do2 = [torch.randn(t.shape, generator=g).to(torch.bfloat16)[:, heads] for t in (four["q1"], four["q2"])]
+        d = dict(dev, q1=dev["q1"][:, heads].contiguous(), q2=dev["q2"][:, heads].contiguous())
+        sched = ops.duo_schedule(d["cu_q1"], d["cu_k1"], d["cu_q2"], d["cu_k2"], d["pos_q2"], d["q1"].shape[1], 1, d["q1"].shape[0],
+                                 d["k1"].shape[0], d["k2"].shape[0]) if table else None
+        o1, l1, o2, l2 = [t[:, heads].contiguous() if t.dim() == 3 else t[heads].contiguous() for t in whole]
+        got = ops.duo_bwd_varlen(d["q1"], d["k1"], d["v1"], o1, l1, do1.contiguous(), d["cu_q1"], d["cu_k1"], d["q2"], d["k2"], d["v2"], o2, l2,
+                                 do2.contiguous(), d["pos_q2"], d["pos_k2"], d["cu_q2"], d["cu_k2"], d["scale"], schedule=sched)
+        return got[0], got[3]
+
+    with emu_util.emulated():
+        whole = ops.duo_fwd_varlen(*varlen_args(four))
+        want = grads(four, slice(0, 4), False)
+        for heads in (slice(0, 2), slice(3, 4)):
+            for table in ((False, True) if heads.start == 0 else (True,)):
+                for a, b in zip(grads(four, heads, table), want):
+                    assert torch.equal(a, b[:, heads])
