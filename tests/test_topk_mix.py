@@ -37,6 +37,18 @@ def test_topk_mix_on_cpu_shim(seed, rows, V, H, k, kw):
 
 
 @pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+@pytest.mark.parametrize("V,H,k", [(90, 32, 17), (300, 96, 100)])
+def test_columns_of_a_row_shared_by_workgroups_have_the_bits_of_one(V, H, k):
+    """Up to 64 rows several workgroups share a row's columns, above one has them all."""
+    from tah_amd import ops
+    logits, emb = [to_torch(t, "cpu") for t in make_case(7, 1, V, H, ties=0.1)]
+    with emu_util.emulated():
+        few = ops.topk_mix(logits, emb, k)
+        many = ops.topk_mix(logits.expand(65, V).contiguous(), emb, k)
+    assert torch.equal(many, few.expand(65, H))
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
 def test_topk_mix_golden_and_row_enable_on_cpu_shim():
     from tah_amd import ops
     z = np.load(GOLDEN)
