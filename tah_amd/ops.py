@@ -198,8 +198,8 @@ def sample_rows(logits: torch.Tensor, uniforms: torch.Tensor, temperature: float
     inverse-CDF draw over the tokens in descending order of probability, equal ones by ascending index.  Rows whose
     ``add_prev`` entry (int32 [rows]) is not 0 draw from ``logits_prev + logits`` (summed in bf16).  ``uniform_step`` (int32
     [rows]): ``uniforms`` is a table [steps, rows] and row r takes ``uniforms[uniform_step[r], r]``.  Returns int64 [rows]."""
-    if out is None:
-        out = torch.zeros(logits.size(0), dtype=torch.int64, device=logits.device)
+    if out is None:  # (every row that is not left out is written)
+        out = (torch.empty if row_enable is None else torch.zeros)(logits.size(0), dtype=torch.int64, device=logits.device)
     _call("sample_rows", logits, logits_prev, add_prev, uniforms, out, None, row_enable, float(temperature), float(top_p), float(min_p),
           uniform_step)
     return out

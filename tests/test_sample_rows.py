@@ -29,6 +29,14 @@ def make_rows(seed, rows, V, style):
     elif style == "wide":      # values across both halves of the key space, with -inf entries (masked tokens)
         x = rng.standard_normal((rows, V)) * 8.0
         x[:, ::7] = -np.inf
+    elif style == "clear":     # a trained model's shape: a few tokens stand clear, top_p cuts among them, masked tokens
+        x = rng.standard_normal((rows, V))
+        x[:, 11::97] = -np.inf
+        x[:, [3, V // 2, V - 1, 5, 7]] = 30.0 + rng.uniform(-2.0, 0.0, size=(rows, 5))
+    elif style == "edge":      # (at temperature 0.7, top_p 0.9) whether the second token is kept hangs on the sum of all the light ones
+        x = np.full((rows, V), 20.0 + 0.7 * np.log(0.05 / V))
+        x[:, V // 3] = 20.0
+        x[:, V // 2] = 20.0 + 0.7 * np.log(np.where(np.arange(rows) % 2, 0.02, 0.08))
     else:
         raise ValueError(style)
     return bf16_round(x.astype(np.float32))
@@ -84,6 +92,10 @@ EMU_CASES = [
     (5, 1, 700, "ties", 1.0, 1.0, 0.3, False),        # min_p alone, cutting between two levels
     (6, 2, 900, "peaked", 1.3, 1.0, 0.0, True),       # plain temperature sampling
     (7, 1, 17000, "flat", 0.6, 0.3, 0.0, False),
+    (8, 2, 9003, "clear", 0.7, 0.9, 0.0, False),      # only the heavy tokens are counted
+    (9, 2, 4000, "clear", 0.7, 0.6, 0.1, True),
+    (10, 2, 3000, "edge", 0.7, 0.9, 0.0, False),      # begun so, and counted again: kept in one row, left out in the other
+    (11, 1, 1500, "clear", 9.0, 0.97, 0.0, False),    # so hot that every token is heavy
 ]
 
 
@@ -148,6 +160,8 @@ GPU_CASES = [
     (25, 5, 32000, "peaked", 1.0, 0.5, 0.0, False),
     (26, 2, 155648, "flat", 1.5, 1.0, 0.0, False),
     (27, 3, 50257, "peaked", 0.8, 0.9, 0.05, False),
+    (28, 3, 151936, "clear", 0.7, 0.9, 0.0, True),
+    (29, 2, 151936, "edge", 0.7, 0.9, 0.0, False),
 ]
 
 
