@@ -682,20 +682,21 @@ __global__ __launch_bounds__(kChunkThreads) void delta_chunk_kernel(const tah_de
     }
 }
 
-// One workgroup per 16-column slice of a (sequence, head).  Workgroups go to the XCDs round robin: the slices of a head are
+// One workgroup per slice of 16 CS columns of a (sequence, head).  Workgroups go to the XCDs round robin: the slices of a head are
 // placed on one XCD, whose L2 then fetches what they share once.  Waves 0 and 1 form u, waves 2 and 3 the results; a
-// wave holds 16 kOwn rows of the state's slice: register r of lane (c, g) of its tile i is S[kOwn (16 wave + c) + i][4 g + r].
-template <int NT>
-__global__ __launch_bounds__(kDeltaThreads) void delta_chunk_scan_kernel(const tah_delta_layer L, const tah_portions P, const float* q, const float* k,
+// wave holds 16 kOwn rows of the state's slice: register r of lane (c, g) of its tile i is S[kOwn (16 wave + c) + i][4 g + r]
+// of the slice's first 16 columns (then of the next).  CS = 2: scan_columns.
+template <int NT, int CS>
+__global__ __launch_bounds__(kDeltaThreads) TAH_WAVES_PER_EU((NT <= 8 ? 2 : 1), 2) void delta_chunk_scan_kernel(const tah_delta_layer L, const tah_portions P, const float* q, const float* k,
                                                                          const float* work, float* o) {
     constexpr int D = 16 * NT, kOwn = (NT + 3) / 4;
     typedef __attribute__((__vector_size__(kOwn * sizeof(float)))) float own_t;
-    __shared__ __align__(16) float st[16][D + 4];           // S^T
-    __shared__ __align__(16) float ut[16][kChunk + 4], us[16][kChunk + 4];  // u^T, and times exp(G_last - G_s)
+    __shared__ __align__(16) float st[16 * CS][D + 4];           // S^T
+    __shared__ __align__(16) float ut[16 * CS][kChunk + 4], us[16 * CS][kChunk + 4];  // u^T, and times exp(G_last - G_s)
     const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), c = lane % 16, g = lane / 16;
-    const int slices = L.vdim / 16, item = blockIdx.x / 8 / slices * 8 + blockIdx.x % 8;
+    const int slices = L.vdim / (16 * CS), item = blockIdx.x / 8 / slices * 8 + blockIdx.x % 8;
     if (item >= L.heads * P.nseq) return;
-    const int h = item % L.heads, b = item / L.heads, kh = h / (L.heads / L.kv_heads), v0 = 16 * (blockIdx.x / 8 % slices);
+    const int h = item % L.heads, b = item / L.heads, kh = h / (L.heads / L.kv_heads), v0 = 16 * CS * (blockIdx.x / 8 % slices);
     const int first = P.cu[b], n = P.cu[b + 1] - first, slot = P.slot[b];
     if (n <= 0 || slot < 0 || slot >= L.nslots) return;
     int64_t chunk0 = 0;  // chunks of the sequences before
@@ -704,25 +705,29 @@ __global__ __launch_bounds__(kDeltaThreads) void delta_chunk_scan_kernel(const t
     const bool holds = wave * kOwn < NT, fresh = P.pos0[b] == 0;
     const int own = holds ? kOwn * (16 * wave + c) : 0;  // its first row of the state
     float* const S = L.state + ((int64_t)slot * L.heads + h) * D * L.vdim + (int64_t)own * L.vdim + v0 + 4 * g;
-    f32x4 s[kOwn];
+    f32x4 s[CS][kOwn];
     auto publish = [&]() __attribute__((always_inline)) {
         if (!holds) return;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            own_t y;
+        for (int e = 0; e < CS; ++e)
 #pragma unroll
-            for (int i = 0; i < kOwn; ++i) y[i] = s[i][r];
-            *reinterpret_cast<own_t*>(&st[4 * g + r][own]) = y;
-        }
+            for (int r = 0; r < 4; ++r) {
+                own_t y;
+#pragma unroll
+                for (int i = 0; i < kOwn; ++i) y[i] = s[e][i][r];
+                *reinterpret_cast<own_t*>(&st[16 * e + 4 * g + r][own]) = y;
+            }
     };
 #pragma unroll
-    for (int i = 0; i < kOwn; ++i)
-        s[i] = holds && !fresh ? *reinterpret_cast<const f32x4*>(S + (int64_t)i * L.vdim) : f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int e = 0; e < CS; ++e)
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i)
+            s[e][i] = holds && !fresh ? *reinterpret_cast<const f32x4*>(S + (int64_t)i * L.vdim + 16 * e) : f32x4{0.f, 0.f, 0.f, 0.f};
     publish();
     const bool former = wave < 2;
     const int tr = 16 * (wave % 2);  // the wave's rows of a chunk
     struct Loads {
-        f32x4 a[NT], p[2], u0, gam;
+        f32x4 a[NT], p[2], u0[CS], gam;
         own_t kk[8];
         float all;
     } buf0, buf1;
@@ -741,7 +746,9 @@ __global__ __launch_bounds__(kDeltaThreads) void delta_chunk_scan_kernel(const t
 #pragma unroll
         for (int i = 0; i < NT; ++i) x.a[i] = *reinterpret_cast<const f32x4*>(ab + (ao + 16 * i + 4 * g));
 #pragma unroll
-        for (int r = 0; r < 4; ++r) x.u0[r] = wu[(unsigned)((tr + 4 * g + r) * L.vdim + c)];
+        for (int e = 0; e < CS; ++e)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x.u0[e][r] = wu[(unsigned)((tr + 4 * g + r) * L.vdim + 16 * e + c)];
 #pragma unroll
         for (int i = 0; i < 2; ++i) x.p[i] = *reinterpret_cast<const f32x4*>(wp + (unsigned)((tr + c) * kChunk + 16 * i + 4 * g));
         x.gam = *reinterpret_cast<const f32x4*>(wg + (unsigned)((former ? kChunk : 0) + tr + 4 * g));
@@ -753,65 +760,93 @@ __global__ __launch_bounds__(kDeltaThreads) void delta_chunk_scan_kernel(const t
         }
     };
     // the results of a chunk are written during the next one, so that no load waits behind a store just issued
-    f32x4 done = {0.f, 0.f, 0.f, 0.f};
+    f32x4 done[CS];
+#pragma unroll
+    for (int e = 0; e < CS; ++e) done[e] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto flush = [&](int ch) __attribute__((always_inline)) {
         if (former || ch < 0) return;
         float* const ob = o + ((int64_t)(first + ch * kChunk) * L.heads + h) * L.vdim + v0;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int t = tr + 4 * g + r;
-            if (ch * kChunk + t < n) ob[(unsigned)(t * L.heads * L.vdim + c)] = done[r];
+            if (ch * kChunk + t < n) {
+#pragma unroll
+                for (int e = 0; e < CS; ++e) ob[(unsigned)(t * L.heads * L.vdim + 16 * e + c)] = done[e][r];
+            }
         }
     };
     auto step = [&](int ch, const Loads& cur, Loads& nxt) __attribute__((always_inline)) {
         fetch(ch + 1 < chunks ? ch + 1 : ch, nxt);
         __builtin_amdgcn_sched_barrier(0);
         // W S or Q S
-        f32x4 x0 = {0.f, 0.f, 0.f, 0.f}, x1 = x0;
+        f32x4 x0[CS], x1[CS];
+#pragma unroll
+        for (int e = 0; e < CS; ++e) x0[e] = x1[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < NT; ++i) {
-            const f32x4 y = *reinterpret_cast<const f32x4*>(&st[c][16 * i + 4 * g]);
-            x0 = mfma_f32(cur.a[i][0], y[0], x0);
-            x1 = mfma_f32(cur.a[i][1], y[1], x1);
-            x0 = mfma_f32(cur.a[i][2], y[2], x0);
-            x1 = mfma_f32(cur.a[i][3], y[3], x1);
+            f32x4 y[CS];
+#pragma unroll
+            for (int e = 0; e < CS; ++e) y[e] = *reinterpret_cast<const f32x4*>(&st[16 * e + c][16 * i + 4 * g]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int e = 0; e < CS; ++e) {
+                    f32x4& x = r % 2 ? x1[e] : x0[e];
+                    x = mfma_f32(cur.a[i][r], y[e][r], x);
+                }
         }
         flush(ch - 1);
-        f32x4 res;
+        f32x4 res[CS];
         if (former) {
-            f32x4 u, w;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                u[r] = cur.u0[r] - (x0[r] + x1[r]);
-                w[r] = u[r] * cur.gam[r];
+            for (int e = 0; e < CS; ++e) {
+                f32x4 u, w;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    u[r] = cur.u0[e][r] - (x0[e][r] + x1[e][r]);
+                    w[r] = u[r] * cur.gam[r];
+                }
+                *reinterpret_cast<f32x4*>(&ut[16 * e + c][tr + 4 * g]) = u;
+                *reinterpret_cast<f32x4*>(&us[16 * e + c][tr + 4 * g]) = w;
             }
-            *reinterpret_cast<f32x4*>(&ut[c][tr + 4 * g]) = u;
-            *reinterpret_cast<f32x4*>(&us[c][tr + 4 * g]) = w;
         } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) res[r] = (x0[r] + x1[r]) * cur.gam[r];
+            for (int e = 0; e < CS; ++e)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) res[e][r] = (x0[e][r] + x1[e][r]) * cur.gam[r];
         }
         __syncthreads();
-        f32x4 uw[2];
+        f32x4 uw[CS][2];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) uw[i] = *reinterpret_cast<const f32x4*>(&us[c][16 * i + 4 * g]);
+        for (int e = 0; e < CS; ++e)
 #pragma unroll
-        for (int i = 0; i < kOwn; ++i)
+            for (int i = 0; i < 2; ++i) uw[e][i] = *reinterpret_cast<const f32x4*>(&us[16 * e + c][16 * i + 4 * g]);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) s[i][r] *= cur.all;
+        for (int e = 0; e < CS; ++e)
+#pragma unroll
+            for (int i = 0; i < kOwn; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[e][i][r] *= cur.all;
 #pragma unroll
         for (int y = 0; y < 8; ++y)
 #pragma unroll
-            for (int i = 0; i < kOwn; ++i) s[i] = mfma_f32(uw[y / 4][y % 4], cur.kk[y][i], s[i]);
+            for (int e = 0; e < CS; ++e)
+#pragma unroll
+                for (int i = 0; i < kOwn; ++i) s[e][i] = mfma_f32(uw[e][y / 4][y % 4], cur.kk[y][i], s[e][i]);
         publish();
         if (!former) {
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                const f32x4 u = *reinterpret_cast<const f32x4*>(&ut[c][16 * i + 4 * g]);
+                f32x4 u[CS];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) res = mfma_f32(cur.p[i][e], u[e], res);
+                for (int e = 0; e < CS; ++e) u[e] = *reinterpret_cast<const f32x4*>(&ut[16 * e + c][16 * i + 4 * g]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int e = 0; e < CS; ++e) res[e] = mfma_f32(cur.p[i][r], u[e][r], res[e]);
             }
-            done = res;
+#pragma unroll
+            for (int e = 0; e < CS; ++e) done[e] = res[e];
         }
         __syncthreads();
     };
@@ -825,8 +860,10 @@ __global__ __launch_bounds__(kDeltaThreads) void delta_chunk_scan_kernel(const t
     }
     flush(chunks - 1);
 #pragma unroll
-    for (int i = 0; i < kOwn; ++i)
-        if (holds) *reinterpret_cast<f32x4*>(S + (int64_t)i * L.vdim) = s[i];
+    for (int e = 0; e < CS; ++e)
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i)
+            if (holds) *reinterpret_cast<f32x4*>(S + (int64_t)i * L.vdim + 16 * e) = s[e][i];
 }
 
 // one wave per (row, head)
@@ -950,12 +987,27 @@ bool chunked(const tah_delta_layer& L, int rows, int nseq) {
 }
 int64_t chunk_slots(int rows, int nseq) { return (int64_t)rows / kChunk + nseq; }
 
+// State columns of a scan's workgroup.  A chunk's W, q and k rows (36 KB) are read for 16 columns or for 32, and those reads out of the L2
+// are what a full launch waits for; with fewer than two workgroups of 16 per compute unit the wider one leaves too many idle.  32 heads of 128 x 128, us
+// with 16 and with 32: one sequence of 1337 101 -> 141 (256 workgroups of 16), two of up to 1500 175 -> 168 (512), four 309 -> 256, eight 530 -> 422, sixteen
+// of 256 255 -> 190, 32 of 128 306 -> 217.  Every sum is the same: the same bits.  Two tiles of columns beside dim = 256 do not fit the registers.
+int scan_columns(const tah_delta_layer& L, int nseq) {
+    return L.dim <= 128 && L.vdim % 32 == 0 && (int64_t)L.heads * nseq * (L.vdim / 16) >= 512 ? 32 : 16;
+}
+
 template <int NT>
 void launch_chunked(const tah_delta_layer& L, const tah_portions& P, const float* q, const float* k, const float* v, const float* lg, const float* beta,
                     float* o, float* work, hipStream_t st) {
     hipLaunchKernelGGL((delta_chunk_kernel<NT>), dim3((unsigned)chunk_slots(P.rows, P.nseq), L.heads), dim3(kChunkThreads), 0, st, L, P, q, k, v, lg,
                        beta, work);
-    hipLaunchKernelGGL((delta_chunk_scan_kernel<NT>), dim3((unsigned)((L.heads * P.nseq + 7) / 8 * 8 * (L.vdim / 16))), dim3(kDeltaThreads), 0, st, L, P, q, k, work, o);
+    const int items = (L.heads * P.nseq + 7) / 8 * 8;
+    if constexpr (NT <= 8) {
+        if (scan_columns(L, P.nseq) == 32) {
+            hipLaunchKernelGGL((delta_chunk_scan_kernel<NT, 2>), dim3((unsigned)(items * (L.vdim / 32))), dim3(kDeltaThreads), 0, st, L, P, q, k, work, o);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((delta_chunk_scan_kernel<NT, 1>), dim3((unsigned)(items * (L.vdim / 16))), dim3(kDeltaThreads), 0, st, L, P, q, k, work, o);
 }
 
 template <class E>

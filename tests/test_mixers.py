@@ -79,6 +79,37 @@ def test_linear_batches_on_cpu_shim():
         Z.linear_batch_case("cpu", 3, 16, 32, 3)
 
 
+def check_delta_columns(dev, dtype, m, lens):
+    """Many sequences' scans hold 32 state columns to a workgroup, one's 16: the same results and states, to the bit."""
+    assert m["heads"] * len(lens) * (m["vdim"] // 16) >= 512 > m["heads"] * (m["vdim"] // 16) and min(lens) >= 48
+    layer, w, cols, width, S = Z.delta_layer(dev, dtype, m, 2 * len(lens), torch.Generator().manual_seed(5))
+    proj = [Z.rnd(torch.Generator().manual_seed(6 + b), n, width).to(dtype) for b, n in enumerate(lens)]
+    out_cols = (m["heads"] * m["vdim"] + 31) // 32 * 32
+
+    def run(seqs, first_slot):
+        P, _ = Z.portions_of([lens[b] for b in seqs], [0] * len(seqs), [first_slot + b for b in seqs], dev)
+        out = torch.zeros((sum(lens[b] for b in seqs), out_cols), dtype=dtype, device=dev)
+        layer.portions(torch.cat([proj[b] for b in seqs]).to(dev), P, out)
+        return out
+
+    together = run(range(len(lens)), 0)
+    alone = torch.cat([run([b], len(lens)) for b in range(len(lens))])
+    assert together.any() and torch.equal(together, alone)
+    assert torch.equal(S[:len(lens)], S[len(lens):])
+
+
+@needs_clang
+def test_delta_scan_columns_on_cpu_shim():
+    with emu_util.emulated():
+        check_delta_columns("cpu", torch.bfloat16, delta(64, 32, 16, 32, 4), (64, 49, 97, 48))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,lens", [(delta(32, 16, 128, 128, 4), (333, 48, 64, 97)), (delta(8, 8, 64, 96, 2), (65,) * 11), (delta(16, 4, 32, 64, 3), (50,) * 9)])
+def test_delta_scan_columns_gpu(m, lens):
+    check_delta_columns("cuda", torch.bfloat16, m, lens)
+
+
 @needs_clang
 @BOTH
 @pytest.mark.parametrize("case", range(len(DELTA_SMALL)))
