@@ -643,6 +643,9 @@ typedef struct tah_decider_tail_args {
     int32_t* q_pos;           /* [rows] out or NULL */
 } tah_decider_tail_args;
 int tah_decider_tail(const tah_decider_tail_args* args, tah_stream_t stream);
+/* tah_decider_tail and, of the rows it calls hard, tah_topk_mix in one launch: the bits of the two calls.  mix->row_enable is
+ * decider->hard, mix->out is not NULL and both have the same rows. */
+int tah_decide_mix(const tah_decider_tail_args* decider, const tah_topk_mix_args* mix, tah_stream_t stream);
 
 /* End of a tick of a generation loop in which every row advances by one latent iteration of its own token, so that a
  * row whose token needs no second iteration does not wait for those that do (the reference's loop,

@@ -367,6 +367,7 @@ PROTOTYPES = {
     "tah_step_begin": (C.c_int, [C.POINTER(StepBeginArgs), c_void_p]),
     "tah_greedy_tick": (C.c_int, [C.POINTER(GreedyTickArgs), c_void_p]),
     "tah_decider_tail": (C.c_int, [C.POINTER(DeciderTailArgs), c_void_p]),
+    "tah_decide_mix": (C.c_int, [C.POINTER(DeciderTailArgs), C.POINTER(TopkMixArgs), c_void_p]),
     "tah_linear_pack_weight": (C.c_int, [c_void_p, c_int64, c_void_p, c_int32, c_int32, c_int32, c_void_p]),
     "tah_linear_pack_rows": (C.c_int, [c_void_p, c_int64, c_void_p, c_int32, c_int32, c_void_p]),
     "tah_linear_rows": (C.c_int, [C.POINTER(LinearRowsArgs), c_void_p]),

@@ -2,15 +2,10 @@
 // they save is launches, one per fused pair per layer per latent iteration).
 #include <hip/hip_runtime.h>
 
-#include "duo_device.h"
-#include "tah_duo.h"
+#include "decide_row.h"
 
 namespace tah {
 namespace {
-
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2e __attribute__((ext_vector_type(2)));
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
 
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {  // two floats -> packed bf16 pair (nearest even)
     const f32x2 v = {lo, hi};
@@ -388,38 +383,11 @@ __global__ __launch_bounds__(256) void step_begin_kernel(const StepBeginParams p
     }
 }
 
-struct DeciderTailParams {
-    const __bf16 *h, *w2, *b2;
-    int64_t h_rs;
-    int32_t width;
-    float threshold;
-    const uint8_t* active;
-    const int32_t* pos;
-    uint8_t* hard;
-    int32_t *hard_i, *slot, *q_pos;
-};
-
-// One wave per row.  z = bf16(h . w2) (float32 sum), + b2 in bf16, sigmoid in float32, > threshold, and active.
+// One wave per row.
 __global__ __launch_bounds__(64) void decider_tail_kernel(const DeciderTailParams p) {
     const int row = blockIdx.x, lane = threadIdx.x;
-    float s = 0.f;
-    for (int c = 8 * lane; c < p.width; c += 8 * 64) {
-        const u32x4 a = *reinterpret_cast<const u32x4*>(p.h + (int64_t)row * p.h_rs + c);
-        const u32x4 b = *reinterpret_cast<const u32x4*>(p.w2 + c);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) s += lo_f(a[q]) * lo_f(b[q]) + hi_f(a[q]) * hi_f(b[q]);
-    }
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m);
-    if (lane != 0) return;
-    float z = lo_f(pack2(s, 0.f));
-    if (p.b2) z = lo_f(pack2(z + (float)p.b2[0], 0.f));
-    const float prob = 1.0f / (1.0f + fast_exp2(-z * kLog2e));
-    const bool hard = prob > p.threshold && (p.active == nullptr || p.active[row] != 0);
-    p.hard[row] = hard ? 1 : 0;
-    if (p.hard_i) p.hard_i[row] = hard ? 1 : 0;
-    if (p.slot) p.slot[row] = hard ? row : -1;
-    if (p.q_pos) p.q_pos[row] = hard ? p.pos[row] : -1;
+    const bool hard = decide_row(p, row, lane);
+    if (lane == 0) put_decision(p, row, hard);
 }
 
 }  // namespace
@@ -520,14 +488,9 @@ extern "C" int tah_step_begin(const tah_step_begin_args* a, tah_stream_t stream)
 extern "C" int tah_decider_tail(const tah_decider_tail_args* a, tah_stream_t stream) {
     using namespace tah;
     if (!a) return TAH_E_NULL;
-    if (a->rows < 0 || a->rows > 65535 || a->width <= 0 || a->width % 8 != 0) return TAH_E_SHAPE;
+    if (int rc = check_decider(*a)) return rc;
     if (a->rows == 0) return TAH_OK;
-    if (!a->hidden || !a->w2 || !a->hard || (a->q_pos && !a->pos)) return TAH_E_NULL;
-    if ((reinterpret_cast<uintptr_t>(a->hidden) & 15) || (reinterpret_cast<uintptr_t>(a->w2) & 15) || a->hidden_row_stride % 8 != 0) return TAH_E_ALIGN;
-    DeciderTailParams p;
-    p.h = static_cast<const __bf16*>(a->hidden); p.w2 = static_cast<const __bf16*>(a->w2); p.b2 = static_cast<const __bf16*>(a->b2);
-    p.h_rs = a->hidden_row_stride; p.width = a->width; p.threshold = a->threshold;
-    p.active = a->active; p.pos = a->pos; p.hard = a->hard; p.hard_i = a->hard_i32; p.slot = a->slot; p.q_pos = a->q_pos;
+    const DeciderTailParams p = decider_params(*a);
     hipLaunchKernelGGL(decider_tail_kernel, dim3(a->rows), dim3(64), 0, static_cast<hipStream_t>(stream), p);
     return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
 }

@@ -14,9 +14,7 @@
 // accumulated in float over bf16-rounded products, as the bf16 eager arithmetic it replaces rounds them.
 #include <hip/hip_runtime.h>
 
-#include "duo_device.h"
-#include "row_keys.h"
-#include "tah_duo.h"
+#include "decide_row.h"
 
 namespace tah {
 namespace {
@@ -45,6 +43,7 @@ struct MixParams {
     int32_t* idxs;  // their vocabulary indices ([rows, v_rs]), or null
     int64_t v_rs;
     const uint8_t* row_enable;
+    DeciderTailParams dec;  // dec.h: the rows are those that this decider calls hard, decided here
     int64_t l_rs, e_rs, o_rs;
     int32_t rows, vocab, hidden, topk;
 };
@@ -121,7 +120,12 @@ __global__ __launch_bounds__(kMixThreads) void topk_mix_kernel(const MixParams p
 
     const int row = blockIdx.x;
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-    if (p.row_enable && !p.row_enable[row]) {  // uniform per workgroup
+    bool on = !p.row_enable || p.row_enable[row];  // uniform per workgroup
+    if (p.dec.h) {  // (every wave for itself, the same sums)
+        on = decide_row(p.dec, row, lane);
+        if (blockIdx.y == 0 && tid == 0) put_decision(p.dec, row, on);
+    }
+    if (!on) {
         if (p.zero_disabled && p.out && blockIdx.y == 0) {
             const bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
             for (int cg = tid; cg < p.hidden / 8; cg += kMixThreads) {
@@ -496,9 +500,9 @@ __global__ __launch_bounds__(kMixThreads) void topk_mix_kernel(const MixParams p
 }  // namespace
 }  // namespace tah
 
-extern "C" int tah_topk_mix(const tah_topk_mix_args* a, tah_stream_t stream) {
-    using namespace tah;
-    if (!a) return TAH_E_NULL;
+namespace tah {
+namespace {
+int run_topk_mix(const tah_topk_mix_args* a, const tah_decider_tail_args* decider, tah_stream_t stream) {
     const bool mix = a->out != nullptr;  // without `out` only values_out is produced
     if (a->rows < 0 || a->vocab <= 0 || a->topk <= 0 || (mix && a->hidden <= 0)) return TAH_E_SHAPE;
     if (a->topk > kMaxTopk || a->vocab > kMaxVec * 8 * kMixThreads || (mix && a->hidden % 8 != 0)) return TAH_E_SHAPE;
@@ -522,7 +526,8 @@ extern "C" int tah_topk_mix(const tah_topk_mix_args* a, tah_stream_t stream) {
     p.vals = static_cast<__bf16*>(a->values_out);
     p.idxs = a->indices_out;
     p.v_rs = a->values_row_stride;
-    p.row_enable = a->row_enable;
+    p.row_enable = decider ? nullptr : a->row_enable;
+    p.dec = decider ? decider_params(*decider) : DeciderTailParams{};
     p.l_rs = a->logits_row_stride; p.e_rs = a->embedding_row_stride; p.o_rs = a->out_row_stride;
     p.rows = a->rows; p.vocab = a->vocab; p.hidden = a->hidden; p.topk = a->topk;
     const int cgs = mix ? a->hidden / 8 : 1;
@@ -537,4 +542,19 @@ extern "C" int tah_topk_mix(const tah_topk_mix_args* a, tah_stream_t stream) {
     else if (nvec <= 14) hipLaunchKernelGGL(topk_mix_kernel<14>, grid, block, smem, st, p);
     else hipLaunchKernelGGL(topk_mix_kernel<kMaxVec>, grid, block, smem, st, p);
     return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
+}
+}  // namespace
+}  // namespace tah
+
+extern "C" int tah_topk_mix(const tah_topk_mix_args* a, tah_stream_t stream) {
+    if (!a) return TAH_E_NULL;
+    return tah::run_topk_mix(a, nullptr, stream);
+}
+
+extern "C" int tah_decide_mix(const tah_decider_tail_args* decider, const tah_topk_mix_args* a, tah_stream_t stream) {
+    if (!a || !decider) return TAH_E_NULL;
+    if (int rc = tah::check_decider(*decider)) return rc;
+    if (decider->rows != a->rows || !a->out) return TAH_E_SHAPE;
+    if (a->row_enable != decider->hard) return TAH_E_NULL;
+    return tah::run_topk_mix(a, decider, stream);
 }

@@ -44,6 +44,7 @@ void load_library(const std::string& path, bool allow_host) {
     bind(g.step_begin, "tah_step_begin");
     bind(g.greedy_tick, "tah_greedy_tick");
     bind(g.decider_tail, "tah_decider_tail");
+    bind(g.decide_mix, "tah_decide_mix");
     bind(g.linear_pack_weight, "tah_linear_pack_weight");
     bind(g.linear_pack_rows, "tah_linear_pack_rows");
     bind(g.linear_rows, "tah_linear_rows");
@@ -729,18 +730,14 @@ void rows_copy(const Tensor& src, const optional<Tensor>& src_rows, const Tensor
              "tah_rows_copy");
 }
 
-Tensor topk_mix(const Tensor& logits, const Tensor& embedding, int64_t topk, const optional<Tensor>& row_enable, const optional<Tensor>& out_,
-                const optional<Tensor>& out_packed, bool zero_disabled, const optional<Tensor>& values_out) {
-    need_lib();
-    Dev d; d.see(logits); d.see(embedding); d.see(row_enable); d.see(out_); d.see(out_packed); d.see(values_out);
+tah_topk_mix_args mix_args(const Tensor& logits, const Tensor& embedding, int64_t topk, const optional<Tensor>& row_enable, const Tensor& out,
+                           const optional<Tensor>& out_packed, bool zero_disabled, Dev& d) {
+    d.see(logits); d.see(embedding); d.see(row_enable); d.see(out); d.see(out_packed);
     TORCH_CHECK(logits.dim() == 2 && embedding.dim() == 2 && logits.scalar_type() == at::kBFloat16 && embedding.scalar_type() == at::kBFloat16,
                 "topk_mix: logits [rows, V] and embedding [V, H] must be bf16");
     TORCH_CHECK(logits.size(1) == embedding.size(0) && logits.stride(1) == 1 && embedding.stride(1) == 1,
                 "topk_mix: vocabulary sizes differ or the inner dimension is not contiguous");
     const int64_t rows = logits.size(0), H = embedding.size(1);
-    // rows that are not enabled: zeros in a fresh tensor (it is zero-filled); in the caller's tensor they keep their
-    // contents unless zero_disabled asks the kernel to write zeros
-    Tensor out = out_.has_value() ? *out_ : (row_enable.has_value() ? at::zeros({rows, H}, embedding.options()) : at::empty({rows, H}, embedding.options()));
     if (out_packed.has_value())
         TORCH_CHECK(out_packed->scalar_type() == at::kBFloat16 && out_packed->is_contiguous() && out_packed->numel() == 32 * H,
                     "topk_mix: out_packed must be a contiguous bf16 tensor of 32 * H elements");
@@ -751,7 +748,7 @@ Tensor topk_mix(const Tensor& logits, const Tensor& embedding, int64_t topk, con
                         row_enable->is_contiguous(),
                     "topk_mix: row_enable must be a contiguous bool/uint8 [rows] tensor");
     tah_topk_mix_args a{};
-    a.logits = ptr(logits); a.embedding = ptr(embedding); a.out = mptr(out);
+    a.logits = ptr(logits); a.embedding = ptr(embedding); a.out = out.data_ptr();
     a.row_enable = static_cast<const uint8_t*>(ptr(row_enable));
     a.logits_row_stride = rows > 1 ? logits.stride(0) : logits.size(1);
     a.embedding_row_stride = embedding.stride(0);
@@ -759,6 +756,19 @@ Tensor topk_mix(const Tensor& logits, const Tensor& embedding, int64_t topk, con
     a.rows = (int32_t)rows; a.vocab = (int32_t)logits.size(1); a.hidden = (int32_t)H; a.topk = (int32_t)topk;
     a.out_packed = out_packed.has_value() ? out_packed->data_ptr() : nullptr;
     a.zero_disabled = zero_disabled ? 1 : 0;
+    return a;
+}
+
+Tensor topk_mix(const Tensor& logits, const Tensor& embedding, int64_t topk, const optional<Tensor>& row_enable, const optional<Tensor>& out_,
+                const optional<Tensor>& out_packed, bool zero_disabled, const optional<Tensor>& values_out) {
+    need_lib();
+    Dev d; d.see(logits); d.see(embedding); d.see(row_enable); d.see(out_); d.see(out_packed); d.see(values_out);
+    TORCH_CHECK(logits.dim() == 2 && embedding.dim() == 2, "topk_mix: logits [rows, V] and embedding [V, H] must be bf16");
+    const int64_t rows = logits.size(0), H = embedding.size(1);
+    // rows that are not enabled: zeros in a fresh tensor (it is zero-filled); in the caller's tensor they keep their
+    // contents unless zero_disabled asks the kernel to write zeros
+    Tensor out = out_.has_value() ? *out_ : (row_enable.has_value() ? at::zeros({rows, H}, embedding.options()) : at::empty({rows, H}, embedding.options()));
+    tah_topk_mix_args a = mix_args(logits, embedding, topk, row_enable, out, out_packed, zero_disabled, d);
     if (values_out.has_value()) {
         TORCH_CHECK(values_out->dim() == 2 && values_out->size(0) == rows && values_out->size(1) == std::min<int64_t>(topk, logits.size(1)) &&
                         values_out->scalar_type() == at::kBFloat16 && values_out->stride(1) == 1,
@@ -1029,11 +1039,10 @@ void greedy_tick(const Tensor& logits, const Tensor& logits_prev, int64_t eos, i
 }
 
 // tah_decider_tail: second layer of the decider, the decision, and the second iteration's per-row bookkeeping.
-void decider_tail(const Tensor& hidden, const Tensor& w2, const optional<Tensor>& b2, double threshold, const optional<Tensor>& active,
-                  const optional<Tensor>& pos, const Tensor& hard, const optional<Tensor>& hard_i32, const optional<Tensor>& slot,
-                  const optional<Tensor>& q_pos) {
-    need_lib();
-    Dev d; d.see(hidden); d.see(w2); d.see(b2); d.see(active); d.see(pos); d.see(hard); d.see(hard_i32); d.see(slot); d.see(q_pos);
+tah_decider_tail_args decider_args(const Tensor& hidden, const Tensor& w2, const optional<Tensor>& b2, double threshold, const optional<Tensor>& active,
+                                   const optional<Tensor>& pos, const Tensor& hard, const optional<Tensor>& hard_i32, const optional<Tensor>& slot,
+                                   const optional<Tensor>& q_pos, Dev& d) {
+    d.see(hidden); d.see(w2); d.see(b2); d.see(active); d.see(pos); d.see(hard); d.see(hard_i32); d.see(slot); d.see(q_pos);
     TORCH_CHECK(hidden.dim() == 2 && hidden.scalar_type() == at::kBFloat16 && (hidden.numel() == 0 || hidden.stride(1) == 1), "decider_tail: hidden must be bf16 [rows, width]");
     const int64_t rows = hidden.size(0), width = hidden.size(1);
     TORCH_CHECK(vec_of(w2, at::kBFloat16, width), "decider_tail: w2 must be a contiguous bf16 tensor of `width` elements");
@@ -1052,7 +1061,28 @@ void decider_tail(const Tensor& hidden, const Tensor& w2, const optional<Tensor>
     a.hard_i32 = hard_i32.has_value() ? static_cast<int32_t*>(hard_i32->data_ptr()) : nullptr;
     a.slot = slot.has_value() ? static_cast<int32_t*>(slot->data_ptr()) : nullptr;
     a.q_pos = q_pos.has_value() ? static_cast<int32_t*>(q_pos->data_ptr()) : nullptr;
+    return a;
+}
+
+void decider_tail(const Tensor& hidden, const Tensor& w2, const optional<Tensor>& b2, double threshold, const optional<Tensor>& active,
+                  const optional<Tensor>& pos, const Tensor& hard, const optional<Tensor>& hard_i32, const optional<Tensor>& slot,
+                  const optional<Tensor>& q_pos) {
+    need_lib();
+    Dev d;
+    const tah_decider_tail_args a = decider_args(hidden, w2, b2, threshold, active, pos, hard, hard_i32, slot, q_pos, d);
     check_rc(g.decider_tail(&a, d.stream()), "tah_decider_tail");
+}
+
+// tah_decide_mix: decider_tail, and topk_mix of the rows it calls hard
+void decide_mix(const Tensor& hidden, const Tensor& w2, const optional<Tensor>& b2, double threshold, const optional<Tensor>& active,
+                const optional<Tensor>& pos, const Tensor& hard, const optional<Tensor>& hard_i32, const optional<Tensor>& slot,
+                const optional<Tensor>& q_pos, const Tensor& logits, const Tensor& embedding, int64_t topk, Tensor out,
+                const optional<Tensor>& out_packed, bool zero_disabled) {
+    need_lib();
+    Dev d;
+    const tah_decider_tail_args a = decider_args(hidden, w2, b2, threshold, active, pos, hard, hard_i32, slot, q_pos, d);
+    const tah_topk_mix_args m = mix_args(logits, embedding, topk, hard, out, out_packed, zero_disabled, d);
+    check_rc(g.decide_mix(&a, &m, d.stream()), "tah_decide_mix");
 }
 
 // ---- linear layers of a decode step (tah_linear_rows) ------------------------------------------------------
@@ -1236,6 +1266,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("step_begin", &step_begin);
     m.def("greedy_tick", &greedy_tick);
     m.def("decider_tail", &decider_tail);
+    m.def("decide_mix", &decide_mix);
     m.def("linear_pack_weight", &linear_pack_weight);
     m.def("linear_pack_rows", &linear_pack_rows);
     m.def("linear_rows", &linear_rows);

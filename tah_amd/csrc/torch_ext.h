@@ -42,6 +42,7 @@ struct Api {
     Entry<decltype(&tah_step_begin)> step_begin;
     Entry<decltype(&tah_greedy_tick)> greedy_tick;
     Entry<decltype(&tah_decider_tail)> decider_tail;
+    Entry<decltype(&tah_decide_mix)> decide_mix;
     Entry<decltype(&tah_linear_pack_weight)> linear_pack_weight;
     Entry<decltype(&tah_linear_pack_rows)> linear_pack_rows;
     Entry<decltype(&tah_norm_linear_supported)> norm_linear_supported;

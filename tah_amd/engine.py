@@ -833,11 +833,11 @@ class TaHDecodeEngine(DecodeEngine):
             self.hard_i.copy_(self.hard)
             torch.where(self.hard, self.rows, self.minus1, out=self.slot1)
             torch.where(self.hard, self.pos, self.minus1, out=self.qpos1)
+            ops.topk_mix(l0, w.embed, c.topk, row_enable=self.hard, out=self.x1, out_packed=self.xp, zero_disabled=True)
         else:
             hr = ops.linear_rows(w.dec_w1_p, self.xp, B, c.decider_hidden, c.hidden, norm_eps=c.rms_eps, bias=w.dec_b1, relu=True)
-            ops.decider_tail(hr, w.dec_w2.reshape(-1), w.dec_b2, w.threshold, hard=self.hard, active=self.act, pos=self.pos,
-                             hard_i32=self.hard_i, slot=self.slot1, q_pos=self.qpos1)
-        ops.topk_mix(l0, w.embed, c.topk, row_enable=self.hard, out=self.x1, out_packed=self.xp, zero_disabled=True)
+            ops.decide_mix(hr, w.dec_w2.reshape(-1), w.dec_b2, w.threshold, l0, w.embed, c.topk, hard=self.hard, active=self.act, pos=self.pos,
+                           hard_i32=self.hard_i, slot=self.slot1, q_pos=self.qpos1, out=self.x1, out_packed=self.xp, zero_disabled=True)
         h1 = self._pass_single_packed(self.x1, self.pos, 1, self.slot1, self.qpos1, self.hard_i, self.cos_rows, self.sin_rows,
                                       rows_packed=True)
         self.hard_len += self.hard_i  # after all layers appended at the old count
@@ -1032,10 +1032,10 @@ class TaHDecodeEngine(DecodeEngine):
         logits = ops.linear_rows(w.lm_head_p, self.xp, B, c.vocab, c.hidden, norm_eps=c.rms_eps, out=self.logits2[parity])
         if self.decider is not None:  # (rows at their second iteration are not eligible: what they left in hs_buf is not used)
             torch.logical_and(self._decide_rows(logits, self.hs_buf), self.eligible, out=self.hard)
+            ops.topk_mix(logits, w.embed, c.topk, row_enable=self.hard, out=self.x1)  # (other rows of x1 are not read)
         else:
             hr = ops.linear_rows(w.dec_w1_p, self.xp, B, c.decider_hidden, c.hidden, norm_eps=c.rms_eps, bias=w.dec_b1, relu=True)
-            ops.decider_tail(hr, w.dec_w2.reshape(-1), w.dec_b2, w.threshold, hard=self.hard, active=self.eligible)
-        ops.topk_mix(logits, w.embed, c.topk, row_enable=self.hard, out=self.x1)  # (other rows of x1 are not read)
+            ops.decide_mix(hr, w.dec_w2.reshape(-1), w.dec_b2, w.threshold, logits, w.embed, c.topk, hard=self.hard, active=self.eligible, out=self.x1)
         chosen = None
         if temperature > 0.0:
             # one draw per row from the final logits as the step-wise loop forms them (first iteration, plus the second

@@ -256,6 +256,13 @@ def decider_tail(hidden, w2, b2, threshold: float, *, hard, active=None, pos=Non
     _call("decider_tail", hidden, w2, b2, float(threshold), active, pos, hard, hard_i32, slot, q_pos)
 
 
+def decide_mix(hidden, w2, b2, threshold: float, logits, embedding, topk: int, *, hard, out, active=None, pos=None, hard_i32=None, slot=None, q_pos=None,
+               out_packed=None, zero_disabled: bool = False) -> None:
+    """``decider_tail`` and ``topk_mix`` of the rows it calls hard (``row_enable=hard``) in one launch (``tah_decide_mix``)."""
+    _call("decide_mix", hidden, w2, b2, float(threshold), active, pos, hard, hard_i32, slot, q_pos, logits, embedding, int(topk), out, out_packed,
+          bool(zero_disabled))
+
+
 LINEAR_MAX_ROWS = 32
 
 

@@ -159,3 +159,63 @@ def test_step_glue_gpu():
     _greedy_tick_case("cuda", V=151936)
     _greedy_tick_case("cuda", V=20480 + 8, workspace=True)
     _greedy_tick_case("cuda", V=151936, workspace=True)
+
+
+def _decide_mix_case(dev, B, W, V, H, k, optional):
+    """The decision and the mix of the rows it calls hard in one launch: the bits of the two calls, with and without what is optional."""
+    from tah_amd import ops
+    g = torch.Generator().manual_seed(11)
+    h = torch.relu(torch.randn(B, W, generator=g)).to(BF).to(dev)
+    w2 = (torch.randn(W, generator=g) * 0.3).to(BF).to(dev)
+    logits, embed = torch.randn(B, V, generator=g).to(BF).to(dev), torch.randn(V, H, generator=g).to(BF).to(dev)
+    pos = torch.arange(B, dtype=torch.int32, device=dev)
+    act = torch.arange(B, device=dev) > 0
+    thr = float(torch.sigmoid(h[1:].float() @ w2.float()).sort().values[:2].mean())  # (the lowest active row is not hard)
+
+    def run(together):
+        hard, out = torch.zeros(B, dtype=torch.bool, device=dev), torch.full((B, H), 7.0, dtype=BF, device=dev)
+        xp = torch.full((32 * H,), 5.0, dtype=BF, device=dev) if optional else None
+        hi, slot, qp = (torch.full((B,), 3, dtype=torch.int32, device=dev) for _ in range(3))
+        tail = dict(active=act, pos=pos, hard_i32=hi, slot=slot, q_pos=qp) if optional else {}
+        if together:
+            ops.decide_mix(h, w2, None, thr, logits, embed, k, hard=hard, out=out, out_packed=xp, zero_disabled=optional, **tail)
+        else:
+            ops.decider_tail(h, w2, None, thr, hard=hard, **tail)
+            ops.topk_mix(logits, embed, k, row_enable=hard, out=out, out_packed=xp, zero_disabled=optional)
+        return [hard, out, hi, slot, qp] + ([xp] if optional else [])
+
+    got, want = run(True), run(False)
+    assert want[0].any() and not want[0].all()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def _decide_mix_refusals(dev, lib):
+    """A mask that is not the decision's, or other rows: refused before anything is launched."""
+    import ctypes as C
+
+    from tah_amd import _capi
+    t = torch.zeros(4096, dtype=BF, device=dev)
+    hard, other = (torch.zeros(4, dtype=torch.bool, device=dev) for _ in range(2))
+    d = _capi.DeciderTailArgs(hidden=t.data_ptr(), hidden_row_stride=64, w2=t.data_ptr(), rows=4, width=64, hard=hard.data_ptr())
+    m = _capi.TopkMixArgs(logits=t.data_ptr(), embedding=t.data_ptr(), out=t.data_ptr(), row_enable=other.data_ptr(), logits_row_stride=32,
+                          embedding_row_stride=32, out_row_stride=32, rows=4, vocab=32, hidden=32, topk=5)
+    call = lambda: lib.tah_decide_mix(C.byref(d), C.byref(m), None)
+    assert call() == -1  # TAH_E_NULL
+    m.row_enable, m.rows = hard.data_ptr(), 3
+    assert call() == -2  # TAH_E_SHAPE
+    m.rows, m.out = 4, None
+    assert call() == -2
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_decide_mix_on_cpu_shim():
+    with emu_util.emulated() as lib:
+        _decide_mix_case("cpu", 5, 64, 300, 32, 17, True)
+        _decide_mix_case("cpu", 3, 520, 90, 16, 100, False)
+        _decide_mix_refusals("cpu", lib)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,W,V,H,k,optional", [(32, 512, 151936, 2048, 100, True), (8, 512, 151936, 2048, 100, False), (70, 64, 3000, 24, 50, False)])
+def test_decide_mix_gpu(B, W, V, H, k, optional):
+    _decide_mix_case("cuda", B, W, V, H, k, optional)
