@@ -371,6 +371,8 @@ PROTOTYPES = {
     "tah_linear_pack_weight": (C.c_int, [c_void_p, c_int64, c_void_p, c_int32, c_int32, c_int32, c_void_p]),
     "tah_linear_pack_rows": (C.c_int, [c_void_p, c_int64, c_void_p, c_int32, c_int32, c_void_p]),
     "tah_linear_rows": (C.c_int, [C.POINTER(LinearRowsArgs), c_void_p]),
+    "tah_linear_beside_supported": (C.c_int, [c_int32, c_int32, c_int32, c_int32]),
+    "tah_linear_beside": (C.c_int, [C.POINTER(LinearRowsArgs), C.POINTER(LinearRowsArgs), c_void_p]),
     "tah_linear_chain_supported": (C.c_int, [c_int32] * 5),
     "tah_linear_chain": (C.c_int, [C.POINTER(LinearChainArgs), c_void_p]),
     "tah_kv_append": (C.c_int, [C.POINTER(KvAppendArgs), c_void_p]),

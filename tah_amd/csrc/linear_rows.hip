@@ -70,6 +70,12 @@ struct LinParams {
     bool by_list;            // products are: seven of eight of 64 experts' workgroups would start only to leave (one row, eight experts of
                              // 2048 x 768, in a captured sequence: gate|up 10.3 -> 8.8 us a launch, down 8.4 -> 5.4; eight rows 10.9 -> 9.5, 9.2 -> 5.7)
     float c0, c1;           // constants of the activation
+    // a second layer over the same rows, with the same norm, as the column groups from groups1 on (or w2 == null): tah_linear_beside
+    const bf16x8* w2;
+    const __bf16* bias2;
+    __bf16* y2;
+    int64_t y2_rs;
+    int32_t act2, groups1;
 };
 
 // 16-byte unit of the packed rows form that holds row r, columns k ... k + 7 (k % 8 == 0)
@@ -128,7 +134,7 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
             if (__ballot(hit) == 0) return;
         }
     }
-    const bf16x8* const pw = p.w + batch * (p.w_bs / 8);
+    const bf16x8* pw = p.w + batch * (p.w_bs / 8);
     const bf16x8* const px = p.x + batch * (p.x_bs / 8);
     int group = blockIdx.x, half = 0;
     if (NH == 1 && (int)gridDim.x == 2 * p.groups) {
@@ -138,6 +144,20 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
         } else {
             group = blockIdx.x / 2;
             half = blockIdx.x % 2;
+        }
+    }
+    const __bf16* bias = p.bias;
+    __bf16* y = p.y + batch * p.y_bs;
+    int64_t y_rs = p.y_rs;
+    int act = p.act;
+    if constexpr (NC == 2 && EPI == kPlainNorm) {
+        if (p.w2 && group >= p.groups1) {  // (uniform)
+            group -= p.groups1;
+            pw = p.w2;
+            bias = p.bias2;
+            y = p.y2;
+            y_rs = p.y2_rs;
+            act = p.act2;
         }
     }
     // The epilogue's own operands (residual, bias: 16 bytes each for a thread that writes results) are asked for here:
@@ -153,7 +173,7 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
         const bool live_row = erow < p.rows;
         // (addresses picked by selects, so that no load sits under a branch)
         const __bf16* ra = (p.res && live_row) ? p.res + (int64_t)erow * p.res_rs + en0 : reinterpret_cast<const __bf16*>(px);
-        const __bf16* ba = p.bias ? p.bias + en0 : reinterpret_cast<const __bf16*>(px);
+        const __bf16* ba = bias ? bias + en0 : reinterpret_cast<const __bf16*>(px);
         res_early = *reinterpret_cast<const bf16x8*>(ra);
         bias_early = *reinterpret_cast<const bf16x8*>(ba);
     }
@@ -394,7 +414,7 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
         } else {
 #pragma unroll
             for (int i = 0; i < 8; ++i) out[i] = (__bf16)(sg[i] * rin);
-            if (p.bias) {
+            if (bias) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) out[i] = (__bf16)((float)out[i] + (float)bias_early[i]);
             }
@@ -402,27 +422,27 @@ __global__ __launch_bounds__(kLinThreads) void linear_rows_kernel(const LinParam
 #pragma unroll
                 for (int i = 0; i < 8; ++i) out[i] = (__bf16)((float)out[i] + (float)res_early[i]);
             }
-            if (p.act == TAH_ACT_RELU) {
+            if (act == TAH_ACT_RELU) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) out[i] = (float)out[i] > 0.f ? out[i] : (__bf16)0.f;
-            } else if (p.act == TAH_ACT_GELU) {
+            } else if (act == TAH_ACT_GELU) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     const float v = (float)out[i];
                     out[i] = (__bf16)(0.5f * v * (1.0f + erff(v * 0.70710678118654752f)));
                 }
-            } else if (p.act == TAH_ACT_GELU_TANH) {
+            } else if (act == TAH_ACT_GELU_TANH) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     const float v = (float)out[i];
                     out[i] = (__bf16)(0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v))));
                 }
-            } else if (p.act == TAH_ACT_XIELU) {
+            } else if (act == TAH_ACT_XIELU) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) out[i] = (__bf16)xielu((float)out[i], p.c0, p.c1);
             }
         }
-        if (p.y) *reinterpret_cast<bf16x8*>(p.y + batch * p.y_bs + (int64_t)row * p.y_rs + n0) = out;
+        if (p.y) *reinterpret_cast<bf16x8*>(y + (int64_t)row * y_rs + n0) = out;
     }
     if (p.yp) {
         bf16x8* const yp = p.yp + batch * (p.yp_bs / 8);
@@ -1349,9 +1369,10 @@ extern "C" int tah_linear_pack_rows(const void* x, int64_t x_row_stride, void* x
     return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
 }
 
-extern "C" int tah_linear_rows(const tah_linear_rows_args* a, tah_stream_t stream) {
-    using namespace tah;
-    if (!a) return TAH_E_NULL;
+namespace tah {
+namespace {
+// beside: a second layer of the same rows in the launch (tah_linear_beside has checked it), or null
+int run_linear_rows(const tah_linear_rows_args* a, const tah_linear_rows_args* beside, tah_stream_t stream) {
     if (a->kind != TAH_LINEAR_PLAIN && a->kind != TAH_LINEAR_GATE_UP) return TAH_E_SHAPE;
     if (a->rows < 0 || a->rows > kLinRows || a->n < 0 || a->k < 0 || a->k % kStepK != 0) return TAH_E_SHAPE;
     const bool gate_up = a->kind == TAH_LINEAR_GATE_UP;
@@ -1407,7 +1428,16 @@ extern "C" int tah_linear_rows(const tah_linear_rows_args* a, tah_stream_t strea
     const int pw = steps % kLinWaves == 0 ? steps / kLinWaves : 0;  // compile-time K for the sizes of the end-to-end model
     if (!gate_up && a->input_norm != TAH_NORM_LAYER && a->n >= kWideFromCols && a->n % (2 * kTileCols) == 0) {
         // an output head: two tiles per workgroup, the rows' operand is read half as often
-        const int groups = a->n / (2 * kTileCols);
+        int groups = a->n / (2 * kTileCols);
+        if (beside) {
+            p.w2 = static_cast<const bf16x8*>(beside->w_packed);
+            p.bias2 = static_cast<const __bf16*>(beside->bias);
+            p.y2 = static_cast<__bf16*>(beside->out);
+            p.y2_rs = beside->out_row_stride;
+            p.act2 = beside->activation;
+            p.groups1 = groups;
+            groups += beside->n / (2 * kTileCols);
+        }
         if (pw == 8 && p.rows > 16 && batch == 1 && p.y && !p.yp && !p.res && !p.bias && p.act == TAH_ACT_NONE && !p.select) {
             if (p.norm) launch_wide<kPlainNorm, 8>(p, groups, st);
             else launch_wide<kPlain, 8>(p, groups, st);
@@ -1447,6 +1477,37 @@ extern "C" int tah_linear_rows(const tah_linear_rows_args* a, tah_stream_t strea
         else launch<2, 2, kGateUp16, 0>(p, groups, batch, st);
     }
     return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
+}
+
+}  // namespace
+}  // namespace tah
+
+extern "C" int tah_linear_rows(const tah_linear_rows_args* a, tah_stream_t stream) {
+    if (!a) return TAH_E_NULL;
+    return tah::run_linear_rows(a, nullptr, stream);
+}
+
+// (More than sixteen rows: the resident workgroups of the head walk ranges of column groups, and with a second layer's among them 32
+// prompts and 96 tokens took 79.6 instead of 77.4 ms.)
+extern "C" int tah_linear_beside_supported(int32_t rows, int32_t n, int32_t k, int32_t beside) {
+    using namespace tah;
+    return rows >= 0 && rows <= 16 && n >= kWideFromCols && n % (2 * kTileCols) == 0 && k > 0 && k % kStepK == 0 && beside > 0 && beside % (2 * kTileCols) == 0;
+}
+
+extern "C" int tah_linear_beside(const tah_linear_rows_args* a, const tah_linear_rows_args* b, tah_stream_t stream) {
+    using namespace tah;
+    if (!a || !b) return TAH_E_NULL;
+    if (!tah_linear_beside_supported(a->rows, a->n, a->k, b->n) || a->kind != TAH_LINEAR_PLAIN || a->batch > 1 || a->residual || a->bias || a->out_packed || a->n_select != 0 ||
+        a->activation != TAH_ACT_NONE || a->input_norm != TAH_NORM_RMS)
+        return TAH_E_SHAPE;
+    if (b->kind != TAH_LINEAR_PLAIN || b->batch < 0 || b->batch > 1 || b->residual || b->out_packed || b->n_select != 0 ||
+        (b->activation != TAH_ACT_NONE && b->activation != TAH_ACT_RELU) || b->input_norm != TAH_NORM_RMS || b->rows != a->rows || b->k != a->k ||
+        b->norm_eps != a->norm_eps || b->out_row_stride < b->n)
+        return TAH_E_SHAPE;
+    if (a->rows == 0) return TAH_OK;
+    if (!a->out || !b->w_packed || !b->out || b->x_packed != a->x_packed) return TAH_E_NULL;
+    if (!aligned16(b->w_packed) || !aligned16(b->out) || !aligned16(b->bias) || b->out_row_stride % 8 != 0) return TAH_E_ALIGN;
+    return run_linear_rows(a, b, stream);
 }
 
 extern "C" int tah_norm_linear_supported(int32_t rows, int32_t cols, int32_t n) {

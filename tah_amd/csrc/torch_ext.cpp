@@ -48,6 +48,8 @@ void load_library(const std::string& path, bool allow_host) {
     bind(g.linear_pack_weight, "tah_linear_pack_weight");
     bind(g.linear_pack_rows, "tah_linear_pack_rows");
     bind(g.linear_rows, "tah_linear_rows");
+    bind(g.linear_beside_supported, "tah_linear_beside_supported");
+    bind(g.linear_beside, "tah_linear_beside");
     bind(g.norm_linear_supported, "tah_norm_linear_supported");
     bind(g.norm_linear, "tah_norm_linear");
     bind(g.norm_route_supported, "tah_norm_route_supported");
@@ -1173,6 +1175,36 @@ optional<Tensor> linear_rows(const Tensor& w_packed, const Tensor& x_packed, int
     return y;
 }
 
+bool linear_beside_supported(int64_t rows, int64_t n, int64_t k, int64_t beside) {
+    need_lib();
+    const auto fits = [](int64_t x) { return x >= 0 && x <= 0x7fffffff; };
+    return fits(rows) && fits(n) && fits(k) && fits(beside) && g.linear_beside_supported((int32_t)rows, (int32_t)n, (int32_t)k, (int32_t)beside) != 0;
+}
+
+// An output head [n, k] and a second layer [n2, k] (bias, ReLU) over the same rows with the same RMSNorm (tah_linear_beside).
+std::tuple<Tensor, Tensor> linear_beside(const Tensor& w_packed, const Tensor& w2_packed, const Tensor& x_packed, int64_t rows, int64_t n, int64_t n2, int64_t k,
+                                         double norm_eps, const optional<Tensor>& out, const optional<Tensor>& bias2, bool relu2) {
+    need_lib();
+    Dev d; d.see(w_packed); d.see(w2_packed); d.see(x_packed); d.see(out); d.see(bias2);
+    TORCH_CHECK(rows >= 0 && n >= 0 && n2 >= 0 && k >= 0, "linear_beside: negative size");
+    TORCH_CHECK(packed_vec(w_packed, n * k) && packed_vec(w2_packed, n2 * k), "linear_beside: weights must come from linear_pack_weight for these sizes");
+    TORCH_CHECK(packed_vec(x_packed, 32 * k), "linear_beside: x_packed must be a contiguous bf16 tensor of 32 * K elements");
+    if (bias2.has_value()) TORCH_CHECK(packed_vec(*bias2, n2), "linear_beside: bias must be a contiguous bf16 [N] tensor");
+    Tensor y = out.has_value() ? *out : at::empty({rows, n}, x_packed.options()), y2 = at::empty({rows, n2}, x_packed.options());
+    TORCH_CHECK(y.dim() == 2 && y.size(0) == rows && y.size(1) == n && y.scalar_type() == at::kBFloat16 && (y.numel() == 0 || y.stride(1) == 1),
+                "linear_beside: out must be bf16 [rows, N]");
+    tah_linear_rows_args a{};
+    a.w_packed = w_packed.data_ptr(); a.x_packed = x_packed.data_ptr();
+    a.out = mptr(y); a.out_row_stride = rows > 1 ? y.stride(0) : n;
+    a.rows = (int32_t)rows; a.n = (int32_t)n; a.k = (int32_t)k;
+    a.kind = TAH_LINEAR_PLAIN; a.input_norm = TAH_NORM_RMS; a.norm_eps = (float)norm_eps;
+    tah_linear_rows_args b = a;
+    b.w_packed = w2_packed.data_ptr(); b.out = mptr(y2); b.out_row_stride = n2; b.n = (int32_t)n2;
+    b.bias = bias2.has_value() ? bias2->data_ptr() : nullptr; b.activation = relu2 ? TAH_ACT_RELU : TAH_ACT_NONE;
+    check_rc(g.linear_beside(&a, &b, d.stream()), "tah_linear_beside");
+    return {y, y2};
+}
+
 bool linear_chain_supported(int64_t rows, int64_t hidden, int64_t o_cols, int64_t ff, int64_t qkv_cols) {
     need_lib();
     const auto fits = [](int64_t v) { return v >= 0 && v <= 0x7fffffff; };
@@ -1267,6 +1299,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("greedy_tick", &greedy_tick);
     m.def("decider_tail", &decider_tail);
     m.def("decide_mix", &decide_mix);
+    m.def("linear_beside_supported", &linear_beside_supported);
+    m.def("linear_beside", &linear_beside);
     m.def("linear_pack_weight", &linear_pack_weight);
     m.def("linear_pack_rows", &linear_pack_rows);
     m.def("linear_rows", &linear_rows);

@@ -43,6 +43,8 @@ struct Api {
     Entry<decltype(&tah_greedy_tick)> greedy_tick;
     Entry<decltype(&tah_decider_tail)> decider_tail;
     Entry<decltype(&tah_decide_mix)> decide_mix;
+    Entry<decltype(&tah_linear_beside_supported)> linear_beside_supported;
+    Entry<decltype(&tah_linear_beside)> linear_beside;
     Entry<decltype(&tah_linear_pack_weight)> linear_pack_weight;
     Entry<decltype(&tah_linear_pack_rows)> linear_pack_rows;
     Entry<decltype(&tah_norm_linear_supported)> norm_linear_supported;

@@ -776,6 +776,15 @@ class TaHDecodeEngine(DecodeEngine):
             return self._rms(h, self.w.norm) @ self.w.lm_head.t()
         return ops.linear_rows(self.w.lm_head_p, self.xp, h.shape[0], c.vocab, c.hidden, norm_eps=c.rms_eps)
 
+    def _head_and_decider(self, out: Optional[torch.Tensor] = None):
+        """Logits [B, V] and the decider's first layer [B, 512] of the rows operand the last layer left in ``self.xp``."""
+        c, w, B = self.cfg, self.w, self.B
+        if ops.linear_beside_supported(B, c.vocab, c.hidden, c.decider_hidden):  # (in the head's launch: one prompt and 96 tokens 41.6 -> 41.3 ms)
+            return ops.linear_beside(w.lm_head_p, w.dec_w1_p, self.xp, B, c.vocab, c.decider_hidden, c.hidden, norm_eps=c.rms_eps, out=out, bias2=w.dec_b1,
+                                     relu2=True)
+        logits = ops.linear_rows(w.lm_head_p, self.xp, B, c.vocab, c.hidden, norm_eps=c.rms_eps, out=out)
+        return logits, ops.linear_rows(w.dec_w1_p, self.xp, B, c.decider_hidden, c.hidden, norm_eps=c.rms_eps, bias=w.dec_b1, relu=True)
+
     def step_logits(self, tok: torch.Tensor, force_hard: Optional[torch.Tensor] = None, active: Optional[torch.Tensor] = None):
         """The iteration loop of tah_model.py:580-706 for one new token per sequence, on ``self.pos``.
 
@@ -827,15 +836,15 @@ class TaHDecodeEngine(DecodeEngine):
                        cos_rows=self.cos_rows, sin_rows=self.sin_rows, slot=self.slot0, q_pos=self.qpos0, active=self.act)
         self._pass_single_packed(self.x0, self.pos, 0, self.slot0, self.qpos0, self.zeros_i, self.cos_rows, self.sin_rows,
                                  rows_packed=True)
-        l0 = self._head(self.x0)
         if self.decider is not None:
+            l0 = self._head(self.x0)
             torch.logical_and(self._decide_rows(l0, self.hs_buf), self.act, out=self.hard)
             self.hard_i.copy_(self.hard)
             torch.where(self.hard, self.rows, self.minus1, out=self.slot1)
             torch.where(self.hard, self.pos, self.minus1, out=self.qpos1)
             ops.topk_mix(l0, w.embed, c.topk, row_enable=self.hard, out=self.x1, out_packed=self.xp, zero_disabled=True)
         else:
-            hr = ops.linear_rows(w.dec_w1_p, self.xp, B, c.decider_hidden, c.hidden, norm_eps=c.rms_eps, bias=w.dec_b1, relu=True)
+            l0, hr = self._head_and_decider()
             ops.decide_mix(hr, w.dec_w2.reshape(-1), w.dec_b2, w.threshold, l0, w.embed, c.topk, hard=self.hard, active=self.act, pos=self.pos,
                            hard_i32=self.hard_i, slot=self.slot1, q_pos=self.qpos1, out=self.x1, out_packed=self.xp, zero_disabled=True)
         h1 = self._pass_single_packed(self.x1, self.pos, 1, self.slot1, self.qpos1, self.hard_i, self.cos_rows, self.sin_rows,
@@ -1029,12 +1038,13 @@ class TaHDecodeEngine(DecodeEngine):
                        append_at=self.append_at, eligible=self.eligible)
         self._pass_single_packed(self.x0, self.pos, None, self.slot0, self.qpos0, self.q_depth_rows, self.cos_rows,
                                  self.sin_rows, rows_packed=True)
-        logits = ops.linear_rows(w.lm_head_p, self.xp, B, c.vocab, c.hidden, norm_eps=c.rms_eps, out=self.logits2[parity])
+        logits = self.logits2[parity]
         if self.decider is not None:  # (rows at their second iteration are not eligible: what they left in hs_buf is not used)
+            ops.linear_rows(w.lm_head_p, self.xp, B, c.vocab, c.hidden, norm_eps=c.rms_eps, out=logits)
             torch.logical_and(self._decide_rows(logits, self.hs_buf), self.eligible, out=self.hard)
             ops.topk_mix(logits, w.embed, c.topk, row_enable=self.hard, out=self.x1)  # (other rows of x1 are not read)
         else:
-            hr = ops.linear_rows(w.dec_w1_p, self.xp, B, c.decider_hidden, c.hidden, norm_eps=c.rms_eps, bias=w.dec_b1, relu=True)
+            _, hr = self._head_and_decider(logits)
             ops.decide_mix(hr, w.dec_w2.reshape(-1), w.dec_b2, w.threshold, logits, w.embed, c.topk, hard=self.hard, active=self.eligible, out=self.x1)
         chosen = None
         if temperature > 0.0:

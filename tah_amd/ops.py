@@ -279,6 +279,17 @@ def linear_pack_rows(x: torch.Tensor, out: Optional[torch.Tensor] = None) -> tor
     return _call("linear_pack_rows", x, out)
 
 
+def linear_beside_supported(rows: int, n: int, k: int, n2: int) -> bool:
+    return bool(lib().linear_beside_supported(int(rows), int(n), int(k), int(n2)))
+
+
+def linear_beside(w_packed, w2_packed, x_packed, rows: int, n: int, n2: int, k: int, *, norm_eps: float, out: Optional[torch.Tensor] = None,
+                  bias2: Optional[torch.Tensor] = None, relu2: bool = False):
+    """An output head and a second layer over the same rows in one launch (``tah_linear_beside``): the results of ``linear_rows(w_packed, ...,
+    norm_eps=, out=)`` and ``linear_rows(w2_packed, ..., norm_eps=, bias=bias2, relu=relu2)``, for ``linear_beside_supported`` sizes."""
+    return _call("linear_beside", w_packed, w2_packed, x_packed, int(rows), int(n), int(n2), int(k), float(norm_eps), out, bias2, bool(relu2))
+
+
 def linear_rows(w_packed: torch.Tensor, x_packed: torch.Tensor, rows: int, n: int, k: int, *, gate_up: bool = False,
                 residual: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None,
                 out_packed: Optional[torch.Tensor] = None, want_out: bool = True, norm_eps: Optional[float] = None,

@@ -549,3 +549,39 @@ def test_linear_rows_select_on_the_cpu_shim():
 @pytest.mark.parametrize("rows,n,k,gate_up", [(1, 768, 2048, True), (9, 48, 2048, True), (20, 96, 320, True), (1, 2048, 768, False), (8, 64, 2048, False), (32, 32, 96, False)])
 def test_linear_rows_select_gpu(rows, n, k, gate_up):
     _select_case("cuda", rows, n, k, gate_up, SELECT_LISTS)
+
+
+def _beside_case(dev, rows, n, n2, k, bias, relu):
+    """An output head and a second layer of the same rows in one launch: the bits of the two calls, and nothing behind either result."""
+    from tah_amd import ops
+    d = lambda t: t.to(dev)
+    w, w2, x = d(_rand((n, k), 1, k ** -0.5)), d(_rand((n2, k), 2, k ** -0.5)), d(_rand((rows, k), 3))
+    b2 = d(_rand((n2,), 4)) if bias else None
+    wp, w2p, xp = ops.linear_pack_weight(w), ops.linear_pack_weight(w2), ops.linear_pack_rows(x)
+    assert ops.linear_beside_supported(rows, n, k, n2)
+    out = torch.full((rows + 1, n + 16), 3.0, dtype=BF, device=dev)
+    y, y2 = ops.linear_beside(wp, w2p, xp, rows, n, n2, k, norm_eps=1e-6, out=out[:rows, :n], bias2=b2, relu2=relu)
+    assert torch.equal(y, ops.linear_rows(wp, xp, rows, n, k, norm_eps=1e-6))
+    assert torch.equal(y2, ops.linear_rows(w2p, xp, rows, n2, k, norm_eps=1e-6, bias=b2, relu=relu))
+    assert (out[rows:] == 3.0).all() and (out[:, n:] == 3.0).all() and y2.any()
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_linear_beside_on_cpu_shim():
+    from tah_amd import ops
+    from tah_amd._capi import TahDuoError
+    with emu_util.emulated():
+        _beside_case("cpu", 3, 16384, 64, 32, True, True)
+        # no head, widths of half a workgroup's, too many rows
+        for rows, n, n2, k in ((1, 16352, 64, 32), (1, 16384 + 16, 64, 32), (1, 16384, 48, 32), (17, 16384, 64, 32)):
+            assert not ops.linear_beside_supported(rows, n, k, n2)
+            z = torch.zeros(n * k, dtype=BF)
+            with pytest.raises(TahDuoError):
+                ops.linear_beside(z, z[:n2 * k], torch.zeros(32 * k, dtype=BF), rows, n, n2, k, norm_eps=1e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 8, 9, 16])
+@pytest.mark.parametrize("n,n2,k,bias,relu", [(151936, 512, 2048, True, True), (16384, 32, 2048, False, False), (32000, 96, 1024, True, False)])
+def test_linear_beside_gpu(rows, n, n2, k, bias, relu):
+    _beside_case("cuda", rows, n, n2, k, bias, relu)
