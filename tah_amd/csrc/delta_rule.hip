@@ -18,7 +18,7 @@
 //    a unit lower triangular system.  The first kernel solves it for all chunks at once, for the two parts of the right
 //    hand side: U0 (from v) and W (from k), so that u = U0 - W S; and forms P[t][s] = exp(G_t - G_s) (q_t . k_s), s <= t.
 //    The second walks the chunks of a sequence: u = U0 - W S, o_t = exp(G_t) S^T q_t + (P u)_t,
-//    S <- exp(G_last) S + sum_s exp(G_last - G_s) k_s u_s^T, a workgroup holding sixteen columns of a head's state.
+//    S <- exp(G_last) S + sum_s exp(G_last - G_s) k_s u_s^T, a workgroup holding sixteen or 32 columns of a head's state.
 //  State and inputs are float32 throughout: no reduced-precision matrix instruction touches the recurrence.
 //
 // The convolution's inputs of the last `taps` tokens are kept as a ring (token p at p % taps): a step writes the entry

@@ -554,7 +554,9 @@ extern "C" int tah_topk_mix(const tah_topk_mix_args* a, tah_stream_t stream) {
 extern "C" int tah_decide_mix(const tah_decider_tail_args* decider, const tah_topk_mix_args* a, tah_stream_t stream) {
     if (!a || !decider) return TAH_E_NULL;
     if (int rc = tah::check_decider(*decider)) return rc;
-    if (decider->rows != a->rows || !a->out) return TAH_E_SHAPE;
+    if (decider->rows != a->rows) return TAH_E_SHAPE;
+    if (a->rows == 0) return TAH_OK;
+    if (!a->out) return TAH_E_SHAPE;
     if (a->row_enable != decider->hard) return TAH_E_NULL;
     return tah::run_topk_mix(a, decider, stream);
 }

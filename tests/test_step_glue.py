@@ -205,6 +205,8 @@ def _decide_mix_refusals(dev, lib):
     assert call() == -2  # TAH_E_SHAPE
     m.rows, m.out = 4, None
     assert call() == -2
+    m.rows = d.rows = 0
+    assert call() == 0  # nothing to do, as for the two calls
 
 
 @pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
