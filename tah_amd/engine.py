@@ -607,32 +607,7 @@ class TaHDecodeEngine(DecodeEngine):
     def _rms(self, x, w):
         return F.rms_norm(x, (x.shape[-1],), w, self.cfg.rms_eps)
 
-    def _few(self, n: int) -> bool:
-        """Whether n rows of a prompt (its hard tokens, a short prompt) take the decode step's linear layers: a product costs its weights there,
-        which they read at two to three times the rate of the library's.  One prompt of 203 tokens, 12 of them hard, and 96 tokens of eight
-        layers: 42.36 -> 41.71 ms (the output heads 205 -> 90 us each)."""
-        return self.packed_linear and 0 < n <= ops.LINEAR_MAX_ROWS
-
-    def _dense(self, x, L, name: str):
-        if self._few(x.shape[0]):
-            n, k = L[name].shape
-            return ops.linear_rows(L[name + "_p"], ops.linear_pack_rows(x.contiguous()), x.shape[0], n, k)
-        return x @ L[name].t()
-
-    def _prompt_head(self, x, rows, normed):
-        """Logits of some rows of ``x``, the last layer's result, or of ``normed``, the same behind the final norm."""
-        if self._few(rows.numel()) and self.w.lm_head_p is not None:
-            c = self.cfg
-            return ops.linear_rows(self.w.lm_head_p, ops.linear_pack_rows(x[rows]), rows.numel(), c.vocab, c.hidden, norm_eps=c.rms_eps)
-        return normed[rows] @ self.w.lm_head.t()
-
     def _mlp(self, x, L):
-        if self._few(x.shape[0]):
-            c = self.cfg
-            act = torch.empty(32 * c.intermediate, dtype=x.dtype, device=x.device)
-            ops.linear_rows(L["wgu_p"], ops.linear_pack_rows(x), x.shape[0], c.intermediate, c.hidden, gate_up=True, out_packed=act, want_out=False,
-                            norm_eps=c.rms_eps)
-            return ops.linear_rows(L["wdown_p"], act, x.shape[0], c.hidden, c.intermediate, residual=x, out=x)
         if self.w.norms_folded:  # the norm's weight sits in wgu, its per-row factor is applied with the gate
             h = ops.silu_mul(x @ L["wgu"].t(), norm_input=x, norm_eps=self.cfg.rms_eps)
         else:
@@ -643,7 +618,7 @@ class TaHDecodeEngine(DecodeEngine):
         """Prepared q, k and v of packed prompt rows (input norm, projections, q/k norm, rotary embedding)."""
         c = self.cfg
         if self.w.norms_folded:
-            q, k, v = self._split_qkv(self._dense(x, L, "wqkv"))
+            q, k, v = self._split_qkv(x @ L["wqkv"].t())
             return qk_norm_rope(q, k, L["qn"], L["kn"], cos, sin, c.rms_eps, v=v, norm_input=x, norm_eps=c.rms_eps)
         q, k, v = self._split_qkv(self._rms(x, L["ln1"]) @ L["wqkv"].t())
         qo, ko = qk_norm_rope(q, k, L["qn"], L["kn"], cos, sin, c.rms_eps)
@@ -901,7 +876,7 @@ class TaHDecodeEngine(DecodeEngine):
                                              schedule=sched0)
             self.slabs0[l].append(ko, v, cu)
             kv_tok.append((ko, v))
-            x = x + self._dense(o1.view(N, -1), L, "wo")
+            x = x + o1.view(N, -1) @ L["wo"].t()
             x = self._mlp(x, L)
             self._keep_hidden(l + 1, x, hs_sel)
         h0 = self._rms(x, w.norm)
@@ -924,7 +899,7 @@ class TaHDecodeEngine(DecodeEngine):
                 w.threshold = float(torch.quantile(prob, 1.0 - calibrate))
             hard = (prob > w.threshold) if force_hard is None else force_hard
         last = (cu[1:] - 1).long()
-        logits_last = self._prompt_head(x, last, h0)  # model dtype, like the reference's logits buffers
+        logits_last = (h0[last] @ w.lm_head.t())  # model dtype, like the reference's logits buffers
         rows2 = torch.nonzero(hard).flatten()
         n2 = rows2.numel()
         if n2:
@@ -932,7 +907,7 @@ class TaHDecodeEngine(DecodeEngine):
             if int(counts.max()) > self.max_hard:
                 raise TahDuoError("more hard tokens in a prompt than the depth-1 cache holds")
             cu2 = torch.cat([torch.zeros(1, dtype=torch.long, device=dev), counts.cumsum(0)]).to(torch.int32)
-            l0h = self._prompt_head(x, rows2, h0)
+            l0h = h0[rows2] @ w.lm_head.t()
             x2 = ops.topk_mix(l0h, w.embed, c.topk)
             pos2 = pos[rows2].contiguous()
             cos2, sin2 = self.cos[pos2.long()], self.sin[pos2.long()]
@@ -943,9 +918,9 @@ class TaHDecodeEngine(DecodeEngine):
                 _, _, o2, _ = ops.duo_fwd_varlen(qo[:0], k1, v1, zc, cu, qo, ko, v, pos2, pos2, cu2, cu2, self.scale,
                                                  schedule=sched1)
                 self.slabs1[l].append(ko, v, cu2, pos_new=pos2)
-                x2 = x2 + self._dense(o2.view(n2, -1), L, "wo")
+                x2 = x2 + o2.view(n2, -1) @ L["wo"].t()
                 x2 = self._mlp(x2, L)
-            l1h = self._prompt_head(x2, torch.arange(n2, device=dev), self._rms(x2, w.norm))
+            l1h = self._rms(x2, w.norm) @ w.lm_head.t()
             both = l0h + l1h
             # a prompt whose last token is hard: its final logits are the sum of both iterations'
             is_last = torch.isin(rows2, last)
