@@ -309,30 +309,31 @@ class _BlockAttn(torch.autograd.Function):
         else:
             o, lse, _, _ = ops.duo_fwd_varlen(qp, k1, v1, b.cu_q, b.cu_k1, none, k2p, v2p, b.none_pos, b.none_pos, b.none_cu, b.none_cu, b.scale,
                                               b.schedule, b.pairs)
-        ctx.save_for_backward(qp, k1, v1, k2p, v2p, o, lse)
-        ctx.b = b
+        # (positions and boundaries may be views of the caller's: a change in place before the backward is an error there)
+        ctx.save_for_backward(qp, k1, v1, k2p, v2p, o, lse, b.cu_q, b.pos_q, b.cu_k1, b.cu_k2, b.pos_k, b.none_cu, b.none_pos)
+        ctx.second, ctx.scale, ctx.schedule, ctx.pairs, ctx.max_k, ctx.pack_q, ctx.packs = (
+            b.second, b.scale, b.schedule, b.pairs, (b.max_k1, b.max_k2), b.pack_q, b.packs)
         out = o if b.pack_q.rows is None else ops.rows_select([o], b.pack_q.rank, b.pack_q.B * b.pack_q.T)[0]
         return out.view(b.pack_q.B, b.pack_q.T, *out.shape[1:])
 
     @staticmethod
     def backward(ctx, g):
-        b = ctx.b
-        qp, k1, v1, k2p, v2p, o, lse = ctx.saved_tensors
-        pack = b.pack_q
+        qp, k1, v1, k2p, v2p, o, lse, cu_q, pos_q, cu_k1, cu_k2, pos_k, none_cu, none_pos = ctx.saved_tensors
+        pack = ctx.pack_q
         g = _readable(g.reshape(pack.B * pack.T, *g.shape[2:]).contiguous())
         if pack.rows is not None:
             g = ops.rows_select([g], pack.rows, pack.n, pack.n_dev)[0]
         none = qp.new_empty((0,) + tuple(qp.shape[1:]))
         no_lse = lse.new_empty((lse.shape[0], 0))
-        if b.second:
-            grads = ops.duo_bwd_varlen(none, k1, v1, none, no_lse, none, b.none_cu, b.cu_k1, qp, k2p, v2p, o, lse, g, b.pos_q, b.pos_k, b.cu_q,
-                                       b.cu_k2, b.scale, b.schedule, max_seqlen_k1=b.max_k1, max_seqlen_k2=b.max_k2, pairs=b.pairs)
+        more = dict(schedule=ctx.schedule, max_seqlen_k1=ctx.max_k[0], max_seqlen_k2=ctx.max_k[1], pairs=ctx.pairs)
+        if ctx.second:
+            grads = ops.duo_bwd_varlen(none, k1, v1, none, no_lse, none, none_cu, cu_k1, qp, k2p, v2p, o, lse, g, pos_q, pos_k, cu_q, cu_k2, ctx.scale, **more)
             rows = [grads[3], grads[4], grads[5]]
         else:
-            grads = ops.duo_bwd_varlen(qp, k1, v1, o, lse, g, b.cu_q, b.cu_k1, none, k2p, v2p, none, no_lse, none, b.none_pos, b.none_pos, b.none_cu,
-                                       b.none_cu, b.scale, b.schedule, max_seqlen_k1=b.max_k1, max_seqlen_k2=b.max_k2, pairs=b.pairs)
+            grads = ops.duo_bwd_varlen(qp, k1, v1, o, lse, g, cu_q, cu_k1, none, k2p, v2p, none, no_lse, none, none_pos, none_pos, none_cu, none_cu, ctx.scale,
+                                       **more)
             rows = [grads[0], None, None]
-        for pack, at in b.packs:
+        for pack, at in ctx.packs:
             for i, t in zip(at, ops.rows_select([rows[i] for i in at], pack.rank, pack.B * pack.T)):
                 rows[i] = t
         return None, rows[0], grads[1], grads[2], rows[1], rows[2]
@@ -524,7 +525,7 @@ def _attend_block(m: "DuoMask", cache: TaHDuoCache, layer: int, pq: _Packed, que
             k1, v1, b.cu_k1, b.max_k1 = k2.detach()[:0], v2.detach()[:0], b.none_cu, 0
     else:
         k2 = v2 = k1.detach()[:0]
-        b.max_k2 = n_k2 = 0
+        b.cu_k2, b.pos_k, b.max_k2 = b.none_cu, b.none_pos, 0
     Hkv = k1.shape[1]
     if b.second:
         b.pairs = 2 if k1_paired else 0

@@ -242,6 +242,36 @@ def test_forward_loop_gradients(emu):
         assert err < 3e-2, (n, float(err))
 
 
+def test_positions_changed_between_forward_and_backward_are_an_error(emu):
+    """32-bit positions of a block without a valid mask are taken where they lie: a caller that writes to them before the backward
+    gets autograd's error, not gradients of other positions; left alone, the same gradients come out as from a copy."""
+    from tah_amd.attention import build_attention_mask, duo_attention_forward
+    from tah_amd.cache import TaHDuoCache
+    g = torch.Generator().manual_seed(9)
+    make = lambda n, h: (torch.randn(1, h, n, 128, generator=g) * 0.5).to(torch.bfloat16)
+    x = [make(12, 2), make(12, 1), make(12, 1), make(4, 2), make(4, 1), make(4, 1)]
+
+    def loop(pos2):
+        t = [a.clone().requires_grad_(True) for a in x]
+        cache, o = TaHDuoCache(), None
+        for depth, pos, (q, k, v) in ((0, torch.arange(12, dtype=torch.int32)[None], t[:3]), (1, pos2, t[3:])):
+            m = build_attention_mask(pos, None, cache, depth)
+            cache.current_iter_depth, cache.position_ids_to_cache, cache.valid_mask_to_cache = depth, pos, None
+            kk, vv = cache.update(k, v, 0)
+            o = duo_attention_forward(_layer(), q, kk, vv, m, scaling=128 ** -0.5)[0]
+        return t, o
+
+    pos2 = torch.tensor([[1, 4, 7, 11]], dtype=torch.int32)
+    (t, o), (t2, o2) = loop(pos2), loop(pos2.long())
+    for a, b in ((t, o), (t2, o2)):
+        b.float().square().sum().backward()
+    assert all(torch.equal(a.grad, b.grad) for a, b in zip(t[1:], t2[1:]))
+    _, o = loop(pos2)
+    pos2 += 1
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        o.float().sum().backward()
+
+
 def test_decode_steps_through_cache_and_callable(emu):
     """Prefill then decode steps at both depths with slabs; compare with the dense reference over the grown cache."""
     from tests.decode_steps_case import run
