@@ -140,26 +140,20 @@ class _RowsMove(torch.autograd.Function):
         return grad_src, None, None, None, None, None, None, None
 
 
-class _RowsSelect(torch.autograd.Function):
-    """out[r] = src[index[r]], zeros where that is negative, for several tensors in one launch.  ``back``: the table of the other
-    direction (every source row goes to one row of the result at most)."""
+class _Selected(torch.autograd.Function):
+    """Rows that ``ops.rows_select`` took out of ``src`` (``box``: a list that holds them).  ``back``: the table of the other direction
+    (every source row went to one row of the result at most).  A node per tensor around the one launch: what happens to the
+    gradient of one of them (when it is asked for, or that it never is) is nothing to the others."""
 
     @staticmethod
-    def forward(ctx, index, rows, back, *srcs):
+    def forward(ctx, src, box, back):
         ctx.save_for_backward(back)
-        ctx.totals = [s.shape[0] for s in srcs]
-        out = ops.rows_select(srcs, index, rows)
-        ctx.mark_non_differentiable(*[o for i, o in enumerate(out) if not ctx.needs_input_grad[3 + i]])
-        return tuple(out)
+        ctx.total = src.shape[0]
+        return box.pop()
 
     @staticmethod
-    def backward(ctx, *grads):
-        (back,) = ctx.saved_tensors
-        at = [i for i in range(len(grads)) if ctx.needs_input_grad[3 + i]]
-        out = [None] * len(grads)
-        for i, g in zip(at, ops.rows_select([grads[i] for i in at], back, ctx.totals[at[0]]) if at else ()):
-            out[i] = g
-        return (None, None, None, *out)
+    def backward(ctx, grad):
+        return ops.rows_select([grad], ctx.saved_tensors[0], ctx.total)[0], None, None
 
 
 def _flat_rows(t: torch.Tensor, lead: int) -> torch.Tensor:
@@ -195,7 +189,9 @@ def gather_active(current_iter_mask: torch.Tensor, *tensors, pad_value=0, max_ac
                 raise TahDuoError(f"gather_active: tensor shape {tuple(t.shape)} does not start with ({B}, {S})")
         W = idx.width
         left, back, pad_mask = ops.left_index_build(idx.cu, idx.flat, idx.rank, S, W)
-        moved = iter(_RowsSelect.apply(left, B * W, back, *[_flat_rows(t, B * S) for t in given]) if given else ())
+        srcs = [_flat_rows(t, B * S) for t in given]
+        rows = ops.rows_select(srcs, left, B * W) if given else []
+        moved = iter([_Selected.apply(t, [r], back) if t.is_floating_point() or t.is_complex() else r for t, r in zip(srcs, rows)])
         return (pad_mask, *[None if t is None else next(moved).view(B, W, *t.shape[2:]) for t in tensors])
     overflow = None
     if max_active is None:

@@ -233,3 +233,28 @@ def test_gathered_tensors_want_gradients_as_before():
         for b in range(3):
             want[b, mask[b]] = w[b, :int(mask[b].sum())]
         assert torch.equal(x.grad, want)
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_gathered_tensors_have_gradients_of_their_own():
+    """Tensors packed together stay apart for autograd: one backward leaves the others' gradients alone and frees nothing of theirs,
+    and forward mode is refused as by any node that has no rule for it."""
+    import torch.autograd.forward_ad as fwd
+
+    from tah_amd.pack import gather_active
+
+    with emu_util.emulated():
+        g = torch.Generator().manual_seed(2)
+        mask = torch.rand(3, 11, generator=g) < 0.4
+        x, y = [torch.randn(3, 11, 4, generator=g, requires_grad=True) for _ in range(2)]
+        want = mask[..., None].expand(3, 11, 4).float()
+        pad, gx, gy, ids = gather_active(mask, x, y, torch.arange(33).view(3, 11))
+        gx.sum().backward()
+        assert torch.equal(x.grad, want) and y.grad is None
+        gy.sum().backward()
+        assert torch.equal(y.grad, want) and torch.equal(x.grad, want)
+        gx = gather_active(mask, x)[1]
+        gx *= 2.0  # (a result of its own, not a view of anything)
+        assert torch.equal(torch.autograd.grad(gx.sum(), x)[0], 2.0 * want)
+        with fwd.dual_level(), pytest.raises(RuntimeError):
+            gather_active(mask, fwd.make_dual(x.detach(), torch.ones_like(x)))
