@@ -41,7 +41,7 @@
 extern "C" {
 #endif
 
-#define TAH_DUO_ABI_VERSION 12
+#define TAH_DUO_ABI_VERSION 13
 
 enum {
     TAH_OK = 0,
@@ -171,6 +171,10 @@ typedef struct tah_duo_bwd_args {
     size_t ds_workspace_bytes;
     int32_t max_seqlen_k1;      /* upper bound on one sequence's depth-0 key rows, 0: unknown (total_k is used) */
     int32_t max_seqlen_k2;      /* same for depth 1 */
+    const int32_t* packed_q1;   /* NULL, or where s1.cu_q holds pairs: int32 [nseq+1], the boundaries the same sequences' query rows
+                                 * would have one behind the other (packed_q1[b] rows before sequence b) ... */
+    int32_t rows_q1;            /* ... and their number, packed_q1[nseq] or more, 1 .. s1.total_q.  The workspace then holds blocks
+                                 * for these rows alone: tah_duo_bwd_workspace_bytes with rows_q1 in place of total_q1 */
 } tah_duo_bwd_args;
 
 /* Backward of tah_duo_fwd_varlen: dQ, dK, dV of both depths.  Replaces torch

@@ -8,7 +8,7 @@ from __future__ import annotations
 
 import ctypes as C
 
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 c_void_p, c_int32, c_int64, c_float = C.c_void_p, C.c_int32, C.c_int64, C.c_float
 
@@ -72,7 +72,8 @@ class DuoBwdArgs(C.Structure):
 
     _fields_ = [("fwd", DuoFwdArgs), ("g1", DuoBwdStream), ("g2", DuoBwdStream),
                 ("ds_workspace", c_void_p), ("ds_workspace_bytes", C.c_size_t),
-                ("max_seqlen_k1", c_int32), ("max_seqlen_k2", c_int32)]
+                ("max_seqlen_k1", c_int32), ("max_seqlen_k2", c_int32),
+                ("packed_q1", c_void_p), ("rows_q1", c_int32)]
 
 
 class AdditiveMask(C.Structure):

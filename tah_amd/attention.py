@@ -225,8 +225,9 @@ class _Packed:
     they lie, ``cu`` then holds (first row, one past the last) pairs, ``paired``.  Its pad rows come out as zeros, as from a scatter, and
     what they hold is not read.  Two layers of four sequences of 1024 to 3210 rows, forward and backward: 2.62 -> 2.05 ms with
     :class:`_BlockAttn` (row moves, clears and the gradients of empty slices were 0.5 of it, and the host's 105 launches behind the hard
-    tokens' read-back the rest).  Blocks that are mostly padding are packed: the dS
-    workspace of the backward grows with the rows a block has, and its pad rows are cleared in every result.
+    tokens' read-back the rest).  The backward's dS workspace counts the valid rows alone, as for packed ones.  Two layers' depth-0 calls, forward and
+    backward, in place and packed: 2.03 and 2.33 ms (8 x 4096, 57 % valid), 6.90 and 7.47 (8 x 8192, 57 %), 4.22 and 4.52 (38 %), 0.83 and
+    0.90 (4 x 3210, 32 %), 2.89 and 2.96 (8 x 8192, 21 %): below a half little is left of it, and such blocks are packed.
 
     With ``tah_amd.pack.HOST_SYNC`` off nothing is read back from the device: packed tensors keep the full
     B*T rows, the kernels find the real extent in ``cu`` (and read no row behind it: those are undefined), and the row copies
@@ -252,6 +253,7 @@ class _Packed:
             self.cu = torch.arange(0, (B + 1) * T, T, dtype=torch.int32, device=device)
         elif pos is None and idx.intervals is not None and 2 * idx.n >= B * T:
             self.rows, self.n, self.cu, self.paired = None, B * T, idx.intervals, True
+            self.packed_cu, self.packed_n = idx.cu, idx.n
         else:
             self.rows, self.n, self.cu, self.n_dev, self.rank = idx.flat, idx.bound, idx.cu, idx.n_dev, idx.rank
         self.pos = None
@@ -330,6 +332,8 @@ class _BlockAttn(torch.autograd.Function):
             grads = ops.duo_bwd_varlen(none, k1, v1, none, no_lse, none, none_cu, cu_k1, qp, k2p, v2p, o, lse, g, pos_q, pos_k, cu_q, cu_k2, ctx.scale, **more)
             rows = [grads[3], grads[4], grads[5]]
         else:
+            if pack.paired:
+                more.update(packed_q1=pack.packed_cu, rows_q1=pack.packed_n)
             grads = ops.duo_bwd_varlen(qp, k1, v1, o, lse, g, cu_q, cu_k1, none, k2p, v2p, none, no_lse, none, none_pos, none_pos, none_cu, none_cu, ctx.scale,
                                        **more)
             rows = [grads[0], None, None]

@@ -57,6 +57,7 @@ struct BwdParams {
     // dS exchange between the key-tile kernel and the dQ kernel that reads it back (see ds_block)
     unsigned char* ds_ws;
     int32_t ds_q1slots, ds_kt1, ds_kt;
+    const int32_t* ds_packed_q1;  // boundaries of the depth-0 query rows without those in between, or nullptr: the call's own
 };
 
 // ---------------------------------------------------------------------------
@@ -65,7 +66,8 @@ struct BwdParams {
 // recomputes S and dP: 5 products per (query tile, key tile) pair instead of 7.
 // The workspace is a table of 16 KiB blocks, one per (64 query rows, query head, 128 keys):
 //   block = ((qslot * hq + head) * ds_kt + ktile)
-//   qslot = first row / 64 + seq + tile                   depth-0 query rows  (ds_q1slots slots)
+//   qslot = first row / 64 + seq + tile                   depth-0 query rows  (ds_q1slots slots; first row: among the sequences' rows alone
+//                                                         where the call says where that is, so that padding has no blocks)
 //           ds_q1slots + first row / 64 + seq + tile      depth-1 query rows
 //   ktile = key tile inside its sequence (depth 0), ds_kt1 + key tile (depth 1)
 // (cu / 64 + seq numbers the 64-row tiles of successive sequences without collisions and needs no prefix
@@ -487,7 +489,7 @@ __global__ __launch_bounds__(kKvThreads) TAH_WAVES_PER_EU(2, 2) void duo_bwd_dkd
     [[maybe_unused]] int64_t ds_base1 = 0, ds_base2 = 0;
     if constexpr (kExport) {
         const int ktile = (second ? p.ds_kt1 : 0) + kl0 / kBK;
-        const int slot1 = q1_lo / kBQ + seq + t1_begin;
+        const int slot1 = (p.ds_packed_q1 ? const_i32(p.ds_packed_q1, seq) : q1_lo) / kBQ + seq + t1_begin;
         const int slot2 = p.ds_q1slots + q2_lo / kBQ + seq + t2_begin;
         ds_base1 = (((int64_t)slot1 * p.hq + hk * G) * p.ds_kt + ktile) * kDsBlockBytes + wave * kDsWaveBytes;
         ds_base2 = (((int64_t)slot2 * p.hq + hk * G) * p.ds_kt + ktile) * kDsBlockBytes + wave * kDsWaveBytes;
@@ -896,7 +898,8 @@ __global__ __launch_bounds__(lq_threads(kUnits)) TAH_WAVES_PER_EU(2, 2) void duo
 
     // where my unit's blocks start: (qslot, head), key tile 0.  A unit without a tile copies the first unit's
     // blocks (memory that exists; never used).
-    const int qslot = (second ? p.ds_q1slots : 0) + q_lo / kBN + seq + tile0 + (unit_ok ? utile : 0);
+    const int first_row = !second && p.ds_packed_q1 ? const_i32(p.ds_packed_q1, seq) : q_lo;
+    const int qslot = (second ? p.ds_q1slots : 0) + first_row / kBN + seq + tile0 + (unit_ok ? utile : 0);
     const unsigned char* ds_unit = p.ds_ws + (int64_t)(qslot * p.hq + uhead) * p.ds_kt * kDsBlockBytes;
 
     // asynchronous copies of one step: K rows as in the dQ kernel (4 rows per copy, two copies per wave), then four
@@ -1149,13 +1152,17 @@ int dispatch_bwd(const tah_duo_bwd_args* a, const tah_additive_mask* m, tah_stre
     p.sched = kDense ? nullptr : static_cast<const int32_t*>(f.schedule);
     p.ds_ws = nullptr;
     p.ds_q1slots = p.ds_kt1 = p.ds_kt = 0;
+    p.ds_packed_q1 = nullptr;
     if (!kDense && a->ds_workspace && g <= 4) {
         if (reinterpret_cast<uintptr_t>(a->ds_workspace) & 15) return TAH_E_ALIGN;
-        const size_t need = tah_duo_bwd_workspace_bytes(f.nseq, f.hq, f.hkv, f.s1.total_q, f.s1.total_k, f.s2.total_q, f.s2.total_k,
+        if ((f.cu_pairs & 1) && a->packed_q1) p.ds_packed_q1 = a->packed_q1;
+        if (p.ds_packed_q1 && (a->rows_q1 < 0 || a->rows_q1 > f.s1.total_q || (a->rows_q1 == 0) != (f.s1.total_q == 0))) return TAH_E_SHAPE;
+        const int32_t rows_q1 = p.ds_packed_q1 ? a->rows_q1 : f.s1.total_q;
+        const size_t need = tah_duo_bwd_workspace_bytes(f.nseq, f.hq, f.hkv, rows_q1, f.s1.total_k, f.s2.total_q, f.s2.total_k,
                                                         a->max_seqlen_k1, a->max_seqlen_k2);
         if (a->ds_workspace_bytes < need) return TAH_E_WORKSPACE;
         p.ds_ws = static_cast<unsigned char*>(a->ds_workspace);
-        p.ds_q1slots = ds_query_slots(f.s1.total_q, f.nseq);
+        p.ds_q1slots = ds_query_slots(rows_q1, f.nseq);
         p.ds_kt1 = ds_key_slots(f.s1.total_k, a->max_seqlen_k1);
         p.ds_kt = p.ds_kt1 + ds_key_slots(f.s2.total_k, a->max_seqlen_k2);
     }

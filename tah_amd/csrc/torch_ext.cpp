@@ -225,7 +225,7 @@ std::vector<Tensor> duo_bwd_varlen(const Tensor& q1, const Tensor& k1, const Ten
                                    const Tensor& v2, const Tensor& o2, const Tensor& lse2, const Tensor& do2, const Tensor& pos_q2,
                                    const Tensor& pos_k2, const Tensor& cu_q2, const Tensor& cu_k2, double scale,
                                    const optional<Tensor>& schedule, const optional<Tensor>& ds_workspace,
-                                   int64_t max_seqlen_k1, int64_t max_seqlen_k2, int64_t pairs) {
+                                   int64_t max_seqlen_k1, int64_t max_seqlen_k2, int64_t pairs, const optional<Tensor>& packed_q1, int64_t rows_q1) {
     need_lib();
     for (auto p : {std::make_pair(&q1, "q1"), {&k1, "k1"}, {&v1, "v1"}, {&o1, "o1"}, {&do1, "do1"}, {&q2, "q2"}, {&k2, "k2"},
                    {&v2, "v2"}, {&o2, "o2"}, {&do2, "do2"}})
@@ -259,6 +259,14 @@ std::vector<Tensor> duo_bwd_varlen(const Tensor& q1, const Tensor& k1, const Ten
         a.ds_workspace_bytes = (size_t)ds_workspace->numel() * ds_workspace->element_size();
         a.max_seqlen_k1 = (int32_t)max_seqlen_k1;
         a.max_seqlen_k2 = (int32_t)max_seqlen_k2;
+    }
+    if (packed_q1.has_value()) {
+        i32(*packed_q1, "packed_q1");
+        d.see(*packed_q1);
+        TORCH_CHECK((pairs & 1) && packed_q1->numel() == (int64_t)a.fwd.nseq + 1 && rows_q1 > 0 && rows_q1 <= q1.size(0),
+                    "packed_q1: nseq+1 boundaries of rows_q1 query rows, beside pairs");
+        a.packed_q1 = static_cast<const int32_t*>(packed_q1->data_ptr());
+        a.rows_q1 = (int32_t)rows_q1;
     }
     check_rc(g.bwd_varlen(&a, d.stream()), "tah_duo_bwd_varlen");
     Gaps gaps;

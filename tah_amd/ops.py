@@ -82,23 +82,26 @@ def _ds_workspace(device, nbytes: int):
 
 
 def duo_bwd_varlen(q1, k1, v1, o1, lse1, do1, cu_q1, cu_k1, q2, k2, v2, o2, lse2, do2, pos_q2, pos_k2, cu_q2, cu_k2,
-                   scale: float, schedule=None, ds_workspace=None, max_seqlen_k1: int = 0, max_seqlen_k2: int = 0, pairs: int = 0):
+                   scale: float, schedule=None, ds_workspace=None, max_seqlen_k1: int = 0, max_seqlen_k2: int = 0, pairs: int = 0,
+                   packed_q1: Optional[torch.Tensor] = None, rows_q1: int = 0):
     """Backward of :func:`duo_fwd_varlen`; returns dq1, dk1, dv1, dq2, dk2, dv2 (bf16).
 
     ``ds_workspace``: a uint8 tensor of at least :func:`duo_bwd_workspace_bytes` bytes, ``False`` for the three-kernel
     backward, or None: the package's own buffer when ``DS_EXCHANGE`` is on and the call fits ``DS_EXCHANGE_MAX_BYTES``.
     ``max_seqlen_k1`` / ``max_seqlen_k2``: upper bounds on one sequence's key rows per depth (0: unknown); they only
     make the workspace smaller.  ``pairs``: as in :func:`duo_fwd_varlen` (gradients of rows in between are zeros).
+    ``packed_q1`` (int32 [nseq+1]) and ``rows_q1``: the boundaries that the depth-0 query rows given as pairs would have one behind
+    the other, and their number; the workspace then counts these rows and not those in between.
     """
     if ds_workspace is None and DS_EXCHANGE:
-        need = duo_bwd_workspace_bytes(cu_q1.numel() // 2 if pairs & 1 else cu_q1.numel() - 1, q1.shape[1], k1.shape[1], q1.shape[0], k1.shape[0], q2.shape[0],
-                                       k2.shape[0], max_seqlen_k1, max_seqlen_k2)
+        need = duo_bwd_workspace_bytes(cu_q1.numel() // 2 if pairs & 1 else cu_q1.numel() - 1, q1.shape[1], k1.shape[1],
+                                       q1.shape[0] if packed_q1 is None else rows_q1, k1.shape[0], q2.shape[0], k2.shape[0], max_seqlen_k1, max_seqlen_k2)
         if 0 < need <= DS_EXCHANGE_MAX_BYTES:
             ds_workspace = _ds_workspace(q1.device, need)
     if ds_workspace is False:
         ds_workspace = None
     return tuple(_call("duo_bwd_varlen", q1, k1, v1, o1, lse1, do1, cu_q1, cu_k1, q2, k2, v2, o2, lse2, do2, pos_q2, pos_k2,
-                       cu_q2, cu_k2, float(scale), schedule, ds_workspace, int(max_seqlen_k1), int(max_seqlen_k2), int(pairs)))
+                       cu_q2, cu_k2, float(scale), schedule, ds_workspace, int(max_seqlen_k1), int(max_seqlen_k2), int(pairs), packed_q1, int(rows_q1)))
 
 
 def duo_fwd_masked(q, k, v, mask, nseq: int, scale: float):

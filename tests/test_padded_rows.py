@@ -258,3 +258,58 @@ def test_gathered_tensors_have_gradients_of_their_own():
         assert torch.equal(torch.autograd.grad(gx.sum(), x)[0], 2.0 * want)
         with fwd.dual_level(), pytest.raises(RuntimeError):
             gather_active(mask, fwd.make_dual(x.detach(), torch.ones_like(x)))
+
+
+def check_workspace_of_padded_blocks(dev, monkeypatch, lens, left, hq, hkv):
+    """dS of a padded block in place: blocks for the rows that exist and no others, none written behind them, and the gradients of the
+    same block packed, to the bit."""
+    import types
+
+    from tah_amd import attention as A, ops
+    from tah_amd.cache import TaHDuoCache
+
+    g = torch.Generator().manual_seed(sum(lens))
+    B, T = len(lens), max(lens)
+    at, n = torch.arange(T)[None], torch.tensor(lens)[:, None]
+    valid = ((at >= T - n) if left else (at < n)).to(dev)
+    x = [(torch.randn(B, T, h, D, generator=g) * 0.5).to(torch.bfloat16).to(dev) for h in (hq, hkv, hkv, hq)]
+    asked = []
+
+    def buffer(device, nbytes):
+        whole = torch.full((nbytes + 65536,), 171, dtype=torch.uint8, device=device)
+        asked.append((nbytes, whole))
+        return whole[:nbytes]
+
+    monkeypatch.setattr(ops, "_ds_workspace", buffer)
+    monkeypatch.setattr(A, "NO_SYNC_ROWS", 0)
+    results = []
+    for paired in (True, False):
+        v = valid.clone()
+        pos = (v.long().cumsum(-1) - 1).clamp(min=0)
+        if not paired:
+            A.HardIndex.of(v).intervals = None
+        t = [a.clone().requires_grad_(True) for a in x[:3]]
+        cache = TaHDuoCache()
+        mask = A.build_attention_mask(pos, v, cache, 0)
+        cache.current_iter_depth, cache.position_ids_to_cache, cache.valid_mask_to_cache = 0, pos, v
+        kk, vv = cache.update(t[1].transpose(1, 2), t[2].transpose(1, 2), 0)
+        o = A.duo_attention_forward(types.SimpleNamespace(layer_idx=0), t[0].transpose(1, 2), kk, vv, mask, scaling=SCALE)[0]
+        assert mask._packed.paired == paired
+        results.append([o.detach()] + list(torch.autograd.grad(o, t, x[3])))
+    assert len(asked) == 2 and asked[0][0] == asked[1][0] > 0
+    assert all((whole[nbytes:] == 171).all() for nbytes, whole in asked)
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+@pytest.mark.parametrize("lens,left,hq,hkv", [([130, 70, 66], False, 2, 1), ([65, 33], True, 1, 1)])
+def test_workspace_of_padded_blocks_emu(monkeypatch, lens, left, hq, hkv):
+    with emu_util.emulated():
+        check_workspace_of_padded_blocks("cpu", monkeypatch, lens, left, hq, hkv)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,left,hq,hkv", [([1000, 520, 513, 600], False, 16, 8), ([400] + [210] * 69, True, 4, 1)])
+def test_workspace_of_padded_blocks_gpu(monkeypatch, lens, left, hq, hkv):
+    check_workspace_of_padded_blocks("cuda", monkeypatch, lens, left, hq, hkv)
