@@ -528,7 +528,8 @@ typedef struct tah_linear_rows_args {
 int tah_linear_rows(const tah_linear_rows_args* args, tah_stream_t stream);
 /* Two plain layers over the same rows (x_packed, rows, k) with the same RMSNorm in one launch, the bits of the two calls: an
  * output head, and a layer beside it with an optional bias and ReLU (a decider's first one).  Sizes: those
- * tah_linear_beside_supported says 1 for; anything else, other epilogues among it, is TAH_E_SHAPE. */
+ * tah_linear_beside_supported says 1 for; anything else, other epilogues, results that lie on each other or on what is read,
+ * and rows that are not the same among it, is TAH_E_SHAPE. */
 int tah_linear_beside_supported(int32_t rows, int32_t n, int32_t k, int32_t beside);
 int tah_linear_beside(const tah_linear_rows_args* head, const tah_linear_rows_args* beside, tah_stream_t stream);
 

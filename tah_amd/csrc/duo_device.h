@@ -54,6 +54,25 @@ __device__ __forceinline__ void device_or(uint32_t* p, uint32_t v) { __hip_atomi
 __device__ __forceinline__ void device_max(unsigned long long* p, unsigned long long v) { __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 #endif
 
+// Memory that a call's rows take up, on the host: `rows` rows of `bytes`, `stride` bytes apart (nothing where `at` is null).
+struct RowSpan {
+    const void* at;
+    int64_t bytes, stride;
+    int32_t rows;
+};
+inline RowSpan one_span(const void* at, int64_t bytes) { return RowSpan{at, bytes, bytes, 1}; }
+// Whether two of them share a byte (columns of one array side by side do not; otherwise a gap between rows counts as taken).
+inline bool spans_meet(const RowSpan& x, const RowSpan& y) {
+    if (!x.at || !y.at || x.bytes <= 0 || y.bytes <= 0 || x.rows <= 0 || y.rows <= 0) return false;
+    const int64_t from = reinterpret_cast<intptr_t>(x.at), other = reinterpret_cast<intptr_t>(y.at);
+    if (other >= from + (x.rows - 1) * x.stride + x.bytes || from >= other + (y.rows - 1) * y.stride + y.bytes) return false;
+    if (x.rows > 1 && y.rows > 1 && x.stride == y.stride && x.stride >= x.bytes && x.stride >= y.bytes) {
+        const int64_t d = ((other - from) % x.stride + x.stride) % x.stride;
+        return d < x.bytes || x.stride - d < y.bytes;
+    }
+    return true;
+}
+
 #ifndef TAH_WAIT_VMEM
 // s_waitcnt vmcnt(0) (expcnt/lgkmcnt untouched) as a builtin, so the compiler's own wait-count
 // bookkeeping also learns that no ordinary load is pending past this point.

@@ -1505,7 +1505,17 @@ extern "C" int tah_linear_beside(const tah_linear_rows_args* a, const tah_linear
         b->norm_eps != a->norm_eps || b->out_row_stride < b->n)
         return TAH_E_SHAPE;
     if (a->rows == 0) return TAH_OK;
-    if (!a->out || !b->w_packed || !b->out || b->x_packed != a->x_packed) return TAH_E_NULL;
+    if (!a->out || !a->x_packed || !a->w_packed || !b->w_packed || !b->out) return TAH_E_NULL;
+    if (b->x_packed != a->x_packed) return TAH_E_SHAPE;
+    // (in two calls a result that lies on another, or on what the second one reads, has an order)
+    const auto result = [&](const tah_linear_rows_args* l) { return RowSpan{l->out, 2ll * l->n, 2 * l->out_row_stride, l->rows}; };
+    const RowSpan written[] = {result(a), result(b)};
+    const RowSpan read[] = {one_span(a->x_packed, 64ll * a->k), one_span(a->w_packed, 2ll * a->n * a->k), one_span(b->w_packed, 2ll * b->n * b->k),
+                            one_span(b->bias, 2ll * b->n)};
+    if (spans_meet(written[0], written[1])) return TAH_E_SHAPE;
+    for (const RowSpan& w : written)
+        for (const RowSpan& r : read)
+            if (spans_meet(w, r)) return TAH_E_SHAPE;
     if (!aligned16(b->w_packed) || !aligned16(b->out) || !aligned16(b->bias) || b->out_row_stride % 8 != 0) return TAH_E_ALIGN;
     return run_linear_rows(a, b, stream);
 }

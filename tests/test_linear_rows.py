@@ -580,6 +580,33 @@ def test_linear_beside_on_cpu_shim():
                 ops.linear_beside(z, z[:n2 * k], torch.zeros(32 * k, dtype=BF), rows, n, n2, k, norm_eps=1e-6)
 
 
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_linear_beside_refuses_results_on_each_other_and_on_what_it_reads():
+    """Two calls have an order that one launch has not; columns of one array side by side share nothing and are taken (with a bias off
+    its alignment: refused by the check behind, before a launch)."""
+    import ctypes as C
+
+    from tah_amd import _capi
+    rows, n, n2, k = 3, 16384, 32, 32
+    w, w2, x = torch.zeros(n * k, dtype=BF), torch.zeros(n2 * k, dtype=BF), torch.zeros(64 * k, dtype=BF)
+    buf, b2 = torch.zeros(rows, n + n2 + 32, dtype=BF), torch.zeros(n2 + 8, dtype=BF)[1:]
+    with emu_util.emulated() as lib:
+        def call(out, out2, x2=x, bias=b2, stride=buf.stride(0), stride2=buf.stride(0)):
+            a, b = [_capi.LinearRowsArgs(w_packed=ww.data_ptr(), x_packed=xx.data_ptr(), out=o.data_ptr(), out_row_stride=s, rows=rows, n=nn, k=k, input_norm=1,
+                                         norm_eps=1e-6) for ww, xx, o, s, nn in ((w, x, out, stride, n), (w2, x2, out2, stride2, n2))]
+            b.bias = bias.data_ptr()
+            return lib.tah_linear_beside(C.byref(a), C.byref(b), None)
+
+        other = torch.zeros(rows, n2, dtype=BF)
+        shape, taken = _capi.TAH_E_SHAPE, _capi.TAH_E_ALIGN
+        assert call(buf, buf[:, n:]) == taken and call(buf[:, n2:], buf) == taken and call(buf, other, stride2=n2) == taken
+        assert call(buf, buf[:, n - 16:]) == shape and call(buf[:, 16:], buf) == shape  # half of the narrow result's columns
+        assert call(buf, buf[1:, :n2]) == shape                                     # rows of the same array, one further down
+        assert call(buf, x, stride2=n2) == shape and call(buf, w2, stride2=n2) == shape and call(buf, w, stride2=n2) == shape
+        assert call(buf, other, stride2=n2, bias=other) == shape and call(buf, other, stride2=n2, bias=buf) == shape
+        assert call(buf, other, x2=torch.zeros(64 * k, dtype=BF), stride2=n2) == shape
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows", [1, 8, 9, 16])
 @pytest.mark.parametrize("n,n2,k,bias,relu", [(151936, 512, 2048, True, True), (16384, 32, 2048, False, False), (32000, 96, 1024, True, False)])
