@@ -654,7 +654,8 @@ typedef struct tah_decider_tail_args {
 } tah_decider_tail_args;
 int tah_decider_tail(const tah_decider_tail_args* args, tah_stream_t stream);
 /* tah_decider_tail and, of the rows it calls hard, tah_topk_mix in one launch: the bits of the two calls.  mix->row_enable is
- * decider->hard, mix->out is not NULL and both have the same rows. */
+ * decider->hard, mix->out is not NULL and both have the same rows; the results lie neither on each other nor on what is read, but
+ * for the 32-bit words of the decision, which may be the positions or each other (TAH_E_SHAPE otherwise). */
 int tah_decide_mix(const tah_decider_tail_args* decider, const tah_topk_mix_args* mix, tah_stream_t stream);
 
 /* End of a tick of a generation loop in which every row advances by one latent iteration of its own token, so that a

@@ -557,6 +557,26 @@ extern "C" int tah_decide_mix(const tah_decider_tail_args* decider, const tah_to
     if (decider->rows != a->rows) return TAH_E_SHAPE;
     if (a->rows == 0) return TAH_OK;
     if (!a->out) return TAH_E_SHAPE;
-    if (a->row_enable != decider->hard) return TAH_E_NULL;
+    if (!a->row_enable) return TAH_E_NULL;
+    if (a->row_enable != decider->hard) return TAH_E_SHAPE;
+    // Two calls have an order: here the first of a row's workgroups stores the decision while the others still read what it came from.  (The
+    // 32-bit words of the decision are stored by the thread that reads the row's position: they may be the positions or each other.)
+    using namespace tah;
+    const int32_t rows = a->rows, k = a->topk < a->vocab ? a->topk : a->vocab;
+    const auto matrix = [&](const void* at, int64_t cols, int64_t stride) { return RowSpan{at, 2 * cols, 2 * stride, rows}; };
+    const RowSpan hidden = matrix(decider->hidden, decider->width, decider->hidden_row_stride), logits = matrix(a->logits, a->vocab, a->logits_row_stride);
+    const RowSpan read[] = {hidden, logits, one_span(decider->w2, 2ll * decider->width), one_span(decider->b2, 2), one_span(decider->active, rows),
+                            RowSpan{a->embedding, 2ll * a->hidden, 2 * a->embedding_row_stride, a->vocab}, one_span(decider->pos, 4ll * rows)};
+    constexpr int kWords = 3;  // of the results: those of 32 bits per row
+    const RowSpan written[] = {one_span(decider->hard_i32, 4ll * rows), one_span(decider->slot, 4ll * rows), one_span(decider->q_pos, 4ll * rows),
+                               one_span(decider->hard, rows), matrix(a->out, a->hidden, a->out_row_stride), one_span(a->out_packed, 64ll * a->hidden),
+                               matrix(a->values_out, k, a->values_row_stride), RowSpan{a->indices_out, 4ll * k, 4 * a->values_row_stride, rows}};
+    constexpr int kWritten = sizeof(written) / sizeof(written[0]);
+    for (int i = 0; i < kWritten; ++i) {
+        for (const RowSpan& r : read)
+            if (!(i < kWords && written[i].at == decider->pos) && spans_meet(written[i], r)) return TAH_E_SHAPE;
+        for (int j = 0; j < i; ++j)
+            if (!(i < kWords && written[i].at == written[j].at) && spans_meet(written[i], written[j])) return TAH_E_SHAPE;
+    }
     return tah::run_topk_mix(a, decider, stream);
 }

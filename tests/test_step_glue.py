@@ -200,6 +200,8 @@ def _decide_mix_refusals(dev, lib):
     m = _capi.TopkMixArgs(logits=t.data_ptr(), embedding=t.data_ptr(), out=t.data_ptr(), row_enable=other.data_ptr(), logits_row_stride=32,
                           embedding_row_stride=32, out_row_stride=32, rows=4, vocab=32, hidden=32, topk=5)
     call = lambda: lib.tah_decide_mix(C.byref(d), C.byref(m), None)
+    assert call() == -2  # TAH_E_SHAPE
+    m.row_enable = None
     assert call() == -1  # TAH_E_NULL
     m.row_enable, m.rows = hard.data_ptr(), 3
     assert call() == -2  # TAH_E_SHAPE
@@ -207,6 +209,27 @@ def _decide_mix_refusals(dev, lib):
     assert call() == -2
     m.rows = d.rows = 0
     assert call() == 0  # nothing to do, as for the two calls
+    # results on what is read, or on each other (the decision's 32-bit words aside): an order that one launch has not
+    B, W, V, H = 4, 64, 90, 32
+    new = lambda *shape, dtype=BF: torch.zeros(*shape, dtype=dtype, device=dev)
+    h, w2, b2, logits, embed = new(B, W), new(W), new(8), new(B, V + H), new(V, H)
+    out, xp, words, act = new(B, 2 * H), new(32 * H), new(4, B, dtype=torch.int32), new(2 * B, dtype=torch.uint8)
+
+    def over(**at):
+        p = dict(hidden=h, w2=w2, b2=b2, active=act, pos=words[0], hard=hard, hard_i32=words[1], slot=words[2], q_pos=words[3], logits=logits, embedding=embed, out=out,
+                 out_packed=xp)
+        p.update(at)
+        p = {k: t.data_ptr() for k, t in p.items()}
+        d = _capi.DeciderTailArgs(hidden_row_stride=W, rows=B, width=W, **{k: p[k] for k in ("hidden", "w2", "b2", "active", "pos", "hard", "hard_i32", "slot",
+                                                                                             "q_pos")})
+        m = _capi.TopkMixArgs(row_enable=p["hard"], logits_row_stride=V + H, embedding_row_stride=H, out_row_stride=2 * H, rows=B, vocab=V, hidden=H, topk=5,
+                              **{k: p[k] for k in ("logits", "embedding", "out", "out_packed")})
+        return lib.tah_decide_mix(C.byref(d), C.byref(m), None)
+
+    assert over() == 0 and over(q_pos=words[0]) == 0 and over(slot=words[1]) == 0 and over(active=act[B:]) == 0
+    for bad in (dict(hard=act), dict(hard=act[1:]), dict(hard=h), dict(out=h), dict(out_packed=h), dict(out=logits), dict(out_packed=embed), dict(hard_i32=w2),
+                dict(q_pos=words.view(-1)[1:]), dict(slot=words.view(-1)[5:]), dict(out_packed=out), dict(hard=b2), dict(hard=words[2].view(torch.uint8))):
+        assert over(**bad) == -2, list(bad)
 
 
 @pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
