@@ -535,7 +535,16 @@ int run_topk_mix(const tah_topk_mix_args* a, const tah_decider_tail_args* decide
     const size_t smem = mix ? (size_t)parts * a->hidden * sizeof(float) : 0;
     if (smem > 48 * 1024) return TAH_E_SHAPE;  // (32 KiB whenever hidden < 8192)
     const int nvec = (a->vocab + 8 * kMixThreads - 1) / (8 * kMixThreads);
-    const dim3 grid(a->rows, mix && a->rows <= kMixSplitRows && cgs < kMixThreads && cgs % kMixSplit == 0 ? kMixSplit : 1), block(kMixThreads);
+    // (results on the row that they come from: one workgroup has read all of it before it stores, several have not)
+    const RowSpan logits{a->logits, 2ll * a->vocab, 2 * a->logits_row_stride, a->rows}, enable = one_span(a->row_enable, a->rows);
+    const int32_t values = a->topk < a->vocab ? a->topk : a->vocab;
+    bool alone = false;
+    for (const RowSpan& w : {RowSpan{a->out, 2ll * a->hidden, 2 * a->out_row_stride, a->rows}, one_span(a->out_packed, 64ll * a->hidden),
+                             RowSpan{a->values_out, 2ll * values, 2 * a->values_row_stride, a->rows},
+                             RowSpan{a->indices_out, 4ll * values, 4 * a->values_row_stride, a->rows}})
+        alone = alone || spans_meet(w, logits) || spans_meet(w, enable);
+    const bool split = mix && !alone && a->rows <= kMixSplitRows && cgs < kMixThreads && cgs % kMixSplit == 0;
+    const dim3 grid(a->rows, split ? kMixSplit : 1), block(kMixThreads);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (nvec <= 2) hipLaunchKernelGGL(topk_mix_kernel<2>, grid, block, smem, st, p);
     else if (nvec <= 8) hipLaunchKernelGGL(topk_mix_kernel<8>, grid, block, smem, st, p);

@@ -49,6 +49,21 @@ def test_columns_of_a_row_shared_by_workgroups_have_the_bits_of_one(V, H, k):
 
 
 @pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_results_on_the_row_s_own_logits():
+    """A result that takes the place of the logits it comes from is what it is beside them, also where workgroups share the columns."""
+    from tah_amd import ops
+    logits, emb = [to_torch(t, "cpu") for t in make_case(11, 2, 300, 96)]
+    with emu_util.emulated():
+        values = torch.empty(2, 17, dtype=torch.bfloat16)
+        want = ops.topk_mix(logits, emb, 17, values_out=values)
+        wide = torch.zeros(2, 304, dtype=torch.bfloat16)  # (rows 16 bytes apart)
+        wide[:, :300] = logits
+        assert torch.equal(ops.topk_mix(wide[:, :300], emb, 17, out=wide[:, :96]), want)
+        wide[:, :300] = logits
+        assert torch.equal(ops.topk_mix(wide[:, :300], emb, 17, values_out=wide[:, :17]), want) and torch.equal(wide[:, :17], values)
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
 def test_topk_mix_golden_and_row_enable_on_cpu_shim():
     from tah_amd import ops
     z = np.load(GOLDEN)
