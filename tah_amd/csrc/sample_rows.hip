@@ -34,6 +34,10 @@ constexpr int kBinsPerThread = kWinKeys / kSmpThreads;  // 32: a thread's group 
 constexpr int kHistWords = kWinKeys + kWinKeys / 32;    // bin b lives at word b + b / 32 (a thread's 32 bins: stride 33)
 constexpr size_t kSmpSmem = (size_t)kHistWords * sizeof(uint32_t);
 constexpr int kFewThreads = kSmpThreads / 4;  // threads with a token among the heavy ones, at most, for only those to be counted
+// How far two float32 sums of the same masses can lie apart, as a share of them: one is rounded at most 33 times inside a thread (32 keys, each
+// a product), 6 over a wave's lanes, 16 over the waves and once over the windows, each time by 2^-24 at most; two of them, the bound
+// added to one and the products with top_p: fewer than 128 roundings.
+constexpr float kSumSlack = 0x1p-17f;
 constexpr uint32_t kNoCut = 0x20000u;  // a distance past every key
 
 struct SampleParams {
@@ -460,11 +464,11 @@ __global__ __launch_bounds__(kSmpThreads) void sample_rows_kernel(const SamplePa
     if constexpr (!kProbs) {
         if (sparse) {
             count();
-            // the largest target S may have (the margin of 2^-20 is for the sums' rounding); the cut stands if every target the light
-            // tokens leave possible keeps the last kept token and leaves out the next
-            const float target = p.top_p * (S + light_mass) * (1.f + 0x1p-20f);
+            // the largest target that a count of everything may have; the cut stands if every target the light tokens leave possible keeps
+            // the last kept token and leaves out the next
+            const float target = p.top_p * (S + light_mass) * (1.f + kSumSlack);
             const float before_last = cut(target);
-            sparse = target < S && before_last <= p.top_p * S * (1.f - 0x1p-20f);
+            sparse = target < S && before_last <= p.top_p * S * (1.f - kSumSlack);
             if (!sparse) {  // (uniform) count everything after all
                 __syncthreads();  // the histogram and s_code have been read
                 if (tid == 0) s_code[0] = 0;

@@ -165,6 +165,51 @@ GPU_CASES = [
 ]
 
 
+def rounded_up_row():
+    """A row whose count of all tokens rounds up at every step: two tokens, and light ones in eighteen places of the key space (two of the
+    first wave's lanes, the other waves, the far window), each with a little more than half a unit of the total's last place.  Whole
+    threads (40 tokens, eight of every 8192) hold light tokens of one kind, so that the bound of their sum is tight."""
+    V, top, T = 40960, 20.0, 20.0 / 24.0
+    x = np.full(V, -np.inf)
+    x[0], x[1] = top, 10.0
+    thread = 1
+    for d in [776, 1544] + [2048 * w + 700 for w in range(1, 16)] + [32778]:  # distance from the largest key
+        key = (0x8000 | 0x41A0) - d
+        bits = np.uint32(key & 0x7FFF if key >= 0x8000 else ~key & 0xFFFF)
+        value = float((bits << np.uint32(16)).view(np.float32))
+        for _ in range(int(np.ceil(0.52 * 2.0 ** -23 / np.exp((value - top) / T) / 40))):
+            x[[8192 * j + 8 * thread + i for j in range(5) for i in range(8)]] = value
+            thread += 1
+    return torch.from_numpy(x.astype(np.float32)).to(torch.bfloat16)[None], T
+
+
+def sum_edge_case(dev, near):
+    """Targets around the edge where the second token is kept: the draw's cut is that of the count of all tokens, which the
+    distribution comes from, to the last bit of top_p."""
+    from tah_amd import ops
+    x, T = rounded_up_row()
+    x = x.to(dev)
+    u = torch.full((1,), 1.0 - 2.0 ** -24, device=dev)
+    edge = np.float32(ops.sample_probs(x, T)[0, 0].item())  # (one over the total)
+    kept = []
+    for k in near:
+        p = float(edge + np.float32(k * 2.0 ** -24))
+        kept.append(int((ops.sample_probs(x, T, top_p=p)[0] > 0).sum()))
+        assert ops.sample_rows(x, u, T, top_p=p).item() == kept[-1] - 1, (k, kept)
+    assert set(kept) == {1, 2}
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_cut_at_the_edge_of_the_sums_on_cpu_shim():
+    with emu_util.emulated():
+        sum_edge_case("cpu", (-12, -3, -1, 0, 1, 2, 6))
+
+
+@pytest.mark.gpu
+def test_cut_at_the_edge_of_the_sums_gpu():
+    sum_edge_case("cuda", range(-24, 25))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("seed,rows,V,style,temperature,top_p,min_p,with_prev", GPU_CASES)
 def test_sample_rows_gpu(seed, rows, V, style, temperature, top_p, min_p, with_prev):
