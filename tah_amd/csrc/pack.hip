@@ -91,7 +91,9 @@ __global__ __launch_bounds__(kScanThreads) void hard_index_kernel(const uint8_t*
 // entry f in that form, both -1 where there is none, and the form's padding.
 __global__ __launch_bounds__(256) void left_index_kernel(const int32_t* cu, const int32_t* flat, const int32_t* rank, int B, int S, int width,
                                                          int32_t* left, int32_t* back, uint8_t* pad) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int64_t at0 = (int64_t)blockIdx.x * 256 + threadIdx.x;  // (the last workgroup's may lie past 2^31)
+    if (at0 >= (int64_t)B * (S > width ? S : width)) return;
+    const int i = (int)at0;
     if (i < B * width) {
         const int b = i / width, at = cu[b] + i % width;
         const bool there = at < cu[b + 1];
@@ -148,8 +150,8 @@ __device__ __forceinline__ void select_rows(const tah_select_rows& t, const int3
     unsigned char* const dst = static_cast<unsigned char*>(t.dst);
     if (per_row < kWave / 2) {  // short rows: as many as fit to a wave
         const int in_wave = kWave / per_row, lane = threadIdx.x % kWave, mine = lane / per_row, c = lane - mine * per_row;
-        for (int r0 = ((int)blockIdx.x * 4 + (int)threadIdx.x / kWave) * in_wave; r0 < rows; r0 += (int)gridDim.x * 4 * in_wave) {
-            const int r = r0 + mine;
+        for (int64_t r0 = ((int64_t)blockIdx.x * 4 + threadIdx.x / kWave) * in_wave; r0 < rows; r0 += (int64_t)gridDim.x * 4 * in_wave) {
+            const int64_t r = r0 + mine;
             if (mine >= in_wave || r >= rows) continue;
             const int from = index[r];
             V v = {};
@@ -158,7 +160,7 @@ __device__ __forceinline__ void select_rows(const tah_select_rows& t, const int3
         }
         return;
     }
-    for (int r = (int)blockIdx.x * 4 + (int)threadIdx.x / kWave; r < rows; r += (int)gridDim.x * 4) {  // a wave to a row
+    for (int64_t r = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave; r < rows; r += (int64_t)gridDim.x * 4) {  // a wave to a row
         const int from = index[r];
         const V* const s = reinterpret_cast<const V*>(src + from * t.src_stride_bytes);
         V* const d = reinterpret_cast<V*>(dst + r * t.row_bytes);
@@ -248,7 +250,7 @@ extern "C" int tah_left_index_build(const int32_t* cu, const int32_t* flat, cons
     const int n = B * (S > width ? S : width);
     if (n == 0) return TAH_OK;
     if (!cu || (B * S > 0 && (!flat || !rank || !back)) || (B * width > 0 && (!left || !pad))) return TAH_E_NULL;
-    hipLaunchKernelGGL(left_index_kernel, dim3((n + 255) / 256), dim3(256), 0, static_cast<hipStream_t>(stream), cu, flat, rank, B, S, width, left,
+    hipLaunchKernelGGL(left_index_kernel, dim3((unsigned)(((int64_t)n + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream), cu, flat, rank, B, S, width, left,
                        back, pad);
     return hipGetLastError() == hipSuccess ? TAH_OK : TAH_E_LAUNCH;
 }
