@@ -6,7 +6,7 @@ import torch
 from oracle import duo_oracle as O
 from tests.cases import make_dense_case
 from tests.test_host_layer import (_deeper_levels, caller_position_ids, _forward_two_depths, _forward_two_depths_reference_style, _loops_over_depths,
-                                   _oracle_two_depths, check_depth_gradients, check_depth_outputs)
+                                   _oracle_two_depths, check_depth_gradients, check_depth_outputs, padded_gradients_case)
 
 pytestmark = pytest.mark.gpu
 
@@ -22,6 +22,13 @@ def test_forward_loop_matches_dense_reference_gpu(B, T, p, left_pad):
     np.testing.assert_allclose(o1.cpu()[valid].float().numpy(), w1[valid].numpy(), atol=2e-2, rtol=2e-2)
     assert (o1.cpu()[~valid] == 0).all()
     np.testing.assert_allclose(o2.cpu()[~pad.cpu()].float().numpy(), w2[~wpad].numpy(), atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("B,T,lens,left,Hq,Hkv,paired", [(3, 300, [300, 170, 64], False, 4, 2, True), (4, 260, [129, 260, 200, 100], True, 16, 8, True),
+                                                         (1, 512, [300], True, 4, 1, True), (2, 200, [64, 33], False, 4, 4, False)])
+def test_gradients_of_padded_blocks_gpu(monkeypatch, B, T, lens, left, Hq, Hkv, paired):
+    """Where they lie, and (less than half of them valid) packed."""
+    padded_gradients_case(monkeypatch, B, T, lens, left, Hq, Hkv, paired=paired, device="cuda")
 
 
 def test_reference_style_loop_with_dense_masks_gpu():

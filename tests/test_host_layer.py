@@ -242,6 +242,52 @@ def test_forward_loop_gradients(emu):
         assert err < 3e-2, (n, float(err))
 
 
+def padded_gradients_case(monkeypatch, B, T, lens, left, Hq, Hkv, paired=True, device="cpu"):
+    """Gradients of both depths through the callable, blocks of padded rows where they lie (every block reads its count back, as large ones
+    do): against the dense oracle in float64, NaN in every pad row of the inputs and of the outputs' gradients, exact zeros in the
+    pad rows' gradients and in those of rows that are not hard."""
+    import tah_amd.attention as A
+    from tah_amd.cache import TaHDuoCache
+    monkeypatch.setattr(A, "NO_SYNC_ROWS", 0)
+    masks = []
+    real = A.build_attention_mask
+    monkeypatch.setattr(A, "build_attention_mask", lambda *a, **k: masks.append(real(*a, **k)) or masks[-1])
+    c = make_dense_case(90 + sum(lens), B=B, T=T, p_hard=0.25, Hq=Hq, Hkv=Hkv, D=128)
+    at, n = torch.arange(T)[None], torch.tensor(lens)[:, None]
+    c["valid"] = ((at >= T - n) if left else (at < n)).long()
+    valid = c["valid"].bool()
+    c["hard"] &= valid
+    c["hard"][:, T - 1 if left else 0] = True  # (every sequence has one)
+    rows = lambda m: m[:, None, :, None]
+    names = ("q1", "k1", "v1", "q2", "k2", "v2")
+    kept = {x: valid if x[1] == "1" else c["hard"] for x in names}
+    ref = {x: torch.where(rows(kept[x]), c[x], 0.0).to(torch.bfloat16).double().requires_grad_(True) for x in names}
+    c.update({x: torch.where(rows(kept[x]), c[x], float("nan")) for x in names})
+    t, o1, o2, pad = _forward_two_depths(c, TaHDuoCache(), requires_grad=True, device=device)
+    assert masks[0]._packed.paired == paired and (masks[0]._packed.rows is None) == paired and not masks[1]._packed.paired
+    g = torch.Generator().manual_seed(4)
+    w1, w2 = [torch.randn(o.shape, generator=g).to(torch.bfloat16) for o in (o1, o2)]
+    pad = pad.cpu()
+    nan = lambda w, m: torch.where(m[:, :, None, None], w, float("nan")).to(device)
+    got = torch.autograd.grad((o1, o2), [t[x] for x in names], (nan(w1, valid), nan(w2, ~pad)))
+    r1, r2, rpad = O.duo_prefill_dense(*[ref[x] for x in names], c["hard"], c["scale"], valid_mask=c["valid"])
+    assert torch.equal(pad, rpad)
+    zero = lambda w, m: torch.where(m[:, :, None, None], w.double(), 0.0)
+    want = torch.autograd.grad((r1, r2), [ref[x] for x in names], (zero(w1, valid), zero(w2, ~pad)))
+    for x, a, b in zip(names, got, want):
+        a = a.float().cpu()
+        assert (a.masked_select(~rows(kept[x])) == 0).all(), x
+        # (the bound of the other gradient tests of this loop)
+        err = (a - b).abs().max() / b.abs().max()
+        assert err < 3e-2, (x, float(err))
+
+
+@pytest.mark.parametrize("B,T,lens,left,Hq,Hkv", [(2, 40, [40, 23], False, 2, 1), (2, 36, [36, 20], True, 2, 2),
+                                                  (1, 70, [66], True, 2, 1)])  # (one sequence, heads apart: rows 128 elements apart)
+def test_gradients_of_padded_blocks_where_they_lie(emu, monkeypatch, B, T, lens, left, Hq, Hkv):
+    padded_gradients_case(monkeypatch, B, T, lens, left, Hq, Hkv)
+
+
 def test_positions_changed_between_forward_and_backward_are_an_error(emu):
     """32-bit positions of a block without a valid mask are taken where they lie: a caller that writes to them before the backward
     gets autograd's error, not gradients of other positions; left alone, the same gradients come out as from a copy."""
