@@ -266,10 +266,10 @@ def bench_fwd_bwd(name: str, seqlens, p_hard: float, seed: int, steps: int, warm
                          "three_kernel_backward": "dQ and dK/dV each recompute S and dP (7 products per tile pair), no workspace"},
             "tflops": tf, "roofline": {"bound": "mfma", "achieved": tf, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                                        "frac": tf / PEAK_BF16_TFLOPS, "traffic": traffic,
-                                       "kernels": "duo_fwd_kernel + duo_bwd_delta_kernel x2 + duo_bwd_dkdv_kernel (dS export) + "
+                                       "kernels": "duo_fwd_kernel + duo_bwd_delta_kernel + duo_bwd_dkdv_kernel (dS export) + "
                                                   "duo_bwd_dq_from_ds_kernel",
                                        "kernel_ms": {"forward (duo_fwd_kernel)": half["fwd"],
-                                                     "backward (delta x2, dkdv + dS export, dq from dS)": half["bwd"]},
+                                                     "backward (delta, dkdv + dS export, dq from dS)": half["bwd"]},
                                        "frac_forward": fwd_flops / (half["fwd"] * 1e-3) / 1e12 / PEAK_BF16_TFLOPS,
                                        "frac_backward": 2.5 * fwd_flops / (half["bwd"] * 1e-3) / 1e12 / PEAK_BF16_TFLOPS},
             "tokens_per_s": sum(seqlens) / (ms * 1e-3)}

@@ -11,7 +11,8 @@
  * [cu[b], cu[b+1]) of a [rows, heads, D] bf16 tensor whose innermost D elements
  * are contiguous; row and head strides are given in elements.  (Boundaries given as
  * pairs, `cu_pairs`: rows [cu[2b], cu[2b+1]), ascending, with rows in between that belong
- * to no sequence and are neither read nor written -- padded batches where they lie.)  Only valid tokens
+ * to no sequence -- padded batches where they lie.  Such rows have to be addressable; no result depends on what
+ * they hold, and of a call's results they are left as they are.)  Only valid tokens
  * are packed, so within a sequence the depth-0 ("iteration 1") key at local
  * index j has position j, and a depth-0 query at local index i has position
  * i + (Lk1 - Lq1) (queries are the newest rows of the sequence).  Depth-1

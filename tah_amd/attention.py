@@ -223,7 +223,7 @@ class _Packed:
 
     A padded block (every sequence's valid rows lie together, depth 0: no positions) is not moved at all: the kernels take its rows where
     they lie, ``cu`` then holds (first row, one past the last) pairs, ``paired``.  Its pad rows come out as zeros, as from a scatter, and
-    what they hold is not read.  Two layers of four sequences of 1024 to 3210 rows, forward and backward: 2.62 -> 2.05 ms with
+    what they hold changes nothing.  Two layers of four sequences of 1024 to 3210 rows, forward and backward: 2.62 -> 2.05 ms with
     :class:`_BlockAttn` (row moves, clears and the gradients of empty slices were 0.5 of it, and the host's 105 launches behind the hard
     tokens' read-back the rest).  The backward's dS workspace counts the valid rows alone, as for packed ones.  Two layers' depth-0 calls, forward and
     backward, in place and packed: 2.03 and 2.33 ms (8 x 4096, 57 % valid), 6.90 and 7.47 (8 x 8192, 57 %), 4.22 and 4.52 (38 %), 0.83 and

@@ -1160,7 +1160,9 @@ __global__ __launch_bounds__(kLinThreads, kMore ? 2 : 4) void norm_linear_kernel
 // ---- the parts of a windowed attention's split call and the output projection behind them in one launch -------
 // One or two rows: merging a call's parts was a launch of 4.7 us for 42 KB a row, and the projection behind it another of 4.5. Here
 // every workgroup of the projection merges the row for itself (a compute unit takes 42 KB in in 0.4 us), its weights on their way.  The
-// same bits as window_merge_kernel and tah_linear_rows leave.  From three rows on the parts cost more than the launch: two launches.
+// same bits as window_merge_kernel and tah_linear_rows leave.  From three rows on the parts cost more than the launch: two launches.  Heads
+// of 2048 columns together and no other width (K per wave is the template's, as in norm_linear_kernel: no other is built or measured):
+// there, too, two launches.
 // One row of 16 heads in five parts, 2048 -> 2048, in a captured step: 4.7 + 4.5 -> 5.5 us.
 template <int F, bool H8>
 __global__ __launch_bounds__(kLinThreads) void merge_linear_kernel(const MergeLinear p, const LinearOut out, const bf16x8* weights) {

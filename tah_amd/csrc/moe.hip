@@ -28,95 +28,95 @@ constexpr int kTile = TAH_MOE_TILE;
 // One row's experts from its logits, by one wave.  zr: the logits in LDS, behind them the shared expert's where there is a gate.
 __device__ __forceinline__ void choose_experts(const tah_moe_route_args& p, float* const zr, int row, int lane) {
     const int experts = p.experts, top = p.top;
-            if (p.gate_w && lane == 0) p.shared_gate[row] = sigmoid_exact(zr[experts]);
-            if (p.score == TAH_MOE_SIGMOID) {
-                for (int e = lane; e < experts; e += kWave) zr[e] = sigmoid_exact(zr[e]);
-                TAH_WAVE_LDS_SYNC();
+    if (p.gate_w && lane == 0) p.shared_gate[row] = sigmoid_exact(zr[experts]);
+    if (p.score == TAH_MOE_SIGMOID) {
+        for (int e = lane; e < experts; e += kWave) zr[e] = sigmoid_exact(zr[e]);
+        TAH_WAVE_LDS_SYNC();
+    }
+    if (p.keep < p.groups) {
+        // a lane's groups: the sum of their two largest scores; then the best groups one after another, and the others'
+        // experts leave the race
+        const int size = experts / p.groups;
+        float gs[kGroupsPerLane];
+#pragma unroll
+        for (int u = 0; u < kGroupsPerLane; ++u) {
+            const int gr = lane + kWave * u;
+            float a = kNegInf, b = kNegInf;
+            for (int i = 0; gr < p.groups && i < size; ++i) {
+                const float v = zr[gr * size + i];
+                b = fmaxf(b, fminf(a, v));
+                a = fmaxf(a, v);
             }
-            if (p.keep < p.groups) {
-                // a lane's groups: the sum of their two largest scores; then the best groups one after another, and the others'
-                // experts leave the race
-                const int size = experts / p.groups;
-                float gs[kGroupsPerLane];
-    #pragma unroll
-                for (int u = 0; u < kGroupsPerLane; ++u) {
-                    const int gr = lane + kWave * u;
-                    float a = kNegInf, b = kNegInf;
-                    for (int i = 0; gr < p.groups && i < size; ++i) {
-                        const float v = zr[gr * size + i];
-                        b = fmaxf(b, fminf(a, v));
-                        a = fmaxf(a, v);
-                    }
-                    gs[u] = gr < p.groups ? (size > 1 ? a + b : a) : kNegInf;
-                }
-                uint32_t open = 0;  // bit u: group lane + 64 u is open
-                if (p.groups <= kWave) {  // a lane's group is open when fewer than `keep` are in front of it
-                    int before = 0;
-                    for (int g = 0; g < p.groups; ++g) {
-                        const float o = lane_value(gs[0], g);
-                        before += o > gs[0] || (o == gs[0] && g < lane);
-                    }
-                    open = gs[0] > kNegInf && before < p.keep;
-                } else for (int j = 0; j < p.keep; ++j) {
-                    float bv = kNegInf;
-                    int bi = 0x7fffffff;
-    #pragma unroll
-                    for (int u = 0; u < kGroupsPerLane; ++u)
-                        if (!(open >> u & 1) && gs[u] > bv) { bv = gs[u]; bi = lane + kWave * u; }
-    #pragma unroll
-                    for (int m = 32; m >= 1; m >>= 1) {
-                        const float ov = __shfl_xor(bv, m);
-                        const int oi = __shfl_xor(bi, m);
-                        if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-                    }
-                    if (bi % kWave == lane && bi < p.groups) open |= 1u << (bi / kWave);
-                }
-    #pragma unroll
-                for (int u = 0; u < kGroupsPerLane; ++u) {
-                    const int gr = lane + kWave * u;
-                    for (int i = 0; gr < p.groups && !(open >> u & 1) && i < size; ++i) zr[gr * size + i] = kNegInf;
-                }
-                TAH_WAVE_LDS_SYNC();
+            gs[u] = gr < p.groups ? (size > 1 ? a + b : a) : kNegInf;
+        }
+        uint32_t open = 0;  // bit u: group lane + 64 u is open
+        if (p.groups <= kWave) {  // a lane's group is open when fewer than `keep` are in front of it
+            int before = 0;
+            for (int g = 0; g < p.groups; ++g) {
+                const float o = lane_value(gs[0], g);
+                before += o > gs[0] || (o == gs[0] && g < lane);
             }
-            // the largest scores one after another, the lower index among equals; a chosen one leaves the race
-            float mine = kNegInf, first = 0.f;
-            int my_index = 0;
-            float v[kUnitsHeld];  // scores of experts lane, lane + 64, ... while they are in the race
-    #pragma unroll
-            for (int u = 0; u < kUnitsHeld; ++u) v[u] = lane + kWave * u < experts ? zr[lane + kWave * u] : kNegInf;
-            const bool held = experts <= kUnitsHeld * kWave;
-            for (int j = 0; j < top; ++j) {
-                float bv = kNegInf;
-                int bi = 0x7fffffff;
-                if (held) {
-    #pragma unroll
-                    for (int u = 0; u < kUnitsHeld; ++u)
-                        if (v[u] > bv) { bv = v[u]; bi = lane + kWave * u; }
-                } else {
-                    for (int e = lane; e < experts; e += kWave) {
-                        const float o = zr[e];
-                        if (o > bv) { bv = o; bi = e; }
-                    }
-                }
-                const float largest = wave_max_quick(bv);
-                bi = wave_min_quick(bv == largest ? bi : 0x7fffffff);
-                if (bi >= experts) bi = j;  // (only when the logits are not numbers)
-                if (j == 0) first = largest;
-                if (lane == j) { mine = largest; my_index = bi; }
-                if (held) {
-    #pragma unroll
-                    for (int u = 0; u < kUnitsHeld; ++u) v[u] = lane + kWave * u == bi ? kNegInf : v[u];
-                } else {
-                    if (lane == 0) zr[bi] = kNegInf;
-                    TAH_WAVE_LDS_SYNC();
-                }
+            open = gs[0] > kNegInf && before < p.keep;
+        } else for (int j = 0; j < p.keep; ++j) {
+            float bv = kNegInf;
+            int bi = 0x7fffffff;
+#pragma unroll
+            for (int u = 0; u < kGroupsPerLane; ++u)
+                if (!(open >> u & 1) && gs[u] > bv) { bv = gs[u]; bi = lane + kWave * u; }
+#pragma unroll
+            for (int m = 32; m >= 1; m >>= 1) {
+                const float ov = __shfl_xor(bv, m);
+                const int oi = __shfl_xor(bi, m);
+                if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
             }
-            const float w = lane < top ? expf(mine - first) : 0.f;
-            const float sum = wave_sum(w);
-            if (lane < top) {
-                p.index[(int64_t)row * top + lane] = my_index;
-                p.weight[(int64_t)row * top + lane] = p.score == TAH_MOE_SIGMOID ? mine : w / sum;
+            if (bi % kWave == lane && bi < p.groups) open |= 1u << (bi / kWave);
+        }
+#pragma unroll
+        for (int u = 0; u < kGroupsPerLane; ++u) {
+            const int gr = lane + kWave * u;
+            for (int i = 0; gr < p.groups && !(open >> u & 1) && i < size; ++i) zr[gr * size + i] = kNegInf;
+        }
+        TAH_WAVE_LDS_SYNC();
+    }
+    // the largest scores one after another, the lower index among equals; a chosen one leaves the race
+    float mine = kNegInf, first = 0.f;
+    int my_index = 0;
+    float v[kUnitsHeld];  // scores of experts lane, lane + 64, ... while they are in the race
+#pragma unroll
+    for (int u = 0; u < kUnitsHeld; ++u) v[u] = lane + kWave * u < experts ? zr[lane + kWave * u] : kNegInf;
+    const bool held = experts <= kUnitsHeld * kWave;
+    for (int j = 0; j < top; ++j) {
+        float bv = kNegInf;
+        int bi = 0x7fffffff;
+        if (held) {
+#pragma unroll
+            for (int u = 0; u < kUnitsHeld; ++u)
+                if (v[u] > bv) { bv = v[u]; bi = lane + kWave * u; }
+        } else {
+            for (int e = lane; e < experts; e += kWave) {
+                const float o = zr[e];
+                if (o > bv) { bv = o; bi = e; }
             }
+        }
+        const float largest = wave_max_quick(bv);
+        bi = wave_min_quick(bv == largest ? bi : 0x7fffffff);
+        if (bi >= experts) bi = j;  // (only when the logits are not numbers)
+        if (j == 0) first = largest;
+        if (lane == j) { mine = largest; my_index = bi; }
+        if (held) {
+#pragma unroll
+            for (int u = 0; u < kUnitsHeld; ++u) v[u] = lane + kWave * u == bi ? kNegInf : v[u];
+        } else {
+            if (lane == 0) zr[bi] = kNegInf;
+            TAH_WAVE_LDS_SYNC();
+        }
+    }
+    const float w = lane < top ? expf(mine - first) : 0.f;
+    const float sum = wave_sum(w);
+    if (lane < top) {
+        p.index[(int64_t)row * top + lane] = my_index;
+        p.weight[(int64_t)row * top + lane] = p.score == TAH_MOE_SIGMOID ? mine : w / sum;
+    }
 }
 
 // LDS: rows [RB][cols] float32, logits [RB][experts + 1]

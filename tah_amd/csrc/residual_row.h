@@ -1,6 +1,7 @@
 // A row of the residual stream on its way past a norm: the sum with a sublayer's normed result and the norm and short convolution in
-// front of the next sublayer.  Shared by residual_norm_kernel (row_norm.hip), which writes what the next launch reads, and by
-// norm_linear_kernel (linear_rows.hip), whose workgroups each make the rows' operand for themselves.
+// front of the next sublayer.  Shared by residual_norm_kernel (row_norm.hip), which writes what the next launch reads, by
+// norm_linear_kernel (linear_rows.hip), whose workgroups each make the rows' operand for themselves, and by
+// moe_norm_route_kernel (moe.hip), whose workgroup goes on to choose its row's experts.
 #pragma once
 #include "mixer_device.h"
 

@@ -544,8 +544,8 @@ class TaHDecodeEngine(DecodeEngine):
             self.x_mid, *self.x_turn = [torch.zeros(batch, cfg.hidden, dtype=torch.bfloat16, device=dev) for _ in range(3)]
             self.arrived = torch.zeros(cfg.layers, ops.LINEAR_CHAIN_WORDS, dtype=torch.int32, device=dev)
         self.pass_open = False  # a pass has begun and not ended: the words are not to be relied on
-        # the step's element-wise glue in two launches (tah_step_begin, tah_decider_tail) and the decider's first layer
-        # on the linear-layer kernel, instead of some twenty torch launches; needs the packed rows
+        # the step's element-wise glue in two launches (tah_step_begin; the decision with the mix, tah_decide_mix) and the
+        # decider's first layer on the linear-layer kernel, instead of some twenty torch launches; needs the packed rows
         self.fused_glue = bool(self.packed_linear and weights.lm_head_p is not None and
                                (decider is not None or (weights.dec_w1_p is not None and cfg.decider_hidden % 8 == 0)))
         if self.fused_glue:

@@ -49,7 +49,7 @@ def duo_fwd_varlen(q1, k1, v1, cu_q1, cu_k1, q2, k2, v2, pos_q2, pos_k2, cu_q2, 
     q2 [T2q,Hq,D], k2/v2 [T2k,Hkv,D], pos_q2/pos_k2 int32, cu_q2/cu_k2: depth-1 stream
     (hard tokens).  ``schedule``: table from :func:`duo_schedule` or None.  ``pairs``: the sum of 1, 2, 4, 8 for
     cu_q1, cu_k1, cu_q2, cu_k2 that hold (first row, one past the last) pairs, int32 [2 * nseq], ascending, with rows in between that
-    belong to no sequence: what they hold is not read, their rows of o are zeros (of lse undefined).
+    belong to no sequence: what they hold changes nothing, their rows of o are zeros (of lse undefined).
     Returns o1, lse1 [Hq,T1q], o2, lse2 [Hq,T2q].
     """
     return _call("duo_fwd_varlen", q1, k1, v1, cu_q1, cu_k1, q2, k2, v2, pos_q2, pos_k2, cu_q2, cu_k2, float(scale), schedule, int(pairs))

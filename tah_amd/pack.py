@@ -3,8 +3,8 @@
 ``gather_active`` and ``scatter_back`` mirror tah/model/tah_model.py:96-176:
 same arguments, same return values, same row-major packing order, same
 padding.  The index work (stream compaction of the mask) and every row move run
-in HIP kernels (tah_hard_index_build, tah_pad_rows_build, tah_rows_copy); torch
-only allocates and fills buffers.  Floating-point tensors stay differentiable:
+in HIP kernels (tah_mask_index_build, tah_left_index_build, tah_rows_select,
+tah_pad_rows_build, tah_rows_copy); torch only allocates and fills buffers.  Floating-point tensors stay differentiable:
 the backward of a row gather is a row scatter and vice versa.
 """
 from __future__ import annotations
