@@ -259,8 +259,8 @@ typedef struct tah_moe_route_args {
 int tah_moe_route(const tah_moe_route_args* args, tah_stream_t stream);
 /* tah_residual_norm and tah_moe_route on what comes out of it (the normed row, x_elem, or without next_coef the new residual row) in one
  * launch, for rows of tah_norm_route_supported() sizes, bf16: the bits of the two calls.  norm: without experts' rows and
- * convolution.  The new residual rows go to x_out [rows, cols], which lies on nothing that is read (TAH_E_SHAPE where it does);
- * route->x is not read. */
+ * convolution.  The new residual rows go to x_out [rows, cols], which lies on nothing that is read, the choice of experts lies on nothing that
+ * the norm reads or leaves, and neither on the router (TAH_E_SHAPE where they do); route->x is not read. */
 int tah_norm_route_supported(int32_t rows, int32_t cols, int32_t experts, int32_t gate);
 int tah_norm_route(const tah_residual_norm_args* norm, float* x_out, const tah_moe_route_args* route, tah_stream_t stream);
 /* Rows sorted by expert, every expert's rows padded to whole tiles of TAH_MOE_TILE: source row of every place (-1:

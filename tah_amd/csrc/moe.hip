@@ -574,6 +574,21 @@ extern "C" int tah_norm_route(const tah_residual_norm_args* norm, float* x_out, 
         meet(norm->coef, 4ll * norm->cols) || meet(norm->next_coef, 4ll * norm->cols) || meet(norm->y_scale, 4ll * norm->rows) ||
         meet(a->router, 2ll * a->experts * a->cols) || meet(a->gate_w, 2ll * a->cols))
         return TAH_E_SHAPE;
+    // (in two calls the choice is stored when every row has been normed, and the router read; here while other rows are on their way)
+    const int64_t rows = norm->rows, cols = norm->cols;
+    const RowSpan chosen[] = {one_span(a->index, 4 * rows * a->top), one_span(a->weight, 4 * rows * a->top), one_span(a->gate_w ? a->shared_gate : nullptr, 4 * rows)};
+    const RowSpan left[] = {one_span(norm->xe, 2 * rows * cols), one_span(norm->x_packed, 64 * cols), one_span(norm->normed, 2 * rows * cols),
+                            one_span(norm->normed_packed, 64 * cols), one_span(x_out, 4 * rows * cols)};
+    const RowSpan read[] = {one_span(norm->x, 4 * rows * cols), RowSpan{norm->y, 2 * cols, 2 * norm->y_row_stride, norm->rows}, one_span(norm->coef, 4 * cols),
+                            one_span(norm->next_coef, 4 * cols), one_span(norm->y_scale, 4 * rows)};
+    const RowSpan router[] = {one_span(a->router, 2ll * a->experts * cols), one_span(a->gate_w, 2 * cols)};
+    const auto any_meet = [](const auto& some, const auto& others) {
+        for (const RowSpan& s : some)
+            for (const RowSpan& o : others)
+                if (spans_meet(s, o)) return true;
+        return false;
+    };
+    if (any_meet(chosen, left) || any_meet(chosen, read) || any_meet(chosen, router) || any_meet(left, router)) return TAH_E_SHAPE;
     if (!a->router || !a->index || !a->weight || (a->gate_w && !a->shared_gate)) return TAH_E_NULL;
     if (!aligned_16(a->router) || !aligned_16(a->gate_w) || !aligned_16(x_out)) return TAH_E_ALIGN;
     const NormRoute p{*norm, *a, x_out};

@@ -78,6 +78,32 @@ def test_norm_route_refuses_what_it_is_not_built_for():
             ops._call("norm_route", *args(x))  # results on what is read
 
 
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+def test_norm_route_refuses_a_choice_on_what_other_rows_read_or_leave():
+    """Two calls have an order, one launch has none: a row's experts may be stored before another row's norm has read its own."""
+    from tah_amd import ops
+
+    bf = torch.bfloat16
+    with emu_util.emulated():
+        def call(**kw):
+            t = dict(x=torch.randn(4, 64), out=torch.zeros(4, 64), coef=torch.ones(64), y=torch.randn(4, 64).to(bf), y_scale=torch.ones(4), nxt=torch.ones(64),
+                     normed=torch.zeros(4, 64, dtype=bf), packed=torch.zeros(32 * 64, dtype=bf), router=torch.randn(8, 64).to(bf),
+                     gate_w=torch.randn(1, 64).to(bf), index=torch.zeros(4, 2, dtype=torch.int32), weight=torch.zeros(4, 2), sg=torch.zeros(4))
+            for name, on in kw.items():  # (the result `name` at the start of tensor `on`)
+                t[name] = t[on].view(-1).view(t[name].dtype)[:t[name].numel()].view(t[name].shape)
+            ops._call("norm_route", t["x"], t["out"], t["coef"], 64, 1e-6, t["y"], t["y_scale"], None, t["nxt"], t["normed"], t["packed"], 1, 64, t["router"],
+                      t["gate_w"], t["index"], t["weight"], t["sg"], 0, 1, 1)
+
+        call()
+        call(normed="y")  # (row by row, as the norm alone takes it)
+        for name in ("index", "weight", "sg"):
+            for on in ("x", "y", "coef", "nxt", "out", "normed", "packed", "router") + (("y_scale", "gate_w") if name == "sg" else ()):
+                with pytest.raises(ops._capi.TahDuoError):
+                    call(**{name: on})
+        with pytest.raises(ops._capi.TahDuoError):
+            call(normed="router")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", CASES)
 def test_norm_route_gpu(case):
