@@ -83,10 +83,8 @@ class Linear:
         self.packed = ops.linear_pack_weight(self.w) if w.dtype == torch.bfloat16 else None
 
     def __call__(self, x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-        # Few rows (the wanted rows in front of the output head, a short turn): a product costs its weights there, which the decode
-        # step's kernel reads at the memory's rate and the library at half of it (one row, 622 MB: 90 us and 205).
-        if self.packed is not None and out is None and x.dim() == 2 and 0 < x.shape[0] <= ops.LINEAR_MAX_ROWS:
-            return self.rows(ops.linear_pack_rows(x.contiguous()), x.shape[0])
+        # (few rows too: the decode step's kernel takes one row of an output head of 622 MB in 90 us and the library in 205, but adds up in another
+        # order, and float32 logits that were rounded to bf16 then differ by whole bf16 steps)
         return torch.matmul(x, self.w.t(), out=out) if out is not None else x @ self.w.t()
 
     def rows(self, xp: torch.Tensor, rows: int, **kw):

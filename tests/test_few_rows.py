@@ -31,6 +31,29 @@ def test_linear_of_few_rows_gpu(rows):
     linear_case("cuda", rows, 4128, 2048)
 
 
+def library_case(dev, rows, n, k):
+    from tah_amd.mixers import Linear
+
+    g = torch.Generator().manual_seed(rows)
+    x, w = torch.randn(rows, k, generator=g).to(BF).to(dev), (torch.randn(n, k, generator=g) * k ** -0.5).to(BF).to(dev)
+    assert torch.equal(Linear(w)(x), x @ w.t())
+
+
+@pytest.mark.skipif(not emu_util.have_host_clang(), reason="host clang++ not available")
+@pytest.mark.parametrize("rows", [1, 32])
+def test_linear_of_few_rows_is_the_library_s(rows):
+    """Products of a prompt take the library's bits, few rows or many.  (Logits come as float32 numbers that were rounded to bf16: another order of
+    the sum moves some of them by a whole bf16 step.)"""
+    with emu_util.emulated():
+        library_case("cpu", rows, 1024, 2048)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 12, 32, 33])
+def test_linear_of_few_rows_is_the_library_s_gpu(rows):
+    library_case("cuda", rows, 4128, 2048)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("lens,hard", [([5], 2), ([20, 12], 32), ([20, 13], 33), ([200, 90], 3)])
 def test_prompts_of_few_rows_against_library_products_gpu(lens, hard):
